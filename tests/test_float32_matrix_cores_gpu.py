@@ -43,3 +43,65 @@ def test_product_at_the_edges_of_its_tiles(ops, N, K):  # noqa: F811
             gate, up = f64(full[:M, :N // 2]), f64(full[:M, N // 2:])
             want = gate / (1 + torch.exp(-gate)) * up
             assert ((f64(out) - want).abs() <= 16 * EPS * want.abs() + 1e-30).all(), M
+
+
+def case(entries, nh, nkv, hd, P, window, seed):
+    """Requests with pages scattered over a pool of rubbish; the queries of a step's last tokens, and float64's result."""
+    g = torch.Generator().manual_seed(seed)
+    lens = [s + n for n, s in entries]
+    each = [-(-n // P) for n in lens]
+    pages = sum(each) + 3
+    perm = torch.randperm(pages - 1, generator=g) + 1
+    pool = torch.full((pages, 2, nkv, P, hd), float("nan"))
+    vt = pool[:, 1].reshape(pages, nkv, hd, P)
+    table = torch.full((len(lens), max(each) + 1), -1, dtype=torch.int32)
+    qs, want, used = [], [], 0
+    for e, ((n, start), size) in enumerate(zip(entries, lens)):
+        k, v = torch.randn(size, nkv, hd, generator=g), torch.randn(size, nkv, hd, generator=g)
+        q = torch.randn(n, nh, hd, generator=g)
+        mine = perm[used:used + each[e]]
+        used += each[e]
+        for t in range(size):
+            pool[mine[t // P], 0, :, t % P] = k[t]
+            vt[mine[t // P], :, :, t % P] = v[t]
+        first = max(0, start - window + 1) // P if window else 0
+        table[e, first:each[e]] = mine[first:].to(torch.int32)        # pages behind the window were given back
+        i = torch.arange(start, size)[:, None]
+        j = torch.arange(size)[None, :]
+        hidden = (j > i) | ((i - j >= window) if window else False)
+        o = torch.empty(n, nh, hd, dtype=torch.float64)
+        for h in range(nh):
+            s = (f64(q[:, h]) @ f64(k[:, h * nkv // nh]).T / math.sqrt(hd)).masked_fill(hidden, float("-inf"))
+            o[:, h] = torch.softmax(s, -1) @ f64(v[:, h * nkv // nh])
+        qs.append(q.reshape(n, nh * hd))
+        want.append(o.reshape(n, nh * hd))
+    pool[:, 1] = vt.reshape(pages, nkv, P, hd)
+    return qs, dev(pool.reshape(pages, 2 * nkv, P, hd).contiguous()), table, want
+
+
+@pytest.mark.parametrize("nh,nkv,hd,P,window", [(2, 1, 16, 4, None), (6, 2, 48, 12, 37), (16, 8, 128, 16, None), (17, 1, 64, 16, 70),
+                                                (5, 5, 256, 4, None)])
+def test_attention_under_every_cut_of_a_step(ops, nh, nkv, hd, P, window):  # noqa: F811
+    """Portions that start at 0 and in the middle, of one row beyond a tile and of two, beside single tokens, one of them
+    alone in its context; rows never written hold NaN.  Within 2e-5 of float64 (a row's weights sum to one; scores of
+    some 4 sqrt(hd) / 2^24 and sums of hundreds of keys), and each row taken as a single token has the same bits."""
+    entries = [(65, 0), (1, 0), (18, 131), (1, 300), (2, 15), (1, 16)]
+    qs, pool, table, want = case(entries, nh, nkv, hd, P, window, seed=nh + hd)
+    q = dev(torch.cat(qs))
+    out = torch.full_like(q, 7.0)
+    args = (nh, nkv, hd, 1.0 / math.sqrt(hd), window)
+    ops.attention(FakeCtx(entries), View(dev(table)), q, pool, out, *args)
+    assert (f64(out) - torch.cat(want)).abs().max() < 2e-5
+    for row_in, e in ((0, 0), (40, 0), (64, 0), (7, 2), (17, 2), (1, 4)):
+        row = sum(n for n, _ in entries[:e]) + row_in
+        one = torch.empty(1, nh * hd, device="cuda")
+        ops.attention(FakeCtx([(1, entries[e][1] + row_in)]), View(dev(table[e:e + 1].contiguous())), q[row:row + 1].contiguous(), pool,
+                      one, *args)
+        assert torch.equal(one[0], out[row]), (row_in, e)
+    try:
+        ops.use_fast_attention = False
+        rows = torch.empty_like(q)
+        ops.attention(FakeCtx(entries), View(dev(table)), q, pool, rows, *args)
+    finally:
+        ops.use_fast_attention = True
+    assert (f64(rows) - f64(out)).abs().max() < 2e-5

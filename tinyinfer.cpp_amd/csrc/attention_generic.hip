@@ -1,10 +1,14 @@
-// Paged causal grouped-query attention, one workgroup per (token row, q head),
-// for any head size that is a multiple of 16 up to 256, any number of heads and
-// groups, any page size, with an optional window.  This is the attention of the
-// float32 path (chunk rows and decode rows alike) and the fallback of the
-// bfloat16 path for head sizes its fast kernels refuse.
+// Paged causal grouped-query attention for any head size that is a multiple of
+// 16 up to 256, any number of heads and groups, any page size, with an optional
+// window.
 //
-// A workgroup is 16 groups of 16 lanes.  Lane j of a group owns dims j, j+16, ...
+//   attention_f32_kernel   the float32 path: a step's portions and single tokens
+//                          on the 32-bit matrix instructions, pages of whole 4s
+//   attention_rows_kernel  one workgroup per (token row, q head): float32 in
+//                          other pages or without a step's lists, and the
+//                          bfloat16 path for head sizes its fast kernels refuse
+//
+// In attention_rows_kernel a workgroup is 16 groups of 16 lanes.  Lane j of a group owns dims j, j+16, ...
 // Group g walks keys lo+g, lo+g+16, ... with an online softmax; the 16 partial
 // results are merged in LDS with the usual rescaling.  Scores, softmax statistics
 // and the output accumulate in 32-bit.
@@ -128,7 +132,212 @@ extern "C" int ti_attention_rows(int dtype, const void* q, const void* pool, con
 }
 
 // ------------------------------------------------------------------------------------------------
-// The same walk for attention whose keys and values differ in size and whose scores are soft-capped:
+// float32 on the matrix cores.  A workgroup's eight wavefronts hold 16 columns: 16 consecutive tokens of one q head
+// (a portion; four workgroups a tile of 64 rows), or the q heads of one token that share a kv head (single tokens).
+// They walk the keys in blocks of 16:
+//   S^T (16 keys x 16 columns) = K (16 x hd) . Q^T      O^T (hd x 16) += V^T (hd x 16 keys) . P^T
+// both by v_mfma_f32_16x16x4_f32 with four consecutive entries a lane (loaded as one float4; both operands of a product
+// are permuted alike), so that the scores' layout is the second product's operand.  Block b belongs to wavefront
+// b mod 8 whatever the tile, and a block that a column may not see leaves it bit by bit as it was: a token's result
+// depends on its keys alone, however a step is cut.  Keys and values come straight from memory, the next block's while
+// one is multiplied; short contexts are bounded by the start and the merge.  (With the rows kernel below, one workgroup
+// per row and head, lane sums and one value a load, a portion of 300 tokens with 16 heads of 128 on 8 kv heads took
+// 201 us a layer, 5.6 ms of a prompt of Qwen3-0.6B's sizes.)
+#define AF_WAVES 8
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float af4;
+
+template <int DB, bool SINGLE>
+__global__ void __launch_bounds__(64 * AF_WAVES)
+attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool, const int* __restrict__ table,
+                     int table_stride, const int* __restrict__ pos, const int* __restrict__ slot,
+                     const int* __restrict__ rows, const int* __restrict__ tiles, const int* __restrict__ entries,
+                     float* __restrict__ out, int n_head, int n_kv, int P, float scale, int window) {
+  constexpr int HD = DB * 16;
+  __shared__ __attribute__((aligned(16))) float s_o[AF_WAVES][16][HD + 4];
+  __shared__ float s_m[AF_WAVES][16], s_l[AF_WAVES][16];
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r16 = lane & 15, quad = lane >> 4;
+  const int G = n_head / n_kv;
+  // the workgroup's columns: rows m_row .. of head `head0`, or heads head0 .. of row m_row
+  int m_row, head0, n_cols, kvh, p_first, p_last;
+  const int* tab;
+  if constexpr (SINGLE) {
+    const int parts = (G + 15) / 16;
+    m_row = rows ? rows[blockIdx.x] : blockIdx.x;
+    kvh = blockIdx.y / parts;
+    head0 = kvh * G + (blockIdx.y % parts) * 16;
+    n_cols = min(16, (kvh + 1) * G - head0);
+    p_first = p_last = pos[m_row];
+    tab = table + (size_t)slot[m_row] * table_stride;
+  } else {
+    const int entry = tiles[(blockIdx.x >> 2) * 2], row0 = entries[entry * 4];
+    m_row = tiles[(blockIdx.x >> 2) * 2 + 1] + (blockIdx.x & 3) * 16;
+    head0 = blockIdx.y;
+    kvh = head0 / G;
+    n_cols = min(16, row0 + entries[entry * 4 + 1] - m_row);
+    if (n_cols <= 0) return;
+    p_first = entries[entry * 4 + 2] + m_row - row0;
+    p_last = p_first + n_cols - 1;
+    tab = table + (size_t)entry * table_stride;
+  }
+  const int col = min(r16, n_cols - 1);             // columns past the end repeat the last one and are not stored
+  const size_t q_row = SINGLE ? (size_t)m_row * n_head + head0 + col : (size_t)(m_row + col) * n_head + head0;
+  const int hi = SINGLE ? p_last : p_first + col;
+  const int lo = (window > 0 && hi - window + 1 > 0) ? hi - window + 1 : 0;
+  const int lo_min = (window > 0 && p_first - window + 1 > 0) ? p_first - window + 1 : 0;
+
+  const size_t page_elems = (size_t)2 * n_kv * P * HD;
+  const float* k_head = pool + (size_t)kvh * P * HD;
+  const float* v_head = pool + ((size_t)n_kv + kvh) * P * HD;
+  af4 qf[DB], o[DB];
+#pragma unroll
+  for (int s = 0; s < DB; ++s) {
+    qf[s] = *reinterpret_cast<const af4*>(q + q_row * HD + s * 16 + quad * 4);
+    o[s] = af4{0.f, 0.f, 0.f, 0.f};
+  }
+  struct Block { af4 k[DB], v[DB]; int key0; bool have; };
+  auto load = [&](Block& f, int b) {                // keys past the last one repeat it, whatever their place holds
+    f.key0 = b * 16;
+    const int key = min(b * 16 + r16, p_last), v4 = min(b * 16 + quad * 4, p_last & ~3);
+    const int pk = tab[key / P], pv = tab[v4 / P];
+    f.have = pv >= 0;                               // a page given back behind the window holds nothing that is seen
+    const float* kp = k_head + (size_t)max(pk, 0) * page_elems + (size_t)(key % P) * HD + quad * 4;
+    const float* vp = v_head + (size_t)max(pv, 0) * page_elems + (size_t)r16 * P + (v4 % P);
+#pragma unroll
+    for (int s = 0; s < DB; ++s) f.k[s] = *reinterpret_cast<const af4*>(kp + s * 16);
+#pragma unroll
+    for (int d = 0; d < DB; ++d) f.v[d] = *reinterpret_cast<const af4*>(vp + (size_t)d * 16 * P);
+  };
+  float mx = -INFINITY, l = 0.f;
+  auto attend = [&](Block& f) {
+    af4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < DB; ++s) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (s % 2 == 0) s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(f.k[s][j], qf[s][j], s0, 0, 0, 0);
+        else s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(f.k[s][j], qf[s][j], s1, 0, 0, 0);
+      }
+    }
+    float sc[4], bm = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int key = f.key0 + quad * 4 + i;
+      sc[i] = (f.have && key >= lo && key <= hi) ? (s0[i] + s1[i]) * scale : -INFINITY;
+      bm = fmaxf(bm, sc[i]);
+      if (!f.have || key > p_last) {                // never written: any bits, and 0 times NaN is NaN
+#pragma unroll
+        for (int d = 0; d < DB; ++d) f.v[d][i] = 0.f;
+      }
+    }
+    bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
+    bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+    const float m_new = fmaxf(mx, bm);
+    const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+    const float alpha = expf(mx - m_safe);          // 1 where nothing new is seen; 0 in front of the first key
+    float w[4];
+    l *= alpha;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      w[i] = expf(sc[i] - m_safe);
+      l += w[i];
+    }
+    mx = m_new;
+#pragma unroll
+    for (int d = 0; d < DB; ++d) {
+      o[d] *= alpha;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.v[d][j], w[j], o[d], 0, 0, 0);
+    }
+  };
+  const int b_last = p_last / 16;
+  int b = lo_min / 16;
+  b += (wave - b % AF_WAVES + AF_WAVES) % AF_WAVES;
+  if (b <= b_last) {
+    Block f0;
+    if constexpr (DB > 8) {                         // two blocks of such heads do not fit in the registers
+      for (; b <= b_last; b += AF_WAVES) {
+        load(f0, b);
+        attend(f0);
+      }
+    } else {
+    Block f1;
+    load(f0, b);
+    for (;;) {
+      load(f1, min(b + AF_WAVES, b_last));
+      __builtin_amdgcn_sched_barrier(0);
+      attend(f0);
+      if ((b += AF_WAVES) > b_last) break;
+      load(f0, min(b + AF_WAVES, b_last));
+      __builtin_amdgcn_sched_barrier(0);
+      attend(f1);
+      if ((b += AF_WAVES) > b_last) break;
+    }
+    }
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+#pragma unroll
+  for (int d = 0; d < DB; ++d) *reinterpret_cast<af4*>(&s_o[wave][r16][d * 16 + quad * 4]) = o[d];
+  if (quad == 0) {
+    s_m[wave][r16] = mx;
+    s_l[wave][r16] = l;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < n_cols * HD; e += 64 * AF_WAVES) {
+    const int c = e / HD, d = e % HD;
+    float mm = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < AF_WAVES; ++w) mm = fmaxf(mm, s_m[w][c]);
+    float lt = 0.f, acc = 0.f;
+#pragma unroll
+    for (int w = 0; w < AF_WAVES; ++w) {
+      const float f = (s_m[w][c] == -INFINITY) ? 0.f : expf(s_m[w][c] - mm);
+      lt += s_l[w][c] * f;
+      acc += s_o[w][c][d] * f;
+    }
+    const size_t row = SINGLE ? (size_t)m_row * n_head + head0 + c : (size_t)(m_row + c) * n_head + head0;
+    out[row * HD + d] = acc / lt;
+  }
+}
+
+// A step's attention in float32: n_tiles tiles of up to 64 rows of portions (tiles int32 [n_tiles][2] = (entry, first
+// row), entries int32 [.][4] = (row0, tokens, first position, .), an entry being its own row of the block table) and
+// n_single rows of single tokens (row numbers in `rows`, or 0 .. n_single - 1).  3: sizes not served (what the head
+// and page sizes say, never the step: one kernel serves all steps of a model).
+extern "C" int ti_attention_f32(const void* q, const void* pool, const int* table, int table_stride, const int* pos, const int* slot,
+                                const int* rows, int n_single, const int* tiles, const int* entries, int n_tiles, void* out,
+                                int n_head, int n_kv, int hd, int page_size, float scale, int window, hipStream_t stream) {
+  TI_REQUIRE(n_head > 0 && n_kv > 0 && n_head % n_kv == 0, "attention: heads %d / kv_heads %d", n_head, n_kv);
+  TI_REQUIRE(n_head <= 65535, "attention: too many heads (%d)", n_head);
+  TI_REQUIRE(page_size > 0 && table_stride > 0, "attention: bad page_size %d / table_stride %d", page_size, table_stride);
+  TI_REQUIRE(n_tiles >= 0 && n_single >= 0 && (n_tiles == 0 || (tiles && entries)), "attention: %d tiles without their lists", n_tiles);
+  if (hd < 16 || hd > 256 || hd % 16 != 0 || page_size % 4 != 0) return 3;
+  const int parts = (n_head / n_kv + 15) / 16;
+#define AF_CASE(D)                                                                                                            \
+  case D:                                                                                                                     \
+    if (n_tiles)                                                                                                              \
+      attention_f32_kernel<D, false><<<dim3(n_tiles * 4, n_head), 64 * AF_WAVES, 0, stream>>>(                                \
+          (const float*)q, (const float*)pool, table, table_stride, pos, slot, rows, tiles, entries, (float*)out, n_head,     \
+          n_kv, page_size, scale, window);                                                                                    \
+    if (n_single)                                                                                                             \
+      attention_f32_kernel<D, true><<<dim3(n_single, n_kv * parts), 64 * AF_WAVES, 0, stream>>>(                              \
+          (const float*)q, (const float*)pool, table, table_stride, pos, slot, rows, tiles, entries, (float*)out, n_head,     \
+          n_kv, page_size, scale, window);                                                                                    \
+    break;
+  switch (hd / 16) {
+    AF_CASE(1) AF_CASE(2) AF_CASE(3) AF_CASE(4) AF_CASE(5) AF_CASE(6) AF_CASE(7) AF_CASE(8)
+    AF_CASE(9) AF_CASE(10) AF_CASE(11) AF_CASE(12) AF_CASE(13) AF_CASE(14) AF_CASE(15) AF_CASE(16)
+    default:
+      return 3;
+  }
+#undef AF_CASE
+  TI_LAUNCH_CHECK();
+  return 0;
+}
+
+// ------------------------------------------------------------------------------------------------
+// The same walk (a workgroup per row and head) for attention whose keys and values differ in size and whose scores are soft-capped:
 //   s = (q . k) * scale;  s <- softcap * tanh(s / softcap)  (softcap <= 0: none);  softmax over the
 // visible keys.  Any key size dk and value size dv up to 256 (lanes beyond a size idle).  A page is
 // K [n_kv][P][dk] | V [n_kv][dv][P]; with dk == dv that is the layout above.

@@ -95,7 +95,14 @@ int ti_attention_rows(int dtype, const void* q, const void* pool, const int* tab
                       const int* slot, void* out, int M, int n_head, int n_kv, int hd, int page_size, float scale,
                       int window, hipStream_t stream);
 
-// the same for keys and values of different sizes (dk, dv up to 256, any value in that range) and soft-capped scores:
+// a step's attention in float32 on the matrix cores: n_tiles tiles of up to 64 rows of portions, tiles int32 [n_tiles][2] =
+// (entry, first row) of entries int32 [.][4] = (row0, tokens, first position, .), and n_single rows of single tokens (their numbers
+// in rows, or the first n_single where it is null).  3: head or page size not served.
+int ti_attention_f32(const void* q, const void* pool, const int* table, int table_stride, const int* pos, const int* slot,
+                     const int* rows, int n_single, const int* tiles, const int* entries, int n_tiles, void* out, int n_head,
+                     int n_kv, int hd, int page_size, float scale, int window, hipStream_t stream);
+
+// attention of every row for keys and values of different sizes (dk, dv up to 256, any value in that range) and soft-capped scores:
 // s = (q . k) scale, then softcap tanh(s / softcap) if softcap > 0.  A page is K [n_kv][P][dk] | V [n_kv][dv][P].
 int ti_attention_capped_rows(int dtype, const void* q, const void* pool, const int* table, int table_stride,
                              const int* pos, const int* slot, void* out, int M, int n_head, int n_kv, int dk, int dv,

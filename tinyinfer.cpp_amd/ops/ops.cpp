@@ -875,6 +875,19 @@ bool Ops::attention(const AttentionWork& work, Workspace& ws, const CacheView& v
       }
     }
   }
+  if (q.dtype == DType::F32 && softcap <= 0.f && use.fast_attention && (work.n_tiles_small == 0 || (work.tiles_small && work.entry_meta)) &&
+      (work.decode_only || work.n_tiles_small || work.n_decode_rows)) {
+    check_pool("attention", pool, kv_heads, head_dim, DType::F32);
+    require(q.contiguous() && out.contiguous() && q.ndim == 2 && q.shape[1] == (int64_t)heads * head_dim && out.ndim == 2 &&
+                out.shape[0] == q.shape[0] && out.shape[1] == q.shape[1] && out.dtype == q.dtype,
+            "attention: q/out shapes or dtypes do not fit");
+    int rc = KERNEL("attention_generic", ti_attention_f32)(
+        q.data, pool.data, view.table, view.table_width, work.positions, work.slots, work.decode_only ? nullptr : work.decode_rows,
+        work.decode_only ? (int)work.M : work.n_decode_rows, work.tiles_small, work.entry_meta, work.decode_only ? 0 : work.n_tiles_small,
+        out.data, heads, kv_heads, head_dim, (int)pool.shape[2], scale, window, (hipStream_t)launch_stream());
+    done = rc == 0;
+    if (rc != 3) check("attention_generic", rc, "attention(float32)");
+  }
   took(done ? "[mfma]" : "[generic]");
   if (!done && sink) throw KernelError("attention: the matrix-core kernels refused sizes they were asked about, with a sink to join");
   if (!done && softcap > 0.f)
