@@ -18,6 +18,8 @@
 // per row of A for M <= 32.)
 #include <algorithm>
 #include <string>
+#include <type_traits>
+#include <utility>
 #include "common.h"
 #include "tinyinfer_kernels.h"
 #include "tinyinfer_kernels_tuning.h"
@@ -815,31 +817,26 @@ gemm_tiled_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, vo
 }
 
 // ====================================================== tiled kernel, pipelined
-// The same product with the tiles brought in by direct global-to-LDS loads
-// (global_load_lds_dwordx4: each lane fetches 16 bytes, the wavefront's 64 pieces
-// land in 1 KiB of LDS in lane order) three stages deep, so that two k-tiles are in
-// flight while one is multiplied (K must be a multiple of 64; other K take the plain
-// tiled kernel).  BK = 64: a tile row is 128 bytes = 8 pieces.  Rows
-// are stored unpadded, and piece c of row r sits in slot c ^ ((r >> 1) & 7): the 16
-// rows that one phase of a 16-byte LDS read touches then fall on all 64 banks once.
-// The lane that fills slot (r, c) simply fetches piece c ^ ((r >> 1) & 7) of row r.
+// The same product with the tiles brought in by direct memory-to-LDS loads
+// (buffer_load_dwordx4 ... lds: each lane fetches 16 bytes, the wavefront's 64 pieces
+// land in 1 KiB of LDS in lane order), STAGES - 1 k-tiles ahead of the one that is
+// multiplied (K must be a multiple of 64; other K take the plain tiled kernel).
+// BK = 64: a tile row is 128 bytes = 8 pieces, one line of the caches (k-tiles of 32,
+// half a line a row, take a third longer from memory).  Rows are stored unpadded, and
+// piece c of row r sits in slot c ^ ((r >> 1) & 7): the 16 rows that one phase of a
+// 16-byte LDS read touches then fall on all 64 banks once.  The lane that fills slot
+// (r, c) simply fetches piece c ^ ((r >> 1) & 7) of row r.
 //
-// WG tile BM x BN, four wavefronts as WAVES_M x WAVES_N, each (BM / WAVES_M) x
+// WG tile BM x BN, four or eight wavefronts as WAVES_M x WAVES_N, each (BM / WAVES_M) x
 // (BN / WAVES_N) out of 32 x 32 x 16 MFMAs.  SwiGLU needs two 32-column tiles per
-// wavefront: tile 0 holds gate columns, tile 1 the matching up columns.
+// wavefront: the first half holds gate columns, the second the matching up columns.
 #define PBK 64
 #define PSTAGES 3
 
-__device__ __forceinline__ void wait_vmcnt(int n) {
-  // s_waitcnt with only vmcnt set (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14)
-  switch (n) {
-    case 0: __builtin_amdgcn_s_waitcnt(0x0F70); break;
-#define TI_W(N) case N: __builtin_amdgcn_s_waitcnt(0x0F70 | ((N) & 15) | (((N) >> 4) << 14)); break;
-    TI_W(1) TI_W(2) TI_W(3) TI_W(4) TI_W(5) TI_W(6) TI_W(7) TI_W(8) TI_W(9) TI_W(10) TI_W(11) TI_W(12)
-    TI_W(13) TI_W(14) TI_W(15) TI_W(16) TI_W(20) TI_W(24)
-#undef TI_W
-    default: __builtin_amdgcn_s_waitcnt(0x0F70); break;
-  }
+// s_waitcnt with only vmcnt set (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14)
+template <int N> __device__ __forceinline__ void wait_vmcnt() {
+  static_assert(N >= 0 && N <= 63, "vmcnt counts to 63");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
 // What the epilogue TI_EPI_QKV_PREP needs: the product is the fused q/k/v projection of a step's
@@ -922,13 +919,18 @@ __device__ __forceinline__ void qkv_rows_by_lanes(const QKVEpilogue& ep, float* 
     qkv_rows_by_lanes<HD, BM, NWV, FS, false, false>(ep, ft, s_pos, s_page, s_prow, s_live, hh, u, m0);
 }
 
-// k-steps whose fragments are on their way from LDS while one is multiplied (two: a prompt of 2,048 tokens at
-// Qwen3-0.6B's sizes 0.7 % faster, at Qwen3-8B's 3.7 % slower)
-#define FRAG_AHEAD 1
-template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int STAGES = PSTAGES, int KT = PBK>
+// tile(n_k - LEFT, LEFT) for LEFT = STAGES - 2, ..., 0, as far as there are tiles
+template <class Tile, int... I>
+__device__ __forceinline__ void last_tiles(int n_k, Tile&& tile, std::integer_sequence<int, I...>) {
+  constexpr int N = (int)sizeof...(I);
+  ((n_k >= N - I ? (tile(n_k - (N - I), std::integral_constant<int, N - 1 - I>{}), 0) : 0), ...);
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int STAGES = PSTAGES>
 __global__ void __launch_bounds__(WAVES_M * WAVES_N * 64)
 gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ out_arg,
                       int M, int N, int K, long lda, int n_first, int xcd_rows, QKVEpilogue ep = QKVEpilogue{}) {
+#if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass has no buffer descriptors)
   // n_first: the output column the grid's first workgroup starts at (a launch may cover a range of columns)
   // xcd_rows > 0 (the grid's width is a multiple of 8 then): which tile a workgroup takes follows the eight
   // dies.  Workgroups go to the dies in turn, so die c has numbers c, c + 8, ...; it takes an eighth of the
@@ -954,13 +956,10 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
   constexpr int NWV = WAVES_M * WAVES_N;                     // wavefronts: 4 or 8
   static_assert(NWV == 4 || NWV == 8, "four or eight wavefronts");
   static_assert(!SW || TN % 2 == 0, "SwiGLU pairs the column tiles of a wavefront: the first half gate, the second half up");
-  static_assert(STAGES >= 2 && STAGES <= 4, "two to four stages");
-  // KT: the depth of a k-tile, 64 or 32.  A row of a stage is KT bfloat16 (CPR pieces of 16 bytes); a wavefront's
-  // load of 1 KiB covers RPL rows; piece c of row r lies in slot c ^ swz(r), so that the sixteen lanes of a
-  // fragment read (sixteen rows, one piece) touch sixteen different 16-byte columns of the banks
-  static_assert(KT == 64 || KT == 32, "k-tiles of 64 or 32");
-  constexpr int CPR = KT / 8, RPL = 64 / CPR, ROWB = KT * 2;
-  auto swz = [](int r) { return KT == 64 ? (r >> 1) & 7 : (r >> 2) & 3; };
+  static_assert(STAGES >= 2, "one stage is multiplied, the others are on their way");
+  // a row of a stage is KT bfloat16 (CPR pieces of 16 bytes); a wavefront's load of 1 KiB covers RPL rows
+  constexpr int KT = PBK, CPR = KT / 8, RPL = 64 / CPR, ROWB = KT * 2, KSTEPS = KT / 16;
+  auto swz = [](int r) { return (r >> 1) & 7; };
 
   constexpr int STAGE_BYTES = (BM + BN) * ROWB;
   constexpr int GROUPS_A = BM / RPL, GROUPS_B = BN / RPL;    // RPL rows = 1 KiB = one wavefront load
@@ -979,49 +978,36 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
   const int m0 = by * BM;
   const int n0 = n_first + bx * (SW ? BN / 2 : BN);
   const int lr = lane / CPR, lc = lane % CPR;                // row within a load's group of rows, slot within the row
-  const bool spread = K >= 4096;
 
-  // the global row each of this lane's loads reads (clamped into the matrix: rows
-  // beyond it are computed and thrown away), as a pointer to its first element
-  const bf16_t* gsrc[LOADS];
-  int gpiece[LOADS];                                         // which 8-element piece of the row this lane fetches
+  // A load's rows lie behind one of three descriptors (tokens, weight rows, up rows), which are scalar, as is where a k-tile
+  // starts; a lane's own offset stays the same from tile to tile, so that a load costs no vector arithmetic.  Rows beyond
+  // the matrix are clamped into it: they are computed and thrown away.
+  unsigned voff[LOADS];
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
     const int g = wave + NWV * i;                            // groups 0..GROUPS_A-1: A, then B
     if (g < GROUPS_A) {
       const int row = g * RPL + lr;
-      const int gm = min(m0 + row, M - 1);
-      gsrc[i] = A + (size_t)gm * lda;
-      gpiece[i] = lc ^ swz(row);
+      voff[i] = (unsigned)min(row, M - 1 - m0) * (unsigned)(lda * 2) + (lc ^ swz(row)) * 16;
     } else {
       const int row = (g - GROUPS_A) * RPL + lr;
-      int wr;
-      if (SW) {
-        constexpr int span = BN / WAVES_N, half = span / 2;  // LDS rows of one wavefront's columns: gate rows, then up rows
-        const int n = n0 + (row / span) * half + (row % half);
-        wr = ((row % span) >= half ? N : 0) + min(n, N - 1);
-      } else {
-        wr = min(n0 + row, N - 1);
-      }
-      gsrc[i] = W + (size_t)wr * K;
-      gpiece[i] = lc ^ swz(row);
+      constexpr int span = BN / WAVES_N, half = span / 2;    // SwiGLU: a wavefront's columns are gate rows, then up rows
+      const int n = SW ? (row / span) * half + (row % half) : row;
+      voff[i] = (unsigned)min(n, N - 1 - n0) * (unsigned)(K * 2) + (lc ^ swz(row)) * 16;
     }
   }
-
-  // load i of this wavefront's LOADS loads of k-tile kt
-  auto issue_one = [&](int kt, int i) {
-    unsigned char* stage = smem + (kt % STAGES) * STAGE_BYTES;
-    const int k0 = (kt0 + kt) * KT;
+  auto rows_at = [](const bf16_t* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
+  const auto rsA = rows_at(A + (size_t)m0 * lda + (size_t)kt0 * KT);
+  const auto rsW = rows_at(W + (size_t)n0 * K + (size_t)kt0 * KT);
+  const auto rsU = rows_at(W + (size_t)(n0 + (SW ? N : 0)) * K + (size_t)kt0 * KT);
+  // load i of this wavefront's LOADS loads of k-tile kt, into the stage at that byte
+  auto issue_one = [&](int kt, unsigned stage, int i) {
     const int g = wave + NWV * i;
-    unsigned char* dst = stage + g * 1024;                   // the same in every lane
-    // K is a multiple of 64 here (the dispatcher sees to it): no piece lies past the end
-    __builtin_amdgcn_global_load_lds(
-        (const __attribute__((address_space(1))) void*)(gsrc[i] + k0 + gpiece[i] * 8),
-        (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-  };
-  auto issue = [&](int kt) {
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) issue_one(kt, i);
+    auto* dst = (__attribute__((address_space(3))) void*)(smem + stage + g * 1024);      // the same in every lane
+    constexpr int span = BN / WAVES_N;
+    if (g < GROUPS_A) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, dst, 16, voff[i], kt * KT * 2, 0, 0);
+    else if (SW && ((g - GROUPS_A) * RPL) % span >= span / 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsU, dst, 16, voff[i], kt * KT * 2, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsW, dst, 16, voff[i], kt * KT * 2, 0, 0);
   };
 
   floatx16 acc[TM][TN];
@@ -1034,114 +1020,128 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
 
   // The multiply loop is scheduled by hand.  The compiler does not know which LDS
   // bytes a direct load will write, so before any LDS read it can see, and at every
-  // fence, it waits for all of them, the two k-tiles in flight included; that would
+  // fence, it waits for all of them, the k-tiles in flight included; that would
   // undo the pipeline.  So LDS is read with ds_read_b128 in inline assembly, the
-  // barrier is the bare instruction, and the waits are written out: vmcnt before the
-  // barrier (the tile about to be multiplied has landed), lgkmcnt before each group of
-  // MFMAs (its fragments have arrived; those of the next k-step are still in flight).
+  // barrier is the bare instruction, and the waits are written out.
+  //
+  // A k-step's matrix instructions stand one by one, and between them what the steps ahead need: the
+  // next step's fragments from LDS, and the loads of k-tile kt + STAGES - 1 (the unit that takes their
+  // addresses handles 64 bytes a cycle for the whole compute unit: asked for at once they would queue
+  // there with nothing on the matrix cores).  The last k-step's fragments are in registers before any
+  // of its matrix instructions, so the workgroup meets behind number GB of that step: then the tile's
+  // stage is free, tile kt + 1 has landed for every wavefront, and its first fragments are read behind
+  // the remaining instructions; no k-tile begins with a wait for LDS.  Whole tiles run without a branch,
+  // the last STAGES - 1 by themselves.
+  // (Against a loop that met in front of each k-tile, read its first fragments there and asked by lane
+  // addresses, us: 2048 x 24576 x 4096 with SwiGLU 382 -> 328, 2048 x 4096 x 12288 193 -> 167,
+  // 2048 x 4096 x 4096 70 -> 61, 2048 x 4096 x 1024 24 -> 22; the library's kernels 296, 180, 62 and 24.)
   const int fr = lane & 31, fh = lane >> 5;                  // fragment row, and which half of a 16-wide k-step
   const unsigned lds0 = (unsigned)(size_t)smem;              // LDS byte address of the first stage
   const unsigned rowA = lds0 + (wm * (BM / WAVES_M) + fr) * ROWB;
   const unsigned rowB = lds0 + BM * ROWB + (wn * (BN / WAVES_N) + fr) * ROWB;
-  unsigned xo[KT / 16];                                      // swizzled byte offset of this lane's piece, per k-step
+  unsigned xo[KSTEPS];                                       // swizzled byte offset of this lane's piece, per k-step
 #pragma unroll
-  for (int ks = 0; ks < KT / 16; ++ks) xo[ks] = ((ks * 2 + fh) ^ swz(fr)) << 4;
+  for (int ks = 0; ks < KSTEPS; ++ks) xo[ks] = ((ks * 2 + fh) ^ swz(fr)) << 4;
 
   // the residual an adding epilogue adds to: asked for while the last k-tile is multiplied
   // (elements outside the matrix read a valid one and are not stored)
   // (a tile of many accumulators has no registers for it and reads the residual in the epilogue)
   constexpr bool PREV = EPI == TI_EPI_ADD_F32 && (NWV == 4 || TM * TN <= 4);
   float prev[PREV ? TM : 1][PREV ? TN : 1][16];
+  constexpr int NR = TM + TN, NM = TM * TN;                  // fragment reads and matrix instructions of a k-step
+  constexpr int GB = NM >= 8 ? 2 : 0;
+  // matrix instructions of a k-tile that its loads are spread over: up to the barrier; where only one k-tile is ahead the
+  // first quarter, so that the loads have the rest of the tile to arrive in
+  constexpr int SPAN = STAGES == 2 ? NM : (KSTEPS - 1) * NM + GB + 1;
+  v4u fa[2][TM], fb[2][TN];
+  // fragment j of k-step ks of the stage at byte st
+  auto read_one = [&](unsigned st, int ks, int set, int j) {
+    const unsigned pa = rowA + st + xo[ks], pb = rowB + st + xo[ks];
 #pragma unroll
-  for (int st = 0; st < STAGES - 1; ++st)
-    if (st < n_k) issue(st);
-  for (int kt = 0; kt < n_k; ++kt) {
-    // tile kt has landed (its loads are older than those of the tiles after it), in every wavefront,
-    // and every wavefront has finished with the stage that tile kt + STAGES - 1 goes into
-    wait_vmcnt(min(STAGES - 2, n_k - 1 - kt) * LOADS);
-    __builtin_amdgcn_s_barrier();
-    // Tile kt + 2 goes into the stage that everyone has left.  Its loads go out between the k-steps
-    // below, each behind a k-step's matrix instructions: the unit that takes the addresses handles 64
-    // bytes a cycle for the whole compute unit, and eight wavefronts that ask for a whole tile at once
-    // queue there with nothing on the matrix cores meanwhile.
-    // (a prompt of 2,048 tokens 2.5 % faster at Qwen3-0.6B's sizes, 2.1 % at Qwen3-8B's; a k-tile of a 256 x 128
-    // tile from 2,480 to 2,200 cycles)
-    // (spread evenly between the matrix instructions where K is long, k-step by k-step where it is short: see below)
-    const bool more = kt + STAGES - 1 < n_k, more_spread = more && spread, more_steps = more && !spread;
-    if constexpr (PREV) {
-      if (kt == n_k - 1) {
+    for (int a = 0; a < TM; ++a)
+      if (a == j) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][a]) : "v"(pa), "n"(a * 32 * ROWB));
 #pragma unroll
-        for (int a = 0; a < TM; ++a)
+    for (int b = 0; b < TN; ++b)
+      if (b == j - TM) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[set][b]) : "v"(pb), "n"(b * 32 * ROWB));
+  };
 #pragma unroll
-          for (int b = 0; b < TN; ++b)
+  for (int t = 0; t < STAGES - 1; ++t)
+    if (t < n_k) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-              const int m = m0 + wm * (BM / WAVES_M) + a * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-              const int n = n0 + wn * (BN / WAVES_N) + b * 32 + (lane & 31);
-              prev[a][b][i] = ((const float*)out_)[(size_t)min(m, M - 1) * N + min(n, N - 1)];
-            }
-      }
+      for (int i = 0; i < LOADS; ++i) issue_one(t, t * STAGE_BYTES, i);
     }
-    const unsigned st = (kt % STAGES) * STAGE_BYTES;
-    // the fragments of FRAG_AHEAD k-steps are on their way from LDS while one is multiplied
-    constexpr int SETS = FRAG_AHEAD + 1, KSTEPS = KT / 16;
-    v4u fa[SETS][TM], fb[SETS][TN];
-    auto read_step = [&](int ks, int set) {
-      const unsigned pa = rowA + st + xo[ks], pb = rowB + st + xo[ks];
+  if (n_k >= STAGES - 1) wait_vmcnt<(STAGES - 2) * LOADS>();
+  else wait_vmcnt<0>();
+  __builtin_amdgcn_s_barrier();
+  if (n_k > 0) {
+#pragma unroll
+    for (int j = 0; j < NR; ++j) read_one(0, 0, 0, j);
+  }
+  unsigned st = 0, st_new = (STAGES - 1) * STAGE_BYTES;      // where tile kt lies, where tile kt + STAGES - 1 goes
+  // LEFT: how many tiles follow tile kt (STAGES: at least STAGES - 1)
+  auto tile = [&](int kt, auto left) {
+    constexpr int LEFT = decltype(left)::value;
+    constexpr bool MORE = LEFT >= STAGES - 1, NEXT = LEFT >= 1;
+    const unsigned st_next = st == (STAGES - 1) * STAGE_BYTES ? 0 : st + STAGE_BYTES;
+    if constexpr (PREV && LEFT == 0) {
 #pragma unroll
       for (int a = 0; a < TM; ++a)
-        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][a]) : "v"(pa), "n"(a * 32 * ROWB));
 #pragma unroll
-      for (int b = 0; b < TN; ++b)
-        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[set][b]) : "v"(pb), "n"(b * 32 * ROWB));
-    };
+        for (int b = 0; b < TN; ++b)
 #pragma unroll
-    for (int ks = 0; ks < FRAG_AHEAD; ++ks) read_step(ks, ks);
+          for (int i = 0; i < 16; ++i) {
+            const int m = m0 + wm * (BM / WAVES_M) + a * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
+            const int n = n0 + wn * (BN / WAVES_N) + b * 32 + (lane & 31);
+            prev[a][b][i] = ((const float*)out_)[(size_t)min(m, M - 1) * N + min(n, N - 1)];
+          }
+    }
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
-      const int set = ks % SETS;
-      if (ks + FRAG_AHEAD < KSTEPS) read_step(ks + FRAG_AHEAD, (ks + FRAG_AHEAD) % SETS);
-      // this k-step's fragments are there when only the reads issued after them are outstanding:
-      // those of the k-steps up to FRAG_AHEAD further on
-      constexpr int PER = TM + TN;
-      const int later = (KSTEPS - 1 - ks < FRAG_AHEAD ? KSTEPS - 1 - ks : FRAG_AHEAD) * PER;
-      static_assert(FRAG_AHEAD * PER <= 15, "lgkmcnt counts to 15");
-      switch (later) {
-#define TI_LGKM(N) case N: asm volatile("s_waitcnt lgkmcnt(" #N ")" ::: "memory"); break;
-        TI_LGKM(0) TI_LGKM(2) TI_LGKM(3) TI_LGKM(4) TI_LGKM(6) TI_LGKM(7) TI_LGKM(8) TI_LGKM(12) TI_LGKM(14)
-#undef TI_LGKM
-        default: asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); break;
-      }
-      // tie the fragments to the wait, so that no MFMA is moved above it
+      const int set = ks & 1;
+      constexpr int LAST = KSTEPS - 1;
+      // this step's fragments have arrived (the next step's are asked for below); tied to the wait, so that no
+      // matrix instruction is moved above it
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
       for (int a = 0; a < TM; ++a) asm volatile("" : "+v"(fa[set][a]));
 #pragma unroll
       for (int b = 0; b < TN; ++b) asm volatile("" : "+v"(fb[set][b]));
 #pragma unroll
-      for (int a = 0; a < TM; ++a)
+      for (int g = 0; g < NM; ++g) {
+        const int a = g / TN, b = g % TN;
+        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[set][a]),
+                                                            __builtin_bit_cast(bf16x8, fb[set][b]), acc[a][b], 0, 0, 0);
+        if (MORE) {
 #pragma unroll
-        for (int b = 0; b < TN; ++b) {
-          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[set][a]),
-                                                              __builtin_bit_cast(bf16x8, fb[set][b]), acc[a][b],
-                                                              0, 0, 0);
-          // load i goes out behind matrix instruction (2 i + 1) NM / (2 LOADS) of the k-tile's NM: spread evenly,
-          // no two wavefronts' loads queue at the unit that takes the addresses (a prompt of 2,048 tokens at
-          // Qwen3-8B's sizes 2.2 % faster, at Qwen3-32B's 3.1 %; at Qwen3-0.6B's, K = 1,024 to 3,072, 0.6 % slower
-          // than with the loads behind each k-step's matrix instructions, which stays for K below 4,096)
-          constexpr int NM = KSTEPS * TM * TN;
-          const int g = (ks * TM + a) * TN + b;
-          if (more_spread) {
+          for (int i = 0; i < LOADS; ++i)
+            if ((2 * i + 1) * SPAN / (2 * LOADS) == ks * NM + g) issue_one(kt + STAGES - 1, st_new, i);
+        }
+        if (ks < LAST) {
 #pragma unroll
-            for (int i = 0; i < LOADS; ++i)
-              if ((2 * i + 1) * NM / (2 * LOADS) == g) issue_one(kt + STAGES - 1, i);
+          for (int j = 0; j < NR; ++j)
+            if (j * (NM - 1) / NR == g) read_one(st, ks + 1, set ^ 1, j);
+        } else if (NEXT) {
+          if (g == GB) {
+            // the loads of the tiles behind kt + 1 may still be out
+            __builtin_amdgcn_sched_barrier(0);
+            wait_vmcnt<(MORE ? STAGES - 2 : LEFT >= 1 ? LEFT - 1 : 0) * LOADS>();
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (g >= GB) {
+#pragma unroll
+            for (int j = 0; j < NR; ++j)
+              if (GB + j * (NM - 1 - GB) / NR == g) read_one(st_next, 0, set ^ 1, j);
           }
         }
-      if (more_steps) {
-#pragma unroll
-        for (int i = ks; i < LOADS; i += KT / 16) issue_one(kt + STAGES - 1, i);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-  }
+    st_new = st;
+    st = st_next;
+  };
+  for (int kt = 0; kt + STAGES - 1 < n_k; ++kt) tile(kt, std::integral_constant<int, STAGES>{});
+  last_tiles(n_k, tile, std::make_integer_sequence<int, STAGES - 1>{});
 
   // acc[a][b][i]: row wm*(BM/WAVES_M) + a*32 + 8*(i/4) + 4*(lane/32) + i%4, column wn*(BN/WAVES_N) + b*32 + lane%32
   const int ccol = lane & 31, crow = (lane >> 5) * 4;
@@ -1249,6 +1249,7 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
       }
     }
   }
+#endif
 }
 
 // Row tiles per block of the order in which a die takes its tiles (see the kernel), 0: tiles in the grid's
@@ -1263,11 +1264,11 @@ static int xcd_rows_for(const dim3& grid, int N, int K) {
   return (long)N * K * 2 >= (192L << 20) ? 8 : 0;
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int STAGES = PSTAGES, int KT = PBK>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int STAGES = PSTAGES>
 static int launch_pipelined(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda,
                             hipStream_t s, int ksplit = 1, int n_first = 0, int n_end = -1) {
-  constexpr int bytes = STAGES * (BM + BN) * KT * 2;
-  auto kernel = gemm_pipelined_kernel<BM, BN, WAVES_M, WAVES_N, EPI, STAGES, KT>;
+  constexpr int bytes = STAGES * (BM + BN) * PBK * 2;
+  auto kernel = gemm_pipelined_kernel<BM, BN, WAVES_M, WAVES_N, EPI, STAGES>;
   static bool ready = false;          // per instantiation: allow more than 64 KiB of dynamic LDS
   if (!ready) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
@@ -1435,11 +1436,11 @@ static int launch_tiled_best(const bf16_t* A, const bf16_t* W, void* out, int M,
     const long huge = (long)((M + 255) / 256) * ((N * cols + 255) / 256);
     if (!g_force_tile && g_tiles_256 && M > 256 && K >= 4096 && huge >= units) {
       const int row_tiles = (M + 255) / 256;
-      if (huge % units == 0 || huge % units >= units * 7 / 8) return launch_pipelined<256, 256, 4, 2, EPI, 4, 32>(A, W, out, M, N, K, lda, s);
+      if (huge % units == 0 || huge % units >= units * 7 / 8) return launch_pipelined<256, 256, 4, 2, EPI, 2>(A, W, out, M, N, K, lda, s);
       const int col_tiles = (int)(huge / units * units / row_tiles);
       const int n_big = col_tiles * 128;                // output columns of the first range
       if (huge >= 2L * units && col_tiles >= 1 && n_big < N) {
-        if (int rc = launch_pipelined<256, 256, 4, 2, EPI, 4, 32>(A, W, out, M, N, K, lda, s, 1, 0, n_big)) return rc;
+        if (int rc = launch_pipelined<256, 256, 4, 2, EPI, 2>(A, W, out, M, N, K, lda, s, 1, 0, n_big)) return rc;
         return launch_pipelined<256, 128, 4, 2, EPI>(A, W, out, M, N, K, lda, s, 1, n_big, N);
       }
     }
@@ -1464,7 +1465,7 @@ static int launch_tiled_best(const bf16_t* A, const bf16_t* W, void* out, int M,
     if (tile == 9) return launch_pipelined<256, 160, 4, 1, EPI>(A, W, out, M, N, K, lda, s);
   }
   if (tile == 1) return launch_pipelined<256, 128, 4, 2, EPI>(A, W, out, M, N, K, lda, s);
-  if (tile == 10) return launch_pipelined<256, 256, 4, 2, EPI, 4, 32>(A, W, out, M, N, K, lda, s);
+  if (tile == 10) return launch_pipelined<256, 256, 4, 2, EPI, 2>(A, W, out, M, N, K, lda, s);
   if constexpr (EPI == TI_EPI_SWIGLU)
     if (tile == 5) return launch_pipelined<64, 128, 2, 2, EPI>(A, W, out, M, N, K, lda, s);
   if constexpr (EPI != TI_EPI_SWIGLU)                // a SwiGLU wavefront needs two column tiles
