@@ -1,0 +1,82 @@
+"""The pipelined product's tiles beyond the ones tests of the whole dispatch name, loops shorter than the ring of stages,
+the dies' blocks of tiles, and the q/k/v product in tiles of 64 rows."""
+import pytest
+import torch
+
+from test_kernels_gpu import dev, f64, ops, qkv_prepared_case, ref_linear  # noqa: F401  (the fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 320, 448])
+@pytest.mark.parametrize("M,N", [(65, 160), (129, 256), (300, 136)])
+def test_every_tile_over_few_k_tiles(ops, M, N, K):  # noqa: F811
+    """One to seven k-tiles (the rings hold two to five) under every tile: the bits of the 128 x 64 tile, which are the sums in
+    ascending steps of 16, within K 2^-24 of float64 for each of the K sums' terms; the row behind the last is left alone."""
+    lib = ops.lib("gemm_bf16")
+    g = torch.Generator().manual_seed(M + K)
+    a = dev((torch.rand(M, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    w = dev((torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    ref, size = ref_linear(a.cpu(), w.cpu()), f64(a).abs() @ f64(w).abs().T
+    want = {}
+    try:
+        for tile in (3, 1, 2, 4, 5, 6, 7, 8, 9, 10, 11):
+            lib.ti_tuning_set(b"force_tile", tile)
+            out = torch.full((M + 1, N), 7.0, device="cuda")
+            ops.linear(a, w, out[:M], "store")
+            act = torch.full((M + 1, N // 2), 7.0, device="cuda", dtype=torch.bfloat16)
+            ops.linear(a, w, act[:M], "swiglu")
+            assert bool((out[M] == 7.0).all()) and bool((act[M] == 7.0).all())
+            added = torch.ones(M, N, device="cuda")
+            ops.linear(a, w, added, "add")
+            got = (out[:M], act[:M], added)
+            want = want or got
+            for x, y in zip(got, want):
+                assert torch.equal(x, y), tile
+    finally:
+        lib.ti_tuning_set(b"force_tile", 0)
+    assert ((f64(want[0]) - ref).abs() <= (K + 1) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1024, 1024, 128), (2048, 512, 128), (512, 2048, 64), (384, 1152, 64)])
+def test_dies_blocks_cover_every_tile_once(ops, M, N, K):  # noqa: F811
+    """Grids that the eight dies cut by rows, by columns and by both, and one that none of the cuts divides."""
+    lib = ops.lib("gemm_bf16")
+    g = torch.Generator().manual_seed(M + N)
+    a = dev((torch.rand(M, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    w = dev((torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    outs = []
+    try:
+        for tile in (2, 4, 6):
+            lib.ti_tuning_set(b"force_tile", tile)
+            for order in (0, 1):
+                lib.ti_tuning_set(b"die_order", order)
+                out = torch.full((M, N), float("nan"), device="cuda")
+                ops.linear(a, w, out, "store")
+                outs.append(out)
+    finally:
+        lib.ti_tuning_set(b"force_tile", 0)
+        lib.ti_tuning_set(b"die_order", 1)
+    for out in outs[1:]:
+        assert torch.equal(out, outs[0])
+    assert (f64(outs[0]) - ref_linear(a.cpu(), w.cpu())).abs().max() < 2e-5 * K
+
+
+@pytest.mark.parametrize("M,N,K", [(77, 1024, 3072), (256, 1024, 2048), (512, 2048, 512), (130, 4096, 4096), (700, 1000, 1024)])
+def test_sums_of_a_split_product(ops, M, N, K):  # noqa: F811
+    """Products into the residual whose launch is cut into two, four or eight runs of K, or left whole, as their cost says."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = dev((torch.rand(M, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    w = dev((torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    base = dev(torch.randn(M, N, generator=g))
+    ref, size = ref_linear(a.cpu(), w.cpu()) + f64(base), f64(a).abs() @ f64(w).abs().T + f64(base).abs()
+    for may_defer in (True, False):
+        x = base.clone()
+        ops.linear(a, w, x, "add", may_defer=may_defer)
+        ops.flush()
+        assert ((f64(x) - ref).abs() <= (K + 9) * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("M,nh,nkv,hd,K", [(65, 16, 8, 128, 64), (129, 6, 2, 64, 128), (200, 4, 1, 128, 320), (512, 16, 8, 128, 192)])
+def test_qkv_product_with_prepared_heads_in_tiles_of_64_rows(ops, M, nh, nkv, hd, K):  # noqa: F811
+    qkv_prepared_case(ops, 64, M, nh, nkv, hd, K, 16, True, "table")

@@ -929,27 +929,26 @@ __device__ __forceinline__ void last_tiles(int n_k, Tile&& tile, std::integer_se
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int STAGES = PSTAGES>
 __global__ void __launch_bounds__(WAVES_M * WAVES_N * 64)
 gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ out_arg,
-                      int M, int N, int K, long lda, int n_first, int xcd_rows, QKVEpilogue ep = QKVEpilogue{}) {
+                      int M, int N, int K, long lda, int n_first, int xcd_rows, int die_rows, QKVEpilogue ep = QKVEpilogue{}) {
 #if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass has no buffer descriptors)
   // n_first: the output column the grid's first workgroup starts at (a launch may cover a range of columns)
-  // xcd_rows > 0 (the grid's width is a multiple of 8 then): which tile a workgroup takes follows the eight
-  // dies.  Workgroups go to the dies in turn, so die c has numbers c, c + 8, ...; it takes an eighth of the
-  // column tiles, in blocks of xcd_rows row tiles, down the rows of a column first: the workgroups of a die
-  // that run at the same time then share a few column tiles of the weight and xcd_rows row tiles of the
-  // tokens in the die's own L2.
+  // xcd_rows > 0: which tile a workgroup takes follows the eight dies.  Workgroups go to the dies in turn, so die c has
+  // numbers c, c + 8, ...; it takes one block of the tiles (the rows cut in die_rows, the columns in 8 / die_rows, both
+  // dividing the grid), in groups of xcd_rows row tiles, down the rows of a column first: the workgroups of a die then read
+  // only the block's rows of A and W into the die's own L2, and those that run together share them.
   int bx = blockIdx.x, by = blockIdx.y;
   if (xcd_rows > 0) {
-    const int nx = gridDim.x, ny = gridDim.y, cx = nx >> 3;
+    const int die_cols = 8 / die_rows, nx = gridDim.x, cx = nx / die_cols, cy = gridDim.y / die_rows;
     const int id = bx + nx * by, die = id & 7, local = id >> 3;
-    const int full = ny / xcd_rows, per = xcd_rows * cx;
+    const int full = cy / xcd_rows, per = xcd_rows * cx;
     int rb = local / per, rem = local - rb * per, rows = xcd_rows;
     if (rb >= full) {
       rb = full;
       rem = local - full * per;
-      rows = ny - full * xcd_rows;
+      rows = cy - full * xcd_rows;
     }
-    by = rb * xcd_rows + rem % rows;
-    bx = die * cx + rem / rows;
+    by = (die / die_cols) * cy + rb * xcd_rows + rem % rows;
+    bx = (die % die_cols) * cx + rem / rows;
   }
   constexpr bool SW = (EPI == TI_EPI_SWIGLU);
   constexpr int TM = BM / WAVES_M / 32, TN = BN / WAVES_N / 32;
@@ -1150,7 +1149,7 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
     // lanes finish a row of a q or k head (the arithmetic of the kernel that prepares whole steps; a
     // row's eight lanes read its angles and write its result as runs of consecutive bytes), and a
     // thread a dim of a v head.
-    static_assert((BM == 256 || BM == 128) && NWV == 8, "the first wavefronts look up a row each; 64 rows per pass of all eight");
+    static_assert(BM % 64 == 0 && BM <= 256 && NWV == 8, "the first wavefronts look up a row each; 64 rows per pass of all eight");
     constexpr int FS = BN + 8;                              // row stride: the eight rows x eight lanes of a wavefront
                                                             // read 64 different banks
     static_assert(BM * FS * 4 + 4 * BM * 4 <= STAGES * STAGE_BYTES, "the 32-bit tile fits into the stages");
@@ -1252,16 +1251,36 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
 #endif
 }
 
-// Row tiles per block of the order in which a die takes its tiles (see the kernel), 0: tiles in the grid's
-// order.  The dies' order pays where the weight is larger than the cache in front of the memory holds (256 MB):
-// in the grid's order every row tile pulls the whole weight from memory again (Qwen3-32B's gate/up and down
-// over 2,048 rows, 524 and 262 MB: a prompt of 2,048 tokens 9.6 % faster); a weight that cache holds is served
-// from it either way (Qwen3-8B's, 201 MB: no change; Qwen3-0.6B's: 0.7 % slower).
-static int g_xcd_rows = 0;       // a hook for measurements: > 0 forces the block's rows, -1 the grid's order
-static int xcd_rows_for(const dim3& grid, int N, int K) {
-  if (grid.x % 8 != 0 || g_xcd_rows < 0) return 0;
-  if (g_xcd_rows > 0) return g_xcd_rows;
-  return (long)N * K * 2 >= (192L << 20) ? 8 : 0;
+// The order in which the dies take a product's tiles (see the kernel): rows = 0 is the grid's own, which deals the columns
+// out to the dies where 8 divides them and mixes everything where not.
+struct DieOrder {
+  int rows = 0, die_rows = 1;
+};
+static int g_xcd_rows = 0;       // a hook for measurements: > 0 forces the group's rows (all rows to a die), -1 the grid's order
+static int g_die_order = 1;      // a hook for measurements: 0: no blocks of rows
+// A: bytes of the token rows, W: of the weight rows.  Large weights: an eighth of the columns to a die, in groups of eight row
+// tiles.  In the grid's order every row tile pulls the whole weight from memory again once it is larger than the cache
+// in front of the memory holds (256 MB; Qwen3-32B's gate/up and down over 2,048 rows, 524 and 262 MB: a prompt of 2,048
+// tokens 9.6 % faster).  Otherwise the cut that brings the fewest bytes into the eight L2s, A / die_rows + W / die_cols each.
+static DieOrder die_order(const dim3& grid, long A, long W) {
+  DieOrder o;
+  if (g_xcd_rows < 0) return o;
+  if (g_xcd_rows > 0 || W >= (192L << 20)) {
+    if (grid.x % 8 == 0) o.rows = g_xcd_rows > 0 ? g_xcd_rows : 8;
+    return o;
+  }
+  if (!g_die_order) return o;
+  long least = grid.x % 8 == 0 ? A + W / 8 : A + W;
+  for (int r = 1; r <= 8; r *= 2) {
+    if (grid.y % r || grid.x % (8 / r)) continue;
+    const long bytes = A / r + W / (8 / r);
+    if (bytes * 10 < least * 9) {
+      least = bytes;
+      o.rows = 8;
+      o.die_rows = r;
+    }
+  }
+  return o;
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int STAGES = PSTAGES>
@@ -1281,8 +1300,8 @@ static int launch_pipelined(const bf16_t* A, const bf16_t* W, void* out, int M, 
   // columns [n_first, n_end) of the output (all of them by default); n_end short of N is a multiple of the tile
   if (n_end < 0) n_end = N;
   dim3 grid((n_end - n_first + bn - 1) / bn, (M + BM - 1) / BM, (EPI == TI_EPI_STORE_F32) ? ksplit : 1);
-  kernel<<<grid, WAVES_M * WAVES_N * 64, bytes, s>>>(A, W, out, M, N, K, lda, n_first,
-                                                     xcd_rows_for(grid, (EPI == TI_EPI_SWIGLU ? 2 : 1) * N, K), QKVEpilogue{});
+  const DieOrder o = die_order(grid, (long)M * K * 2, (EPI == TI_EPI_SWIGLU ? 2L : 1L) * N * K * 2);
+  kernel<<<grid, WAVES_M * WAVES_N * 64, bytes, s>>>(A, W, out, M, N, K, lda, n_first, o.rows, o.die_rows, QKVEpilogue{});
   return 0;
 }
 
@@ -1291,6 +1310,9 @@ static int g_tiles_256 = 1;      // a hook for measurements: 0 = no tiles of 256
 static int g_two_ranges = 1;     // a hook for measurements: 0 = never split the columns between two tile shapes
 static int g_qkv_rows = 0;       // hooks for measurements: 128 or 256 forces the tile's rows;
 static int g_qkv_min_rows = 17;  // the fewest rows served (fewer take the kernels with the norm in front)
+
+// What the pipelined kernel takes: k-tiles of 64, and rows whose offsets inside a tile fit its 32-bit load offsets.
+static bool pipelined_serves(int M, int K, long lda) { return K % PBK == 0 && K < (1 << 21) && lda < (1 << 21); }
 
 static int compute_units() {
   static int n = 0;
@@ -1303,12 +1325,12 @@ static int compute_units() {
   return n;
 }
 
-template <int BM, int WAVES_M, int WAVES_N>
+template <int BM, int WAVES_M, int WAVES_N, int STAGES>
 static int launch_qkv_prep(const void* A, const void* W, int M, int N, int K, long lda, const QKVEpilogue& ep,
                            hipStream_t stream, int n_first = 0, int n_end = -1) {
   constexpr int BN = 128;
-  constexpr int bytes = PSTAGES * (BM + BN) * PBK * 2;
-  auto kernel = gemm_pipelined_kernel<BM, BN, WAVES_M, WAVES_N, TI_EPI_QKV_PREP>;
+  constexpr int bytes = STAGES * (BM + BN) * PBK * 2;
+  auto kernel = gemm_pipelined_kernel<BM, BN, WAVES_M, WAVES_N, TI_EPI_QKV_PREP, STAGES>;
   static bool ready = false;
   if (!ready) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
@@ -1319,9 +1341,82 @@ static int launch_qkv_prep(const void* A, const void* W, int M, int N, int K, lo
   }
   if (n_end < 0) n_end = N;               // columns [n_first, n_end): whole heads
   dim3 grid((n_end - n_first + BN - 1) / BN, (M + BM - 1) / BM);
-  kernel<<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, nullptr, M, N, K, lda, n_first,
-                                       xcd_rows_for(grid, N, K), ep);
+  const DieOrder o = die_order(grid, (long)M * K * 2, (long)N * K * 2);
+  kernel<<<grid, 512, bytes, stream>>>((const bf16_t*)A, (const bf16_t*)W, nullptr, M, N, K, lda, n_first, o.rows, o.die_rows, ep);
   return 0;
+}
+
+// for measurements: 0 = choose the tile by the shape, else a tile's id below
+static int g_force_tile = 0;
+
+// The tiles, and what one costs.  A launch is rounds of workgroups; a round lasts start + k-tiles x (each + fill x the share
+// of the compute units that is busy), for workgroups alone on a unit and, where two fit in its LDS, for two.  The numbers
+// (us, k-tiles of 64) are fitted to 300 products: 65 to 6,000 rows times the four weights of a layer of Qwen3-0.6B's, 1.7B's,
+// 4B's and 8B's sizes, weights not in the caches, K also cut in two, four and eight.  The median error is 3 to 9 %, and the
+// tile that is the cheapest by them is on average 0.8 % slower than the fastest (with K split 1.8 %, SwiGLU 0.9 %).
+// Fewer rows of A than a tile has cost what the whole tile costs.
+struct TileRate {
+  int id, bm, bn, stages;
+  float start1, each1, fill1;        // one workgroup to a unit
+  float start2, each2, fill2;        // two (0: they do not fit)
+};
+static const TileRate TILES_PLAIN[] = {
+    {1, 256, 128, 3, 4.96f, 0.54f, 0.35f, 0.f, 0.f, 0.f},     {11, 256, 128, 3, 6.58f, 0.55f, 0.30f, 0.f, 0.f, 0.f},
+    {2, 128, 128, 4, 3.25f, 0.39f, 0.16f, 0.f, 0.f, 0.f},     {4, 128, 64, 4, 2.46f, 0.28f, 0.05f, 0.f, 0.f, 0.f},
+    {3, 128, 64, 3, 2.17f, 0.38f, 0.06f, 3.48f, 0.26f, 0.39f}, {6, 64, 64, 5, 1.27f, 0.20f, 0.05f, 1.96f, 0.19f, 0.22f},
+    {8, 128, 160, 3, 4.98f, 0.51f, 0.13f, 0.f, 0.f, 0.f},     {9, 256, 160, 3, 8.03f, 0.63f, 0.35f, 0.f, 0.f, 0.f}};
+static const TileRate TILES_SWIGLU[] = {
+    {10, 256, 256, 2, 5.46f, 1.39f, 0.20f, 0.f, 0.f, 0.f},    {1, 256, 128, 3, 3.08f, 0.56f, 0.28f, 0.f, 0.f, 0.f},
+    {2, 128, 128, 4, 0.f, 0.54f, 0.05f, 0.f, 0.f, 0.f},       {7, 64, 128, 4, 0.f, 0.40f, 0.03f, 0.f, 0.f, 0.f},
+    {5, 64, 128, 3, 0.f, 0.45f, 0.09f, 0.f, 0.55f, 0.20f}};
+static const double LAUNCH_US = 2.0;
+
+static double tile_us(const TileRate& t, long workgroups, int k_tiles) {
+  const long units = compute_units();
+  const long round = t.each2 > 0.f ? 2 * units : units;
+  const long full = workgroups / round, rest = workgroups % round;
+  auto one = [&](double share) { return t.start1 + k_tiles * (t.each1 + t.fill1 * share); };
+  auto two = [&](double share) { return t.start2 + k_tiles * (t.each2 + t.fill2 * share); };
+  double us = full * (t.each2 > 0.f ? two(1.0) : one(1.0));
+  if (rest) us += rest <= units ? one((double)rest / units) : two((double)rest / round);
+  return us;
+}
+
+struct TileChoice {
+  int id = 0;
+  double us = 0.0;
+  int n_big = 0;            // > 0: only that many rows of W, the others by tile `rest`
+  int rest = 0;
+};
+// The cheapest tile for M rows times `rows` rows of W (for SwiGLU both halves), k_tiles deep, the launch `copies` times as
+// large (K split).  two_ranges: also two launches, whole rounds of one tile and the columns left over in another.
+static TileChoice choose_tile(bool swiglu, int M, int rows, int k_tiles, int copies, bool two_ranges) {
+  const TileRate* tiles = swiglu ? TILES_SWIGLU : TILES_PLAIN;
+  const int n = swiglu ? (int)(sizeof(TILES_SWIGLU) / sizeof(TileRate)) : (int)(sizeof(TILES_PLAIN) / sizeof(TileRate));
+  auto allowed = [&](const TileRate& t) { return !((t.id == 10 && !g_tiles_256) || (t.bn == 160 && !g_tiles_160)); };
+  auto row_tiles = [&](const TileRate& t) { return (long)((M + t.bm - 1) / t.bm); };
+  auto us = [&](const TileRate& t, int r) { return LAUNCH_US + tile_us(t, row_tiles(t) * ((r + t.bn - 1) / t.bn) * copies, k_tiles); };
+  TileChoice best;
+  for (int i = 0; i < n; ++i) {
+    if (!allowed(tiles[i])) continue;
+    const double c = us(tiles[i], rows);
+    if (!best.id || c < best.us) best = {tiles[i].id, c, 0, 0};
+  }
+  if (!two_ranges || !g_two_ranges || copies != 1) return best;
+  for (int i = 0; i < n; ++i) {
+    const TileRate& t = tiles[i];
+    const long units = compute_units(), rt = row_tiles(t), all = rt * ((rows + t.bn - 1) / t.bn);
+    if (!allowed(t) || t.each2 > 0.f || all < units || all % units == 0) continue;
+    const int n_big = (int)(all / units * units / rt) * t.bn;
+    if (n_big <= 0 || n_big >= rows) continue;
+    const double first = us(t, n_big);
+    for (int j = 0; j < n; ++j) {
+      if (!allowed(tiles[j])) continue;
+      const double c = first + us(tiles[j], rows - n_big);
+      if (c < best.us) best = {t.id, c, n_big, tiles[j].id};
+    }
+  }
+  return best;
 }
 
 // The fused q/k/v projection of a step's rows with the per-head work in its epilogue (see
@@ -1335,7 +1430,7 @@ extern "C" int ti_gemm_bf16_qkv_prep(const void* A, const void* W, int M, int K,
                                      int page_size, hipStream_t stream) {
   TI_REQUIRE(M >= 0 && K > 0 && lda >= K && n_head > 0 && n_kv >= 0 && hd > 0 && page_size > 0 && table_stride > 0,
              "gemm_bf16_qkv_prep: bad sizes");
-  if (M < g_qkv_min_rows || K % 64 != 0 || lda % 8 != 0 || !(hd == 64 || hd == 128) || ((uintptr_t)A & 15) ||
+  if (M < g_qkv_min_rows || !pipelined_serves(M, K, lda) || lda % 8 != 0 || !(hd == 64 || hd == 128) || ((uintptr_t)A & 15) ||
       ((uintptr_t)W & 15) || ((uintptr_t)q_out & 15) || ((uintptr_t)pool & 15) || ((uintptr_t)rope_table & 15)) {
     ti_set_error("gemm_bf16_qkv_prep: M=%d K=%d head_dim=%d is not served (M > 16, K %% 64 == 0, head_dim 64 or 128)",
                  M, K, hd);
@@ -1346,131 +1441,100 @@ extern "C" int ti_gemm_bf16_qkv_prep(const void* A, const void* W, int M, int K,
   QKVEpilogue ep{q_w, k_w, eps, inv_freq, (const float2*)rope_table, table_len, pos, slot, table, table_stride,
                  (bf16_t*)pool, (bf16_t*)q_out, n_head, n_kv, hd, page_size};
   const int N = (n_head + 2 * n_kv) * hd;
-  // 128-row tiles while they make no more workgroups than there are compute units (1,024 rows of
-  // the 32 column tiles of Qwen3-0.6B), else 256-row tiles, which load less per flop
-  const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-  // Few tiles (a short portion beside decoded tokens): a launch of tiles whose columns are whole heads
-  // leaves most compute units idle, and each workgroup that does run finishes 128 rows of heads by
-  // itself; the product in 64 x 64 tiles followed by the kernel that prepares whole steps is faster
-  // then (8 decoded tokens beside 128 of a prompt, Qwen3-0.6B's sizes: 2.47 -> 2.29 ms a step; from
-  // 512 rows on this kernel wins).  Not when a test asks for a tile.
-  if (!g_qkv_rows && tiles128 * 2 < compute_units()) {
-    ti_set_error("gemm_bf16_qkv_prep: %ld tiles of 128 x 128 are left to the product and the preparation kernel", tiles128);
-    return 3;
+  // The tile of 64, 128 or 256 rows whose launch costs the least, 256-row tiles also as whole rounds of the units with the
+  // heads left over in 128-row tiles behind them (Qwen3-8B's 48 heads over 2,048 rows), beside the plain product in its own best
+  // tile followed by the kernel that prepares whole steps, which reads the product's 32-bit sums again.  Finishing the heads
+  // costs a tile about 3 us (tiles of 128 x 128 for 512 rows of Qwen3-0.6B's sizes, the only ones below 1,024 rows before:
+  // 18.9 us; of 64 x 128, on all units: 12).  Not when a test asks for a tile; steps of up to 64 rows whose tiles
+  // leave most units idle always go to the product.
+  const long units = compute_units();
+  const int k_tiles = K / PBK, col_tiles = (N + 127) / 128;
+  auto tile_of = [&](int id) -> const TileRate& {
+    for (const auto& t : TILES_PLAIN)
+      if (t.id == id) return t;
+    return TILES_PLAIN[0];
+  };
+  auto us = [&](int rows, int cols) {               // (a tile of 64 x 128 does what one of 128 x 64 does)
+    const TileRate& t = tile_of(rows == 256 ? 1 : rows == 128 ? 2 : 4);
+    return LAUNCH_US + 3.0 + tile_us(t, (long)((M + rows - 1) / rows) * cols, k_tiles);
+  };
+  int rows = g_qkv_rows, n_big = 0;                 // n_big > 0: that many columns in 256-row tiles, the others in 128-row tiles
+  if (!rows) {
+    double least = us(64, col_tiles);
+    rows = 64;
+    for (int r = 128; r <= 256; r *= 2)
+      if (us(r, col_tiles) < least) {
+        least = us(r, col_tiles);
+        rows = r;
+      }
+    const long row_tiles = (M + 255) / 256, big = row_tiles * col_tiles;
+    if (g_two_ranges && big > units && big % units != 0) {
+      const int cols = (int)(big / units * units / row_tiles);
+      if (cols >= 1 && us(256, cols) + us(128, col_tiles - cols) < least) {
+        least = us(256, cols) + us(128, col_tiles - cols);
+        rows = 256;
+        n_big = cols * 128;
+      }
+    }
+    const double apart = choose_tile(false, M, N, k_tiles, 1, true).us + LAUNCH_US + 2.0 + 2.0 * M * N * 4 / 4.0e6;
+    if (M <= 64 ? (long)((M + 127) / 128) * col_tiles * 2 < units : apart < least) {
+      ti_set_error("gemm_bf16_qkv_prep: %d rows are left to the product and the preparation kernel", M);
+      return 3;
+    }
   }
-  const bool rows128 = g_qkv_rows ? g_qkv_rows == 128 : tiles128 <= compute_units();
-  // 256-row tiles that leave a round short of three quarters (Qwen3-8B's 48 heads over 2,048 rows: 8 x 48
-  // tiles on 256 units): the heads that make whole rounds take them, the other heads 128-row tiles in a
-  // launch of their own, as in the plain product
-  const int units = compute_units(), row_tiles = (M + 255) / 256;
-  const long big = (long)row_tiles * ((N + 127) / 128);
   int rc_;
-  if (!rows128 && !g_qkv_rows && g_two_ranges && big >= units && big < 4L * units && big % units != 0 &&
-      big % units < units * 3 / 4 && (int)(big / units * units / row_tiles) >= 1) {
-    const int n_big = (int)(big / units * units / row_tiles) * 128;
-    rc_ = launch_qkv_prep<256, 4, 2>(A, W, M, N, K, lda, ep, stream, 0, n_big);
-    if (!rc_) rc_ = launch_qkv_prep<128, 2, 4>(A, W, M, N, K, lda, ep, stream, n_big, N);
+  if (n_big) {
+    rc_ = launch_qkv_prep<256, 4, 2, 3>(A, W, M, N, K, lda, ep, stream, 0, n_big);
+    if (!rc_) rc_ = launch_qkv_prep<128, 4, 2, 4>(A, W, M, N, K, lda, ep, stream, n_big, N);
+  } else if (rows == 64) {
+    rc_ = launch_qkv_prep<64, 2, 4, 4>(A, W, M, N, K, lda, ep, stream);
+  } else if (rows == 128) {
+    rc_ = launch_qkv_prep<128, 4, 2, 4>(A, W, M, N, K, lda, ep, stream);
   } else {
-    rc_ = rows128 ? launch_qkv_prep<128, 2, 4>(A, W, M, N, K, lda, ep, stream)
-                  : launch_qkv_prep<256, 4, 2>(A, W, M, N, K, lda, ep, stream);
+    rc_ = launch_qkv_prep<256, 4, 2, 3>(A, W, M, N, K, lda, ep, stream);
   }
   if (rc_) return rc_;
   TI_LAUNCH_CHECK();
   return 0;
 }
 
-// for measurements: 0 = choose the tile by the shape, 1 = 256 x 128, 3 = 128 x 64, 5 = 64 x 128 (SwiGLU only), 6 = 64 x 64,
-// 8 = 128 x 160, 9 = 256 x 160 (neither for SwiGLU), 10 = 256 x 256
-static int g_force_tile = 0;
+template <int EPI>
+static int launch_tile(int id, const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda, hipStream_t s,
+                       int ksplit = 1, int n_first = 0, int n_end = -1) {
+  constexpr bool SW = EPI == TI_EPI_SWIGLU;          // a SwiGLU wavefront needs two column tiles
+  switch (id) {
+    case 1: return launch_pipelined<256, 128, 4, 2, EPI>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+    case 2: return launch_pipelined<128, 128, 4, 2, EPI, 4>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+  }
+  if constexpr (SW) {
+    switch (id) {
+      case 5: return launch_pipelined<64, 128, 2, 2, EPI>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+      case 7: return launch_pipelined<64, 128, 2, 2, EPI, 4>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+      case 10: return launch_pipelined<256, 256, 4, 2, EPI, 2>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+    }
+    return launch_pipelined<128, 64, 4, 1, EPI>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);      // 3, and a forced tile
+  } else {                                                                                                // that it does not have
+    switch (id) {
+      case 4: return launch_pipelined<128, 64, 2, 2, EPI, 4>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+      case 6: return launch_pipelined<64, 64, 2, 2, EPI, 5>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+      case 8: return launch_pipelined<128, 160, 4, 1, EPI>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+      case 9: return launch_pipelined<256, 160, 4, 1, EPI>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+      case 11: return launch_pipelined<256, 128, 4, 1, EPI>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);      // for a long K
+    }
+    return launch_pipelined<128, 64, 2, 2, EPI>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+  }
+}
 
-// Three tiles.  256 x 128 with eight wavefronts does the most per byte it loads, one workgroup
-// to a compute unit: it is taken when its workgroups come in (nearly) whole rounds of the 256
-// units or in many rounds.  Otherwise 128 x 64 with four wavefronts, two workgroups to a unit;
-// and where even those are fewer than two to a unit, 64 x 64 (three to a unit).
 template <int EPI>
 static int launch_tiled_best(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda,
                              hipStream_t s) {
-  const int cols = (EPI == TI_EPI_SWIGLU) ? 2 : 1;   // a SwiGLU workgroup covers BN / 2 output columns
   constexpr bool SW = EPI == TI_EPI_SWIGLU;
-  const long big = (long)((M + 255) / 256) * ((N * cols + 127) / 128);
-  const long mid = (long)((M + 127) / 128) * ((N * cols + 63) / 64);
-  const int units = compute_units();
-  const bool whole_rounds = big >= units && (big % units == 0 || big % units >= units * 3 / 4);
-  int tile = (big >= 4 * units || whole_rounds) ? 1 : (mid >= 2 * units ? 3 : 6);
-  if (M <= 64 && tile == 1) tile = 6;                // few rows times a wide weight: no 256-row tile
-  // Up to 64 rows times a stacked [gate; up] weight: such a product waits for the weight from memory, and
-  // a 128 x 64 tile, half of whose rows are empty then, has 8 of its 24 KB a stage in weights.  A 64 x 128
-  // tile has 16 of 24, two workgroups to a unit as well: twice the weight under way (Qwen3-32B's gate/up
-  // at 64 rows 141 -> 115 us, 8B's 52 -> 45); a weight that gives it fewer workgroups than half the
-  // units stays with the narrower tile (0.6B's: 10.0 against 10.6 us).
-  if (SW && M <= 64 && (long)(N * cols + 127) / 128 * 2 >= compute_units()) tile = 5;
-  // 65 to 520 rows (a portion of a prompt beside decoded tokens) times a large weight wait for the weight,
-  // and every tile of rows pulls all of it in again.  129 to 256 rows under a stacked [gate; up] weight take
-  // one 256-row tile, not two of 128 (Qwen3-8B's at 136 rows 89 -> 65 us, 32B's 185 -> 163, 4B's 48 -> 40);
-  // from 385 rows on 128 x 64 tiles, not 64 x 64 (8B's q/k/v, o and down at 520 rows 63, 42 and 132 ->
-  // 47, 39 and 104 us).  Small weights are not what such a step waits for: they stay as they were.
-  const bool large = (long)N * cols * K >= (8L << 20);
-  if (SW && large && M > 128 && M <= 256 && tile == 3) tile = 1;
-  if (!SW && large && M > 384 && tile == 6) tile = 3;
-  // Widths that 160 columns divide (2,560 and 5,120 among Qwen3's): where tiles of 256 x 160 or 128 x 160,
-  // four wavefronts of 64 x 160 or 32 x 160, make whole rounds of the units, they are taken: a workgroup
-  // to a unit, fewer LDS reads and bytes from memory per matrix instruction than 256 x 128 (Qwen3-32B's o
-  // and down over 2,048 rows, 8 x 32 tiles: 212 and 604 us -> 180 and 554; Qwen3-4B's, 16 x 16 tiles of
-  // 128 x 160: 88 and 170 -> 75 and 141).
-  if constexpr (!SW) {
-    if (!g_force_tile && g_tiles_160 && M > 64 && N % 160 == 0) {
-      const long cols160 = N / 160;
-      const long wg256 = (long)((M + 255) / 256) * cols160, wg128 = (long)((M + 127) / 128) * cols160;
-      auto whole = [&](long wg) { return wg >= units && (wg % units == 0 || wg % units >= units * 7 / 8); };
-      if (whole(wg256)) tile = 9;
-      else if (whole(wg128) && wg128 <= 2L * units) tile = 8;
-    }
-  }
-  // A stacked [gate; up] weight over many rows, K long: 256 x 256 tiles (eight wavefronts of 64 x 128, two
-  // stages of 64 KB) load two thirds of what 256 x 128 tiles load per flop.  Taken where they come in whole
-  // rounds of the units (Qwen3-8B's gate/up over 2,048 rows, 8 x 96 tiles: 382 -> 343 us); where rounds are
-  // left over, the columns of the whole rounds take them and the rest 256 x 128 tiles in a launch of its own
-  // (Qwen3-32B's, 8 x 200 tiles).  With the other epilogues they gain nothing or lose (o over 8,192 rows: 285 ->
-  // 314 us).
-  if constexpr (SW) {
-    const long huge = (long)((M + 255) / 256) * ((N * cols + 255) / 256);
-    if (!g_force_tile && g_tiles_256 && M > 256 && K >= 4096 && huge >= units) {
-      const int row_tiles = (M + 255) / 256;
-      if (huge % units == 0 || huge % units >= units * 7 / 8) return launch_pipelined<256, 256, 4, 2, EPI, 2>(A, W, out, M, N, K, lda, s);
-      const int col_tiles = (int)(huge / units * units / row_tiles);
-      const int n_big = col_tiles * 128;                // output columns of the first range
-      if (huge >= 2L * units && col_tiles >= 1 && n_big < N) {
-        if (int rc = launch_pipelined<256, 256, 4, 2, EPI, 2>(A, W, out, M, N, K, lda, s, 1, 0, n_big)) return rc;
-        return launch_pipelined<256, 128, 4, 2, EPI>(A, W, out, M, N, K, lda, s, 1, n_big, N);
-      }
-    }
-  }
-  // 256 x 128 tiles that fill the units once or more and leave a round short of three quarters (Qwen3-32B's
-  // o and down projections over 2,048 rows: 8 x 40 tiles on 256 units): the columns that make whole rounds
-  // take those tiles, the rest 128 x 64 tiles in a launch of their own behind them, rather than everything
-  // the smaller tile, which needs a third more time per flop (those projections 548 -> 420 us on average;
-  // Qwen3-0.6B's gate/up, 8 x 48 tiles, likewise).
-  if (tile == 3 && big >= units && !g_force_tile && g_two_ranges) {   // (not where a 160-column tile was chosen)
-    const int row_tiles = (M + 255) / 256;
-    const int col_tiles = (int)(big / units * units / row_tiles);
-    const int n_big = col_tiles * (128 / cols);         // output columns of the first range
-    if (col_tiles >= 1 && n_big < N) {
-      if (int rc = launch_pipelined<256, 128, 4, 2, EPI>(A, W, out, M, N, K, lda, s, 1, 0, n_big)) return rc;
-      return launch_pipelined<128, 64, 4, 1, EPI>(A, W, out, M, N, K, lda, s, 1, n_big, N);
-    }
-  }
-  if (g_force_tile) tile = g_force_tile;
-  if constexpr (!SW) {
-    if (tile == 8) return launch_pipelined<128, 160, 4, 1, EPI>(A, W, out, M, N, K, lda, s);
-    if (tile == 9) return launch_pipelined<256, 160, 4, 1, EPI>(A, W, out, M, N, K, lda, s);
-  }
-  if (tile == 1) return launch_pipelined<256, 128, 4, 2, EPI>(A, W, out, M, N, K, lda, s);
-  if (tile == 10) return launch_pipelined<256, 256, 4, 2, EPI, 2>(A, W, out, M, N, K, lda, s);
-  if constexpr (EPI == TI_EPI_SWIGLU)
-    if (tile == 5) return launch_pipelined<64, 128, 2, 2, EPI>(A, W, out, M, N, K, lda, s);
-  if constexpr (EPI != TI_EPI_SWIGLU)                // a SwiGLU wavefront needs two column tiles
-    if (tile == 6) return launch_pipelined<64, 64, 2, 2, EPI>(A, W, out, M, N, K, lda, s);
-  return launch_pipelined<128, 64, 4, 1, EPI>(A, W, out, M, N, K, lda, s);
+  if (g_force_tile) return launch_tile<EPI>(g_force_tile, A, W, out, M, N, K, lda, s);
+  const TileChoice c = choose_tile(SW, M, SW ? 2 * N : N, K / PBK, 1, true);
+  if (!c.n_big) return launch_tile<EPI>(c.id, A, W, out, M, N, K, lda, s);
+  const int n_big = SW ? c.n_big / 2 : c.n_big;
+  if (int rc = launch_tile<EPI>(c.id, A, W, out, M, N, K, lda, s, 1, 0, n_big)) return rc;
+  return launch_tile<EPI>(c.rest, A, W, out, M, N, K, lda, s, 1, n_big, N);
 }
 
 // ------------------------------------------------------------------- dispatch
@@ -2060,59 +2124,49 @@ extern "C" int ti_gemm_bf16_add_split(const void* A, const void* W, void* out, i
       return 0;
     }
   }
-  int KS = 1;
+  int KS = 1, tile = 0;      // (tile: of the pipelined kernel, 0: not taken)
   const bool small = M <= 64 && !(large_weight(M, N, K, epi) && g_use_pipelined);
   if (g_add_split && epi == TI_EPI_ADD_F32 && partial && M > 16 && K % 64 == 0 && lda % 8 == 0 &&
       !((uintptr_t)A & 15) && !((uintptr_t)W & 15) && !((uintptr_t)partial & 15) && (small || g_use_pipelined)) {
-    // split K until the launch has about a workgroup per compute unit
-    const long tiles = small ? (N + 15) / 16 : (long)((M + 63) / 64) * ((N + 63) / 64);
     const int nb = K / 64;
-    // (a large weight is waited for from memory: then about four workgroups per unit, so that enough
-    // of it is on its way at any time)
-    // as long as the partial sums stay a small part of what the weight has in bytes
-    const bool streamed = !small && (long)N * K >= (8L << 20);
-    while (KS < 8 && tiles * KS * 2 <= compute_units() && nb / (KS * 2) >= 4) KS *= 2;
-    if (streamed)
-      while (KS < 8 && tiles * KS * 2 <= 4L * compute_units() && nb / (KS * 2) >= 4 && (long)KS * 2 * M * 16 <= K) KS *= 2;
-    while (KS > 1 && (long)KS * M * N * 4 > partial_bytes) KS /= 2;
-    // with the addition as a kernel of its own, only large products gain
-    if (!defer && small && !((long)M * K >= 128 * 1024 || (K >= 3072 && (long)M * K >= 96 * 1024))) KS = 1;
-    if (!defer && !small && KS < 4) KS = 1;
-  }
-  // Many rows times a weight of few rows (o and down of a whole prompt): 64 x 64 tiles are what fills
-  // the chip, and they pull four bytes into a compute unit where a 128 x 128 tile pulls two.  When the
-  // 128 x 128 tiles are at most half as many as the units, K is split between two to four workgroups
-  // per tile instead: the same bytes as one round of 128 x 128 tiles, on all units.
-  // (not under a weight of 64 Mi elements or more: Qwen3-32B's down projection at 264 rows 164 -> 199 us)
-  if (KS == 1 && !small && g_add_split && g_use_pipelined && defer && epi == TI_EPI_ADD_F32 && partial && M >= 256 &&
-      (long)N * K < (64L << 20) && K % 64 == 0 && lda % 8 == 0 && !((uintptr_t)A & 15) && !((uintptr_t)W & 15) && !((uintptr_t)partial & 15)) {
-    const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-    int ks = (int)std::min<long>(4, compute_units() / std::max<long>(1, tiles128));
-    while (ks > 1 && ((K / 64) / ks < 8 || (long)ks * M * N * 4 > partial_bytes)) --ks;
-    if (ks >= 2) {
-      int rc_ = launch_pipelined<128, 128, 2, 4, TI_EPI_STORE_F32>((const bf16_t*)A, (const bf16_t*)W, partial, M, N, K, lda,
-                                                                   stream, ks);
-      if (rc_) return rc_;
-      if (defer == 1) {
-        *splits = ks;
-      } else {
-        const size_t count = (size_t)M * N;
-        gemm_partials_add_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>((float*)out, (const float*)partial,
-                                                                                    ks, count);
+    if (small) {
+      // split K until the launch has about a workgroup per compute unit
+      const long tiles = (N + 15) / 16;
+      while (KS < 8 && tiles * KS * 2 <= compute_units() && nb / (KS * 2) >= 4) KS *= 2;
+      while (KS > 1 && (long)KS * M * N * 4 > partial_bytes) KS /= 2;
+      // with the addition as a kernel of its own, only large products gain
+      if (!defer && !((long)M * K >= 128 * 1024 || (K >= 3072 && (long)M * K >= 96 * 1024))) KS = 1;
+    } else if (pipelined_serves(M, K, lda)) {
+      // A product of few tiles, a short loop each, leaves units idle: K split between workgroups fills them, and the sums
+      // cost their bytes once more where they are added (by the norm behind, or a kernel of its own).  Split as many
+      // ways as tile and sums together are the cheapest (512 x 1024 x 3072: 13 us whole, 9.5 in two; the norm 0.6 more).
+      // One way means that the sums of whole tiles are left to the norm, which spares the product the wait for the
+      // residual behind its last k-tile; only where few tiles of many rows leave it short of other work (o and down of a
+      // whole prompt at small widths).
+      const double sums = (double)M * N * 4 / 10e6;      // us: the norm reads them at about 10 TB/s, out of the caches
+      const long tiles128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+      const bool few = defer && M >= 256 && tiles128 * 2 <= compute_units();
+      double least = choose_tile(false, M, N, nb, 1, true).us + 1.5;
+      for (int ks = few ? 1 : 2; ks <= 8; ks *= 2) {
+        if (nb / ks < 4 || (long)ks * M * N * 4 > partial_bytes) break;
+        const TileChoice c = choose_tile(false, M, N, nb / ks, ks, false);
+        const double us = c.us + ks * sums + (defer ? 1.0 : 4.0 + 2 * sums);
+        if (us < least || (few && !tile)) {
+          least = us;
+          KS = ks;
+          tile = c.id;
+        }
       }
-      TI_LAUNCH_CHECK();
-      return 0;
     }
   }
-  if (KS == 1) {
+  if (KS == 1 && !tile) {
     ti_set_error("gemm_bf16_add_split: serves more than 16 rows added into a product of few tiles, K a multiple of 64");
     return 3;
   }
   if (small) {
     launch_mblocks<TI_EPI_ADD_F32>((const bf16_t*)A, (const bf16_t*)W, out, (float*)partial, M, N, K, lda, KS, stream);
   } else {
-    int rc_ = launch_pipelined<64, 64, 2, 2, TI_EPI_STORE_F32>((const bf16_t*)A, (const bf16_t*)W, partial, M, N, K, lda,
-                                                               stream, KS);
+    int rc_ = launch_tile<TI_EPI_STORE_F32>(tile, (const bf16_t*)A, (const bf16_t*)W, partial, M, N, K, lda, stream, KS);
     if (rc_) return rc_;
   }
   if (defer == 1) {
@@ -2192,8 +2246,7 @@ extern "C" int ti_gemm_bf16_store_split(const void* A, const void* W, void* out,
     ti_set_error("gemm_bf16_store_split: serves 17 to 64 rows times a large weight of few tiles, K a multiple of 64");
     return 3;
   }
-  int rc_ = launch_pipelined<64, 64, 2, 2, TI_EPI_STORE_F32>((const bf16_t*)A, (const bf16_t*)W, partial, M, N, K, lda, stream,
-                                                             KS);
+  int rc_ = launch_tile<TI_EPI_STORE_F32>(6, (const bf16_t*)A, (const bf16_t*)W, partial, M, N, K, lda, stream, KS);
   if (rc_) return rc_;
   const size_t count = (size_t)M * N;
   gemm_partials_sum_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>((float*)out, (const float*)partial, KS, count);
@@ -2283,7 +2336,7 @@ extern "C" int ti_gemm_bf16(const void* A, const void* W, void* out, int M, int 
       if (rc_) return rc_;                                        \
     } else if (skinny)                                            \
       launch_skinny<E>(a, w, out, M, N, K, lda, stream);          \
-    else if (g_use_pipelined && K % PBK == 0) {                   \
+    else if (g_use_pipelined && pipelined_serves(M, K, lda)) {    \
       int rc_ = launch_tiled_best<E>(a, w, out, M, N, K, lda, stream); \
       if (rc_) return rc_;                                        \
     } else                                                        \
@@ -2309,7 +2362,7 @@ extern "C" int ti_gemm_bf16(const void* A, const void* W, void* out, int M, int 
 // The rules are the library's, process-wide; the host library's Ops applies an object's own
 // overrides around its calls and resets them afterwards.  Returns 0, or 1 for an unknown name.
 extern "C" void ti_tuning_reset() {
-  g_xcd_rows = 0; g_tiles_160 = 1; g_tiles_256 = 1; g_two_ranges = 1; g_qkv_rows = 0; g_qkv_min_rows = 17; g_force_tile = 0; g_skinny_waves = 0;
+  g_xcd_rows = 0; g_die_order = 1; g_tiles_160 = 1; g_tiles_256 = 1; g_two_ranges = 1; g_qkv_rows = 0; g_qkv_min_rows = 17; g_force_tile = 0; g_skinny_waves = 0;
   g_skinny_deep = 1; g_use_pipelined = 1; set_tiled_from(280L << 20); g_row_per_wave = 1;
   g_normed_weight_below = NORMED_WEIGHT_BELOW; g_skinny_copy = 1; g_wide_rows = 1; g_pieces = 1; g_add_split = 1;
   g_rows_direct = 1;
@@ -2324,6 +2377,7 @@ extern "C" int ti_tuning_set(const char* name, long value) {
   else if (n == "tiles_256") g_tiles_256 = (int)value;
   else if (n == "two_ranges") g_two_ranges = (int)value;
   else if (n == "xcd_rows") g_xcd_rows = (int)value;
+  else if (n == "die_order") g_die_order = (int)value;
   else if (n == "skinny_waves") g_skinny_waves = (int)value;
   else if (n == "qkv_prep_min_rows") g_qkv_min_rows = (int)value;
   else if (n == "qkv_prep_rows") g_qkv_rows = (int)value;

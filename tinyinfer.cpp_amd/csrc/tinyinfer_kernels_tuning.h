@@ -5,16 +5,19 @@
 // (Ops::tune) and resets them afterwards.
 //
 // libti_gemm_bf16:
-//   force_tile           1: 256 x 128, 3: 128 x 64, 5: 64 x 128 (SwiGLU only), 6: 64 x 64, 8: 128 x 160, 9: 256 x 160, 10: 256 x 256; 0: by the shape
+//   force_tile           1: 256 x 128, 2: 128 x 128, 3 / 4: 128 x 64 (4: not SwiGLU), 5 / 7: 64 x 128 (SwiGLU only), 6: 64 x 64, 8: 128 x 160,
+//                        9: 256 x 160 (6, 8, 9: not SwiGLU), 10: 256 x 256 (SwiGLU only), 11: 256 x 128 by four wavefronts (not
+//                        SwiGLU); 0: by the shape
 //   normed_weight_below  weights of fewer elements keep the norm inside the product (0: the default)
 //   tiles_160            0: no tiles of 160 columns
 //   tiles_256            0: no tiles of 256 x 256
-//   two_ranges           0: never split a product's columns between 256 x 128 and 128 x 64 tiles
+//   two_ranges           0: never split a product's columns between two tiles
 //   xcd_rows             row tiles per block of the order in which a die takes the tiles of a tiled product (-1: the grid's order,
 //                        0: by the weight's size)
+//   die_order            0: the dies take the tiles of a small weight in the grid's order
 //   skinny_waves         4 or 8 wavefronts in the kernel for M <= 64 (0: by the shape)
 //   qkv_prep_min_rows    the fewest rows ti_gemm_bf16_qkv_prep serves (17)
-//   qkv_prep_rows        128 / 256: the rows of ti_gemm_bf16_qkv_prep's tile; 0: by the shape
+//   qkv_prep_rows        64 / 128 / 256: the rows of ti_gemm_bf16_qkv_prep's tile; 0: by the shape
 //   wide_rows            0: 17..64 rows times a weight of 16,384 rows or more take the other kernels
 //   tiled_from           17..64 rows x weight elements from which they take the tiled kernels (280 Mi)
 //   add_split            0: ti_gemm_bf16_add_split serves nothing
