@@ -71,7 +71,9 @@ __global__ void rmsnorm_kernel(const float* __restrict__ x, const float* __restr
 }
 
 // the same for widths that are multiples of four: a wavefront per row, four rows a workgroup
-template <typename T>
+// PIECES: 16-byte pieces of a row a lane keeps in registers, its weights asked for beside them and not behind the
+// sum (rows up to 256 PIECES floats wide: one round trip to memory and not two); 0: any width
+template <typename T, int PIECES = 0>
 __global__ void __launch_bounds__(256)
 rmsnorm_wave_kernel(const float* __restrict__ x, const float* __restrict__ w, const int* __restrict__ rows,
                     T* __restrict__ out, int n_rows, int H, float eps) {
@@ -79,6 +81,30 @@ rmsnorm_wave_kernel(const float* __restrict__ x, const float* __restrict__ w, co
   if (r >= n_rows) return;
   const float* src = x + (size_t)(rows ? rows[r] : r) * H;
   float ss = 0.f;
+  if constexpr (PIECES > 0) {
+    float4 v[PIECES], g[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int k = lane * 4 + i * 256;
+      v[i] = *reinterpret_cast<const float4*>(src + (k < H ? k : 0));
+      g[i] = *reinterpret_cast<const float4*>(w + (k < H ? k : 0));
+    }
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i)
+      if (lane * 4 + i * 256 < H) ss = rms_accumulate(ss, v[i]);
+    const float scale = rms_scale(ss, H, eps);
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int k = lane * 4 + i * 256;
+      if (k >= H) continue;
+      T* dst = out + (size_t)r * H + k;
+      st<T>(dst, v[i].x * scale * g[i].x);
+      st<T>(dst + 1, v[i].y * scale * g[i].y);
+      st<T>(dst + 2, v[i].z * scale * g[i].z);
+      st<T>(dst + 3, v[i].w * scale * g[i].w);
+    }
+    return;
+  }
 #pragma unroll 8
   for (int k = lane * 4; k < H; k += 256) ss = rms_accumulate(ss, *reinterpret_cast<const float4*>(src + k));
   const float scale = rms_scale(ss, H, eps);
@@ -197,10 +223,15 @@ extern "C" int ti_rmsnorm(int out_dtype, const float* x, const float* w, const i
   }
   if (H % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0) {
     const int grid = (n_rows + 3) / 4;
-    if (out_dtype == TI_F32)
-      rmsnorm_wave_kernel<float><<<grid, 256, 0, stream>>>(x, w, rows, (float*)out, n_rows, H, eps);
-    else
-      rmsnorm_wave_kernel<bf16_t><<<grid, 256, 0, stream>>>(x, w, rows, (bf16_t*)out, n_rows, H, eps);
+#define TI_GO(T, PIECES) rmsnorm_wave_kernel<T, PIECES><<<grid, 256, 0, stream>>>(x, w, rows, (T*)out, n_rows, H, eps)
+    if (out_dtype == TI_F32) {
+      if (H <= 1024) TI_GO(float, 4);
+      else TI_GO(float, 0);
+    } else {
+      if (H <= 1024) TI_GO(bf16_t, 4);
+      else TI_GO(bf16_t, 0);
+    }
+#undef TI_GO
     TI_LAUNCH_CHECK();
     return 0;
   }
@@ -244,8 +275,7 @@ rmsnorm_add_partials_kernel(float* __restrict__ x, const float* __restrict__ par
     }
     return v;
   };
-  auto scaled = [&](int k, float4 v, float scale) {
-    const float4 g = *reinterpret_cast<const float4*>(w + k);
+  auto scaled = [&](int k, float4 v, float4 g, float scale) {
     T* dst = out + (size_t)r * H;
     st<T>(dst + k, v.x * scale * g.x);
     st<T>(dst + k + 1, v.y * scale * g.y);
@@ -254,7 +284,12 @@ rmsnorm_add_partials_kernel(float* __restrict__ x, const float* __restrict__ par
   };
   float ss = 0.f;
   {
-    float4 v[PIECES];
+    float4 v[PIECES], g[PIECES];      // (the weights are asked for beside the row, not behind the sum)
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+      const int k = lane * 4 + i * 256;
+      g[i] = *reinterpret_cast<const float4*>(w + (k < H ? k : 0));
+    }
     if (KS_T) {
 #pragma unroll
       for (int i = 0; i < PIECES; ++i) {
@@ -297,46 +332,47 @@ rmsnorm_add_partials_kernel(float* __restrict__ x, const float* __restrict__ par
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
       const int k = lane * 4 + i * 256;
-      if (k < H) scaled(k, v[i], scale);
+      if (k < H) scaled(k, v[i], g[i], scale);
     }
   }
 }
 
-// The same for rows of 1,025 to 4,096 floats: a workgroup per row, so that four times as many loads
-// are on their way as with a wavefront per row (64 rows of 4,096 with 8 partial sums: 26 -> ~7 us).
-// Thread t adds up the 16-byte pieces t, t + 256, ... (the partial sums four at a time), writes them
-// back and leaves them in LDS; wavefront 0 takes the sum of squares from there in the order of
+// The same with a workgroup per row, so that four times as many loads are on their way as with a
+// wavefront per row (64 rows of 4,096 with 8 partial sums: 26 -> ~7 us; 77 rows of 1,024 with 8: 5.6 -> 3.4).
+// Thread t adds up the 16-byte pieces t, t + 256, ... (VP of them; the partial sums BATCH at a time),
+// writes them back and leaves them in LDS; wavefront 0 takes the sum of squares from there in the order of
 // rmsnorm_wave_kernel (lane l the pieces l, l + 64, ...), so the bits are that kernel's.
-template <typename T>
+template <typename T, int VP, int BATCH>
 __global__ void __launch_bounds__(256)
 rmsnorm_add_partials_row_kernel(float* __restrict__ x, const float* __restrict__ partial, int KS,
                                 const float* __restrict__ w, T* __restrict__ out, int n_rows, int H, float eps) {
-  __shared__ __attribute__((aligned(16))) float row[4096];
+  __shared__ __attribute__((aligned(16))) float row[VP * 1024];
   __shared__ float s_scale;
   const int r = blockIdx.x, lane = threadIdx.x & 63;
   float* src = x + (size_t)r * H;
   const size_t count = (size_t)n_rows * H;
   const float* prow = partial + (size_t)r * H;
-  float4 v[4];
+  float4 v[VP], g[VP];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < VP; ++i) {
     const int k = threadIdx.x * 4 + i * 1024;
     v[i] = *reinterpret_cast<const float4*>(src + (k < H ? k : 0));
+    g[i] = *reinterpret_cast<const float4*>(w + (k < H ? k : 0));
   }
-  for (int s0 = 0; s0 < KS; s0 += 4) {
-    float4 q[4][4];
+  for (int s0 = 0; s0 < KS; s0 += BATCH) {
+    float4 q[BATCH][VP];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < BATCH; ++j)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < VP; ++i) {
         const int k = threadIdx.x * 4 + i * 1024;
         q[j][i] = *reinterpret_cast<const float4*>(prow + (size_t)(s0 + j < KS ? s0 + j : s0) * count + (k < H ? k : 0));
       }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < BATCH; ++j)
       if (s0 + j < KS) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < VP; ++i) {
           v[i].x += q[j][i].x;
           v[i].y += q[j][i].y;
           v[i].z += q[j][i].z;
@@ -345,7 +381,7 @@ rmsnorm_add_partials_row_kernel(float* __restrict__ x, const float* __restrict__
       }
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < VP; ++i) {
     const int k = threadIdx.x * 4 + i * 1024;
     if (k < H) {
       *reinterpret_cast<float4*>(src + k) = v[i];
@@ -363,18 +399,19 @@ rmsnorm_add_partials_row_kernel(float* __restrict__ x, const float* __restrict__
   const float scale = s_scale;
   T* dst = out + (size_t)r * H;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < VP; ++i) {
     const int k = threadIdx.x * 4 + i * 1024;
     if (k < H) {
-      const float4 g = *reinterpret_cast<const float4*>(w + k);
-      st<T>(dst + k, v[i].x * scale * g.x);
-      st<T>(dst + k + 1, v[i].y * scale * g.y);
-      st<T>(dst + k + 2, v[i].z * scale * g.z);
-      st<T>(dst + k + 3, v[i].w * scale * g.w);
+      st<T>(dst + k, v[i].x * scale * g[i].x);
+      st<T>(dst + k + 1, v[i].y * scale * g[i].y);
+      st<T>(dst + k + 2, v[i].z * scale * g[i].z);
+      st<T>(dst + k + 3, v[i].w * scale * g[i].w);
     }
   }
 }
 
+// rows up to this many: a workgroup each (beyond, the units have enough wavefronts with four rows a workgroup, and no barrier)
+#define RMS_ROW_EACH 1024
 template <typename T>
 static void launch_rmsnorm_add_partials(float* x, const float* partial, int KS, const float* w, T* out, int n_rows,
                                         int H, float eps, hipStream_t stream) {
@@ -385,11 +422,12 @@ static void launch_rmsnorm_add_partials(float* x, const float* partial, int KS, 
   const int grid = (n_rows + 3) / 4;
 #define TI_GO(KS_T, PIECES) \
   rmsnorm_add_partials_kernel<T, KS_T, PIECES><<<grid, 256, 0, stream>>>(x, partial, KS, w, out, n_rows, H, eps)
-  if (H <= 1024 && KS == 4) TI_GO(4, 4);
-  else if (H <= 1024 && KS == 2) TI_GO(2, 4);
-  else if (H <= 1024 && KS == 8) TI_GO(8, 4);
-  else if (H <= 1024) TI_GO(0, 4);
-  else rmsnorm_add_partials_row_kernel<T><<<n_rows, 256, 0, stream>>>(x, partial, KS, w, out, n_rows, H, eps);
+  if (H > 1024) rmsnorm_add_partials_row_kernel<T, 4, 4><<<n_rows, 256, 0, stream>>>(x, partial, KS, w, out, n_rows, H, eps);
+  else if (n_rows <= RMS_ROW_EACH) rmsnorm_add_partials_row_kernel<T, 1, 8><<<n_rows, 256, 0, stream>>>(x, partial, KS, w, out, n_rows, H, eps);
+  else if (KS == 1) TI_GO(1, 4);
+  else if (KS == 2) TI_GO(2, 4);
+  else if (KS == 4) TI_GO(4, 4);
+  else TI_GO(0, 4);
 #undef TI_GO
 }
 
