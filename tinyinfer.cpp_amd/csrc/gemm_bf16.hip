@@ -8,8 +8,9 @@
 //    weight rows; the wavefronts split K between them in interleaved 128-byte
 //    pieces and reduce through LDS in a fixed order.  The weights are the "A"
 //    operand of v_mfma_f32_16x16x32_bf16, the tokens are the 16 columns.
-//  * tiled (M > 64, prefill): 128 x 128 x 32 tiles through double-buffered LDS,
-//    four wavefronts in 2 x 2, each 64 x 64 out of v_mfma_f32_32x32x16_bf16.
+//  * tiled (M > 64, prefill): tiles of 64 x 64 to 256 x 256, k-tiles of 64 through two to
+//    five stages of LDS, wavefronts' shares out of v_mfma_f32_32x32x16_bf16.  K that is
+//    no multiple of 64: 128 x 128 x 32 through double-buffered LDS.
 //
 // Epilogues: store float, add into a float residual, store bfloat16, or SwiGLU
 // over a stacked [gate; up] weight.  The reduction order of an output element
