@@ -105,3 +105,36 @@ def test_attention_under_every_cut_of_a_step(ops, nh, nkv, hd, P, window):  # no
     finally:
         ops.use_fast_attention = True
     assert (f64(rows) - f64(out)).abs().max() < 2e-5
+
+
+def hold(pool, table, P, nkv, hd, e, j, key, value):
+    """What the cache holds of request e's token j: its key and its value, the same number everywhere."""
+    page = pool[int(table[e, j // P])]
+    page[:nkv, j % P] = key
+    page[nkv:].view(nkv, hd, P)[:, :, j % P] = value
+
+
+@pytest.mark.parametrize("hd,P,window", [(16, 4, None), (64, 16, None), (128, 16, 20), (256, 4, 20), (144, 16, 33)])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_rows_do_not_feel_what_they_cannot_see(ops, bad, hd, P, window):  # noqa: F811
+    """Infinite and not-a-number keys and values of tokens in the middle of a text: rows in front of them, and rows whose
+    window has left them behind, keep their bits in every cut of the step; the rows that see them are spoiled."""
+    nh, nkv = 4, 2
+    entries = [(65, 0), (40, 37), (1, 50)]
+    qs, pool, table, _ = case(entries, nh, nkv, hd, P, window, seed=hd)
+    q, view, args = dev(torch.cat(qs)), View(dev(table)), (nh, nkv, hd, 1.0 / math.sqrt(hd), window)
+    clean, out = torch.empty_like(q), torch.empty_like(q)
+    ops.attention(FakeCtx(entries), view, q, pool, clean, *args)
+    told = [(0, 9, 0.0, bad), (0, 21, bad, 0.0), (1, 44, 0.0, -bad), (1, 61, bad, bad), (2, 50 - (window or 0) if window else 50, 0.0, bad)]
+    for e, j, key, value in told:
+        hold(pool, table, P, nkv, hd, e, j, key, value)
+    ops.attention(FakeCtx(entries), view, q, pool, out, *args)
+    row = 0
+    for e, (n, start) in enumerate(entries):
+        for p in range(start, start + n):
+            seen = any(x == e and j <= p and (not window or p - j < window) for x, j, _, _ in told)
+            if seen:
+                assert not torch.isfinite(out[row]).any(), (e, p)
+            else:
+                assert torch.equal(out[row], clean[row]), (e, p)
+            row += 1

@@ -138,8 +138,8 @@ extern "C" int ti_attention_rows(int dtype, const void* q, const void* pool, con
 //   S^T (16 keys x 16 columns) = K (16 x hd) . Q^T      O^T (hd x 16) += V^T (hd x 16 keys) . P^T
 // both by v_mfma_f32_16x16x4_f32 with four consecutive entries a lane (loaded as one float4; both operands of a product
 // are permuted alike), so that the scores' layout is the second product's operand.  Block b belongs to wavefront
-// b mod 8 whatever the tile, and a block that a column may not see leaves it bit by bit as it was: a token's result
-// depends on its keys alone, however a step is cut.  Keys and values come straight from memory, the next block's while
+// b mod 8 whatever the tile, and a key that a column may not see leaves it bit by bit as it was, whatever the key and its
+// value hold: a token's result depends on its keys alone, however a step is cut.  Keys and values come straight from memory, the next block's while
 // one is multiplied; short contexts are bounded by the start and the merge.  (With the rows kernel below, one workgroup
 // per row and head, lane sums and one value a load, a portion of 300 tokens with 16 heads of 128 on 8 kv heads took
 // 201 us a layer, 5.6 ms of a prompt of Qwen3-0.6B's sizes.)
@@ -185,6 +185,7 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
   const int hi = SINGLE ? p_last : p_first + col;
   const int lo = (window > 0 && hi - window + 1 > 0) ? hi - window + 1 : 0;
   const int lo_min = (window > 0 && p_first - window + 1 > 0) ? p_first - window + 1 : 0;
+  const int lo_max = (window > 0 && p_last - window + 1 > 0) ? p_last - window + 1 : 0;
 
   const size_t page_elems = (size_t)2 * n_kv * P * HD;
   const float* k_head = pool + (size_t)kvh * P * HD;
@@ -225,7 +226,7 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
       const int key = f.key0 + quad * 4 + i;
       sc[i] = (f.have && key >= lo && key <= hi) ? (s0[i] + s1[i]) * scale : -INFINITY;
       bm = fmaxf(bm, sc[i]);
-      if (!f.have || key > p_last) {                // never written: any bits, and 0 times NaN is NaN
+      if (!f.have || key > p_last || key < lo_min) {  // seen by no column: any bits, and 0 times NaN is NaN
 #pragma unroll
         for (int d = 0; d < DB; ++d) f.v[d][i] = 0.f;
       }
@@ -244,11 +245,39 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
     }
     mx = m_new;
 #pragma unroll
-    for (int d = 0; d < DB; ++d) {
-      o[d] *= alpha;
+    for (int d = 0; d < DB; ++d) o[d] *= alpha;
+    // A key that some columns see and others do not: a weight of 0 leaves those out unless the value is infinite or not a
+    // number.  Such values are taken out of the product and given to the columns that see them one by one.
+    if (!SINGLE && (f.key0 + 15 > p_first || f.key0 < lo_max)) {
+      float nil = 0.f;
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) nil = fmaf(f.v[d][j], 0.f, nil);
+      if (__any(nil != 0.f)) {
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int key = f.key0 + g * 4 + j;
+            const float weight = __shfl(w[j], g * 16 + r16, 64);
+#pragma unroll
+            for (int d = 0; d < DB; ++d)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const float v = __shfl(f.v[d][j], g * 16 + quad * 4 + i, 64);
+                if (v * 0.f != 0.f && key >= lo && key <= hi) o[d][i] = fmaf(v, weight, o[d][i]);
+              }
+          }
+#pragma unroll
+        for (int d = 0; d < DB; ++d)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) f.v[d][j] = f.v[d][j] * 0.f != 0.f ? 0.f : f.v[d][j];
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
 #pragma unroll
       for (int j = 0; j < 4; ++j) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.v[d][j], w[j], o[d], 0, 0, 0);
-    }
   };
   const int b_last = p_last / 16;
   int b = lo_min / 16;
