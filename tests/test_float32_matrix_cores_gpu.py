@@ -138,3 +138,15 @@ def test_rows_do_not_feel_what_they_cannot_see(ops, bad, hd, P, window):  # noqa
             else:
                 assert torch.equal(out[row], clean[row]), (e, p)
             row += 1
+
+
+def test_portions_without_a_list_of_small_tiles(ops):  # noqa: F811
+    """A work list that names its portions by tiles of 128 rows alone, beside a single token: every row is written."""
+    nh, nkv, hd, P = 4, 2, 64, 16
+    entries = [(65, 0), (1, 40)]
+    qs, pool, table, want = case(entries, nh, nkv, hd, P, None, seed=3)
+    ctx, q = FakeCtx(entries), dev(torch.cat(qs))
+    ctx.tiles_small, ctx.n_tiles_small = None, 0
+    out = torch.full_like(q, 7.0)
+    ops.attention(ctx, View(dev(table)), q, pool, out, nh, nkv, hd, 1.0 / math.sqrt(hd), None)
+    assert (f64(out) - torch.cat(want)).abs().max() < 2e-5

@@ -875,8 +875,10 @@ bool Ops::attention(const AttentionWork& work, Workspace& ws, const CacheView& v
       }
     }
   }
-  if (q.dtype == DType::F32 && softcap <= 0.f && use.fast_attention && (work.n_tiles_small == 0 || (work.tiles_small && work.entry_meta)) &&
-      (work.decode_only || work.n_tiles_small || work.n_decode_rows)) {
+  // float32: portions come by their small tiles; a list that names them by large tiles alone goes row by row
+  const bool small_tiles = work.n_tiles_small > 0 && work.tiles_small && work.entry_meta;
+  if (q.dtype == DType::F32 && softcap <= 0.f && use.fast_attention &&
+      (work.decode_only || small_tiles || (work.n_tiles == 0 && work.n_tiles_small == 0 && work.n_decode_rows))) {
     check_pool("attention", pool, kv_heads, head_dim, DType::F32);
     require(q.contiguous() && out.contiguous() && q.ndim == 2 && q.shape[1] == (int64_t)heads * head_dim && out.ndim == 2 &&
                 out.shape[0] == q.shape[0] && out.shape[1] == q.shape[1] && out.dtype == q.dtype,
