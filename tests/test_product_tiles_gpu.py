@@ -1,5 +1,7 @@
 """The pipelined product's tiles beyond the ones tests of the whole dispatch name, loops shorter than the ring of stages,
 the dies' blocks of tiles, and the q/k/v product in tiles of 64 rows."""
+import ctypes
+
 import pytest
 import torch
 
@@ -80,3 +82,20 @@ def test_sums_of_a_split_product(ops, M, N, K):  # noqa: F811
 @pytest.mark.parametrize("M,nh,nkv,hd,K", [(65, 16, 8, 128, 64), (129, 6, 2, 64, 128), (200, 4, 1, 128, 320), (512, 16, 8, 128, 192)])
 def test_qkv_product_with_prepared_heads_in_tiles_of_64_rows(ops, M, nh, nkv, hd, K):  # noqa: F811
     qkv_prepared_case(ops, 64, M, nh, nkv, hd, K, 16, True, "table")
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 5120, 17408), (32, 5120, 8192), (64, 5120, 17408)])
+def test_large_weights_under_few_rows_keep_eight_runs_of_k(ops, M, N, K):  # noqa: F811
+    """17 to 64 rows times a weight that is waited for from memory: eight runs of K, whose sums are within (K + 9) 2^-24 of
+    float64 for each of the terms."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a = (torch.rand(M, K, generator=g, device="cuda") * 2 - 1).to(torch.bfloat16)
+    w = (torch.rand(N, K, generator=g, device="cuda") * 2 - 1).to(torch.bfloat16)
+    x, partial, splits = torch.zeros(M, N, device="cuda"), torch.full((8, M, N), float("nan"), device="cuda"), ctypes.c_int(0)
+    lib, ptr = ops.lib("gemm_bf16"), lambda t: ctypes.c_void_p(t.data_ptr())
+    rc = lib.ti_gemm_bf16_add_split(ptr(a), ptr(w), ptr(x), M, N, K, ctypes.c_long(K), 1, ptr(partial),
+                                    ctypes.c_long(partial.numel() * 4), 1, ctypes.byref(splits), None)
+    torch.cuda.synchronize()
+    assert rc == 0 and splits.value == 8
+    ref, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    assert ((partial.double().sum(0) - ref).abs() <= (K + 9) * 2.0 ** -24 * size).all()

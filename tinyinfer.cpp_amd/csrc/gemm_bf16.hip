@@ -2068,6 +2068,10 @@ static int pieces_splits(int N, int K, long partial_bytes) {
 
 static int g_add_split = 1;        // a hook for measurements: 0: ti_gemm_bf16_add_split serves nothing
 
+// Elements from which up to 64 rows times a weight cut K by the weight's bytes and not by the tiles' cost.  Below it the cost
+// is right or better (4096 x 4096 at 24 rows: 12.3 us in four runs, 14.0 in eight), from here on it is slower or the same.
+#define STREAMED_WEIGHT (24L << 20)
+
 template <int EPI>
 static void launch_mblocks(const bf16_t* a, const bf16_t* w, void* out, float* partial, int M, int N, int K,
                            long lda, int KS, hipStream_t s) {
@@ -2137,6 +2141,16 @@ extern "C" int ti_gemm_bf16_add_split(const void* A, const void* W, void* out, i
       while (KS > 1 && (long)KS * M * N * 4 > partial_bytes) KS /= 2;
       // with the addition as a kernel of its own, only large products gain
       if (!defer && !((long)M * K >= 128 * 1024 || (K >= 3072 && (long)M * K >= 96 * 1024))) KS = 1;
+    } else if (pipelined_serves(M, K, lda) && M <= 64 && (long)N * K >= STREAMED_WEIGHT) {
+      // Up to 64 rows times a weight that is waited for from memory: about four workgroups of 64 x 64 per unit, so that
+      // enough of it is on its way at any time, as long as the sums stay a small part of its bytes.  The costs below know
+      // nothing of a weight's bytes and cut such a K in four (us at 32 rows, eight runs and four: 5120 x 25600 56.6 and
+      // 65.4, 5120 x 17408 40.3 and 45.9, 5120 x 8192 26.3 and 27.8).
+      const long tiles = (N + 63) / 64;
+      while (KS < 8 && tiles * KS * 2 <= 4L * compute_units() && nb / (KS * 2) >= 4 && (long)KS * 2 * M * 16 <= K) KS *= 2;
+      while (KS > 1 && (long)KS * M * N * 4 > partial_bytes) KS /= 2;
+      if (!defer && KS < 4) KS = 1;
+      if (KS > 1) tile = choose_tile(false, M, N, nb / KS, KS, false).id;
     } else if (pipelined_serves(M, K, lda)) {
       // A product of few tiles, a short loop each, leaves units idle: K split between workgroups fills them, and the sums
       // cost their bytes once more where they are added (by the norm behind, or a kernel of its own).  Split as many
