@@ -99,3 +99,18 @@ def test_large_weights_under_few_rows_keep_eight_runs_of_k(ops, M, N, K):  # noq
     assert rc == 0 and splits.value == 8
     ref, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
     assert ((partial.double().sum(0) - ref).abs() <= (K + 9) * 2.0 ** -24 * size).all()
+
+
+def test_rows_too_long_for_the_tiled_kernel(ops):  # noqa: F811
+    """A row of 2^21 entries: the kernel whose loads have 32-bit offsets inside a tile leaves it to others, split or not.
+    Sums of ones and zeros are exact."""
+    M, N, K = 17, 64, 1 << 21
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a = (torch.rand(M, K, generator=g, device="cuda") < 0.5).to(torch.bfloat16)
+    w = (torch.rand(N, K, generator=g, device="cuda") < 0.5).to(torch.bfloat16)
+    out, partial = torch.empty(M, N, device="cuda"), torch.empty(8, M, N, device="cuda")
+    lib, ptr = ops.lib("gemm_bf16"), lambda t: ctypes.c_void_p(t.data_ptr())
+    assert lib.ti_gemm_bf16_store_split(ptr(a), ptr(w), ptr(out), M, N, K, ctypes.c_long(K), ptr(partial),
+                                        ctypes.c_long(partial.numel() * 4), None) == 3
+    ops.linear(a, w, out, "store")
+    assert torch.equal(out, (a.float() @ w.float().T).round())

@@ -1313,7 +1313,7 @@ static int g_qkv_rows = 0;       // hooks for measurements: 128 or 256 forces th
 static int g_qkv_min_rows = 17;  // the fewest rows served (fewer take the kernels with the norm in front)
 
 // What the pipelined kernel takes: k-tiles of 64, and rows whose offsets inside a tile fit its 32-bit load offsets.
-static bool pipelined_serves(int M, int K, long lda) { return K % PBK == 0 && K < (1 << 21) && lda < (1 << 21); }
+static bool pipelined_serves(int K, long lda) { return K % PBK == 0 && K < (1 << 21) && lda < (1 << 21); }
 
 static int compute_units() {
   static int n = 0;
@@ -1431,7 +1431,7 @@ extern "C" int ti_gemm_bf16_qkv_prep(const void* A, const void* W, int M, int K,
                                      int page_size, hipStream_t stream) {
   TI_REQUIRE(M >= 0 && K > 0 && lda >= K && n_head > 0 && n_kv >= 0 && hd > 0 && page_size > 0 && table_stride > 0,
              "gemm_bf16_qkv_prep: bad sizes");
-  if (M < g_qkv_min_rows || !pipelined_serves(M, K, lda) || lda % 8 != 0 || !(hd == 64 || hd == 128) || ((uintptr_t)A & 15) ||
+  if (M < g_qkv_min_rows || !pipelined_serves(K, lda) || lda % 8 != 0 || !(hd == 64 || hd == 128) || ((uintptr_t)A & 15) ||
       ((uintptr_t)W & 15) || ((uintptr_t)q_out & 15) || ((uintptr_t)pool & 15) || ((uintptr_t)rope_table & 15)) {
     ti_set_error("gemm_bf16_qkv_prep: M=%d K=%d head_dim=%d is not served (M > 16, K %% 64 == 0, head_dim 64 or 128)",
                  M, K, hd);
@@ -2141,7 +2141,7 @@ extern "C" int ti_gemm_bf16_add_split(const void* A, const void* W, void* out, i
       while (KS > 1 && (long)KS * M * N * 4 > partial_bytes) KS /= 2;
       // with the addition as a kernel of its own, only large products gain
       if (!defer && !((long)M * K >= 128 * 1024 || (K >= 3072 && (long)M * K >= 96 * 1024))) KS = 1;
-    } else if (pipelined_serves(M, K, lda) && M <= 64 && (long)N * K >= STREAMED_WEIGHT) {
+    } else if (pipelined_serves(K, lda) && M <= 64 && (long)N * K >= STREAMED_WEIGHT) {
       // Up to 64 rows times a weight that is waited for from memory: about four workgroups of 64 x 64 per unit, so that
       // enough of it is on its way at any time, as long as the sums stay a small part of its bytes.  The costs below know
       // nothing of a weight's bytes and cut such a K in four (us at 32 rows, eight runs and four: 5120 x 25600 56.6 and
@@ -2151,7 +2151,7 @@ extern "C" int ti_gemm_bf16_add_split(const void* A, const void* W, void* out, i
       while (KS > 1 && (long)KS * M * N * 4 > partial_bytes) KS /= 2;
       if (!defer && KS < 4) KS = 1;
       if (KS > 1) tile = choose_tile(false, M, N, nb / KS, KS, false).id;
-    } else if (pipelined_serves(M, K, lda)) {
+    } else if (pipelined_serves(K, lda)) {
       // A product of few tiles, a short loop each, leaves units idle: K split between workgroups fills them, and the sums
       // cost their bytes once more where they are added (by the norm behind, or a kernel of its own).  Split as many
       // ways as tile and sums together are the cheapest (512 x 1024 x 3072: 13 us whole, 9.5 in two; the norm 0.6 more).
@@ -2249,7 +2249,7 @@ extern "C" int ti_gemm_bf16_store_split(const void* A, const void* W, void* out,
                                         void* partial, long partial_bytes, hipStream_t stream) {
   TI_REQUIRE(M >= 0 && N > 0 && K > 0 && lda >= K, "gemm_bf16_store_split: bad sizes M=%d N=%d K=%d lda=%ld", M, N, K, lda);
   int KS = 1;
-  if (g_add_split && g_use_pipelined && partial && M > 16 && M <= 64 && K % 64 == 0 && lda % 8 == 0 &&
+  if (g_add_split && g_use_pipelined && partial && M > 16 && M <= 64 && pipelined_serves(K, lda) && lda % 8 == 0 &&
       !((uintptr_t)A & 15) && !((uintptr_t)W & 15) && !((uintptr_t)partial & 15) &&
       large_weight(M, N, K, TI_EPI_STORE_F32) && !wide_rows_serves(M, N, K, TI_EPI_STORE_F32)) {
     const long tiles = (N + 63) / 64;
@@ -2351,7 +2351,7 @@ extern "C" int ti_gemm_bf16(const void* A, const void* W, void* out, int M, int 
       if (rc_) return rc_;                                        \
     } else if (skinny)                                            \
       launch_skinny<E>(a, w, out, M, N, K, lda, stream);          \
-    else if (g_use_pipelined && pipelined_serves(M, K, lda)) {    \
+    else if (g_use_pipelined && pipelined_serves(K, lda)) {    \
       int rc_ = launch_tiled_best<E>(a, w, out, M, N, K, lda, stream); \
       if (rc_) return rc_;                                        \
     } else                                                        \
