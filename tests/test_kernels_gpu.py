@@ -1,6 +1,7 @@
 """Each kernel alone against a plain PyTorch reference of the same op (float64
 on the CPU), at sizes other than the engine's.  Vectors that the reference's own
 selftest holds are marked with its file:line."""
+import ctypes
 import math
 
 import numpy as np
@@ -1001,11 +1002,13 @@ def test_partial_sums_left_to_the_next_norm(ops, M, N, K):
 
 
 @pytest.mark.parametrize("rows,H,KS", [(5, 2304, 3), (3, 1028, 5), (9, 64, 1), (2, 1024, 4), (70, 1536, 2),
-                                       (8, 5120, 4), (3, 4100, 2), (2, 8192, 3), (5, 9220, 2), (1, 20480, 1)])
+                                       (8, 5120, 4), (3, 4100, 2), (2, 8192, 3), (5, 9220, 2), (1, 20480, 1),
+                                       (1024, 1024, 8), (1025, 1024, 8), (1025, 1024, 2), (1100, 1020, 1), (1030, 516, 4),
+                                       (1027, 260, 3)])
 def test_rmsnorm_that_adds_partial_sums(ops, rows, H, KS):
     """The norm that first adds KS partial sums to its rows, alone, at widths and counts that the
-    products of the engine do not produce: the rows afterwards are x + p0 + ... in that order
-    (bit for bit), and the output is the norm of them, in the bits of the plain norm kernel."""
+    products of the engine do not produce, and on either side of the 1,024 rows up to which narrow
+    rows have a workgroup each: the rows afterwards are x + p0 + ... in that order (bit for bit), and the output is the norm of them, in the bits of the plain norm kernel."""
     import ctypes
     g = torch.Generator().manual_seed(rows + H + KS)
     x0 = torch.randn(rows, H, generator=g)
@@ -1033,10 +1036,9 @@ def test_rmsnorm_that_adds_partial_sums(ops, rows, H, KS):
 @pytest.mark.parametrize("tile", [1, 3, 5, 6, 8, 9, 10])
 @pytest.mark.parametrize("M,N,K", [(300, 520, 128), (257, 384, 192), (130, 200, 64), (700, 96, 320)])
 def test_linear_bf16_every_tile(ops, tile, M, N, K):
-    """Each tile of the pipelined kernel (256 x 128 with eight wavefronts, 128 x 64, 64 x 128 for the SwiGLU
-    epilogue, 64 x 64, 128 x 160 and 256 x 160 with four wavefronts, which the SwiGLU epilogue does not
-    take, and 256 x 256 with k-tiles of 32 in a ring of four stages), whatever the dispatch would have chosen
-    for the shape, with every epilogue, against float64."""
+    """Tiles of the pipelined kernel (256 x 128 with eight wavefronts, 128 x 64, 64 x 64, 128 x 160 and 256 x 160
+    with four wavefronts, which the SwiGLU epilogue does not take, and for it alone 64 x 128 and 256 x 256 in two
+    stages), whatever the dispatch would have chosen for the shape, with every epilogue, against float64."""
     assert ops.use_fast_gemm, "the bfloat16 MFMA kernels are switched off or not built"
     lib = ops.lib("gemm_bf16")
     g = torch.Generator().manual_seed(M + N + tile)
@@ -1069,16 +1071,20 @@ def test_linear_bf16_every_tile(ops, tile, M, N, K):
         ops.tune()
 
 
-@pytest.mark.parametrize("M,N,K", [(2000, 5130, 192), (2048, 5120, 64), (1100, 9000, 128)])
+def takes_two_ranges(ops, swiglu, M, N, K):
+    rest, n_big = ctypes.c_int(0), ctypes.c_int(0)
+    tile = ops.lib("gemm_bf16").ti_gemm_bf16_tile_choice(int(swiglu), M, N, K, ctypes.byref(rest), ctypes.byref(n_big))
+    return 0 < n_big.value < N and rest.value not in (0, tile)
+
+
+@pytest.mark.parametrize("M,N,K", [(2000, 5130, 2048), (2048, 6144, 1024), (1100, 9000, 1024)])
 def test_columns_split_between_two_tile_shapes(ops, M, N, K):
-    """256 x 128 tiles that fill the compute units once or more and leave a round mostly empty: the columns
-    that make whole rounds take those tiles, the rest 128 x 64 tiles in a second launch.  Same bits as the
-    smaller tile everywhere, and the values of float64, for every epilogue."""
+    """Large tiles that fill the compute units once or more and leave a round mostly empty: the columns that
+    make whole rounds take those tiles, the rest smaller ones in a second launch.  Same bits as one tile
+    everywhere, and the values of float64, for every epilogue."""
     assert ops.use_fast_gemm, "the bfloat16 MFMA kernels are switched off or not built"
     lib = ops.lib("gemm_bf16")
-    units = torch.cuda.get_device_properties(0).multi_processor_count
-    big = -(-M // 256) * -(-N // 128)
-    assert big >= units and 0 < big % units < units * 3 // 4 and big < 4 * units, "the shape does not take the rule"
+    assert takes_two_ranges(ops, False, M, N, K) and takes_two_ranges(ops, True, M, N // 2, K), "the shape does not take two ranges"
     g = torch.Generator().manual_seed(M + N)
     a = (torch.rand(M, K, generator=g) * 2 - 1).to(torch.bfloat16)
     w = (torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16)
@@ -1145,7 +1151,7 @@ def test_widths_that_160_divides_take_tiles_of_160_columns(ops, M, N, K):
 
 
 @pytest.mark.parametrize("tile,M,N,K", [(1, 700, 2048, 128), (1, 2300, 1024, 64), (3, 700, 1024, 192), (9, 1100, 1280, 64),
-                                        (0, 1500, 2048, 128)])
+                                        (0, 2048, 6144, 1024)])
 @pytest.mark.parametrize("rows", [1, 3, 8])
 def test_tiles_taken_in_the_dies_order(ops, tile, M, N, K, rows):
     """The order in which workgroups take a tiled product's tiles when the weight is larger than the cache
@@ -1154,6 +1160,7 @@ def test_tiles_taken_in_the_dies_order(ops, tile, M, N, K, rows):
     block of row tiles is short where `rows` does not divide their number; tile 0 is a launch in two ranges."""
     assert ops.use_fast_gemm, "the bfloat16 MFMA kernels are switched off or not built"
     lib = ops.lib("gemm_bf16")
+    assert tile or (takes_two_ranges(ops, False, M, N, K) and takes_two_ranges(ops, True, M, N // 2, K))
     g = torch.Generator().manual_seed(M + N + rows)
     a = dev((torch.rand(M, K, generator=g) * 2 - 1).to(torch.bfloat16))
     w = dev((torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16))
@@ -1189,7 +1196,7 @@ def test_tiles_taken_in_the_dies_order(ops, tile, M, N, K, rows):
 def test_stacked_gate_up_over_many_rows_takes_tiles_of_256_x_256(ops, M, F, K):
     """A [gate; up] weight over many rows with a long K: 256 x 256 tiles where they make whole rounds of the
     compute units (8 x 32 tiles), and where rounds are left over (8 x 72 tiles: two rounds and a quarter) the
-    whole rounds' columns take them and the rest 256 x 128 tiles; rows and columns that fill no tile.
+    whole rounds' columns take them and the rest 128 x 128 tiles; rows and columns that fill no tile.
     The bits of the product with the rule switched off, and the values of float64."""
     assert ops.use_fast_gemm, "the bfloat16 MFMA kernels are switched off or not built"
     lib = ops.lib("gemm_bf16")
@@ -1723,8 +1730,7 @@ def decode_from_projections_case(ops, nh, nkv, hd, P, window, norm, rope, starts
 @pytest.mark.parametrize("tile_rows", [128, 256])
 def test_qkv_product_with_prepared_heads(ops, tile_rows, M, nh, nkv, hd, K, P, norm, rope):
     """The q/k/v product whose epilogue norms, rotates and caches, with tiles of 128 and of 256
-    rows (the dispatch takes the first while it makes no more workgroups than the chip has
-    units), against the product followed by the kernel that prepares whole steps: the same bits
+    rows, against the product followed by the kernel that prepares whole steps: the same bits
     in q and in the cache (rows that are no multiple of the tile, a last tile with a head beyond
     the matrix, no k/v heads)."""
     qkv_prepared_case(ops, tile_rows, M, nh, nkv, hd, K, P, norm, rope)
@@ -1734,10 +1740,10 @@ def test_qkv_product_with_prepared_heads(ops, tile_rows, M, nh, nkv, hd, K, P, n
 def test_qkv_product_with_prepared_heads_in_two_ranges(ops, M, nh, nkv, hd):
     """256-row tiles that would leave a round of workgroups mostly empty: the heads that make whole
     rounds take them, the other heads 128-row tiles in a second launch.  The same bits."""
-    units = torch.cuda.get_device_properties(0).multi_processor_count
-    big = -(-M // 256) * ((nh + 2 * nkv) * hd // 128)
-    assert big >= units and 0 < big % units < units * 3 // 4, "the shape does not take the rule"
-    qkv_prepared_case(ops, 0, M, nh, nkv, hd, 64, 16, True, "table")
+    K, n_big = 2048, ctypes.c_int(0)
+    rows = ops.lib("gemm_bf16").ti_gemm_bf16_qkv_choice(M, (nh + 2 * nkv) * hd, K, ctypes.byref(n_big))
+    assert rows == 256 and 0 < n_big.value < (nh + 2 * nkv) * hd, "the shape does not take two ranges"
+    qkv_prepared_case(ops, 0, M, nh, nkv, hd, K, 16, True, "table")
 
 
 @pytest.mark.parametrize("tile_rows,rows", [(128, 4), (256, 2)])

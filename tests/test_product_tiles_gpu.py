@@ -64,19 +64,28 @@ def test_dies_blocks_cover_every_tile_once(ops, M, N, K):  # noqa: F811
     assert (f64(outs[0]) - ref_linear(a.cpu(), w.cpu())).abs().max() < 2e-5 * K
 
 
-@pytest.mark.parametrize("M,N,K", [(77, 1024, 3072), (256, 1024, 2048), (512, 2048, 512), (130, 4096, 4096), (700, 1000, 1024)])
+@pytest.mark.parametrize("M,N,K", [(77, 1024, 3072), (256, 1024, 2048), (512, 2048, 512), (130, 4096, 4096), (700, 1000, 1024),
+                                   (2048, 1024, 3072)])
 def test_sums_of_a_split_product(ops, M, N, K):  # noqa: F811
-    """Products into the residual whose launch is cut into two, four or eight runs of K, or left whole, as their cost says."""
+    """Products into the residual whose launch is cut into two, four or eight runs of K, or left whole, as their cost says.  The
+    norm behind a product whose sums were left adds them to the same bits and has the bits of the norm of their sum."""
     g = torch.Generator().manual_seed(M + N + K)
     a = dev((torch.rand(M, K, generator=g) * 2 - 1).to(torch.bfloat16))
     w = dev((torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16))
     base = dev(torch.randn(M, N, generator=g))
     ref, size = ref_linear(a.cpu(), w.cpu()) + f64(base), f64(a).abs() @ f64(w).abs().T + f64(base).abs()
-    for may_defer in (True, False):
+    for may_defer in (False, True):
         x = base.clone()
         ops.linear(a, w, x, "add", may_defer=may_defer)
         ops.flush()
         assert ((f64(x) - ref).abs() <= (K + 9) * 2.0 ** -24 * size).all()
+    nw = dev(torch.rand(N, generator=g) + 0.5)
+    normed, want = (torch.empty(M, N, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    ops.rmsnorm(x, nw, 1e-6, want)
+    y = base.clone()
+    ops.linear(a, w, y, "add", may_defer=True)
+    ops.rmsnorm(y, nw, 1e-6, normed)
+    assert torch.equal(y, x) and torch.equal(normed, want)
 
 
 @pytest.mark.parametrize("M,nh,nkv,hd,K", [(65, 16, 8, 128, 64), (129, 6, 2, 64, 128), (200, 4, 1, 128, 320), (512, 16, 8, 128, 192)])

@@ -1033,8 +1033,9 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
   // the remaining instructions; no k-tile begins with a wait for LDS.  Whole tiles run without a branch,
   // the last STAGES - 1 by themselves.
   // (Against a loop that met in front of each k-tile, read its first fragments there and asked by lane
-  // addresses, us: 2048 x 24576 x 4096 with SwiGLU 382 -> 328, 2048 x 4096 x 12288 193 -> 167,
-  // 2048 x 4096 x 4096 70 -> 61, 2048 x 4096 x 1024 24 -> 22; the library's kernels 296, 180, 62 and 24.)
+  // addresses, us alone: 2048 x 24576 x 4096 with SwiGLU 382 -> 328, 2048 x 4096 x 12288 193 -> 167,
+  // 2048 x 4096 x 4096 70 -> 61, 2048 x 4096 x 1024 24 -> 22.  Inside a prompt, where the chip is warmer, the first
+  // takes 340.)
   const int fr = lane & 31, fh = lane >> 5;                  // fragment row, and which half of a 16-wide k-step
   const unsigned lds0 = (unsigned)(size_t)smem;              // LDS byte address of the first stage
   const unsigned rowA = lds0 + (wm * (BM / WAVES_M) + fr) * ROWB;
@@ -1309,7 +1310,7 @@ static int launch_pipelined(const bf16_t* A, const bf16_t* W, void* out, int M, 
 static int g_tiles_160 = 1;      // a hook for measurements: 0 = no tiles of 160 columns
 static int g_tiles_256 = 1;      // a hook for measurements: 0 = no tiles of 256 x 256
 static int g_two_ranges = 1;     // a hook for measurements: 0 = never split the columns between two tile shapes
-static int g_qkv_rows = 0;       // hooks for measurements: 128 or 256 forces the tile's rows;
+static int g_qkv_rows = 0;       // hooks for measurements: 64, 128 or 256 forces the tile's rows;
 static int g_qkv_min_rows = 17;  // the fewest rows served (fewer take the kernels with the norm in front)
 
 // What the pipelined kernel takes: k-tiles of 64, and rows whose offsets inside a tile fit its 32-bit load offsets.
@@ -1355,21 +1356,25 @@ static int g_force_tile = 0;
 // (us, k-tiles of 64) are fitted to 300 products: 65 to 6,000 rows times the four weights of a layer of Qwen3-0.6B's, 1.7B's,
 // 4B's and 8B's sizes, weights not in the caches, K also cut in two, four and eight.  The median error is 3 to 9 %, and the
 // tile that is the cheapest by them is on average 0.8 % slower than the fastest (with K split 1.8 %, SwiGLU 0.9 %).
+// Beyond what it was fitted to, 17 to 2,048 rows times the weights of Qwen3-14B's and 32B's sizes against the rules measured
+// before it: 0 to 49 % faster (5120 x 25600 under 264 rows 206 -> 124 us), but for 200 rows times 32B's gate/up, 2 % slower,
+// and for the runs of K under up to 64 rows, which ti_gemm_bf16_add_split therefore counts itself.  Inside the fit the worst
+// seen against them is 2560 x 4096 under 264 to 300 rows, 21.7 -> 23.9 us.
 // Fewer rows of A than a tile has cost what the whole tile costs.
 struct TileRate {
-  int id, bm, bn, stages;
+  int id, bm, bn;
   float start1, each1, fill1;        // one workgroup to a unit
   float start2, each2, fill2;        // two (0: they do not fit)
 };
 static const TileRate TILES_PLAIN[] = {
-    {1, 256, 128, 3, 4.96f, 0.54f, 0.35f, 0.f, 0.f, 0.f},     {11, 256, 128, 3, 6.58f, 0.55f, 0.30f, 0.f, 0.f, 0.f},
-    {2, 128, 128, 4, 3.25f, 0.39f, 0.16f, 0.f, 0.f, 0.f},     {4, 128, 64, 4, 2.46f, 0.28f, 0.05f, 0.f, 0.f, 0.f},
-    {3, 128, 64, 3, 2.17f, 0.38f, 0.06f, 3.48f, 0.26f, 0.39f}, {6, 64, 64, 5, 1.27f, 0.20f, 0.05f, 1.96f, 0.19f, 0.22f},
-    {8, 128, 160, 3, 4.98f, 0.51f, 0.13f, 0.f, 0.f, 0.f},     {9, 256, 160, 3, 8.03f, 0.63f, 0.35f, 0.f, 0.f, 0.f}};
+    {1, 256, 128, 4.96f, 0.54f, 0.35f, 0.f, 0.f, 0.f},     {11, 256, 128, 6.58f, 0.55f, 0.30f, 0.f, 0.f, 0.f},
+    {2, 128, 128, 3.25f, 0.39f, 0.16f, 0.f, 0.f, 0.f},     {4, 128, 64, 2.46f, 0.28f, 0.05f, 0.f, 0.f, 0.f},
+    {3, 128, 64, 2.17f, 0.38f, 0.06f, 3.48f, 0.26f, 0.39f}, {6, 64, 64, 1.27f, 0.20f, 0.05f, 1.96f, 0.19f, 0.22f},
+    {8, 128, 160, 4.98f, 0.51f, 0.13f, 0.f, 0.f, 0.f},     {9, 256, 160, 8.03f, 0.63f, 0.35f, 0.f, 0.f, 0.f}};
 static const TileRate TILES_SWIGLU[] = {
-    {10, 256, 256, 2, 5.46f, 1.39f, 0.20f, 0.f, 0.f, 0.f},    {1, 256, 128, 3, 3.08f, 0.56f, 0.28f, 0.f, 0.f, 0.f},
-    {2, 128, 128, 4, 0.f, 0.54f, 0.05f, 0.f, 0.f, 0.f},       {7, 64, 128, 4, 0.f, 0.40f, 0.03f, 0.f, 0.f, 0.f},
-    {5, 64, 128, 3, 0.f, 0.45f, 0.09f, 0.f, 0.55f, 0.20f}};
+    {10, 256, 256, 5.46f, 1.39f, 0.20f, 0.f, 0.f, 0.f},    {1, 256, 128, 3.08f, 0.56f, 0.28f, 0.f, 0.f, 0.f},
+    {2, 128, 128, 0.f, 0.54f, 0.05f, 0.f, 0.f, 0.f},       {7, 64, 128, 0.f, 0.40f, 0.03f, 0.f, 0.f, 0.f},
+    {5, 64, 128, 0.f, 0.45f, 0.09f, 0.f, 0.55f, 0.20f}};
 static const double LAUNCH_US = 2.0;
 
 static double tile_us(const TileRate& t, long workgroups, int k_tiles) {
@@ -1420,10 +1425,66 @@ static TileChoice choose_tile(bool swiglu, int M, int rows, int k_tiles, int cop
   return best;
 }
 
+// The tile of the q/k/v product that finishes its heads: of 64, 128 or 256 rows the one whose launch costs the least,
+// 256-row tiles also as whole rounds of the units with the heads left over in 128-row tiles behind them (Qwen3-8B's 48 heads
+// over 2,048 rows), beside the plain product in its own best tile followed by the kernel that prepares whole steps, which
+// reads the product's 32-bit sums again.  Finishing the heads costs a tile about 3 us (512 rows of Qwen3-0.6B's sizes in
+// tiles of 128 x 128: 18.9 us; of 64 x 128, on all units: 12).  Steps of up to 64 rows whose tiles leave most units idle
+// always go to the product.
+struct QKVChoice {
+  int rows = 0;             // of a tile; 0: left to the product and the preparation kernel
+  int n_big = 0;            // > 0: that many columns in 256-row tiles, the others in 128-row tiles
+};
+static QKVChoice qkv_choice(int M, int N, int K) {
+  QKVChoice c{g_qkv_rows, 0};
+  if (c.rows) return c;                             // (a test asks for a tile)
+  const long units = compute_units();
+  const int k_tiles = K / PBK, col_tiles = (N + 127) / 128;
+  auto us = [&](int rows, int cols) {               // (a tile of 64 x 128 does what one of 128 x 64 does)
+    const int id = rows == 256 ? 1 : rows == 128 ? 2 : 4;
+    const TileRate* t = TILES_PLAIN;
+    while (t->id != id) ++t;
+    return LAUNCH_US + 3.0 + tile_us(*t, (long)((M + rows - 1) / rows) * cols, k_tiles);
+  };
+  double least = us(64, col_tiles);
+  c.rows = 64;
+  for (int r = 128; r <= 256; r *= 2)
+    if (us(r, col_tiles) < least) {
+      least = us(r, col_tiles);
+      c.rows = r;
+    }
+  const long row_tiles = (M + 255) / 256, big = row_tiles * col_tiles;
+  if (g_two_ranges && big > units && big % units != 0) {
+    const int cols = (int)(big / units * units / row_tiles);
+    if (cols >= 1 && us(256, cols) + us(128, col_tiles - cols) < least) {
+      least = us(256, cols) + us(128, col_tiles - cols);
+      c = {256, cols * 128};
+    }
+  }
+  const double apart = choose_tile(false, M, N, k_tiles, 1, true).us + LAUNCH_US + 2.0 + 2.0 * M * N * 4 / 4.0e6;
+  if (M <= 64 ? (long)((M + 127) / 128) * col_tiles * 2 < units : apart < least) c = {0, 0};
+  return c;
+}
+
+// What the two rules choose, for tests: the tile of a product of N output columns (and, where the columns are split, the
+// second tile and the column it begins at), the rows of the q/k/v product's tile (0: left to the product, and likewise).
+extern "C" int ti_gemm_bf16_tile_choice(int swiglu, int M, int N, int K, int* rest, int* n_big) {
+  const TileChoice c = choose_tile(swiglu != 0, M, swiglu ? 2 * N : N, K / PBK, 1, true);
+  *rest = c.rest;
+  *n_big = swiglu ? c.n_big / 2 : c.n_big;
+  return c.id;
+}
+extern "C" int ti_gemm_bf16_qkv_choice(int M, int N, int K, int* n_big) {
+  const QKVChoice c = qkv_choice(M, N, K);
+  *n_big = c.n_big;
+  return c.rows;
+}
+
 // The fused q/k/v projection of a step's rows with the per-head work in its epilogue (see
 // QKVEpilogue): A [M, K] bf16, W [(n_head + 2 n_kv) hd, K] bf16 (n_kv = 0: q heads only, nothing is
 // written to the cache).  Returns 3 for what it does not serve: M <= 16, K not a multiple of 64,
-// head sizes other than 64 and 128.
+// head sizes other than 64 and 128, and sizes at which the product and the preparation kernel cost
+// less (qkv_choice).
 extern "C" int ti_gemm_bf16_qkv_prep(const void* A, const void* W, int M, int K, long lda, const float* q_w,
                                      const float* k_w, float eps, const float* inv_freq, const float* rope_table,
                                      int table_len, const int* pos, const int* slot, const int* table,
@@ -1442,54 +1503,18 @@ extern "C" int ti_gemm_bf16_qkv_prep(const void* A, const void* W, int M, int K,
   QKVEpilogue ep{q_w, k_w, eps, inv_freq, (const float2*)rope_table, table_len, pos, slot, table, table_stride,
                  (bf16_t*)pool, (bf16_t*)q_out, n_head, n_kv, hd, page_size};
   const int N = (n_head + 2 * n_kv) * hd;
-  // The tile of 64, 128 or 256 rows whose launch costs the least, 256-row tiles also as whole rounds of the units with the
-  // heads left over in 128-row tiles behind them (Qwen3-8B's 48 heads over 2,048 rows), beside the plain product in its own best
-  // tile followed by the kernel that prepares whole steps, which reads the product's 32-bit sums again.  Finishing the heads
-  // costs a tile about 3 us (tiles of 128 x 128 for 512 rows of Qwen3-0.6B's sizes, the only ones below 1,024 rows before:
-  // 18.9 us; of 64 x 128, on all units: 12).  Not when a test asks for a tile; steps of up to 64 rows whose tiles
-  // leave most units idle always go to the product.
-  const long units = compute_units();
-  const int k_tiles = K / PBK, col_tiles = (N + 127) / 128;
-  auto tile_of = [&](int id) -> const TileRate& {
-    for (const auto& t : TILES_PLAIN)
-      if (t.id == id) return t;
-    return TILES_PLAIN[0];
-  };
-  auto us = [&](int rows, int cols) {               // (a tile of 64 x 128 does what one of 128 x 64 does)
-    const TileRate& t = tile_of(rows == 256 ? 1 : rows == 128 ? 2 : 4);
-    return LAUNCH_US + 3.0 + tile_us(t, (long)((M + rows - 1) / rows) * cols, k_tiles);
-  };
-  int rows = g_qkv_rows, n_big = 0;                 // n_big > 0: that many columns in 256-row tiles, the others in 128-row tiles
-  if (!rows) {
-    double least = us(64, col_tiles);
-    rows = 64;
-    for (int r = 128; r <= 256; r *= 2)
-      if (us(r, col_tiles) < least) {
-        least = us(r, col_tiles);
-        rows = r;
-      }
-    const long row_tiles = (M + 255) / 256, big = row_tiles * col_tiles;
-    if (g_two_ranges && big > units && big % units != 0) {
-      const int cols = (int)(big / units * units / row_tiles);
-      if (cols >= 1 && us(256, cols) + us(128, col_tiles - cols) < least) {
-        least = us(256, cols) + us(128, col_tiles - cols);
-        rows = 256;
-        n_big = cols * 128;
-      }
-    }
-    const double apart = choose_tile(false, M, N, k_tiles, 1, true).us + LAUNCH_US + 2.0 + 2.0 * M * N * 4 / 4.0e6;
-    if (M <= 64 ? (long)((M + 127) / 128) * col_tiles * 2 < units : apart < least) {
-      ti_set_error("gemm_bf16_qkv_prep: %d rows are left to the product and the preparation kernel", M);
-      return 3;
-    }
+  const QKVChoice c = qkv_choice(M, N, K);
+  if (!c.rows) {
+    ti_set_error("gemm_bf16_qkv_prep: %d rows are left to the product and the preparation kernel", M);
+    return 3;
   }
   int rc_;
-  if (n_big) {
-    rc_ = launch_qkv_prep<256, 4, 2, 3>(A, W, M, N, K, lda, ep, stream, 0, n_big);
-    if (!rc_) rc_ = launch_qkv_prep<128, 4, 2, 4>(A, W, M, N, K, lda, ep, stream, n_big, N);
-  } else if (rows == 64) {
+  if (c.n_big) {
+    rc_ = launch_qkv_prep<256, 4, 2, 3>(A, W, M, N, K, lda, ep, stream, 0, c.n_big);
+    if (!rc_) rc_ = launch_qkv_prep<128, 4, 2, 4>(A, W, M, N, K, lda, ep, stream, c.n_big, N);
+  } else if (c.rows == 64) {
     rc_ = launch_qkv_prep<64, 2, 4, 4>(A, W, M, N, K, lda, ep, stream);
-  } else if (rows == 128) {
+  } else if (c.rows == 128) {
     rc_ = launch_qkv_prep<128, 4, 2, 4>(A, W, M, N, K, lda, ep, stream);
   } else {
     rc_ = launch_qkv_prep<256, 4, 2, 3>(A, W, M, N, K, lda, ep, stream);
@@ -1513,8 +1538,9 @@ static int launch_tile(int id, const bf16_t* A, const bf16_t* W, void* out, int 
       case 7: return launch_pipelined<64, 128, 2, 2, EPI, 4>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
       case 10: return launch_pipelined<256, 256, 4, 2, EPI, 2>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
     }
-    return launch_pipelined<128, 64, 4, 1, EPI>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);      // 3, and a forced tile
-  } else {                                                                                                // that it does not have
+    // (a forced tile that it does not have)
+    return launch_pipelined<128, 128, 4, 2, EPI, 4>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+  } else {
     switch (id) {
       case 4: return launch_pipelined<128, 64, 2, 2, EPI, 4>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
       case 6: return launch_pipelined<64, 64, 2, 2, EPI, 5>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
@@ -2098,8 +2124,8 @@ extern "C" int ti_gemm_bf16_partials_add(float* out, const float* partial, int K
 // leave most compute units idle (few rows times a weight of few rows): K is split over workgroups,
 // which leave their sums in `partial` [KS][M][N] (workspace of partial_bytes).  17..64 rows:
 // gemm_mblocks_kernel (measured against the kernels without MFMA at 64 rows: 1024 x 3072 19.7 ->
-// 9.7 us with the addition of the partial sums as a kernel of its own, ~6 us without).  More rows:
-// the pipelined kernel with 64 x 64 tiles, storing (136 rows: 18.5 -> ~8 us).
+// 9.7 us with the addition of the partial sums as a kernel of its own, ~6 us without).  More rows, and
+// 17..64 under a large weight: the pipelined kernel, storing, in the tile that costs the least.
 // Up to 16 rows: the kernel with the token rows in pieces, where pieces_splits says so.
 // defer = 0: the partial sums are added to `out` here, and only what gains even so is served.
 // defer = 1: they are left in `partial`, *splits gets their number, and the caller sees to the

@@ -5,9 +5,9 @@
 // (Ops::tune) and resets them afterwards.
 //
 // libti_gemm_bf16:
-//   force_tile           1: 256 x 128, 2: 128 x 128, 3 / 4: 128 x 64 (4: not SwiGLU), 5 / 7: 64 x 128 (SwiGLU only), 6: 64 x 64, 8: 128 x 160,
-//                        9: 256 x 160 (6, 8, 9: not SwiGLU), 10: 256 x 256 (SwiGLU only), 11: 256 x 128 by four wavefronts (not
-//                        SwiGLU); 0: by the shape
+//   force_tile           1: 256 x 128, 2: 128 x 128; not for SwiGLU 3 / 4: 128 x 64, 6: 64 x 64, 8: 128 x 160, 9: 256 x 160,
+//                        11: 256 x 128 by four wavefronts; for SwiGLU alone 5 / 7: 64 x 128, 10: 256 x 256 (another's number:
+//                        128 x 128 for SwiGLU, 128 x 64 for the others); 0: by the shape
 //   normed_weight_below  weights of fewer elements keep the norm inside the product (0: the default)
 //   tiles_160            0: no tiles of 160 columns
 //   tiles_256            0: no tiles of 256 x 256
@@ -39,6 +39,11 @@ extern "C" {
 #endif
 int ti_tuning_set(const char* name, long value);     // 0, or 1 for a name the library does not know
 void ti_tuning_reset();                              // every choice back to the library's own
+// libti_gemm_bf16: what is chosen for M rows times N output columns.  The tile (by its number above) and, where the columns are
+// split between two (n_big > 0), the second one from column n_big on; the rows of the q/k/v product's tile (0: left to the
+// product and the preparation kernel), 256 and 128 where n_big > 0.
+int ti_gemm_bf16_tile_choice(int swiglu, int M, int N, int K, int* rest, int* n_big);
+int ti_gemm_bf16_qkv_choice(int M, int N, int K, int* n_big);
 #ifdef __cplusplus
 }
 #endif
