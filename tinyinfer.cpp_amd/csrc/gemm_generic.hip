@@ -123,8 +123,9 @@ static int launch(const void* A, const void* W, void* out, int M, int N, int K, 
 // Few tokens: the weights' bytes bound it, each is read once, and eight runs keep eight wavefronts loading per tile.
 // Many: a 16x16x4 lasts 32 cycles, so 32-bit products are bound by the matrix cores' 157 TFLOP/s long before L1 or
 // LDS; operands need no staging, and what counts is that the tiles fill whole rounds of the compute units.
-// Measured beside the generic kernel, us at 300 tokens: 4096 x 1024 36.7 (157), [gate; up] 6144 x 1024 47.9 (273),
-// 151936 x 1024 1046 (2984); a prompt of 300 tokens of Qwen3-0.6B's sizes spends 5.3 ms in its products (31.5).
+// Measured inside a prompt of 300 tokens of Qwen3-0.6B's sizes, us (the generic kernel): 4096 x 1024 37.1 (157), [gate; up]
+// 6144 x 1024 47.8 (273), 1024 x 2048 and 1024 x 3072 29.4 on average (294), 151936 x 1024 1,055 (2,984); its products
+// together 5.1 ms (31.5).
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gf4;
 #define GF_RUNS 8
 
@@ -258,6 +259,17 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
   }
 }
 
+static int compute_units() {
+  static int n = 0;
+  if (!n) {
+    int dev = 0;
+    hipDeviceProp_t prop;
+    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess) n = prop.multiProcessorCount;
+    if (n <= 0) n = 256;
+  }
+  return n;
+}
+
 // The tile: of those that are built, the one whose rounds of the compute units take the least time in all.  A round costs a
 // start, its products (RB NB) and its operands' loads (RB + NB, four times a product's weight each: sixteen lines a load).
 // Fitted to 1 to 1,000 rows times the weights of Qwen3-0.6B's sizes: the tile it picks is on average 0.9 % slower than the
@@ -276,7 +288,7 @@ static int launch_f32(const float* A, const float* W, float* out, int M, int N, 
   long best = -1;
   for (const auto& t : TILES) {
     if (sw && t[0] * t[1] > 8) continue;           // two planes of it would not fit in LDS
-    const long cost = f32_tile_cost(t[0], t[1], sw, M, N, 256);
+    const long cost = f32_tile_cost(t[0], t[1], sw, M, N, compute_units());
     if (best < 0 || cost < best) {
       best = cost;
       rb = t[0];
