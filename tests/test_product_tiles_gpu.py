@@ -1,5 +1,6 @@
 """The pipelined product's tiles beyond the ones tests of the whole dispatch name, loops shorter than the ring of stages,
-the dies' blocks of tiles, and the q/k/v product in tiles of 64 rows."""
+the dies' blocks of tiles, split sums and the norm behind them, the q/k/v product in tiles of 64 rows, and what large weights
+under few rows and very long rows take."""
 import ctypes
 
 import pytest
