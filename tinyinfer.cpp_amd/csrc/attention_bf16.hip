@@ -62,9 +62,10 @@ struct PagedKV {
 // v_mfma_f32_16x16x32_bf16 over both blocks at once.
 template <int HD>
 struct KVPair {
-  Frag8 k[2][HD / 32];   // K:   row lane % 16, dims 32 s + 8 (lane / 16) .. + 7
-  Frag8 v[HD / 16];      // V^T: row (dim) 16 d + lane % 16; elements 0..3: keys 4 (lane / 16) .. + 3 of
-                         //      block A, elements 4..7: the same keys of block B
+  // Of the pair's 32 keys (block A's, then block B's) a lane's eight scores are those of keys 8 (lane / 16) .. + 7, so that the
+  // values they weigh lie in one run of 16 bytes: half as many loads as with four keys of either block.
+  Frag8 k[2][HD / 32];   // K:   k[j]: key 8 (row / 4) + row % 4 + 4 j of the pair, row = lane % 16; dims 32 s + 8 (lane / 16) .. + 7
+  Frag8 v[HD / 16];      // V^T: row (dim) 16 d + lane % 16; keys 8 (lane / 16) .. + 7
 };
 
 // Issue the loads of a pair.  They are unconditional (the caller passes pages that
@@ -75,28 +76,29 @@ __device__ __forceinline__ void load_pair(const PagedKV& kv, int pageA, int keyA
                                           KVPair<HD>& f) {
   const int lane = threadIdx.x & 63;
   const int r16 = lane & 15, quad = lane >> 4;
-  // where a block's keys and values start is the same in every lane (scalar registers); a lane
-  // adds one offset of its own, and the steps are constants in the load instructions
-  const size_t page_elems = (size_t)2 * kv.n_kv * kv.P * HD;
-  const int rowA = keyA % kv.P, rowB = keyB % kv.P;
-  const bf16_t* ka = kv.pool + (size_t)pageA * page_elems + (size_t)kv.kvh * kv.P * HD + (size_t)rowA * HD;
-  const bf16_t* kb = kv.pool + (size_t)pageB * page_elems + (size_t)kv.kvh * kv.P * HD + (size_t)rowB * HD;
-  const bf16_t* va = kv.pool + (size_t)pageA * page_elems + (size_t)(kv.n_kv + kv.kvh) * kv.P * HD + rowA;
-  const bf16_t* vb = kv.pool + (size_t)pageB * page_elems + (size_t)(kv.n_kv + kv.kvh) * kv.P * HD + rowB;
-  const unsigned k_lane = (unsigned)(r16 * HD + quad * 8);          // elements
-  const unsigned v_lane = (unsigned)(r16 * kv.P + quad * 4);
+  // where a block's keys and values start is the same in every lane (scalar registers)
+  const size_t page_elems = (size_t)2 * kv.n_kv * kv.P * HD, head_elems = (size_t)kv.P * HD;
+  const bf16_t* ka = kv.pool + (size_t)pageA * page_elems + kv.kvh * head_elems;
+  const bf16_t* kb = kv.pool + (size_t)pageB * page_elems + kv.kvh * head_elems;
+  const bf16_t* va = ka + kv.n_kv * head_elems;
+  const bf16_t* vb = kb + kv.n_kv * head_elems;
+  if (kv.P != 16) {      // blocks that start inside their page
+    const int rowA = keyA % kv.P, rowB = keyB % kv.P;
+    ka += (size_t)rowA * HD;
+    kb += (size_t)rowB * HD;
+    va += rowA;
+    vb += rowB;
+  }
+  const bf16_t* k = (r16 < 8 ? ka : kb) + (((r16 >> 2) & 1) * 8 + (r16 & 3)) * HD + quad * 8;
+  const bf16_t* v = (quad < 2 ? va : vb) + r16 * kv.P + (quad & 1) * 8;
 #pragma unroll
   for (int s = 0; s < HD / 32; ++s) {
-    f.k[0][s].u = *reinterpret_cast<const uint4*>(ka + k_lane + s * 32);
-    f.k[1][s].u = *reinterpret_cast<const uint4*>(kb + k_lane + s * 32);
+    f.k[0][s].u = *reinterpret_cast<const uint4*>(k + s * 32);
+    f.k[1][s].u = *reinterpret_cast<const uint4*>(k + 4 * HD + s * 32);
   }
   const unsigned v_step = 16u * kv.P;                                // elements between blocks of 16 dims
 #pragma unroll
-  for (int d = 0; d < HD / 16; ++d) {
-    const uint2 a = *reinterpret_cast<const uint2*>(va + v_lane + d * v_step);
-    const uint2 b = *reinterpret_cast<const uint2*>(vb + v_lane + d * v_step);
-    f.v[d].u = make_uint4(a.x, a.y, b.x, b.y);
-  }
+  for (int d = 0; d < HD / 16; ++d) f.v[d].u = *reinterpret_cast<const uint4*>(v + d * v_step);
 }
 
 // What the walk knows of one block.
@@ -141,40 +143,44 @@ __device__ __forceinline__ void attend_pair(KVPair<HD>& f, const Frag8* qf, Bloc
       sb[i] = tanh_fast(sb[i] * r) * back;
     }
   }
-  // this lane: keys key0 + 4 quad + i of column lane % 16, in each block
+  // this lane: eight keys in a row of one block
   float sv[8];
   const bool plain = A.valid && B.valid && !A.check && !B.check;   // the same in every lane
-  if (plain) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      sv[i] = sa[i] * scale;
-      sv[4 + i] = sb[i] * scale;
-    }
-  } else {
+  for (int i = 0; i < 4; ++i) {
+    sv[i] = sa[i] * scale;
+    sv[4 + i] = sb[i] * scale;
+  }
+  if (!plain) {
+    const int key0 = (quad < 2 ? A.key0 : B.key0) + (quad & 1) * 8;
+    const bool valid = quad < 2 ? A.valid : B.valid, check = quad < 2 ? A.check : B.check;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ka = A.key0 + quad * 4 + i, kb = B.key0 + quad * 4 + i;
-      const bool see_a = A.valid & (!A.check | ((ka >= lo) & (ka <= hi)));   // bitwise: selects, no branches
-      const bool see_b = B.valid & (!B.check | ((kb >= lo) & (kb <= hi)));
-      sv[i] = see_a ? sa[i] * scale : -INFINITY;
-      sv[4 + i] = see_b ? sb[i] * scale : -INFINITY;
-      // rows never written may hold anything, NaN included, and 0 * NaN is NaN
-      const bool zero_a = !A.valid | (ka > kv_last), zero_b = !B.valid | (kb > kv_last);
-      const unsigned keep_a = zero_a ? ((i & 1) ? 0x0000FFFFu : 0xFFFF0000u) : 0xFFFFFFFFu;
-      const unsigned keep_b = zero_b ? ((i & 1) ? 0x0000FFFFu : 0xFFFF0000u) : 0xFFFFFFFFu;
+    for (int w = 0; w < 4; ++w) {
+      unsigned keep = 0xFFFFFFFFu;
 #pragma unroll
-      for (int d = 0; d < HD / 16; ++d) {
-        unsigned* wv = reinterpret_cast<unsigned*>(&f.v[d].u);
-        wv[i >> 1] &= keep_a;             // element i of block A
-        wv[2 + (i >> 1)] &= keep_b;       // element 4 + i: block B
+      for (int i = 2 * w; i < 2 * w + 2; ++i) {
+        const int key = key0 + i;
+        const bool see = valid & (!check | ((key >= lo) & (key <= hi)));   // bitwise: selects, no branches
+        sv[i] = see ? sv[i] : -INFINITY;
+        // rows never written may hold anything, NaN included, and 0 * NaN is NaN
+        const bool zero = !valid | (key > kv_last);
+        keep &= zero ? ((i & 1) ? 0x0000FFFFu : 0xFFFF0000u) : 0xFFFFFFFFu;
       }
+#pragma unroll
+      for (int d = 0; d < HD / 16; ++d) reinterpret_cast<unsigned*>(&f.v[d].u)[w] &= keep;
     }
   }
   float bm = sv[0];
 #pragma unroll
   for (int i = 1; i < 8; ++i) bm = fmaxf(bm, sv[i]);
-  bm = fmaxf(bm, __shfl_xor(bm, 16, 64));
-  bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+  {
+    const LanePair p = lane_pair<32>(bm);
+    bm = fmaxf(p.a, p.b);
+  }
+  {
+    const LanePair p = lane_pair<16>(bm);
+    bm = fmaxf(p.a, p.b);
+  }
   const float m_new = fmaxf(m, bm);
   const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
   Frag8 pf;
@@ -205,7 +211,7 @@ __device__ __forceinline__ void attend_pair(KVPair<HD>& f, const Frag8* qf, Bloc
 // Walk blocks first, first + stride, ... (n of them) of one request, two at a time.
 // The page ids of 64 blocks are fetched at once, one per lane, so that the walk waits
 // for the block table once per 1024 positions and not once per block; within such a
-// run the loads of the next pair are in flight while a pair is computed (two fragment
+// run the loads of the next pairs are in flight while a pair is computed (two fragment
 // sets take turns; loads past the end repeat the last block and are not used).
 // `check(block)` tells whether a block needs masks.
 struct NoHook {
@@ -213,21 +219,30 @@ struct NoHook {
 };
 
 // `after_table` runs once, right after the first load of page ids has been issued, and
-// `before_attend` once, after the loads of the first pair have been issued and before the
-// first pair is computed (both also when there is no block to walk; every wavefront of a
+// `before_attend` once, after the loads of the first pair have been issued, `after_second` once, after those of
+// the second, and before the first pair is computed (all also when there is no block to walk; every wavefront of a
 // workgroup runs each exactly once, so they may hold a barrier).  Loads come back in the
 // order they were issued: what a caller asks for in `after_table` arrives before the keys
 // and values, and what it computes in `before_attend` runs while those are in flight.
-template <int HD, typename Check, typename AfterTable = NoHook, typename BeforeAttend = NoHook>
+// `held`: how many lanes already have the page id of their first block (`held_id`; the others and later
+// blocks ask the table); FIRST4: `first4` holds the ids of the first four blocks as well, in scalar registers,
+// so that the first loads do not wait for the lanes'.
+template <int HD, bool FIRST4 = false, typename Check, typename AfterTable = NoHook, typename BeforeAttend = NoHook,
+          typename AfterSecond = NoHook>
 __device__ __forceinline__ void walk_blocks(const PagedKV& kv, const Frag8* qf, int first, int stride, int n,
                                             int lo, int hi, int kv_last, float scale, Check check, float& m,
                                             float& l, floatx4* o, AfterTable after_table = NoHook{},
-                                            BeforeAttend before_attend = NoHook{}, float cap2 = 0.f) {
+                                            BeforeAttend before_attend = NoHook{}, float cap2 = 0.f, int held = 0,
+                                            int held_id = -1, const int* first4 = nullptr,
+                                            AfterSecond after_second = NoHook{}) {
   const int lane = threadIdx.x & 63;
+  constexpr int ASK = -0x7fffffff;
   bool hooks_due = true;
-  for (int c0 = 0; c0 < n; c0 += 64) {
-    const int nc = min(64, n - c0);
-    const int mine = (lane < nc) ? kv.table[((first + (c0 + lane) * stride) * 16) / kv.P] : -1;
+  for (int c0 = 0; c0 == 0 || c0 < n; c0 += 64) {      // (once at least: the hooks)
+    const int nc = max(0, min(64, n - c0));
+    const int have = c0 == 0 ? held : 0;
+    int mine = lane < min(nc, have) ? held_id : -1;
+    if (nc > have && lane >= have && lane < nc) mine = kv.table[((first + (c0 + lane) * stride) * 16) / kv.P];
     if (hooks_due) {
       __builtin_amdgcn_sched_barrier(0);
       after_table();
@@ -237,34 +252,38 @@ __device__ __forceinline__ void walk_blocks(const PagedKV& kv, const Frag8* qf, 
     BlockInfo a0, b0, a1, b1;
     // block j of this run, clamped to the run's last block
     auto info = [&](int j, int& page) {
-      const int jc = min(j, nc - 1);
+      const int jc = max(0, min(j, nc - 1));
       const int blk = first + (c0 + jc) * stride;
-      page = __builtin_amdgcn_readlane(mine, jc);
+      if (page == ASK) page = __builtin_amdgcn_readlane(mine, jc);
       return BlockInfo{blk * 16, j < nc && page >= 0, check(blk)};
     };
-    auto issue = [&](int j, KVPair<HD>& f, BlockInfo& A, BlockInfo& B) {
-      int pa, pb;
+    auto issue = [&](int j, KVPair<HD>& f, BlockInfo& A, BlockInfo& B, int pa = ASK, int pb = ASK) {
       A = info(j, pa);
       B = info(j + 1, pb);
       load_pair<HD>(kv, max(pa, 0), A.key0, max(pb, 0), B.key0, f);
     };
-    issue(0, f0, a0, b0);
+    const bool given = FIRST4 && c0 == 0;
+    if (given) issue(0, f0, a0, b0, first4[0], first4[1]);
+    else issue(0, f0, a0, b0);
     if (hooks_due) {
       __builtin_amdgcn_sched_barrier(0);
       before_attend();
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if (given) issue(2, f1, a1, b1, first4[2], first4[3]);
+    else issue(2, f1, a1, b1);
+    if (hooks_due) {
+      __builtin_amdgcn_sched_barrier(0);
+      after_second();
       hooks_due = false;
     }
     for (int i = 0; i < nc; i += 4) {
-      issue(i + 2, f1, a1, b1);
       attend_pair<HD>(f0, qf, a0, b0, lo, hi, kv_last, scale, m, l, o, cap2);
+      if (i + 2 >= nc) break;
       issue(i + 4, f0, a0, b0);
-      if (i + 2 < nc) attend_pair<HD>(f1, qf, a1, b1, lo, hi, kv_last, scale, m, l, o, cap2);
+      attend_pair<HD>(f1, qf, a1, b1, lo, hi, kv_last, scale, m, l, o, cap2);
+      issue(i + 6, f1, a1, b1);
     }
-  }
-  if (hooks_due) {
-    after_table();
-    before_attend();
   }
 }
 
@@ -284,96 +303,47 @@ struct QKPrep {
   bf16_t* pool_w;            // the cache to write the new key and value into; nullptr: nothing is written
 };
 
+// One head of the row by one wavefront, in two steps, so that the loads of keys and values can go out between them: lane i
+// holds pair i.  The arithmetic is qk_head_wave's (the same bits); w null: a value head, rounded alone.
 template <int HD>
-struct QueryLoads {
-  static_assert(HD == 64 || HD == 128, "a lane holds whole rotation pairs for these head sizes only");
-  static constexpr int NS = HD / 32, NP = NS / 2, HALF = HD / 2;
-  float x[NS][8];
-  float wl[NP][8], wh[NP][8];
-  float2 cs[NP][8];
+struct HeadJob {
+  static_assert(HD == 64 || HD == 128, "a lane holds one rotation pair at most");
+  static constexpr int HALF = HD / 2;
+  float lo, hi, wl, wh;
+  float2 cs;
   bool from_table;
-
-  // everything the preparation reads, asked for in one go (the table case and the computed case
-  // of the angles are told apart once, not per element, so that the loads go out together)
-  __device__ __forceinline__ void load(const QKPrep& pr, const float* __restrict__ src, int p) {
-    const int lane = threadIdx.x & 63, quad = lane >> 4;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const float4 a = *reinterpret_cast<const float4*>(src + s * 32 + quad * 8);
-      const float4 b = *reinterpret_cast<const float4*>(src + s * 32 + quad * 8 + 4);
-      x[s][0] = a.x; x[s][1] = a.y; x[s][2] = a.z; x[s][3] = a.w;
-      x[s][4] = b.x; x[s][5] = b.y; x[s][6] = b.z; x[s][7] = b.w;
+  __device__ __forceinline__ void load(const QKPrep& pr, const float* __restrict__ src, const float* __restrict__ w, int p) {
+    const int i = (threadIdx.x & 63) & (HALF - 1);
+    lo = src[i];
+    hi = src[i + HALF];
+    wl = wh = 1.f;
+    if (w) {
+      wl = w[i];
+      wh = w[i + HALF];
     }
     from_table = pr.inv_freq && pr.rope_table && p < pr.table_len;   // the same in every lane
-#pragma unroll
-    for (int sp = 0; sp < NP; ++sp) {
-      const int i0 = sp * 32 + quad * 8;
-      if (pr.q_w) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const float4 a = *reinterpret_cast<const float4*>(pr.q_w + i0 + 4 * h);
-          const float4 b = *reinterpret_cast<const float4*>(pr.q_w + i0 + HALF + 4 * h);
-          wl[sp][4 * h] = a.x; wl[sp][4 * h + 1] = a.y; wl[sp][4 * h + 2] = a.z; wl[sp][4 * h + 3] = a.w;
-          wh[sp][4 * h] = b.x; wh[sp][4 * h + 1] = b.y; wh[sp][4 * h + 2] = b.z; wh[sp][4 * h + 3] = b.w;
-        }
-      }
-      if (from_table) {
-        const float4* t = reinterpret_cast<const float4*>(pr.rope_table + (size_t)p * HALF + i0);
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const float4 v = t[h];
-          cs[sp][2 * h] = make_float2(v.x, v.y);
-          cs[sp][2 * h + 1] = make_float2(v.z, v.w);
-        }
-      }
-    }
+    if (from_table) cs = pr.rope_table[(size_t)p * HALF + i];
   }
-
-  // Q^T fragments of this lane's column (one q head): the same arithmetic as qk_head_wave, in
-  // the layout of the first product.  A lane holds the dims 32 s + 8 quad + j (s < HD / 32,
-  // j < 8), which are both halves of its rotation pairs; the sum of squares goes up the same
-  // tree as the butterfly of a wavefront with one pair per lane.
-  __device__ __forceinline__ void finish(const QKPrep& pr, int p, bool valid, Frag8* qf) {
-    const int lane = threadIdx.x & 63, quad = lane >> 4;
-    float scale = 1.f;
-    if (pr.q_w) {
-      float u[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        u[j] = qk_pair_square(x[0][j], x[NP][j]);
-        if (NP == 2) u[j] += qk_pair_square(x[1][j], x[1 + NP][j]);   // pairs i and i + 32
+  // `dst`: HD consecutive elements
+  __device__ __forceinline__ void finish(const QKPrep& pr, const float* w, bool value, int p, bf16_t* dst) {
+    const int lane = threadIdx.x & 63;
+    float a = lo, b = hi;
+    if (!value) {
+      if (w) {
+        const float scale = qk_norm_scale(group_sum<TI_WAVE>(lane < HALF ? qk_pair_square(lo, hi) : 0.f), HD, pr.eps);
+        a *= scale;
+        b *= scale;
+        a *= wl;
+        b *= wh;
       }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) u[j] += __shfl_xor(u[j], 32, 64);   // pairs i and i ^ 16
-#pragma unroll
-      for (int j = 0; j < 8; ++j) u[j] += __shfl_xor(u[j], 16, 64);   // i ^ 8
-#pragma unroll
-      for (int j = 0; j < 4; ++j) u[j] += u[j + 4];                   // i ^ 4
-      u[0] += u[2];                                                   // i ^ 2
-      u[1] += u[3];
-      scale = qk_norm_scale(u[0] + u[1], HD, pr.eps);                 // i ^ 1
-    }
-    if (pr.inv_freq && !from_table) {
-#pragma unroll
-      for (int sp = 0; sp < NP; ++sp)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) cs[sp][j] = qk_cos_sin(sp * 32 + quad * 8 + j, HALF, p, pr.inv_freq, nullptr, 0);
-    }
-#pragma unroll
-    for (int sp = 0; sp < NP; ++sp) {
-      bf16_t* lo_h = reinterpret_cast<bf16_t*>(&qf[sp].u);
-      bf16_t* hi_h = reinterpret_cast<bf16_t*>(&qf[sp + NP].u);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float lo = x[sp][j] * scale, hi = x[sp + NP][j] * scale;
-        if (pr.q_w) {
-          lo *= wl[sp][j];
-          hi *= wh[sp][j];
-        }
-        if (pr.inv_freq) qk_rotate(lo, hi, cs[sp][j]);
-        lo_h[j] = f2bf(valid ? lo : 0.f);
-        hi_h[j] = f2bf(valid ? hi : 0.f);
+      if (pr.inv_freq) {
+        if (!from_table) cs = qk_cos_sin(lane & (HALF - 1), HALF, p, pr.inv_freq, nullptr, 0);
+        qk_rotate(a, b, cs);
       }
+    }
+    if (lane < HALF) {
+      dst[lane] = f2bf(a);
+      dst[lane + HALF] = f2bf(b);
     }
   }
 };
@@ -381,12 +351,10 @@ struct QueryLoads {
 // =================================================================== decode
 // grid (rows, n_kv * head_parts, splits), 256 threads.  Partials (splits > 1):
 //   part_o [row][head][split][hd], part_ml [row][head][split][2] = (max, sum)
-// PREP: the queries come from the 32-bit projections (see QKPrep); needs parts == 1.
-// SHARED (with PREP): the four wavefronts need the same query; one prepares it, after the
-// first keys and values have been asked for by all four, and hands it over through LDS.  The
-// others' load units are then free for keys and values from the start, and the preparation
-// runs while those are on their way.  It costs registers (one wavefront per SIMD): for launches
-// of at most one workgroup per compute unit, where the start of the kernel is most of its time.
+// PREP: the queries come from the 32-bit projections (see QKPrep); needs parts == 1.  The row's query heads, and its own
+// key and value where a workgroup walks their block, are prepared a head a wavefront and shared through LDS while the first
+// keys and values are on their way.  (A lane that prepared its column's head by itself asked for 64 to 112 bytes in 28 loads
+// in front of its keys, and kept 100 registers for them: 8 requests of 2,048 tokens at 0.6B 21.8 us a layer, now FIG1.)
 // A learned sink in the softmax's denominator: exp(sink[head]) joins the sum where a column is finished (no key, no value,
 // not scaled).  m, lt: the column's maximum (in units of log 2) and the sum of its weights; lt becomes the new denominator
 // and the factor on the column's unscaled outputs comes back.  sink null: nothing changes.
@@ -400,23 +368,57 @@ __device__ __forceinline__ float sink_join(const float* __restrict__ sink, int h
 }
 
 #define DEC_TABLE_LDS 1024     // entries of a block-table row that the decode kernel can hold in LDS
-template <int HD, bool PREP, bool SHARED = false>
-__global__ void __launch_bounds__(256)
-attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool, const int* __restrict__ table,
-                   int table_stride, const int* __restrict__ pos, const int* __restrict__ slot,
-                   const int* __restrict__ rows, bf16_t* __restrict__ out, float* __restrict__ part_o,
-                   float* __restrict__ part_ml, int n_head, int n_kv, int P, float scale, int window,
-                   int n_splits, QKPrep prep, float softcap = 0.f, const float* __restrict__ sink = nullptr) {
-  __shared__ float s_o[4][HD / 16][4][64];
-  __shared__ float s_m[4][16], s_l[4][16];
-  __shared__ __attribute__((aligned(16))) bf16_t s_kv[PREP ? 2 * HD : 2];   // the row's own key, then its value
-  const int ridx = blockIdx.x;
-  const int m_row = rows ? rows[ridx] : ridx;
-  const int G = n_head / n_kv;
-  const int parts = (G + 15) / 16;   // q heads per kv head, in sets of up to 16 columns
-  const int kvh = blockIdx.y / parts, part = blockIdx.y % parts;
-  const int split = blockIdx.z;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+// The workgroup's LDS: what its NW wavefronts leave for the merge, and their maxima and sums.
+template <int HD, int NW>
+struct DecodeMerge {
+  floatx4 o[NW][HD / 16][64];
+  float m[NW][16], l[NW][16];
+};
+// A launch by records (TI_RUN_* in tinyinfer_kernels.h): the host cuts every row's context into runs of its own choice and says what each
+// workgroup walks.  Record i, of a launch's `run_stride` ints: the header below, then for each of the workgroup's
+// NW wavefronts (run_stride - TI_RUN_HEAD) / NW page ids, at least four: those of the first blocks that it walks (-1: given back;
+// beyond the run's end anything).  A workgroup's first loads are then its header and its page ids, side by side, and its
+// keys' are the next.  Runs of no blocks are nobody's:
+// their workgroups end at once (a captured graph launches as many records for every step).
+struct DecodeRuns {
+  const int* runs;      // null: no records, `split` of n_splits equal runs of every row
+  int run_stride;
+};
+// One workgroup of NW wavefronts: row `ridx` of the launch, kv head and set of q heads `y`, run `split` of n_splits; or record `ridx`.
+template <int HD, bool PREP, int NW, bool RUNS>
+__device__ __forceinline__ void
+decode_run(DecodeMerge<HD, NW>& sm, int ridx, int y, int split, const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool,
+           const int* __restrict__ table, int table_stride, const int* __restrict__ pos, const int* __restrict__ slot,
+           const int* __restrict__ rows, bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
+           int n_head, int n_kv, int P, float scale, int window, int n_splits, const QKPrep& prep, float softcap,
+           const float* __restrict__ sink, DecodeRuns by = DecodeRuns{nullptr, 0}, int group = 0) {
+  static_assert(!PREP || NW == 4, "the preparation is written for four wavefronts");
+  auto& s_o = sm.o;
+  auto& s_m = sm.m;
+  auto& s_l = sm.l;
+  // the wavefront's number in scalar registers, and with it what it walks
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int held = RUNS ? (by.run_stride - TI_RUN_HEAD) / NW : 0;      // lanes whose first block's page id comes with the record
+  int held_id = -1, first4[4] = {};
+  int rh[TI_RUN_HEAD] = {};
+  if constexpr (RUNS) {
+    const int* rec = by.runs + (size_t)ridx * by.run_stride;
+    const int* ids = rec + TI_RUN_HEAD + wave * held;
+    if (lane < held) held_id = ids[lane];
+#pragma unroll
+    for (int i = 0; i < TI_RUN_HEAD; ++i) rh[i] = rec[i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) first4[i] = ids[i];
+#pragma unroll
+    for (int i = 0; i < TI_RUN_HEAD; ++i) asm volatile("" : "+s"(rh[i]));      // all of it at once
+#pragma unroll
+    for (int i = 0; i < 4; ++i) asm volatile("" : "+s"(first4[i]));
+    if (rh[TI_RUN_BLOCKS] == 0) return;
+  }
+  const int m_row = RUNS ? rh[TI_RUN_ROW] : rows ? rows[ridx] : ridx;
+  const int G = group ? group : n_head / n_kv;       // (a division in the kernel takes longer than an argument)
+  const int parts = PREP ? 1 : (G + 15) / 16;        // q heads per kv head, in sets of up to 16 columns
+  const int kvh = y / parts, part = y % parts;
   const int r16 = lane & 15, quad = lane >> 4;
   const int n_cols = min(16, G - part * 16);
   const int head = kvh * G + part * 16 + r16;   // valid if r16 < n_cols
@@ -426,8 +428,10 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool
   // for at once, all of them, beside the position instead of behind it (which pages the workgroup walks
   // depends on the position), and looked up in LDS afterwards: one round trip to memory less before the
   // first keys can be asked for (0.15 us of the kernel's 19 at batch 8 of Qwen3-0.6B's sizes).
-  __shared__ int s_table[DEC_TABLE_LDS];
-  const bool early = slot == nullptr;
+  constexpr bool CAN_EARLY = NW == 4 && !RUNS;
+  constexpr int EARLY = CAN_EARLY ? DEC_TABLE_LDS : 1;
+  __shared__ int s_table[EARLY];
+  const bool early = CAN_EARLY && slot == nullptr;
   int ids[DEC_TABLE_LDS / 256];
   if (early) {
     const int* table_row = table + (size_t)m_row * table_stride;
@@ -437,87 +441,95 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool
       ids[j] = i < table_stride ? table_row[i] : -1;
     }
   }
-  const int p_q = pos[m_row];
+  const int p_q = RUNS ? rh[TI_RUN_POS] : pos[m_row];
   const int lo = (window > 0 && p_q - window + 1 > 0) ? p_q - window + 1 : 0;
   const int blk_lo = lo / 16, blk_hi = p_q / 16;
   const int n_blk = blk_hi - blk_lo + 1;
   const int per = (n_blk + n_splits - 1) / n_splits;
-  const int b0 = blk_lo + split * per;
-  const int b1 = min(blk_hi + 1, b0 + per);
+  const int b0 = RUNS ? rh[TI_RUN_FIRST] : blk_lo + split * per;
+  const int b1 = RUNS ? b0 + rh[TI_RUN_BLOCKS] : min(blk_hi + 1, b0 + per);
+  // where the results go: straight out, or to place part_at + part_step * head of the partial results
+  const bool whole = RUNS ? rh[TI_RUN_PART] < 0 : n_splits == 1;
+  const size_t part_at = RUNS ? (size_t)rh[TI_RUN_PART] * n_head : (size_t)ridx * n_head * n_splits + split;
+  const int part_step = RUNS ? 1 : n_splits;
   if (early) {
 #pragma unroll
-    for (int j = 0; j < DEC_TABLE_LDS / 256; ++j) s_table[threadIdx.x + 256 * j] = ids[j];
+    for (int j = 0; j < DEC_TABLE_LDS / 256; ++j)
+      if constexpr (CAN_EARLY) s_table[threadIdx.x + 256 * j] = ids[j];
     __syncthreads();
   }
 
-  PagedKV kv{pool, early ? s_table : table + (size_t)slot[m_row] * table_stride, P, n_kv, kvh};
+  PagedKV kv{pool, early ? s_table : table + (size_t)(RUNS ? rh[TI_RUN_TABLE_ROW] : slot[m_row]) * table_stride, P, n_kv, kvh};
   Frag8 qf[HD / 32];
   float mx = -INFINITY, l = 0.f;
   floatx4 o[HD / 16];
 #pragma unroll
   for (int d = 0; d < HD / 16; ++d) o[d] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const int mine = (b1 - (b0 + wave) + 3) / 4;   // blocks b0 + wave, + 4, ... below b1
-  auto edge = [=](int b) { return b == blk_lo || b == blk_hi; };
-  bool own_key = false;   // PREP: this workgroup takes the row's own key and value from LDS, not from the cache
+  const int mine = (b1 - (b0 + wave) + NW - 1) / NW;   // blocks b0 + wave, + NW, ... below b1
+  auto edge = [=](int b) { return (lo > 0 && b == blk_lo) || b == blk_hi; };
   if constexpr (PREP) {
+    __shared__ __attribute__((aligned(16))) bf16_t s_q[16][HD];       // the query heads
+    __shared__ __attribute__((aligned(16))) bf16_t s_kv[2][HD];       // the row's own key, then its value
     const float* row = prep.qkv + (size_t)m_row * prep.row_width;
-    own_key = prep.pool_w && blk_hi >= b0 && blk_hi < b1;
+    // The workgroup that walks the block of the row's own position prepares the position's key and value as well: from LDS
+    // they go into the cache for later steps, and into this step's attention as a block of their own, so nothing waits for
+    // the cache to hold them.
+    const bool own_key = prep.pool_w && blk_hi >= b0 && blk_hi < b1;
     const int last = own_key ? p_q - 1 : p_q;      // what the cache holds for this workgroup
-    const float* q_src = row + (size_t)(r16 < n_cols ? head : kvh * G) * HD;
-    // this workgroup walks the block of the row's own position: the position's key and value
-    // are computed here (by the code that prepares whole steps) into LDS; from there they go
-    // into the cache for later steps, and into this step's attention as a block of their own,
-    // so nothing waits for the cache to hold them.
-    auto own_key_to_lds = [&]() {
-      if (wave == (SHARED ? 1 : 0))
-        qk_head_wave<bf16_t>(row + (size_t)(n_head + kvh) * HD, s_kv, 1, prep.k_w, prep.eps, prep.inv_freq,
-                             prep.rope_table, prep.table_len, p_q, HD);
-      if (wave == (SHARED ? 2 : 1)) v_head_wave<bf16_t>(row + (size_t)(n_head + n_kv + kvh) * HD, s_kv + HD, 1, HD);
+    const int n_jobs = n_cols + (own_key ? 2 : 0);
+    HeadJob<HD> job;
+    auto job_load = [&](int j) {
+      const int h = j < n_cols ? kvh * G + j : j == n_cols ? n_head + kvh : n_head + n_kv + kvh;
+      job.load(prep, row + (size_t)h * HD, j < n_cols ? prep.q_w : j == n_cols ? prep.k_w : nullptr, p_q);
     };
-    auto own_key_to_cache = [&]() {          // after a barrier
-      const int page = kv.table[p_q / P];
-      if (page >= 0) {    // the host reserves pages first; never write astray
-        bf16_t* kd = kv_page_slot<bf16_t>(prep.pool_w, page, 0, kvh, p_q % P, n_kv, P, HD);
-        bf16_t* vd = kv_page_slot<bf16_t>(prep.pool_w, page, 1, kvh, p_q % P, n_kv, P, HD);
-        for (int i = threadIdx.x; i < HD; i += 256) {
-          kd[i] = s_kv[i];
-          vd[(size_t)i * P] = s_kv[HD + i];
-        }
-      }
+    auto job_finish = [&](int j) {
+      job.finish(prep, j < n_cols ? prep.q_w : prep.k_w, j > n_cols, p_q, j < n_cols ? s_q[j] : s_kv[j - n_cols]);
     };
-    if constexpr (SHARED) {
-      __shared__ uint4 s_q[HD / 32][64];
-      QueryLoads<HD> ql;
-      walk_blocks<HD>(
-          kv, qf, b0 + wave, 4, mine, lo, last, last, scale * TI_LOG2E, edge, mx, l, o,
-          [&]() {
-            if (wave == 0) ql.load(prep, q_src, p_q);   // the same for every lane of the wavefront
-          },
-          [&]() {
-            if (own_key) own_key_to_lds();
-            if (wave == 0) {
-              ql.finish(prep, p_q, r16 < n_cols, qf);
+    walk_blocks<HD, RUNS>(
+        kv, qf, b0 + wave, NW, mine, lo, last, last, scale * TI_LOG2E, edge, mx, l, o,
+        [&]() {
+          if (wave < n_jobs) job_load(wave);
+        },
+        [&]() {
+          for (int j = wave; j < n_jobs; j += NW) {
+            if (j != wave) job_load(j);
+            job_finish(j);
+          }
+          __syncthreads();
 #pragma unroll
-              for (int s = 0; s < HD / 32; ++s) s_q[s][lane] = qf[s].u;
-            }
-            __syncthreads();
-            if (wave != 0) {
+          for (int s = 0; s < HD / 32; ++s)
+            qf[s].u = r16 < n_cols ? *reinterpret_cast<const uint4*>(&s_q[r16][s * 32 + quad * 8]) : make_uint4(0, 0, 0, 0);
+        },
+        0.f, held, held_id, first4,
+        [&]() {
+          if (!own_key) return;
+          if (wave == 0) {
+            // the row's own key and value come first: their score is the maximum, their weight 1
+            floatx4 sc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-              for (int s = 0; s < HD / 32; ++s) qf[s].u = s_q[s][lane];
+            for (int s = 0; s < HD / 32; ++s) {
+              Frag8 k;
+              k.u = (r16 == 0) ? *reinterpret_cast<const uint4*>(&s_kv[0][s * 32 + quad * 8]) : make_uint4(0, 0, 0, 0);
+              sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k.v, qf[s].v, sc, 0, 0, 0);
             }
-            if (own_key) own_key_to_cache();
-          });
-    } else {
-      if (own_key) own_key_to_lds();
-      QueryLoads<HD> ql;
-      ql.load(prep, q_src, p_q);
-      ql.finish(prep, p_q, r16 < n_cols, qf);
-      if (own_key) {
-        __syncthreads();
-        own_key_to_cache();
-      }
-      walk_blocks<HD>(kv, qf, b0 + wave, 4, mine, lo, last, last, scale * TI_LOG2E, edge, mx, l, o);
-    }
+            mx = __shfl(sc[0], r16, 64) * (scale * TI_LOG2E);      // row 0 of the tile lies in the first sixteen lanes
+            l = quad == 0 ? 1.f : 0.f;                             // the lanes of a column are added at the end
+#pragma unroll
+            for (int d = 0; d < HD / 16; ++d)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) o[d][i] = bf2f(s_kv[1][d * 16 + quad * 4 + i]);
+          } else if (wave == NW - 1) {
+            const int page = RUNS ? rh[TI_RUN_OWN_PAGE] : kv.table[p_q / P];
+            if (page >= 0) {    // the host reserves pages first; never write astray
+              bf16_t* kd = kv_page_slot<bf16_t>(prep.pool_w, page, 0, kvh, p_q % P, n_kv, P, HD);
+              bf16_t* vd = kv_page_slot<bf16_t>(prep.pool_w, page, 1, kvh, p_q % P, n_kv, P, HD);
+              for (int i = lane; i < HD; i += 64) {
+                kd[i] = s_kv[0][i];
+                vd[(size_t)i * P] = s_kv[1][i];
+              }
+            }
+          }
+        });
   } else {
 #pragma unroll
     for (int s = 0; s < HD / 32; ++s) {
@@ -525,31 +537,15 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool
       if (r16 < n_cols)
         qf[s].u = *reinterpret_cast<const uint4*>(q + ((size_t)m_row * n_head + head) * HD + s * 32 + quad * 8);
     }
-    walk_blocks<HD>(kv, qf, b0 + wave, 4, mine, lo, p_q, p_q, scale * TI_LOG2E, edge, mx, l, o, NoHook{}, NoHook{},
-                    softcap * TI_LOG2E);
-  }
-  if (PREP && own_key && wave == 0) {
-    // the row's own key and value: a block whose first key is the only one that counts
-    KVPair<HD> f;
-#pragma unroll
-    for (int s = 0; s < HD / 32; ++s) {
-      f.k[0][s].u = (r16 == 0) ? *reinterpret_cast<const uint4*>(s_kv + s * 32 + quad * 8) : make_uint4(0, 0, 0, 0);
-      f.k[1][s].u = make_uint4(0, 0, 0, 0);
-    }
-#pragma unroll
-    for (int d = 0; d < HD / 16; ++d)
-      f.v[d].u = make_uint4(quad == 0 ? (unsigned)s_kv[HD + d * 16 + r16] : 0u, 0, 0, 0);
-    attend_pair<HD>(f, qf, BlockInfo{p_q, true, true}, BlockInfo{p_q, false, false}, p_q, p_q, p_q, scale * TI_LOG2E,
-                    mx, l, o);
+    walk_blocks<HD, RUNS>(kv, qf, b0 + wave, NW, mine, lo, p_q, p_q, scale * TI_LOG2E, edge, mx, l, o, NoHook{}, NoHook{},
+                          softcap * TI_LOG2E, held, held_id, first4);
   }
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
 
-  // merge the four wavefronts: lane keeps its (column, dims) in all of them
+  // merge the wavefronts: lane keeps its (column, dims) in all of them
 #pragma unroll
-  for (int d = 0; d < HD / 16; ++d)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s_o[wave][d][i][lane] = o[d][i];
+  for (int d = 0; d < HD / 16; ++d) s_o[wave][d][lane] = o[d];
   if (quad == 0) {
     s_m[wave][r16] = mx;
     s_l[wave][r16] = l;
@@ -557,25 +553,25 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool
   __syncthreads();
   float mm = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) mm = fmaxf(mm, s_m[w][r16]);
-  float wgt[4], lt = 0.f;
+  for (int w = 0; w < NW; ++w) mm = fmaxf(mm, s_m[w][r16]);
+  float wgt[NW], lt = 0.f;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
+  for (int w = 0; w < NW; ++w) {
     wgt[w] = (s_m[w][r16] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(s_m[w][r16] - mm);
     lt += s_l[w][r16] * wgt[w];
   }
   if (r16 >= n_cols) return;
-  // wavefront w finishes dim blocks w, w + 4, ...
-  for (int d = wave; d < HD / 16; d += 4) {
-    float acc[4];
+  // wavefront w finishes dim blocks w, w + NW, ...
+  for (int d = wave; d < HD / 16; d += NW) {
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      acc[i] = 0.f;
+    for (int w = 0; w < NW; ++w) {
+      const floatx4 v = s_o[w][d][lane];
 #pragma unroll
-      for (int w = 0; w < 4; ++w) acc[i] += s_o[w][d][i][lane] * wgt[w];
+      for (int i = 0; i < 4; ++i) acc[i] += v[i] * wgt[w];
     }
     const int dim = d * 16 + quad * 4;
-    if (n_splits == 1) {
+    if (whole) {
       float den = lt;
       const float inv = sink_join(sink, head, mm, den) / den;
       Frag4 r;
@@ -583,33 +579,77 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool
       for (int i = 0; i < 4; ++i) r.h[i] = f2bf(acc[i] * inv);
       *reinterpret_cast<uint2*>(out + ((size_t)m_row * n_head + head) * HD + dim) = r.u;
     } else {
-      float* po = part_o + (((size_t)ridx * n_head + head) * n_splits + split) * HD + dim;
+      float* po = part_o + (part_at + (size_t)part_step * head) * HD + dim;
       *reinterpret_cast<float4*>(po) = make_float4(acc[0], acc[1], acc[2], acc[3]);
     }
   }
-  if (n_splits > 1 && wave == 0 && quad == 0) {
-    float* pm = part_ml + (((size_t)ridx * n_head + head) * n_splits + split) * 2;
+  if (!whole && wave == 0 && quad == 0) {
+    float* pm = part_ml + (part_at + (size_t)part_step * head) * 2;
     pm[0] = mm;
     pm[1] = lt;
   }
+}
+
+template <int HD, bool PREP>
+__global__ void __launch_bounds__(256, 2)
+attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool, const int* __restrict__ table,
+                   int table_stride, const int* __restrict__ pos, const int* __restrict__ slot,
+                   const int* __restrict__ rows, bf16_t* __restrict__ out, float* __restrict__ part_o,
+                   float* __restrict__ part_ml, int n_head, int n_kv, int P, float scale, int window,
+                   int n_splits, QKPrep prep, float softcap = 0.f, const float* __restrict__ sink = nullptr) {
+  __shared__ DecodeMerge<HD, 4> sm;
+  decode_run<HD, PREP, 4, false>(sm, blockIdx.x, blockIdx.y, blockIdx.z, q, pool, table, table_stride, pos, slot, rows,
+                                         out, part_o, part_ml, n_head, n_kv, P, scale, window, n_splits, prep, softcap, sink);
+}
+
+// The same from the projections, by records: grid (n_kv, records).  A launch's workgroups differ by what the host gave them:
+// with every row in as many runs a launch lasted as long as the longest row asks.
+// (The arguments that the first loads need come first: they arrive in scalar registers with the wavefront.)
+template <int HD>
+__global__ void __launch_bounds__(256, 2)
+attn_decode_runs_kernel(const int* __restrict__ runs, int run_stride, int group, const float* __restrict__ qkv, int row_width,
+                        int n_kv, const float* __restrict__ q_w, const float* __restrict__ k_w,
+                        const float2* __restrict__ rope_table, const bf16_t* __restrict__ pool, const int* __restrict__ table,
+                        int table_stride, int P, const float* __restrict__ inv_freq, int table_len, float eps,
+                        bf16_t* __restrict__ pool_w, bf16_t* __restrict__ out, float* __restrict__ part_o,
+                        float* __restrict__ part_ml, float scale, int window) {
+  __shared__ DecodeMerge<HD, 4> sm;
+  const QKPrep prep{qkv, row_width, q_w, k_w, eps, inv_freq, rope_table, table_len, pool_w};
+  decode_run<HD, true, 4, true>(sm, blockIdx.y, blockIdx.x, 0, nullptr, pool, table, table_stride, nullptr, nullptr, nullptr,
+                                out, part_o, part_ml, group * n_kv, n_kv, P, scale, window, 1, prep, 0.f, nullptr,
+                                DecodeRuns{runs, run_stride}, group);
 }
 
 // grid (rows, n_head), max(HD, 64) threads: out = sum_s w_s o_s / sum_s w_s l_s, w_s = 2^(m_s - max m).
 // The partial outputs are fetched in batches of eight independent loads: the kernel waits for
 // memory a few times, not once per split.
 #define MERGE_MAX_SPLITS 64
-template <int HD>
+// RECORDS: `rows` holds (row, first run's place, runs, -) of every row, whose run s lies at [first + s][head]; a row of one
+// run has its result already.
+template <int HD, bool RECORDS = false>
 __global__ void __launch_bounds__(HD < 64 ? 64 : HD)
 attn_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                   const int* __restrict__ rows, bf16_t* __restrict__ out, int n_head, int n_splits,
                   const float* __restrict__ sink = nullptr) {
   const int ridx = blockIdx.x, head = blockIdx.y, d = threadIdx.x;
   if (d >= HD) return;
-  const int m_row = rows ? rows[ridx] : ridx;
-  const float2* pm = reinterpret_cast<const float2*>(part_ml) + ((size_t)ridx * n_head + head) * n_splits;
-  const float* po = part_o + ((size_t)ridx * n_head + head) * n_splits * HD + d;
+  int m_row;
+  size_t at, step;                    // the runs' places: at, at + step, ...
+  if constexpr (RECORDS) {
+    n_splits = rows[4 * ridx + 2];
+    if (n_splits < 2) return;
+    m_row = rows[4 * ridx];
+    at = (size_t)rows[4 * ridx + 1] * n_head + head;
+    step = n_head;
+  } else {
+    m_row = rows ? rows[ridx] : ridx;
+    at = ((size_t)ridx * n_head + head) * n_splits;
+    step = 1;
+  }
+  const float2* pm = reinterpret_cast<const float2*>(part_ml) + at;
+  const float* po = part_o + at * HD + d;
   // every thread works the weights of the splits out for itself: they are few, and no thread waits
-  // for another.  Up to 16 splits: everything asked for at once, one round trip to memory (splits
+  // for another.  Up to 32 splits: everything asked for at once, one round trip to memory (splits
   // beyond the last repeat it and count for nothing).
   auto at_once = [&](auto cap_tag) {
     constexpr int CAP = decltype(cap_tag)::value;
@@ -618,8 +658,8 @@ attn_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ pa
 #pragma unroll
     for (int j = 0; j < CAP; ++j) {
       const int sj = j < n_splits ? j : n_splits - 1;
-      ml[j] = pm[sj];
-      v[j] = po[(size_t)sj * HD];
+      ml[j] = pm[sj * step];
+      v[j] = po[sj * step * HD];
     }
     float mm = -INFINITY;
 #pragma unroll
@@ -644,8 +684,12 @@ attn_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ pa
     at_once(std::integral_constant<int, 16>{});
     return;
   }
+  if (n_splits <= 32) {      // (run by run 17 took 6 us longer than 16)
+    at_once(std::integral_constant<int, 32>{});
+    return;
+  }
   float mm = -INFINITY;
-  for (int s = 0; s < n_splits; ++s) mm = fmaxf(mm, pm[s].x);
+  for (int s = 0; s < n_splits; ++s) mm = fmaxf(mm, pm[s * step].x);
   float acc = 0.f, lt = 0.f;
   int s = 0;
   for (; s + 8 <= n_splits; s += 8) {
@@ -653,8 +697,8 @@ attn_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ pa
     float2 ml[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      v[j] = po[(size_t)(s + j) * HD];
-      ml[j] = pm[s + j];
+      v[j] = po[(s + j) * step * HD];
+      ml[j] = pm[(s + j) * step];
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -664,10 +708,10 @@ attn_merge_kernel(const float* __restrict__ part_o, const float* __restrict__ pa
     }
   }
   for (; s < n_splits; ++s) {
-    const float2 ml = pm[s];
+    const float2 ml = pm[s * step];
     const float w = split_weight(ml.x, mm);
     lt = fmaf(ml.y, w, lt);
-    acc = split_accumulate(acc, po[(size_t)s * HD], w);
+    acc = split_accumulate(acc, po[s * step * HD], w);
   }
   const float f = sink_join(sink, head, mm, lt);
   out[((size_t)m_row * n_head + head) * HD + d] = f2bf(acc * (f / lt));
@@ -808,17 +852,17 @@ __device__ __forceinline__ void unrolled_while(F&& f) {
 // PAIRED: a workgroup takes two tiles, one after the other: tiles[blockIdx.x] and
 // tiles[n_tiles - 1 - blockIdx.x] of a list ordered from the most keys to the fewest, so that
 // under a causal mask every workgroup of a launch has about the same work.
-template <int HD, int NG, int NW = 4, int ST = PF_STAGES, bool PAIRED = false, int CB = 1>
-__global__ void __launch_bounds__(64 * NW * NG)
-attn_prefill_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool,
-                        const int* __restrict__ table, int table_stride, const int* __restrict__ tiles,
-                        int n_tiles, const int* __restrict__ entries, bf16_t* __restrict__ out, int n_head,
-                        int n_kv, int P, float scale, int window, float* __restrict__ part_o = nullptr,
-                        float* __restrict__ part_ml = nullptr, float softcap = 0.f, const float* __restrict__ sink = nullptr) {
-  // gridDim.z > 1: the keys a tile sees are cut into gridDim.z runs of whole turns, workgroup z takes
-  // run z and leaves its maxima, sums and unscaled outputs in part_ml [row][head][z] = (m, l) and
-  // part_o [row][head][z][HD] for the kernel that merges them
-  const int n_splits = gridDim.z, split = blockIdx.z;
+// Workgroup (bx, by) of a grid of gx x n_head.
+//   n_splits > 1: the keys a tile sees are cut into n_splits runs of whole turns, the workgroup takes
+//   run `split` and leaves its maxima, sums and unscaled outputs in part_ml [row][head][split] = (m, l) and
+//   part_o [row][head][split][HD] for the kernel that merges them
+template <int HD, int NG, int NW, int ST, bool PAIRED, int CB>
+__device__ __forceinline__ void
+prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int split, const bf16_t* __restrict__ q,
+              const bf16_t* __restrict__ pool, const int* __restrict__ table, int table_stride,
+              const int* __restrict__ tiles, int n_tiles, const int* __restrict__ entries, bf16_t* __restrict__ out,
+              int n_head, int n_kv, int P, float scale, int window, float* __restrict__ part_o,
+              float* __restrict__ part_ml, float softcap, const float* __restrict__ sink) {
   constexpr int WROWS = 32 * CB;                      // tokens per wavefront
   constexpr int TROWS = NW * WROWS;                   // tokens per tile
   constexpr int NP = HD / 8;                          // 16-byte pieces per K row
@@ -831,19 +875,18 @@ attn_prefill_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
   constexpr int MY_K = K_LOADS / NW, MY_LOADS = (K_LOADS + V_LOADS) / NW;   // per wavefront and turn
   constexpr int KS = HD / 16;                         // k-steps of the first product
   constexpr int DB = HD / 32;                         // 32-dim blocks of the output
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
   // Which (tile, head) this workgroup takes.  Workgroups go to the eight XCDs in turn (linear id
   // mod 8) and each XCD has an L2 of its own: with a multiple of eight kv heads, an XCD is given
   // whole kv heads, so that the keys and values of a head are read into one L2 only.
-  int head = blockIdx.y, bx = blockIdx.x;
+  int head = by;
   if (n_kv % 8 == 0) {
-    const int id = blockIdx.y * gridDim.x + blockIdx.x;
+    const int id = by * gx + bx;
     const int xcd = id & 7, local = id >> 3;
-    const int per_kv = (n_head / n_kv) * gridDim.x;       // workgroups of one kv head
+    const int per_kv = (n_head / n_kv) * gx;              // workgroups of one kv head
     const int rest = local % per_kv;
-    head = (xcd + 8 * (local / per_kv)) * (n_head / n_kv) + rest / gridDim.x;
-    bx = rest % gridDim.x;
+    head = (xcd + 8 * (local / per_kv)) * (n_head / n_kv) + rest / gx;
+    bx = rest % gx;
   }
   // the wavefront's number in scalar registers: what follows from it (which turns it loads, where they
   // go, which rows are its own) is then worked out once per wavefront, not once per lane
@@ -1292,6 +1335,43 @@ attn_prefill_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
   }   // slot
 }
 
+template <int HD, int NG, int NW = 4, int ST = PF_STAGES, bool PAIRED = false, int CB = 1>
+__global__ void __launch_bounds__(64 * NW * NG)
+attn_prefill_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool,
+                        const int* __restrict__ table, int table_stride, const int* __restrict__ tiles,
+                        int n_tiles, const int* __restrict__ entries, bf16_t* __restrict__ out, int n_head,
+                        int n_kv, int P, float scale, int window, float* __restrict__ part_o = nullptr,
+                        float* __restrict__ part_ml = nullptr, float softcap = 0.f, const float* __restrict__ sink = nullptr) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  prefill_tiles<HD, NG, NW, ST, PAIRED, CB>(smem, blockIdx.x, blockIdx.y, gridDim.x, gridDim.z, blockIdx.z, q, pool, table,
+                                            table_stride, tiles, n_tiles, entries, out, n_head, n_kv, P, scale, window, part_o,
+                                            part_ml, softcap, sink);
+}
+
+// ============================================== portions and single tokens in one launch
+// A step that holds portions beside decoded tokens: the first n_tiles * n_head workgroups take a tile of 64 rows
+// each (the unpaired kernel above), the others a run of a single token's context (by records), walked by eight
+// wavefronts.  The tiles are bound by their softmax and leave memory idle, the single tokens by what a compute unit
+// reads: side by side they take about as long as the longer of the two.
+template <int HD>
+__global__ void __launch_bounds__(512)
+attn_step_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool, const int* __restrict__ table, int table_stride,
+                 const int* __restrict__ tiles, int n_tiles, const int* __restrict__ entries, const int* __restrict__ runs,
+                 int run_stride, int group, bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
+                 int n_head, int n_kv, int P, float scale, int window, float softcap, const float* __restrict__ sink) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int n_pre = n_tiles * n_head, id = blockIdx.x;
+  if (id < n_pre) {
+    prefill_tiles<HD, 4, 2, 2, false, 1>(smem, id % n_tiles, id / n_tiles, n_tiles, 1, 0, q, pool, table, table_stride, tiles,
+                                         n_tiles, entries, out, n_head, n_kv, P, scale, window, nullptr, nullptr, softcap, sink);
+  } else {
+    const int at = id - n_pre, ways = n_kv * ((group + 15) / 16);
+    decode_run<HD, false, 8, true>(*reinterpret_cast<DecodeMerge<HD, 8>*>(smem), at / ways, at % ways, 0, q, pool, table,
+                                          table_stride, nullptr, nullptr, nullptr, out, part_o, part_ml, n_head, n_kv, P, scale,
+                                          window, 1, QKPrep{}, softcap, sink, DecodeRuns{runs, run_stride}, group);
+  }
+}
+
 // ------------------------------------------------------------------ dispatch
 static int check_common(const char* what, int n_head, int n_kv, int hd, int P, int table_stride) {
   if (!(hd == 32 || hd == 64 || hd == 128)) {
@@ -1322,8 +1402,6 @@ static int compute_units() {
   }
   return n;
 }
-// 1 (default): small decode launches from the projections let one wavefront prepare the query
-static int g_decode_shared_query = 1;
 
 // Decode rows.  rows: which rows of the step (nullptr: rows 0..n_rows-1).  n_splits > 1 needs
 // part_o (float [n_rows, n_head, n_splits, hd]) and part_ml (float [n_rows, n_head, n_splits, 2]).
@@ -1349,19 +1427,12 @@ static int launch_decode(const void* q, const void* pool, const int* table, int 
   const int parts = (n_head / n_kv + 15) / 16;
   TI_REQUIRE(n_kv * parts <= 65535, "attention_decode: too many heads");
   dim3 grid(n_rows, n_kv * parts, n_splits);
-  // at most one workgroup per compute unit: one wavefront prepares the query for all four
-  const bool shared = PREP && g_decode_shared_query && (long)n_rows * n_kv * parts * n_splits <= compute_units();
 #define TI_DEC(H)                                                                                          \
   case H:                                                                                                  \
-    if (shared)                                                                                            \
-      attn_decode_kernel<H, PREP, PREP><<<grid, 256, 0, stream>>>(                                         \
-          (const bf16_t*)q, (const bf16_t*)pool, table, table_stride, pos, slot, rows, (bf16_t*)out,        \
-          part_o, part_ml, n_head, n_kv, page_size, scale, window, n_splits, prep, g_softcap, g_sink);      \
-    else                                                                                                   \
-      attn_decode_kernel<H, PREP><<<grid, 256, 0, stream>>>((const bf16_t*)q, (const bf16_t*)pool, table,   \
-                                                            table_stride, pos, slot, rows, (bf16_t*)out,    \
-                                                            part_o, part_ml, n_head, n_kv, page_size,       \
-                                                            scale, window, n_splits, prep, g_softcap, g_sink); \
+    attn_decode_kernel<H, PREP><<<grid, 256, 0, stream>>>((const bf16_t*)q, (const bf16_t*)pool, table,     \
+                                                          table_stride, pos, slot, rows, (bf16_t*)out,      \
+                                                          part_o, part_ml, n_head, n_kv, page_size,         \
+                                                          scale, window, n_splits, prep, g_softcap, g_sink);  \
     if (n_splits > 1)                                                                                       \
       attn_merge_kernel<H><<<dim3(n_rows, n_head), (H < 64 ? 64 : H), 0, stream>>>(part_o, part_ml, rows,   \
                                                                                   (bf16_t*)out, n_head,    \
@@ -1552,6 +1623,95 @@ extern "C" int ti_attention_prefill_paired_bf16(const void* q, const void* pool,
   return 0;
 }
 
+// What a launch by records needs: n_runs records of run_stride ints, and where rows are cut (n_rows > 0) the rows' records
+// int [n_rows][4] and buffers for the runs' results, [n_runs][n_head][hd] and [n_runs][n_head][2].
+static int check_runs(const char* what, const int* runs, int n_runs, int run_stride, const int* rows, int n_rows, const float* part_o,
+                      const float* part_ml) {
+  TI_REQUIRE(runs && n_runs > 0 && n_runs <= 65535 && run_stride >= TI_RUN_HEAD, "%s: records (%d of %d ints)", what, n_runs, run_stride);
+  TI_REQUIRE(n_rows == 0 || (n_rows > 0 && rows && part_o && part_ml), "%s: rows in several runs need records and buffers", what);
+  return 0;
+}
+
+// ti_attention_decode_prepared_bf16 by records (see DecodeRuns).  Serves the same sizes.
+extern "C" int ti_attention_decode_runs_bf16(const float* qkv, int row_width, const float* q_w, const float* k_w, float eps,
+                                             const float* inv_freq, const float* rope_table, int table_len, void* pool, int write_kv,
+                                             const int* table, int table_stride, const int* runs, int n_runs, int run_stride,
+                                             const int* rows, int n_rows, void* out, float* part_o, float* part_ml, int n_head, int n_kv,
+                                             int hd, int page_size, float scale, int window, hipStream_t stream) {
+  int rc = check_common("attention_decode_runs", n_head, n_kv, hd, page_size, table_stride);
+  if (rc) return rc;
+  if (hd == 32 || n_head / n_kv > 16 || ((uintptr_t)q_w & 15) || ((uintptr_t)rope_table & 15)) {
+    ti_set_error("attention_decode_runs: head_dim %d with %d q heads per kv head is not served (or a norm "
+                 "weight or the sin/cos table is not 16-byte aligned)", hd, n_head / n_kv);
+    return 3;
+  }
+  TI_REQUIRE(qkv && row_width >= (n_head + (write_kv ? 2 * n_kv : 0)) * hd && row_width % 4 == 0 && ((uintptr_t)qkv & 15) == 0,
+             "attention_decode_runs: the projections do not fit (row_width %d)", row_width);
+  TI_REQUIRE(inv_freq || !rope_table, "attention_decode_runs: a sin/cos table without inv_freq");
+  rc = check_runs("attention_decode_runs", runs, n_runs, run_stride, rows, n_rows, part_o, part_ml);
+  if (rc) return rc;
+#define TI_GO(H)                                                                                                          \
+  attn_decode_runs_kernel<H><<<dim3(n_kv, n_runs), 256, 0, stream>>>(                                                     \
+      runs, run_stride, n_head / n_kv, qkv, row_width, n_kv, q_w, k_w, (const float2*)rope_table, (const bf16_t*)pool, table, \
+      table_stride, page_size, inv_freq, table_len, eps, write_kv ? (bf16_t*)pool : nullptr, (bf16_t*)out, part_o, part_ml,   \
+      scale, window)
+  if (hd == 128) TI_GO(128);
+  else TI_GO(64);
+#undef TI_GO
+  if (n_rows) {
+    if (hd == 128) attn_merge_kernel<128, true><<<dim3(n_rows, n_head), 128, 0, stream>>>(part_o, part_ml, rows, (bf16_t*)out, n_head, 0, nullptr);
+    else attn_merge_kernel<64, true><<<dim3(n_rows, n_head), 64, 0, stream>>>(part_o, part_ml, rows, (bf16_t*)out, n_head, 0, nullptr);
+  }
+  TI_LAUNCH_CHECK();
+  return 0;
+}
+
+// Portions (tiles of 64 rows as above, unpaired, whole) and the single-token rows of the same step (by records) in one
+// launch; softcap as for the entry points below.  Returns 3 for head sizes other than 64 and 128.
+extern "C" int ti_attention_step_bf16(const void* q, const void* pool, const int* table, int table_stride, const int* tiles,
+                                      const int* entries, int n_tiles, const int* runs, int n_runs, int run_stride, const int* rows,
+                                      int n_rows, void* out, float* part_o, float* part_ml, int n_head, int n_kv, int hd, int page_size,
+                                      float scale, float softcap, int window, hipStream_t stream) {
+  int rc = check_common("attention_step", n_head, n_kv, hd, page_size, table_stride);
+  if (rc) return rc;
+  if (hd == 32) {
+    ti_set_error("attention_step: head_dim 32 is not served (64, 128)");
+    return 3;
+  }
+  TI_REQUIRE(n_tiles > 0 && tiles && entries, "attention_step: no tiles");
+  rc = check_runs("attention_step", runs, n_runs, run_stride, rows, n_rows, part_o, part_ml);
+  if (rc) return rc;
+  const int parts = (n_head / n_kv + 15) / 16;
+  const long grid = (long)n_tiles * n_head + (long)n_runs * n_kv * parts;
+  TI_REQUIRE(grid <= 0x7fffffL, "attention_step: too many workgroups");
+  constexpr int STAGES = 4 * 2 * 2 * PF_KEYS * 2;      // bytes of the tiles' stages per head dimension
+  static_assert(sizeof(DecodeMerge<128, 8>) <= STAGES * 128 && sizeof(DecodeMerge<64, 8>) <= STAGES * 64, "the merge fits the stages");
+  static bool ready = false;          // allow more than 64 KiB of dynamic LDS, once
+  if (!ready) {
+    if (hipFuncSetAttribute((const void*)attn_step_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, STAGES * 128) != hipSuccess ||
+        hipFuncSetAttribute((const void*)attn_step_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize, STAGES * 64) != hipSuccess) {
+      ti_set_error("attention_step: cannot reserve the LDS");
+      return 2;
+    }
+    ready = true;
+  }
+  const float cap = softcap > 0.f ? softcap : 0.f;
+#define TI_GO(H)                                                                                                              \
+  do {                                                                                                                        \
+    attn_step_kernel<H><<<(unsigned)grid, 512, STAGES * H, stream>>>((const bf16_t*)q, (const bf16_t*)pool, table, table_stride, \
+                                                                     tiles, n_tiles, entries, runs, run_stride, n_head / n_kv,  \
+                                                                     (bf16_t*)out, part_o, part_ml,                              \
+                                                                     n_head, n_kv, page_size, scale, window, cap, g_sink);       \
+    if (n_rows)                                                                                                               \
+      attn_merge_kernel<H, true><<<dim3(n_rows, n_head), H, 0, stream>>>(part_o, part_ml, rows, (bf16_t*)out, n_head, 0, g_sink); \
+  } while (0)
+  if (hd == 128) TI_GO(128);
+  else TI_GO(64);
+#undef TI_GO
+  TI_LAUNCH_CHECK();
+  return 0;
+}
+
 // The three entry points above with soft-capped scores: s <- softcap tanh(s / softcap) before the softmax.
 struct CapScope {
   explicit CapScope(float cap) { g_softcap = cap > 0.f ? cap : 0.f; }
@@ -1588,14 +1748,12 @@ extern "C" int ti_attention_prefill_paired_capped_bf16(const void* q, const void
 // tinyinfer_kernels_tuning.h); process-wide in the library, applied and reset around its calls by the
 // host library's Ops.  Returns 0, or 1 for an unknown name.
 extern "C" void ti_tuning_reset() {
-  g_decode_shared_query = 1;
   g_prefill_groups = 0;
   g_prefill_lds = 1;
 }
 extern "C" int ti_tuning_set(const char* name, long value) {
   const std::string n = name ? name : "";
-  if (n == "decode_shared_query") g_decode_shared_query = (int)value;
-  else if (n == "prefill_groups") g_prefill_groups = (int)value;
+  if (n == "prefill_groups") g_prefill_groups = (int)value;
   else if (n == "prefill_use_lds") g_prefill_lds = (int)value;
   else return 1;
   return 0;

@@ -441,6 +441,24 @@ int ti_attention_decode_prepared_bf16(const float* qkv, int row_width, const flo
                                       const int* slot, void* out, float* part_o, float* part_ml, int n_rows,
                                       int n_head, int n_kv, int hd, int page_size, float scale, int window,
                                       int n_splits, hipStream_t stream);
+// the same by records (int32 [n_runs][run_stride]: what each workgroup walks, TI_RUN_*, then the page ids of its first blocks,
+// (run_stride - TI_RUN_HEAD) / wavefronts of them, at least four, for each of its four wavefronts): every row in as many runs as
+// the host chose.  n_rows > 0: rows in several runs are merged, by the rows' records int32 [n_rows][4] = (row, first run's place,
+// runs, -); part_o f32 [places][n_head][hd], part_ml f32 [places][n_head][2]
+int ti_attention_decode_runs_bf16(const float* qkv, int row_width, const float* q_w, const float* k_w, float eps,
+                                  const float* inv_freq, const float* rope_table, int table_len, void* pool, int write_kv,
+                                  const int* table, int table_stride, const int* runs, int n_runs, int run_stride, const int* rows,
+                                  int n_rows, void* out, float* part_o, float* part_ml, int n_head, int n_kv, int hd, int page_size,
+                                  float scale, int window, hipStream_t stream);
+// a step's portions (tiles of 64 rows, see ti_attention_prefill_paired_bf16) and its single-token rows (by records, for eight
+// wavefronts a workgroup) in one launch (head sizes 64, 128)
+int ti_attention_step_bf16(const void* q, const void* pool, const int* table, int table_stride, const int* tiles, const int* entries,
+                           int n_tiles, const int* runs, int n_runs, int run_stride, const int* rows, int n_rows, void* out,
+                           float* part_o, float* part_ml, int n_head, int n_kv, int hd, int page_size, float scale, float softcap,
+                           int window, hipStream_t stream);
+// a record's header: row of the step, its position, the run's first block of 16 positions, its blocks (0: nobody's), the place of
+// its partial result (-1: it is the whole row), the row of the block tables, the page of the row's own position
+enum { TI_RUN_ROW, TI_RUN_POS, TI_RUN_FIRST, TI_RUN_BLOCKS, TI_RUN_PART, TI_RUN_TABLE_ROW, TI_RUN_OWN_PAGE, TI_RUN_HEAD = 8 };
 // portions of prompts: tiles int32 [n_tiles][2] = (entry, first row) of 128 rows each, entries int32
 // [n_entries][4] = (row0, n_tokens, start_pos, -)
 int ti_attention_prefill_bf16(const void* q, const void* pool, const int* table, int table_stride, const int* tiles,

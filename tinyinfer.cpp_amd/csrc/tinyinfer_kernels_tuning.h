@@ -30,7 +30,6 @@
 //   wide_rows_min_n      the fewest weight rows from which 17..64 rows take the kernel that keeps them in registers (16,384)
 //   wide_rows_grid       its number of workgroups (0: a tile of 16 weight rows each, at most one per compute unit)
 // libti_attention_bf16:
-//   decode_shared_query  0: every wavefront of a decode workgroup prepares the query itself
 //   prefill_groups       1 or 2 groups of wavefronts per workgroup, 0: by the launch
 //   prefill_use_lds      0: the kernel without LDS for every head size
 #pragma once

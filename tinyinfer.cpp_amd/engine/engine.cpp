@@ -37,6 +37,13 @@ int* StepPlan::ints(const std::string& key, size_t n) {
   return l.host.data();
 }
 
+int StepPlan::group_of(const Part* part) const {
+  if (!groups_) return -1;
+  const auto it = groups_->find(part);
+  return it == groups_->end() ? -1 : it->second;
+}
+const int* StepPlan::table_row(int group, size_t entry) const { return cache_->table_row(group, requests_->at(entry)); }
+
 struct Engine::Impl {
   struct Graph {
     hipGraph_t graph = nullptr;
@@ -56,11 +63,15 @@ struct Engine::Impl {
     std::vector<int64_t> requests;
     std::vector<int> n_tokens;
     std::vector<int64_t> admitted_here;
-    bool decode_fast = false;
+    std::vector<EntryRecord> entries;
+    int64_t M = 0, n_want = 0;
+    int max_context = 0;
+    bool decode_only = false, decode_fast = false;
   };
 
   Engine& e;
   std::vector<Part*> parts;                 // every part, once
+  std::map<const Part*, int> groups;        // the group of cache layers a part is bound to
   // storage behind the cache manager: per group, [cache layer][page][K|V][kv head][row][hd] of the
   // compute dtype, or [cache layer][slot][...] float32
   std::vector<DeviceBuffer> storage;
@@ -151,15 +162,15 @@ struct Engine::Impl {
     return true;
   }
 
-  std::unique_ptr<Prepared> prepare(const std::vector<StepEntry>& entries, Graph* graph, bool capturing) {
+  // The step's pages are reserved and its lists planned: what it will launch is known, nothing has been launched.
+  // for_graph: the step may be captured, or replay a captured one.
+  std::unique_ptr<Prepared> begin(const std::vector<StepEntry>& entries, bool for_graph) {
     if (entries.empty()) throw EngineError("a step needs at least one entry");
     CacheManager& c = *e.cache;
     const int64_t V = e.model->spec.vocab_size;
     auto p = std::unique_ptr<Prepared>(new Prepared());
     std::vector<int> starts;
     p->decode_fast = reserve_decode_step(entries, starts);
-    int64_t M = 0, n_want = 0;
-    const size_t R = entries.size();
     if (!p->decode_fast) {
       std::set<int64_t> seen;
       for (const auto& en : entries) {
@@ -207,15 +218,38 @@ struct Engine::Impl {
       }
     }
     for (const auto& en : entries) {
-      M += (int64_t)en.tokens.size();
-      n_want += (int64_t)en.want.size();
       p->requests.push_back(en.request);
       p->n_tokens.push_back((int)en.tokens.size());
     }
     // the pages are taken: whatever fails from here on (a part's plan, a buffer that cannot be had)
     // gives them back before the error leaves
     try {
-      fill(*p, entries, starts, M, n_want, graph, capturing);
+      const size_t R = entries.size();
+      p->entries.reserve(R);
+      p->decode_only = true;
+      for (size_t i = 0; i < R; ++i) {
+        const int n = p->n_tokens[i];
+        const int start = p->decode_fast ? starts[i] : c.length(p->requests[i]);
+        p->entries.push_back({(int)p->M, n, start, c.slot(p->requests[i])});
+        p->decode_only = p->decode_only && n == 1;
+        p->max_context = std::max(p->max_context, start + n);
+        p->M += n;
+        p->n_want += (int64_t)entries[i].want.size();
+      }
+      // what the parts add to the step's metadata
+      StepPlan& plan = p->plan;
+      plan.entries_ = &p->entries;
+      plan.M_ = p->M;
+      plan.decode_only_ = p->decode_only;
+      plan.max_seq_ = e.max_seq;
+      plan.for_graph_ = for_graph;
+      plan.act_dtype_ = e.act_dtype;
+      plan.page_size_ = e.page_size;
+      plan.ops_ = &e.ops;
+      plan.cache_ = &c;
+      plan.requests_ = &p->requests;
+      plan.groups_ = &groups;
+      for (Part* part : parts) part->plan(plan);
     } catch (...) {
       undo(*p);
       throw;
@@ -223,11 +257,20 @@ struct Engine::Impl {
     return p;
   }
 
-  void fill(Prepared& prepared, const std::vector<StepEntry>& entries, const std::vector<int>& starts, int64_t M, int64_t n_want,
-            Graph* graph, bool capturing) {
+  // The step's metadata on its way to the device, and its context.  What fails gives the pages back.
+  void fill(Prepared& prepared, const std::vector<StepEntry>& entries, Graph* graph, bool capturing) {
+    try {
+      fill_in(prepared, entries, graph, capturing);
+    } catch (...) {
+      undo(prepared);
+      throw;
+    }
+  }
+  void fill_in(Prepared& prepared, const std::vector<StepEntry>& entries, Graph* graph, bool capturing) {
     Prepared* p = &prepared;
     CacheManager& c = *e.cache;
     const size_t R = entries.size();
+    const int64_t M = p->M, n_want = p->n_want;
     clear_slots();
 
     Workspace& work = graph ? graph->ws : ws;
@@ -236,29 +279,11 @@ struct Engine::Impl {
     ctx.engine = &e;
     ctx.M = M;
     ctx.n_out = n_want;
-    ctx.entries.reserve(R);
-    bool decode_only = true;
-    int row0 = 0, max_context = 0;
-    for (size_t i = 0; i < R; ++i) {
-      const auto& en = entries[i];
-      const int n = (int)en.tokens.size();
-      const int start = p->decode_fast ? starts[i] : c.length(en.request);
-      ctx.entries.push_back({row0, n, start, c.slot(en.request)});
-      decode_only = decode_only && n == 1;
-      max_context = std::max(max_context, start + n);
-      row0 += n;
-    }
-    ctx.decode_only = decode_only;
-    ctx.max_context = max_context;
-
-    // what the parts add to the step's metadata
+    ctx.entries = p->entries;
+    ctx.decode_only = p->decode_only;
+    ctx.max_context = p->max_context;
     StepPlan& plan = p->plan;
-    plan.entries_ = &ctx.entries;
-    plan.M_ = M;
-    plan.decode_only_ = decode_only;
-    plan.max_seq_ = e.max_seq;
     plan.sized_for_longest_ = capturing;
-    for (Part* part : parts) part->plan(plan);
     ctx.plan = &plan;
 
     // layout: tokens | positions | slots | out_rows | entries [R,4] | the parts' lists | tables
@@ -372,8 +397,9 @@ struct Engine::Impl {
       if (e.cache->has(r)) e.cache->release(r);
   }
 
-  Tensor step(const std::vector<StepEntry>& entries) {
-    auto p = prepare(entries, nullptr, false);
+  Tensor step(const std::vector<StepEntry>& entries) { return step(entries, begin(entries, false)); }
+  Tensor step(const std::vector<StepEntry>& entries, std::unique_ptr<Prepared> p) {
+    fill(*p, entries, nullptr, false);
     Tensor logits;
     try {
       logits = run(*p->ctx);
@@ -398,9 +424,9 @@ struct Engine::Impl {
     return key;
   }
 
-  Tensor capture(const std::vector<StepEntry>& entries, const std::string& key, bool decode) {
+  Tensor capture(const std::vector<StepEntry>& entries, const std::string& key, bool decode, std::unique_ptr<Prepared> p) {
     std::unique_ptr<Graph> g(new Graph());
-    auto p = prepare(entries, g.get(), true);
+    fill(*p, entries, g.get(), true);
     try {
       // a first run outside the graph: it computes this step's result and makes every workspace
       // buffer the graph will use
@@ -447,23 +473,26 @@ struct Engine::Impl {
   Tensor step_graph(const std::vector<StepEntry>& entries) {
     if (foreign) return step(entries);      // parts outside the library launch on streams of their own
     bool decode = false;
-    const std::string key = shape_key(entries, decode);
+    std::string key = shape_key(entries, decode);
+    auto p = begin(entries, true);
+    // a step of single tokens has two graphs: with the kernels that merge the runs of a row, and without
+    if (decode && p->plan.runs_planned_ && !p->plan.merges_) key += "w";
     auto it = graphs.find(key);
     if (it == graphs.end()) {
       if (!decode) {
         if (shapes_seen.size() > 4096) shapes_seen.clear();
         const int seen = ++shapes_seen[key];
-        if (seen < STEP_GRAPH_AFTER) return step(entries);
+        if (seen < STEP_GRAPH_AFTER) return step(entries, std::move(p));
         shapes_seen.erase(key);
       }
-      return capture(entries, key, decode);
+      return capture(entries, key, decode, std::move(p));
     }
     if (!decode) {
       shape_order.remove(key);
       shape_order.push_back(key);
     }
     Graph& g = *it->second;
-    auto p = prepare(entries, &g, false);
+    fill(*p, entries, &g, false);
     try {
       hip_check(hipGraphLaunch(g.exec, stream), "hipGraphLaunch");
     } catch (...) {
@@ -570,6 +599,8 @@ Engine::Engine(std::shared_ptr<Model> model_, const EngineOptions& o)
     impl_->parts.push_back(&p);
     p.prepare(ops, max_seq);          // tables that depend on the longest sequence
   });
+  for (const auto& run : model->bindings)
+    for (const auto& b : run) impl_->groups.emplace(b.first, b.second.first);
   impl_->foreign = model->has_foreign_parts();
   if (!impl_->foreign) {
     impl_->feedback_rows = cache->max_requests;

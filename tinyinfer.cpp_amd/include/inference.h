@@ -299,6 +299,7 @@ class Ops {
   void* stream() const { return stream_; }
   void set_stream(void* s) { flush(); stream_ = s; }
   int compute_units();
+  int units() const { return const_cast<Ops*>(this)->compute_units(); }
 
   // a token below zero stands for fed[-1 - token] (device memory, n_fed ids; may be null)
   // scale: a factor on every element, in 32-bit
@@ -585,6 +586,21 @@ class Ops {
   void tune(const std::string& library, const std::string& name, long value);
   void untune();
   static int decode_splits(int n_rows, int kv_heads, int heads, int context, int typical, int units, int head_dim = 128);
+  // The decode attention by records: what each workgroup walks of the single-token rows' contexts.
+  struct RunsLaunch { int wavefronts = 4, records = 0, stride = 0; };
+  struct RunsRow { int row, pos, first_block, blocks, table_row; const int* pages; };      // pages: by position / page size
+  // the sizes of the lists, from what every step of a shape shares: rows, the most blocks of 16 positions a row may have, workgroups a
+  // record (`ways`), compute units that portions of the same launch take (`busy`; wavefronts: 4 alone, 8 beside portions);
+  // listed_blocks: the blocks of a run whose page ids come with its record
+  static RunsLaunch runs_launch(int n_rows, int most_blocks, int listed_blocks, int ways, int units, int busy, int wavefronts);
+  // runs [records][stride], rows [n_rows][4]; how many places partial results take (0: every row in one run), and the records in use.
+  // beside_us: how long the portions of the same launch take
+  static int plan_runs(const std::vector<RunsRow>& list, const RunsLaunch& launch, int ways, int units, int busy, double beside_us,
+                       int head_dim, int page_size, int* runs, int* rows, int* used);
+  // a step's portions and single-token rows in one launch (else one after the other)?  portion_us: how long the portions take in it
+  static bool portions_with_rows(int n_tiles_small, int n_rows, int heads, int kv_heads, int portion_context, int rows_context, int window,
+                                 int units, int head_dim);
+  static double portion_us(int portion_context, int window);
   // runs of keys for the prefill kernel with 64-row tiles, and whether it pairs a heavy with a light tile
   static int portion_launch(int n_tiles_small, int heads, int portion_context, int window, int units, bool* paired);
 
@@ -641,6 +657,11 @@ struct AttentionWork {
   int n_tiles_small = 0;
   const int* decode_rows = nullptr;  // rows of single-token entries (null when every entry is one)
   int n_decode_rows = 0;
+  const int* runs = nullptr;         // [n_runs][run_stride] what each workgroup walks of the single-token rows' contexts (see Ops::plan_runs);
+  int n_runs = 0, run_stride = 0;    // null: every row in as many equal runs
+  const int* run_rows = nullptr;     // [n_run_rows][4] how many runs a row is in, for the merge
+  int n_run_rows = 0;                // 0: every row is in one run
+  bool runs_with_tiles = false;      // the records are for a launch that holds the portions as well
   bool decode_only = false;
   bool slots_are_rows = false;       // slots[m] == m for every row (a step of single tokens, one entry a row)
   int max_context = 0;               // longest context any row reads
@@ -662,6 +683,7 @@ struct StepEntry {
 struct EntryRecord { int row0, n_tokens, start, state_slot; };
 
 class Engine;
+class CacheManager;
 class Part;
 // What a part may add to a step before its metadata goes to the device: integer lists of its
 // own.  `ints(key, n)` returns host memory for n ints that will lie in the step's metadata;
@@ -673,6 +695,15 @@ class StepPlan {
   bool decode_only() const { return decode_only_; }
   int max_seq() const { return max_seq_; }
   bool sized_for_longest() const { return sized_for_longest_; }   // a graph is being captured: size launches for max_seq
+  bool for_graph() const { return for_graph_; }                   // the step may be a replay: lists of the same sizes for every step of its shape
+  DType act_dtype() const { return act_dtype_; }
+  int page_size() const { return page_size_; }
+  const Ops* ops() const { return ops_; }
+  int group_of(const Part* part) const;                           // the part's group of cache layers, -1: none
+  const int* table_row(int group, size_t entry) const;            // the entry's page ids, as many as a table row holds
+  // whether a step's launches merge runs of a row: a captured step of single tokens is kept for either
+  void set_merges(bool any) { runs_planned_ = true; merges_ = merges_ || any; }
+  bool merges() const { return merges_; }
   bool has(const std::string& key) const { return lists_.count(key) != 0; }
   int* ints(const std::string& key, size_t n);
   void set_value(const std::string& key, int64_t v) { values_[key] = v; }
@@ -684,8 +715,13 @@ class StepPlan {
   std::map<std::string, int64_t> values_;
   const std::vector<EntryRecord>* entries_ = nullptr;
   int64_t M_ = 0;
-  bool decode_only_ = false, sized_for_longest_ = false;
-  int max_seq_ = 0;
+  bool decode_only_ = false, sized_for_longest_ = false, for_graph_ = false, runs_planned_ = false, merges_ = false;
+  int max_seq_ = 0, page_size_ = 16;
+  DType act_dtype_ = DType::F32;
+  const Ops* ops_ = nullptr;
+  const CacheManager* cache_ = nullptr;
+  const std::vector<int64_t>* requests_ = nullptr;                // of the entries
+  const std::map<const Part*, int>* groups_ = nullptr;
 };
 
 // Everything a part may touch during one step.

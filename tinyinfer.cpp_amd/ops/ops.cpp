@@ -736,6 +736,128 @@ int Ops::decode_splits(int n_rows, int kv_heads, int heads, int context, int typ
   return best;
 }
 
+// ---- launches by records.  What one costs, as measured at a head size of 128 in a chain of 28 (us): a workgroup that walks 16 n
+// positions of one row takes 6.0 + 0.147 n alone (13 blocks 7.8, 129 25.2); rows in several runs need the merge, 2.7; all
+// workgroups together read at most 6.4e6 bytes a us, and the two bounds wear on each other as the root of their squares' sum does
+// (8 rows of 129 blocks: in runs of 129 30.9, 65 23.4, 43 20.4, 33 19.9, 22 21.5; 23 rows of 6 to 107 blocks: 107 29.3, 72 26.3,
+// 36 27.1, 27 25.0; 32 equal runs of them would be 24).  Beside portions eight wavefronts walk a run at 0.2 a block.
+static const double RUN_START_US = 6.0, RUN_MERGE_US = 2.7, RUN_BLOCK_US = 0.147, RUN_BLOCK_BESIDE_US = 0.2, RUN_BYTES_US = 6.4e6;
+static const double RUN_NEXT_US = 4.0;       // a workgroup that starts behind another on its unit
+static const int RUN_LEAST_BLOCKS = 4;       // a block a wavefront
+static const int RUN_MOST = 32;              // runs a row (the merge asks for so many at once)
+static const int RUN_LIST_INTS = 64 * 1024;  // the records' room in a step's metadata
+
+Ops::RunsLaunch Ops::runs_launch(int n_rows, int most_blocks, int listed_blocks, int ways, int units, int busy, int wavefronts) {
+  RunsLaunch l;
+  l.wavefronts = wavefronts;
+  // a round of the compute units where half of it holds a record a row (finer runs gain nothing then), two rounds where it does not
+  const int round = std::max(1, std::max(units / 4, units - busy) / std::max(1, ways));
+  int records = n_rows <= round / 2 ? round : 2 * round * ((n_rows + 2 * round - 1) / (2 * round));
+  const int most_runs = std::min(RUN_MOST, (most_blocks + RUN_LEAST_BLOCKS - 1) / RUN_LEAST_BLOCKS);
+  records = (int)std::min<long>(records, (long)n_rows * std::max(1, most_runs));
+  l.records = std::max(records, n_rows);
+  // page ids with the record: of up to 64 blocks a wavefront, as many as the list has room for
+  const int each = std::max(4, std::min({64, (listed_blocks + wavefronts - 1) / wavefronts, (RUN_LIST_INTS / l.records - TI_RUN_HEAD) / wavefronts}));
+  l.stride = TI_RUN_HEAD + wavefronts * each;
+  return l;
+}
+
+int Ops::plan_runs(const std::vector<RunsRow>& list, const RunsLaunch& launch, int ways, int units, int busy, double beside_us,
+                   int head_dim, int page_size, int* runs, int* rows, int* used) {
+  int longest = 1;
+  long total = 0;
+  for (const RunsRow& r : list) {
+    longest = std::max(longest, r.blocks);
+    total += r.blocks;
+  }
+  const double size = head_dim / 128.0, block = (busy ? RUN_BLOCK_BESIDE_US : RUN_BLOCK_US) * size;
+  const double read = (double)total * ways * 16 * 512 * size / RUN_BYTES_US;
+  int length = longest;
+  double best = -1.0;
+  for (int s = 1; s <= RUN_MOST; ++s) {
+    const int len = std::max((longest + s - 1) / s, std::min(longest, RUN_LEAST_BLOCKS));
+    long items = 0;
+    for (const RunsRow& r : list) items += (r.blocks + len - 1) / len;
+    if (items > launch.records && s > 1) break;
+    const long groups = items * ways;
+    double load;      // runs that a unit walks one after the other
+    if (busy) load = groups <= units - busy ? 1.0 : 1.0 + (double)(groups - std::max(0, units - busy)) / units;
+    else load = (double)((groups + units - 1) / units);
+    const double walk = load * len * block;
+    double us = RUN_START_US + std::sqrt(walk * walk + read * read) + (items > (long)list.size() ? RUN_MERGE_US : 0.0);
+    us += RUN_NEXT_US * (busy ? load - 1.0 : std::max(0.0, std::ceil(load / 2) - 1.0));      // (two workgroups fit a unit, one beside portions)
+    us = std::max(us, beside_us + (items > (long)list.size() ? RUN_MERGE_US : 0.0));
+    if (best < 0 || us < best - 1e-9) {
+      best = us;
+      length = len;
+    }
+    if (len <= RUN_LEAST_BLOCKS) break;
+  }
+  struct Item { int row, first, blocks, part; };
+  std::vector<Item> items;
+  items.reserve(launch.records);
+  int places = 0;
+  for (size_t i = 0; i < list.size(); ++i) {
+    const RunsRow& r = list[i];
+    int k = (r.blocks + length - 1) / length;
+    const int per = (r.blocks + k - 1) / k;
+    k = (r.blocks + per - 1) / per;
+    rows[4 * i] = r.row;
+    rows[4 * i + 1] = k > 1 ? places : -1;
+    rows[4 * i + 2] = k;
+    rows[4 * i + 3] = 0;
+    for (int s = 0; s < k; ++s) items.push_back({(int)i, s * per, std::min(per, r.blocks - s * per), k > 1 ? places++ : -1});
+  }
+  // the longest first
+  std::stable_sort(items.begin(), items.end(), [](const Item& a, const Item& b) { return a.blocks > b.blocks; });
+  const int each = (launch.stride - TI_RUN_HEAD) / launch.wavefronts;
+  for (int n = 0; n < launch.records; ++n) {
+    int* rec = runs + (size_t)n * launch.stride;
+    if (n >= (int)items.size()) {
+      rec[TI_RUN_BLOCKS] = 0;
+      continue;
+    }
+    const Item& it = items[n];
+    const RunsRow& r = list[it.row];
+    rec[TI_RUN_ROW] = r.row;
+    rec[TI_RUN_POS] = r.pos;
+    rec[TI_RUN_FIRST] = r.first_block + it.first;
+    rec[TI_RUN_BLOCKS] = it.blocks;
+    rec[TI_RUN_PART] = it.part;
+    rec[TI_RUN_TABLE_ROW] = r.table_row;
+    rec[TI_RUN_OWN_PAGE] = r.pages[r.pos / page_size];
+    for (int w = 0; w < launch.wavefronts; ++w) {
+      int* ids = rec + TI_RUN_HEAD + w * each;
+      for (int j = 0; j < each && w + launch.wavefronts * j < it.blocks; ++j)
+        ids[j] = r.pages[(size_t)(r.first_block + it.first + w + launch.wavefronts * j) * 16 / page_size];
+    }
+  }
+  if (used) *used = (int)items.size();
+  return places;
+}
+
+// The portions' workgroups (a tile of 64 rows each, not paired, their keys in one run) and the rows' in one launch.  Portions whose keys
+// want several runs (a short portion behind a long context) would last longer than both launches one after the other;
+// portions that fill the chip by themselves are better off in pairs.  Measured at 16 heads, 8 of them for keys (us, both launches, then
+// one): 504 tokens beside 8 rows of 1,000 30.9 -> 18.2, behind 504 others 37.1 -> 23.5; 512 beside 64 rows of 200 35.3 -> 25.8, of 1,000
+// 81.9 -> 59.8; 32 beside 8 of 1,000 23.1 -> 16.3.
+static const double PORTION_START_US = 7.8, PORTION_TURN_US = 1.57 / 4;     // of a tile: its start, and a turn of 32 keys (four groups take them in rotation)
+double Ops::portion_us(int portion_context, int window) {
+  const int seen = window == 0 ? portion_context : std::min(portion_context, window + 64);
+  return PORTION_START_US + PORTION_TURN_US * ((seen + 31) / 32);
+}
+bool Ops::portions_with_rows(int n_tiles_small, int n_rows, int heads, int kv_heads, int portion_context, int rows_context, int window,
+                             int units, int head_dim) {
+  if (n_tiles_small == 0 || n_rows == 0 || (long)n_tiles_small * heads > units) return false;
+  const int S = portion_launch(n_tiles_small, heads, portion_context, window, units, nullptr);
+  if (S == 1) return true;
+  const double whole = portion_us(portion_context, window);
+  const double apart = PORTION_START_US + (whole - PORTION_START_US) / S + RUN_MERGE_US + RUN_START_US +
+                       RUN_BLOCK_US * (head_dim / 128.0) * (rows_context / 16.0) *
+                           std::max(1.0, (double)n_rows * kv_heads / units);
+  return whole < apart;
+}
+
 static int typical_context(const AttentionWork& w) {
   return w.split_context > w.max_context ? std::max(w.max_context, w.split_context / 2) : w.max_context;
 }
@@ -778,6 +900,21 @@ bool Ops::attention_from_projections(const AttentionWork& work, Workspace& ws, c
   const int P = (int)pool.shape[2];
   if ((head_dim != 64 && head_dim != 128) || P % 16 != 0 || heads / kv_heads > 16) return false;
   const int n = (int)work.M;
+  if (work.runs && !work.runs_with_tiles) {
+    float *part_o = nullptr, *part_ml = nullptr;
+    if (work.n_run_rows) {
+      part_o = (float*)ws.get("attn.part_o", (size_t)work.n_runs * heads * head_dim * 4);
+      part_ml = (float*)ws.get("attn.part_ml", (size_t)work.n_runs * heads * 2 * 4);
+    }
+    int rc = KERNEL("attention_bf16", ti_attention_decode_runs_bf16)(
+        (const float*)qkv.data, (int)qkv.shape[1], q_w, k_w, eps, rot.inv_freq, rot.table, rot.table_len, pool.data, write_kv ? 1 : 0,
+        view.table, view.table_width, work.runs, work.n_runs, work.run_stride, work.run_rows, work.n_run_rows, out.data, part_o, part_ml,
+        heads, kv_heads, head_dim, P, scale, window, (hipStream_t)launch_stream());
+    if (rc == 3) return false;
+    check("attention_bf16", rc, "attention(decode, by records)");
+    took(work.n_run_rows ? "[fused, runs]" : "[fused]");
+    return true;
+  }
   const int context = window == 0 ? work.split_context : std::min(work.split_context, window + 16);
   int S = decode_splits(n, kv_heads, heads, context, std::min(context, typical_context(work)), compute_units(), head_dim);
   if (use.force_decode_splits > 0) S = std::min(use.force_decode_splits, std::max(1, (context + 15) / 16));
@@ -828,6 +965,23 @@ bool Ops::attention(const AttentionWork& work, Workspace& ws, const CacheView& v
       done = true;
       void* stream = launch_stream();
       const int units = compute_units();
+      if (work.runs && work.runs_with_tiles && work.n_tiles_small && work.tiles_small && use.paired_prefill && use.force_paired_tiles < 0 &&
+          use.force_decode_splits == 0 && !work.decode_only) {
+        float *part_o = nullptr, *part_ml = nullptr;
+        if (work.n_run_rows) {
+          part_o = (float*)ws.get("attn.part_o", (size_t)work.n_runs * heads * head_dim * 4);
+          part_ml = (float*)ws.get("attn.part_ml", (size_t)work.n_runs * heads * 2 * 4);
+        }
+        const int rc = KERNEL("attention_bf16", ti_attention_step_bf16)(
+            q.data, pool.data, view.table, view.table_width, work.tiles_small, work.entry_meta, work.n_tiles_small, work.runs, work.n_runs,
+            work.run_stride, work.run_rows, work.n_run_rows, out.data, part_o, part_ml, heads, kv_heads, head_dim, P, scale, softcap,
+            window, (hipStream_t)stream);
+        if (rc != 3) {
+          check("attention_bf16", rc, "attention(portions and rows)");
+          took("[mfma, one launch]");
+          return true;
+        }
+      }
       // the portions first: with their keys cut into runs, the merge writes every row of the step, and
       // the rows of single tokens get their own result afterwards
       if (work.n_tiles && (head_dim == 64 || head_dim == 128) && work.n_tiles * heads < PAIRED_BELOW && work.tiles_small &&

@@ -767,7 +767,63 @@ class Attention final : public MixerPart {
   // fewest, and the rows of single-token entries.  Every attention part of a model asks for the
   // same lists; the first one builds them.
   void plan(StepPlan& plan) const override {
-    if (plan.decode_only() || plan.has("attention.tiles")) return;
+    if (!plan.decode_only() && !plan.has("attention.tiles")) plan_tiles(plan);
+    plan_runs(plan);
+  }
+  // The single-token rows of a step that the plain attention serves on the matrix cores, by records (Ops::plan_runs): all of a step of
+  // single tokens, or those beside portions in the portions' launch.  One list for all parts whose pages are the same.
+  std::string runs_key(int group) const {
+    return "attention.runs." + std::to_string(group) + "." + std::to_string(kv_heads * ((heads / kv_heads + 15) / 16)) + "." + std::to_string(heads);
+  }
+  void plan_runs(StepPlan& plan) const {
+    const Ops* ops = plan.ops();
+    const int P = plan.page_size();
+    if (general || gated || !ops || plan.act_dtype() != DType::BF16 || (head_dim != 64 && head_dim != 128) || P % 16 != 0) return;
+    if (!ops->use.fast_attention || !ops->use.early_page_ids || ops->use.force_decode_splits > 0) return;
+    if (plan.decode_only() && (!ops->use.fused_qk_decode || heads / kv_heads > 16)) return;
+    const int group = plan.group_of(this);
+    if (group < 0) return;
+    const std::string key = runs_key(group);
+    if (plan.has(key)) return;
+    const auto& entries = plan.entries();
+    std::vector<Ops::RunsRow> rows;
+    int n_tiles = 0, portion_context = 0, longest = 0;
+    for (size_t i = 0; i < entries.size(); ++i) {
+      const auto& e = entries[i];
+      if (e.n_tokens > 1) {
+        n_tiles += (e.n_tokens + PREFILL_TILE_SMALL - 1) / PREFILL_TILE_SMALL;
+        portion_context = std::max(portion_context, e.start + e.n_tokens);
+        continue;
+      }
+      const int first = window > 0 ? std::max(0, e.start - window + 1) / 16 : 0;
+      rows.push_back({e.row0, e.start, first, e.start / 16 + 1 - first, (int)i, plan.table_row(group, i)});
+      longest = std::max(longest, e.start + 1);
+    }
+    if (rows.empty()) return;
+    // What decides how a captured step launches holds for every replay of it, and so do the lists' sizes; what the lists hold is
+    // the same for a step that is captured and one that is not.
+    const auto blocks = [&](int context) { return (window > 0 ? std::min(context, window + 16) : context) / 16 + 1; };
+    const int most = plan.for_graph() ? plan.max_seq() : longest;
+    const int ways = kv_heads * ((heads / kv_heads + 15) / 16), units = ops->units();
+    double beside_us = 0.0;
+    if (!plan.decode_only()) {
+      if (!ops->use.paired_prefill || !ops->use.portion_splits || ops->use.force_paired_tiles >= 0) return;
+      const int context = plan.for_graph() ? plan.max_seq() : portion_context;
+      if (!Ops::portions_with_rows(n_tiles, (int)rows.size(), heads, kv_heads, context, most, window, units, head_dim)) return;
+      beside_us = Ops::portion_us(portion_context, window);
+    }
+    const int busy = plan.decode_only() ? 0 : n_tiles * heads;
+    const Ops::RunsLaunch launch = Ops::runs_launch((int)rows.size(), blocks(plan.max_seq()), blocks(most), ways, units, busy, plan.decode_only() ? 4 : 8);
+    int used = 0;
+    int* row_list = plan.ints(key + ".rows", 4 * rows.size());
+    int* runs = plan.ints(key, (size_t)launch.records * launch.stride);
+    const int places = Ops::plan_runs(rows, launch, ways, units, busy, beside_us, head_dim, P, runs, row_list, &used);
+    plan.set_value(key + ".stride", launch.stride);
+    plan.set_value(key + ".n", plan.for_graph() ? launch.records : used);
+    plan.set_value(key + ".merge", places > 0 ? 1 : 0);
+    plan.set_merges(places > 0);
+  }
+  void plan_tiles(StepPlan& plan) const {
     const auto& entries = plan.entries();
     size_t n_tiles = 0, n_small = 0, n_dec = 0;
     for (const auto& e : entries) {
@@ -826,6 +882,19 @@ class Attention final : public MixerPart {
       w.decode_rows = ctx.planned("attention.decode_rows");
       w.n_decode_rows = (int)ctx.planned_size("attention.decode_rows");
       w.portion_context = (int)ctx.value("attention.portion_context");
+    }
+    if (ctx.plan && ctx.engine && !general && !gated) {
+      const std::string key = runs_key(ctx.binding(this).first);
+      if (ctx.planned_size(key)) {
+        w.runs = ctx.planned(key);
+        w.n_runs = (int)ctx.value(key + ".n");
+        w.run_stride = (int)ctx.value(key + ".stride");
+        w.run_rows = ctx.planned(key + ".rows");
+        w.runs_with_tiles = !ctx.decode_only;
+        // a captured step of single tokens serves those that merge or those that do not; any other merges what needs it
+        const bool merge = !ctx.plan->for_graph() ? ctx.value(key + ".merge") != 0 : ctx.decode_only ? ctx.plan->merges() : true;
+        w.n_run_rows = merge ? (int)(ctx.planned_size(key + ".rows") / 4) : 0;
+      }
     }
     if (ctx.plan && ctx.plan->sized_for_longest()) {
       // a graph is being captured: what a replay launches must cover the longest sequence
