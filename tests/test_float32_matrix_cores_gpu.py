@@ -14,7 +14,7 @@ EPS = 2.0 ** -24
 
 @pytest.mark.parametrize("N,K", [(16, 4), (1000, 20), (65, 132), (1024, 1024), (36, 3076)])
 def test_product_at_the_edges_of_its_tiles(ops, N, K):  # noqa: F811
-    """Rows on either side of every tile's edge, runs of K that end inside a step of 16 or are empty, a last tile of few
+    """Rows on either side of every tile's edge, runs of K that end inside a step of 32 or are empty, a last tile of few
     columns.  A sum of K products in 32 bits, added in any order, is within (K + 1) 2^-24 of sum |a| |w|; the error is
     held to that bound, the row beyond the last is left alone, and a row alone has the bits of the row among others."""
     g = torch.Generator().manual_seed(N + K)
@@ -43,6 +43,32 @@ def test_product_at_the_edges_of_its_tiles(ops, N, K):  # noqa: F811
             gate, up = f64(full[:M, :N // 2]), f64(full[:M, N // 2:])
             want = gate / (1 + torch.exp(-gate)) * up
             assert ((f64(out) - want).abs() <= 16 * EPS * want.abs() + 1e-30).all(), M
+
+
+@pytest.mark.parametrize("M,N,K", [(7, 64, 20), (37, 132, 1056), (300, 96, 260)])
+def test_product_of_what_three_bfloat16_do_not_hold(ops, M, N, K):  # noqa: F811
+    """Operands from 1e-30 to the largest float, infinite ones and NaN, beside zeros: what float64 gives in 32 bits is what comes out, of
+    the same kind where it is not finite, within the bound of a 32-bit sum where it is.  Every row by every weight row's own kind."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g) * 1e-3
+    big = torch.finfo(torch.float32).max
+    for i, x in enumerate((1e-30, big, -big, float("inf"), float("nan"), 3.39e38)):
+        a[(3 * i) % M, (5 * i + 1) % K] = x
+    a[M // 2] *= 1e-30
+    w[3] *= 1e-6
+    w[5, :] = 0.0
+    w[7, 6 % K] = float("-inf")
+    w[9, K - 1] = float("nan")
+    ref = f64(a) @ f64(w).T
+    size = f64(a).abs() @ f64(w).abs().T
+    out = torch.empty(M, N, device="cuda")
+    ops.linear(dev(a), dev(w), out, "store")
+    out = f64(out)
+    fine = torch.isfinite(ref) & (ref.abs() < big)
+    assert fine.any() and not fine.all()
+    assert ((out - ref).abs() <= (K + 1) * EPS * size + 1e-36)[fine].all()
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    assert torch.equal(torch.isposinf(out), torch.isposinf(ref)) and torch.equal(torch.isneginf(out), torch.isneginf(ref))
 
 
 def case(entries, nh, nkv, hd, P, window, seed):

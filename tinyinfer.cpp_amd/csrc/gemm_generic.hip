@@ -6,11 +6,12 @@
 // Every output element sums its K products in an order that K alone decides,
 // so a token's result does not depend on what else is in the batch.
 //
-//   gemm_f32_kernel      float32 with rows of whole, aligned float4s: the 32-bit
-//                        matrix instructions (fused multiply-adds of full
-//                        precision, twice the rate of the vector unit's)
+//   gemm_f32_kernel      float32 with rows of whole, aligned float4s: matrix
+//                        instructions on the floats cut into three bfloat16
 //   gemm_generic_kernel  everything else: one fused multiply-add at a time, in
 //                        ascending k
+#include <float.h>
+#include <type_traits>
 #include "common.h"
 #include "tinyinfer_kernels.h"
 
@@ -114,29 +115,127 @@ static int launch(const void* A, const void* W, void* out, int M, int N, int K, 
 }
 
 // ------------------------------------------------------------------------------------------------ float32, matrix cores
-// A workgroup of eight wavefronts owns 16 RB weight rows x 16 NB tokens and cuts K into eight runs of whole 16s (the
-// same runs whatever M, N and the tile are), one a wavefront.  A wavefront walks its run in steps of 16: each lane
-// loads four consecutive k of one weight row and of one token straight from memory, and four v_mfma_f32_16x16x4_f32
-// take one of the four each (both operands are permuted alike, so every k meets itself).  The runs' sums meet in LDS
-// and are added in ascending order.
+// A workgroup of eight wavefronts owns 16 RB weight rows x 16 NB tokens and cuts K into eight runs of whole 32s (the
+// same runs whatever M, N and the tile are), one a wavefront.  The runs' sums meet in LDS and are added in ascending order.
 //
-// Few tokens: the weights' bytes bound it, each is read once, and eight runs keep eight wavefronts loading per tile.
-// Many: a 16x16x4 lasts 32 cycles, so 32-bit products are bound by the matrix cores' 157 TFLOP/s long before L1 or
-// LDS; operands need no staging, and what counts is that the tiles fill whole rounds of the compute units.
-// Measured inside a prompt of 300 tokens of Qwen3-0.6B's sizes, us (the generic kernel): 4096 x 1024 37.1 (157), [gate; up]
-// 6144 x 1024 47.8 (273), 1024 x 2048 and 1024 x 3072 29.4 on average (294), 151936 x 1024 1,055 (2,984); its products
-// together 5.1 ms (31.5).
+// A float is the sum of three bfloat16 (8 + 8 + 8 bits: the nearest, what is left cut to eight bits, and the rest, without a remainder),
+// so a product of floats is nine products of bfloat16, which v_mfma_f32_16x16x32_bf16 multiplies exactly and adds in 32 bits.  Six of them
+// are taken, the smallest first; the three left out are below 2^-22 of the product, where each addition already rounds at 2^-24 of the
+// sum, and 32 products share a rounding in place of one each.  Six of these take 96 cycles where the 32-bit instructions take 256.  Error
+// against 64 bits, 2-norm over 2-norm, with N(0, 1) tokens and N(0, 0.02) weights (by 32-bit instructions): K = 1024 1.6e-7 (2.1e-7),
+// 3072 3.0e-7 (3.6e-7), 12288 6.4e-7 (7.1e-7), 36 4.7e-8 (8.0e-8).
+// The matrix unit cuts what it adds downwards, which leaves every sum too low by some 5e-8 of the outputs' size: small, but the same way
+// in every layer (a prompt's logits 9.2e-7 off, by 32-bit instructions 8.1e-7).  The odd runs therefore take the tokens' negatives
+// and their sums are subtracted: the mean error is then 1e-9.
+// What the three pieces cannot hold (infinite, not a number, above the largest bfloat16) leaves a sum that is not finite; such an element
+// is computed again by fused multiply-adds.  (Below 2^-110 the last piece may lie below the normal numbers, 2^-133 at least.)
+//
+// A wavefront's rows come through its own part of LDS by direct loads, eight lanes to a row's 128 bytes, and are read back as the operands
+// lie.  (Loaded as operands straight into registers, neighbouring lanes ask for different rows: 64 cycles a load of 1 KiB whatever the
+// tile, four times what the direct loads take, and all that bounded these products.)  No barrier: a wavefront waits for its own loads,
+// and asks for the next step as soon as it has read one.  What bounds them now is the splitting (52 instructions a block of 16 rows
+// and step beside 16 cycles each of six matrix instructions a pair of blocks), and for 1,024 columns the ends: the first loads and the
+// sums' way through LDS are a third of the 13 us.
+// us a call, before (32-bit instructions, operands straight from memory) and now: 300 rows x 4096 x 1024 36.9 -> 25.7, [gate; up]
+// 6144 x 1024 47.9 -> 31.9, 1024 x 2048 24.3 -> 13.3, 1024 x 3072 33.6 -> 19.5, 151936 x 1024 1,040 -> 697; 53 rows 14.0 -> 9.2,
+// 20.6 -> 12.6, 13.1 -> 7.7, 16.9 -> 10.2, 242 -> 186; one row 8.4 -> 6.9, 12.7 -> 9.3, 11.5 -> 9.0 (1024 x 3072), 171 -> 127.
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gf4;
 #define GF_RUNS 8
+#define GF_STEP 32
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 gbf8;
+
+// Eight floats, times `sign` (1 or -1), as three bfloat16 each, the sum of which they are: the nearest, and twice the upper half of what
+// is left.
+struct Planes {
+  gbf8 p[3];
+};
+__device__ __forceinline__ Planes split_planes(const gf4& x, const gf4& y, float sign) {
+  const uint32_t flip = __float_as_uint(sign) & 0x80000000u;
+  uint32_t u[3][4];
+  float r[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    r[i] = x[i];
+    r[4 + i] = y[i];
+  }
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    uint32_t h[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      h[i] = j == 0 ? (__float_as_uint(r[i]) ^ flip) + 0x8000u : __float_as_uint(r[i]);
+      if (j == 0) r[i] = fmaf(r[i], sign, -__uint_as_float(h[i] & 0xffff0000u));
+      if (j == 1) r[i] -= __uint_as_float(h[i] & 0xffff0000u);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[j][i] = __builtin_amdgcn_perm(h[2 * i + 1], h[2 * i], 0x07060302u);
+  }
+  Planes s;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) s.p[j] = __builtin_bit_cast(gbf8, make_uint4(u[j][0], u[j][1], u[j][2], u[j][3]));
+  return s;
+}
+
+// One element by fused multiply-adds, in the same runs: where the three pieces do not hold an operand.
+__device__ __forceinline__ float dot_by_fma(const float* __restrict__ a, const float* __restrict__ w, int K, int run) {
+  float total = 0.f;
+  for (int k0 = 0; k0 < K; k0 += run) {
+    float s = 0.f;
+    for (int k = k0; k < min(K, k0 + run); ++k) s = fmaf(a[k], w[k], s);
+    total = k0 ? total + s : s;
+  }
+  return total;
+}
+
+// s_waitcnt with only vmcnt set (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14)
+template <int N> __device__ __forceinline__ void wait_vmcnt() {
+  static_assert(N >= 0 && N <= 63, "vmcnt counts to 63");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+struct Eight { gf4 x, y; };      // eight consecutive k of one row
+// N blocks of 16 rows of a stage, the first at LDS byte `at`, have arrived in registers when this returns; x, y: a lane's two pieces
+template <int N> __device__ __forceinline__ void read_blocks(Eight* e, unsigned x, unsigned y) {
+  static_assert(N >= 1 && N <= 4, "up to eight reads at a time");
+  if constexpr (N == 1)
+    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(e[0].x), "=&v"(e[0].y) : "v"(x), "v"(y) : "memory");
+  if constexpr (N == 2)
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %4 offset:2048\n\tds_read_b128 %3, %5 offset:2048\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(e[0].x), "=&v"(e[0].y), "=&v"(e[1].x), "=&v"(e[1].y) : "v"(x), "v"(y) : "memory");
+  if constexpr (N == 3)
+    asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %7\n\tds_read_b128 %2, %6 offset:2048\n\tds_read_b128 %3, %7 offset:2048\n\t"
+                 "ds_read_b128 %4, %6 offset:4096\n\tds_read_b128 %5, %7 offset:4096\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(e[0].x), "=&v"(e[0].y), "=&v"(e[1].x), "=&v"(e[1].y), "=&v"(e[2].x), "=&v"(e[2].y)
+                 : "v"(x), "v"(y) : "memory");
+  if constexpr (N == 4)
+    asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\tds_read_b128 %2, %8 offset:2048\n\tds_read_b128 %3, %9 offset:2048\n\t"
+                 "ds_read_b128 %4, %8 offset:4096\n\tds_read_b128 %5, %9 offset:4096\n\tds_read_b128 %6, %8 offset:6144\n\t"
+                 "ds_read_b128 %7, %9 offset:6144\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(e[0].x), "=&v"(e[0].y), "=&v"(e[1].x), "=&v"(e[1].y), "=&v"(e[2].x), "=&v"(e[2].y), "=&v"(e[3].x), "=&v"(e[3].y)
+                 : "v"(x), "v"(y) : "memory");
+}
+
+template <int RB, int NB, bool SW> struct F32Tile {
+  static constexpr int PL = SW ? 2 : 1;               // planes of weight rows: gate and up
+  static constexpr int TR = 16 * RB, TM = 16 * NB;
+  static constexpr int LD = TR + 4;                   // floats between tokens of a tile in LDS
+  static constexpr int BLOCKS = PL * RB + NB;         // of 16 rows: what a step of a wavefront reads
+  static constexpr int STEP_BYTES = BLOCKS * 2048;
+  static constexpr int STAGES = BLOCKS <= 2 ? 4 : BLOCKS <= 3 ? 3 : BLOCKS <= 4 ? 2 : 1;
+  static constexpr int SUMS = GF_RUNS * PL * TM * LD * 4, STAGED = GF_RUNS * STAGES * STEP_BYTES;
+  static constexpr int LDS = SUMS > STAGED ? SUMS : STAGED;
+};
 
 template <int RB, int NB, bool SW>
 __global__ void __launch_bounds__(64 * GF_RUNS)
 gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ out, int M, int N, int K,
                 long lda, int run, int m_tiles, int n_tiles, int epi, int wide_out) {
-  constexpr int PL = SW ? 2 : 1;                    // planes of weight rows: gate and up
-  constexpr int TR = 16 * RB, TM = 16 * NB;
-  constexpr int LD = TR + 4;                        // floats between tokens of a tile in LDS
-  __shared__ __attribute__((aligned(16))) float s_tile[GF_RUNS][PL][TM][LD];
+#if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass has no buffer descriptors)
+  using T = F32Tile<RB, NB, SW>;
+  constexpr int PL = T::PL, TR = T::TR, TM = T::TM, LD = T::LD, BLOCKS = T::BLOCKS, STAGES = T::STAGES;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  float (*s_tile)[PL][TM][LD] = reinterpret_cast<float (*)[PL][TM][LD]>(smem);
   // the dies take workgroups in turn: a die gets all token tiles of a set of weight rows, one after the other, so
   // that the rows come from memory once
   const int die = blockIdx.x & 7, local = blockIdx.x >> 3;
@@ -147,16 +246,6 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r16 = lane & 15, quad = lane >> 4;
 
-  // rows past the end repeat the last one; their sums are not stored
-  const float* wp[PL][RB];
-  const float* ap[NB];
-#pragma unroll
-  for (int p = 0; p < PL; ++p)
-#pragma unroll
-    for (int r = 0; r < RB; ++r) wp[p][r] = W + (size_t)(min(n0 + r * 16 + r16, N - 1) + p * N) * K + quad * 4;
-#pragma unroll
-  for (int b = 0; b < NB; ++b) ap[b] = A + (size_t)min(m0 + b * 16 + r16, M - 1) * lda + quad * 4;
-
   gf4 acc[PL][RB][NB];
 #pragma unroll
   for (int p = 0; p < PL; ++p)
@@ -165,62 +254,92 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
 #pragma unroll
       for (int b = 0; b < NB; ++b) acc[p][r][b] = gf4{0.f, 0.f, 0.f, 0.f};
 
-  struct Step { gf4 w[PL][RB], a[NB]; };
-  auto load = [&](Step& s, int k) {
+  const float sign = wave & 1 ? -1.f : 1.f;
+  // one step's products: blocks of weight rows (gate, then up), then blocks of tokens
+  const auto multiply = [&](const Eight* e) {
+    Planes w[PL * RB];
 #pragma unroll
-    for (int p = 0; p < PL; ++p)
+    for (int r = 0; r < PL * RB; ++r) w[r] = split_planes(e[r].x, e[r].y, 1.f);
 #pragma unroll
-      for (int r = 0; r < RB; ++r) s.w[p][r] = *reinterpret_cast<const gf4*>(wp[p][r] + k);
+    for (int b = 0; b < NB; ++b) {
+      const Planes a = split_planes(e[PL * RB + b].x, e[PL * RB + b].y, sign);
 #pragma unroll
-    for (int b = 0; b < NB; ++b) s.a[b] = *reinterpret_cast<const gf4*>(ap[b] + k);
-  };
-  auto multiply = [&](const Step& s) {
+      for (int j = 0; j < 6; ++j) {
+        constexpr int WJ[6] = {2, 0, 1, 1, 0, 0}, AJ[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int p = 0; p < PL; ++p)
-#pragma unroll
-        for (int r = 0; r < RB; ++r)
-#pragma unroll
-          for (int b = 0; b < NB; ++b)
-            acc[p][r][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(s.w[p][r][j], s.a[b][j], acc[p][r][b], 0, 0, 0);
-  };
-  const int k0 = wave * run, k1 = min(K, k0 + run);
-  const int steps = k1 > k0 ? (k1 - k0) / 16 : 0;   // whole steps; K's last 4, 8 or 12 are a step of their own
-  // loads run DEPTH steps ahead; past the run's end they repeat its last step
-  constexpr int DEPTH = (PL * RB + NB <= 3) ? 8 : (PL * RB + NB <= 6) ? 4 : 2;
-  if (steps > 0) {
-    Step s[DEPTH];
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) load(s[d], k0 + 16 * min(d, steps - 1));
-    int i = 0;
-    for (; i + DEPTH <= steps; i += DEPTH) {
-#pragma unroll
-      for (int d = 0; d < DEPTH; ++d) {
-        multiply(s[d]);
-        load(s[d], k0 + 16 * min(i + DEPTH + d, steps - 1));
-        __builtin_amdgcn_sched_barrier(0);          // the loads leave here, not where the next product needs them
+        for (int r = 0; r < PL * RB; ++r)
+          acc[r / RB][r % RB][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[r].p[WJ[j]], a.p[AJ[j]], acc[r / RB][r % RB][b], 0, 0, 0);
       }
     }
+  };
+  const int k0 = wave * run, k1 = min(K, k0 + run);
+  const int steps = k1 > k0 ? (k1 - k0) / GF_STEP : 0;   // whole steps; what is left of K is a step of its own
+  if (steps > 0) {
+    // A load of 1 KiB covers eight rows of a block: eight lanes a row, its 128 bytes in pieces of 16, piece c of row r in place
+    // c ^ (r & 7), so that the sixteen rows that are read together lie in different banks.  Rows past the end repeat the last one;
+    // their sums are not stored.
+    unsigned voff[BLOCKS][2];
+    const int lr = lane >> 3, piece = (lane & 7) ^ lr;
 #pragma unroll
-    for (int d = 0; d < DEPTH; ++d)
-      if (i + d < steps) multiply(s[d]);
-  }
-  if (k1 > k0 && (k1 - k0) % 16) {
-    const int k = k0 + steps * 16;
-    Step s;
-    if (k + quad * 4 < K) {                         // K is a multiple of 4: a lane's four are there or not
-      load(s, k);
-    } else {
+    for (int i = 0; i < BLOCKS; ++i)
 #pragma unroll
-      for (int p = 0; p < PL; ++p)
+      for (int h = 0; h < 2; ++h)
+        voff[i][h] = (i < PL * RB ? (unsigned)min((i % RB) * 16 + h * 8 + lr, N - 1 - n0) * (unsigned)(K * 4)
+                                  : (unsigned)min((i - PL * RB) * 16 + h * 8 + lr, M - 1 - m0) * (unsigned)(lda * 4)) + piece * 16;
+    const auto rows_at = [](const float* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
+    const auto rsW = rows_at(W + (size_t)n0 * K + k0), rsU = rows_at(W + (size_t)(n0 + (SW ? N : 0)) * K + k0);
+    const auto rsA = rows_at(A + (size_t)m0 * lda + k0);
+    unsigned char* mine = smem + wave * STAGES * T::STEP_BYTES;
+    const auto load = [&](int step, unsigned stage) {
 #pragma unroll
-        for (int r = 0; r < RB; ++r) s.w[p][r] = gf4{0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < BLOCKS; ++i)
 #pragma unroll
-      for (int b = 0; b < NB; ++b) s.a[b] = gf4{0.f, 0.f, 0.f, 0.f};
+        for (int h = 0; h < 2; ++h) {
+          auto* dst = (__attribute__((address_space(3))) void*)(mine + stage + i * 2048 + h * 1024);      // the same in every lane
+          if (i < RB) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsW, dst, 16, voff[i][h], step * GF_STEP * 4, 0, 0);
+          else if (i < PL * RB) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsU, dst, 16, voff[i][h], step * GF_STEP * 4, 0, 0);
+          else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, dst, 16, voff[i][h], step * GF_STEP * 4, 0, 0);
+        }
+    };
+    const unsigned at = (unsigned)(size_t)mine + r16 * 128, x = at + (((2 * quad) ^ (r16 & 7)) << 4), y = at + (((2 * quad + 1) ^ (r16 & 7)) << 4);
+#pragma unroll
+    for (int d = 0; d < STAGES; ++d)
+      if (d < steps) load(d, d * T::STEP_BYTES);
+    unsigned stage = 0;
+    for (int i = 0; i < steps; ++i) {
+      // this step's loads are back; those of the steps behind it may still be out
+      const int behind = min(STAGES, steps - i) - 1;      // the same in every lane
+      if (STAGES >= 4 && behind == 3) wait_vmcnt<STAGES >= 4 ? 6 * BLOCKS : 0>();
+      else if (STAGES >= 3 && behind == 2) wait_vmcnt<STAGES >= 3 ? 4 * BLOCKS : 0>();
+      else if (STAGES >= 2 && behind == 1) wait_vmcnt<STAGES >= 2 ? 2 * BLOCKS : 0>();
+      else wait_vmcnt<0>();
+      Eight e[BLOCKS];
+      constexpr int R = BLOCKS % 4;
+#pragma unroll
+      for (int b = 0; b + 4 <= BLOCKS; b += 4) read_blocks<4>(e + b, x + stage + b * 2048, y + stage + b * 2048);
+      if constexpr (R) read_blocks<(R ? R : 1)>(e + BLOCKS - R, x + stage + (BLOCKS - R) * 2048, y + stage + (BLOCKS - R) * 2048);
+      if (i + STAGES < steps) load(i + STAGES, stage);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(e);
+      stage = stage == (STAGES - 1) * T::STEP_BYTES ? 0 : stage + T::STEP_BYTES;
     }
-    multiply(s);
   }
+  if (k1 > k0 && (k1 - k0) % GF_STEP) {
+    const int k = k0 + steps * GF_STEP + quad * 8;
+    const auto part = [&](const float* p) {                // K is a multiple of 4: a lane's fours are there or not
+      Eight e = {gf4{0.f, 0.f, 0.f, 0.f}, gf4{0.f, 0.f, 0.f, 0.f}};
+      if (k < K) e.x = *reinterpret_cast<const gf4*>(p + k);
+      if (k + 4 < K) e.y = *reinterpret_cast<const gf4*>(p + k + 4);
+      return e;
+    };
+    Eight e[BLOCKS];
+#pragma unroll
+    for (int i = 0; i < BLOCKS; ++i)
+      e[i] = part(i < PL * RB ? W + (size_t)(min(n0 + (i % RB) * 16 + r16, N - 1) + (i / RB) * N) * K
+                              : A + (size_t)min(m0 + (i - PL * RB) * 16 + r16, M - 1) * lda);
+    multiply(e);
+  }
+  __syncthreads();                                         // the stages are free
   // a lane holds four weight rows of one token
 #pragma unroll
   for (int p = 0; p < PL; ++p)
@@ -236,10 +355,23 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
     const int m = m0 + t, n = n0 + c;
     if (m >= M || n >= N) continue;
     gf4 v = *reinterpret_cast<const gf4*>(&s_tile[0][0][t][c]);
-    for (int w = 1; w < runs; ++w) v += *reinterpret_cast<const gf4*>(&s_tile[w][0][t][c]);
+    for (int w = 1; w < runs; ++w) {
+      const gf4 x = *reinterpret_cast<const gf4*>(&s_tile[w][0][t][c]);
+      v = w & 1 ? v - x : v + x;
+    }
+    const auto settle = [&](gf4& x, size_t row0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (!(fabsf(x[i]) <= FLT_MAX) && n + i < N) x[i] = dot_by_fma(A + (size_t)m * lda, W + (row0 + n + i) * K, K, run);
+    };
+    settle(v, 0);
     if (SW) {
       gf4 u = *reinterpret_cast<const gf4*>(&s_tile[0][PL - 1][t][c]);
-      for (int w = 1; w < runs; ++w) u += *reinterpret_cast<const gf4*>(&s_tile[w][PL - 1][t][c]);
+      for (int w = 1; w < runs; ++w) {
+        const gf4 x = *reinterpret_cast<const gf4*>(&s_tile[w][PL - 1][t][c]);
+        u = w & 1 ? u - x : u + x;
+      }
+      settle(u, N);
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[i] = v[i] / (1.0f + expf(-v[i])) * u[i];
     }
@@ -257,6 +389,7 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
         if (n + i < N) o[i] = epi == TI_EPI_ADD_F32 ? o[i] + v[i] : v[i];
     }
   }
+#endif
 }
 
 static int compute_units() {
@@ -271,9 +404,9 @@ static int compute_units() {
 }
 
 // The tile: of those that are built, the one whose rounds of the compute units take the least time in all.  A round costs a
-// start, its products (RB NB) and its operands' loads (RB + NB, four times a product's weight each: sixteen lines a load).
+// start, its products (RB NB) and its operands (RB + NB blocks to split, four times a product's weight each).
 // Fitted to 1 to 1,000 rows times the weights of Qwen3-0.6B's sizes: the tile it picks is on average 0.9 % slower than the
-// fastest (300 x 1024 x 3072: 32 x 48 35.7 us, 16 x 80 40.8).
+// fastest (300 x 1024 x 3072: 32 x 48 20.2 us, 16 x 80 22.4), and 0.3 % over those and the 1.7B to 4B sizes with the present kernel.
 static long f32_tile_cost(int rb, int nb, bool sw, int M, int N, int units) {
   const long tiles = (long)((M + 16 * nb - 1) / (16 * nb)) * ((N + 16 * rb - 1) / (16 * rb));
   const int pl = sw ? 2 : 1;
@@ -296,22 +429,30 @@ static int launch_f32(const float* A, const float* W, float* out, int M, int N, 
     }
   }
   const int wide_out = N % 4 == 0 && ((uintptr_t)out & 15) == 0;
-  const int run = ((K + GF_RUNS - 1) / GF_RUNS + 15) / 16 * 16;
+  const int run = ((K + GF_RUNS - 1) / GF_RUNS + GF_STEP - 1) / GF_STEP * GF_STEP;
   const int m_tiles = (M + 16 * nb - 1) / (16 * nb), n_tiles = (N + 16 * rb - 1) / (16 * rb);
   const long grid = m_tiles == 1 ? n_tiles : (long)((n_tiles + 7) / 8) * 8 * m_tiles;
+#define GF_LAUNCH(R, B, S)                                                                                                \
+  do {                                                                                                                    \
+    constexpr int lds = F32Tile<R, B, S>::LDS;                                                                            \
+    static const hipError_t room = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_f32_kernel<R, B, S>),           \
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);                  \
+    TI_REQUIRE(room == hipSuccess, "gemm_generic: %d bytes of LDS: %s", lds, hipGetErrorString(room));                    \
+    gemm_f32_kernel<R, B, S><<<(unsigned)grid, 64 * GF_RUNS, lds, stream>>>(A, W, out, M, N, K, lda, run, m_tiles, n_tiles, epi, wide_out); \
+  } while (0)
 #define GF_CASE(R, B)                                                                                                     \
   if (rb == R && nb == B) {                                                                                               \
     if (sw) {                                                                                                             \
-      if constexpr (R * B <= 8)                                                                                          \
-        gemm_f32_kernel<R, B, true><<<(unsigned)grid, 64 * GF_RUNS, 0, stream>>>(A, W, out, M, N, K, lda, run, m_tiles, n_tiles, epi, wide_out); \
+      if constexpr (R * B <= 8) GF_LAUNCH(R, B, true);                                                                    \
     } else {                                                                                                              \
-      gemm_f32_kernel<R, B, false><<<(unsigned)grid, 64 * GF_RUNS, 0, stream>>>(A, W, out, M, N, K, lda, run, m_tiles, n_tiles, epi, wide_out); \
+      GF_LAUNCH(R, B, false);                                                                                             \
     }                                                                                                                     \
     return 0;                                                                                                             \
   }
   GF_CASE(1, 1) GF_CASE(1, 2) GF_CASE(1, 3) GF_CASE(1, 4) GF_CASE(1, 5) GF_CASE(2, 2) GF_CASE(2, 3) GF_CASE(2, 4) GF_CASE(2, 5)
   GF_CASE(4, 2) GF_CASE(4, 4)
 #undef GF_CASE
+#undef GF_LAUNCH
   return 1;
 }
 
@@ -323,7 +464,8 @@ extern "C" int ti_gemm_generic(int dtype, const void* A, const void* W, void* ou
   if (M == 0) return 0;
   int rc;
   // rows of whole float4s on 16-byte boundaries (what K, lda and the addresses say, never M: a token's sum keeps its order)
-  const bool f4 = dtype == TI_F32 && K % 4 == 0 && lda % 4 == 0 &&
+  // (and a tile's rows within 2 GiB, which is what a buffer's descriptor spans)
+  const bool f4 = dtype == TI_F32 && K % 4 == 0 && lda % 4 == 0 && lda < (1 << 22) &&
                   (((uintptr_t)A | (uintptr_t)W) & 15) == 0;
   if (f4 && epi >= TI_EPI_STORE_F32 && epi <= TI_EPI_RELU2 && epi != TI_EPI_QKV_PREP)
     rc = launch_f32((const float*)A, (const float*)W, (float*)out, M, N, K, lda, epi, stream);
