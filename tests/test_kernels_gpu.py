@@ -565,6 +565,34 @@ def test_sample_with_more_equal_logits_at_the_cut_than_are_collected(ops):
     check_draws(row, 1.0, 30, 1.0, us, got)
 
 
+@pytest.mark.parametrize("V,skip", [(151936, 0), (151935, 0), (20002, 2), (20000, 1), (1500, 0)])
+def test_sample_rows_whose_first_bin_holds_too_many(ops, V, skip):
+    """Logits all of a size (around 1,000: a bin of the first count holds most of the row) beside ordinary rows, cuts above and
+    below what a thread each sorts, rows of no whole float4s or off their boundaries: the draws lie where the plain CDF puts
+    them and are the walking kernel's (a sum taken in another order may move one edge a setting)."""
+    g = torch.Generator().manual_seed(V + skip)
+    us = np.linspace(0.01, 0.99, 12).astype(np.float32)
+    rows = torch.randn(2, V, generator=g) * 2
+    rows[0] += 1000.0
+    rows[0, V // 3:V // 3 + 9] = rows[0].topk(30).values[-1]
+    flat = torch.zeros(skip + 12 * V)
+    flat[skip:] = rows.repeat(6, 1).reshape(-1)
+    logits = dev(flat)[skip:].view(12, V)
+    for T, top_k, top_p in ((0.8, 512, 1.0), (1.0, 30, 0.9), (1.5, 1400, 0.95), (0.0, 5, 1.0)):
+        got = run_sample(ops, logits, T, top_k, top_p, us.tolist())
+        for i in range(2):
+            if T > 0:
+                check_draws(rows[i], T, top_k, top_p, us[i::2], got[i::2])
+            else:
+                assert set(got[i::2]) == {int(rows[i].argmax())}
+        ops.use_radix_sample = False
+        try:
+            walked = run_sample(ops, logits, T, top_k, top_p, us.tolist())
+        finally:
+            ops.use_radix_sample = True
+        assert sum(a != b for a, b in zip(got, walked)) <= 1, (T, top_k, top_p, got, walked)
+
+
 # ------------------------------------------------- bfloat16 matrix-core products
 @pytest.mark.parametrize("M,N,K", [
     (1, 48, 64), (5, 261, 1024), (8, 1000, 96), (16, 17, 200), (17, 130, 72), (33, 64, 3072), (64, 151, 256),

@@ -265,30 +265,36 @@ sample_kernel(const float* __restrict__ logits, const float* __restrict__ temp, 
   sample_row_by_bisection(logits, temp, top_k, top_p, uni, out, V, blockIdx.x);
 }
 
-// ------------------------------------------------------------ the same draw in four short kernels
+// ------------------------------------------------------------ the same draw in two short kernels
 // A row of 151,936 logits cut to its 512 largest: the kernel above takes 0.9 ms (1.8 with a top-p
 // cut), as long as a whole decode step, because one workgroup reads the row once per bit of the
-// answer.  Here the k-th largest key is found by radix and many workgroups share a row:
-//   pass 0  counts the keys of a row by their upper 11 bits (counts in LDS first, then added to the
-//           row's histogram in memory: sums of integers, the same in any order);
-//   pass 1  finds the bin that holds the k-th largest and counts its keys by their next 11 bits;
-//   pass 2  collects the keys at or above the 22-bit prefix that holds the k-th largest: the k - 1
-//           above it and those that share its prefix (few: for logits between 16 and 32 a prefix
-//           is 0.002 wide), as (key, index) pairs;
-//   finish  one workgroup per row sorts the collected pairs by (logit down, index up), cuts at the
-//           k-th key (equals stay), sums the weights in that order for the top-p cut, sorts what
-//           is left by index and draws by inverse CDF.  Sums are scans of a fixed shape.
+// answer.  Here the k-th largest key is found by radix, and many workgroups share a row:
+//   part    a workgroup holds S_SPAN keys of a row in registers, finds its own k-th largest (counts of the keys'
+//           upper 12 bits in LDS, and of the next 10 and the last 10 where a bin holds too many) and leaves
+//           what is at or above it, or in its bin, as (key, index) pairs: the row's k largest are among them.  It says as
+//           well from where up its own share of the k, k / parts, lies;
+//   finish  one workgroup per row: at least k keys lie at or above the least of the parts' shares, so it takes those pairs alone (some
+//           700 of 10,000 for k = 512), finds the k-th key among them the same way, keeps it and those above,
+//           sorts what is kept by logit where there is a top-p cut and sums the weights in that order, sorts
+//           what is left by index and draws by inverse CDF.  Sums are scans of a fixed shape.
 // It draws what the kernel above draws, up to the rounding of sums that are taken in another order.
-// Rows that it does not serve (no top-k cut, a cut beyond S_MAX_K, more than S_CAND keys collected:
-// thousands of equal logits at the cut) are left to that kernel's walk, inside the last kernel.
-// The row's words of the workspace start at zero and are left at zero.
-#define S_BINS 2048
-#define S_CAND 4096                              // pairs a row may collect (and the finish sorts in LDS)
-#define S_MAX_K 3584                             // the largest cut served: room for equals and prefix-mates
-#define S_LOADS 8                                // loads of a thread that are under way at a time
-#define S_STAGE 512                              // pairs a workgroup gathers in LDS before it asks for room
-#define S_HEAD_WORDS (2 * S_BINS + 64)           // two histograms, the count of pairs, pass 1's bin (and padding)
-#define S_ROW_WORDS (S_HEAD_WORDS + 2 * S_CAND)
+// Rows that it does not serve (no top-k cut, a cut beyond S_MAX_K, more than S_CAND keys that are equal
+// at the cut) are left to that kernel's walk, inside the last kernel.
+//
+// 64 rows of 151,936, greedy, top-k 50 and top-p, 512 and 20 in turn, us: three passes over the row's memory and a finish
+// with two sorts by rank 9.9 + 12.9 + 14.3 + 23.0; this 13.4 + 16.8.  Of the first, 9.5 are the loads and the counts (39 MB, and a
+// workgroup's counts wait for its loads); the second is a chain of some thirty short steps with a barrier each (a greedy row's 6.8).
+// Parts of 8,192 keys 13.1 + 18.1; without the shares the finish's counts of 10,000 pairs a row took 3 us more.
+#define S_BITS 12
+#define S_BINS (1 << S_BITS)
+#define S_BITS2 10                               // the next digits
+#define S_BINS2 (1 << S_BITS2)
+#define S_CAND 4096                              // pairs a workgroup may leave of its part, and the finish may keep
+#define S_MAX_K 3584                             // the largest cut served: room for equals and for a bin's others
+#define S_NT 512
+#define S_LOADS 20                               // keys a thread holds
+#define S_SPAN (S_NT * S_LOADS)
+static_assert(S_BITS + 2 * S_BITS2 == 32, "a key is three digits");
 
 __device__ __forceinline__ float key_value(uint32_t key) {
   return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key);
@@ -299,154 +305,183 @@ __device__ __forceinline__ int served_cut(const float* temp, const int* top_k, i
   return (k > 0 && k < V && k <= S_MAX_K) ? k : 0;
 }
 
-// Which of the S_BINS bins holds the k-th largest key, and how many keys lie in the bins above it.  Every
-// thread of the workgroup calls it (256 or more: thread t < 256 owns bins 8 t .. 8 t + 7) and gets both.
-// k beyond the number of keys: the lowest bin that holds a key.  No keys: bin -1.
-__device__ void bin_of_kth(const int* __restrict__ hist, int k, int* s_sum, int* s_above, int* s_res, int& bin, int& above) {
-  const int t = threadIdx.x;
-  const bool own = t < 256;
-  int c[8], mine = 0;
+// The sum of v over this lane and those below it: shifts inside rows of 16 lanes and two broadcasts, no trip through LDS.
+__device__ __forceinline__ int wave_prefix(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);      // row_shr:1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);      // lane 15 of a row to the next, 31 to the upper half
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return v;
+}
+
+// Which of BINS counts in LDS holds the k-th largest key, how many keys lie in the bins above it, and how many in it.  Every
+// thread of the workgroup's NT calls it and gets all three; what it leaves in the counts is zero.
+// k beyond the number of keys: the lowest bin that holds a key.  No keys: bin -1.  share_bin: the bin of the share-th largest, 0 where
+// there are fewer.
+template <int BINS, int NT>
+__device__ void bin_of_kth(int* s_bins, int k, int* s_wave, int* s_res, int& bin, int& above, int& in, int share = 0, int* share_bin = nullptr) {
+  constexpr int OWN = BINS / NT, WAVES = NT / TI_WAVE;
+  const int t = threadIdx.x, lane = t & (TI_WAVE - 1), wave = t / TI_WAVE;
+  int* own = s_bins + BINS - OWN * (t + 1);        // the first threads own the highest bins
+  int c[OWN], mine = 0;
+  if constexpr (OWN % 4 == 0) {
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    c[j] = own ? hist[8 * t + j] : 0;
-    mine += c[j];
+    for (int j = 0; j < OWN; j += 4) {
+      int4* p = reinterpret_cast<int4*>(own + j);
+      const int4 q = *p;
+      *p = make_int4(0, 0, 0, 0);
+      c[j] = q.x, c[j + 1] = q.y, c[j + 2] = q.z, c[j + 3] = q.w;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < OWN; ++j) {
+      c[j] = own[j];
+      own[j] = 0;
+    }
   }
-  if (own) s_sum[t] = mine;
-  if (t == 0) s_res[0] = -1, s_res[1] = 0;
+#pragma unroll
+  for (int j = 0; j < OWN; ++j) mine += c[j];
+  int run = wave_prefix(mine), total = 0;
+  if (lane == TI_WAVE - 1) s_wave[wave] = run;
+  run -= mine;                                     // keys in the bins above this thread's
+  if (t == 0) s_res[0] = -1, s_res[1] = 0, s_res[2] = 0, s_res[3] = 0;
   __syncthreads();
-  if (t < TI_WAVE) {
-    int q[4], s4 = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      q[j] = s_sum[4 * t + j];
-      s4 += q[j];
-    }
-    int suf = s4;                                  // keys of the owners that lanes >= t stand for
-#pragma unroll
-    for (int o = 1; o < TI_WAVE; o <<= 1) {
-      const int v = __shfl_down(suf, o, TI_WAVE);
-      if (t + o < TI_WAVE) suf += v;
-    }
-    int run = suf - s4;
-#pragma unroll
-    for (int j = 3; j >= 0; --j) {
-      s_above[4 * t + j] = run;                    // keys in the bins of owners beyond 4 t + j
-      run += q[j];
-    }
-    if (t == 0) s_above[256] = run;                // all keys
+  for (int w = 0; w < WAVES; ++w) {
+    const int n = s_wave[w];
+    if (w < wave) run += n;
+    total += n;
   }
-  __syncthreads();
-  const int total = s_above[256];
   const int kk = k < total ? k : total;
-  if (own && kk >= 1) {
-    int run = s_above[t];
+  if (kk >= 1) {
 #pragma unroll
-    for (int j = 7; j >= 0; --j) {
-      if (run < kk && run + c[j] >= kk) s_res[0] = 8 * t + j, s_res[1] = run;
+    for (int j = OWN - 1; j >= 0; --j) {
+      if (run < kk && run + c[j] >= kk) s_res[0] = BINS - OWN * (t + 1) + j, s_res[1] = run, s_res[2] = c[j];
+      if (run < share && run + c[j] >= share) s_res[3] = BINS - OWN * (t + 1) + j;
       run += c[j];
     }
   }
   __syncthreads();
   bin = s_res[0];
   above = s_res[1];
+  in = s_res[2];
+  if (share_bin) *share_bin = s_res[3];
   __syncthreads();
 }
 
-template <int PASS>
-__global__ void __launch_bounds__(256)
-sample_pass_kernel(const float* __restrict__ logits, const float* __restrict__ temp, const int* __restrict__ top_k,
-                   int* __restrict__ scratch, int V) {
-  __shared__ int s_hist[PASS == 2 ? 1 : S_BINS];
-  __shared__ unsigned long long s_stage[PASS == 2 ? S_STAGE : 1];
-  __shared__ int s_sum[256], s_above[257], s_res[2], s_count, s_base;
-  const int r = blockIdx.y;
+// Where this lane's `n` entries go behind *s_count: one counter's step a wavefront.  All lanes call it.
+__device__ __forceinline__ int next_places(int* s_count, int n) {
+  const int upto = wave_prefix(n), all = __builtin_amdgcn_readlane(upto, TI_WAVE - 1);
+  if (all == 0) return 0;
+  int at = 0;
+  if ((threadIdx.x & (TI_WAVE - 1)) == 0) at = atomicAdd(s_count, all);
+  return __builtin_amdgcn_readfirstlane(at) + upto - n;
+}
+
+// grid (parts of `span` keys, rows), span a multiple of 4, at most S_SPAN.  WIDE: rows of whole float4s on their boundaries, four
+// neighbours a load.  counts [row][parts][2] (pairs, the key from which the part's share lies), pairs [row][parts][S_CAND]
+// (key << 32 | ~index).  (64 registers a thread: four workgroups to a unit, so that 64 rows of 15 parts are one round.)
+template <bool WIDE>
+__global__ void __launch_bounds__(S_NT)
+sample_part_kernel(const float* __restrict__ logits, const float* __restrict__ temp, const int* __restrict__ top_k,
+                   int2* __restrict__ counts, unsigned long long* __restrict__ pairs, int V, int span) {
+  __shared__ __attribute__((aligned(16))) int s_bins[S_BINS];
+  __shared__ int s_wave[S_NT / TI_WAVE], s_res[4], s_count;
+  const int r = blockIdx.y, t = threadIdx.x;
   const int k = served_cut(temp, top_k, r, V);
   if (k == 0) return;                              // the whole workgroup
   const float* row = logits + (size_t)r * V;
-  int* hist1 = scratch + (size_t)r * S_ROW_WORDS;
-  int* hist2 = hist1 + S_BINS;
-  int* n_cand = hist2 + S_BINS;
-  unsigned long long* cand = reinterpret_cast<unsigned long long*>(hist1 + S_HEAD_WORDS);
-  int b1 = 0, above1 = 0, b2 = 0, above2 = 0;
-  if (PASS == 1) {
-    bin_of_kth(hist1, k, s_sum, s_above, s_res, b1, above1);
-    if (blockIdx.x == 0 && threadIdx.x == 0) n_cand[1] = b1, n_cand[2] = above1;   // pass 2 need not look again
-    if (b1 < 0) return;                            // a row of NaN
-  }
-  if (PASS == 2) {
-    b1 = n_cand[1];
-    above1 = n_cand[2];
-    if (b1 < 0) return;
-    bin_of_kth(hist2, k - above1, s_sum, s_above, s_res, b2, above2);
-    if (b2 < 0) return;
-    if (threadIdx.x == 0) s_count = 0;
-    __syncthreads();
-  } else {
-    for (int i = threadIdx.x; i < S_BINS; i += 256) s_hist[i] = 0;
-    __syncthreads();
-  }
-  const uint32_t prefix = ((uint32_t)b1 << 11) | (uint32_t)b2;
-  // S_LOADS loads are under way at a time: one load a turn leaves a wavefront waiting for memory 37 times over
-  for (int base = blockIdx.x * (256 * S_LOADS) + threadIdx.x; base < V; base += gridDim.x * (256 * S_LOADS)) {
-    float v[S_LOADS];
+  const size_t part = (size_t)r * gridDim.x + blockIdx.x;
+  const int base = blockIdx.x * span, end = min(V, base + span);
+  const float none = __uint_as_float(0x7fc00000u);
+  float v[S_LOADS];
+  // key u of a thread is the row's base + place(u)
+  const auto place = [&](int u) { return WIDE ? S_NT * (u & ~3) + 4 * t + (u & 3) : S_NT * u + t; };
 #pragma unroll
-    for (int u = 0; u < S_LOADS; ++u) v[u] = base + 256 * u < V ? row[base + 256 * u] : __uint_as_float(0x7fc00000u);
-#pragma unroll
-    for (int u = 0; u < S_LOADS; ++u) {
-      if (!(v[u] == v[u])) continue;               // NaN is never drawn
-      const int i = base + 256 * u;
-      const uint32_t key = order_key(v[u]);
-      if (PASS == 0) {
-        atomicAdd(&s_hist[key >> 21], 1);
-      } else if (PASS == 1) {
-        if ((key >> 21) == (uint32_t)b1) atomicAdd(&s_hist[(key >> 10) & (S_BINS - 1)], 1);
-      } else if ((key >> 10) >= prefix) {
-        const unsigned long long pair = ((unsigned long long)key << 32) | (uint32_t)~i;
-        const int at = atomicAdd(&s_count, 1);
-        if (at < S_STAGE) {
-          s_stage[at] = pair;
-        } else {                                   // more than the stage holds: one by one
-          const int g = atomicAdd(n_cand, 1);
-          if (g < S_CAND) cand[g] = pair;
-        }
-      }
+  for (int u = 0; u < S_LOADS; u += WIDE ? 4 : 1) {
+    const int i = base + place(u);
+    if (WIDE) {
+      const float4 q = i < end ? *reinterpret_cast<const float4*>(row + i) : make_float4(none, none, none, none);
+      v[u] = q.x, v[u + 1] = q.y, v[u + 2] = q.z, v[u + 3] = q.w;
+    } else {
+      v[u] = i < end ? row[i] : none;
     }
   }
+  for (int i = t; i < S_BINS / 4; i += S_NT) reinterpret_cast<int4*>(s_bins)[i] = make_int4(0, 0, 0, 0);
+  if (t == 0) s_count = 0;
   __syncthreads();
-  if (PASS == 2) {
-    const int mine = min(s_count, S_STAGE);
-    if (threadIdx.x == 0 && mine > 0) s_base = atomicAdd(n_cand, mine);
-    __syncthreads();
-    for (int i = threadIdx.x; i < mine; i += 256)
-      if (s_base + i < S_CAND) cand[s_base + i] = s_stage[i];
-  } else {
-    int* hist = PASS == 0 ? hist1 : hist2;
-    for (int i = threadIdx.x; i < S_BINS; i += 256)
-      if (s_hist[i]) atomicAdd(&hist[i], s_hist[i]);
+  uint32_t key[S_LOADS];                           // 0, which is no number's: NaN is never drawn
+#pragma unroll
+  for (int u = 0; u < S_LOADS; ++u) {
+    key[u] = v[u] == v[u] ? order_key(v[u]) : 0;
+    if (key[u]) atomicAdd(&s_bins[key[u] >> (32 - S_BITS)], 1);
   }
+  __syncthreads();
+  int bin, above, in, share_bin, taken = 0, need = k, shift = 32 - S_BITS;      // taken: keys above the prefix
+  bin_of_kth<S_BINS, S_NT>(s_bins, need, s_wave, s_res, bin, above, in, (k + gridDim.x - 1) / gridDim.x, &share_bin);
+  if (bin < 0) {
+    if (t == 0) counts[part] = make_int2(0, 0);
+    return;
+  }
+  uint32_t prefix = bin;
+  // few more than k is good enough: the finish looks at 15 such parts of a row of 151,936
+  const int enough = min(S_CAND, max(1024, k + 512));
+  while (above + taken + in > enough && shift > 0) {
+    taken += above;
+    need -= above;
+#pragma unroll
+    for (int u = 0; u < S_LOADS; ++u)
+      if (key[u] && (key[u] >> shift) == prefix) atomicAdd(&s_bins[(key[u] >> (shift - S_BITS2)) & (S_BINS2 - 1)], 1);
+    __syncthreads();
+    bin_of_kth<S_BINS2, S_NT>(s_bins, need, s_wave, s_res, bin, above, in);
+    prefix = (prefix << S_BITS2) | (uint32_t)bin;
+    shift -= S_BITS2;
+  }
+  unsigned long long* mine = pairs + part * S_CAND;
+  const uint32_t least = max(prefix << shift, 1u);
+  int n = 0;
+#pragma unroll
+  for (int u = 0; u < S_LOADS; ++u) n += key[u] >= least ? 1 : 0;
+  int at = next_places(&s_count, n);
+#pragma unroll
+  for (int u = 0; u < S_LOADS; ++u)
+    if (key[u] >= least) {
+      if (at < S_CAND) mine[at] = ((unsigned long long)key[u] << 32) | (uint32_t)~(base + place(u));
+      ++at;
+    }
+  __syncthreads();
+  if (t == 0) counts[part] = make_int2(s_count, share_bin << (32 - S_BITS));       // more than S_CAND: the row is walked
 }
 
 // sorts a[0..n) of LDS downwards by the entries' upper words, n <= S_CAND; every thread of the workgroup
-// calls it.  Up to S_BY_RANK entries each thread counts the entries above its own and puts it there (n reads
-// that the whole wavefront shares, a compare and an add each, no barrier between them); entries with equal
+// calls it.  Up to S_BY_RANK entries each thread counts the entries above its own and puts it there (reads of four keys
+// that the whole wavefront shares, no barrier between them); entries with equal
 // upper words take neighbouring places in the order in which they come.  More entries are sorted by a
-// bitonic network on the whole entries, a barrier a stage.  tmp: room for S_BY_RANK entries and as many counters.
+// bitonic network on the whole entries, a barrier a stage.  tmp: room for S_BY_RANK entries, as many counters and as many keys.
 #define S_BY_RANK 1024
 __device__ void sort_down(unsigned long long* a, int n, unsigned long long* tmp) {
   if (n <= S_BY_RANK) {
     int* taken = reinterpret_cast<int*>(tmp + S_BY_RANK);
+    uint32_t* keys = reinterpret_cast<uint32_t*>(taken + S_BY_RANK);
     const int i = threadIdx.x;
-    if (i < n) taken[i] = 0;
+    unsigned long long x = 0;
+    if (i < n) {
+      x = a[i];
+      taken[i] = 0;
+    }
+    if (i < ((n + 3) & ~3)) keys[i] = (uint32_t)(x >> 32);         // beyond n: 0, above nothing
     __syncthreads();
     if (i < n) {
-      const unsigned long long x = a[i];
       const uint32_t mine = (uint32_t)(x >> 32);
       int above = 0;
-      for (int j = 0; j < n; ++j) above += (uint32_t)(a[j] >> 32) > mine ? 1 : 0;
-      tmp[above + atomicAdd(&taken[above], 1)] = x;
+      for (int j = 0; j < n; j += 4) {
+        const uint4 q = *reinterpret_cast<const uint4*>(keys + j);
+        above += (q.x > mine) + (q.y > mine) + (q.z > mine) + (q.w > mine);
+      }
+      a[above + atomicAdd(&taken[above], 1)] = x;
     }
-    __syncthreads();
-    if (i < n) a[i] = tmp[i];
     __syncthreads();
     return;
   }
@@ -515,76 +550,216 @@ __device__ int pairs_at_least(const unsigned long long* a, int n, uint32_t key, 
   return m;
 }
 
+// sorts the pairs a[0..n) of LDS, (key, ~index) with indices below V, by index; the result is in b as (~index, key).  A count by the
+// indices' upper bits gives every pair its bucket's range, and within a bucket it counts the smaller ones.  n <= S_CAND; every thread
+// calls it.  s_bins: 2 SNT counters.
+__device__ void sort_by_index(const unsigned long long* a, unsigned long long* tmp, unsigned long long* b, int n, int V, int* s_bins, int* s_wave) {
+  const int t = threadIdx.x, lane = t & (TI_WAVE - 1), wave = t / TI_WAVE;
+  const int bits = max(0, 32 - __clz(V - 1) - 11);           // indices of a bucket: 2^bits, 2 SNT buckets
+  static_assert(2 * SNT == 2048, "eleven bits of buckets");
+  s_bins[2 * t] = s_bins[2 * t + 1] = 0;
+  __syncthreads();
+  for (int i = t; i < n; i += SNT) atomicAdd(&s_bins[~(uint32_t)a[i] >> bits], 1);
+  __syncthreads();
+  const int c0 = s_bins[2 * t], c1 = s_bins[2 * t + 1];
+  int run = wave_prefix(c0 + c1);
+  if (lane == TI_WAVE - 1) s_wave[wave] = run;
+  __syncthreads();
+  run -= c0 + c1;
+#pragma unroll
+  for (int w = 0; w < SNT / TI_WAVE; ++w)
+    if (w < wave) run += s_wave[w];
+  s_bins[2 * t] = run;                                       // where the bucket starts; after the next loop where it ends
+  s_bins[2 * t + 1] = run + c0;
+  __syncthreads();
+  for (int i = t; i < n; i += SNT) tmp[atomicAdd(&s_bins[~(uint32_t)a[i] >> bits], 1)] = a[i];
+  __syncthreads();
+  for (int i = t; i < n; i += SNT) {
+    const unsigned long long x = tmp[i];
+    const uint32_t index = ~(uint32_t)x, bucket = index >> bits;
+    const int lo = bucket ? s_bins[bucket - 1] : 0, hi = s_bins[bucket];
+    int at = lo;
+    for (int j = lo; j < hi; ++j) at += ~(uint32_t)tmp[j] < index ? 1 : 0;
+    b[at] = (x << 32) | (x >> 32);
+  }
+  __syncthreads();
+}
+
 __global__ void __launch_bounds__(SNT)
 sample_finish_kernel(const float* __restrict__ logits, const float* __restrict__ temp, const int* __restrict__ top_k,
                      const float* __restrict__ top_p, const float* __restrict__ uni, int* __restrict__ out,
-                     int* __restrict__ scratch, int V) {
-  __shared__ unsigned long long s_pair[S_CAND];
+                     const int2* __restrict__ counts, const unsigned long long* __restrict__ pairs, int parts, int V) {
+  __shared__ __attribute__((aligned(16))) unsigned long long s_pair[S_CAND], s_tmp[S_CAND];
   __shared__ float s_w[S_CAND];
+  __shared__ __attribute__((aligned(16))) int s_bins[S_BINS];
   __shared__ float s_wave[SNT / TI_WAVE];
-  __shared__ int s_n, s_at;
-  const int r = blockIdx.x;
+  __shared__ int s_iwave[SNT / TI_WAVE], s_res[4];
+  __shared__ int s_n, s_at, s_m, s_over;
+  __shared__ uint32_t s_max, s_from;
+  const int r = blockIdx.x, t = threadIdx.x, lane = t & (TI_WAVE - 1), wave = t / TI_WAVE;
   const int k = served_cut(temp, top_k, r, V);
   if (k == 0) {
     sample_row_by_bisection(logits, temp, top_k, top_p, uni, out, V, r);
     return;
   }
   const float T = temp[r], p_keep = top_p[r], u = uni[r];
-  int* head = scratch + (size_t)r * S_ROW_WORDS;
-  const unsigned long long* cand = reinterpret_cast<const unsigned long long*>(head + S_HEAD_WORDS);
-  const int n = head[2 * S_BINS];
-  if (threadIdx.x == 0) s_at = 0x7fffffff;
-  __syncthreads();                                 // every thread has the count: now the row's words go back to zero
-  for (int i = threadIdx.x; i < S_HEAD_WORDS; i += SNT) head[i] = 0;
-  if (n > S_CAND) {
+  // a wavefront takes parts wave, wave + 16, ...: f(eight pairs, or 0) by all lanes, eight loads under way at a time;
+  // a part's first go out beside the load of its count (what lies beyond it is room of the part's, whatever it holds)
+  const auto each = [&](auto f) {
+    for (int b = wave; b < parts; b += SNT / TI_WAVE) {
+      const unsigned long long* seg = pairs + ((size_t)r * parts + b) * S_CAND + lane;
+      unsigned long long x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = seg[TI_WAVE * j];
+      const int n = min(counts[(size_t)r * parts + b].x, S_CAND);
+      for (int i0 = 0; i0 < n; i0 += 8 * TI_WAVE) {
+        if (i0) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) x[j] = i0 + TI_WAVE * j + lane < n ? seg[i0 + TI_WAVE * j] : 0ull;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (i0 + TI_WAVE * j + lane >= n) x[j] = 0ull;
+        f(x);
+      }
+    }
+  };
+  reinterpret_cast<int4*>(s_bins)[t] = make_int4(0, 0, 0, 0);
+  static_assert(S_BINS == 4 * SNT, "four bins a thread");
+  if (t == 0) s_at = 0x7fffffff, s_m = 0, s_max = 0, s_over = 0, s_from = 0xffffffffu;
+  __syncthreads();
+  for (int b = t; b < parts; b += SNT) {
+    const int2 c = counts[(size_t)r * parts + b];
+    if (c.x > S_CAND) s_over = 1;
+    atomicMin(&s_from, (uint32_t)c.y);
+  }
+  __syncthreads();
+  const uint32_t from = s_from;
+  const bool over = s_over != 0;
+  // the pairs at or above `key`, in LDS as far as they fit
+  const auto gather = [&](uint32_t key) {
+    const uint32_t least = max(key, 1u);           // (0 is no pair)
+    each([&](const unsigned long long* x) {
+      int n = 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) n += (uint32_t)(x[j] >> 32) >= least ? 1 : 0;
+      int at = next_places(&s_m, n);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if ((uint32_t)(x[j] >> 32) >= least) {
+          if (at < S_CAND) s_tmp[at] = x[j];
+          ++at;
+        }
+    });
+    __syncthreads();
+  };
+  gather(from);
+  int bin, above, in, taken = 0, need = k, shift = 32, got = s_m;      // taken: keys above the prefix
+  uint32_t prefix = 0;
+  const auto digit = [&](unsigned long long x) {
+    const uint32_t key = (uint32_t)(x >> 32);
+    if (x && (shift == 32 || (key >> shift) == prefix))
+      atomicAdd(&s_bins[shift == 32 ? key >> (32 - S_BITS) : (key >> (shift - S_BITS2)) & (S_BINS2 - 1)], 1);
+  };
+  const auto next = [&]() {                        // the digit that `digit` has counted
+    __syncthreads();
+    if (shift == 32) {
+      bin_of_kth<S_BINS, SNT>(s_bins, need, s_iwave, s_res, bin, above, in);
+      prefix = bin;
+      shift = 32 - S_BITS;
+    } else {
+      bin_of_kth<S_BINS2, SNT>(s_bins, need, s_iwave, s_res, bin, above, in);
+      prefix = (prefix << S_BITS2) | (uint32_t)bin;
+      shift -= S_BITS2;
+    }
+    taken += above;
+    need -= above;
+  };
+  if (got == 0) {                                  // a row of NaN
+    if (t == 0) out[r] = 0;
+    return;
+  }
+  if (got > S_CAND && !over) {                     // shares that are no guide: by digits over all pairs, until few enough are left
+    do {
+      each([&](const unsigned long long* x) {
+        for (int j = 0; j < 8; ++j) digit(x[j]);
+      });
+      next();
+    } while (taken + in > S_CAND && shift > 0);
+    got = taken + in;
+    if (got <= S_CAND) {
+      if (t == 0) s_m = 0;
+      __syncthreads();
+      gather(prefix << shift);
+    }
+  }
+  if (over || got > S_CAND) {
     sample_row_by_bisection(logits, temp, top_k, top_p, uni, out, V, r);
     return;
   }
-  if (n == 0) {                                    // a row of NaN
-    if (threadIdx.x == 0) out[r] = 0;
-    return;
-  }
-  for (int i = threadIdx.x; i < n; i += SNT) s_pair[i] = cand[i];
+  const int n = s_m;                               // the rest of the k-th key from these
+  constexpr int PER = S_CAND / SNT;
+  unsigned long long mine[PER];                    // pairs t, t + SNT, ...
+#pragma unroll
+  for (int j = 0; j < PER; ++j) mine[j] = t + SNT * j < n ? s_tmp[t + SNT * j] : 0ull;
   __syncthreads();
-  sort_down(s_pair, n, reinterpret_cast<unsigned long long*>(s_w));                            // by key
+  if (t == 0) s_m = 0;
+  __syncthreads();
+  while (shift > 0) {
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      digit(mine[j]);
+    next();
+  }
+  const uint32_t cut = prefix;
   if (!(T > 0.f)) {                                // of equal logits the lowest index
-    const uint32_t top = (uint32_t)(s_pair[0] >> 32);
-    for (int i = threadIdx.x; i < n; i += SNT)
-      if ((uint32_t)(s_pair[i] >> 32) == top) atomicMin(&s_at, (int)~(uint32_t)s_pair[i]);
+#pragma unroll
+    for (int j = 0; j < PER; ++j)
+      if (mine[j] && (uint32_t)(mine[j] >> 32) == cut) atomicMin(&s_at, (int)~(uint32_t)mine[j]);
     __syncthreads();
-    if (threadIdx.x == 0) out[r] = s_at;
+    if (t == 0) out[r] = s_at;
     return;
   }
-  int m = pairs_at_least(s_pair, n, (uint32_t)(s_pair[min(k, n) - 1] >> 32), &s_n);
-  const float mx = key_value((uint32_t)(s_pair[0] >> 32));
+  uint32_t largest = 0;
+  int kept = 0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const uint32_t key = (uint32_t)(mine[j] >> 32);
+    kept += key >= cut ? 1 : 0;                    // (the cut is some number's key, not 0)
+    largest = max(largest, key);
+  }
+  int place = next_places(&s_m, kept);
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    if ((uint32_t)(mine[j] >> 32) >= cut) s_pair[place++] = mine[j];
+  if (largest) atomicMax(&s_max, largest);
+  __syncthreads();
+  int m = s_m;
+  const float mx = key_value(s_max);
   const float inv_t = 1.0f / T;
   if (p_keep < 1.0f) {
-    for (int i = threadIdx.x; i < m; i += SNT) s_w[i] = expf((key_value((uint32_t)(s_pair[i] >> 32)) - mx) * inv_t);
+    sort_down(s_pair, m, s_tmp);
+    for (int i = t; i < m; i += SNT) s_w[i] = expf((key_value((uint32_t)(s_pair[i] >> 32)) - mx) * inv_t);
     __syncthreads();
-    const float need = p_keep * scan_in_place(s_w, m, s_wave);
-    for (int i = threadIdx.x; i < m; i += SNT)
-      if (s_w[i] >= need) atomicMin(&s_at, i);
+    const float need_mass = p_keep * scan_in_place(s_w, m, s_wave);
+    for (int i = t; i < m; i += SNT)
+      if (s_w[i] >= need_mass) atomicMin(&s_at, i);
     __syncthreads();
-    const int j = s_at;                            // the first pair at which the mass from the top reaches need
+    const int j = s_at;                            // the first pair at which the mass from the top reaches it
     __syncthreads();
-    if (threadIdx.x == 0) s_at = 0x7fffffff;
+    if (t == 0) s_at = 0x7fffffff;
     if (j < m) m = pairs_at_least(s_pair, m, (uint32_t)(s_pair[j] >> 32), &s_n);   // its equals stay
     else __syncthreads();
   }
   // what is left, in the order of the indices
-  for (int i = threadIdx.x; i < m; i += SNT) {
-    const unsigned long long pr = s_pair[i];
-    s_pair[i] = (pr << 32) | (pr >> 32);           // (~index, key)
-  }
-  __syncthreads();
-  sort_down(s_pair, m, reinterpret_cast<unsigned long long*>(s_w));
-  for (int i = threadIdx.x; i < m; i += SNT) s_w[i] = expf((key_value((uint32_t)s_pair[i]) - mx) * inv_t);
+  sort_by_index(s_pair, s_tmp, s_pair, m, V, s_bins, s_iwave);
+  for (int i = t; i < m; i += SNT) s_w[i] = expf((key_value((uint32_t)s_pair[i]) - mx) * inv_t);
   __syncthreads();
   const float target = u * scan_in_place(s_w, m, s_wave);
-  for (int i = threadIdx.x; i < m; i += SNT)
+  for (int i = t; i < m; i += SNT)
     if (target < s_w[i]) atomicMin(&s_at, i);
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (t == 0) {
     const int at = s_at < m ? s_at : m - 1;        // rounding pushed the target past the end: the last one kept
     out[r] = (int)~(uint32_t)(s_pair[at] >> 32);
   }
@@ -648,10 +823,10 @@ extern "C" int ti_argmax_static(const float* logits, int* out, int n_rows, int V
   return 0;
 }
 
-extern "C" long ti_sample_scratch_bytes(int n_rows) { return (long)n_rows * S_ROW_WORDS * 4; }
+static int sample_parts(int V) { return std::max(1, (V + S_SPAN - 1) / S_SPAN); }
+extern "C" long ti_sample_scratch_bytes(int n_rows, int V) { return (long)n_rows * sample_parts(V) * (S_CAND * 8 + 8); }
 
-// scratch: ti_sample_scratch_bytes(n_rows) bytes that were zero before the first call and that only calls of
-// this function (one at a time) have touched since, or nullptr (then one workgroup walks a whole row)
+// scratch: ti_sample_scratch_bytes(n_rows, V) bytes on a boundary of 8, or nullptr (then one workgroup walks a whole row)
 extern "C" int ti_sample(const float* logits, const float* temp, const int* top_k, const float* top_p,
                          const float* uni, int* out, void* scratch, int n_rows, int V, hipStream_t stream) {
   TI_REQUIRE(n_rows >= 0 && V > 0, "sample: bad sizes rows=%d V=%d", n_rows, V);
@@ -659,12 +834,15 @@ extern "C" int ti_sample(const float* logits, const float* temp, const int* top_
   if (!scratch) {
     sample_kernel<<<n_rows, SNT, 0, stream>>>(logits, temp, top_k, top_p, uni, out, V);
   } else {
-    const int most = n_rows <= 8 ? 80 : (n_rows <= 32 ? 32 : 16), span = 256 * S_LOADS;
-    const dim3 grid(std::min(most, (V + span - 1) / span), n_rows);
-    sample_pass_kernel<0><<<grid, 256, 0, stream>>>(logits, temp, top_k, (int*)scratch, V);
-    sample_pass_kernel<1><<<grid, 256, 0, stream>>>(logits, temp, top_k, (int*)scratch, V);
-    sample_pass_kernel<2><<<grid, 256, 0, stream>>>(logits, temp, top_k, (int*)scratch, V);
-    sample_finish_kernel<<<n_rows, SNT, 0, stream>>>(logits, temp, top_k, top_p, uni, out, (int*)scratch, V);
+    const int parts = sample_parts(V), span = ((V + parts - 1) / parts + 3) & ~3;      // parts of a size: equal shares
+    const dim3 grid(parts, n_rows);
+    auto* pairs = (unsigned long long*)scratch;
+    int2* counts = (int2*)(pairs + (size_t)n_rows * parts * S_CAND);
+    if (V % 4 == 0 && ((uintptr_t)logits & 15) == 0)
+      sample_part_kernel<true><<<grid, S_NT, 0, stream>>>(logits, temp, top_k, counts, pairs, V, span);
+    else
+      sample_part_kernel<false><<<grid, S_NT, 0, stream>>>(logits, temp, top_k, counts, pairs, V, span);
+    sample_finish_kernel<<<n_rows, SNT, 0, stream>>>(logits, temp, top_k, top_p, uni, out, counts, pairs, parts, V);
   }
   TI_LAUNCH_CHECK();
   return 0;

@@ -501,11 +501,10 @@ int ti_argmax(const float* logits, int* out, void* scratch, int n_rows, int V, h
 // allocating routine; calls that overlap on one GPU share the array and race.  It has no counterpart in
 // the reference: it is there for callers that cannot allocate.
 int ti_argmax_static(const float* logits, int* out, int n_rows, int V, hipStream_t stream);
-// temperature, top-k (0: all), top-p and one uniform number per row.  scratch: ti_sample_scratch_bytes(n_rows)
-// bytes, zero before the first call and touched by nothing else since (the kernels leave them at zero; calls
-// that overlap on one workspace race), or null: then one workgroup walks a whole row, as it does for the rows
-// that have no top-k cut.
-long ti_sample_scratch_bytes(int n_rows);
+// temperature, top-k (0: all), top-p and one uniform number per row.  scratch: ti_sample_scratch_bytes(n_rows, V)
+// bytes on a boundary of 8, whatever they hold (calls that overlap on one workspace race), or null: then one workgroup walks a whole
+// row, as it does for the rows that have no top-k cut.
+long ti_sample_scratch_bytes(int n_rows, int V);
 int ti_sample(const float* logits, const float* temp, const int* top_k, const float* top_p, const float* uni, int* out,
               void* scratch, int n_rows, int V, hipStream_t stream);
 

@@ -614,7 +614,7 @@ class Ops {
   int units_ = 0;
   DeviceBuffer partials_;
   DeviceBuffer argmax_scratch_;
-  DeviceBuffer sample_scratch_;       // zero between calls
+  DeviceBuffer sample_scratch_;
   struct { void* out = nullptr; int64_t count = 0; int splits = 0; } pending_;
   std::map<std::string, std::map<std::string, long>> tuning_;
   friend struct TunedScope;

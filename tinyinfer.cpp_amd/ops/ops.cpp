@@ -1977,11 +1977,10 @@ void Ops::sample(const Tensor& logits, const float* temperature, const int* top_
   void* scratch = nullptr;
   if (use.radix_sample) {
     const int64_t rows = std::max<int64_t>(logits.shape[0], 8);
-    const size_t need = (size_t)KERNEL("sampling", ti_sample_scratch_bytes)((int)rows);
+    const size_t need = (size_t)KERNEL("sampling", ti_sample_scratch_bytes)((int)rows, (int)logits.shape[1]);
     if (sample_scratch_.bytes() < need) {
       flush();
       sample_scratch_ = DeviceBuffer(need);
-      fill_zero(sample_scratch_.data(), need);     // the kernels leave it at zero
     }
     scratch = sample_scratch_.data();
   }
