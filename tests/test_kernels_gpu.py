@@ -593,6 +593,29 @@ def test_sample_rows_whose_first_bin_holds_too_many(ops, V, skip):
         assert sum(a != b for a, b in zip(got, walked)) <= 1, (T, top_k, top_p, got, walked)
 
 
+@pytest.mark.parametrize("n,V", [(1, 1000), (65, 20001), (150, 4096)])
+def test_sampler_of_more_rows_than_travel_with_a_launch(ops, n, V):
+    """What the rows ask for goes with the launches, 64 rows at a time, and the ids come straight into the host's memory: the ids
+    are those of the kernel that reads both from device memory, in turns of two calls under way at once."""
+    from tinyinfer_amd.sampling import Sampler, SamplingParams
+    from tinyinfer_amd.sampling.sampler import uniform
+    g = torch.Generator().manual_seed(n)
+    asked = [SamplingParams(), SamplingParams(0.8, 50, 0.9, 3), SamplingParams(1.2, 0, 1.0, 9)]
+    sampler, tickets, wants = Sampler(ops), [], []
+    for turn in range(2):
+        logits = dev(torch.randn(n, V, generator=g) * 3)
+        params = [asked[(i + turn) % 3] for i in range(n)]
+        requests, counters = [7 * i + turn for i in range(n)], [i % 5 for i in range(n)]
+        out = torch.empty(n, dtype=torch.int32, device="cuda")
+        ops.sample(logits, dev(torch.tensor([p.temperature for p in params])),
+                   dev(torch.tensor([p.effective_top_k() for p in params], dtype=torch.int32)), dev(torch.tensor([p.top_p for p in params])),
+                   dev(torch.tensor([uniform(p.seed, r, c) for p, r, c in zip(params, requests, counters)])), out)
+        wants.append((logits, out.tolist()))
+        tickets.append(sampler.sample_async(logits, params, requests, counters))
+    for ticket, (_, want) in zip(tickets, wants):
+        assert sampler.collect(ticket) == want
+
+
 # ------------------------------------------------- bfloat16 matrix-core products
 @pytest.mark.parametrize("M,N,K", [
     (1, 48, 64), (5, 261, 1024), (8, 1000, 96), (16, 17, 200), (17, 130, 72), (33, 64, 3072), (64, 151, 256),

@@ -153,18 +153,35 @@ argmax_final_kernel(const float* __restrict__ part_val, const int* __restrict__ 
   if (threadIdx.x == 0) out[r] = bi == 0x7fffffff ? 0 : bi;
 }
 
+// What the rows of a call ask for: in memory of the device's, or up to S_VALUES rows of it in the launch's own arguments, which
+// costs no copy (one of 1 KiB takes 3 us on the stream and as long on the host).
+struct SampleRow {
+  float temp;
+  int top_k;
+  float top_p, uni;
+};
+struct RowsInMemory {
+  const float* temp;
+  const int* top_k;
+  const float *top_p, *uni;
+  __device__ __forceinline__ SampleRow at(int r) const { return SampleRow{temp[r], top_k[r], top_p[r], uni[r]}; }
+};
+#define S_VALUES 64
+struct RowsByValue {
+  SampleRow row[S_VALUES];
+  __device__ __forceinline__ SampleRow at(int r) const { return row[r]; }
+};
+
 // temp[r] <= 0: greedy.  top_k[r] <= 0 or >= V: no top-k cut.  top_p[r] >= 1: no top-p cut.
 // One workgroup walks the whole row some seventy times: the way for the rows that the four short
 // kernels below do not serve, and for a caller without their workspace.
-__device__ void sample_row_by_bisection(const float* __restrict__ logits, const float* __restrict__ temp,
-                                        const int* __restrict__ top_k, const float* __restrict__ top_p,
-                                        const float* __restrict__ uni, int* __restrict__ out, int V, int r) {
+__device__ void sample_row_by_bisection(const float* __restrict__ logits, SampleRow want, int* __restrict__ out, int V, int r) {
   __shared__ float s_val[SNT / TI_WAVE];
   __shared__ int s_idx[SNT / TI_WAVE];
   __shared__ float s_chunk[SNT];
   __shared__ int s_pick;
   const float* row = logits + (size_t)r * V;
-  const float T = temp[r];
+  const float T = want.temp;
   const int best = row_argmax(row, V, s_val, s_idx);
   if (!(T > 0.f)) {
     if (threadIdx.x == 0) out[r] = best;
@@ -174,7 +191,7 @@ __device__ void sample_row_by_bisection(const float* __restrict__ logits, const 
   const float inv_t = 1.0f / T;
 
   uint32_t cut = 0;   // keep keys >= cut
-  const int k = top_k[r];
+  const int k = want.top_k;
   if (k > 0 && k < V) {
     uint32_t prefix = 0;
     for (int bit = 31; bit >= 0; --bit) {
@@ -186,7 +203,7 @@ __device__ void sample_row_by_bisection(const float* __restrict__ logits, const 
     }
     cut = prefix;
   }
-  const float p_keep = top_p[r];
+  const float p_keep = want.top_p;
   if (p_keep < 1.0f) {
     float s = 0.f;
     for (int i = threadIdx.x; i < V; i += SNT) {
@@ -223,7 +240,7 @@ __device__ void sample_row_by_bisection(const float* __restrict__ logits, const 
   if (threadIdx.x == 0) {
     float total = 0.f;
     for (int i = 0; i < SNT; ++i) total += s_chunk[i];
-    const float target = uni[r] * total;
+    const float target = want.uni * total;
     float acc = 0.f;
     int owner = -1, last_nonzero = 0;
     for (int i = 0; i < SNT; ++i) {
@@ -259,10 +276,10 @@ __device__ void sample_row_by_bisection(const float* __restrict__ logits, const 
   if (threadIdx.x == 0) out[r] = s_pick;
 }
 
+template <class Rows>
 __global__ void __launch_bounds__(SNT)
-sample_kernel(const float* __restrict__ logits, const float* __restrict__ temp, const int* __restrict__ top_k,
-              const float* __restrict__ top_p, const float* __restrict__ uni, int* __restrict__ out, int V) {
-  sample_row_by_bisection(logits, temp, top_k, top_p, uni, out, V, blockIdx.x);
+sample_kernel(const float* __restrict__ logits, Rows rows, int* __restrict__ out, int V) {
+  sample_row_by_bisection(logits, rows.at(blockIdx.x), out, V, blockIdx.x);
 }
 
 // ------------------------------------------------------------ the same draw in two short kernels
@@ -299,9 +316,9 @@ static_assert(S_BITS + 2 * S_BITS2 == 32, "a key is three digits");
 __device__ __forceinline__ float key_value(uint32_t key) {
   return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key);
 }
-// the cut that the radix kernels find for row r: a greedy row is a cut to the largest key; 0: not served
-__device__ __forceinline__ int served_cut(const float* temp, const int* top_k, int r, int V) {
-  const int k = temp[r] > 0.f ? top_k[r] : 1;
+// the cut that the radix kernels find for a row: a greedy row is a cut to the largest key; 0: not served
+__device__ __forceinline__ int served_cut(const SampleRow& want, int V) {
+  const int k = want.temp > 0.f ? want.top_k : 1;
   return (k > 0 && k < V && k <= S_MAX_K) ? k : 0;
 }
 
@@ -383,14 +400,14 @@ __device__ __forceinline__ int next_places(int* s_count, int n) {
 // grid (parts of `span` keys, rows), span a multiple of 4, at most S_SPAN.  WIDE: rows of whole float4s on their boundaries, four
 // neighbours a load.  counts [row][parts][2] (pairs, the key from which the part's share lies), pairs [row][parts][S_CAND]
 // (key << 32 | ~index).  (64 registers a thread: four workgroups to a unit, so that 64 rows of 15 parts are one round.)
-template <bool WIDE>
+template <bool WIDE, class Rows>
 __global__ void __launch_bounds__(S_NT)
-sample_part_kernel(const float* __restrict__ logits, const float* __restrict__ temp, const int* __restrict__ top_k,
-                   int2* __restrict__ counts, unsigned long long* __restrict__ pairs, int V, int span) {
+sample_part_kernel(const float* __restrict__ logits, Rows rows, int2* __restrict__ counts, unsigned long long* __restrict__ pairs,
+                   int V, int span) {
   __shared__ __attribute__((aligned(16))) int s_bins[S_BINS];
   __shared__ int s_wave[S_NT / TI_WAVE], s_res[4], s_count;
   const int r = blockIdx.y, t = threadIdx.x;
-  const int k = served_cut(temp, top_k, r, V);
+  const int k = served_cut(rows.at(r), V);
   if (k == 0) return;                              // the whole workgroup
   const float* row = logits + (size_t)r * V;
   const size_t part = (size_t)r * gridDim.x + blockIdx.x;
@@ -585,10 +602,10 @@ __device__ void sort_by_index(const unsigned long long* a, unsigned long long* t
   __syncthreads();
 }
 
+template <class Rows>
 __global__ void __launch_bounds__(SNT)
-sample_finish_kernel(const float* __restrict__ logits, const float* __restrict__ temp, const int* __restrict__ top_k,
-                     const float* __restrict__ top_p, const float* __restrict__ uni, int* __restrict__ out,
-                     const int2* __restrict__ counts, const unsigned long long* __restrict__ pairs, int parts, int V) {
+sample_finish_kernel(const float* __restrict__ logits, Rows rows, int* __restrict__ out, const int2* __restrict__ counts,
+                     const unsigned long long* __restrict__ pairs, int parts, int V) {
   __shared__ __attribute__((aligned(16))) unsigned long long s_pair[S_CAND], s_tmp[S_CAND];
   __shared__ float s_w[S_CAND];
   __shared__ __attribute__((aligned(16))) int s_bins[S_BINS];
@@ -597,12 +614,13 @@ sample_finish_kernel(const float* __restrict__ logits, const float* __restrict__
   __shared__ int s_n, s_at, s_m, s_over;
   __shared__ uint32_t s_max, s_from;
   const int r = blockIdx.x, t = threadIdx.x, lane = t & (TI_WAVE - 1), wave = t / TI_WAVE;
-  const int k = served_cut(temp, top_k, r, V);
+  const SampleRow want = rows.at(r);
+  const int k = served_cut(want, V);
   if (k == 0) {
-    sample_row_by_bisection(logits, temp, top_k, top_p, uni, out, V, r);
+    sample_row_by_bisection(logits, want, out, V, r);
     return;
   }
-  const float T = temp[r], p_keep = top_p[r], u = uni[r];
+  const float T = want.temp, p_keep = want.top_p, u = want.uni;
   // a wavefront takes parts wave, wave + 16, ...: f(eight pairs, or 0) by all lanes, eight loads under way at a time;
   // a part's first go out beside the load of its count (what lies beyond it is room of the part's, whatever it holds)
   const auto each = [&](auto f) {
@@ -694,7 +712,7 @@ sample_finish_kernel(const float* __restrict__ logits, const float* __restrict__
     }
   }
   if (over || got > S_CAND) {
-    sample_row_by_bisection(logits, temp, top_k, top_p, uni, out, V, r);
+    sample_row_by_bisection(logits, want, out, V, r);
     return;
   }
   const int n = s_m;                               // the rest of the k-th key from these
@@ -826,24 +844,42 @@ extern "C" int ti_argmax_static(const float* logits, int* out, int n_rows, int V
 static int sample_parts(int V) { return std::max(1, (V + S_SPAN - 1) / S_SPAN); }
 extern "C" long ti_sample_scratch_bytes(int n_rows, int V) { return (long)n_rows * sample_parts(V) * (S_CAND * 8 + 8); }
 
+template <class Rows>
+static void launch_sample(const float* logits, const Rows& rows, int* out, void* scratch, int n_rows, int V, hipStream_t stream) {
+  if (!scratch) {
+    sample_kernel<<<n_rows, SNT, 0, stream>>>(logits, rows, out, V);
+    return;
+  }
+  const int parts = sample_parts(V), span = ((V + parts - 1) / parts + 3) & ~3;      // parts of a size: equal shares
+  const dim3 grid(parts, n_rows);
+  auto* pairs = (unsigned long long*)scratch;
+  int2* counts = (int2*)(pairs + (size_t)n_rows * parts * S_CAND);
+  if (V % 4 == 0 && ((uintptr_t)logits & 15) == 0)
+    sample_part_kernel<true><<<grid, S_NT, 0, stream>>>(logits, rows, counts, pairs, V, span);
+  else
+    sample_part_kernel<false><<<grid, S_NT, 0, stream>>>(logits, rows, counts, pairs, V, span);
+  sample_finish_kernel<<<n_rows, SNT, 0, stream>>>(logits, rows, out, counts, pairs, parts, V);
+}
+
 // scratch: ti_sample_scratch_bytes(n_rows, V) bytes on a boundary of 8, or nullptr (then one workgroup walks a whole row)
 extern "C" int ti_sample(const float* logits, const float* temp, const int* top_k, const float* top_p,
                          const float* uni, int* out, void* scratch, int n_rows, int V, hipStream_t stream) {
   TI_REQUIRE(n_rows >= 0 && V > 0, "sample: bad sizes rows=%d V=%d", n_rows, V);
   if (n_rows == 0) return 0;
-  if (!scratch) {
-    sample_kernel<<<n_rows, SNT, 0, stream>>>(logits, temp, top_k, top_p, uni, out, V);
-  } else {
-    const int parts = sample_parts(V), span = ((V + parts - 1) / parts + 3) & ~3;      // parts of a size: equal shares
-    const dim3 grid(parts, n_rows);
-    auto* pairs = (unsigned long long*)scratch;
-    int2* counts = (int2*)(pairs + (size_t)n_rows * parts * S_CAND);
-    if (V % 4 == 0 && ((uintptr_t)logits & 15) == 0)
-      sample_part_kernel<true><<<grid, S_NT, 0, stream>>>(logits, temp, top_k, counts, pairs, V, span);
-    else
-      sample_part_kernel<false><<<grid, S_NT, 0, stream>>>(logits, temp, top_k, counts, pairs, V, span);
-    sample_finish_kernel<<<n_rows, SNT, 0, stream>>>(logits, temp, top_k, top_p, uni, out, counts, pairs, parts, V);
-  }
+  launch_sample(logits, RowsInMemory{temp, top_k, top_p, uni}, out, scratch, n_rows, V, stream);
   TI_LAUNCH_CHECK();
+  return 0;
+}
+
+extern "C" int ti_sample_by_value(const float* logits, const float* temp, const int* top_k, const float* top_p,
+                                  const float* uni, int* out, void* scratch, int n_rows, int V, hipStream_t stream) {
+  TI_REQUIRE(n_rows >= 0 && V > 0, "sample: bad sizes rows=%d V=%d", n_rows, V);
+  for (int r0 = 0; r0 < n_rows; r0 += S_VALUES) {
+    const int n = std::min(S_VALUES, n_rows - r0);
+    RowsByValue rows = {};
+    for (int i = 0; i < n; ++i) rows.row[i] = SampleRow{temp[r0 + i], top_k[r0 + i], top_p[r0 + i], uni[r0 + i]};
+    launch_sample(logits + (size_t)r0 * V, rows, out + r0, scratch, n, V, stream);
+    TI_LAUNCH_CHECK();
+  }
   return 0;
 }

@@ -507,6 +507,10 @@ int ti_argmax_static(const float* logits, int* out, int n_rows, int V, hipStream
 long ti_sample_scratch_bytes(int n_rows, int V);
 int ti_sample(const float* logits, const float* temp, const int* top_k, const float* top_p, const float* uni, int* out,
               void* scratch, int n_rows, int V, hipStream_t stream);
+// the same with what the rows ask for in the host's memory, read before the call returns: it travels with the launches.  `out` may be
+// pinned memory of the host's.  (Rows are served 64 at a time.)
+int ti_sample_by_value(const float* logits, const float* temp, const int* top_k, const float* top_p, const float* uni, int* out,
+                       void* scratch, int n_rows, int V, hipStream_t stream);
 
 
 // ---- libti_measure: what the GPU delivers, for the bench tool's fractions

@@ -553,6 +553,9 @@ class Ops {
   void argmax(const Tensor& logits, int* out);
   void sample(const Tensor& logits, const float* temperature, const int* top_k, const float* top_p, const float* uniform,
               int* out);
+  // the same with the rows' numbers in the host's memory (no copy of them on the stream); `out` may be pinned memory of the host's
+  void sample_by_value(const Tensor& logits, const float* temperature, const int* top_k, const float* top_p, const float* uniform,
+                       int* out);
   void fill_zero(void* p, size_t bytes);
   void fill_random(const Tensor& t, const std::string& init, double a, double b, uint64_t seed);
   // Partial sums that a product left in the workspace are added now (same order, same bits as
@@ -615,6 +618,7 @@ class Ops {
   DeviceBuffer partials_;
   DeviceBuffer argmax_scratch_;
   DeviceBuffer sample_scratch_;
+  void* sample_scratch(const Tensor& logits, int64_t rows);
   struct { void* out = nullptr; int64_t count = 0; int splits = 0; } pending_;
   std::map<std::string, std::map<std::string, long>> tuning_;
   friend struct TunedScope;

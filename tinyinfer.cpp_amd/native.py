@@ -147,9 +147,9 @@ _SIGNATURES = {
     "ti_engine_state": [c_void_p, c_int, c_int, _TT],
     "ti_engine_synchronize": [c_void_p],
     "ti_sampler_create": [c_void_p, _OUT_PTR],
-    "ti_sampler_sample": [c_void_p, _TT, c_int, P(c_float), P(c_int), P(c_float), P(c_u64), P(c_i64), P(c_i64), P(c_int)],
-    "ti_sampler_sample_async": [c_void_p, _TT, c_int, P(c_float), P(c_int), P(c_float), P(c_u64), P(c_i64), P(c_i64), c_void_p,
-                                P(c_u64)],
+    # (the rows' arrays as ctypes arrays or as packed bytes)
+    "ti_sampler_sample": [c_void_p, _TT, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, P(c_int)],
+    "ti_sampler_sample_async": [c_void_p, _TT, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, P(c_u64)],
     "ti_sampler_collect": [c_void_p, c_u64, c_int, P(c_int)],
     "ti_scheduler_create": [c_void_p, c_int, c_int, c_int, _OUT_PTR],
     "ti_scheduler_add": [c_void_p, c_int, P(c_int), c_int, c_float, c_int, c_float, c_u64, c_int, P(c_int), P(c_i64)],

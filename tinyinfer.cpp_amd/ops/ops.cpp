@@ -1969,23 +1969,35 @@ void Ops::argmax(const Tensor& logits, int* out) {
   check("sampling", rc, "argmax");
 }
 
+void* Ops::sample_scratch(const Tensor& logits, int64_t rows) {
+  if (!use.radix_sample) return nullptr;
+  const size_t need = (size_t)KERNEL("sampling", ti_sample_scratch_bytes)((int)std::max<int64_t>(rows, 8), (int)logits.shape[1]);
+  if (sample_scratch_.bytes() < need) {
+    flush();
+    sample_scratch_ = DeviceBuffer(need);
+  }
+  return sample_scratch_.data();
+}
+
 void Ops::sample(const Tensor& logits, const float* temperature, const int* top_k, const float* top_p,
                  const float* uniform, int* out) {
   TIMED("sample " + dims(logits));
   require(logits.ndim == 2 && logits.dtype == DType::F32 && logits.contiguous(),
           "sample: logits must be contiguous float32 [n, V]");
-  void* scratch = nullptr;
-  if (use.radix_sample) {
-    const int64_t rows = std::max<int64_t>(logits.shape[0], 8);
-    const size_t need = (size_t)KERNEL("sampling", ti_sample_scratch_bytes)((int)rows, (int)logits.shape[1]);
-    if (sample_scratch_.bytes() < need) {
-      flush();
-      sample_scratch_ = DeviceBuffer(need);
-    }
-    scratch = sample_scratch_.data();
-  }
+  void* scratch = sample_scratch(logits, logits.shape[0]);
   int rc = KERNEL("sampling", ti_sample)((const float*)logits.data, temperature, top_k, top_p, uniform, out, scratch,
                                          (int)logits.shape[0], (int)logits.shape[1], (hipStream_t)launch_stream());
+  check("sampling", rc, "sample");
+}
+
+void Ops::sample_by_value(const Tensor& logits, const float* temperature, const int* top_k, const float* top_p,
+                          const float* uniform, int* out) {
+  TIMED("sample " + dims(logits));
+  require(logits.ndim == 2 && logits.dtype == DType::F32 && logits.contiguous(),
+          "sample: logits must be contiguous float32 [n, V]");
+  void* scratch = sample_scratch(logits, std::min<int64_t>(logits.shape[0], 64));
+  int rc = KERNEL("sampling", ti_sample_by_value)((const float*)logits.data, temperature, top_k, top_p, uniform, out, scratch,
+                                                  (int)logits.shape[0], (int)logits.shape[1], (hipStream_t)launch_stream());
   check("sampling", rc, "sample");
 }
 

