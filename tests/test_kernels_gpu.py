@@ -963,6 +963,38 @@ def test_linear_bf16_large_weight_at_13_to_16_rows(ops):
         assert torch.equal(outs[0], outs[1]) == (M == 12), M
 
 
+@pytest.mark.parametrize("N,K", [(40, 64), (1000, 1088), (2056, 1024), (4104, 192), (6144, 1024)])
+def test_linear_bf16_rows_through_lds_at_17_to_64_rows(ops, N, K):
+    """The 16-row workgroups whose rows come through LDS: fewer steps than stages and than wavefronts, four and eight wavefronts, a
+    launch of one workgroup a unit and of more, a last tile of few weight rows, both sides of every 16 tokens.  Within the bound
+    of 32-bit sums of float64, the row beyond the last left alone, and a row's bits those it has among 64."""
+    ops.lib("gemm_bf16").ti_tuning_reset()
+    g = torch.Generator().manual_seed(N + K)
+    a = (torch.rand(64, K, generator=g) * 2 - 1).to(torch.bfloat16)
+    w = (torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16)
+    ref, tol = ref_linear(a, w), 2e-5 * K
+    ad, wd = dev(a), dev(w)
+    full = torch.empty(64, N, device="cuda")
+    ops.linear(ad, wd, full, "store")
+    assert (f64(full) - ref).abs().max() < tol
+    pair = torch.empty(64, N // 2, device="cuda", dtype=torch.bfloat16)
+    ops.linear(ad, wd, pair, "swiglu")
+    gate, up = ref[:, :N // 2], ref[:, N // 2:]
+    want = gate / (1 + torch.exp(-gate)) * up
+    assert (f64(pair) - want).abs().max() < 0.005 * want.abs().max() + 10 * tol
+    for M in (17, 32, 33, 48, 49, 63):
+        out = torch.full((M + 1, N), 7.0, device="cuda")
+        ops.linear(ad[:M], wd, out[:M], "store")
+        assert torch.equal(out[:M], full[:M]) and bool((out[M] == 7.0).all()), M
+        out = torch.empty(M, N // 2, device="cuda", dtype=torch.bfloat16)
+        ops.linear(ad[:M], wd, out, "swiglu")
+        assert torch.equal(out, pair[:M]), M
+        out = torch.zeros(M, N, device="cuda")
+        ops.linear(ad[:M], wd, out, "add", may_defer=True)
+        ops.flush()
+        assert (f64(out) - ref[:M]).abs().max() < tol, M
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 16400, 64), (64, 20000, 1024), (40, 16387, 2048), (33, 17000, 192),
                                    (48, 16384, 1088)])
 def test_linear_bf16_wide_weight_at_17_to_64_rows(ops, M, N, K):

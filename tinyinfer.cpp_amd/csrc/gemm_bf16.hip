@@ -25,6 +25,7 @@
 #include "tinyinfer_kernels.h"
 #include "tinyinfer_kernels_tuning.h"
 #include "qk_prep.h"
+#include "staged_rows.h"
 
 TI_ERROR_API
 
@@ -48,13 +49,26 @@ __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f +
 // UN: 64-element chunks of K a wavefront has in flight at a time.  All loads of a pass are
 // issued before the first product: out-of-range pieces read a valid address (piece 0 of the
 // row) and get a zeroed weight instead of a branch, so that nothing waits in between.
-template <int MT, int EPI, int NW = 4, int UN = 4>
+// STAGES > 0 (more than 16 tokens, K of whole chunks): the rows come through LDS (staged_rows.h), a chunk a step; the same sums in the
+// same order.  Every workgroup pulls in all token rows, which as operands from memory was most of its time.  us, before and now, at 17,
+// 32, 48 and 64 rows: 4096 x 1024 4.3 4.9 5.9 6.9 -> 3.9 4.0 3.9 4.6; [gate; up] 6144 x 1024 6.7 7.8 9.8 10.0 -> 5.3 5.8 6.9 7.9 (the
+// latter two were tiles); 4096 x 2048 8.7 9.3 10.9 11.9 -> 6.0 6.4 7.2 8.3; 12288 x 2048 16.1 17.0 17.8 18.4 -> 11.5 13.5 16.3 18.6.
+struct RowPieces { v4u x, y; };
+template <int MT, int EPI, int NW = 4, int UN = 4, int STAGES = 0>
 __global__ void __launch_bounds__(NW * 64)
 gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ out_,
                    int M, int N, int K, long lda) {
+#if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass has no buffer descriptors)
   constexpr bool SW = (EPI == TI_EPI_SWIGLU);
-  __shared__ float red[NW][MT][16][17];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  constexpr int BLOCKS = MT + 1, STAGED = STAGES * BLOCKS * 2048;      // a wavefront's stages, where its sums lie afterwards
+  static_assert(STAGES == 0 || STAGED >= MT * 16 * 17 * 4, "a wavefront's sums fit into its stages");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  __shared__ float s_red[STAGES ? 1 : NW][MT][16][17];
+  const auto red = [&](int w, int t, int a, int b) -> float& {
+    if constexpr (STAGES) return reinterpret_cast<float (*)[16][17]>(smem + w * STAGED)[t][a][b];
+    else return s_red[w][t][a][b];
+  };
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r = lane & 15, j = lane >> 4;   // MFMA row / column, and k group
   // the weight row this lane feeds
   int wrow;
@@ -89,6 +103,43 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
   const uint4 zero = make_uint4(0, 0, 0, 0);
   // chunk c covers k in [64 c, 64 c + 64); lane group j takes [64 c + 16 j, +16)
   const int chunks = (K + 63) / 64;
+  if constexpr (STAGES > 0) {
+    const int lr = lane >> 3, piece = ((lane & 7) ^ lr) * 16;
+    const int n0 = blockIdx.x * (SW ? 8 : 16);
+    unsigned voff[BLOCKS][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      voff[0][h] = (unsigned)min((SW ? 0 : 8 * h) + lr, N - 1 - n0) * (unsigned)(K * 2) + piece;
+#pragma unroll
+      for (int t = 0; t < MT; ++t) voff[1 + t][h] = (unsigned)min(16 * t + 8 * h + lr, M - 1) * (unsigned)(lda * 2) + piece;
+    }
+    const auto rows_at = [](const bf16_t* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
+    const auto rsW = rows_at(W + (size_t)n0 * K + wave * 64), rsU = rows_at(W + (size_t)(n0 + (SW ? N : 0)) * K + wave * 64);
+    const auto rsA = rows_at(A + wave * 64);
+    unsigned char* mine = smem + wave * STAGED;
+    const auto load = [&](int step, unsigned stage) {
+#pragma unroll
+      for (int i = 0; i < BLOCKS; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          auto* dst = (__attribute__((address_space(3))) void*)(mine + stage + i * 2048 + h * 1024);      // the same in every lane
+          if (i > 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, dst, 16, voff[i][h], step * NW * 128, 0, 0);
+          else if (SW && h == 1) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsU, dst, 16, voff[i][h], step * NW * 128, 0, 0);
+          else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsW, dst, 16, voff[i][h], step * NW * 128, 0, 0);
+        }
+    };
+    const unsigned at = (unsigned)(size_t)mine + r * 128;
+    const int steps = wave < chunks ? (chunks - wave + NW - 1) / NW : 0;
+    staged_steps<BLOCKS, STAGES, RowPieces>(steps, at + (((2 * j) ^ (r & 7)) << 4), at + (((2 * j + 1) ^ (r & 7)) << 4), load,
+                                            [&](const RowPieces* e) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, e[0].x), __builtin_bit_cast(bf16x8, e[1 + t].x), acc[t], 0, 0, 0);
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, e[0].y), __builtin_bit_cast(bf16x8, e[1 + t].y), acc[t], 0, 0, 0);
+      }
+    });
+  }
+  if constexpr (STAGES == 0)
   for (int c0 = wave; c0 < chunks; c0 += NW * UN) {
     Frag w0[UN], w1[UN], a0[UN][MT], a1[UN][MT];
     bool ok0[UN], ok1[UN];
@@ -125,7 +176,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
 #pragma unroll
   for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[wave][t][r][4 * j + i] = acc[t][i];
+    for (int i = 0; i < 4; ++i) red(wave, t, r, 4 * j + i) = acc[t][i];
   __syncthreads();
   // thread -> (token = tid / 16, row = tid % 16): consecutive threads, consecutive columns
   if (NW > 4 && threadIdx.x >= 256) return;
@@ -140,8 +191,8 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
       float g = 0.f, u = 0.f;
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
-        g += red[w][t][tok][row];
-        u += red[w][t][tok][row + 8];
+        g += red(w, t, tok, row);
+        u += red(w, t, tok, row + 8);
       }
       ((bf16_t*)out_)[(size_t)m * N + n] = f2bf(silu_mul(g, u));
     } else {
@@ -149,13 +200,14 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
       if (n >= N) continue;
       float s = 0.f;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) s += red[w][t][tok][row];
+      for (int w = 0; w < NW; ++w) s += red(w, t, tok, row);
       const size_t o = (size_t)m * N + n;
       if (EPI == TI_EPI_STORE_F32) ((float*)out_)[o] = s;
       if (EPI == TI_EPI_ADD_F32) ((float*)out_)[o] = prev[t] + s;
       if (TI_EPI_ACT(EPI)) ((bf16_t*)out_)[o] = f2bf(epi_act<EPI>(s));
     }
   }
+#endif
 }
 
 // ================================== skinny kernel whose token rows are made in the kernel
@@ -833,12 +885,6 @@ gemm_tiled_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, vo
 // wavefront: the first half holds gate columns, the second the matching up columns.
 #define PBK 64
 #define PSTAGES 3
-
-// s_waitcnt with only vmcnt set (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14)
-template <int N> __device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N <= 63, "vmcnt counts to 63");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
 
 // What the epilogue TI_EPI_QKV_PREP needs: the product is the fused q/k/v projection of a step's
 // rows, and instead of storing it the kernel finishes each head of each row: per-head norm and
@@ -1572,14 +1618,38 @@ static int g_skinny_waves = 0;
 // 1 (default): eight chunks of K in flight per wavefront where its share of K is more than four
 static int g_skinny_deep = 1;
 
+// Stages of the kernel for 17 to 64 rows: all of 1,024 columns under way where a workgroup has its compute unit for itself, room for two
+// workgroups where they share it.
+template <int MT, int EPI, int NW, int STAGES>
+static int launch_skinny_staged(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda, int grid, hipStream_t s) {
+  constexpr int lds = NW * STAGES * (MT + 1) * 2048;
+  auto kernel = gemm_skinny_kernel<MT, EPI, NW, 4, STAGES>;
+  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  TI_REQUIRE(room == hipSuccess, "gemm_bf16: %d bytes of LDS: %s", lds, hipGetErrorString(room));
+  kernel<<<grid, NW * 64, lds, s>>>(A, W, out, M, N, K, lda);
+  return 0;
+}
+
 template <int EPI>
-static void launch_skinny(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda,
+static int launch_skinny(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda,
                           hipStream_t s) {
   const int grid = (EPI == TI_EPI_SWIGLU) ? (N + 7) / 8 : (N + 15) / 16;
   const int mt = (M + 15) / 16;
   int waves = g_skinny_waves;
   // by the weight's shape only, so that a row's bits do not depend on the rows beside it
   if (waves == 0) waves = (grid <= 128 && K >= 1024) ? 8 : 4;
+  // rows within 2 GiB, which is what a buffer's descriptor spans
+  const bool staged = mt > 1 && K % 64 == 0 && lda < (1L << 24) && K < (1 << 24);
+#define TI_STAGED(MTV)                                                                                      \
+  if (mt == MTV && staged) {                                                                               \
+    if (waves == 8) return launch_skinny_staged<MTV, EPI, 8, 2>(A, W, out, M, N, K, lda, grid, s);          \
+    if (grid <= compute_units()) return launch_skinny_staged<MTV, EPI, 4, 4>(A, W, out, M, N, K, lda, grid, s); \
+    return launch_skinny_staged<MTV, EPI, 4, 2>(A, W, out, M, N, K, lda, grid, s);                          \
+  }
+  TI_STAGED(2)
+  TI_STAGED(3)
+  TI_STAGED(4)
+#undef TI_STAGED
 #define TI_SKINNY(MTV)                                                               \
   if (mt == MTV) {                                                                   \
     if (waves == 8)                                                                  \
@@ -1594,13 +1664,14 @@ static void launch_skinny(const bf16_t* A, const bf16_t* W, void* out, int M, in
       gemm_skinny_kernel<1, EPI, 8, 8><<<grid, 512, 0, s>>>(A, W, out, M, N, K, lda);
     else
       gemm_skinny_kernel<1, EPI, 4, 8><<<grid, 256, 0, s>>>(A, W, out, M, N, K, lda);
-    return;
+    return 0;
   }
   TI_SKINNY(1)
   TI_SKINNY(2)
   TI_SKINNY(3)
   TI_SKINNY(4)
 #undef TI_SKINNY
+  return 0;
 }
 
 template <int EPI>
@@ -1625,17 +1696,23 @@ static int g_use_pipelined = 1;
 // gate/up at 16 rows: 72 us with the norm inside, 62 us as norm + tiled product; Qwen3-4B's: 50
 // against 37 us); from rows x weight elements = 600 Mi on these take the tiled kernels too, and
 // the norm a kernel of its own.  (At 9 to 12 rows that was measured as well, and loses.)
+// With the rows through LDS the 16-row workgroups hold out longer where the product stores and is not cut over K (which it is into
+// the residual, and from K = 4096 on): to 1000 Mi (us, tiles and 16-row workgroups: 6144 x 2560 at 64 rows, 960 Mi, 16.7 and 16.5, at 32
+// 14.7 and 12.0; [gate; up] 12288 x 2048 at 48 rows, 1152 Mi, 17.8 and 16.3, at 64, 1536 Mi, 18.4 and 18.6; 19456 x 2560 at 17 rows,
+// 807 Mi, 24.7 and 23.9, at 32, 1520 Mi, 26.4 and 28.7).
 static long g_tiled_from = 280L << 20;           // 17..64 rows x weight elements from which steps take the tiled kernels
 static long g_tiled_from_16 = 600L << 20;        // the same for 13..16 rows
+#define TILED_FROM_STORED (1000L << 20)
+static long g_tiled_from_stored = TILED_FROM_STORED;      // the same for 17..64 rows whose product stores, K below 4096
 static void set_tiled_from(long rows_times_elems) {
-  g_tiled_from = rows_times_elems;
+  g_tiled_from = g_tiled_from_stored = rows_times_elems;
   g_tiled_from_16 = rows_times_elems >= (280L << 20) && rows_times_elems < (1L << 59) ? rows_times_elems / 280 * 600
                                                                                      : rows_times_elems;
 }
 static bool large_weight(int M, int N, int K, int epi) {
   const long rows = (epi == TI_EPI_SWIGLU) ? 2L * N : (long)N;
   if (M <= 12 || M > 64 || K % PBK != 0) return false;
-  return rows * K * M >= (M <= 16 ? g_tiled_from_16 : g_tiled_from);
+  return rows * K * M >= (M <= 16 ? g_tiled_from_16 : epi == TI_EPI_ADD_F32 || K >= 4096 ? g_tiled_from : g_tiled_from_stored);
 }
 
 // 1 (default): up to GR_MMAX tokens and a weight of fewer than GR_ROWS_BELOW rows take the kernel
@@ -1797,25 +1874,30 @@ static int launch_skinny_copied(const bf16_t* A, const bf16_t* W, void* out, int
 }
 
 // ---------------------------------------------------------------------------------------------
-// 17 to 64 rows: 16x16x32 MFMAs fed straight from memory.  A workgroup takes 16 rows of W (16
+// 17 to 64 rows: 16x16x32 MFMAs fed through LDS (staged_rows.h).  A workgroup takes 16 rows of W (16
 // output columns; SwiGLU: 8 gate and 8 up rows) and a range of K; its four wavefronts take the
-// 64-wide k-blocks of that range in turn, each block as MB + 1 pairs of 16-byte loads per lane
-// (lane -> row lane % 16, 8 k at 8 (lane / 16), first and second half of the block) and 2 MB
-// MFMAs over all 16 MB rows of A.  The four wavefronts' sums meet in LDS, in the order 0..3.
+// 64-wide k-blocks of that range in turn, each block as MB + 1 blocks of rows (a lane's two pieces: 8 k at 8 (lane / 16) in the first
+// and in the second half) and 2 MB MFMAs over all 16 MB rows of A.  (Operands straight from memory: 1024 x 3072 at 64 rows 6.0 us, now
+// 4.5; 1024 x 2048 4.9, now 4.6; 2048 x 2048 7.1, now 5.3; up to 32 rows the same.)  The four wavefronts' sums meet in LDS, in the order 0..3.
 // With a weight of few rows the launch would fill a fraction of the compute units and every
 // workgroup would pull in all of A: then K is split over KS workgroups, which leave their sums
 // in `partial` [KS][M][N], and gemm_partials_add_kernel adds them to the residual in the order
 // 0..KS-1.  A row's bits do not depend on the other rows.
+#define MBK_STAGES 2
 #define MBK_STRIDE 20   // floats per row of the LDS tile: the 4 x 16 lanes of a store hit 64 banks
 
 template <int MB, int EPI>
 __global__ void __launch_bounds__(256)
 gemm_mblocks_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ out_,
                     float* __restrict__ partial, int M, int N, int K, long lda) {
+#if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass has no buffer descriptors)
   constexpr bool SW = (EPI == TI_EPI_SWIGLU);
   constexpr int TILE = SW ? 8 : 16;                          // output columns of a workgroup
-  __shared__ __attribute__((aligned(16))) float red[4][MB * 16][MBK_STRIDE];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  constexpr int BLOCKS = MB + 1, STAGES = MBK_STAGES, STAGED = STAGES * BLOCKS * 2048;
+  static_assert(4 * STAGED >= 4 * MB * 16 * MBK_STRIDE * 4, "the sums fit into the stages");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  float (*red)[MB * 16][MBK_STRIDE] = reinterpret_cast<float (*)[MB * 16][MBK_STRIDE]>(smem);
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int r = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * TILE;
   const int KS = gridDim.y, split = blockIdx.y;
@@ -1823,46 +1905,43 @@ gemm_mblocks_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, 
   const int kb0 = (int)((long)nb * split / KS), kb1 = (int)((long)nb * (split + 1) / KS);
 
   // rows outside the matrices read a valid row; what they give is not stored
-  const bf16_t* arow[MB];
+  unsigned voff[BLOCKS][2];
+  const int lr = lane >> 3, piece = ((lane & 7) ^ lr) * 16;
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) arow[mb] = A + (size_t)min(mb * 16 + r, M - 1) * lda + g * 8;
-  int wr;
-  if (SW) wr = (r < 8) ? min(n0 + r, N - 1) : N + min(n0 + r - 8, N - 1);
-  else wr = min(n0 + r, N - 1);
-  const bf16_t* wrow = W + (size_t)wr * K + g * 8;
-
-  struct Block { uint4 a[MB][2]; uint4 b[2]; };
-  auto load = [&](Block& f, int kb) {
-    const int k = kb * 64;
-    f.b[0] = *reinterpret_cast<const uint4*>(wrow + k);
-    f.b[1] = *reinterpret_cast<const uint4*>(wrow + k + 32);
+  for (int h = 0; h < 2; ++h) {
+    voff[0][h] = (unsigned)min((SW ? 0 : 8 * h) + lr, N - 1 - n0) * (unsigned)(K * 2) + piece;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      f.a[mb][0] = *reinterpret_cast<const uint4*>(arow[mb] + k);
-      f.a[mb][1] = *reinterpret_cast<const uint4*>(arow[mb] + k + 32);
-    }
+    for (int mb = 0; mb < MB; ++mb) voff[1 + mb][h] = (unsigned)min(mb * 16 + 8 * h + lr, M - 1) * (unsigned)(lda * 2) + piece;
+  }
+  const auto rows_at = [](const bf16_t* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
+  const size_t k0 = (size_t)(kb0 + wave) * 64;
+  const auto rsW = rows_at(W + (size_t)n0 * K + k0), rsU = rows_at(W + (size_t)(n0 + (SW ? N : 0)) * K + k0), rsA = rows_at(A + k0);
+  unsigned char* mine = smem + wave * STAGED;
+  const auto load = [&](int step, unsigned stage) {
+#pragma unroll
+    for (int i = 0; i < BLOCKS; ++i)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        auto* dst = (__attribute__((address_space(3))) void*)(mine + stage + i * 2048 + h * 1024);      // the same in every lane
+        if (i > 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, dst, 16, voff[i][h], step * 4 * 128, 0, 0);
+        else if (SW && h == 1) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsU, dst, 16, voff[i][h], step * 4 * 128, 0, 0);
+        else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsW, dst, 16, voff[i][h], step * 4 * 128, 0, 0);
+      }
   };
   floatx4 acc[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) acc[mb] = floatx4{0.f, 0.f, 0.f, 0.f};
-  int kb = kb0 + wave;
-  if (kb < kb1) {
-    Block cur;
-    load(cur, kb);
-    while (kb < kb1) {
-      // the next block is asked for before this one is multiplied (after the last one, the last again)
-      Block next;
-      load(next, min(kb + 4, kb1 - 1));
+  const unsigned at = (unsigned)(size_t)mine + r * 128;
+  const int steps = kb0 + wave < kb1 ? (kb1 - kb0 - wave + 3) / 4 : 0;
+  staged_steps<BLOCKS, STAGES, RowPieces>(steps, at + ((g ^ (r & 7)) << 4), at + (((g + 4) ^ (r & 7)) << 4), load, [&](const RowPieces* e) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+    for (int mb = 0; mb < MB; ++mb)
+      acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, e[1 + mb].x), __builtin_bit_cast(bf16x8, e[0].x), acc[mb], 0, 0, 0);
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-          acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, cur.a[mb][h]),
-                                                            __builtin_bit_cast(bf16x8, cur.b[h]), acc[mb], 0, 0, 0);
-      cur = next;
-      kb += 4;
-    }
-  }
+    for (int mb = 0; mb < MB; ++mb)
+      acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, e[1 + mb].y), __builtin_bit_cast(bf16x8, e[0].y), acc[mb], 0, 0, 0);
+  });
+  __syncthreads();                                           // the stages are free
   // acc[mb][q]: row 16 mb + 4 g + q, column r
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
@@ -1903,6 +1982,7 @@ gemm_mblocks_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, 
     else if (EPI == TI_EPI_STORE_F32) ((float*)out_)[o] = v[i];
     else ((bf16_t*)out_)[o] = f2bf(epi_act<EPI>(v[i]));
   }
+#endif
 }
 
 // out[i] += partial[0][i] + ... + partial[KS - 1][i], in that order
@@ -2099,15 +2179,21 @@ static int g_add_split = 1;        // a hook for measurements: 0: ti_gemm_bf16_a
 #define STREAMED_WEIGHT (24L << 20)
 
 template <int EPI>
-static void launch_mblocks(const bf16_t* a, const bf16_t* w, void* out, float* partial, int M, int N, int K,
+static int launch_mblocks(const bf16_t* a, const bf16_t* w, void* out, float* partial, int M, int N, int K,
                            long lda, int KS, hipStream_t s) {
   const int tile = (EPI == TI_EPI_SWIGLU) ? 8 : 16;
   dim3 grid((N + tile - 1) / tile, KS);
   const int mb = (M + 15) / 16;
-  if (mb == 1) gemm_mblocks_kernel<1, EPI><<<grid, 256, 0, s>>>(a, w, out, partial, M, N, K, lda);
-  else if (mb == 2) gemm_mblocks_kernel<2, EPI><<<grid, 256, 0, s>>>(a, w, out, partial, M, N, K, lda);
-  else if (mb == 3) gemm_mblocks_kernel<3, EPI><<<grid, 256, 0, s>>>(a, w, out, partial, M, N, K, lda);
-  else gemm_mblocks_kernel<4, EPI><<<grid, 256, 0, s>>>(a, w, out, partial, M, N, K, lda);
+  const int lds = 4 * MBK_STAGES * (mb + 1) * 2048;
+  if (mb == 1) gemm_mblocks_kernel<1, EPI><<<grid, 256, lds, s>>>(a, w, out, partial, M, N, K, lda);
+  else if (mb == 2) gemm_mblocks_kernel<2, EPI><<<grid, 256, lds, s>>>(a, w, out, partial, M, N, K, lda);
+  else if (mb == 3) gemm_mblocks_kernel<3, EPI><<<grid, 256, lds, s>>>(a, w, out, partial, M, N, K, lda);
+  else {
+    static const hipError_t room = hipFuncSetAttribute((const void*)gemm_mblocks_kernel<4, EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    TI_REQUIRE(room == hipSuccess, "gemm_bf16: %d bytes of LDS: %s", lds, hipGetErrorString(room));
+    gemm_mblocks_kernel<4, EPI><<<grid, 256, lds, s>>>(a, w, out, partial, M, N, K, lda);
+  }
+  return 0;
 }
 
 // out[i] += partial[0][i] + ... + partial[KS - 1][i] for count elements: what a product with a split
@@ -2156,7 +2242,7 @@ extern "C" int ti_gemm_bf16_add_split(const void* A, const void* W, void* out, i
     }
   }
   int KS = 1, tile = 0;      // (tile: of the pipelined kernel, 0: not taken)
-  const bool small = M <= 64 && !(large_weight(M, N, K, epi) && g_use_pipelined);
+  const bool small = M <= 64 && lda < (1L << 24) && !(large_weight(M, N, K, epi) && g_use_pipelined);
   if (g_add_split && epi == TI_EPI_ADD_F32 && partial && M > 16 && K % 64 == 0 && lda % 8 == 0 &&
       !((uintptr_t)A & 15) && !((uintptr_t)W & 15) && !((uintptr_t)partial & 15) && (small || g_use_pipelined)) {
     const int nb = K / 64;
@@ -2205,7 +2291,8 @@ extern "C" int ti_gemm_bf16_add_split(const void* A, const void* W, void* out, i
     return 3;
   }
   if (small) {
-    launch_mblocks<TI_EPI_ADD_F32>((const bf16_t*)A, (const bf16_t*)W, out, (float*)partial, M, N, K, lda, KS, stream);
+    int rc_ = launch_mblocks<TI_EPI_ADD_F32>((const bf16_t*)A, (const bf16_t*)W, out, (float*)partial, M, N, K, lda, KS, stream);
+    if (rc_) return rc_;
   } else {
     int rc_ = launch_tile<TI_EPI_STORE_F32>(tile, (const bf16_t*)A, (const bf16_t*)W, partial, M, N, K, lda, stream, KS);
     if (rc_) return rc_;
@@ -2299,19 +2386,20 @@ extern "C" int ti_gemm_bf16_store_split(const void* A, const void* W, void* out,
 // are added here)
 extern "C" int ti_gemm_bf16_mblocks_any(const void* A, const void* W, void* out, int M, int N, int K, long lda,
                                         int epi, void* partial, int ks, hipStream_t stream) {
-  TI_REQUIRE(M > 0 && M <= 64 && N > 0 && K > 0 && K % 64 == 0 && lda >= K && lda % 8 == 0 && ks >= 1 && ks <= K / 64,
+  TI_REQUIRE(M > 0 && M <= 64 && N > 0 && K > 0 && K % 64 == 0 && lda >= K && lda % 8 == 0 && lda < (1L << 24) && ks >= 1 && ks <= K / 64,
              "gemm_bf16_mblocks_any: bad sizes M=%d N=%d K=%d lda=%ld ks=%d", M, N, K, lda, ks);
   TI_REQUIRE(ks == 1 || (epi == TI_EPI_ADD_F32 && partial), "gemm_bf16_mblocks_any: a split K needs the adding epilogue");
   const bf16_t* a = (const bf16_t*)A;
   const bf16_t* w = (const bf16_t*)W;
+  int rc_ = 0;
   switch (epi) {
-    case TI_EPI_STORE_F32: launch_mblocks<TI_EPI_STORE_F32>(a, w, out, nullptr, M, N, K, lda, 1, stream); break;
-    case TI_EPI_STORE_ACT: launch_mblocks<TI_EPI_STORE_ACT>(a, w, out, nullptr, M, N, K, lda, 1, stream); break;
-    case TI_EPI_RELU2: launch_mblocks<TI_EPI_RELU2>(a, w, out, nullptr, M, N, K, lda, 1, stream); break;
-    case TI_EPI_SWIGLU: launch_mblocks<TI_EPI_SWIGLU>(a, w, out, nullptr, M, N, K, lda, 1, stream); break;
+    case TI_EPI_STORE_F32: rc_ = launch_mblocks<TI_EPI_STORE_F32>(a, w, out, nullptr, M, N, K, lda, 1, stream); break;
+    case TI_EPI_STORE_ACT: rc_ = launch_mblocks<TI_EPI_STORE_ACT>(a, w, out, nullptr, M, N, K, lda, 1, stream); break;
+    case TI_EPI_RELU2: rc_ = launch_mblocks<TI_EPI_RELU2>(a, w, out, nullptr, M, N, K, lda, 1, stream); break;
+    case TI_EPI_SWIGLU: rc_ = launch_mblocks<TI_EPI_SWIGLU>(a, w, out, nullptr, M, N, K, lda, 1, stream); break;
     case TI_EPI_ADD_F32:
-      launch_mblocks<TI_EPI_ADD_F32>(a, w, out, (float*)partial, M, N, K, lda, ks, stream);
-      if (ks > 1) {
+      rc_ = launch_mblocks<TI_EPI_ADD_F32>(a, w, out, (float*)partial, M, N, K, lda, ks, stream);
+      if (rc_ == 0 && ks > 1) {
         const size_t count = (size_t)M * N;
         gemm_partials_add_kernel<<<(unsigned)((count + 255) / 256), 256, 0, stream>>>((float*)out, (const float*)partial,
                                                                                     ks, count);
@@ -2320,6 +2408,7 @@ extern "C" int ti_gemm_bf16_mblocks_any(const void* A, const void* W, void* out,
     default:
       TI_REQUIRE(false, "gemm_bf16_mblocks_any: unknown epilogue %d", epi);
   }
+  if (rc_) return rc_;
   TI_LAUNCH_CHECK();
   return 0;
 }
@@ -2375,9 +2464,10 @@ extern "C" int ti_gemm_bf16(const void* A, const void* W, void* out, int M, int 
     if (copied) {                                                 \
       int rc_ = launch_skinny_copied<E>(a, w, out, M, N, K, lda, stream); \
       if (rc_) return rc_;                                        \
-    } else if (skinny)                                            \
-      launch_skinny<E>(a, w, out, M, N, K, lda, stream);          \
-    else if (g_use_pipelined && pipelined_serves(K, lda)) {    \
+    } else if (skinny) {                                          \
+      int rc_ = launch_skinny<E>(a, w, out, M, N, K, lda, stream); \
+      if (rc_) return rc_;                                        \
+    } else if (g_use_pipelined && pipelined_serves(K, lda)) {    \
       int rc_ = launch_tiled_best<E>(a, w, out, M, N, K, lda, stream); \
       if (rc_) return rc_;                                        \
     } else                                                        \
@@ -2404,7 +2494,7 @@ extern "C" int ti_gemm_bf16(const void* A, const void* W, void* out, int M, int 
 // overrides around its calls and resets them afterwards.  Returns 0, or 1 for an unknown name.
 extern "C" void ti_tuning_reset() {
   g_xcd_rows = 0; g_die_order = 1; g_tiles_160 = 1; g_tiles_256 = 1; g_two_ranges = 1; g_qkv_rows = 0; g_qkv_min_rows = 17; g_force_tile = 0; g_skinny_waves = 0;
-  g_skinny_deep = 1; g_use_pipelined = 1; set_tiled_from(280L << 20); g_row_per_wave = 1;
+  g_skinny_deep = 1; g_use_pipelined = 1; set_tiled_from(280L << 20); g_tiled_from_stored = TILED_FROM_STORED; g_row_per_wave = 1;
   g_normed_weight_below = NORMED_WEIGHT_BELOW; g_skinny_copy = 1; g_wide_rows = 1; g_pieces = 1; g_add_split = 1;
   g_rows_direct = 1;
   g_wide_rows_min_n = WIDE_ROWS_MIN_N;

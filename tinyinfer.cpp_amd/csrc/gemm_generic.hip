@@ -14,6 +14,7 @@
 #include <type_traits>
 #include "common.h"
 #include "tinyinfer_kernels.h"
+#include "staged_rows.h"
 
 TI_ERROR_API
 
@@ -130,10 +131,8 @@ static int launch(const void* A, const void* W, void* out, int M, int N, int K, 
 // What the three pieces cannot hold (infinite, not a number, above the largest bfloat16) leaves a sum that is not finite; such an element
 // is computed again by fused multiply-adds.  (Below 2^-110 the last piece may lie below the normal numbers, 2^-133 at least.)
 //
-// A wavefront's rows come through its own part of LDS by direct loads, eight lanes to a row's 128 bytes, and are read back as the operands
-// lie.  (Loaded as operands straight into registers, neighbouring lanes ask for different rows: 64 cycles a load of 1 KiB whatever the
-// tile, four times what the direct loads take, and all that bounded these products.)  No barrier: a wavefront waits for its own loads,
-// and asks for the next step as soon as it has read one.  What bounds them now is the splitting (52 instructions a block of 16 rows
+// A wavefront's rows come through its own part of LDS by direct loads (staged_rows.h; loaded as operands straight into registers they were
+// all that bounded these products).  What bounds them now is the splitting (52 instructions a block of 16 rows
 // and step beside 16 cycles each of six matrix instructions a pair of blocks), and for 1,024 columns the ends: the first loads and the
 // sums' way through LDS are a third of the 13 us.
 // us a call, before (32-bit instructions, operands straight from memory) and now: 300 rows x 4096 x 1024 36.9 -> 25.7, [gate; up]
@@ -187,34 +186,7 @@ __device__ __forceinline__ float dot_by_fma(const float* __restrict__ a, const f
   return total;
 }
 
-// s_waitcnt with only vmcnt set (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14)
-template <int N> __device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N <= 63, "vmcnt counts to 63");
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
 struct Eight { gf4 x, y; };      // eight consecutive k of one row
-// N blocks of 16 rows of a stage, the first at LDS byte `at`, have arrived in registers when this returns; x, y: a lane's two pieces
-template <int N> __device__ __forceinline__ void read_blocks(Eight* e, unsigned x, unsigned y) {
-  static_assert(N >= 1 && N <= 4, "up to eight reads at a time");
-  if constexpr (N == 1)
-    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(e[0].x), "=&v"(e[0].y) : "v"(x), "v"(y) : "memory");
-  if constexpr (N == 2)
-    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %4 offset:2048\n\tds_read_b128 %3, %5 offset:2048\n\t"
-                 "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(e[0].x), "=&v"(e[0].y), "=&v"(e[1].x), "=&v"(e[1].y) : "v"(x), "v"(y) : "memory");
-  if constexpr (N == 3)
-    asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %7\n\tds_read_b128 %2, %6 offset:2048\n\tds_read_b128 %3, %7 offset:2048\n\t"
-                 "ds_read_b128 %4, %6 offset:4096\n\tds_read_b128 %5, %7 offset:4096\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(e[0].x), "=&v"(e[0].y), "=&v"(e[1].x), "=&v"(e[1].y), "=&v"(e[2].x), "=&v"(e[2].y)
-                 : "v"(x), "v"(y) : "memory");
-  if constexpr (N == 4)
-    asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\tds_read_b128 %2, %8 offset:2048\n\tds_read_b128 %3, %9 offset:2048\n\t"
-                 "ds_read_b128 %4, %8 offset:4096\n\tds_read_b128 %5, %9 offset:4096\n\tds_read_b128 %6, %8 offset:6144\n\t"
-                 "ds_read_b128 %7, %9 offset:6144\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(e[0].x), "=&v"(e[0].y), "=&v"(e[1].x), "=&v"(e[1].y), "=&v"(e[2].x), "=&v"(e[2].y), "=&v"(e[3].x), "=&v"(e[3].y)
-                 : "v"(x), "v"(y) : "memory");
-}
 
 template <int RB, int NB, bool SW> struct F32Tile {
   static constexpr int PL = SW ? 2 : 1;               // planes of weight rows: gate and up
@@ -275,9 +247,7 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
   const int k0 = wave * run, k1 = min(K, k0 + run);
   const int steps = k1 > k0 ? (k1 - k0) / GF_STEP : 0;   // whole steps; what is left of K is a step of its own
   if (steps > 0) {
-    // A load of 1 KiB covers eight rows of a block: eight lanes a row, its 128 bytes in pieces of 16, piece c of row r in place
-    // c ^ (r & 7), so that the sixteen rows that are read together lie in different banks.  Rows past the end repeat the last one;
-    // their sums are not stored.
+    // Rows past the end repeat the last one; their sums are not stored.
     unsigned voff[BLOCKS][2];
     const int lr = lane >> 3, piece = (lane & 7) ^ lr;
 #pragma unroll
@@ -302,27 +272,7 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
         }
     };
     const unsigned at = (unsigned)(size_t)mine + r16 * 128, x = at + (((2 * quad) ^ (r16 & 7)) << 4), y = at + (((2 * quad + 1) ^ (r16 & 7)) << 4);
-#pragma unroll
-    for (int d = 0; d < STAGES; ++d)
-      if (d < steps) load(d, d * T::STEP_BYTES);
-    unsigned stage = 0;
-    for (int i = 0; i < steps; ++i) {
-      // this step's loads are back; those of the steps behind it may still be out
-      const int behind = min(STAGES, steps - i) - 1;      // the same in every lane
-      if (STAGES >= 4 && behind == 3) wait_vmcnt<STAGES >= 4 ? 6 * BLOCKS : 0>();
-      else if (STAGES >= 3 && behind == 2) wait_vmcnt<STAGES >= 3 ? 4 * BLOCKS : 0>();
-      else if (STAGES >= 2 && behind == 1) wait_vmcnt<STAGES >= 2 ? 2 * BLOCKS : 0>();
-      else wait_vmcnt<0>();
-      Eight e[BLOCKS];
-      constexpr int R = BLOCKS % 4;
-#pragma unroll
-      for (int b = 0; b + 4 <= BLOCKS; b += 4) read_blocks<4>(e + b, x + stage + b * 2048, y + stage + b * 2048);
-      if constexpr (R) read_blocks<(R ? R : 1)>(e + BLOCKS - R, x + stage + (BLOCKS - R) * 2048, y + stage + (BLOCKS - R) * 2048);
-      if (i + STAGES < steps) load(i + STAGES, stage);
-      __builtin_amdgcn_sched_barrier(0);
-      multiply(e);
-      stage = stage == (STAGES - 1) * T::STEP_BYTES ? 0 : stage + T::STEP_BYTES;
-    }
+    staged_steps<BLOCKS, STAGES, Eight>(steps, x, y, load, multiply);
   }
   if (k1 > k0 && (k1 - k0) % GF_STEP) {
     const int k = k0 + steps * GF_STEP + quad * 8;
