@@ -995,6 +995,34 @@ def test_linear_bf16_rows_through_lds_at_17_to_64_rows(ops, N, K):
         assert (f64(out) - ref[:M]).abs().max() < tol, M
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 4104, 2112), (5, 40, 64), (8, 2056, 4160), (13, 1000, 1088), (16, 6144, 2048)])
+def test_linear_bf16_rows_through_lds_up_to_16_rows(ops, M, N, K):
+    """Up to 16 rows through LDS stages: fewer steps than stages, four and eight wavefronts, a last tile of few weight rows.  Every
+    epilogue gives the bits of the kernels that took these products before (the sums are in the same order), and what lies beyond is left."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = dev((torch.rand(M, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    w = dev((torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    lib, outs = ops.lib("gemm_bf16"), {}
+    lib.ti_tuning_reset()
+    try:
+        for on in (1, 0):
+            lib.ti_tuning_set(b"rows_staged", on)
+            lib.ti_tuning_set(b"row_per_wave", 0)
+            store, pair = torch.full((M + 1, N), 7.0, device="cuda"), torch.full((M + 1, N // 2), 7.0, device="cuda", dtype=torch.bfloat16)
+            act, add = torch.empty(M, N, device="cuda", dtype=torch.bfloat16), torch.ones(M, N, device="cuda")
+            ops.linear(a, w, store[:M], "store")
+            ops.linear(a, w, pair[:M], "swiglu")
+            ops.linear(a, w, act, "store_act")
+            ops.linear(a, w, add, "add")
+            outs[on] = (store, pair, act, add)
+    finally:
+        lib.ti_tuning_reset()
+    for x, y in zip(outs[1], outs[0]):
+        assert torch.equal(x, y)
+    assert bool((outs[1][0][M] == 7.0).all()) and bool((outs[1][1][M] == 7.0).all())
+    assert (f64(outs[1][0][:M]) - ref_linear(a.cpu(), w.cpu())).abs().max() < 2e-5 * K
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 16400, 64), (64, 20000, 1024), (40, 16387, 2048), (33, 17000, 192),
                                    (48, 16384, 1088)])
 def test_linear_bf16_wide_weight_at_17_to_64_rows(ops, M, N, K):

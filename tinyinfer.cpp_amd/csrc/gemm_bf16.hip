@@ -1618,7 +1618,19 @@ static int g_skinny_waves = 0;
 // 1 (default): eight chunks of K in flight per wavefront where its share of K is more than four
 static int g_skinny_deep = 1;
 
-// Stages of the kernel for 17 to 64 rows: all of 1,024 columns under way where a workgroup has its compute unit for itself, room for two
+// rows within 2 GiB, which is what a buffer's descriptor spans
+static bool staged_fits(int K, long lda) { return K % 64 == 0 && lda < (1L << 24) && K < (1 << 24); }
+// Up to 16 rows of it as well (us, by rows in pieces, rows copied to LDS or a weight row a wavefront, and this; the same bits as the
+// former two): 6144 x 4096 under 1 and 8 rows 12.5 13.9 -> 10.5 10.7, [gate; up] 24576 x 4096 34.1 37.5 -> 32.6 33.2, 4096 x 4096 8.9 9.9 ->
+// 7.7 7.9, 4096 x 12288 20.7 22.0 -> 17.5 17.4, 2560 x 9728 14.8 17.0 -> 10.6 12.0, [gate; up] 6144 x 1024 5.2 5.3 -> 4.2 4.3,
+// 151936 x 1024 52.8 61.0 -> 49.0 53.8.  But a weight of a quarter of a GiB and more keeps the pieces under up to
+// 8 rows (151936 x 2048 104 and 117, here 112 and 122; 151936 x 4096 195 and 207, here 203 and 207).
+static int g_rows_staged = 1;      // a hook for measurements: 0: up to 16 rows take the other kernels
+static bool staged_16_serves(int M, int N, int K, long lda, int epi) {
+  const long elements = (epi == TI_EPI_SWIGLU ? 2L * N : (long)N) * K;
+  return g_rows_staged && M <= 16 && staged_fits(K, lda) && (M > 8 || elements < (288L << 20));
+}
+// Stages of the kernel for up to 64 rows: all of 1,024 columns under way where a workgroup has its compute unit for itself, room for two
 // workgroups where they share it.
 template <int MT, int EPI, int NW, int STAGES>
 static int launch_skinny_staged(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda, int grid, hipStream_t s) {
@@ -1638,14 +1650,14 @@ static int launch_skinny(const bf16_t* A, const bf16_t* W, void* out, int M, int
   int waves = g_skinny_waves;
   // by the weight's shape only, so that a row's bits do not depend on the rows beside it
   if (waves == 0) waves = (grid <= 128 && K >= 1024) ? 8 : 4;
-  // rows within 2 GiB, which is what a buffer's descriptor spans
-  const bool staged = mt > 1 && K % 64 == 0 && lda < (1L << 24) && K < (1 << 24);
+  const bool staged = (mt > 1 && staged_fits(K, lda)) || staged_16_serves(M, N, K, lda, EPI);
 #define TI_STAGED(MTV)                                                                                      \
   if (mt == MTV && staged) {                                                                               \
     if (waves == 8) return launch_skinny_staged<MTV, EPI, 8, 2>(A, W, out, M, N, K, lda, grid, s);          \
     if (grid <= compute_units()) return launch_skinny_staged<MTV, EPI, 4, 4>(A, W, out, M, N, K, lda, grid, s); \
     return launch_skinny_staged<MTV, EPI, 4, 2>(A, W, out, M, N, K, lda, grid, s);                          \
   }
+  TI_STAGED(1)
   TI_STAGED(2)
   TI_STAGED(3)
   TI_STAGED(4)
@@ -1726,6 +1738,9 @@ static int g_row_per_wave = 1;
 // against 7.5 us at 8 tokens), not for more rows (Qwen3-4B's o, 2,560 x 4,096: 10.8 us here, 6.1 in
 // workgroups of 16 rows; 1.7B's, 2,048 x 2,048: 3.9 against 3.0).
 static bool row_per_wave_serves(int M, int N, int K, int epi) {
+  // A weight of more than 8 Mi elements streams better with its rows through LDS stages (2048 x 6144 under 1 and 8 rows 9.4 and 11.0 us here,
+  // 7.1 and 8.2 there); a smaller one is a matter of the chain of launches (o and down of 0.6B: a step of 1 request 775 us, there 829).
+  if (g_rows_staged && K % 64 == 0 && (long)N * K > (8L << 20)) return false;
   return g_row_per_wave && M <= GR_MMAX && N < GR_ROWS_BELOW && (M <= 4 || N <= 4 * compute_units()) && K % 8 == 0 &&
          K <= 64 * 8 * GR_LOADS && (epi == TI_EPI_STORE_F32 || epi == TI_EPI_ADD_F32 || epi == TI_EPI_RELU2);
 }
@@ -2431,8 +2446,9 @@ extern "C" int ti_gemm_bf16(const void* A, const void* W, void* out, int M, int 
   const bf16_t* a = (const bf16_t*)A;
   const bf16_t* w = (const bf16_t*)W;
   const bool skinny = M <= 64 && !(large_weight(M, N, K, epi) && g_use_pipelined);
-  const bool copied = g_skinny_copy && M <= 16 && K % 64 == 0 && K <= 4096 && skinny;
-  if (pieces_serves(M, N, K, epi)) {
+  const bool staged = staged_16_serves(M, N, K, lda, epi) && (skinny || pieces_serves(M, N, K, epi));
+  const bool copied = !staged && g_skinny_copy && M <= 16 && K % 64 == 0 && K <= 4096 && skinny;
+  if (!staged && pieces_serves(M, N, K, epi)) {
     int rc_ = 0;
     switch (epi) {
       case TI_EPI_STORE_F32: rc_ = launch_pieces<TI_EPI_STORE_F32, false>(a, lda, w, out, nullptr, M, N, K, 1, stream); break;
@@ -2464,7 +2480,7 @@ extern "C" int ti_gemm_bf16(const void* A, const void* W, void* out, int M, int 
     if (copied) {                                                 \
       int rc_ = launch_skinny_copied<E>(a, w, out, M, N, K, lda, stream); \
       if (rc_) return rc_;                                        \
-    } else if (skinny) {                                          \
+    } else if (skinny || staged) {                                \
       int rc_ = launch_skinny<E>(a, w, out, M, N, K, lda, stream); \
       if (rc_) return rc_;                                        \
     } else if (g_use_pipelined && pipelined_serves(K, lda)) {    \
@@ -2494,7 +2510,7 @@ extern "C" int ti_gemm_bf16(const void* A, const void* W, void* out, int M, int 
 // overrides around its calls and resets them afterwards.  Returns 0, or 1 for an unknown name.
 extern "C" void ti_tuning_reset() {
   g_xcd_rows = 0; g_die_order = 1; g_tiles_160 = 1; g_tiles_256 = 1; g_two_ranges = 1; g_qkv_rows = 0; g_qkv_min_rows = 17; g_force_tile = 0; g_skinny_waves = 0;
-  g_skinny_deep = 1; g_use_pipelined = 1; set_tiled_from(280L << 20); g_tiled_from_stored = TILED_FROM_STORED; g_row_per_wave = 1;
+  g_skinny_deep = 1; g_use_pipelined = 1; set_tiled_from(280L << 20); g_tiled_from_stored = TILED_FROM_STORED; g_row_per_wave = 1; g_rows_staged = 1;
   g_normed_weight_below = NORMED_WEIGHT_BELOW; g_skinny_copy = 1; g_wide_rows = 1; g_pieces = 1; g_add_split = 1;
   g_rows_direct = 1;
   g_wide_rows_min_n = WIDE_ROWS_MIN_N;
@@ -2512,6 +2528,7 @@ extern "C" int ti_tuning_set(const char* name, long value) {
   else if (n == "skinny_waves") g_skinny_waves = (int)value;
   else if (n == "qkv_prep_min_rows") g_qkv_min_rows = (int)value;
   else if (n == "qkv_prep_rows") g_qkv_rows = (int)value;
+  else if (n == "rows_staged") g_rows_staged = (int)value;
   else if (n == "wide_rows") g_wide_rows = (int)value;
   else if (n == "tiled_from") set_tiled_from(value);
   else if (n == "add_split") g_add_split = (int)value;

@@ -24,6 +24,7 @@
 //   add_split            0: ti_gemm_bf16_add_split serves nothing
 //   use_pipelined        0: the plain tiled kernel for every K
 //   row_per_wave         0: few tokens and a weight of few rows take the 16-row kernels too
+//   rows_staged          0: up to 16 rows never take the kernel whose rows come through LDS stages of each wavefront's own
 //   skinny_copy          0: up to 16 tokens, fragments of the token rows straight from memory
 //   pieces               0: up to 16 rows never take the kernel with the token rows in pieces
 //   skinny_deep          0: four chunks of K in flight per wavefront also for a long K
