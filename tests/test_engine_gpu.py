@@ -299,6 +299,53 @@ def test_prepared_decode_attention_changes_only_rounding(model_folders):
         assert not np.array_equal(results[0][r][:1], results[0][r][1:2])
 
 
+@pytest.fixture(scope="module")
+def wide_headed(tmp_path_factory):
+    """Folders of a model with heads of 128, three a group: without a window and with one of 300."""
+    from tinyinfer_amd.weights import write_model_folder
+    made = {}
+    for window in (None, 300):
+        cfg = dict(ODD_CONFIGS["three heads a group, head 128"])
+        if window:
+            cfg.update(use_sliding_window=True, sliding_window=window, max_window_layers=0)
+        made[window] = (str(tmp_path_factory.mktemp("wide_headed")), cfg["vocab_size"])
+        write_model_folder(made[window][0], cfg, seed=77, dtype="bfloat16")
+        sharpen_folder(made[window][0])
+    return made
+
+
+@pytest.mark.parametrize("window", [None, 300])
+@pytest.mark.parametrize("graph,records", [(False, True), (True, True), (False, False)])
+def test_rows_of_very_different_lengths_by_records(wide_headed, window, graph, records):
+    """Rows of 1 to some 1,300 cached tokens decode together, before, beside and after portions of another request (one launch with the
+    rows), so that the attention cuts some of them into several runs and leaves others whole; from graphs too, which are kept with and
+    without the merge: the plain model's logits, and so do the equal runs of every row that the records replace."""
+    from tinyinfer_amd.engine import StepEntry
+    folder, V = wide_headed[window]
+    starts = {"a": 1, "b": 15, "c": 1280}
+    requests = {r: random_tokens(n, V, 90 + n) for r, n in {"a": 20, "b": 34, "c": 1299, "d": 119}.items()}
+    want, tol = plain_logits(folder, requests, "bfloat16", angles32=True)
+    engine = build_engine(folder, "bfloat16", 1600)
+    engine.ops.use_early_page_ids = records
+    run = engine.step_graph if graph else engine.step
+    at, got = dict(starts), {r: {} for r in requests}
+    # short rows alone first (whole rows), then all, then beside d's portions, then with d
+    for r, n in starts.items():
+        engine.step([StepEntry(r, requests[r][:n], ())])
+    plan = [("ab", 0)] * 4 + [("abc", 0)] * 5 + [("abc", 50), ("cab", 61)] + [("abcd", 0)] * 8
+    at["d"] = 0
+    for live, portion in plan:
+        steps = [(r, 1) for r in live] + ([("d", portion)] if portion else [])
+        logits = run([StepEntry(r, requests[r][at[r]:at[r] + n], (n - 1,)) for r, n in steps]).cpu().numpy().astype(np.float64)
+        for row, (r, n) in zip(logits, steps):
+            at[r] += n
+            got[r][at[r] - 1] = row
+    engine.cache.check()
+    for r in got:
+        for position, row in got[r].items():
+            assert np.abs(row - want[r][position]).max() < tol, (r, position)
+
+
 @pytest.mark.parametrize("config,fused", [("D", True), ("D", False), ("B", True)])
 def test_page_ids_fetched_beside_the_position_change_no_bit(model_folders, config, fused):
     """In a step of single tokens the decode attention fetches a row's page ids beside its position

@@ -354,7 +354,7 @@ struct HeadJob {
 // PREP: the queries come from the 32-bit projections (see QKPrep); needs parts == 1.  The row's query heads, and its own
 // key and value where a workgroup walks their block, are prepared a head a wavefront and shared through LDS while the first
 // keys and values are on their way.  (A lane that prepared its column's head by itself asked for 64 to 112 bytes in 28 loads
-// in front of its keys, and kept 100 registers for them: 8 requests of 2,048 tokens at 0.6B 21.8 us a layer, now FIG1.)
+// in front of its keys, and kept 100 registers for them: 8 requests of 2,048 tokens at 0.6B 21.8 us a layer, now 17.5.)
 // A learned sink in the softmax's denominator: exp(sink[head]) joins the sum where a column is finished (no key, no value,
 // not scaled).  m, lt: the column's maximum (in units of log 2) and the sum of its weights; lt becomes the new denominator
 // and the factor on the column's unscaled outputs comes back.  sink null: nothing changes.
