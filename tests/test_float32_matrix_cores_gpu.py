@@ -133,6 +133,28 @@ def test_attention_under_every_cut_of_a_step(ops, nh, nkv, hd, P, window):  # no
     assert (f64(rows) - f64(out)).abs().max() < 2e-5
 
 
+@pytest.mark.parametrize("nh,nkv,hd,P,window", [(2, 1, 16, 16, None), (17, 1, 48, 48, 37), (4, 2, 64, 16, 70), (3, 3, 80, 32, None),
+                                                (4, 4, 112, 16, 20), (16, 8, 128, 16, None), (2, 2, 128, 64, 37)])
+def test_attention_blocks_through_lds_and_straight_from_memory(ops, nh, nkv, hd, P, window):  # noqa: F811
+    """Pages of whole blocks, whose keys and values come through LDS, and the same cache in pages of 4 rows, whose come straight from
+    memory: the same bits, for heads of every remainder of four slices, contexts of no, one and several blocks a wavefront, and pages
+    given back behind a window; rows never written hold NaN."""
+    entries = [(65, 0), (1, 0), (18, 131), (1, 300), (2, 15), (130, 3), (1, 16)]
+    qs, pool, table, want = case(entries, nh, nkv, hd, P, window, seed=nh + hd + P)
+    q, n = dev(torch.cat(qs)), P // 4
+    pages = pool.cpu().view(-1, 2, nkv * P * hd)
+    k = pages[:, 0].reshape(-1, nkv, n, 4, hd).permute(0, 2, 1, 3, 4).reshape(-1, nkv * 4 * hd)
+    v = pages[:, 1].reshape(-1, nkv, hd, n, 4).permute(0, 3, 1, 2, 4).reshape(-1, nkv * hd * 4)
+    small = dev(torch.stack((k, v), 1).reshape(-1, 2 * nkv, 4, hd).contiguous())
+    ids = torch.where(table[:, :, None] < 0, -1, table[:, :, None] * n + torch.arange(n, dtype=torch.int32)).to(torch.int32)
+    args = (nh, nkv, hd, 1.0 / math.sqrt(hd), window)
+    staged, straight = torch.full_like(q, 7.0), torch.full_like(q, 8.0)
+    ops.attention(FakeCtx(entries), View(dev(table)), q, pool, staged, *args)
+    ops.attention(FakeCtx(entries), View(dev(ids.reshape(len(entries), -1).contiguous())), q, small, straight, *args)
+    assert (f64(staged) - torch.cat(want)).abs().max() < 2e-5
+    assert torch.equal(staged, straight)
+
+
 def hold(pool, table, P, nkv, hd, e, j, key, value):
     """What the cache holds of request e's token j: its key and its value, the same number everywhere."""
     page = pool[int(table[e, j // P])]

@@ -14,6 +14,7 @@
 // and the output accumulate in 32-bit.
 #include "common.h"
 #include "tinyinfer_kernels.h"
+#include "staged_rows.h"
 
 TI_ERROR_API
 
@@ -139,21 +140,54 @@ extern "C" int ti_attention_rows(int dtype, const void* q, const void* pool, con
 // both by v_mfma_f32_16x16x4_f32 with four consecutive entries a lane (loaded as one float4; both operands of a product
 // are permuted alike), so that the scores' layout is the second product's operand.  Block b belongs to wavefront
 // b mod 8 whatever the tile, and a key that a column may not see leaves it bit by bit as it was, whatever the key and its
-// value hold: a token's result depends on its keys alone, however a step is cut.  Keys and values come straight from memory, the next block's while
-// one is multiplied; short contexts are bounded by the start and the merge.  (With the rows kernel below, one workgroup
+// value hold: a token's result depends on its keys alone, however a step is cut.  Keys and values come through LDS or straight from memory (below),
+// the next block's while one is multiplied; short contexts are bounded by the start and the merge.  (With the rows kernel below, one workgroup
 // per row and head, lane sums and one value a load, a portion of 300 tokens with 16 heads of 128 on 8 kv heads took
 // 201 us a layer, 5.6 ms of a prompt of Qwen3-0.6B's sizes.)
 #define AF_WAVES 8
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float af4;
 
-template <int DB, bool SINGLE>
+// N slices of 1 KiB of LDS, this lane's 16 bytes of each (`at`: of the first), have arrived in registers when this returns.
+template <int N> __device__ __forceinline__ void read_some_slices(af4* e, unsigned at) {
+  if constexpr (N == 1) asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(e[0]) : "v"(at) : "memory");
+  if constexpr (N == 2)
+    asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:1024\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(e[0]), "=&v"(e[1]) : "v"(at) : "memory");
+  if constexpr (N == 4)
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:1024\n\tds_read_b128 %2, %4 offset:2048\n\t"
+                 "ds_read_b128 %3, %4 offset:3072\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(e[0]), "=&v"(e[1]), "=&v"(e[2]), "=&v"(e[3]) : "v"(at) : "memory");
+}
+template <int DB> __device__ __forceinline__ void read_slices(af4* e, unsigned at) {
+#pragma unroll
+  for (int d = 0; d + 4 <= DB; d += 4) read_some_slices<4>(e + d, at + d * 1024);
+  if constexpr (DB & 2) read_some_slices<2>(e + (DB & ~3), at + (DB & ~3) * 1024);
+  if constexpr (DB & 1) read_some_slices<1>(e + (DB & ~1), at + (DB & ~1) * 1024);
+}
+
+// STAGED (heads of up to 128, pages of whole blocks): the blocks come by direct loads through LDS of each wavefront's own, DB slices of 16
+// rows x 64 bytes for the keys and as many for the values.  As operands straight from memory, neighbouring lanes in different rows, a load
+// takes the unit that takes addresses 64 cycles, and a compute unit's eight wavefronts share it: some 3.4 us a round of eight blocks of
+// heads of 128; four lanes to a row's 64 bytes take 16.  A slice is asked for again, for the wavefront's next block, as soon as it has been
+// read.  Piece c (16 bytes) of row r lies in place 4 r + (c ^ (r / 4)), so that a quarter of the wavefront reads from different banks.  The
+// arithmetic is the same, and so are the bits.  us, straight from memory and so (the portions' with the order of tiles below): a portion
+// of 300 tokens, 16 heads of 128 on 8, 27.9 -> 20.9; 512 tokens behind 300 63 -> 47; 8 single tokens of 900, 31.6 -> 25.7; heads of 64
+// 23.6 -> 20.8 at most (the host's calls are as long).  Left: 320 workgroups on 256 units, one a unit, and each one's start and merge.
+template <int DB, bool SINGLE, bool STAGED>
 __global__ void __launch_bounds__(64 * AF_WAVES)
 attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool, const int* __restrict__ table,
                      int table_stride, const int* __restrict__ pos, const int* __restrict__ slot,
                      const int* __restrict__ rows, const int* __restrict__ tiles, const int* __restrict__ entries,
                      float* __restrict__ out, int n_head, int n_kv, int P, float scale, int window) {
-  constexpr int HD = DB * 16;
-  __shared__ __attribute__((aligned(16))) float s_o[AF_WAVES][16][HD + 4];
+#if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass has no buffer descriptors)
+  constexpr int HD = DB * 16, STAGE = 2 * DB * 1024;       // bytes of a wavefront's stage, where its sums lie afterwards
+  static_assert(STAGE >= 16 * (HD + 4) * 4, "a wavefront's sums fit into its stage");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  __shared__ __attribute__((aligned(16))) float s_sums[STAGED ? 1 : AF_WAVES][16][HD + 4];
+  const auto s_o = [&](int w, int c) -> float* {
+    if constexpr (STAGED) return reinterpret_cast<float*>(smem + w * STAGE) + c * (HD + 4);
+    else return s_sums[w][c];
+  };
   __shared__ float s_m[AF_WAVES][16], s_l[AF_WAVES][16];
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r16 = lane & 15, quad = lane >> 4;
@@ -170,9 +204,11 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
     p_first = p_last = pos[m_row];
     tab = table + (size_t)slot[m_row] * table_stride;
   } else {
-    const int entry = tiles[(blockIdx.x >> 2) * 2], row0 = entries[entry * 4];
-    m_row = tiles[(blockIdx.x >> 2) * 2 + 1] + (blockIdx.x & 3) * 16;
-    head0 = blockIdx.y;
+    // the last tiles, which see the most keys, first and in all heads: what is left for a second round is short
+    const unsigned at = blockIdx.y * gridDim.x + blockIdx.x, part = gridDim.x - 1 - at / n_head;
+    const int entry = tiles[(part >> 2) * 2], row0 = entries[entry * 4];
+    m_row = tiles[(part >> 2) * 2 + 1] + (part & 3) * 16;
+    head0 = at % n_head;
     kvh = head0 / G;
     n_cols = min(16, row0 + entries[entry * 4 + 1] - m_row);
     if (n_cols <= 0) return;
@@ -210,7 +246,7 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
     for (int d = 0; d < DB; ++d) f.v[d] = *reinterpret_cast<const af4*>(vp + (size_t)d * 16 * P);
   };
   float mx = -INFINITY, l = 0.f;
-  auto attend = [&](Block& f) {
+  auto attend = [&](Block& f, auto values) {         // values(): f.v are there when it returns
     af4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < DB; ++s) {
@@ -220,6 +256,7 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
         else s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(f.k[s][j], qf[s][j], s1, 0, 0, 0);
       }
     }
+    values();
     float sc[4], bm = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -282,12 +319,56 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
   const int b_last = p_last / 16;
   int b = lo_min / 16;
   b += (wave - b % AF_WAVES + AF_WAVES) % AF_WAVES;
+  const auto there = [] {};
   if (b <= b_last) {
     Block f0;
-    if constexpr (DB > 8) {                         // two blocks of such heads do not fit in the registers
+    if constexpr (STAGED) {
+      const int row = lane >> 2, piece = (lane & 3) ^ ((row >> 2) & 3);
+      const unsigned k_off = (unsigned)row * (HD * 4) + piece * 16, v_off = (unsigned)row * (unsigned)(P * 4) + piece * 16;
+      unsigned char* mine = smem + wave * STAGE;
+      const unsigned at = (unsigned)(size_t)mine + r16 * 64 + ((quad ^ (r16 >> 2)) << 4);
+      const auto rows_at = [](const float* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
+      const auto page_of = [&](int block) { return __builtin_amdgcn_readfirstlane(tab[block * 16 / P]); };
+      const auto ask_keys = [&](int page, int block) {
+        const auto rs = rows_at(k_head + (size_t)max(page, 0) * page_elems + (size_t)(block * 16 % P) * HD);
+#pragma unroll
+        for (int s = 0; s < DB; ++s)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(mine + s * 1024), 16, k_off, s * 64, 0, 0);
+      };
+      const auto ask_values = [&](int page, int block) {
+        const auto rs = rows_at(v_head + (size_t)max(page, 0) * page_elems + block * 16 % P);
+#pragma unroll
+        for (int d = 0; d < DB; ++d)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(mine + (DB + d) * 1024), 16, v_off, d * 64 * P, 0, 0);
+      };
+      int page = page_of(b);
+      ask_keys(page, b);
+      ask_values(page, b);
+      for (;;) {
+        const int next = b + AF_WAVES;
+        const bool more = next <= b_last;           // the same in every lane
+        const int next_page = more ? page_of(next) : 0;
+        f0.key0 = b * 16;
+        f0.have = page >= 0;
+        wait_vmcnt<DB>();                           // the keys are there; their values may still be out
+        read_slices<DB>(f0.k, at);
+        if (more) ask_keys(next_page, next);
+        __builtin_amdgcn_sched_barrier(0);
+        attend(f0, [&] {
+          if (more) wait_vmcnt<DB>();               // the next keys may still be out
+          else wait_vmcnt<0>();
+          read_slices<DB>(f0.v, at + DB * 1024);
+          if (more) ask_values(next_page, next);
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        if (!more) break;
+        b = next;
+        page = next_page;
+      }
+    } else if constexpr (DB > 8) {                         // two blocks of such heads do not fit in the registers
       for (; b <= b_last; b += AF_WAVES) {
         load(f0, b);
-        attend(f0);
+        attend(f0, there);
       }
     } else {
     Block f1;
@@ -295,11 +376,11 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
     for (;;) {
       load(f1, min(b + AF_WAVES, b_last));
       __builtin_amdgcn_sched_barrier(0);
-      attend(f0);
+      attend(f0, there);
       if ((b += AF_WAVES) > b_last) break;
       load(f0, min(b + AF_WAVES, b_last));
       __builtin_amdgcn_sched_barrier(0);
-      attend(f1);
+      attend(f1, there);
       if ((b += AF_WAVES) > b_last) break;
     }
     }
@@ -307,7 +388,7 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
 #pragma unroll
-  for (int d = 0; d < DB; ++d) *reinterpret_cast<af4*>(&s_o[wave][r16][d * 16 + quad * 4]) = o[d];
+  for (int d = 0; d < DB; ++d) *reinterpret_cast<af4*>(s_o(wave, r16) + d * 16 + quad * 4) = o[d];
   if (quad == 0) {
     s_m[wave][r16] = mx;
     s_l[wave][r16] = l;
@@ -323,11 +404,32 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
     for (int w = 0; w < AF_WAVES; ++w) {
       const float f = (s_m[w][c] == -INFINITY) ? 0.f : expf(s_m[w][c] - mm);
       lt += s_l[w][c] * f;
-      acc += s_o[w][c][d] * f;
+      acc += s_o(w, c)[d] * f;
     }
     const size_t row = SINGLE ? (size_t)m_row * n_head + head0 + c : (size_t)(m_row + c) * n_head + head0;
     out[row * HD + d] = acc / lt;
   }
+#endif
+}
+
+// the stages' LDS; pages of whole blocks whose values lie within what a buffer's offset spans
+template <int DB, bool SINGLE>
+static int launch_attention_f32(dim3 grid, const float* q, const float* pool, const int* table, int table_stride, const int* pos,
+                                const int* slot, const int* rows, const int* tiles, const int* entries, float* out, int n_head, int n_kv,
+                                int P, float scale, int window, hipStream_t stream) {
+  if constexpr (DB <= 8) {
+    if (P % 16 == 0 && P <= 65536) {
+      constexpr int lds = AF_WAVES * 2 * DB * 1024;
+      auto kernel = attention_f32_kernel<DB, SINGLE, true>;
+      static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      TI_REQUIRE(room == hipSuccess, "attention: %d bytes of LDS: %s", lds, hipGetErrorString(room));
+      kernel<<<grid, 64 * AF_WAVES, lds, stream>>>(q, pool, table, table_stride, pos, slot, rows, tiles, entries, out, n_head, n_kv, P, scale, window);
+      return 0;
+    }
+  }
+  attention_f32_kernel<DB, SINGLE, false><<<grid, 64 * AF_WAVES, 0, stream>>>(q, pool, table, table_stride, pos, slot, rows, tiles, entries, out,
+                                                                             n_head, n_kv, P, scale, window);
+  return 0;
 }
 
 // A step's attention in float32: n_tiles tiles of up to 64 rows of portions (tiles int32 [n_tiles][2] = (entry, first
@@ -343,16 +445,15 @@ extern "C" int ti_attention_f32(const void* q, const void* pool, const int* tabl
   TI_REQUIRE(n_tiles >= 0 && n_single >= 0 && (n_tiles == 0 || (tiles && entries)), "attention: %d tiles without their lists", n_tiles);
   if (hd < 16 || hd > 256 || hd % 16 != 0 || page_size % 4 != 0) return 3;
   const int parts = (n_head / n_kv + 15) / 16;
+  int rc_ = 0;
 #define AF_CASE(D)                                                                                                            \
   case D:                                                                                                                     \
     if (n_tiles)                                                                                                              \
-      attention_f32_kernel<D, false><<<dim3(n_tiles * 4, n_head), 64 * AF_WAVES, 0, stream>>>(                                \
-          (const float*)q, (const float*)pool, table, table_stride, pos, slot, rows, tiles, entries, (float*)out, n_head,     \
-          n_kv, page_size, scale, window);                                                                                    \
-    if (n_single)                                                                                                             \
-      attention_f32_kernel<D, true><<<dim3(n_single, n_kv * parts), 64 * AF_WAVES, 0, stream>>>(                              \
-          (const float*)q, (const float*)pool, table, table_stride, pos, slot, rows, tiles, entries, (float*)out, n_head,     \
-          n_kv, page_size, scale, window);                                                                                    \
+      rc_ = launch_attention_f32<D, false>(dim3(n_tiles * 4, n_head), (const float*)q, (const float*)pool, table, table_stride, pos,\
+                                           slot, rows, tiles, entries, (float*)out, n_head, n_kv, page_size, scale, window, stream);\
+    if (rc_ == 0 && n_single)                                                                                                 \
+      rc_ = launch_attention_f32<D, true>(dim3(n_single, n_kv * parts), (const float*)q, (const float*)pool, table, table_stride, pos,\
+                                          slot, rows, tiles, entries, (float*)out, n_head, n_kv, page_size, scale, window, stream);\
     break;
   switch (hd / 16) {
     AF_CASE(1) AF_CASE(2) AF_CASE(3) AF_CASE(4) AF_CASE(5) AF_CASE(6) AF_CASE(7) AF_CASE(8)
@@ -361,6 +462,7 @@ extern "C" int ti_attention_f32(const void* q, const void* pool, const int* tabl
       return 3;
   }
 #undef AF_CASE
+  if (rc_) return rc_;
   TI_LAUNCH_CHECK();
   return 0;
 }
