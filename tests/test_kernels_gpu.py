@@ -593,6 +593,36 @@ def test_sample_rows_whose_first_bin_holds_too_many(ops, V, skip):
         assert sum(a != b for a, b in zip(got, walked)) <= 1, (T, top_k, top_p, got, walked)
 
 
+def masked_row(V, allowed, mask, seed):
+    """A row as a grammar leaves it: ordinary logits at the indices `allowed`, `mask` everywhere else."""
+    row = torch.full((V,), mask)
+    row[allowed] = torch.randn(len(allowed), generator=torch.Generator().manual_seed(seed)) * 2
+    return row
+
+
+@pytest.mark.parametrize("mask", [float("-inf"), torch.finfo(torch.float32).min, -1e4])
+@pytest.mark.parametrize("V,each", [(20480, 30), (151936, 30)])
+def test_sample_rows_whose_parts_hold_fewer_than_the_cut(ops, V, each, mask):
+    """A masked row with `each` logits left in every part of it, the last that a part's wavefronts come to: every part holds fewer than
+    k of them and thousands of equal ones below, which are more than it collects, while the row's own cut lies far above.  The draws
+    lie where the plain CDF puts them, for greedy rows and cuts below, at and above what a part holds."""
+    us = np.linspace(0.01, 0.99, 12).astype(np.float32)
+    parts = -(-V // 10240)
+    span = -(-(V // 4) // parts) * 4
+    allowed = [p * span + 1900 + i for p in range(parts) for i in range(each)]
+    row = masked_row(V, allowed, mask, V)
+    for T, top_k, top_p in ((1.0, 50, 1.0), (0.8, 31, 0.9), (1.0, each, 1.0), (0.0, 5, 1.0)):
+        got = run_sample(ops, dev(row[None, :].repeat(len(us), 1)), T, top_k, top_p, us.tolist())
+        if T > 0:
+            check_draws(row, T, top_k, top_p, us, got)
+        else:
+            assert set(got) == {int(row.argmax())}
+    # as many as all parts hold are left (the row's cut), and one more (its equals are everything else)
+    for top_k in (len(allowed), len(allowed) + 1):
+        got = run_sample(ops, dev(row[None, :].repeat(len(us), 1)), 1.0, top_k, 1.0, us.tolist())
+        check_draws(row, 1.0, top_k, 1.0, us, got)
+
+
 @pytest.mark.parametrize("n,V", [(1, 1000), (65, 20001), (150, 4096)])
 def test_sampler_of_more_rows_than_travel_with_a_launch(ops, n, V):
     """What the rows ask for goes with the launches, 64 rows at a time, and the ids come straight into the host's memory: the ids

@@ -693,7 +693,7 @@ sample_finish_kernel(const float* __restrict__ logits, Rows rows, int* __restric
     taken += above;
     need -= above;
   };
-  if (got == 0) {                                  // a row of NaN
+  if (got == 0 && !over) {                         // a row of NaN
     if (t == 0) out[r] = 0;
     return;
   }
