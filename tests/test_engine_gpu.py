@@ -346,6 +346,72 @@ def test_rows_of_very_different_lengths_by_records(wide_headed, window, graph, r
             assert np.abs(row - want[r][position]).max() < tol, (r, position)
 
 
+def shared_cache_logits(w, cfg, tokens, windows, rnd):
+    """The plain decoder whose layers behind the first keep no keys and values: they read the first layer's, each through a window of
+    its own (None: all keys)."""
+    nh, nkv, hd, eps = cfg["num_attention_heads"], cfg["num_key_value_heads"], cfg["head_dim"], cfg["rms_norm_eps"]
+    T = len(tokens)
+    turned = lambda x, norm: plain.rope_neox(plain.qk_norm(x, norm, eps), range(T), cfg["rope_theta"], rnd)      # noqa: E731
+    x = plain.embed(w["model.embed_tokens.weight"], tokens)
+    for i, window in enumerate(windows):
+        p = f"model.layers.{i}"
+        h = rnd("gemm_in", plain.rms_norm(x, w[p + ".input_layernorm.weight"], eps))
+        if i == 0:
+            k = turned(plain.linear(h, w[p + ".self_attn.k_proj.weight"]).reshape(T, nkv, hd), w[p + ".self_attn.k_norm.weight"])
+            k, v = rnd("kv_cache", k), rnd("kv_cache", plain.linear(h, w[p + ".self_attn.v_proj.weight"]).reshape(T, nkv, hd))
+        q = rnd("q", turned(plain.linear(h, w[p + ".self_attn.q_proj.weight"]).reshape(T, nh, hd), w[p + ".self_attn.q_norm.weight"]))
+        a = plain.attention(q, k, v, window).reshape(T, nh * hd)
+        x = x + plain.linear(rnd("gemm_in", a), w[p + ".self_attn.o_proj.weight"])
+        x = x + plain.ffn_block(plain.rms_norm(x, w[p + ".post_attention_layernorm.weight"], eps), w, p + ".mlp", rnd)
+    return plain.linear(rnd("gemm_in", plain.rms_norm(x, w["model.norm.weight"], eps)), w["model.embed_tokens.weight"])
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("graph", [False, True])
+def test_layers_that_read_one_cache_through_windows_of_their_own(tmp_path, graph, head_dim):
+    """Three layers read the first one's keys and values through windows of 64, all and 150 keys: rows of some 20 to 260 cached tokens
+    decode together, beside another request's portions (one shape four times, so that it is captured) and with it afterwards.  The plain
+    model's logits; the windows' own effect on them is many times the tolerance."""
+    from tinyinfer_amd.engine import Engine, StepEntry
+    from tinyinfer_amd.models.model import Model
+    from tinyinfer_amd.registry import config_and_spec
+    from tinyinfer_amd.weights import write_model_folder
+    from tinyinfer_amd.weights.loader import load_weights
+    cfg = dict(ODD_CONFIGS["three heads a group, head 128"], num_hidden_layers=4, head_dim=head_dim)
+    windows = [None, 64, None, 150]
+    folder = str(tmp_path)
+    write_model_folder(folder, cfg, seed=78, dtype="bfloat16")
+    sharpen_folder(folder)
+    cfg, w = read_folder(folder)
+    _, spec = config_and_spec(cfg)
+    for layer, window in list(zip(spec.layers, windows))[1:]:
+        layer.cache_from = 0
+        layer.parts["mixer"].params["shares_kv"] = True
+        if window:
+            layer.parts["mixer"].params["window"] = window
+    model = Model(spec)
+    load_weights(model, {n: torch.from_numpy(t).to("cuda", torch.float32 if t.ndim == 1 else torch.bfloat16)
+                         for n, t in w.items() if n in model.tensors()}, "bfloat16")
+    engine = Engine(model, "bfloat16", page_size=16, max_tokens=640, max_requests=4, max_seq=320)
+    starts = {"a": 17, "b": 130, "c": 233}
+    requests = {r: random_tokens(n, cfg["vocab_size"], 60 + n) for r, n in {"a": 40, "b": 152, "c": 256, "d": 100}.items()}
+    want = {r: shared_cache_logits(w, cfg, t, windows, ROUNDED) for r, t in requests.items()}
+    exact = {r: shared_cache_logits(w, cfg, t, windows, plain.no_rounding) for r, t in requests.items()}
+    tol = max(float(np.abs(want[r] - exact[r]).max()) for r in want)
+    unseen = shared_cache_logits(w, cfg, requests["c"], [None] * 4, plain.no_rounding)
+    assert np.abs(unseen - exact["c"])[200:].max() > 4 * tol
+    run, at = engine.step_graph if graph else engine.step, dict(starts, d=0)
+    for r, n in starts.items():
+        engine.step([StepEntry(r, requests[r][:n], ())])
+    for live, portion in [("abc", 0)] * 6 + [("abc", 23)] * 4 + [("abcd", 0)] * 8:
+        steps = [(r, 1) for r in live] + ([("d", portion)] if portion else [])
+        logits = run([StepEntry(r, requests[r][at[r]:at[r] + n], (n - 1,)) for r, n in steps]).cpu().numpy().astype(np.float64)
+        for row, (r, n) in zip(logits, steps):
+            at[r] += n
+            assert np.abs(row - want[r][at[r] - 1]).max() < tol, (r, at[r] - 1, portion)
+    engine.cache.check()
+
+
 @pytest.mark.parametrize("config,fused", [("D", True), ("D", False), ("B", True)])
 def test_page_ids_fetched_beside_the_position_change_no_bit(model_folders, config, fused):
     """In a step of single tokens the decode attention fetches a row's page ids beside its position

@@ -771,9 +771,11 @@ class Attention final : public MixerPart {
     plan_runs(plan);
   }
   // The single-token rows of a step that the plain attention serves on the matrix cores, by records (Ops::plan_runs): all of a step of
-  // single tokens, or those beside portions in the portions' launch.  One list for all parts whose pages are the same.
+  // single tokens, or those beside portions in the portions' launch.  One list for all parts whose pages, heads and windows are the
+  // same (layers that read one cache may each have a window of their own).
   std::string runs_key(int group) const {
-    return "attention.runs." + std::to_string(group) + "." + std::to_string(kv_heads * ((heads / kv_heads + 15) / 16)) + "." + std::to_string(heads);
+    return "attention.runs." + std::to_string(group) + "." + std::to_string(kv_heads * ((heads / kv_heads + 15) / 16)) + "." +
+           std::to_string(heads) + "." + std::to_string(head_dim) + "." + std::to_string(window);
   }
   void plan_runs(StepPlan& plan) const {
     const Ops* ops = plan.ops();
