@@ -623,6 +623,46 @@ def test_sample_rows_whose_parts_hold_fewer_than_the_cut(ops, V, each, mask):
         check_draws(row, 1.0, top_k, 1.0, us, got)
 
 
+@pytest.mark.parametrize("V,left", [(151936, 1000), (151935, 40), (25001, 60)])
+def test_sample_masked_rows_without_walking_them(ops, V, left):
+    """Rows of which a mask leaves a few logits, some parts of a row none: greedy rows and cuts that the row as a whole reaches are the
+    plain CDF's and the walking kernel's (a sum taken in another order may move one edge a setting), in a fraction of its time."""
+    g = torch.Generator().manual_seed(V + left)
+    us = np.linspace(0.01, 0.99, 12).astype(np.float32)
+    first = V // 8 if left == 40 else 0                                      # 40: the row's first eighth is masked throughout
+    allowed = (first + torch.randperm(V - first, generator=g)[:left]).sort().values
+    rows = [masked_row(V, allowed, mask, left) for mask in (float("-inf"), torch.finfo(torch.float32).min)]
+    logits = dev(torch.stack(rows * 6))
+
+    def timed(T, top_k, top_p):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        got = run_sample(ops, logits, T, top_k, top_p, us.tolist())
+        args = [dev(t) for t in (torch.full((12,), T), torch.full((12,), top_k, dtype=torch.int32), torch.full((12,), top_p), torch.from_numpy(us))]
+        out = torch.empty(12, dtype=torch.int32, device="cuda")
+        start.record()
+        for _ in range(10):
+            ops.sample(logits, *args, out)
+        end.record()
+        torch.cuda.synchronize()
+        return got, start.elapsed_time(end)
+
+    for T, top_k, top_p in ((0.0, 0, 1.0), (1.0, left, 1.0), (0.8, left // 2, 0.9), (1.0, 7, 1.0)):
+        got, us_got = timed(T, top_k, top_p)
+        ops.use_radix_sample = False
+        try:
+            walked, us_walked = timed(T, top_k, top_p)
+        finally:
+            ops.use_radix_sample = True
+        for i in range(2):
+            if T > 0:
+                check_draws(rows[i], T, top_k, top_p, us[i::2], got[i::2])
+            else:
+                assert set(got[i::2]) == {int(rows[i].argmax())}
+        assert sum(a != b for a, b in zip(got, walked)) <= 1, (T, top_k, top_p, got, walked)
+        if T > 0 and V > 100000:
+            assert us_got < us_walked / 4, (T, top_k, top_p, us_got, us_walked)
+
+
 @pytest.mark.parametrize("n,V", [(1, 1000), (65, 20001), (150, 4096)])
 def test_sampler_of_more_rows_than_travel_with_a_launch(ops, n, V):
     """What the rows ask for goes with the launches, 64 rows at a time, and the ids come straight into the host's memory: the ids

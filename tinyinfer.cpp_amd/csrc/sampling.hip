@@ -295,8 +295,12 @@ sample_kernel(const float* __restrict__ logits, Rows rows, int* __restrict__ out
 //           sorts what is kept by logit where there is a top-p cut and sums the weights in that order, sorts
 //           what is left by index and draws by inverse CDF.  Sums are scans of a fixed shape.
 // It draws what the kernel above draws, up to the rounding of sums that are taken in another order.
-// Rows that it does not serve (no top-k cut, a cut beyond S_MAX_K, more than S_CAND keys that are equal
-// at the cut) are left to that kernel's walk, inside the last kernel.
+// Rows that it does not serve (no top-k cut, a cut beyond S_MAX_K, more keys of a part that are equal
+// at the row's cut than it has room for) are left to that kernel's walk, inside the last kernel.  A part may hold thousands of equal
+// keys at its own k-th while the row's cut lies above them (a masked row: a few logits a part beside as many masked ones as there are):
+// it leaves what is above them and says which they are, and the row is served if k pairs are above all of those.  (64 rows of
+// 151,936 with 1,000 logits left at random, us: a cut of 50 61, of 500 with a top-p cut 81; when such parts sent their rows to the walk
+// 1,016 and 3,872.)
 //
 // 64 rows of 151,936, greedy, top-k 50 and top-p, 512 and 20 in turn, us: three passes over the row's memory and a finish
 // with two sorts by rank 9.9 + 12.9 + 14.3 + 23.0; this 13.4 + 16.8.  Of the first, 9.5 are the loads and the counts (39 MB, and a
@@ -397,12 +401,28 @@ __device__ __forceinline__ int next_places(int* s_count, int n) {
   return __builtin_amdgcn_readfirstlane(at) + upto - n;
 }
 
+// Counts the digits of the lanes that are `on`.  What shares the first such lane's digit is added at once: thousands of masked
+// logits are one key, and a step each on one counter takes 30 us a digit (138 us for the latter rows above).  For the digits behind the
+// first: there it took ordinary rows 3.7 us of 27.  All lanes call it.
+__device__ __forceinline__ void count_digit(int* s_bins, bool on, int digit) {
+  const unsigned long long lanes = __ballot(on);
+  if (lanes == 0) return;
+  const int first = __builtin_ctzll(lanes), shared = __builtin_amdgcn_readlane(digit, first);
+  const int n = __popcll(__ballot(on && digit == shared));
+  if ((int)(threadIdx.x & (TI_WAVE - 1)) == first) atomicAdd(&s_bins[shared], n);
+  else if (on && digit != shared) atomicAdd(&s_bins[digit], 1);
+}
+
 // grid (parts of `span` keys, rows), span a multiple of 4, at most S_SPAN.  WIDE: rows of whole float4s on their boundaries, four
-// neighbours a load.  counts [row][parts][2] (pairs, the key from which the part's share lies), pairs [row][parts][S_CAND]
-// (key << 32 | ~index).  (64 registers a thread: four workgroups to a unit, so that 64 rows of 15 parts are one round.)
+// neighbours a load.  left [row][parts], pairs [row][parts][S_CAND] (key << 32 | ~index).  (64 registers a thread: four workgroups to a unit, so that 64 rows of 15 parts are one round.)
+struct PartLeft {
+  int pairs;
+  uint32_t share;      // the key from which the part's share lies
+  uint32_t over;       // the k-th key, if it has more equals than there is room for: the part's pairs are those above it (0: no such key)
+};
 template <bool WIDE, class Rows>
 __global__ void __launch_bounds__(S_NT)
-sample_part_kernel(const float* __restrict__ logits, Rows rows, int2* __restrict__ counts, unsigned long long* __restrict__ pairs,
+sample_part_kernel(const float* __restrict__ logits, Rows rows, PartLeft* __restrict__ left, unsigned long long* __restrict__ pairs,
                    int V, int span) {
   __shared__ __attribute__((aligned(16))) int s_bins[S_BINS];
   __shared__ int s_wave[S_NT / TI_WAVE], s_res[4], s_count;
@@ -439,7 +459,7 @@ sample_part_kernel(const float* __restrict__ logits, Rows rows, int2* __restrict
   int bin, above, in, share_bin, taken = 0, need = k, shift = 32 - S_BITS;      // taken: keys above the prefix
   bin_of_kth<S_BINS, S_NT>(s_bins, need, s_wave, s_res, bin, above, in, (k + gridDim.x - 1) / gridDim.x, &share_bin);
   if (bin < 0) {
-    if (t == 0) counts[part] = make_int2(0, 0);
+    if (t == 0) left[part] = PartLeft{0, 0, 0};
     return;
   }
   uint32_t prefix = bin;
@@ -450,26 +470,24 @@ sample_part_kernel(const float* __restrict__ logits, Rows rows, int2* __restrict
     need -= above;
 #pragma unroll
     for (int u = 0; u < S_LOADS; ++u)
-      if (key[u] && (key[u] >> shift) == prefix) atomicAdd(&s_bins[(key[u] >> (shift - S_BITS2)) & (S_BINS2 - 1)], 1);
+      count_digit(s_bins, key[u] && (key[u] >> shift) == prefix, (int)((key[u] >> (shift - S_BITS2)) & (S_BINS2 - 1)));
     __syncthreads();
     bin_of_kth<S_BINS2, S_NT>(s_bins, need, s_wave, s_res, bin, above, in);
     prefix = (prefix << S_BITS2) | (uint32_t)bin;
     shift -= S_BITS2;
   }
   unsigned long long* mine = pairs + part * S_CAND;
-  const uint32_t least = max(prefix << shift, 1u);
+  const uint32_t over = above + taken + in > S_CAND ? prefix : 0;         // (a whole key then: all its digits have been looked at)
+  const uint32_t least = over ? over + 1 : max(prefix << shift, 1u);       // fewer than k keys are above the k-th
   int n = 0;
 #pragma unroll
   for (int u = 0; u < S_LOADS; ++u) n += key[u] >= least ? 1 : 0;
   int at = next_places(&s_count, n);
 #pragma unroll
   for (int u = 0; u < S_LOADS; ++u)
-    if (key[u] >= least) {
-      if (at < S_CAND) mine[at] = ((unsigned long long)key[u] << 32) | (uint32_t)~(base + place(u));
-      ++at;
-    }
+    if (key[u] >= least) mine[at++] = ((unsigned long long)key[u] << 32) | (uint32_t)~(base + place(u));
   __syncthreads();
-  if (t == 0) counts[part] = make_int2(s_count, share_bin << (32 - S_BITS));       // more than S_CAND: the row is walked
+  if (t == 0) left[part] = PartLeft{s_count, (uint32_t)share_bin << (32 - S_BITS), over};
 }
 
 // sorts a[0..n) of LDS downwards by the entries' upper words, n <= S_CAND; every thread of the workgroup
@@ -604,15 +622,15 @@ __device__ void sort_by_index(const unsigned long long* a, unsigned long long* t
 
 template <class Rows>
 __global__ void __launch_bounds__(SNT)
-sample_finish_kernel(const float* __restrict__ logits, Rows rows, int* __restrict__ out, const int2* __restrict__ counts,
+sample_finish_kernel(const float* __restrict__ logits, Rows rows, int* __restrict__ out, const PartLeft* __restrict__ left,
                      const unsigned long long* __restrict__ pairs, int parts, int V) {
   __shared__ __attribute__((aligned(16))) unsigned long long s_pair[S_CAND], s_tmp[S_CAND];
   __shared__ float s_w[S_CAND];
   __shared__ __attribute__((aligned(16))) int s_bins[S_BINS];
   __shared__ float s_wave[SNT / TI_WAVE];
   __shared__ int s_iwave[SNT / TI_WAVE], s_res[4];
-  __shared__ int s_n, s_at, s_m, s_over;
-  __shared__ uint32_t s_max, s_from;
+  __shared__ int s_n, s_at, s_m;
+  __shared__ uint32_t s_max, s_from, s_over;
   const int r = blockIdx.x, t = threadIdx.x, lane = t & (TI_WAVE - 1), wave = t / TI_WAVE;
   const SampleRow want = rows.at(r);
   const int k = served_cut(want, V);
@@ -629,7 +647,7 @@ sample_finish_kernel(const float* __restrict__ logits, Rows rows, int* __restric
       unsigned long long x[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = seg[TI_WAVE * j];
-      const int n = min(counts[(size_t)r * parts + b].x, S_CAND);
+      const int n = left[(size_t)r * parts + b].pairs;
       for (int i0 = 0; i0 < n; i0 += 8 * TI_WAVE) {
         if (i0) {
 #pragma unroll
@@ -647,13 +665,13 @@ sample_finish_kernel(const float* __restrict__ logits, Rows rows, int* __restric
   if (t == 0) s_at = 0x7fffffff, s_m = 0, s_max = 0, s_over = 0, s_from = 0xffffffffu;
   __syncthreads();
   for (int b = t; b < parts; b += SNT) {
-    const int2 c = counts[(size_t)r * parts + b];
-    if (c.x > S_CAND) s_over = 1;
-    atomicMin(&s_from, (uint32_t)c.y);
+    const PartLeft c = left[(size_t)r * parts + b];
+    atomicMin(&s_from, c.share);
+    if (c.over) atomicMax(&s_over, c.over);
   }
   __syncthreads();
-  const uint32_t from = s_from;
-  const bool over = s_over != 0;
+  const uint32_t over = s_over;                    // keys up to here may be missing
+  const uint32_t from = over ? max(s_from, over + 1) : s_from;
   // the pairs at or above `key`, in LDS as far as they fit
   const auto gather = [&](uint32_t key) {
     const uint32_t least = max(key, 1u);           // (0 is no pair)
@@ -693,11 +711,15 @@ sample_finish_kernel(const float* __restrict__ logits, Rows rows, int* __restric
     taken += above;
     need -= above;
   };
-  if (got == 0 && !over) {                         // a row of NaN
+  if (over && got < k) {                           // the row's cut is `over`, whose equals are too many
+    sample_row_by_bisection(logits, want, out, V, r);
+    return;
+  }
+  if (got == 0) {                                  // a row of NaN
     if (t == 0) out[r] = 0;
     return;
   }
-  if (got > S_CAND && !over) {                     // shares that are no guide: by digits over all pairs, until few enough are left
+  if (got > S_CAND) {                              // shares that are no guide: by digits over all pairs, until few enough are left
     do {
       each([&](const unsigned long long* x) {
         for (int j = 0; j < 8; ++j) digit(x[j]);
@@ -711,7 +733,7 @@ sample_finish_kernel(const float* __restrict__ logits, Rows rows, int* __restric
       gather(prefix << shift);
     }
   }
-  if (over || got > S_CAND) {
+  if (got > S_CAND) {
     sample_row_by_bisection(logits, want, out, V, r);
     return;
   }
@@ -842,7 +864,7 @@ extern "C" int ti_argmax_static(const float* logits, int* out, int n_rows, int V
 }
 
 static int sample_parts(int V) { return std::max(1, (V + S_SPAN - 1) / S_SPAN); }
-extern "C" long ti_sample_scratch_bytes(int n_rows, int V) { return (long)n_rows * sample_parts(V) * (S_CAND * 8 + 8); }
+extern "C" long ti_sample_scratch_bytes(int n_rows, int V) { return (long)n_rows * sample_parts(V) * (S_CAND * 8 + (long)sizeof(PartLeft)); }
 
 template <class Rows>
 static void launch_sample(const float* logits, const Rows& rows, int* out, void* scratch, int n_rows, int V, hipStream_t stream) {
@@ -853,12 +875,12 @@ static void launch_sample(const float* logits, const Rows& rows, int* out, void*
   const int parts = sample_parts(V), span = ((V + parts - 1) / parts + 3) & ~3;      // parts of a size: equal shares
   const dim3 grid(parts, n_rows);
   auto* pairs = (unsigned long long*)scratch;
-  int2* counts = (int2*)(pairs + (size_t)n_rows * parts * S_CAND);
+  auto* left = (PartLeft*)(pairs + (size_t)n_rows * parts * S_CAND);
   if (V % 4 == 0 && ((uintptr_t)logits & 15) == 0)
-    sample_part_kernel<true><<<grid, S_NT, 0, stream>>>(logits, rows, counts, pairs, V, span);
+    sample_part_kernel<true><<<grid, S_NT, 0, stream>>>(logits, rows, left, pairs, V, span);
   else
-    sample_part_kernel<false><<<grid, S_NT, 0, stream>>>(logits, rows, counts, pairs, V, span);
-  sample_finish_kernel<<<n_rows, SNT, 0, stream>>>(logits, rows, out, counts, pairs, parts, V);
+    sample_part_kernel<false><<<grid, S_NT, 0, stream>>>(logits, rows, left, pairs, V, span);
+  sample_finish_kernel<<<n_rows, SNT, 0, stream>>>(logits, rows, out, left, pairs, parts, V);
 }
 
 // scratch: ti_sample_scratch_bytes(n_rows, V) bytes on a boundary of 8, or nullptr (then one workgroup walks a whole row)
