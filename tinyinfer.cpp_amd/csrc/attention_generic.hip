@@ -170,9 +170,9 @@ template <int DB> __device__ __forceinline__ void read_slices(af4* e, unsigned a
 // takes the unit that takes addresses 64 cycles, and a compute unit's eight wavefronts share it: some 3.4 us a round of eight blocks of
 // heads of 128; four lanes to a row's 64 bytes take 16.  A slice is asked for again, for the wavefront's next block, as soon as it has been
 // read.  Piece c (16 bytes) of row r lies in place 4 r + (c ^ (r / 4)), so that a quarter of the wavefront reads from different banks.  The
-// arithmetic is the same, and so are the bits.  us, straight from memory and so (the portions' with the order of tiles below): a portion
-// of 300 tokens, 16 heads of 128 on 8, 27.9 -> 20.9; 512 tokens behind 300 63 -> 47; 8 single tokens of 900, 31.6 -> 25.7; heads of 64
-// 23.6 -> 20.8 at most (the host's calls are as long).  Left: 320 workgroups on 256 units, one a unit, and each one's start and merge.
+// arithmetic is the same, and so are the bits.  us, straight from memory, so, and with the order of tiles below: a portion
+// of 300 tokens, 16 heads of 128 on 8, 27.7, 20.8, 15.9; 512 tokens behind 300 63.5, 46.9, 43.3; 300 tokens with 32 heads of 64 23.8, 19.8,
+// 17.7; 8 single tokens of 900 31.6 -> 25.7.  Left: 304 workgroups on 256 units, one a unit, and each one's start and merge.
 template <int DB, bool SINGLE, bool STAGED>
 __global__ void __launch_bounds__(64 * AF_WAVES)
 attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool, const int* __restrict__ table,
@@ -204,10 +204,10 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
     p_first = p_last = pos[m_row];
     tab = table + (size_t)slot[m_row] * table_stride;
   } else {
-    // the last tiles, which see the most keys, first and in all heads: what is left for a second round is short
-    const unsigned at = blockIdx.y * gridDim.x + blockIdx.x, part = gridDim.x - 1 - at / n_head;
+    // the list's first tiles, which see the most keys, first and in all heads: what is left for a second round is short
+    const unsigned at = blockIdx.y * gridDim.x + blockIdx.x, part = at / n_head;
     const int entry = tiles[(part >> 2) * 2], row0 = entries[entry * 4];
-    m_row = tiles[(part >> 2) * 2 + 1] + (part & 3) * 16;
+    m_row = tiles[(part >> 2) * 2 + 1] + (3 - (part & 3)) * 16;
     head0 = at % n_head;
     kvh = head0 / G;
     n_cols = min(16, row0 + entries[entry * 4 + 1] - m_row);
