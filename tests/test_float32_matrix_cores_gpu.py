@@ -71,6 +71,27 @@ def test_product_of_what_three_bfloat16_do_not_hold(ops, M, N, K):  # noqa: F811
     assert torch.equal(torch.isposinf(out), torch.isposinf(ref)) and torch.equal(torch.isneginf(out), torch.isneginf(ref))
 
 
+@pytest.mark.parametrize("M,N,K", [(7, 64, 20), (37, 132, 1056), (300, 96, 260), (1000, 64, 96)])
+def test_product_of_the_smallest_floats_and_of_single_ones(ops, M, N, K):  # noqa: F811
+    """Tokens, weights and both down to the subnormal floats: the bound of a 32-bit sum, and half the last place of what a subnormal
+    result holds.  One token element a row that is not zero: each result is one product, rounded once (2^-24 of it), of whose nine products
+    of pieces the three least, 2^-24 of it together, are left out; a zero row gives zeros."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g)
+    out = torch.empty(M, N, device="cuda")
+    for small_a, small_w in ((1e-36, 1.0), (1e-39, 1.0), (1e-43, 1.0), (1.0, 1e-39), (1e-20, 1e-19)):
+        x, y = a * small_a, w * small_w
+        ops.linear(dev(x), dev(y), out, "store")
+        size = f64(x).abs() @ f64(y).abs().T
+        assert ((f64(out) - f64(x) @ f64(y).T).abs() <= (K + 1) * EPS * size + 2.0 ** -150).all(), (small_a, small_w)
+    single = torch.zeros(M, K)
+    single[torch.arange(M), torch.randint(0, K, (M,), generator=g)] = a[:, 0]
+    single[M // 2] = 0.0
+    ops.linear(dev(single), dev(w), out, "store")
+    ref = f64(single) @ f64(w).T
+    assert ((f64(out) - ref).abs() <= 2 * EPS * ref.abs()).all() and not out[M // 2].any()
+
+
 def case(entries, nh, nkv, hd, P, window, seed):
     """Requests with pages scattered over a pool of rubbish; the queries of a step's last tokens, and float64's result."""
     g = torch.Generator().manual_seed(seed)

@@ -1,4 +1,4 @@
-// C = A W^T for any M, N, K, in true 32-bit arithmetic: the matrix product of
+// C = A W^T for any M, N, K, to the precision of 32-bit arithmetic: the matrix product of
 // the float32 path, and the fallback of the bfloat16 path for shapes its fast
 // kernels refuse (operands are widened to float, exactly).  A is [M, K], W is
 // [N, K], both row-major in T.
@@ -119,56 +119,58 @@ static int launch(const void* A, const void* W, void* out, int M, int N, int K, 
 // A workgroup of eight wavefronts owns 16 RB weight rows x 16 NB tokens and cuts K into eight runs of whole 32s (the
 // same runs whatever M, N and the tile are), one a wavefront.  The runs' sums meet in LDS and are added in ascending order.
 //
-// A float is the sum of three bfloat16 (8 + 8 + 8 bits: the nearest, what is left cut to eight bits, and the rest, without a remainder),
-// so a product of floats is nine products of bfloat16, which v_mfma_f32_16x16x32_bf16 multiplies exactly and adds in 32 bits.  Six of them
-// are taken, the smallest first; the three left out are below 2^-22 of the product, where each addition already rounds at 2^-24 of the
-// sum, and 32 products share a rounding in place of one each.  Six of these take 96 cycles where the 32-bit instructions take 256.  Error
-// against 64 bits, 2-norm over 2-norm, with N(0, 1) tokens and N(0, 0.02) weights (by 32-bit instructions): K = 1024 1.6e-7 (2.1e-7),
-// 3072 3.0e-7 (3.6e-7), 12288 6.4e-7 (7.1e-7), 36 4.7e-8 (8.0e-8).
-// The matrix unit cuts what it adds downwards, which leaves every sum too low by some 5e-8 of the outputs' size: small, but the same way
-// in every layer (a prompt's logits 9.2e-7 off, by 32-bit instructions 8.1e-7).  The odd runs therefore take the tokens' negatives
-// and their sums are subtracted: the mean error is then 1e-9.
-// What the three pieces cannot hold (infinite, not a number, above the largest bfloat16) leaves a sum that is not finite; such an element
-// is computed again by fused multiply-adds.  (Below 2^-110 the last piece may lie below the normal numbers, 2^-133 at least.)
+// A float is the sum of three bfloat16 (8 + 8 + 8 bits: the nearest, the nearest to what is left, and the rest, without a remainder; the
+// method of Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations",
+// ARITH 2019), so a product of floats is nine products of bfloat16, which v_mfma_f32_16x16x32_bf16 multiplies exactly and adds in 32 bits.
+// Six of them are taken; the three left out are at most 2^-24 of the product together.  The leading pieces' products have a sum of their
+// own, and the five others, each at most 2^-8 of them, one that is added at the end: what the matrix unit cuts off there is below the
+// leading sum's last place, so a single product comes out rounded once.  Six of these take 96 cycles where the 32-bit instructions take 256.
+// Operands are multiplied by 2^16 first, so that subnormal floats too have three pieces, and sums divided by 2^32.
+// Error against 64 bits, 2-norm over 2-norm, with N(0, 1) tokens and N(0, 0.02) weights (by 32-bit instructions): K = 8 2.8e-8 (5.4e-8), 36
+// 4.6e-8 (8.0e-8), 1024 8.6e-8 (2.1e-7), 3072 1.2e-7 (3.6e-7), 12288 2.4e-7 (7.0e-7); tokens of 1e-36 and of 1e-39 the same; one
+// element that is not zero 2.6e-8 (2.5e-8), at most 8.8e-8 of a product.  (All in one sum, with the second piece cut and no factors: 1024
+// 1.6e-7, one element 3.8e-8 and at most 2.0e-7, tokens of 1e-36 5e-5 and of 1e-39 3e-2; eight products make one element's error
+// 2.5e-8 and calls of 300 rows 10 % longer.)
+// The matrix unit cuts what it adds downwards, which leaves every sum too low: small, but the same way in every layer.  The odd runs
+// therefore take the tokens' negatives and their sums are subtracted: the mean error is then 1e-11.
+// What the three pieces cannot hold (infinite, not a number, above 2^111, sums above 2^95) leaves a sum that is not finite; such an element
+// is computed again by fused multiply-adds.
 //
 // A wavefront's rows come through its own part of LDS by direct loads (staged_rows.h; loaded as operands straight into registers they were
 // all that bounded these products).  What bounds them now is the splitting (52 instructions a block of 16 rows
 // and step beside 16 cycles each of six matrix instructions a pair of blocks), and for 1,024 columns the ends: the first loads and the
-// sums' way through LDS are a third of the 13 us.
-// us a call, before (32-bit instructions, operands straight from memory) and now: 300 rows x 4096 x 1024 36.9 -> 25.7, [gate; up]
-// 6144 x 1024 47.9 -> 31.9, 1024 x 2048 24.3 -> 13.3, 1024 x 3072 33.6 -> 19.5, 151936 x 1024 1,040 -> 697; 53 rows 14.0 -> 9.2,
-// 20.6 -> 12.6, 13.1 -> 7.7, 16.9 -> 10.2, 242 -> 186; one row 8.4 -> 6.9, 12.7 -> 9.3, 11.5 -> 9.0 (1024 x 3072), 171 -> 127.
+// sums' way through LDS are a third of the 15 us.
+// us a call, by 32-bit instructions with operands straight from memory, and now: 300 rows x 4096 x 1024 35.6 -> 26.2, [gate; up]
+// 6144 x 1024 46.7 -> 33.4, 1024 x 2048 23.8 -> 15.2, 1024 x 3072 32.7 -> 21.4, 151936 x 1024 1,043 -> 832; 53 rows 12.7 -> 8.7,
+// 17.8 -> 12.5, 16.2 -> 10.2 (1024 x 3072); one row 6.5 -> 5.1, 9.6 -> 7.1, 10.8 -> 9.6, 172 -> 132.  (In one sum 26.1, 32.4, 13.9, 20.2, 762.)
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gf4;
 #define GF_RUNS 8
 #define GF_STEP 32
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 gbf8;
 
-// Eight floats, times `sign` (1 or -1), as three bfloat16 each, the sum of which they are: the nearest, and twice the upper half of what
-// is left.
+// Eight floats, times `factor`, as three bfloat16 each, the sum of which they are: the nearest, the nearest to what is left, and the rest.
 struct Planes {
   gbf8 p[3];
 };
-__device__ __forceinline__ Planes split_planes(const gf4& x, const gf4& y, float sign) {
-  const uint32_t flip = __float_as_uint(sign) & 0x80000000u;
+#define GF_SCALE 65536.f         // 2^16: multiples of 2^-149 become multiples of 2^-133, the last place of a bfloat16
+__device__ __forceinline__ Planes split_planes(const gf4& x, const gf4& y, float factor) {
   uint32_t u[3][4];
   float r[8];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    r[i] = x[i];
-    r[4 + i] = y[i];
+    r[i] = x[i] * factor;
+    r[4 + i] = y[i] * factor;
   }
 #pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    uint32_t h[8];
+  for (int j = 0; j < 3; ++j)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      h[i] = j == 0 ? (__float_as_uint(r[i]) ^ flip) + 0x8000u : __float_as_uint(r[i]);
-      if (j == 0) r[i] = fmaf(r[i], sign, -__uint_as_float(h[i] & 0xffff0000u));
-      if (j == 1) r[i] -= __uint_as_float(h[i] & 0xffff0000u);
+    for (int i = 0; i < 4; ++i) {
+      u[j][i] = pack_bf16x2(r[2 * i], r[2 * i + 1]);
+      if (j < 2) {
+        r[2 * i] -= __uint_as_float(u[j][i] << 16);
+        r[2 * i + 1] -= __uint_as_float(u[j][i] & 0xffff0000u);
+      }
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) u[j][i] = __builtin_amdgcn_perm(h[2 * i + 1], h[2 * i], 0x07060302u);
-  }
   Planes s;
 #pragma unroll
   for (int j = 0; j < 3; ++j) s.p[j] = __builtin_bit_cast(gbf8, make_uint4(u[j][0], u[j][1], u[j][2], u[j][3]));
@@ -218,29 +220,34 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r16 = lane & 15, quad = lane >> 4;
 
-  gf4 acc[PL][RB][NB];
+  gf4 acc[PL][RB][NB], fine[PL][RB][NB];           // the leading products, the others
 #pragma unroll
   for (int p = 0; p < PL; ++p)
 #pragma unroll
     for (int r = 0; r < RB; ++r)
 #pragma unroll
-      for (int b = 0; b < NB; ++b) acc[p][r][b] = gf4{0.f, 0.f, 0.f, 0.f};
+      for (int b = 0; b < NB; ++b) acc[p][r][b] = fine[p][r][b] = gf4{0.f, 0.f, 0.f, 0.f};
 
-  const float sign = wave & 1 ? -1.f : 1.f;
-  // one step's products: blocks of weight rows (gate, then up), then blocks of tokens
+  const float turned = wave & 1 ? -GF_SCALE : GF_SCALE;
+  // one step's products: blocks of weight rows (gate, then up), then blocks of tokens; the pieces of the fewer are kept
   const auto multiply = [&](const Eight* e) {
-    Planes w[PL * RB];
+    constexpr int NW = PL * RB, KEEP = NW <= NB ? NW : NB, TURN = NW <= NB ? NB : NW;
+    const auto split = [&](int block) { return split_planes(e[block].x, e[block].y, block < NW ? GF_SCALE : turned); };
+    Planes kept[KEEP];
 #pragma unroll
-    for (int r = 0; r < PL * RB; ++r) w[r] = split_planes(e[r].x, e[r].y, 1.f);
+    for (int i = 0; i < KEEP; ++i) kept[i] = split(NW <= NB ? i : NW + i);
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const Planes a = split_planes(e[PL * RB + b].x, e[PL * RB + b].y, sign);
+    for (int t = 0; t < TURN; ++t) {
+      const Planes one = split(NW <= NB ? NW + t : t);
 #pragma unroll
       for (int j = 0; j < 6; ++j) {
         constexpr int WJ[6] = {2, 0, 1, 1, 0, 0}, AJ[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-        for (int r = 0; r < PL * RB; ++r)
-          acc[r / RB][r % RB][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[r].p[WJ[j]], a.p[AJ[j]], acc[r / RB][r % RB][b], 0, 0, 0);
+        for (int i = 0; i < KEEP; ++i) {
+          const int r = NW <= NB ? i : t, b = NW <= NB ? t : i;
+          gf4& sum = j < 5 ? fine[r / RB][r % RB][b] : acc[r / RB][r % RB][b];
+          sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16((NW <= NB ? kept[i] : one).p[WJ[j]], (NW <= NB ? one : kept[i]).p[AJ[j]], sum, 0, 0, 0);
+        }
       }
     }
   };
@@ -297,7 +304,7 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
     for (int r = 0; r < RB; ++r)
 #pragma unroll
       for (int b = 0; b < NB; ++b)
-        *reinterpret_cast<gf4*>(&s_tile[wave][p][b * 16 + r16][r * 16 + quad * 4]) = acc[p][r][b];
+        *reinterpret_cast<gf4*>(&s_tile[wave][p][b * 16 + r16][r * 16 + quad * 4]) = acc[p][r][b] + fine[p][r][b];
   __syncthreads();
   const int runs = (K + run - 1) / run;
   for (int e = threadIdx.x; e < TM * (TR / 4); e += 64 * GF_RUNS) {
@@ -312,7 +319,8 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
     const auto settle = [&](gf4& x, size_t row0) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (!(fabsf(x[i]) <= FLT_MAX) && n + i < N) x[i] = dot_by_fma(A + (size_t)m * lda, W + (row0 + n + i) * K, K, run);
+        if (fabsf(x[i]) <= FLT_MAX) x[i] *= 1.f / (GF_SCALE * GF_SCALE);
+        else if (n + i < N) x[i] = dot_by_fma(A + (size_t)m * lda, W + (row0 + n + i) * K, K, run);
     };
     settle(v, 0);
     if (SW) {
