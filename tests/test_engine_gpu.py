@@ -318,12 +318,13 @@ def wide_headed(tmp_path_factory):
 @pytest.mark.parametrize("graph,records", [(False, True), (True, True), (False, False)])
 def test_rows_of_very_different_lengths_by_records(wide_headed, window, graph, records):
     """Rows of 1 to some 1,300 cached tokens decode together, before, beside and after portions of another request (one launch with the
-    rows), so that the attention cuts some of them into several runs and leaves others whole; from graphs too, which are kept with and
-    without the merge: the plain model's logits, and so do the equal runs of every row that the records replace."""
+    rows; a shape that comes four times, so that it is captured and replayed at other positions), so that the attention cuts some of them
+    into several runs and leaves others whole; from graphs too, which a batch size has one of, with the merge and without: the plain
+    model's logits, and so do the equal runs of every row that the records replace.  What served the steps is seen in the list of calls."""
     from tinyinfer_amd.engine import StepEntry
     folder, V = wide_headed[window]
     starts = {"a": 1, "b": 15, "c": 1280}
-    requests = {r: random_tokens(n, V, 90 + n) for r, n in {"a": 20, "b": 34, "c": 1299, "d": 119}.items()}
+    requests = {r: random_tokens(n, V, 90 + n) for r, n in {"a": 23, "b": 37, "c": 1298, "d": 119}.items()}
     want, tol = plain_logits(folder, requests, "bfloat16", angles32=True)
     engine = build_engine(folder, "bfloat16", 1600)
     engine.ops.use_early_page_ids = records
@@ -332,7 +333,8 @@ def test_rows_of_very_different_lengths_by_records(wide_headed, window, graph, r
     # short rows alone first (whole rows), then all, then beside d's portions, then with d
     for r, n in starts.items():
         engine.step([StepEntry(r, requests[r][:n], ())])
-    plan = [("ab", 0)] * 4 + [("abc", 0)] * 5 + [("abc", 50), ("cab", 61)] + [("abcd", 0)] * 8
+    engine.ops.count_calls(True)
+    plan = [("ab", 0)] * 4 + [("abc", 0)] * 5 + [("abc", 23)] * 4 + [("cab", 19)] + [("abcd", 0)] * 8
     at["d"] = 0
     for live, portion in plan:
         steps = [(r, 1) for r in live] + ([("d", portion)] if portion else [])
@@ -340,10 +342,19 @@ def test_rows_of_very_different_lengths_by_records(wide_headed, window, graph, r
         for row, (r, n) in zip(logits, steps):
             at[r] += n
             got[r][at[r] - 1] = row
+    calls = [c["name"] for c in engine.ops.timing_report()]
+    engine.ops.count_calls(False)
     engine.cache.check()
+    assert at == {r: len(t) for r, t in requests.items()}
     for r in got:
         for position, row in got[r].items():
             assert np.abs(row - want[r][position]).max() < tol, (r, position)
+    if graph:
+        one = (1, (0,))
+        assert sorted(map(str, engine.graph_keys())) == sorted(map(str, [2, 3, 4, (one, one, one, (23, (22,)))]))
+    # (within a window of 300 every row is short enough to stay whole, unless a graph is kept for either)
+    for took in ["[fused, records", "[mfma, one launch]"] + ["[fused, records, runs]"] * (window is None or graph):
+        assert any(took in c for c in calls) == records, (took, sorted(set(calls)))
 
 
 def shared_cache_logits(w, cfg, tokens, windows, rnd):

@@ -45,16 +45,20 @@ int StepPlan::group_of(const Part* part) const {
 const int* StepPlan::table_row(int group, size_t entry) const { return cache_->table_row(group, requests_->at(entry)); }
 
 struct Engine::Impl {
-  struct Graph {
+  // a captured step: its launches, and the buffers that they name
+  struct Captured {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    DeviceBuffer meta;
-    Workspace ws;
-    Tensor logits;
-    ~Graph() {
+    ~Captured() {
       if (exec) (void)hipGraphExecDestroy(exec);
       if (graph) (void)hipGraphDestroy(graph);
     }
+  };
+  struct Graph {
+    DeviceBuffer meta;
+    Workspace ws;
+    Tensor logits;
+    Captured all, whole;       // whole: without the kernels that merge the runs of a row (a step of single tokens that may have either)
   };
   // one step, between prepare and finish
   struct Prepared {
@@ -424,33 +428,47 @@ struct Engine::Impl {
     return key;
   }
 
+  // The step's launches in a HIP graph; the buffers are there already.
+  Tensor record(Prepared& p, Captured& to) {
+    if (!capture_stream) hip_check(hipStreamCreate(&capture_stream), "hipStreamCreate");
+    e.ops.set_stream(capture_stream);
+    Tensor logits;
+    hipError_t err = hipStreamBeginCapture(capture_stream, hipStreamCaptureModeRelaxed);
+    if (err == hipSuccess) {
+      try {
+        logits = run(*p.ctx);
+      } catch (...) {
+        hipGraph_t dead = nullptr;
+        (void)hipStreamEndCapture(capture_stream, &dead);
+        if (dead) (void)hipGraphDestroy(dead);
+        e.ops.set_stream(stream);
+        throw;
+      }
+      err = hipStreamEndCapture(capture_stream, &to.graph);
+    }
+    e.ops.set_stream(stream);
+    hip_check(err, "capturing the step in a HIP graph");
+    hip_check(hipGraphInstantiate(&to.exec, to.graph, nullptr, nullptr, 0), "hipGraphInstantiate");
+    return logits;
+  }
+
   Tensor capture(const std::vector<StepEntry>& entries, const std::string& key, bool decode, std::unique_ptr<Prepared> p) {
     std::unique_ptr<Graph> g(new Graph());
     fill(*p, entries, g.get(), true);
     try {
       // a first run outside the graph: it computes this step's result and makes every workspace
       // buffer the graph will use
+      const bool either = decode && p->plan.may_merge_;
+      if (either) p->plan.merges_ = true;      // (rows in one run are left alone by the merge)
       run(*p->ctx);
       hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-      if (!capture_stream) hip_check(hipStreamCreate(&capture_stream), "hipStreamCreate");
       g->ws.frozen = true;
-      e.ops.set_stream(capture_stream);
-      hipError_t err = hipStreamBeginCapture(capture_stream, hipStreamCaptureModeRelaxed);
-      if (err == hipSuccess) {
-        try {
-          g->logits = run(*p->ctx);
-        } catch (...) {
-          hipGraph_t dead = nullptr;
-          (void)hipStreamEndCapture(capture_stream, &dead);
-          if (dead) (void)hipGraphDestroy(dead);
-          e.ops.set_stream(stream);
-          throw;
-        }
-        err = hipStreamEndCapture(capture_stream, &g->graph);
+      g->logits = record(*p, g->all);
+      // the contexts of later steps decide which of the two is replayed: neither is captured in the middle of serving
+      if (either) {
+        p->plan.merges_ = false;
+        record(*p, g->whole);
       }
-      e.ops.set_stream(stream);
-      hip_check(err, "capturing the step in a HIP graph");
-      hip_check(hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0), "hipGraphInstantiate");
     } catch (...) {
       undo(*p);
       throw;
@@ -473,10 +491,8 @@ struct Engine::Impl {
   Tensor step_graph(const std::vector<StepEntry>& entries) {
     if (foreign) return step(entries);      // parts outside the library launch on streams of their own
     bool decode = false;
-    std::string key = shape_key(entries, decode);
+    const std::string key = shape_key(entries, decode);
     auto p = begin(entries, true);
-    // a step of single tokens has two graphs: with the kernels that merge the runs of a row, and without
-    if (decode && p->plan.runs_planned_ && !p->plan.merges_) key += "w";
     auto it = graphs.find(key);
     if (it == graphs.end()) {
       if (!decode) {
@@ -494,7 +510,8 @@ struct Engine::Impl {
     Graph& g = *it->second;
     fill(*p, entries, &g, false);
     try {
-      hip_check(hipGraphLaunch(g.exec, stream), "hipGraphLaunch");
+      const bool whole = g.whole.exec && !p->plan.merges_;
+      hip_check(hipGraphLaunch(whole ? g.whole.exec : g.all.exec, stream), "hipGraphLaunch");
     } catch (...) {
       undo(*p);
       throw;

@@ -119,13 +119,12 @@ class Engine:
         return self.info()["num_graphs"]
 
     def graph_keys(self):
-        """What the captured graphs are keyed by: a batch size (a decode step; a batch size may have two, one whose
-        attention merges the runs of a row and one whose rows are whole), or a step's shape as ((tokens, (wanted places)), ...)
-        per entry."""
+        """What the captured graphs are keyed by: a batch size (a decode step), or a step's shape as
+        ((tokens, (wanted places)), ...) per entry."""
         keys = []
         for k in self.info()["graphs"]:
             if k.startswith("d"):
-                keys.append(int(k[1:].rstrip("w")))
+                keys.append(int(k[1:]))
             else:
                 shape = []
                 for entry in k[1:].split(";")[:-1]:

@@ -705,8 +705,9 @@ class StepPlan {
   const Ops* ops() const { return ops_; }
   int group_of(const Part* part) const;                           // the part's group of cache layers, -1: none
   const int* table_row(int group, size_t entry) const;            // the entry's page ids, as many as a table row holds
-  // whether a step's launches merge runs of a row: a captured step of single tokens is kept for either
-  void set_merges(bool any) { runs_planned_ = true; merges_ = merges_ || any; }
+  // whether a step's launches merge runs of a row; `ever`: whether any step of this shape may (a captured step of single tokens is
+  // then kept with the merge and without)
+  void set_merges(bool any, bool ever) { merges_ = merges_ || any; may_merge_ = may_merge_ || ever; }
   bool merges() const { return merges_; }
   bool has(const std::string& key) const { return lists_.count(key) != 0; }
   int* ints(const std::string& key, size_t n);
@@ -719,7 +720,7 @@ class StepPlan {
   std::map<std::string, int64_t> values_;
   const std::vector<EntryRecord>* entries_ = nullptr;
   int64_t M_ = 0;
-  bool decode_only_ = false, sized_for_longest_ = false, for_graph_ = false, runs_planned_ = false, merges_ = false;
+  bool decode_only_ = false, sized_for_longest_ = false, for_graph_ = false, may_merge_ = false, merges_ = false;
   int max_seq_ = 0, page_size_ = 16;
   DType act_dtype_ = DType::F32;
   const Ops* ops_ = nullptr;

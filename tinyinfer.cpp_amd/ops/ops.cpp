@@ -912,7 +912,7 @@ bool Ops::attention_from_projections(const AttentionWork& work, Workspace& ws, c
         heads, kv_heads, head_dim, P, scale, window, (hipStream_t)launch_stream());
     if (rc == 3) return false;
     check("attention_bf16", rc, "attention(decode, by records)");
-    took(work.n_run_rows ? "[fused, runs]" : "[fused]");
+    took(work.n_run_rows ? "[fused, records, runs]" : "[fused, records]");
     return true;
   }
   const int context = window == 0 ? work.split_context : std::min(work.split_context, window + 16);

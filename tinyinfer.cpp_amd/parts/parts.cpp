@@ -823,7 +823,7 @@ class Attention final : public MixerPart {
     plan.set_value(key + ".stride", launch.stride);
     plan.set_value(key + ".n", plan.for_graph() ? launch.records : used);
     plan.set_value(key + ".merge", places > 0 ? 1 : 0);
-    plan.set_merges(places > 0);
+    plan.set_merges(places > 0, launch.records > (int)rows.size());
   }
   void plan_tiles(StepPlan& plan) const {
     const auto& entries = plan.entries();
