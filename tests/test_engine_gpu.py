@@ -450,6 +450,7 @@ def test_page_ids_fetched_beside_the_position_change_no_bit(model_folders, confi
     for early in (True, False):
         engine = build_engine(folder, "bfloat16", 256)
         engine.ops.use_early_page_ids = early
+        engine.ops.force_decode_splits = 2                            # (records bring a row's page ids with them)
         engine.ops.use_fused_qk_decode = fused
         results.append(replay(engine, trace))
     for r in requests:
