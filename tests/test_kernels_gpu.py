@@ -1093,6 +1093,23 @@ def test_linear_bf16_rows_through_lds_up_to_16_rows(ops, M, N, K):
     assert (f64(outs[1][0][:M]) - ref_linear(a.cpu(), w.cpu())).abs().max() < 2e-5 * K
 
 
+@pytest.mark.parametrize("N,K,epi", [(2048, 4096, "store"), (2040, 4096, "store"), (2048, 4096, "swiglu"), (2048, 2048, "store"), (2064, 4096, "store")])
+def test_norm_in_front_of_a_weight_of_8_mi_elements_changes_no_bit(ops, N, K, epi):
+    """On either side of the size from which four wavefronts share K in place of eight: the product with the norm inside it and the
+    norm's kernel with the product behind it sum in the same order, for every number of rows that the former serves."""
+    from tinyinfer_amd.ops.kernels import NormedRows
+    g = torch.Generator().manual_seed(N + K)
+    w = dev((torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    x, nw = dev(torch.randn(16, K, generator=g)), dev(torch.rand(K, generator=g) + 0.5)
+    for M in (1, 4, 5, 8, 9, 16):
+        rows, cols = torch.empty(M, K, device="cuda", dtype=torch.bfloat16), N // 2 if epi == "swiglu" else N
+        outs = [torch.empty(M, cols, device="cuda", dtype=torch.bfloat16 if epi == "swiglu" else torch.float32) for _ in range(2)]
+        ops.linear(NormedRows(x[:M], nw, 1e-6, rows), w, outs[0], epi)
+        ops.rmsnorm(x[:M], nw, 1e-6, rows)
+        ops.linear(rows, w, outs[1], epi)
+        assert torch.equal(outs[0], outs[1]), M
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 16400, 64), (64, 20000, 1024), (40, 16387, 2048), (33, 17000, 192),
                                    (48, 16384, 1088)])
 def test_linear_bf16_wide_weight_at_17_to_64_rows(ops, M, N, K):

@@ -1642,14 +1642,16 @@ static int launch_skinny_staged(const bf16_t* A, const bf16_t* W, void* out, int
   return 0;
 }
 
+static int skinny_waves_for(int grid, int K);
 template <int EPI>
 static int launch_skinny(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda,
                           hipStream_t s) {
   const int grid = (EPI == TI_EPI_SWIGLU) ? (N + 7) / 8 : (N + 15) / 16;
   const int mt = (M + 15) / 16;
   int waves = g_skinny_waves;
-  // by the weight's shape only, so that a row's bits do not depend on the rows beside it
-  if (waves == 0) waves = (grid <= 128 && K >= 1024) ? 8 : 4;
+  // by the weight's shape only, so that a row's bits do not depend on the rows beside it; up to K = 4,096 and 16 rows as many as the
+  // kernels with the norm in front take, so that those give the same bits
+  if (waves == 0) waves = mt == 1 && K <= 4096 ? skinny_waves_for(grid, K) : (grid <= 128 && K >= 1024) ? 8 : 4;
   const bool staged = (mt > 1 && staged_fits(K, lda)) || staged_16_serves(M, N, K, lda, EPI);
 #define TI_STAGED(MTV)                                                                                      \
   if (mt == MTV && staged) {                                                                               \
