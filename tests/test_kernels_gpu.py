@@ -663,6 +663,20 @@ def test_sample_masked_rows_without_walking_them(ops, V, left):
             assert us_got < us_walked / 4, (T, top_k, top_p, us_got, us_walked)
 
 
+def test_sample_of_many_rows_within_a_bounded_workspace(ops):
+    """More long rows than the workspace serves at a time: drawn as alone, whichever piece of the call they fall into, in 64 MiB."""
+    from tinyinfer_amd.ops.kernels import Ops
+    g = torch.Generator(device="cuda").manual_seed(3)
+    n, V = 300, 151936
+    logits = torch.randn(n, V, device="cuda", generator=g) * 2
+    u, own = torch.rand(n, generator=g, device="cuda").tolist(), Ops()
+    before = torch.cuda.memory_allocated()
+    got = run_sample(own, logits, 0.9, 40, 0.95, u)
+    assert torch.cuda.memory_allocated() - before <= 65 << 20
+    for r in (0, 63, 135, 136, 137, 271, 272, 299):
+        assert got[r] == run_sample(ops, logits[r:r + 1], 0.9, 40, 0.95, u[r:r + 1])[0], r
+
+
 @pytest.mark.parametrize("n,V", [(1, 1000), (65, 20001), (150, 4096)])
 def test_sampler_of_more_rows_than_travel_with_a_launch(ops, n, V):
     """What the rows ask for goes with the launches, 64 rows at a time, and the ids come straight into the host's memory: the ids

@@ -618,7 +618,7 @@ class Ops {
   DeviceBuffer partials_;
   DeviceBuffer argmax_scratch_;
   DeviceBuffer sample_scratch_;
-  void* sample_scratch(const Tensor& logits, int64_t rows);
+  void* sample_scratch(const Tensor& logits, int64_t* rows);       // rows: how many it serves at a time
   struct { void* out = nullptr; int64_t count = 0; int splits = 0; } pending_;
   std::map<std::string, std::map<std::string, long>> tuning_;
   friend struct TunedScope;

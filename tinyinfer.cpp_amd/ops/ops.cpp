@@ -1969,9 +1969,14 @@ void Ops::argmax(const Tensor& logits, int* out) {
   check("sampling", rc, "argmax");
 }
 
-void* Ops::sample_scratch(const Tensor& logits, int64_t rows) {
+// Rows are drawn as many at a time as this much scratch serves (136 of 151,936 logits; 64 fill the chip).
+static const size_t SAMPLE_SCRATCH_BYTES = (size_t)64 << 20;
+void* Ops::sample_scratch(const Tensor& logits, int64_t* rows) {
+  *rows = std::max<int64_t>(1, logits.shape[0]);
   if (!use.radix_sample) return nullptr;
-  const size_t need = (size_t)KERNEL("sampling", ti_sample_scratch_bytes)((int)std::max<int64_t>(rows, 8), (int)logits.shape[1]);
+  const size_t row = (size_t)KERNEL("sampling", ti_sample_scratch_bytes)(1, (int)logits.shape[1]);
+  *rows = std::max<int64_t>(1, std::min<int64_t>(*rows, (int64_t)(SAMPLE_SCRATCH_BYTES / row)));
+  const size_t need = (size_t)std::max<int64_t>(*rows, std::min<int64_t>(8, (int64_t)(SAMPLE_SCRATCH_BYTES / row))) * row;
   if (sample_scratch_.bytes() < need) {
     flush();
     sample_scratch_ = DeviceBuffer(need);
@@ -1984,10 +1989,14 @@ void Ops::sample(const Tensor& logits, const float* temperature, const int* top_
   TIMED("sample " + dims(logits));
   require(logits.ndim == 2 && logits.dtype == DType::F32 && logits.contiguous(),
           "sample: logits must be contiguous float32 [n, V]");
-  void* scratch = sample_scratch(logits, logits.shape[0]);
-  int rc = KERNEL("sampling", ti_sample)((const float*)logits.data, temperature, top_k, top_p, uniform, out, scratch,
-                                         (int)logits.shape[0], (int)logits.shape[1], (hipStream_t)launch_stream());
-  check("sampling", rc, "sample");
+  int64_t most;
+  void* scratch = sample_scratch(logits, &most);
+  const int64_t n = logits.shape[0], V = logits.shape[1];
+  for (int64_t r = 0; r < n || r == 0; r += most) {
+    int rc = KERNEL("sampling", ti_sample)((const float*)logits.data + r * V, temperature + r, top_k + r, top_p + r, uniform + r, out + r, scratch,
+                                           (int)std::min(most, n - r), (int)V, (hipStream_t)launch_stream());
+    check("sampling", rc, "sample");
+  }
 }
 
 void Ops::sample_by_value(const Tensor& logits, const float* temperature, const int* top_k, const float* top_p,
@@ -1995,10 +2004,14 @@ void Ops::sample_by_value(const Tensor& logits, const float* temperature, const 
   TIMED("sample " + dims(logits));
   require(logits.ndim == 2 && logits.dtype == DType::F32 && logits.contiguous(),
           "sample: logits must be contiguous float32 [n, V]");
-  void* scratch = sample_scratch(logits, std::min<int64_t>(logits.shape[0], 64));
-  int rc = KERNEL("sampling", ti_sample_by_value)((const float*)logits.data, temperature, top_k, top_p, uniform, out, scratch,
-                                                  (int)logits.shape[0], (int)logits.shape[1], (hipStream_t)launch_stream());
-  check("sampling", rc, "sample");
+  int64_t most;
+  void* scratch = sample_scratch(logits, &most);
+  const int64_t n = logits.shape[0], V = logits.shape[1];
+  for (int64_t r = 0; r < n || r == 0; r += most) {
+    int rc = KERNEL("sampling", ti_sample_by_value)((const float*)logits.data + r * V, temperature + r, top_k + r, top_p + r, uniform + r, out + r,
+                                                    scratch, (int)std::min(most, n - r), (int)V, (hipStream_t)launch_stream());
+    check("sampling", rc, "sample");
+  }
 }
 
 void Ops::fill_zero(void* p, size_t bytes) {
