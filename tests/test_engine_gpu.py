@@ -357,6 +357,20 @@ def test_rows_of_very_different_lengths_by_records(wide_headed, window, graph, r
         assert any(took in c for c in calls) == records, (took, sorted(set(calls)))
 
 
+def test_a_step_of_more_rows_than_a_launch_has_records(model_folders):
+    """66,000 requests of one token each in one step: every row has the logits of its token."""
+    from tinyinfer_amd.engine import Engine, StepEntry
+    n, V = 66000, CONFIGS["D"]["vocab_size"]
+    engine = Engine.from_folder(model_folders("D", "bfloat16"), "bfloat16", page_size=16, max_tokens=16 * n, max_requests=n, max_seq=16)
+    logits = engine.step([StepEntry(r, [r % V], (0,)) for r in range(n)])
+    for k in range(V, n, 16 * V):
+        rows = min(V, n - k)
+        assert torch.equal(logits[k:k + rows], logits[:rows]), k
+    few = build_engine(model_folders("D", "bfloat16"), "bfloat16", 64).step([StepEntry(r, [r], (0,)) for r in range(4)])
+    # (other kernels serve four rows: three layers of sums in another order, each rounded to 2^-9, four times over)
+    assert (few - logits[:4]).abs().max() < 12 * 2.0 ** -8 * logits[:4].abs().max()
+
+
 def shared_cache_logits(w, cfg, tokens, windows, rnd):
     """The plain decoder whose layers behind the first keep no keys and values: they read the first layer's, each through a window of
     its own (None: all keys)."""

@@ -777,6 +777,7 @@ class Attention final : public MixerPart {
     return "attention.runs." + std::to_string(group) + "." + std::to_string(kv_heads * ((heads / kv_heads + 15) / 16)) + "." +
            std::to_string(heads) + "." + std::to_string(head_dim) + "." + std::to_string(window);
   }
+  static const int RUN_RECORDS_MAX = 65535;      // a launch's records are one dimension of its grid; steps of more rows have equal runs
   void plan_runs(StepPlan& plan) const {
     const Ops* ops = plan.ops();
     const int P = plan.page_size();
@@ -816,6 +817,7 @@ class Attention final : public MixerPart {
     }
     const int busy = plan.decode_only() ? 0 : n_tiles * heads;
     const Ops::RunsLaunch launch = Ops::runs_launch((int)rows.size(), blocks(plan.max_seq()), blocks(most), ways, units, busy, plan.decode_only() ? 4 : 8);
+    if (launch.records > RUN_RECORDS_MAX) return;
     int used = 0;
     int* row_list = plan.ints(key + ".rows", 4 * rows.size());
     int* runs = plan.ints(key, (size_t)launch.records * launch.stride);
