@@ -81,6 +81,7 @@ uint64_t Sampler::sample_async(const Tensor& logits, const std::vector<SamplingP
     hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
     const int cap = std::max(64, 2 * n);
     b.free_host();
+    b.cap = 0;                   // until both are there: the kernels write to them
     for (Buffers::Turn& u : b.turns) {
       hip_check(hipHostMalloc((void**)&u.i_host, (size_t)cap * 4, hipHostMallocDefault), "hipHostMalloc");
       if (!u.read_back) hip_check(hipEventCreateWithFlags(&u.read_back, hipEventDisableTiming), "hipEventCreate");
