@@ -76,3 +76,15 @@ def test_context_splits_of_the_decode_kernel(monkeypatch):
         for context in (300, 2000, 9000, 40000):
             s = a.decode_splits(rows, 8, 16, context)
             assert 1 <= s <= max(1, min(-(-context // 16) // a.MIN_BLOCKS_PER_SPLIT, a.MAX_SPLITS))
+
+
+def test_what_the_rows_of_a_draw_ask_for_packs_from_any_iterable():
+    """Requests and counters as lists, tuples, views and iterators give the same bytes, numbers beyond their type's range what ctypes
+    makes of them."""
+    from tinyinfer_amd.sampling import Sampler, SamplingParams
+    params = [SamplingParams(0.5, 7, 0.9, -3), SamplingParams()]
+    want = [bytes(a) for a in Sampler._arguments(2, params, [11, 5], [0, 2])]
+    live = {11: "a", 5: "b"}
+    for requests, counters in (((11, 5), (0, 2)), (live.keys(), iter([0, 2])), (iter([11, 5]), (c for c in (0, 2)))):
+        assert [bytes(a) for a in Sampler._arguments(2, params, requests, counters)] == want
+    assert bytes(Sampler._arguments(2, params, iter([11 + (1 << 64), 5]), [0, 2])[4]) == want[4]

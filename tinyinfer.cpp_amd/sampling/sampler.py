@@ -48,6 +48,7 @@ class Sampler:
     @staticmethod
     def _arguments(n, params, requests, counters):
         mask = (1 << 64) - 1
+        requests, counters = tuple(requests), tuple(counters)     # (any iterable)
         try:
             # packed at once: an element of a ctypes array at a time takes longer than the kernels (70 us for 64 rows, this 15)
             if not len(params) == len(requests) == len(counters) == n:
@@ -56,7 +57,7 @@ class Sampler:
             return (struct.pack(floats, *[p.temperature for p in params]), struct.pack(ints, *[p.top_k for p in params]),
                     struct.pack(floats, *[p.top_p for p in params]), struct.pack(f"{n}Q", *[p.seed & mask for p in params]),
                     struct.pack(words, *requests), struct.pack(words, *counters))
-        except (struct.error, OverflowError, ValueError):     # numbers out of their type's range, which ctypes cuts to it, or too few of them
+        except (struct.error, OverflowError, ValueError, TypeError):     # numbers out of their type's range, which ctypes cuts to it, or too few of them
             return ((ctypes.c_float * n)(*[p.temperature for p in params]), (ctypes.c_int * n)(*[p.top_k for p in params]),
                     (ctypes.c_float * n)(*[p.top_p for p in params]), (ctypes.c_uint64 * n)(*[p.seed & mask for p in params]),
                     (ctypes.c_int64 * n)(*requests), (ctypes.c_int64 * n)(*counters))
