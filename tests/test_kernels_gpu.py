@@ -1594,6 +1594,34 @@ def test_linear_with_the_norm_inside_refuses_what_it_does_not_serve(ops):
 
 
 # ---------------------------------------------- bfloat16 matrix-core attention
+@pytest.mark.parametrize("hd", [64, 128])
+def test_decode_records_say_nothing_beyond_their_runs(ops, hd):
+    """Contexts of 1 to 7 blocks, so that some wavefronts walk nothing and some fewer blocks than their record has room for: what the
+    record holds there changes no bit and is loaded from nowhere."""
+    g = torch.Generator().manual_seed(hd)
+    nh, nkv, each, pos = 4, 2, 4, [4, 16, 39, 100]
+    pages = torch.randperm(40, generator=g)[:4 * 7].view(4, 7).to(torch.int32)
+    pool = (torch.randn(40, 2 * nkv, 16, hd, generator=g) * 0.5).to(torch.bfloat16)
+    qkv = dev(torch.randn(4, (nh + 2 * nkv) * hd, generator=g))
+    lib, outs = ops.lib("attention_bf16"), []
+    ptr = lambda t: t.data_ptr()                                       # noqa: E731
+    for beyond in (0, 0x3fffffff, -7):
+        runs = torch.full((4, 8 + 4 * each), beyond, dtype=torch.int32)
+        for r, p in enumerate(pos):
+            blocks = p // 16 + 1
+            runs[r, :8] = torch.tensor([r, p, 0, blocks, -1, r, int(pages[r, p // 16]), 0])
+            for b in range(blocks):
+                runs[r, 8 + (b % 4) * each + b // 4] = pages[r, b]
+        kv, out, table, lists = dev(pool.clone()), torch.empty(4, nh * hd, device="cuda", dtype=torch.bfloat16), dev(pages), dev(runs)
+        rc = lib.ti_attention_decode_runs_bf16(ptr(qkv), qkv.shape[1], None, None, 1e-6, None, None, 0, ptr(kv), 1, ptr(table), 7, ptr(lists), 4,
+                                               runs.shape[1], None, 0, ptr(out), None, None, nh, nkv, hd, 16, hd ** -0.5, 0,
+                                               torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, lib.ti_last_error()
+        outs.append(out.cpu())
+    assert torch.isfinite(outs[0].float()).all() and outs[0].float().abs().max() > 0.1
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 class FakeCtx:
     """The fields of a step context that the attention dispatch reads."""
 
