@@ -823,6 +823,27 @@ def test_linear_bf16_weight_row_per_wavefront(ops, M, N, K):
         assert torch.equal(one[0], results[1][0][M - 1])
 
 
+def test_linear_bf16_rows_further_apart_than_a_descriptor_spans(ops):
+    """Rows 2^24 elements and more apart through the test entry point of the kernel for 17 to 64 rows, and through the plain product, which
+    other kernels serve: the bits, and the values, of rows that lie side by side."""
+    M, N, K, lda = 18, 40, 192, (1 << 24) + 8
+    lib, g = ops.lib("gemm_bf16"), torch.Generator().manual_seed(5)
+    a, w = dev((torch.rand(M, K, generator=g) * 2 - 1).to(torch.bfloat16)), dev((torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    far = torch.empty((M - 1) * lda + K, device="cuda", dtype=torch.bfloat16).as_strided((M, K), (lda, 1))
+    far.copy_(a)
+    partial = torch.empty(2 * M * N, device="cuda")
+    for epi, ks, dtype in ((0, 1, torch.float32), (1, 2, torch.float32), (2, 1, torch.bfloat16)):
+        outs = [torch.ones(M, N, device="cuda", dtype=dtype) for _ in range(2)]
+        for rows, out in zip((a, far), outs):
+            assert lib.ti_gemm_bf16_mblocks_any(rows.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, rows.stride(0), epi, partial.data_ptr(), ks,
+                                                torch.cuda.current_stream().cuda_stream) == 0, lib.ti_last_error()
+        assert torch.equal(*outs), epi
+    for epi in ("store", "add"):
+        out = torch.zeros(M, N, device="cuda")
+        ops.linear(far, w, out, epi)
+        assert (f64(out) - ref_linear(a.cpu(), w.cpu())).abs().max() < 2e-5 * K
+
+
 @pytest.mark.parametrize("M,N,K,ks", [(1, 16, 64, 1), (17, 1024, 2048, 4), (64, 1024, 3072, 8), (33, 50, 256, 3),
                                       (48, 7, 128, 2), (5, 40, 192, 1), (64, 130, 1024, 5)])
 def test_linear_bf16_mfma_fed_from_memory(ops, M, N, K, ks):

@@ -2403,9 +2403,17 @@ extern "C" int ti_gemm_bf16_store_split(const void* A, const void* W, void* out,
 // are added here)
 extern "C" int ti_gemm_bf16_mblocks_any(const void* A, const void* W, void* out, int M, int N, int K, long lda,
                                         int epi, void* partial, int ks, hipStream_t stream) {
-  TI_REQUIRE(M > 0 && M <= 64 && N > 0 && K > 0 && K % 64 == 0 && lda >= K && lda % 8 == 0 && lda < (1L << 24) && ks >= 1 && ks <= K / 64,
+  TI_REQUIRE(M > 0 && M <= 64 && N > 0 && K > 0 && K % 64 == 0 && lda >= K && lda % 8 == 0 && ks >= 1 && ks <= K / 64,
              "gemm_bf16_mblocks_any: bad sizes M=%d N=%d K=%d lda=%ld ks=%d", M, N, K, lda, ks);
   TI_REQUIRE(ks == 1 || (epi == TI_EPI_ADD_F32 && partial), "gemm_bf16_mblocks_any: a split K needs the adding epilogue");
+  if (lda >= (1L << 24) && M > 1) {      // 64 rows lie further apart than a buffer's descriptor spans: one at a time (the same bits)
+    const size_t row = (size_t)N * (epi == TI_EPI_STORE_F32 || epi == TI_EPI_ADD_F32 ? 4 : 2);
+    for (int m = 0; m < M; ++m) {
+      int rc_ = ti_gemm_bf16_mblocks_any((const bf16_t*)A + (size_t)m * lda, W, (char*)out + m * row, 1, N, K, K, epi, partial, ks, stream);
+      if (rc_) return rc_;
+    }
+    return 0;
+  }
   const bf16_t* a = (const bf16_t*)A;
   const bf16_t* w = (const bf16_t*)W;
   int rc_ = 0;
