@@ -783,7 +783,8 @@ class Attention final : public MixerPart {
     const int P = plan.page_size();
     if (general || gated || !ops || plan.act_dtype() != DType::BF16 || (head_dim != 64 && head_dim != 128) || P % 16 != 0) return;
     if (!ops->use.fast_attention || !ops->use.early_page_ids || ops->use.force_decode_splits > 0) return;
-    if (plan.decode_only() && (!ops->use.fused_qk_decode || heads / kv_heads > 16)) return;
+    Ops::Rotation rot;       // (a position encoding without a fused form: single tokens alone go another way)
+    if (plan.decode_only() && (!ops->use.fused_qk_decode || heads / kv_heads > 16 || (pos && !pos->fused(rot)))) return;
     const int group = plan.group_of(this);
     if (group < 0) return;
     const std::string key = runs_key(group);
