@@ -49,7 +49,7 @@ __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f +
 // UN: 64-element chunks of K a wavefront has in flight at a time.  All loads of a pass are
 // issued before the first product: out-of-range pieces read a valid address (piece 0 of the
 // row) and get a zeroed weight instead of a branch, so that nothing waits in between.
-// STAGES > 0 (more than 16 tokens, K of whole chunks): the rows come through LDS (staged_rows.h), a chunk a step; the same sums in the
+// STAGES > 0 (K of whole chunks; up to 16 tokens where staged_16_serves says so): the rows come through LDS (staged_rows.h), a chunk a step; the same sums in the
 // same order.  Every workgroup pulls in all token rows, which as operands from memory was most of its time.  us, before and now, at 17,
 // 32, 48 and 64 rows: 4096 x 1024 4.3 4.9 5.9 6.9 -> 3.9 4.0 3.9 4.6; [gate; up] 6144 x 1024 6.7 7.8 9.8 10.0 -> 5.3 5.8 6.9 7.9 (the
 // latter two were tiles); 4096 x 2048 8.7 9.3 10.9 11.9 -> 6.0 6.4 7.2 8.3; 12288 x 2048 16.1 17.0 17.8 18.4 -> 11.5 13.5 16.3 18.6.
@@ -1623,7 +1623,7 @@ static bool staged_fits(int K, long lda) { return K % 64 == 0 && lda < (1L << 24
 // Up to 16 rows of it as well (us, by rows in pieces, rows copied to LDS or a weight row a wavefront, and this; the same bits as the
 // former two): 6144 x 4096 under 1 and 8 rows 12.5 13.9 -> 10.5 10.7, [gate; up] 24576 x 4096 34.1 37.5 -> 32.6 33.2, 4096 x 4096 8.9 9.9 ->
 // 7.7 7.9, 4096 x 12288 20.7 22.0 -> 17.5 17.4, 2560 x 9728 14.8 17.0 -> 10.6 12.0, [gate; up] 6144 x 1024 5.2 5.3 -> 4.2 4.3,
-// 151936 x 1024 52.8 61.0 -> 49.0 53.8.  But a weight of a quarter of a GiB and more keeps the pieces under up to
+// 151936 x 1024 52.8 61.0 -> 49.0 53.8.  But a weight of 288 Mi elements (576 MiB) and more keeps the pieces under up to
 // 8 rows (151936 x 2048 104 and 117, here 112 and 122; 151936 x 4096 195 and 207, here 203 and 207).
 static int g_rows_staged = 1;      // a hook for measurements: 0: up to 16 rows take the other kernels
 static bool staged_16_serves(int M, int N, int K, long lda, int epi) {

@@ -1,7 +1,7 @@
 // Sampling on the device: greedy argmax (of equal logits the lowest index wins,
 // as /root/reference/src/cuda/sample.cu:5-11) and temperature sampling with
 // optional top-k and top-p cuts (/root/reference/src/main.cpp:40-83 does these
-// on the host with a sort).  One workgroup per row of logits.
+// on the host with a sort).  Several workgroups read a long row, and one finishes it.
 //
 // Temperature sampling draws by inverse CDF over the index order from one
 // uniform number per row, which the host derives from (seed, request, number of
@@ -173,7 +173,7 @@ struct RowsByValue {
 };
 
 // temp[r] <= 0: greedy.  top_k[r] <= 0 or >= V: no top-k cut.  top_p[r] >= 1: no top-p cut.
-// One workgroup walks the whole row some seventy times: the way for the rows that the four short
+// One workgroup walks the whole row some seventy times: the way for the rows that the two short
 // kernels below do not serve, and for a caller without their workspace.
 __device__ void sample_row_by_bisection(const float* __restrict__ logits, SampleRow want, int* __restrict__ out, int V, int r) {
   __shared__ float s_val[SNT / TI_WAVE];

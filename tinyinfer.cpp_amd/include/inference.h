@@ -577,7 +577,8 @@ class Ops {
   struct Switches {
     bool fast_gemm = true, fast_attention = true, fused_norm = true, fused_qk_decode = true, fused_qkv_prefill = true;
     bool split_k_add = true, deferred_add = true, paired_prefill = true, portion_splits = true;
-    bool early_page_ids = true;     // a step of single tokens: the decode attention fetches a row's page ids beside its position
+    bool early_page_ids = true;     // a step of single tokens: the decode attention fetches a row's page ids beside its position (off: no records
+                                    // either, which bring the ids along)
     bool radix_sample = true;       // draws with a top-k cut: many workgroups share a row (else one walks it bit by bit)
     bool shared_tiles = true;       // differential attention over a portion: a tile's wavefronts share keys and values through LDS
     int force_paired_tiles = -1;    // 1 / 0: that kernel with / without pairs, whatever the launch
