@@ -1617,8 +1617,8 @@ def test_linear_with_the_norm_inside_refuses_what_it_does_not_serve(ops):
 # ---------------------------------------------- bfloat16 matrix-core attention
 @pytest.mark.parametrize("hd", [64, 128])
 def test_decode_records_say_nothing_beyond_their_runs(ops, hd):
-    """Contexts of 1 to 7 blocks, so that some wavefronts walk nothing and some fewer blocks than their record has room for: what the
-    record holds there changes no bit and is loaded from nowhere."""
+    """Contexts of 1 to 7 blocks, so that some wavefronts walk nothing and some fewer blocks than their record has room for: which page the
+    record names there, or none, changes no bit."""
     g = torch.Generator().manual_seed(hd)
     nh, nkv, each, pos = 4, 2, 4, [4, 16, 39, 100]
     pages = torch.randperm(40, generator=g)[:4 * 7].view(4, 7).to(torch.int32)
@@ -1626,7 +1626,7 @@ def test_decode_records_say_nothing_beyond_their_runs(ops, hd):
     qkv = dev(torch.randn(4, (nh + 2 * nkv) * hd, generator=g))
     lib, outs = ops.lib("attention_bf16"), []
     ptr = lambda t: t.data_ptr()                                       # noqa: E731
-    for beyond in (0, 0x3fffffff, -7):
+    for beyond in (0, 39, -7):
         runs = torch.full((4, 8 + 4 * each), beyond, dtype=torch.int32)
         for r, p in enumerate(pos):
             blocks = p // 16 + 1

@@ -254,7 +254,7 @@ __device__ __forceinline__ void walk_blocks(const PagedKV& kv, const Frag8* qf, 
     auto info = [&](int j, int& page) {
       const int jc = max(0, min(j, nc - 1));
       const int blk = first + (c0 + jc) * stride;
-      page = page == ASK ? __builtin_amdgcn_readlane(mine, jc) : j < nc ? page : -1;
+      if (page == ASK) page = __builtin_amdgcn_readlane(mine, jc);
       return BlockInfo{blk * 16, j < nc && page >= 0, check(blk)};
     };
     auto issue = [&](int j, KVPair<HD>& f, BlockInfo& A, BlockInfo& B, int pa = ASK, int pb = ASK) {
@@ -377,7 +377,8 @@ struct DecodeMerge {
 // A launch by records (TI_RUN_* in tinyinfer_kernels.h): the host cuts every row's context into runs of its own choice and says what each
 // workgroup walks.  Record i, of a launch's `run_stride` ints: the header below, then for each of the workgroup's
 // NW wavefronts (run_stride - TI_RUN_HEAD) / NW page ids, at least four: those of the first blocks that it walks (-1: given back;
-// beyond the run's end anything, which is not looked at).  A workgroup's first loads are then its header and its page ids, side by side, and its
+// beyond the run's end any page of the pool, or a number below 0: loaded, as every loop's last loads are, and not used; asking for
+// the run's end first took up to 0.2 us a layer).  A workgroup's first loads are then its header and its page ids, side by side, and its
 // keys' are the next.  Runs of no blocks are nobody's:
 // their workgroups end at once (a captured graph launches as many records for every step).
 struct DecodeRuns {
@@ -423,6 +424,7 @@ decode_run(DecodeMerge<HD, NW>& sm, int ridx, int y, int split, const bf16_t* __
   const int n_cols = min(16, G - part * 16);
   const int head = kvh * G + part * 16 + r16;   // valid if r16 < n_cols
 
+  // (By equal runs, for callers of Ops that plan no records and for steps of more rows than a launch has records.)
   // slot == nullptr: row m of the step is row m of the block tables (a step of single tokens, where the
   // host knows it), and a table row has at most DEC_TABLE_LDS entries.  The row's page ids are then asked
   // for at once, all of them, beside the position instead of behind it (which pages the workgroup walks

@@ -442,8 +442,8 @@ int ti_attention_decode_prepared_bf16(const float* qkv, int row_width, const flo
                                       int n_head, int n_kv, int hd, int page_size, float scale, int window,
                                       int n_splits, hipStream_t stream);
 // the same by records (int32 [n_runs][run_stride]: what each workgroup walks, TI_RUN_*, then the page ids of its first blocks,
-// (run_stride - TI_RUN_HEAD) / wavefronts of them, at least four, for each of its four wavefronts): every row in as many runs as
-// the host chose.  n_rows > 0: rows in several runs are merged, by the rows' records int32 [n_rows][4] = (row, first run's place,
+// (run_stride - TI_RUN_HEAD) / wavefronts of them, at least four, for each of its four wavefronts; beyond its end any page of the pool, or
+// a number below 0): every row in as many runs as the host chose.  n_rows > 0: rows in several runs are merged, by the rows' records int32 [n_rows][4] = (row, first run's place,
 // runs, -); part_o f32 [places][n_head][hd], part_ml f32 [places][n_head][2]
 int ti_attention_decode_runs_bf16(const float* qkv, int row_width, const float* q_w, const float* k_w, float eps,
                                   const float* inv_freq, const float* rope_table, int table_len, void* pool, int write_kv,
