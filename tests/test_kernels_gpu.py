@@ -1100,6 +1100,24 @@ def test_linear_bf16_rows_through_lds_at_17_to_64_rows(ops, N, K):
         assert (f64(out) - ref[:M]).abs().max() < tol, M
 
 
+@pytest.mark.parametrize("N,K,epi", [(8192, 1152, "store"), (8208, 1152, "store"), (8208, 1152, "store_act"), (12288, 1024, "swiglu"), (12304, 1024, "swiglu"),
+                                     (12304, 2112, "swiglu")])
+def test_linear_bf16_where_tiles_take_over_from_16_row_workgroups(ops, N, K, epi):
+    """On either side of one round of 16-row workgroups (of one and a half for gate and up): float64's values within the bound of 32-bit
+    sums, for 32, 33 and 64 rows."""
+    g = torch.Generator().manual_seed(N + K)
+    a, w = (torch.rand(64, K, generator=g) * 2 - 1).to(torch.bfloat16), (torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16)
+    ref, tol, ad, wd = ref_linear(a, w), 2e-5 * K, dev(a), dev(w)
+    if epi == "swiglu":
+        gate, up = ref[:, :N // 2], ref[:, N // 2:]
+        ref, tol = gate / (1 + torch.exp(-gate)) * up, None
+    for M in (32, 33, 64):
+        out = torch.empty(M, ref.shape[1], device="cuda", dtype=torch.float32 if epi == "store" else torch.bfloat16)
+        ops.linear(ad[:M], wd, out, epi)
+        most = ref[:M].abs().max()
+        assert (f64(out) - ref[:M]).abs().max() < (tol if epi == "store" else 0.005 * most + 10 * 2e-5 * K), M
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 4104, 2112), (5, 40, 64), (8, 2056, 4160), (13, 1000, 1088), (16, 6144, 2048)])
 def test_linear_bf16_rows_through_lds_up_to_16_rows(ops, M, N, K):
     """Up to 16 rows through LDS stages: fewer steps than stages, four and eight wavefronts, a last tile of few weight rows.  Every

@@ -1713,7 +1713,10 @@ static int g_use_pipelined = 1;
 // With the rows through LDS the 16-row workgroups hold out longer where the product stores and is not cut over K (which it is into
 // the residual, and from K = 4096 on): to 1000 Mi (us, tiles and 16-row workgroups: 6144 x 2560 at 64 rows, 960 Mi, 16.7 and 16.5, at 32
 // 14.7 and 12.0; [gate; up] 12288 x 2048 at 48 rows, 1152 Mi, 17.8 and 16.3, at 64, 1536 Mi, 18.4 and 18.6; 19456 x 2560 at 17 rows,
-// 807 Mi, 24.7 and 23.9, at 32, 1520 Mi, 26.4 and 28.7).
+// 807 Mi, 24.7 and 23.9, at 32, 1520 Mi, 26.4 and 28.7).  But every workgroup pulls in all token rows, and beyond one round of them (two to a
+// unit at 64 rows) the tiles win again from 280 Mi on (weights that are not in the cache; 8192 x 2048 at 48 rows 12.3 and 11.9, 10240 x
+// 2048 12.7 and 15.9, 12288 x 2048 at 24 12.7 and 14.2, 16000 x 1024 at 48 8.7 and 12.3).  [gate; up] tiles cost more, and lose up to three
+// to a unit, up to 32 rows and from K above 2048 on (12288 x 1024 at 48 rows 10.5 and 10.2; 16000 x 1024 at 32 10.7 and 10.2, at 48 10.9 and 12.8).
 static long g_tiled_from = 280L << 20;           // 17..64 rows x weight elements from which steps take the tiled kernels
 static long g_tiled_from_16 = 600L << 20;        // the same for 13..16 rows
 #define TILED_FROM_STORED (1000L << 20)
@@ -1723,10 +1726,16 @@ static void set_tiled_from(long rows_times_elems) {
   g_tiled_from_16 = rows_times_elems >= (280L << 20) && rows_times_elems < (1L << 59) ? rows_times_elems / 280 * 600
                                                                                      : rows_times_elems;
 }
+// 17..64 rows, a product that stores: whether the 16-row workgroups hold out to g_tiled_from_stored
+static bool holds_out(int M, long rows, int K, int epi) {
+  if (epi == TI_EPI_ADD_F32 || K >= 4096) return false;
+  const long groups = (rows + 15) / 16;
+  return epi == TI_EPI_SWIGLU ? groups <= 3L * compute_units() || M <= 32 || K > 2048 : groups <= 2L * compute_units();
+}
 static bool large_weight(int M, int N, int K, int epi) {
   const long rows = (epi == TI_EPI_SWIGLU) ? 2L * N : (long)N;
   if (M <= 12 || M > 64 || K % PBK != 0) return false;
-  return rows * K * M >= (M <= 16 ? g_tiled_from_16 : epi == TI_EPI_ADD_F32 || K >= 4096 ? g_tiled_from : g_tiled_from_stored);
+  return rows * K * M >= (M <= 16 ? g_tiled_from_16 : holds_out(M, rows, K, epi) ? g_tiled_from_stored : g_tiled_from);
 }
 
 // 1 (default): up to GR_MMAX tokens and a weight of fewer than GR_ROWS_BELOW rows take the kernel
