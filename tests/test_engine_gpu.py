@@ -357,6 +357,36 @@ def test_rows_of_very_different_lengths_by_records(wide_headed, window, graph, r
         assert any(took in c for c in calls) == records, (took, sorted(set(calls)))
 
 
+def test_a_captured_shape_whose_portion_grows_long(wide_headed):
+    """One shape, first behind a short context, where the portion and the single token share an attention launch, then behind a long
+    one, where the portion's keys are cut into runs: the steps from graphs launch as the eager ones do, and give their logits up to the
+    rounding of another order of sums (other runs for what is captured)."""
+    from tinyinfer_amd.engine import StepEntry
+    folder, V = wide_headed[None]
+    p, r, got = random_tokens(2100, V, 31), random_tokens(60, V, 32), []
+    for graph in (False, True):
+        engine = build_engine(folder, "bfloat16", 2400)
+        engine.step([StepEntry("p", p[:40], ()), StepEntry("r", r[:30], ())])
+        run, at, rows, served = engine.step_graph if graph else engine.step, 40, [], []
+        for k in range(8):
+            if k == 4:
+                engine.step([StepEntry("p", p[at:1900], ())])
+                at = 1900
+            engine.ops.count_calls(True)
+            rows.append(run([StepEntry("r", r[30 + k:31 + k], (0,)), StepEntry("p", p[at:at + 16], (15,))]).clone())
+            served.append([c["name"] for c in engine.ops.timing_report()])
+            at += 16
+        engine.ops.count_calls(False)
+        got.append(torch.stack(rows))
+        # (a replay issues no calls)
+        assert [any("one launch" in c for c in s) for s in served] == ([True, True] + [False] * 6 if graph else [True] * 4 + [False] * 4)
+        if graph:
+            assert engine.graph_keys() == [((1, (0,)), (16, (15,)))] * 2
+    assert torch.equal(got[0][:4], got[1][:4])
+    # (bfloat16's rounding through two layers, two roundings each: 2^-9 of the largest logit at a time, four times over)
+    assert (got[0] - got[1]).abs().max() < 16 * 2.0 ** -9 * got[0].abs().max()
+
+
 def test_a_step_of_more_rows_than_a_launch_has_records(model_folders):
     """66,000 requests of one token each in one step: every row has the logits of its token."""
     from tinyinfer_amd.engine import Engine, StepEntry

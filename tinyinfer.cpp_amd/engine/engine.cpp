@@ -491,8 +491,9 @@ struct Engine::Impl {
   Tensor step_graph(const std::vector<StepEntry>& entries) {
     if (foreign) return step(entries);      // parts outside the library launch on streams of their own
     bool decode = false;
-    const std::string key = shape_key(entries, decode);
+    std::string key = shape_key(entries, decode);
     auto p = begin(entries, true);
+    if (!decode) key += p->plan.choices_;
     auto it = graphs.find(key);
     if (it == graphs.end()) {
       if (!decode) {

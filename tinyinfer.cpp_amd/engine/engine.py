@@ -120,7 +120,8 @@ class Engine:
 
     def graph_keys(self):
         """What the captured graphs are keyed by: a batch size (a decode step), or a step's shape as
-        ((tokens, (wanted places)), ...) per entry."""
+        ((tokens, (wanted places)), ...) per entry.  (A shape comes twice where its contexts have asked both for one
+        attention launch and for two.)"""
         keys = []
         for k in self.info()["graphs"]:
             if k.startswith("d"):

@@ -710,6 +710,8 @@ class StepPlan {
   // then kept with the merge and without)
   void set_merges(bool any, bool ever) { merges_ = merges_ || any; may_merge_ = may_merge_ || ever; }
   bool merges() const { return merges_; }
+  // a choice that decides what the step launches: steps of one shape that differ in it are captured apart (not steps of single tokens)
+  void add_to_shape(char choice) { choices_ += choice; }
   bool has(const std::string& key) const { return lists_.count(key) != 0; }
   int* ints(const std::string& key, size_t n);
   void set_value(const std::string& key, int64_t v) { values_[key] = v; }
@@ -719,6 +721,7 @@ class StepPlan {
   struct List { size_t offset = 0, n = 0; std::vector<int> host; };
   std::map<std::string, List> lists_;
   std::map<std::string, int64_t> values_;
+  std::string choices_;
   const std::vector<EntryRecord>* entries_ = nullptr;
   int64_t M_ = 0;
   bool decode_only_ = false, sized_for_longest_ = false, for_graph_ = false, may_merge_ = false, merges_ = false;
