@@ -602,8 +602,8 @@ class Ops {
   static int plan_runs(const std::vector<RunsRow>& list, const RunsLaunch& launch, int ways, int units, int busy, double beside_us,
                        int head_dim, int page_size, int* runs, int* rows, int* used);
   // a step's portions and single-token rows in one launch (else one after the other)?  portion_us: how long the portions take in it
-  static bool portions_with_rows(int n_tiles_small, int n_rows, int heads, int kv_heads, int portion_context, int rows_context, int window,
-                                 int units, int head_dim);
+  static bool portions_with_rows(int n_tiles_small, int n_rows, int heads, int kv_heads, int portion_context, int longest_blocks,
+                                 long row_blocks, int window, int units, int head_dim);
   static double portion_us(int portion_context, int window);
   // runs of keys for the prefill kernel with 64-row tiles, and whether it pairs a heavy with a light tile
   static int portion_launch(int n_tiles_small, int heads, int portion_context, int window, int units, bool* paired);

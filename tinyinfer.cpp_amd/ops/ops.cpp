@@ -842,20 +842,40 @@ int Ops::plan_runs(const std::vector<RunsRow>& list, const RunsLaunch& launch, i
 // one): 504 tokens beside 8 rows of 1,000 30.9 -> 18.2, behind 504 others 37.1 -> 23.5; 512 beside 64 rows of 200 35.3 -> 25.8, of 1,000
 // 81.9 -> 59.8; 32 beside 8 of 1,000 23.1 -> 16.3.
 static const double PORTION_START_US = 7.8, PORTION_TURN_US = 1.57 / 4;     // of a tile: its start, and a turn of 32 keys (four groups take them in rotation)
+static const double PORTION_MERGE_US = 4.9;
 double Ops::portion_us(int portion_context, int window) {
   const int seen = window == 0 ? portion_context : std::min(portion_context, window + 64);
   return PORTION_START_US + PORTION_TURN_US * ((seen + 31) / 32);
 }
-bool Ops::portions_with_rows(int n_tiles_small, int n_rows, int heads, int kv_heads, int portion_context, int rows_context, int window,
+// Rows of `total` blocks, the longest of `longest`, in a launch of their own (as plan_runs cuts them)
+static double rows_us(int n_rows, int longest, long total, int ways, int units, int head_dim) {
+  const double size = head_dim / 128.0, read = (double)total * ways * 16 * 512 * size / RUN_BYTES_US;
+  double best = -1.0;
+  for (int s = 1; s <= RUN_MOST; ++s) {
+    const int len = std::max((longest + s - 1) / s, std::min(longest, RUN_LEAST_BLOCKS));
+    const long items = std::max<long>(n_rows, (total + len - 1) / len), load = (items * ways + units - 1) / units;
+    const double walk = load * len * RUN_BLOCK_US * size;
+    const double us = RUN_START_US + std::sqrt(walk * walk + read * read) + (items > n_rows ? RUN_MERGE_US : 0.0);
+    best = best < 0 ? us : std::min(best, us);
+  }
+  return best;
+}
+// Where the portions' keys want runs: one launch lasts as long as the portions whole, whose turns take a quarter longer for a tile by itself (no other reads
+// the keys it reads), and it must not cost the rows another round of the units: what is left over starts when the first are through.  Differences a layer
+// of steps at 16 and 32 heads, one launch less two, us: rows of 2,048 beside 16 tokens behind 2,500 and 4,000: 8 rows +8 and more, 16 -1 and
+// +20, 32 +6 and +14, 48 -10 (4,000), 64 +3 and +1; 8 rows beside 128, 256 and 512 tokens behind 2,000, 3,000 and 2,000 / 4,000 / 8,000 0, +8,
+// -10 / +2 / +26; 2 rows beside 64 behind 1,000 -3, beside 16 behind 8,000 +87.  The rule takes the better of the two or one within 2 us for all.
+bool Ops::portions_with_rows(int n_tiles_small, int n_rows, int heads, int kv_heads, int portion_context, int longest_blocks, long row_blocks, int window,
                              int units, int head_dim) {
   if (n_tiles_small == 0 || n_rows == 0 || (long)n_tiles_small * heads > units) return false;
   const int S = portion_launch(n_tiles_small, heads, portion_context, window, units, nullptr);
   if (S == 1) return true;
-  const double whole = portion_us(portion_context, window);
-  const double apart = PORTION_START_US + (whole - PORTION_START_US) / S + RUN_MERGE_US + RUN_START_US +
-                       RUN_BLOCK_US * (head_dim / 128.0) * (rows_context / 16.0) *
-                           std::max(1.0, (double)n_rows * kv_heads / units);
-  return whole < apart;
+  const int ways = kv_heads * ((heads / kv_heads + 15) / 16), left = units - n_tiles_small * heads;
+  const long groups = (long)n_rows * ways;
+  if (left <= 0 || (groups + left - 1) / left > (groups + units - 1) / units) return false;
+  const double turns = portion_us(portion_context, window) - PORTION_START_US;
+  const double apart = PORTION_START_US + turns / S + PORTION_MERGE_US + rows_us(n_rows, longest_blocks, row_blocks, ways, units, head_dim);
+  return PORTION_START_US + turns * (1.0 + 0.25 / n_tiles_small) < apart;
 }
 
 static int typical_context(const AttentionWork& w) {

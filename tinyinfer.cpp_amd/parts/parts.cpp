@@ -791,7 +791,8 @@ class Attention final : public MixerPart {
     if (plan.has(key)) return;
     const auto& entries = plan.entries();
     std::vector<Ops::RunsRow> rows;
-    int n_tiles = 0, portion_context = 0, longest = 0;
+    int n_tiles = 0, portion_context = 0, longest = 0, longest_blocks = 0;
+    long row_blocks = 0;
     for (size_t i = 0; i < entries.size(); ++i) {
       const auto& e = entries[i];
       if (e.n_tokens > 1) {
@@ -802,6 +803,8 @@ class Attention final : public MixerPart {
       const int first = window > 0 ? std::max(0, e.start - window + 1) / 16 : 0;
       rows.push_back({e.row0, e.start, first, e.start / 16 + 1 - first, (int)i, plan.table_row(group, i)});
       longest = std::max(longest, e.start + 1);
+      longest_blocks = std::max(longest_blocks, rows.back().blocks);
+      row_blocks += rows.back().blocks;
     }
     if (rows.empty()) return;
     // The lists' sizes hold for every replay of a captured step; what they hold, and whether a step's portions and rows share a launch, is the
@@ -813,7 +816,8 @@ class Attention final : public MixerPart {
     double beside_us = 0.0;
     if (!plan.decode_only()) {
       if (!ops->use.paired_prefill || !ops->use.portion_splits || ops->use.force_paired_tiles >= 0) return;
-      const bool together = Ops::portions_with_rows(n_tiles, (int)rows.size(), heads, kv_heads, portion_context, longest, window, units, head_dim);
+      const bool together = Ops::portions_with_rows(n_tiles, (int)rows.size(), heads, kv_heads, portion_context, longest_blocks, row_blocks, window,
+                                                          units, head_dim);
       plan.add_to_shape(together ? '1' : '2');
       if (!together) {
         plan.ints(key, 0);       // asked and answered for the other parts of this list
