@@ -6,6 +6,8 @@ import ctypes
 import os
 import re
 
+import pytest
+
 import tinyinfer_amd  # noqa: F401
 from tinyinfer_amd.csrc import build
 from tinyinfer_amd.ops import kernels
@@ -88,3 +90,20 @@ def test_what_the_rows_of_a_draw_ask_for_packs_from_any_iterable():
     for requests, counters in (((11, 5), (0, 2)), (live.keys(), iter([0, 2])), (iter([11, 5]), (c for c in (0, 2)))):
         assert [bytes(a) for a in Sampler._arguments(2, params, requests, counters)] == want
     assert bytes(Sampler._arguments(2, params, iter([11 + (1 << 64), 5]), [0, 2])[4]) == want[4]
+
+
+@pytest.mark.parametrize("heads,rows,context,tokens,behind,one", [
+    # whole portions: enough units left, or short rows; then long rows beside portions on most units or all, which took up to 12 % longer in one launch
+    (16, 2, 2000, 512, 0, True), (16, 2, 2000, 768, 0, True), (16, 2, 12000, 768, 4000, True), (16, 4, 500, 1024, 8000, True),
+    (16, 6, 12000, 576, 8000, True), (16, 16, 4000, 576, 8000, True), (16, 64, 4000, 1024, 4000, True), (32, 2, 2000, 384, 0, True),
+    (16, 2, 2000, 1024, 4000, False), (16, 2, 12000, 768, 0, False), (16, 2, 12000, 1024, 0, False), (16, 4, 4000, 832, 0, False),
+    (16, 1, 4000, 1024, 8000, False), (16, 6, 12000, 640, 0, False), (32, 2, 2000, 512, 1500, False), (32, 2, 12000, 512, 6000, False),
+    # portions whose keys want runs
+    (16, 48, 2048, 16, 4000, True), (16, 2, 2048, 64, 1000, True), (16, 8, 2048, 16, 2500, False), (16, 32, 2048, 16, 2500, False),
+    (16, 2, 2048, 16, 8000, False), (16, 8, 2048, 512, 8000, False)])
+def test_portions_and_rows_share_a_launch_where_that_was_measured_to_be_faster(heads, rows, context, tokens, behind, one):
+    """Steps of 8 heads for keys on 256 compute units, each timed with one attention launch and with two: the rule takes the faster."""
+    from tinyinfer_amd import native
+    blocks = context // 16 + 1
+    assert native.lib().ti_portions_with_rows(-(-tokens // 64), behind + tokens, behind + min(tokens, 64), rows, blocks, rows * blocks, 16384,
+                                              heads, 8, 0, 256, 128) == one

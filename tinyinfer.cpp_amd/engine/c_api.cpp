@@ -1529,6 +1529,16 @@ int ti_portion_launch(int n_tiles_small, int heads, int portion_context, int win
   if (paired) *paired = p ? 1 : 0;
   return s;
 }
+int ti_portions_with_rows(int n_tiles_small, int context, int least_context, int n_rows, int longest_blocks, long row_blocks, int max_seq, int heads,
+                          int kv_heads, int window, int units, int head_dim) {
+  Ops::PortionsLaunch p;
+  p.n_tiles_small = n_tiles_small;
+  p.context = context;
+  p.least_context = least_context;
+  const int most = (window > 0 ? std::min(max_seq, window + 16) : max_seq) / 16 + 1, ways = kv_heads * ((heads / kv_heads + 15) / 16);
+  const auto launch = Ops::runs_launch(n_rows, most, most, ways, units, n_tiles_small * heads, 8);
+  return Ops::portions_with_rows(p, n_rows, longest_blocks, row_blocks, launch.records, heads, kv_heads, window, units, head_dim) ? 1 : 0;
+}
 int ti_ops_timing_report(void* ops_, const char** out) {
   TI_BEGIN
   Json a = Json::array();

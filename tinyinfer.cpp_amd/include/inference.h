@@ -602,8 +602,11 @@ class Ops {
   static int plan_runs(const std::vector<RunsRow>& list, const RunsLaunch& launch, int ways, int units, int busy, double beside_us,
                        int head_dim, int page_size, int* runs, int* rows, int* used);
   // a step's portions and single-token rows in one launch (else one after the other)?  portion_us: how long the portions take in it
-  static bool portions_with_rows(int n_tiles_small, int n_rows, int heads, int kv_heads, int portion_context, int longest_blocks,
-                                 long row_blocks, int window, int units, int head_dim);
+  struct PortionsLaunch {
+    int n_tiles_small = 0, context = 0, least_context = 0;     // tiles of 64 rows; the keys that the longest and the shortest see
+  };
+  static bool portions_with_rows(const PortionsLaunch& portions, int n_rows, int longest_blocks, long row_blocks, int records, int heads,
+                                 int kv_heads, int window, int units, int head_dim);
   static double portion_us(int portion_context, int window);
   // runs of keys for the prefill kernel with 64-row tiles, and whether it pairs a heavy with a light tile
   static int portion_launch(int n_tiles_small, int heads, int portion_context, int window, int units, bool* paired);
@@ -1379,4 +1382,7 @@ int ti_ops_call(void* ops, const char* op, const ti_tensor* t, int n_t, const do
 int ti_ops_timing_report(void* ops, const char** out_json);     // [{"name", "calls", "us"}] since timing was switched on
 int ti_decode_splits(int n_rows, int kv_heads, int heads, int context, int typical, int units, int head_dim);
 int ti_portion_launch(int n_tiles_small, int heads, int portion_context, int window, int units, int* paired);
+// whether a step's portions and single-token rows share an attention launch (Ops::portions_with_rows; its records for an engine of max_seq)
+int ti_portions_with_rows(int n_tiles_small, int context, int least_context, int n_rows, int longest_blocks, long row_blocks, int max_seq, int heads,
+                          int kv_heads, int window, int units, int head_dim);
 }

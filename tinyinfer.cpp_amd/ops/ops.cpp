@@ -860,22 +860,52 @@ static double rows_us(int n_rows, int longest, long total, int ways, int units, 
   }
   return best;
 }
+// The same beside portions that leave few units free: in the records of that launch, and where the units left do not hold them all, some start when a
+// tile is through: the tiles' ends lie between the shortest's and the longest's, and eight tenths of the way fits what was measured.
+static double rows_beside_us(int n_rows, int longest, long total, int ways, int units, int busy, int records, int head_dim, double portion, double least) {
+  const double size = head_dim / 128.0, read = (double)total * ways * 16 * 512 * size / RUN_BYTES_US;
+  double best = -1.0;
+  for (int s = 1; s <= RUN_MOST; ++s) {
+    const int len = std::max((longest + s - 1) / s, std::min(longest, RUN_LEAST_BLOCKS));
+    const long items = std::max<long>(n_rows, (total + len - 1) / len);
+    if (items > records && s > 1) break;
+    const double load = items * ways <= units - busy ? 1.0 : 1.0 + (double)(items * ways - (units - busy)) / units;
+    const double walk = len * RUN_BLOCK_BESIDE_US * size, merge = items > n_rows ? RUN_MERGE_US : 0.0;
+    double us = RUN_START_US + std::sqrt(load * walk * load * walk + read * read) + RUN_NEXT_US * (load - 1.0);
+    if (load > 1.0) us = std::max(us, least + 0.8 * (portion - least) + RUN_START_US + walk);
+    us = std::max(us, portion) + merge;
+    best = best < 0 ? us : std::min(best, us);
+  }
+  return best;
+}
+// Whole portions, few rows (a quarter of a round of the units, or less): the rows' runs in the one launch are as many as the units left make records, so
+// that a long row beside portions on most units is cut into few, and they may wait for a tile.  Differences a layer, one launch less two, us: 2 rows of
+// 2,000 beside 512, 768 and 1,024 tokens at 16 heads -8, -10, -4, behind 4,000 -11 (768) and +10 (1,024); 2 of 12,000 -4, +6, +12, and -20, +21; 4 of 4,000
+// beside 832 +4, 1 of 4,000 beside 1,024 behind 8,000 +30; 6 of 12,000 beside 640 +14, 576 behind 8,000 -42; 2 of 2,000 at 32 heads beside 384 -9, beside 512
+// behind 1,500 +12.  Of 154 such steps the rule never takes one launch where two are more than 1.5 % faster (one launch always: up to 12 %), nor two where one is 4 % faster.  More rows: one
+// launch (16 of 4,000 within 1 %, others faster).
 // Where the portions' keys want runs: one launch lasts as long as the portions whole, whose turns take a quarter longer for a tile by itself (no other reads
 // the keys it reads), and it must not cost the rows another round of the units: what is left over starts when the first are through.  Differences a layer
 // of steps at 16 and 32 heads, one launch less two, us: rows of 2,048 beside 16 tokens behind 2,500 and 4,000: 8 rows +8 and more, 16 -1 and
 // +20, 32 +6 and +14, 48 -10 (4,000), 64 +3 and +1; 8 rows beside 128, 256 and 512 tokens behind 2,000, 3,000 and 2,000 / 4,000 / 8,000 0, +8,
 // -10 / +2 / +26; 2 rows beside 64 behind 1,000 -3, beside 16 behind 8,000 +87.  The rule takes the better of the two or one within 2 us for all.
-bool Ops::portions_with_rows(int n_tiles_small, int n_rows, int heads, int kv_heads, int portion_context, int longest_blocks, long row_blocks, int window,
-                             int units, int head_dim) {
-  if (n_tiles_small == 0 || n_rows == 0 || (long)n_tiles_small * heads > units) return false;
-  const int S = portion_launch(n_tiles_small, heads, portion_context, window, units, nullptr);
-  if (S == 1) return true;
-  const int ways = kv_heads * ((heads / kv_heads + 15) / 16), left = units - n_tiles_small * heads;
+bool Ops::portions_with_rows(const PortionsLaunch& portions, int n_rows, int longest_blocks, long row_blocks, int records, int heads, int kv_heads,
+                             int window, int units, int head_dim) {
+  if (portions.n_tiles_small == 0 || n_rows == 0 || (long)portions.n_tiles_small * heads > units) return false;
+  const int S = portion_launch(portions.n_tiles_small, heads, portions.context, window, units, nullptr);
+  const int ways = kv_heads * ((heads / kv_heads + 15) / 16), busy = portions.n_tiles_small * heads, left = units - busy;
   const long groups = (long)n_rows * ways;
+  const double whole = portion_us(portions.context, window);
+  const double rows_alone = rows_us(n_rows, longest_blocks, row_blocks, ways, units, head_dim);
+  if (S == 1) {
+    if (groups > units / 4) return true;
+    const double one = rows_beside_us(n_rows, longest_blocks, row_blocks, ways, units, busy, records, head_dim, whole, portion_us(portions.least_context, window));
+    return one < whole + rows_alone;
+  }
   if (left <= 0 || (groups + left - 1) / left > (groups + units - 1) / units) return false;
-  const double turns = portion_us(portion_context, window) - PORTION_START_US;
-  const double apart = PORTION_START_US + turns / S + PORTION_MERGE_US + rows_us(n_rows, longest_blocks, row_blocks, ways, units, head_dim);
-  return PORTION_START_US + turns * (1.0 + 0.25 / n_tiles_small) < apart;
+  const double turns = whole - PORTION_START_US;
+  const double apart = PORTION_START_US + turns / S + PORTION_MERGE_US + rows_alone;
+  return PORTION_START_US + turns * (1.0 + 0.25 / portions.n_tiles_small) < apart;
 }
 
 static int typical_context(const AttentionWork& w) {

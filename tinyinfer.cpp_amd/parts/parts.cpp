@@ -791,13 +791,16 @@ class Attention final : public MixerPart {
     if (plan.has(key)) return;
     const auto& entries = plan.entries();
     std::vector<Ops::RunsRow> rows;
-    int n_tiles = 0, portion_context = 0, longest = 0, longest_blocks = 0;
+    Ops::PortionsLaunch portions;
+    int longest = 0, longest_blocks = 0;
     long row_blocks = 0;
     for (size_t i = 0; i < entries.size(); ++i) {
       const auto& e = entries[i];
       if (e.n_tokens > 1) {
-        n_tiles += (e.n_tokens + PREFILL_TILE_SMALL - 1) / PREFILL_TILE_SMALL;
-        portion_context = std::max(portion_context, e.start + e.n_tokens);
+        const int least = e.start + std::min(e.n_tokens, PREFILL_TILE_SMALL);
+        portions.least_context = portions.n_tiles_small ? std::min(portions.least_context, least) : least;
+        portions.n_tiles_small += (e.n_tokens + PREFILL_TILE_SMALL - 1) / PREFILL_TILE_SMALL;
+        portions.context = std::max(portions.context, e.start + e.n_tokens);
         continue;
       }
       const int first = window > 0 ? std::max(0, e.start - window + 1) / 16 : 0;
@@ -813,20 +816,20 @@ class Attention final : public MixerPart {
     const auto blocks = [&](int context) { return (window > 0 ? std::min(context, window + 16) : context) / 16 + 1; };
     const int most = plan.for_graph() ? plan.max_seq() : longest;
     const int ways = kv_heads * ((heads / kv_heads + 15) / 16), units = ops->units();
+    const int busy = plan.decode_only() ? 0 : portions.n_tiles_small * heads;
+    const Ops::RunsLaunch launch = Ops::runs_launch((int)rows.size(), blocks(plan.max_seq()), blocks(most), ways, units, busy, plan.decode_only() ? 4 : 8);
     double beside_us = 0.0;
     if (!plan.decode_only()) {
       if (!ops->use.paired_prefill || !ops->use.portion_splits || ops->use.force_paired_tiles >= 0) return;
-      const bool together = Ops::portions_with_rows(n_tiles, (int)rows.size(), heads, kv_heads, portion_context, longest_blocks, row_blocks, window,
-                                                          units, head_dim);
+      const bool together = Ops::portions_with_rows(portions, (int)rows.size(), longest_blocks, row_blocks, launch.records, heads, kv_heads, window,
+                                                    units, head_dim);
       plan.add_to_shape(together ? '1' : '2');
       if (!together) {
         plan.ints(key, 0);       // asked and answered for the other parts of this list
         return;
       }
-      beside_us = Ops::portion_us(portion_context, window);
+      beside_us = Ops::portion_us(portions.context, window);
     }
-    const int busy = plan.decode_only() ? 0 : n_tiles * heads;
-    const Ops::RunsLaunch launch = Ops::runs_launch((int)rows.size(), blocks(plan.max_seq()), blocks(most), ways, units, busy, plan.decode_only() ? 4 : 8);
     if (launch.records > RUN_RECORDS_MAX) {
       plan.ints(key, 0);
       return;
