@@ -107,3 +107,13 @@ def test_portions_and_rows_share_a_launch_where_that_was_measured_to_be_faster(h
     blocks = context // 16 + 1
     assert native.lib().ti_portions_with_rows(-(-tokens // 64), behind + tokens, behind + min(tokens, 64), rows, blocks, rows * blocks, 16384,
                                               heads, 8, 0, 256, 128) == one
+
+
+@pytest.mark.parametrize("rows,context,cut", [(33, 300, False), (33, 2000, True), (33, 5000, True), (36, 3000, True), (40, 5000, True), (44, 3000, True),
+                                              (48, 300, False), (48, 3000, True), (52, 3000, False), (64, 3000, False), (66, 300, False),
+                                              (66, 3000, True), (72, 3000, True), (96, 3000, False)])
+def test_rows_on_more_than_a_round_of_the_units_are_cut_where_whole_ones_leave_units_idle(rows, context, cut):
+    """Rows of one length, 8 heads for keys on 256 units: a fifth of the two workgroups a unit idle and long contexts; the others stay whole."""
+    from tinyinfer_amd import native
+    used = native.lib().ti_decode_runs(rows, context // 16 + 1, 8192, 16, 8, 256, 128)
+    assert used > rows if cut else used == rows

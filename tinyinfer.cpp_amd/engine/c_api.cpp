@@ -1539,6 +1539,17 @@ int ti_portions_with_rows(int n_tiles_small, int context, int least_context, int
   const auto launch = Ops::runs_launch(n_rows, most, most, ways, units, n_tiles_small * heads, 8);
   return Ops::portions_with_rows(p, n_rows, longest_blocks, row_blocks, launch.records, heads, kv_heads, window, units, head_dim) ? 1 : 0;
 }
+int ti_decode_runs(int n_rows, int blocks, int max_seq, int heads, int kv_heads, int units, int head_dim) {
+  const int ways = kv_heads * ((heads / kv_heads + 15) / 16);
+  const auto launch = Ops::runs_launch(n_rows, max_seq / 16 + 1, blocks, ways, units, 0, 4);
+  const std::vector<int> pages(blocks, 0);
+  std::vector<Ops::RunsRow> list;
+  for (int i = 0; i < n_rows; ++i) list.push_back({i, 16 * blocks - 1, 0, blocks, i, pages.data()});
+  std::vector<int> runs((size_t)launch.records * launch.stride), rows(4 * (size_t)n_rows);
+  int used = 0;
+  Ops::plan_runs(list, launch, ways, units, 0, 0.0, head_dim, 16, runs.data(), rows.data(), &used);
+  return used;
+}
 int ti_ops_timing_report(void* ops_, const char** out) {
   TI_BEGIN
   Json a = Json::array();

@@ -1382,6 +1382,8 @@ int ti_ops_call(void* ops, const char* op, const ti_tensor* t, int n_t, const do
 int ti_ops_timing_report(void* ops, const char** out_json);     // [{"name", "calls", "us"}] since timing was switched on
 int ti_decode_splits(int n_rows, int kv_heads, int heads, int context, int typical, int units, int head_dim);
 int ti_portion_launch(int n_tiles_small, int heads, int portion_context, int window, int units, int* paired);
+// the runs that a step of n_rows single tokens is cut into, each behind `blocks` blocks of 16 (Ops::plan_runs)
+int ti_decode_runs(int n_rows, int blocks, int max_seq, int heads, int kv_heads, int units, int head_dim);
 // whether a step's portions and single-token rows share an attention launch (Ops::portions_with_rows; its records for an engine of max_seq)
 int ti_portions_with_rows(int n_tiles_small, int context, int least_context, int n_rows, int longest_blocks, long row_blocks, int max_seq, int heads,
                           int kv_heads, int window, int units, int head_dim);

@@ -203,6 +203,8 @@ def lib() -> ctypes.CDLL:
         handle.ti_decode_splits.argtypes = [c_int] * 7
         handle.ti_portion_launch.restype = c_int
         handle.ti_portion_launch.argtypes = [c_int] * 5 + [P(c_int)]
+        handle.ti_decode_runs.restype = c_int
+        handle.ti_decode_runs.argtypes = [c_int] * 7
         handle.ti_portions_with_rows.restype = c_int
         handle.ti_portions_with_rows.argtypes = [c_int] * 5 + [ctypes.c_long] + [c_int] * 6
         handle.ti_detach_allocator.restype = None

@@ -740,8 +740,12 @@ int Ops::decode_splits(int n_rows, int kv_heads, int heads, int context, int typ
 // positions of one row takes 6.0 + 0.147 n alone (13 blocks 7.8, 129 25.2); rows in several runs need the merge, 2.7; all
 // workgroups together read at most 6.4e6 bytes a us, and the two bounds wear on each other as the root of their squares' sum does
 // (8 rows of 129 blocks: in runs of 129 30.9, 65 23.4, 43 20.4, 33 19.9, 22 21.5; 23 rows of 6 to 107 blocks: 107 29.3, 72 26.3,
-// 36 27.1, 27 25.0; 32 equal runs of them would be 24).  Beside portions eight wavefronts walk a run at 0.2 a block.
+// 36 27.1, 27 25.0; 32 equal runs of them would be 24).  Beside portions eight wavefronts walk a run at 0.2 a block.  Where units hold two runs
+// and others one (33 to 48 rows of 8 heads for keys on 256 units) a block of both takes 0.51: 33 whole rows of 63, 188 and 376 blocks 38, 103 and 199,
+// so that such rows may be cut (33 rows of 3,000 and 6,000 tokens 3,813 and 6,504 us a step whole, 3,334 and 5,214 in three and five runs each).
 static const double RUN_START_US = 6.0, RUN_MERGE_US = 2.7, RUN_BLOCK_US = 0.147, RUN_BLOCK_BESIDE_US = 0.2, RUN_BYTES_US = 6.4e6;
+static const double RUN_BLOCK_SHARED_US = 0.257;
+static const double RUN_MERGE_MANY_US = 3.5;  // rows on more than a round of the units: 33 of 400 tokens are better whole, 48 of 3,000 in two
 static const double RUN_NEXT_US = 4.0;       // a workgroup that starts behind another on its unit
 static const int RUN_LEAST_BLOCKS = 4;       // a block a wavefront
 static const int RUN_MOST = 32;              // runs a row (the merge asks for so many at once)
@@ -753,6 +757,8 @@ Ops::RunsLaunch Ops::runs_launch(int n_rows, int most_blocks, int listed_blocks,
   // a round of the compute units where half of it holds a record a row (finer runs gain nothing then), two rounds where it does not
   const int round = std::max(1, std::max(units / 4, units - busy) / std::max(1, ways));
   int records = n_rows <= round / 2 ? round : 2 * round * ((n_rows + 2 * round - 1) / (2 * round));
+  // whole rows that leave a fifth of those empty may be cut, into up to three times what the units hold at once
+  if (!busy && n_rows > round && 5 * n_rows < 4 * records) records = std::max(records, 6 * round);
   const int most_runs = std::min(RUN_MOST, (most_blocks + RUN_LEAST_BLOCKS - 1) / RUN_LEAST_BLOCKS);
   records = (int)std::min<long>(records, (long)n_rows * std::max(1, most_runs));
   l.records = std::max(records, n_rows);
@@ -773,6 +779,7 @@ int Ops::plan_runs(const std::vector<RunsRow>& list, const RunsLaunch& launch, i
   const double size = head_dim / 128.0, block = (busy ? RUN_BLOCK_BESIDE_US : RUN_BLOCK_US) * size;
   const double read = (double)total * ways * 16 * 512 * size / RUN_BYTES_US;
   int length = longest;
+  const double merge = !busy && (long)list.size() * ways > units ? RUN_MERGE_MANY_US : RUN_MERGE_US;
   double best = -1.0;
   for (int s = 1; s <= RUN_MOST; ++s) {
     const int len = std::max((longest + s - 1) / s, std::min(longest, RUN_LEAST_BLOCKS));
@@ -783,10 +790,13 @@ int Ops::plan_runs(const std::vector<RunsRow>& list, const RunsLaunch& launch, i
     double load;      // runs that a unit walks one after the other
     if (busy) load = groups <= units - busy ? 1.0 : 1.0 + (double)(groups - std::max(0, units - busy)) / units;
     else load = (double)((groups + units - 1) / units);
-    const double walk = load * len * block;
-    double us = RUN_START_US + std::sqrt(walk * walk + read * read) + (items > (long)list.size() ? RUN_MERGE_US : 0.0);
-    us += RUN_NEXT_US * (busy ? load - 1.0 : std::max(0.0, std::ceil(load / 2) - 1.0));      // (two workgroups fit a unit, one beside portions)
-    us = std::max(us, beside_us + (items > (long)list.size() ? RUN_MERGE_US : 0.0));
+    // (two workgroups fit a unit, one beside portions; what starts behind them waits for memory as the others do)
+    const double walk = load * len * block + (busy ? 0.0 : RUN_NEXT_US * std::max(0.0, 0.5 * groups / units - 1.0));
+    double us = std::sqrt(walk * walk + read * read);
+    if (!busy && load > 1.0) us = std::max(us, std::ceil((double)total * ways / units / len) * len * RUN_BLOCK_SHARED_US * size);
+    us += RUN_START_US + (items > (long)list.size() ? merge : 0.0);
+    if (busy) us += RUN_NEXT_US * (load - 1.0);
+    us = std::max(us, beside_us + (items > (long)list.size() ? merge : 0.0));
     if (best < 0 || us < best - 1e-9) {
       best = us;
       length = len;
@@ -855,7 +865,9 @@ static double rows_us(int n_rows, int longest, long total, int ways, int units, 
     const int len = std::max((longest + s - 1) / s, std::min(longest, RUN_LEAST_BLOCKS));
     const long items = std::max<long>(n_rows, (total + len - 1) / len), load = (items * ways + units - 1) / units;
     const double walk = load * len * RUN_BLOCK_US * size;
-    const double us = RUN_START_US + std::sqrt(walk * walk + read * read) + (items > n_rows ? RUN_MERGE_US : 0.0);
+    double us = std::sqrt(walk * walk + read * read);
+    if (load > 1) us = std::max(us, load * len * RUN_BLOCK_SHARED_US * size);
+    us += RUN_START_US + (items > n_rows ? RUN_MERGE_US : 0.0);
     best = best < 0 ? us : std::min(best, us);
   }
   return best;
