@@ -2115,3 +2115,15 @@ def test_attention_bf16_far_key(ops):
         ctx = FakeCtx(entries)
         assert run_attention(ops, ctx, View(dev(table)), dev(q), dev(pool), out, 1, 1, hd, 1.0 / 8, None)
         assert (f64(out[-1]) - f64(v[far, 0])).abs().max() < 2e-2
+
+
+@pytest.mark.parametrize("words,skip", [(1, 0), (3, 0), (4, 0), (4097, 0), (4099, 1), (70001, 0), (262144, 0), (262143, 3)])
+def test_words_copied_from_pinned_memory(ops, words, skip):
+    """Whole, with a tail of one to three words, and from a word that sixteen bytes do not start at; nothing beyond is written."""
+    src = torch.empty(words + skip + 4, dtype=torch.int32, pin_memory=True)
+    src.copy_(torch.arange(7, 7 + words + skip + 4, dtype=torch.int32))
+    dst = torch.full((words + 8,), -1, dtype=torch.int32, device="cuda")
+    rc = ops.lib("core").ti_copy_words(dst.data_ptr(), src.data_ptr() + 4 * skip, words, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0
+    assert torch.equal(dst[:words].cpu(), src[skip:skip + words]) and (dst[words:] == -1).all()

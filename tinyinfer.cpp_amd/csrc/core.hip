@@ -631,6 +631,25 @@ extern "C" int ti_fill_zero(void* p, long bytes, hipStream_t stream) {
   return 0;
 }
 
+// Words from memory that the device reads as it stands (pinned host memory), sixteen bytes a lane where both sides allow it.  The runtime copies
+// up to 16 KB by a kernel of its own, and what is longer by an engine that starts when the stream has come to it and is waited for:
+// 34 KB in front of a step 66 us, 6 of them the copy.
+__global__ void copy_words_kernel(uint32_t* __restrict__ to, const uint32_t* __restrict__ from, long words, long quads) {
+  const long stride = (long)gridDim.x * blockDim.x, first = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  for (long i = first; i < quads; i += stride) reinterpret_cast<uint4*>(to)[i] = reinterpret_cast<const uint4*>(from)[i];
+  for (long i = 4 * quads + first; i < words; i += stride) to[i] = from[i];
+}
+
+extern "C" int ti_copy_words(void* to, const void* from, long words, hipStream_t stream) {
+  TI_REQUIRE(words >= 0 && (((uintptr_t)to | (uintptr_t)from) & 3) == 0, "copy_words: %ld words from %p to %p", words, from, to);
+  if (words == 0) return 0;
+  const long quads = (((uintptr_t)to | (uintptr_t)from) & 15) == 0 ? words / 4 : 0;
+  const long lanes = quads ? quads : words;
+  copy_words_kernel<<<(unsigned)std::min<long>((lanes + 255) / 256, 256), 256, 0, stream>>>((uint32_t*)to, (const uint32_t*)from, words, quads);
+  TI_LAUNCH_CHECK();
+  return 0;
+}
+
 // Random weights on the device.  Element i of a tensor is a pure function of (seed, i): two
 // 24-bit uniforms from splitmix64's output function, then Box-Muller for a normal.  The host's
 // generator (the one that writes model folders) is the same function.  The logarithm, root and

@@ -51,6 +51,8 @@ int ti_qk_norm_inplace(float* qkv, int row_width, const float* q_w, const float*
                        float eps, hipStream_t stream);
 // zero `bytes` bytes (whole four-byte words) with a kernel
 int ti_fill_zero(void* p, long bytes, hipStream_t stream);
+// copy four-byte words with a kernel; `from` may be pinned host memory
+int ti_copy_words(void* to, const void* from, long words, hipStream_t stream);
 // random values, element i a pure function of (seed, i).  dtype 0 / 1: kind 0 normal(a, b), 1 uniform
 // [a, b), 2 constant a; dtype 2 (int32): uniform integers in [a, b)
 int ti_fill_random(int dtype, void* p, long n, int kind, float a, float b, unsigned long seed, hipStream_t stream);

@@ -26,6 +26,7 @@ namespace {
 void hip_check(hipError_t e, const char* what) {
   if (e != hipSuccess) throw EngineError(std::string(what) + ": " + hipGetErrorString(e));
 }
+const size_t META_RUNTIME_INTS = 4096, META_KERNEL_INTS = 1 << 18;      // step metadata of more than 16 KB and up to 1 MB is copied by a kernel
 const int STEP_GRAPH_AFTER = 2;    // a step's shape is captured when it comes for this many times ...
                                    // ... and EngineOptions::max_step_graphs such graphs are kept
 }  // namespace
@@ -336,7 +337,11 @@ struct Engine::Impl {
       for (size_t i = 0; i < R; ++i) memcpy(base + i * W, c.table_row(g, entries[i].request), (size_t)W * 4);
       ++gi;
     }
-    hip_check(hipMemcpyAsync(dev, host, total * 4, hipMemcpyHostToDevice, stream), "hipMemcpyAsync(step metadata)");
+    // (beyond 16 KB, which the runtime copies by a kernel, its copy engine would start when the stream has come to it: META_KERNEL_INTS)
+    if (total > META_RUNTIME_INTS && total <= META_KERNEL_INTS)
+      e.ops.copy_words(dev, host, total);
+    else
+      hip_check(hipMemcpyAsync(dev, host, total * 4, hipMemcpyHostToDevice, stream), "hipMemcpyAsync(step metadata)");
     hip_check(hipEventRecord(meta_event[my_turn], stream), "hipEventRecord");
     meta_used[my_turn] = true;
 

@@ -557,6 +557,7 @@ class Ops {
   void sample_by_value(const Tensor& logits, const float* temperature, const int* top_k, const float* top_p, const float* uniform,
                        int* out);
   void fill_zero(void* p, size_t bytes);
+  void copy_words(void* to, const void* from, size_t words);      // four-byte words, by a kernel; `from` may be pinned host memory
   void fill_random(const Tensor& t, const std::string& init, double a, double b, uint64_t seed);
   // Partial sums that a product left in the workspace are added now (same order, same bits as
   // the norm that would have added them).  Every launch through this object does it first.

@@ -2081,6 +2081,11 @@ void Ops::fill_zero(void* p, size_t bytes) {
   check("core", rc, "fill_zero");
 }
 
+void Ops::copy_words(void* to, const void* from, size_t words) {
+  int rc = KERNEL("core", ti_copy_words)(to, from, (long)words, (hipStream_t)launch_stream());
+  check("core", rc, "copy_words");
+}
+
 void Ops::fill_random(const Tensor& t, const std::string& init, double a, double b, uint64_t seed) {
   require(t.contiguous(), "fill_random: the tensor must be contiguous");
   const int kind = init == "normal" ? 0 : init == "uniform" ? 1 : init == "constant" ? 2 : -1;
