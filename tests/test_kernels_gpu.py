@@ -1661,6 +1661,51 @@ def test_decode_records_say_nothing_beyond_their_runs(ops, hd):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
+@pytest.mark.parametrize("stages", [1, 2])
+@pytest.mark.parametrize("hd,P,nh,nkv,window", [(128, 16, 16, 8, 0), (128, 48, 10, 2, 0), (64, 16, 16, 1, 0), (64, 64, 4, 2, 70), (128, 32, 3, 3, 40)])
+def test_decode_records_through_lds(ops, hd, P, nh, nkv, window, stages):
+    """Keys and values through LDS stages: the bits, and the cache, of the kernel that takes them straight from memory.  Contexts around the
+    edges of blocks, of pairs of them, of pages, and beyond the 64 blocks a wavefront holds the page ids of; page ids with the record and
+    behind it."""
+    g = torch.Generator().manual_seed(hd + P)
+    pos = [0, 1, 15, 16, 31, 32, 47, 63, 64, 65, 127, 128, 255, 257, 1000, 4500]
+    n, each, width = len(pos), 6, (nh + 2 * nkv) * hd
+    need = [p // P + 1 for p in pos]
+    table = torch.zeros(n, max(need), dtype=torch.int32)
+    ids = torch.randperm(sum(need), generator=g).to(torch.int32)
+    for r, (a, k) in enumerate(zip(np.cumsum([0] + need), need)):
+        table[r, :k] = ids[a:a + k]
+    pool = (torch.randn(sum(need), 2 * nkv, P, hd, generator=g) * 0.5).to(torch.bfloat16)
+    qkv, q_w, k_w = dev(torch.randn(n, width, generator=g)), dev(1 + 0.1 * torch.randn(hd, generator=g)), dev(1 + 0.1 * torch.randn(hd, generator=g))
+    inv = dev(10000.0 ** (-torch.arange(0, hd, 2).float() / hd))
+    runs = torch.full((n, 8 + 4 * each), -1, dtype=torch.int32)
+    for r, p in enumerate(pos):
+        first = max(0, p - window + 1) // 16 if window else 0
+        blocks = p // 16 + 1 - first
+        runs[r, :8] = torch.tensor([r, p, first, blocks, -1, r, int(table[r, p // P]), 0])
+        for b in range(min(blocks, 4 * each)):
+            runs[r, 8 + (b % 4) * each + b // 4] = table[r, (first + b) * 16 // P]
+    lib, stream = ops.lib("attention_bf16"), torch.cuda.current_stream().cuda_stream
+    ptr = lambda t: t.data_ptr()                                       # noqa: E731
+    tab, at, lists = dev(table), dev(torch.tensor(pos, dtype=torch.int32)), dev(runs)
+    slot = dev(torch.arange(n, dtype=torch.int32))
+    straight, staged = dev(pool.clone()), dev(pool.clone())
+    want, got = (torch.empty(n, nh * hd, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    common = (ptr(qkv), width, ptr(q_w), ptr(k_w), 1e-6, ptr(inv), None, 0)
+    rc = lib.ti_attention_decode_prepared_bf16(*common, ptr(straight), 1, ptr(tab), tab.shape[1], ptr(at), ptr(slot), ptr(want), None, None, n, nh, nkv,
+                                               hd, P, hd ** -0.5, window, 1, stream)
+    assert rc == 0, lib.ti_last_error()
+    try:
+        assert lib.ti_tuning_set(b"decode_stages", stages) == 0
+        rc = lib.ti_attention_decode_runs_bf16(*common, ptr(staged), 1, ptr(tab), tab.shape[1], ptr(lists), n, runs.shape[1], None, 0, ptr(got), None,
+                                               None, nh, nkv, hd, P, hd ** -0.5, window, stream)
+        assert rc == 0, lib.ti_last_error()
+    finally:
+        lib.ti_tuning_reset()
+    assert torch.isfinite(want.float()).all() and want.float().abs().max() > 0.1
+    assert torch.equal(got, want) and torch.equal(staged, straight)
+
+
 class FakeCtx:
     """The fields of a step context that the attention dispatch reads."""
 

@@ -29,6 +29,7 @@
 #include "tinyinfer_kernels.h"
 #include "tinyinfer_kernels_tuning.h"
 #include "qk_prep.h"
+#include "staged_rows.h"
 
 TI_ERROR_API
 
@@ -224,25 +225,19 @@ struct NoHook {
 // workgroup runs each exactly once, so they may hold a barrier).  Loads come back in the
 // order they were issued: what a caller asks for in `after_table` arrives before the keys
 // and values, and what it computes in `before_attend` runs while those are in flight.
-// `held`: how many lanes already have the page id of their first block (`held_id`; the others and later
-// blocks ask the table); FIRST4: `first4` holds the ids of the first four blocks as well, in scalar registers,
-// so that the first loads do not wait for the lanes'.
-template <int HD, bool FIRST4 = false, typename Check, typename AfterTable = NoHook, typename BeforeAttend = NoHook,
+template <int HD, typename Check, typename AfterTable = NoHook, typename BeforeAttend = NoHook,
           typename AfterSecond = NoHook>
 __device__ __forceinline__ void walk_blocks(const PagedKV& kv, const Frag8* qf, int first, int stride, int n,
                                             int lo, int hi, int kv_last, float scale, Check check, float& m,
                                             float& l, floatx4* o, AfterTable after_table = NoHook{},
-                                            BeforeAttend before_attend = NoHook{}, float cap2 = 0.f, int held = 0,
-                                            int held_id = -1, const int* first4 = nullptr,
+                                            BeforeAttend before_attend = NoHook{}, float cap2 = 0.f,
                                             AfterSecond after_second = NoHook{}) {
   const int lane = threadIdx.x & 63;
-  constexpr int ASK = -0x7fffffff;
   bool hooks_due = true;
   for (int c0 = 0; c0 == 0 || c0 < n; c0 += 64) {      // (once at least: the hooks)
     const int nc = max(0, min(64, n - c0));
-    const int have = c0 == 0 ? held : 0;
-    int mine = lane < min(nc, have) ? held_id : -1;
-    if (nc > have && lane >= have && lane < nc) mine = kv.table[((first + (c0 + lane) * stride) * 16) / kv.P];
+    int mine = -1;
+    if (lane < nc) mine = kv.table[((first + (c0 + lane) * stride) * 16) / kv.P];
     if (hooks_due) {
       __builtin_amdgcn_sched_barrier(0);
       after_table();
@@ -254,24 +249,22 @@ __device__ __forceinline__ void walk_blocks(const PagedKV& kv, const Frag8* qf, 
     auto info = [&](int j, int& page) {
       const int jc = max(0, min(j, nc - 1));
       const int blk = first + (c0 + jc) * stride;
-      if (page == ASK) page = __builtin_amdgcn_readlane(mine, jc);
+      page = __builtin_amdgcn_readlane(mine, jc);
       return BlockInfo{blk * 16, j < nc && page >= 0, check(blk)};
     };
-    auto issue = [&](int j, KVPair<HD>& f, BlockInfo& A, BlockInfo& B, int pa = ASK, int pb = ASK) {
+    auto issue = [&](int j, KVPair<HD>& f, BlockInfo& A, BlockInfo& B) {
+      int pa, pb;
       A = info(j, pa);
       B = info(j + 1, pb);
       load_pair<HD>(kv, max(pa, 0), A.key0, max(pb, 0), B.key0, f);
     };
-    const bool given = FIRST4 && c0 == 0;
-    if (given) issue(0, f0, a0, b0, first4[0], first4[1]);
-    else issue(0, f0, a0, b0);
+    issue(0, f0, a0, b0);
     if (hooks_due) {
       __builtin_amdgcn_sched_barrier(0);
       before_attend();
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (given) issue(2, f1, a1, b1, first4[2], first4[3]);
-    else issue(2, f1, a1, b1);
+    issue(2, f1, a1, b1);
     if (hooks_due) {
       __builtin_amdgcn_sched_barrier(0);
       after_second();
@@ -285,6 +278,188 @@ __device__ __forceinline__ void walk_blocks(const PagedKV& kv, const Frag8* qf, 
       issue(i + 6, f1, a1, b1);
     }
   }
+}
+
+// f(integral_constant<int, 0>), f(<1>), ... f(<N - 1>), until one returns false
+template <typename F, int... Is>
+__device__ __forceinline__ void unrolled_while_impl(F&& f, std::integer_sequence<int, Is...>) {
+  (void)(f(std::integral_constant<int, Is>{}) && ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void unrolled_while(F&& f) {
+  unrolled_while_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// ---- the same walk with the operands through LDS
+// As operands straight from memory a pair's keys lie with a row in every lane, and a load of 1 KiB takes the unit that takes addresses 64
+// cycles; direct loads of four whole rows each take 16.
+// A wavefront has ST stages of its own, of a pair each, and meets no barrier; a stage is asked for again as soon as it lies in registers.
+// With it, the arguments asked for beside the record, and the merge of the columns in use alone, a launch at 16 heads, 8 for keys, in a
+// chain of 28 (us, straight from memory before): 1 row of 200 7.6 -> 5.7, 8 of 2,048 in four runs with their merge 19.7 -> 17.9, 2 of
+// 16,000 in sixteen 30.0 -> 27.7, 23 of 900 in two 27.9 -> 22.9, 64 of 200 17.6 -> 14.6, 64 of 2,048 99.5 -> 98.4 (5.5 TB/s).  What is left
+// of the shortest: 1.5 until its loads are out, 2.5 until they are back (a unit takes about 50 bytes a ns), 1.3 for two pairs, 0.7 the merge.
+//
+// Row R of a pair's keys (block A's 16, then block B's) lies at R HD 2 bytes with piece c (16 bytes) in place c ^ f(R),
+// f(R) = R % 4 + 4 ((R / 8) % 4): the rows that sixteen lanes read together differ in it.  The values of a block lie as in a page of 16
+// rows, 32 bytes a dim, with the two halves of dim d changed where bits 2 and 3 of d differ.
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+template <int HD> struct StagedPairs {
+  static constexpr int NP = HD / 8;                      // pieces of a key row
+  static constexpr int ROWS = 64 / NP;                   // key rows a load
+  static constexpr int K_LOADS = 32 / ROWS, V_LOADS = HD / 32;   // of a pair's keys, of one block's values
+  static constexpr int LOADS = K_LOADS + 2 * V_LOADS;
+  static constexpr unsigned K_BYTES = 32 * HD * 2, V_BYTES = 16 * HD * 2, BYTES = K_BYTES + 2 * V_BYTES;
+  static_assert(2 * LOADS <= 63, "vmcnt counts to 63");
+
+  unsigned k_at[HD / 32], v_at;       // LDS: this lane's pieces of the operands in stage 0
+  unsigned k_lane, v_lane;            // memory: this lane's piece of a load, in bytes
+  unsigned lds;                       // stage 0 of this wavefront
+
+  __device__ __forceinline__ StagedPairs(unsigned lds_, int P) : lds(lds_) {
+    const int lane = threadIdx.x & 63, r16 = lane & 15, quad = lane >> 4;
+    const int R = ((r16 >> 2) << 3) | (r16 & 3);
+    const int f = r16 & (NP - 1);                        // f(R): bits 0, 1 and 3, 4 of R
+#pragma unroll
+    for (int s = 0; s < HD / 32; ++s) k_at[s] = lds + R * (HD * 2) + (((s * 4 + quad) ^ f) << 4);
+    v_at = lds + K_BYTES + (quad >> 1) * V_BYTES + r16 * 32 + ((((quad & 1) ^ (r16 >> 2) ^ (r16 >> 3)) & 1) << 4);
+    const int row = lane / NP, c = lane % NP;            // of a load's rows; bits 2 of R and above come with the load's number
+    k_lane = (unsigned)(row * HD * 2 + ((c ^ (row & 3)) << 4));
+    v_lane = (unsigned)((lane >> 1) * P * 2 + (((lane ^ (lane >> 3) ^ (lane >> 4)) & 1) << 4));
+  }
+  // the loads of a pair into the stage at `stage` (bytes); pages that exist, as for load_pair
+  __device__ __forceinline__ void ask(const PagedKV& kv, int pageA, int keyA, int pageB, int keyB, unsigned stage) const {
+    const size_t page_elems = (size_t)2 * kv.n_kv * kv.P * HD, head_elems = (size_t)kv.P * HD;
+    const bf16_t* ka = kv.pool + (size_t)pageA * page_elems + kv.kvh * head_elems;
+    const bf16_t* kb = kv.pool + (size_t)pageB * page_elems + kv.kvh * head_elems;
+    const bf16_t* va = ka + kv.n_kv * head_elems;
+    const bf16_t* vb = kb + kv.n_kv * head_elems;
+    if (kv.P != 16) {
+      const int rowA = keyA % kv.P, rowB = keyB % kv.P;
+      ka += (size_t)rowA * HD;
+      kb += (size_t)rowB * HD;
+      va += rowA;
+      vb += rowB;
+    }
+    const unsigned to = lds + stage;
+    constexpr int HALF = K_LOADS / 2;                    // a block's
+    // (as buffer loads: the compiler waits for everything under way where one of the others' kind is)
+    const auto rows_at = [](const bf16_t* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
+    const auto rs_ka = rows_at(ka), rs_kb = rows_at(kb), rs_va = rows_at(va), rs_vb = rows_at(vb);
+    unrolled_while<K_LOADS>([&](auto tag) __attribute__((always_inline)) {
+      constexpr int g = decltype(tag)::value;
+      constexpr unsigned flip = (unsigned)((((g * ROWS) >> 3) << 2) & (NP - 1)) << 4;      // of the load's first row, the same in every lane
+      // (what is constant is added to both addresses)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(g < HALF ? rs_ka : rs_kb, (__attribute__((address_space(3))) void*)(size_t)(to + (g / HALF) * HALF * 1024),
+                                               16, k_lane ^ flip, 0, (g % HALF) * 1024, 0);
+      return true;
+    });
+#pragma unroll
+    for (int g = 0; g < V_LOADS; ++g) {
+      const unsigned v_to = to + K_BYTES + g * 1024;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_va, (__attribute__((address_space(3))) void*)(size_t)v_to, 16, v_lane, g * 64 * kv.P, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_vb, (__attribute__((address_space(3))) void*)(size_t)(v_to + V_BYTES), 16, v_lane, g * 64 * kv.P, 0, 0);
+    }
+  }
+  // the operands of the pair in stage number S, in registers when this returns (they have landed in LDS before)
+  template <int S> __device__ __forceinline__ void read(KVPair<HD>& f) const {
+    constexpr int OFF = S * (int)BYTES;
+    v4u k[2][HD / 32], v[HD / 16];
+    if constexpr (HD == 128)
+      asm volatile("ds_read_b128 %0, %16 offset:%21\n\tds_read_b128 %1, %17 offset:%21\n\tds_read_b128 %2, %18 offset:%21\n\t"
+                   "ds_read_b128 %3, %19 offset:%21\n\tds_read_b128 %4, %16 offset:%21+1024\n\tds_read_b128 %5, %17 offset:%21+1024\n\t"
+                   "ds_read_b128 %6, %18 offset:%21+1024\n\tds_read_b128 %7, %19 offset:%21+1024\n\t"
+                   "ds_read_b128 %8, %20 offset:%21\n\tds_read_b128 %9, %20 offset:%21+512\n\tds_read_b128 %10, %20 offset:%21+1024\n\t"
+                   "ds_read_b128 %11, %20 offset:%21+1536\n\tds_read_b128 %12, %20 offset:%21+2048\n\tds_read_b128 %13, %20 offset:%21+2560\n\t"
+                   "ds_read_b128 %14, %20 offset:%21+3072\n\tds_read_b128 %15, %20 offset:%21+3584\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(k[0][0]), "=&v"(k[0][1]), "=&v"(k[0][2]), "=&v"(k[0][3]), "=&v"(k[1][0]), "=&v"(k[1][1]), "=&v"(k[1][2]),
+                     "=&v"(k[1][3]), "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7])
+                   : "v"(k_at[0]), "v"(k_at[1]), "v"(k_at[2]), "v"(k_at[3]), "v"(v_at), "n"(OFF)
+                   : "memory");
+    else
+      asm volatile("ds_read_b128 %0, %8 offset:%11\n\tds_read_b128 %1, %9 offset:%11\n\tds_read_b128 %2, %8 offset:%11+512\n\t"
+                   "ds_read_b128 %3, %9 offset:%11+512\n\tds_read_b128 %4, %10 offset:%11\n\tds_read_b128 %5, %10 offset:%11+512\n\t"
+                   "ds_read_b128 %6, %10 offset:%11+1024\n\tds_read_b128 %7, %10 offset:%11+1536\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(k[0][0]), "=&v"(k[0][1]), "=&v"(k[1][0]), "=&v"(k[1][1]), "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+                   : "v"(k_at[0]), "v"(k_at[1]), "v"(v_at), "n"(OFF)
+                   : "memory");
+#pragma unroll
+    for (int s = 0; s < HD / 32; ++s) {
+      f.k[0][s].v = __builtin_bit_cast(bf16x8, k[0][s]);
+      f.k[1][s].v = __builtin_bit_cast(bf16x8, k[1][s]);
+    }
+#pragma unroll
+    for (int d = 0; d < HD / 16; ++d) f.v[d].v = __builtin_bit_cast(bf16x8, v[d]);
+  }
+};
+
+// walk_blocks through ST stages (launches by records: the ids of the first four blocks are given, whatever the run's length).  The hooks
+// come as there, none of them may touch LDS but by instructions of its own (the compiler would wait for every load that is under way).
+// Behind the first pair nothing is asked for beyond the run's end.
+template <int HD, int ST, typename Check, typename AfterTable = NoHook, typename BeforeAttend = NoHook, typename AfterSecond = NoHook>
+__device__ __forceinline__ void walk_staged(const StagedPairs<HD>& st, const PagedKV& kv, const Frag8* qf, int first, int stride, int n,
+                                            int lo, int hi, int kv_last, float scale, Check check, float& m, float& l, floatx4* o,
+                                            AfterTable after_table, BeforeAttend before_attend, float cap2, int held, int held_id,
+                                            const int* first4, AfterSecond after_second) {
+  static_assert(ST == 1 || ST == 2, "a pair, or two");
+  const int lane = threadIdx.x & 63;
+  int c0 = 0, nc = min(64, n);               // the run of up to 64 blocks whose page ids the lanes hold, as in walk_blocks
+  int mine = -1;
+  auto ids = [&](int have) __attribute__((always_inline)) {
+    const auto table = (const __attribute__((address_space(1))) int*)kv.table;      // (in memory, here)
+    if (nc > have && lane >= have && lane < nc) mine = table[((first + (c0 + lane) * stride) * 16) / kv.P];
+  };
+  BlockInfo a[ST], b[ST];
+  // the loads of blocks j and j + 1 of the run, on pages pa and pb
+  auto issue = [&](int j, auto stage_tag, int pa, int pb) __attribute__((always_inline)) {
+    constexpr int S = decltype(stage_tag)::value;
+    const int blk_a = first + (c0 + j) * stride, blk_b = first + (c0 + min(j + 1, max(nc - 1, 0))) * stride;
+    a[S] = BlockInfo{blk_a * 16, j < nc && pa >= 0, check(blk_a)};
+    b[S] = BlockInfo{blk_b * 16, j + 1 < nc && pb >= 0, check(blk_b)};
+    st.ask(kv, max(pa, 0), a[S].key0, max(pb, 0), b[S].key0, S * StagedPairs<HD>::BYTES);
+  };
+  auto issue_held = [&](int j, auto stage_tag) __attribute__((always_inline)) {
+    issue(j, stage_tag, __builtin_amdgcn_readlane(mine, j), __builtin_amdgcn_readlane(mine, min(j + 1, nc - 1)));
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, ST - 1>;
+  ids(held);               // (those that the record does not hold)
+  __builtin_amdgcn_sched_barrier(0);
+  after_table();
+  __builtin_amdgcn_sched_barrier(0);
+  // (without a condition, whatever there is to walk: the compiler counts these loads where `before_attend` waits for what
+  // `after_table` asked for)
+  issue(0, S0{}, first4[0], first4[1]);
+  __builtin_amdgcn_sched_barrier(0);
+  before_attend();
+  __builtin_amdgcn_sched_barrier(0);
+  if (ST > 1 && nc > 2) issue(2, S1{}, first4[2], first4[3]);
+  __builtin_amdgcn_sched_barrier(0);
+  after_second();
+  if (lane < min(nc, held)) mine = held_id;
+  auto turn = [&](int i, auto stage_tag) __attribute__((always_inline)) {
+    constexpr int S = decltype(stage_tag)::value;
+    KVPair<HD> f;
+    if (ST > 1 && i + 2 < nc) wait_vmcnt<StagedPairs<HD>::LOADS>();
+    else wait_vmcnt<0>();
+    st.template read<S>(f);
+    const BlockInfo A = a[S], B = b[S];
+    if (i + 2 * ST < nc) issue_held(i + 2 * ST, stage_tag);
+    attend_pair<HD>(f, qf, A, B, lo, hi, kv_last, scale, m, l, o, cap2);
+  };
+  while (true) {
+    for (int i = 0; i < nc; i += 2 * ST) {
+      turn(i, S0{});
+      if (ST > 1 && i + 2 < nc) turn(i + 2, S1{});
+    }
+    c0 += 64;
+    if (c0 >= n) break;
+    nc = min(64, n - c0);
+    ids(0);
+    issue_held(0, S0{});
+    if (ST > 1 && nc > 2) issue_held(2, S1{});
+  }
+  wait_vmcnt<0>();      // (a wavefront without blocks: what it leaves in its stage comes after the loads)
 }
 
 // ------------------------------------------- queries and the new key prepared in place
@@ -324,8 +499,8 @@ struct HeadJob {
     from_table = pr.inv_freq && pr.rope_table && p < pr.table_len;   // the same in every lane
     if (from_table) cs = pr.rope_table[(size_t)p * HALF + i];
   }
-  // `dst`: HD consecutive elements
-  __device__ __forceinline__ void finish(const QKPrep& pr, const float* w, bool value, int p, bf16_t* dst) {
+  // the pair, finished
+  __device__ __forceinline__ void pair(const QKPrep& pr, const float* w, bool value, int p, bf16_t& first, bf16_t& second) {
     const int lane = threadIdx.x & 63;
     float a = lo, b = hi;
     if (!value) {
@@ -341,10 +516,28 @@ struct HeadJob {
         qk_rotate(a, b, cs);
       }
     }
+    first = f2bf(a);
+    second = f2bf(b);
+  }
+  // `dst`: HD consecutive elements
+  __device__ __forceinline__ void finish(const QKPrep& pr, const float* w, bool value, int p, bf16_t* dst) {
+    const int lane = threadIdx.x & 63;
+    bf16_t a, b;
+    pair(pr, w, value, p, a, b);
     if (lane < HALF) {
-      dst[lane] = f2bf(a);
-      dst[lane + HALF] = f2bf(b);
+      dst[lane] = a;
+      dst[lane + HALF] = b;
     }
+  }
+  // the same into LDS (its byte address) while direct loads into other parts of it are under way: written as an instruction, or the
+  // compiler would have it wait for them
+  __device__ __forceinline__ void finish_lds(const QKPrep& pr, const float* w, bool value, int p, unsigned dst) {
+    const int lane = threadIdx.x & 63;
+    bf16_t a, b;
+    pair(pr, w, value, p, a, b);
+    if (lane < HALF)
+      asm volatile("ds_write_b16 %0, %1\n\tds_write_b16 %0, %2 offset:%3" ::"v"(dst + lane * 2), "v"((unsigned)a), "v"((unsigned)b), "n"(HALF * 2)
+                   : "memory");
   }
 };
 
@@ -368,11 +561,21 @@ __device__ __forceinline__ float sink_join(const float* __restrict__ sink, int h
 }
 
 #define DEC_TABLE_LDS 1024     // entries of a block-table row that the decode kernel can hold in LDS
-// The workgroup's LDS: what its NW wavefronts leave for the merge, and their maxima and sums.
+// The workgroup's LDS: what its NW wavefronts leave for the merge (a column's HD values in a row), and their maxima and sums.
 template <int HD, int NW>
 struct DecodeMerge {
-  floatx4 o[NW][HD / 16][64];
-  float m[NW][16], l[NW][16];
+  float o[NW][16][HD];
+  float2 ml[NW][16];
+};
+// The same where the operands come through LDS stages: a wavefront leaves its outputs in its own first stage.
+template <int HD, int NW, int ST>
+struct StagedMerge {
+  union {
+    unsigned char stages[ST][StagedPairs<HD>::BYTES];
+    float o[16][HD];
+  } w[NW];
+  float2 ml[NW][16];
+  bf16_t q[16][HD], kv[2][HD];      // the query heads, the row's own key and value (16-byte aligned)
 };
 // A launch by records (TI_RUN_* in tinyinfer_kernels.h): the host cuts every row's context into runs of its own choice and says what each
 // workgroup walks.  Record i, of a launch's `run_stride` ints: the header below, then for each of the workgroup's
@@ -385,18 +588,29 @@ struct DecodeRuns {
   const int* runs;      // null: no records, `split` of n_splits equal runs of every row
   int run_stride;
 };
+// A kernel argument that is to have arrived here.  (Pointers as ones to memory: an asm statement makes others point to anything, and flat
+// loads wait for everything under way.)
+template <class T> __device__ __forceinline__ void arrived(T& v) { asm volatile("" : "+s"(v)); }
+template <class T> __device__ __forceinline__ void arrived(T*& p) {
+  auto g = (__attribute__((address_space(1))) T*)p;
+  asm volatile("" : "+s"(g));
+  p = (T*)g;
+}
 // One workgroup of NW wavefronts: row `ridx` of the launch, kv head and set of q heads `y`, run `split` of n_splits; or record `ridx`.
-template <int HD, bool PREP, int NW, bool RUNS>
+// ST: stages of LDS a wavefront takes its operands through, by records; 0: straight from memory, by equal runs
+template <int HD, bool PREP, int NW, int ST, class Shared>
 __device__ __forceinline__ void
-decode_run(DecodeMerge<HD, NW>& sm, int ridx, int y, int split, const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool,
+decode_run(Shared& sm, int ridx, int y, int split, const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool,
            const int* __restrict__ table, int table_stride, const int* __restrict__ pos, const int* __restrict__ slot,
            const int* __restrict__ rows, bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
-           int n_head, int n_kv, int P, float scale, int window, int n_splits, const QKPrep& prep, float softcap,
+           int n_head, int n_kv, int P, float scale, int window, int n_splits, QKPrep prep, float softcap,
            const float* __restrict__ sink, DecodeRuns by = DecodeRuns{nullptr, 0}, int group = 0) {
   static_assert(!PREP || NW == 4, "the preparation is written for four wavefronts");
-  auto& s_o = sm.o;
-  auto& s_m = sm.m;
-  auto& s_l = sm.l;
+  constexpr bool RUNS = ST > 0;
+  auto s_o = [&](int w) -> float(&)[16][HD] {
+    if constexpr (ST > 0) return sm.w[w].o;
+    else return sm.o[w];
+  };
   // the wavefront's number in scalar registers, and with it what it walks
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int held = RUNS ? (by.run_stride - TI_RUN_HEAD) / NW : 0;      // lanes whose first block's page id comes with the record
@@ -414,6 +628,11 @@ decode_run(DecodeMerge<HD, NW>& sm, int ridx, int y, int split, const bf16_t* __
     for (int i = 0; i < TI_RUN_HEAD; ++i) asm volatile("" : "+s"(rh[i]));      // all of it at once
 #pragma unroll
     for (int i = 0; i < 4; ++i) asm volatile("" : "+s"(first4[i]));
+    // so do the arguments that did not come with the wavefront: fetched where they are first needed they are round trips one behind another
+    if constexpr (PREP) {
+      arrived(prep.q_w), arrived(prep.k_w), arrived(table), arrived(table_stride), arrived(window), arrived(prep.inv_freq);
+      arrived(prep.pool_w), arrived(prep.eps), arrived(scale), arrived(out), arrived(part_o), arrived(part_ml);
+    }
     if (rh[TI_RUN_BLOCKS] == 0) return;
   }
   const int m_row = RUNS ? rh[TI_RUN_ROW] : rows ? rows[ridx] : ridx;
@@ -469,14 +688,13 @@ decode_run(DecodeMerge<HD, NW>& sm, int ridx, int y, int split, const bf16_t* __
   for (int d = 0; d < HD / 16; ++d) o[d] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int mine = (b1 - (b0 + wave) + NW - 1) / NW;   // blocks b0 + wave, + NW, ... below b1
   auto edge = [=](int b) { return (lo > 0 && b == blk_lo) || b == blk_hi; };
+  bool own_key = false;
   if constexpr (PREP) {
-    __shared__ __attribute__((aligned(16))) bf16_t s_q[16][HD];       // the query heads
-    __shared__ __attribute__((aligned(16))) bf16_t s_kv[2][HD];       // the row's own key, then its value
     const float* row = prep.qkv + (size_t)m_row * prep.row_width;
     // The workgroup that walks the block of the row's own position prepares the position's key and value as well: from LDS
     // they go into the cache for later steps, and into this step's attention as a block of their own, so nothing waits for
     // the cache to hold them.
-    const bool own_key = prep.pool_w && blk_hi >= b0 && blk_hi < b1;
+    own_key = prep.pool_w && blk_hi >= b0 && blk_hi < b1;
     const int last = own_key ? p_q - 1 : p_q;      // what the cache holds for this workgroup
     const int n_jobs = n_cols + (own_key ? 2 : 0);
     HeadJob<HD> job;
@@ -484,54 +702,125 @@ decode_run(DecodeMerge<HD, NW>& sm, int ridx, int y, int split, const bf16_t* __
       const int h = j < n_cols ? kvh * G + j : j == n_cols ? n_head + kvh : n_head + n_kv + kvh;
       job.load(prep, row + (size_t)h * HD, j < n_cols ? prep.q_w : j == n_cols ? prep.k_w : nullptr, p_q);
     };
-    auto job_finish = [&](int j) {
-      job.finish(prep, j < n_cols ? prep.q_w : prep.k_w, j > n_cols, p_q, j < n_cols ? s_q[j] : s_kv[j - n_cols]);
-    };
-    walk_blocks<HD, RUNS>(
-        kv, qf, b0 + wave, NW, mine, lo, last, last, scale * TI_LOG2E, edge, mx, l, o,
-        [&]() {
-          if (wave < n_jobs) job_load(wave);
-        },
-        [&]() {
-          for (int j = wave; j < n_jobs; j += NW) {
-            if (j != wave) job_load(j);
-            job_finish(j);
-          }
-          __syncthreads();
+    if constexpr (ST > 0) {
+      const unsigned q_lds = (unsigned)(size_t)&sm.q[0][0], kv_lds = (unsigned)(size_t)&sm.kv[0][0];
+      auto finish = [&](int j) {
+        job.finish_lds(prep, j < n_cols ? prep.q_w : prep.k_w, j > n_cols, p_q,
+                       j < n_cols ? q_lds + j * (HD * 2) : kv_lds + (j - n_cols) * (HD * 2));
+      };
+      // HD / 32 operands of 16 bytes, 64 bytes apart
+      auto operands = [&](unsigned at, Frag8* f) {
+        v4u e[HD / 32];
+        if constexpr (HD == 128)
+          asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:64\n\tds_read_b128 %2, %4 offset:128\n\t"
+                       "ds_read_b128 %3, %4 offset:192\n\ts_waitcnt lgkmcnt(0)"
+                       : "=&v"(e[0]), "=&v"(e[1]), "=&v"(e[2]), "=&v"(e[3]) : "v"(at) : "memory");
+        else
+          asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:64\n\ts_waitcnt lgkmcnt(0)"
+                       : "=&v"(e[0]), "=&v"(e[1]) : "v"(at) : "memory");
 #pragma unroll
-          for (int s = 0; s < HD / 32; ++s)
-            qf[s].u = r16 < n_cols ? *reinterpret_cast<const uint4*>(&s_q[r16][s * 32 + quad * 8]) : make_uint4(0, 0, 0, 0);
-        },
-        0.f, held, held_id, first4,
-        [&]() {
-          if (!own_key) return;
-          if (wave == 0) {
+        for (int s = 0; s < HD / 32; ++s) f[s].v = __builtin_bit_cast(bf16x8, e[s]);
+      };
+      const StagedPairs<HD> st((unsigned)(size_t)&sm.w[wave], P);
+      walk_staged<HD, ST>(
+          st, kv, qf, b0 + wave, NW, mine, lo, last, last, scale * TI_LOG2E, edge, mx, l, o,
+          [&]() {
+            if (wave < n_jobs) job_load(wave);
+          },
+          [&]() {
+            for (int j = wave; j < n_jobs; j += NW) {
+              if (j != wave) job_load(j);
+              finish(j);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            operands(q_lds + min(r16, n_cols - 1) * (HD * 2) + quad * 16, qf);
+#pragma unroll
+            for (int s = 0; s < HD / 32; ++s)
+              if (r16 >= n_cols) qf[s].u = make_uint4(0, 0, 0, 0);
+          },
+          0.f, held, held_id, first4,
+          [&]() {
+            if (!own_key || wave != 0) return;
             // the row's own key and value come first: their score is the maximum, their weight 1
             floatx4 sc = {0.f, 0.f, 0.f, 0.f};
+            Frag8 k[HD / 32];
+            operands(kv_lds + quad * 16, k);
 #pragma unroll
             for (int s = 0; s < HD / 32; ++s) {
-              Frag8 k;
-              k.u = (r16 == 0) ? *reinterpret_cast<const uint4*>(&s_kv[0][s * 32 + quad * 8]) : make_uint4(0, 0, 0, 0);
-              sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k.v, qf[s].v, sc, 0, 0, 0);
+              if (r16 != 0) k[s].u = make_uint4(0, 0, 0, 0);
+              sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[s].v, qf[s].v, sc, 0, 0, 0);
             }
             mx = __shfl(sc[0], r16, 64) * (scale * TI_LOG2E);      // row 0 of the tile lies in the first sixteen lanes
             l = quad == 0 ? 1.f : 0.f;                             // the lanes of a column are added at the end
+            // dims 16 d + 4 quad .. + 3, eight bytes of every 32
+            typedef unsigned v2u __attribute__((ext_vector_type(2)));
+            v2u e[HD / 16];
+            const unsigned at = kv_lds + HD * 2 + quad * 8;
+            asm volatile("ds_read_b64 %0, %4\n\tds_read_b64 %1, %4 offset:32\n\tds_read_b64 %2, %4 offset:64\n\t"
+                         "ds_read_b64 %3, %4 offset:96\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(e[0]), "=&v"(e[1]), "=&v"(e[2]), "=&v"(e[3]) : "v"(at) : "memory");
+            if constexpr (HD == 128)
+              asm volatile("ds_read_b64 %0, %4 offset:128\n\tds_read_b64 %1, %4 offset:160\n\tds_read_b64 %2, %4 offset:192\n\t"
+                           "ds_read_b64 %3, %4 offset:224\n\ts_waitcnt lgkmcnt(0)"
+                           : "=&v"(e[HD / 16 - 4]), "=&v"(e[HD / 16 - 3]), "=&v"(e[HD / 16 - 2]), "=&v"(e[HD / 16 - 1]) : "v"(at) : "memory");
 #pragma unroll
             for (int d = 0; d < HD / 16; ++d)
 #pragma unroll
-              for (int i = 0; i < 4; ++i) o[d][i] = bf2f(s_kv[1][d * 16 + quad * 4 + i]);
-          } else if (wave == NW - 1) {
-            const int page = RUNS ? rh[TI_RUN_OWN_PAGE] : kv.table[p_q / P];
-            if (page >= 0) {    // the host reserves pages first; never write astray
-              bf16_t* kd = kv_page_slot<bf16_t>(prep.pool_w, page, 0, kvh, p_q % P, n_kv, P, HD);
-              bf16_t* vd = kv_page_slot<bf16_t>(prep.pool_w, page, 1, kvh, p_q % P, n_kv, P, HD);
-              for (int i = lane; i < HD; i += 64) {
-                kd[i] = s_kv[0][i];
-                vd[(size_t)i * P] = s_kv[1][i];
+              for (int i = 0; i < 4; ++i) o[d][i] = __uint_as_float((i & 1) ? e[d][i >> 1] & 0xffff0000u : e[d][i >> 1] << 16);
+          });
+    } else {
+      __shared__ __attribute__((aligned(16))) bf16_t s_q[16][HD];       // the query heads
+      __shared__ __attribute__((aligned(16))) bf16_t s_kv[2][HD];       // the row's own key, then its value
+      auto job_finish = [&](int j) {
+        job.finish(prep, j < n_cols ? prep.q_w : prep.k_w, j > n_cols, p_q, j < n_cols ? s_q[j] : s_kv[j - n_cols]);
+      };
+      walk_blocks<HD>(
+          kv, qf, b0 + wave, NW, mine, lo, last, last, scale * TI_LOG2E, edge, mx, l, o,
+          [&]() {
+            if (wave < n_jobs) job_load(wave);
+          },
+          [&]() {
+            for (int j = wave; j < n_jobs; j += NW) {
+              if (j != wave) job_load(j);
+              job_finish(j);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < HD / 32; ++s)
+              qf[s].u = r16 < n_cols ? *reinterpret_cast<const uint4*>(&s_q[r16][s * 32 + quad * 8]) : make_uint4(0, 0, 0, 0);
+          },
+          0.f,
+          [&]() {
+            if (!own_key) return;
+            if (wave == 0) {
+              // the row's own key and value come first: their score is the maximum, their weight 1
+              floatx4 sc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+              for (int s = 0; s < HD / 32; ++s) {
+                Frag8 k;
+                k.u = (r16 == 0) ? *reinterpret_cast<const uint4*>(&s_kv[0][s * 32 + quad * 8]) : make_uint4(0, 0, 0, 0);
+                sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k.v, qf[s].v, sc, 0, 0, 0);
+              }
+              mx = __shfl(sc[0], r16, 64) * (scale * TI_LOG2E);      // row 0 of the tile lies in the first sixteen lanes
+              l = quad == 0 ? 1.f : 0.f;                             // the lanes of a column are added at the end
+#pragma unroll
+              for (int d = 0; d < HD / 16; ++d)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[d][i] = bf2f(s_kv[1][d * 16 + quad * 4 + i]);
+            } else if (wave == NW - 1) {
+              const int page = kv.table[p_q / P];
+              if (page >= 0) {    // the host reserves pages first; never write astray
+                bf16_t* kd = kv_page_slot<bf16_t>(prep.pool_w, page, 0, kvh, p_q % P, n_kv, P, HD);
+                bf16_t* vd = kv_page_slot<bf16_t>(prep.pool_w, page, 1, kvh, p_q % P, n_kv, P, HD);
+                for (int i = lane; i < HD; i += 64) {
+                  kd[i] = s_kv[0][i];
+                  vd[(size_t)i * P] = s_kv[1][i];
+                }
               }
             }
-          }
-        });
+          });
+    }
   } else {
 #pragma unroll
     for (int s = 0; s < HD / 32; ++s) {
@@ -539,56 +828,72 @@ decode_run(DecodeMerge<HD, NW>& sm, int ridx, int y, int split, const bf16_t* __
       if (r16 < n_cols)
         qf[s].u = *reinterpret_cast<const uint4*>(q + ((size_t)m_row * n_head + head) * HD + s * 32 + quad * 8);
     }
-    walk_blocks<HD, RUNS>(kv, qf, b0 + wave, NW, mine, lo, p_q, p_q, scale * TI_LOG2E, edge, mx, l, o, NoHook{}, NoHook{},
-                          softcap * TI_LOG2E, held, held_id, first4);
+    if constexpr (ST > 0)
+      walk_staged<HD, ST>(StagedPairs<HD>((unsigned)(size_t)&sm.w[wave], P), kv, qf, b0 + wave, NW, mine, lo, p_q, p_q,
+                          scale * TI_LOG2E, edge, mx, l, o, NoHook{}, NoHook{}, softcap * TI_LOG2E, held, held_id, first4, NoHook{});
+    else
+      walk_blocks<HD>(kv, qf, b0 + wave, NW, mine, lo, p_q, p_q, scale * TI_LOG2E, edge, mx, l, o, NoHook{}, NoHook{},
+                      softcap * TI_LOG2E);
   }
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  {
+    const LanePair p = lane_pair<16>(l);
+    l = p.a + p.b;
+  }
+  {
+    const LanePair p = lane_pair<32>(l);
+    l = p.a + p.b;
+  }
 
-  // merge the wavefronts: lane keeps its (column, dims) in all of them
+  // merge the wavefronts: what the columns in use hold, four values of a column a thread.  (A wavefront's dims of all sixteen columns,
+  // eight of its lanes at work, took 0.95 us from the barrier to the end where this takes 0.45.)
+  if (r16 < n_cols) {
 #pragma unroll
-  for (int d = 0; d < HD / 16; ++d) s_o[wave][d][lane] = o[d];
-  if (quad == 0) {
-    s_m[wave][r16] = mx;
-    s_l[wave][r16] = l;
+    for (int d = 0; d < HD / 16; ++d) *reinterpret_cast<floatx4*>(&s_o(wave)[r16][d * 16 + quad * 4]) = o[d];
+    if (quad == 0) sm.ml[wave][r16] = make_float2(mx, l);
   }
   __syncthreads();
-  float mm = -INFINITY;
+  for (int i = threadIdx.x; i < n_cols * (HD / 4); i += 64 * NW) {
+    const int col = i / (HD / 4), dim = i % (HD / 4) * 4, at = kvh * G + part * 16 + col;
+    floatx4 v[NW];
+    float2 ml[NW];
 #pragma unroll
-  for (int w = 0; w < NW; ++w) mm = fmaxf(mm, s_m[w][r16]);
-  float wgt[NW], lt = 0.f;
+    for (int w = 0; w < NW; ++w) {
+      ml[w] = sm.ml[w][col];
+      v[w] = *reinterpret_cast<const floatx4*>(&s_o(w)[col][dim]);
+    }
+    float mm = -INFINITY, lt = 0.f;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) {
-    wgt[w] = (s_m[w][r16] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(s_m[w][r16] - mm);
-    lt += s_l[w][r16] * wgt[w];
-  }
-  if (r16 >= n_cols) return;
-  // wavefront w finishes dim blocks w, w + NW, ...
-  for (int d = wave; d < HD / 16; d += NW) {
+    for (int w = 0; w < NW; ++w) mm = fmaxf(mm, ml[w].x);
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const floatx4 v = s_o[w][d][lane];
+      const float wgt = (ml[w].x == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(ml[w].x - mm);
+      lt += ml[w].y * wgt;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] += v[i] * wgt[w];
+      for (int e = 0; e < 4; ++e) acc[e] += v[w][e] * wgt;
     }
-    const int dim = d * 16 + quad * 4;
     if (whole) {
       float den = lt;
-      const float inv = sink_join(sink, head, mm, den) / den;
-      Frag4 r;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) r.h[i] = f2bf(acc[i] * inv);
-      *reinterpret_cast<uint2*>(out + ((size_t)m_row * n_head + head) * HD + dim) = r.u;
+      const float inv = sink_join(sink, at, mm, den) / den;
+      *reinterpret_cast<uint2*>(out + ((size_t)m_row * n_head + at) * HD + dim) =
+          make_uint2(pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv));
     } else {
-      float* po = part_o + (part_at + (size_t)part_step * head) * HD + dim;
-      *reinterpret_cast<float4*>(po) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+      const size_t place = part_at + (size_t)part_step * at;
+      *reinterpret_cast<float4*>(part_o + place * HD + dim) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+      if (dim == 0) reinterpret_cast<float2*>(part_ml)[place] = make_float2(mm, lt);
     }
   }
-  if (!whole && wave == 0 && quad == 0) {
-    float* pm = part_ml + (part_at + (size_t)part_step * head) * 2;
-    pm[0] = mm;
-    pm[1] = lt;
+  // the row's own key and value, for later steps: nobody waits for these stores
+  if constexpr (PREP && ST > 0) {
+    if (own_key && wave == NW - 1 && rh[TI_RUN_OWN_PAGE] >= 0) {    // the host reserves pages first; never write astray
+      const int page = rh[TI_RUN_OWN_PAGE];
+      bf16_t* kd = kv_page_slot<bf16_t>(prep.pool_w, page, 0, kvh, p_q % P, n_kv, P, HD);
+      bf16_t* vd = kv_page_slot<bf16_t>(prep.pool_w, page, 1, kvh, p_q % P, n_kv, P, HD);
+      for (int i = lane; i < HD; i += 64) {
+        kd[i] = sm.kv[0][i];
+        vd[(size_t)i * P] = sm.kv[1][i];
+      }
+    }
   }
 }
 
@@ -600,24 +905,23 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool
                    float* __restrict__ part_ml, int n_head, int n_kv, int P, float scale, int window,
                    int n_splits, QKPrep prep, float softcap = 0.f, const float* __restrict__ sink = nullptr) {
   __shared__ DecodeMerge<HD, 4> sm;
-  decode_run<HD, PREP, 4, false>(sm, blockIdx.x, blockIdx.y, blockIdx.z, q, pool, table, table_stride, pos, slot, rows,
+  decode_run<HD, PREP, 4, 0>(sm, blockIdx.x, blockIdx.y, blockIdx.z, q, pool, table, table_stride, pos, slot, rows,
                                          out, part_o, part_ml, n_head, n_kv, P, scale, window, n_splits, prep, softcap, sink);
 }
 
 // The same from the projections, by records: grid (n_kv, records).  A launch's workgroups differ by what the host gave them:
 // with every row in as many runs a launch lasted as long as the longest row asks.
 // (The arguments that the first loads need come first: they arrive in scalar registers with the wavefront.)
-template <int HD>
+template <int HD, int ST>
 __global__ void __launch_bounds__(256, 2)
 attn_decode_runs_kernel(const int* __restrict__ runs, int run_stride, int group, const float* __restrict__ qkv, int row_width,
-                        int n_kv, const float* __restrict__ q_w, const float* __restrict__ k_w,
-                        const float2* __restrict__ rope_table, const bf16_t* __restrict__ pool, const int* __restrict__ table,
-                        int table_stride, int P, const float* __restrict__ inv_freq, int table_len, float eps,
-                        bf16_t* __restrict__ pool_w, bf16_t* __restrict__ out, float* __restrict__ part_o,
-                        float* __restrict__ part_ml, float scale, int window) {
-  __shared__ DecodeMerge<HD, 4> sm;
+                        int n_kv, const float2* __restrict__ rope_table, const bf16_t* __restrict__ pool, int P, int table_len,
+                        const float* __restrict__ q_w, const float* __restrict__ k_w, const int* __restrict__ table,
+                        int table_stride, int window, const float* __restrict__ inv_freq, bf16_t* __restrict__ pool_w, float eps, float scale,
+                        bf16_t* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const QKPrep prep{qkv, row_width, q_w, k_w, eps, inv_freq, rope_table, table_len, pool_w};
-  decode_run<HD, true, 4, true>(sm, blockIdx.y, blockIdx.x, 0, nullptr, pool, table, table_stride, nullptr, nullptr, nullptr,
+  decode_run<HD, true, 4, ST>(*reinterpret_cast<StagedMerge<HD, 4, ST>*>(smem), blockIdx.y, blockIdx.x, 0, nullptr, pool, table, table_stride, nullptr, nullptr, nullptr,
                                 out, part_o, part_ml, group * n_kv, n_kv, P, scale, window, 1, prep, 0.f, nullptr,
                                 DecodeRuns{runs, run_stride}, group);
 }
@@ -800,7 +1104,6 @@ attn_prefill_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ poo
 #define PF_KEYS 32
 #define PF_STAGES 4      // LDS stages: PF_STAGES - 1 turns are in flight while one is computed
 
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float floatx16;
 
 __device__ __forceinline__ void lgkm_wait(int n) {
@@ -829,16 +1132,6 @@ __device__ __forceinline__ void vm_wait_turns(int k) {
     default: TI_VM(0); break;
   }
 #undef TI_VM
-}
-
-// f(integral_constant<int, 0>), f(<1>), ... f(<N - 1>), until one returns false
-template <typename F, int... Is>
-__device__ __forceinline__ void unrolled_while_impl(F&& f, std::integer_sequence<int, Is...>) {
-  (void)(f(std::integral_constant<int, Is>{}) && ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void unrolled_while(F&& f) {
-  unrolled_while_impl(f, std::make_integer_sequence<int, N>{});
 }
 
 // NG groups of NW wavefronts in the workgroup.  A tile is 32 NW rows: a column block of 32
@@ -1368,7 +1661,7 @@ attn_step_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool, 
                                          n_tiles, entries, out, n_head, n_kv, P, scale, window, nullptr, nullptr, softcap, sink);
   } else {
     const int at = id - n_pre, ways = n_kv * ((group + 15) / 16);
-    decode_run<HD, false, 8, true>(*reinterpret_cast<DecodeMerge<HD, 8>*>(smem), at / ways, at % ways, 0, q, pool, table,
+    decode_run<HD, false, 8, 1>(*reinterpret_cast<StagedMerge<HD, 8, 1>*>(smem), at / ways, at % ways, 0, q, pool, table,
                                           table_stride, nullptr, nullptr, nullptr, out, part_o, part_ml, n_head, n_kv, P, scale,
                                           window, 1, QKPrep{}, softcap, sink, DecodeRuns{runs, run_stride}, group);
   }
@@ -1502,6 +1795,7 @@ extern "C" int ti_attention_decode_prepared_bf16(const float* qkv, int row_width
 
 static int g_prefill_groups = 0;   // for measurements: 1 or 2 wavefront groups per workgroup, 0 = by the launch
 static int g_prefill_lds = 1;
+static int g_decode_stages = 0;    // LDS stages a wavefront of the decode kernel by records at a head size of 128, 0 = by the launch
 // 1: head sizes 64 and 128 take the kernel that shares keys and values through LDS
 // (default); 0: every head size takes the kernel that reads them per wavefront
 
@@ -1652,13 +1946,24 @@ extern "C" int ti_attention_decode_runs_bf16(const float* qkv, int row_width, co
   TI_REQUIRE(inv_freq || !rope_table, "attention_decode_runs: a sin/cos table without inv_freq");
   rc = check_runs("attention_decode_runs", runs, n_runs, run_stride, rows, n_rows, part_o, part_ml);
   if (rc) return rc;
-#define TI_GO(H)                                                                                                          \
-  attn_decode_runs_kernel<H><<<dim3(n_kv, n_runs), 256, 0, stream>>>(                                                     \
-      runs, run_stride, n_head / n_kv, qkv, row_width, n_kv, q_w, k_w, (const float2*)rope_table, (const bf16_t*)pool, table, \
-      table_stride, page_size, inv_freq, table_len, eps, write_kv ? (bf16_t*)pool : nullptr, (bf16_t*)out, part_o, part_ml,   \
-      scale, window)
-  if (hd == 128) TI_GO(128);
-  else TI_GO(64);
+  static bool ready = false;          // allow more than 64 KiB of dynamic LDS, once
+  if (!ready) {
+    if (hipFuncSetAttribute((const void*)attn_decode_runs_kernel<128, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(StagedMerge<128, 4, 1>)) != hipSuccess ||
+        hipFuncSetAttribute((const void*)attn_decode_runs_kernel<128, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(StagedMerge<128, 4, 2>)) != hipSuccess ||
+        hipFuncSetAttribute((const void*)attn_decode_runs_kernel<64, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(StagedMerge<64, 4, 2>)) != hipSuccess) {
+      ti_set_error("attention_decode_runs: cannot reserve the LDS");
+      return 2;
+    }
+    ready = true;
+  }
+#define TI_GO(H, S)                                                                                                          \
+  attn_decode_runs_kernel<H, S><<<dim3(n_kv, n_runs), 256, sizeof(StagedMerge<H, 4, S>), stream>>>(                                                     \
+      runs, run_stride, n_head / n_kv, qkv, row_width, n_kv, (const float2*)rope_table, (const bf16_t*)pool, page_size, table_len, \
+      q_w, k_w, table, table_stride, window, inv_freq, write_kv ? (bf16_t*)pool : nullptr, eps, scale, (bf16_t*)out, part_o, part_ml)
+  if (hd == 64) TI_GO(64, 2);
+  // two stages (136 KiB) where a unit has one workgroup at most; one (70 KiB) where two share it, so that one walks while the other starts
+  else if (g_decode_stages ? g_decode_stages == 2 : n_kv * n_runs <= compute_units()) TI_GO(128, 2);
+  else TI_GO(128, 1);
 #undef TI_GO
   if (n_rows) {
     if (hd == 128) attn_merge_kernel<128, true><<<dim3(n_rows, n_head), 128, 0, stream>>>(part_o, part_ml, rows, (bf16_t*)out, n_head, 0, nullptr);
@@ -1686,12 +1991,13 @@ extern "C" int ti_attention_step_bf16(const void* q, const void* pool, const int
   const int parts = (n_head / n_kv + 15) / 16;
   const long grid = (long)n_tiles * n_head + (long)n_runs * n_kv * parts;
   TI_REQUIRE(grid <= 0x7fffffL, "attention_step: too many workgroups");
-  constexpr int STAGES = 4 * 2 * 2 * PF_KEYS * 2;      // bytes of the tiles' stages per head dimension
-  static_assert(sizeof(DecodeMerge<128, 8>) <= STAGES * 128 && sizeof(DecodeMerge<64, 8>) <= STAGES * 64, "the merge fits the stages");
+  // the runs' LDS is the larger: the same stages, and the merge's maxima and sums
+  static_assert(sizeof(StagedMerge<128, 8, 1>) >= 4 * 2 * 2 * PF_KEYS * 2 * 128 && sizeof(StagedMerge<64, 8, 1>) >= 4 * 2 * 2 * PF_KEYS * 2 * 64,
+                "the tiles' stages fit");
   static bool ready = false;          // allow more than 64 KiB of dynamic LDS, once
   if (!ready) {
-    if (hipFuncSetAttribute((const void*)attn_step_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, STAGES * 128) != hipSuccess ||
-        hipFuncSetAttribute((const void*)attn_step_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize, STAGES * 64) != hipSuccess) {
+    if (hipFuncSetAttribute((const void*)attn_step_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(StagedMerge<128, 8, 1>)) != hipSuccess ||
+        hipFuncSetAttribute((const void*)attn_step_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(StagedMerge<64, 8, 1>)) != hipSuccess) {
       ti_set_error("attention_step: cannot reserve the LDS");
       return 2;
     }
@@ -1700,7 +2006,7 @@ extern "C" int ti_attention_step_bf16(const void* q, const void* pool, const int
   const float cap = softcap > 0.f ? softcap : 0.f;
 #define TI_GO(H)                                                                                                              \
   do {                                                                                                                        \
-    attn_step_kernel<H><<<(unsigned)grid, 512, STAGES * H, stream>>>((const bf16_t*)q, (const bf16_t*)pool, table, table_stride, \
+    attn_step_kernel<H><<<(unsigned)grid, 512, sizeof(StagedMerge<H, 8, 1>), stream>>>((const bf16_t*)q, (const bf16_t*)pool, table, table_stride, \
                                                                      tiles, n_tiles, entries, runs, run_stride, n_head / n_kv,  \
                                                                      (bf16_t*)out, part_o, part_ml,                              \
                                                                      n_head, n_kv, page_size, scale, window, cap, g_sink);       \
@@ -1752,11 +2058,13 @@ extern "C" int ti_attention_prefill_paired_capped_bf16(const void* q, const void
 extern "C" void ti_tuning_reset() {
   g_prefill_groups = 0;
   g_prefill_lds = 1;
+  g_decode_stages = 0;
 }
 extern "C" int ti_tuning_set(const char* name, long value) {
   const std::string n = name ? name : "";
   if (n == "prefill_groups") g_prefill_groups = (int)value;
   else if (n == "prefill_use_lds") g_prefill_lds = (int)value;
+  else if (n == "decode_stages") g_decode_stages = (int)value;
   else return 1;
   return 0;
 }

@@ -34,6 +34,7 @@
 // libti_attention_bf16:
 //   prefill_groups       1 or 2 groups of wavefronts per workgroup, 0: by the launch
 //   prefill_use_lds      0: the kernel without LDS for every head size
+//   decode_stages        1 or 2 LDS stages a wavefront in the decode kernel by records (head size 128), 0: by the launch
 #pragma once
 #ifdef __cplusplus
 extern "C" {
