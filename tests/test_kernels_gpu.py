@@ -1612,6 +1612,14 @@ def test_linear_with_the_norm_inside(ops, M, N, K):
             assert (f64(one) - ref).abs().max() < 2e-5 * K + 0.01 * ref.abs().max()
 
 
+@pytest.mark.parametrize("M,N,K", [(16, 4096, 1088), (7, 4100, 2112), (3, 8208, 320), (5, 8200, 2048), (16, 8200, 2048), (2, 12300, 64), (9, 6160, 3136),
+                                   (1, 4112, 128), (4, 6144, 4096)])
+def test_linear_with_the_norm_inside_by_groups(ops, M, N, K):
+    """One to three groups of wavefronts a workgroup, a group beyond the last tile, rows of no whole 256 columns, more rows than a workgroup
+    has wavefronts, more and fewer chunks of K than stages and than wavefronts: the bits of norm and product."""
+    test_linear_with_the_norm_inside(ops, M, N, K)
+
+
 def test_linear_with_the_norm_inside_refuses_what_it_does_not_serve(ops):
     """More rows than the kernel holds, a K that is no multiple of 64, or few tokens with a weight
     of few rows (which another kernel takes): `linear` computes the norm first and the result

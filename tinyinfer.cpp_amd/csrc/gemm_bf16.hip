@@ -210,79 +210,9 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
 #endif
 }
 
-// ================================== skinny kernel whose token rows are made in the kernel
-// out = rows W^T for M <= 16 tokens, where the rows do not exist in memory yet: a producer
-// makes them, as bfloat16 in LDS, in every workgroup for itself.  The rows are few and what
-// they are made from lies in the cache; the first weight loads are already under way while
-// the producer runs; and it costs no launch of its own.  The rounding to bfloat16 is the
-// one every product operand gets, so the result equals that of the producer's own kernel
-// followed by the plain product.
-//
+// ================================== skinny kernel with the token rows in LDS
 // A producer has `template <int NW> __device__ void fill(bf16_t* sA, int lda, int M, int K)`,
 // called by all NW * 64 threads, writing sA[m * lda + k]; the kernel synchronizes after it.
-
-// RMSNorm of float rows X [M, K] with weight Gw [K].  KC: float4 pieces of a row each lane
-// holds (K <= 256 KC).  Wavefront w takes rows w, w + NW, ...; two rows' loads are issued
-// together where the registers allow; a lane's pieces beyond K read piece 0 and are left
-// out of the sum and the store.
-template <int KC>
-struct NormProducer {
-  const float* X;
-  const float* Gw;
-  float eps;
-  template <int NW, class IssueWeights>
-  __device__ __forceinline__ void fill(bf16_t* sA, int lda, int M, int K, IssueWeights issue_weights) const {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    constexpr int RB = KC <= 8 ? 2 : 1;
-    float4 g[KC], v[RB][KC];
-    auto load_rows = [&](int r0) {
-#pragma unroll
-      for (int b = 0; b < RB; ++b) {
-        const int m = r0 + NW * b < M ? r0 + NW * b : (r0 < M ? r0 : 0);
-        const float* xr = X + (size_t)m * K;
-#pragma unroll
-        for (int c = 0; c < KC; ++c) {
-          const int k = lane * 4 + 256 * c;
-          v[b][c] = *reinterpret_cast<const float4*>(xr + (k < K ? k : 0));
-        }
-      }
-    };
-#pragma unroll
-    for (int c = 0; c < KC; ++c) {
-      const int k = lane * 4 + 256 * c;
-      g[c] = *reinterpret_cast<const float4*>(Gw + (k < K ? k : 0));
-    }
-    load_rows(wave);
-    // loads come back in the order they were issued: the rows (from the cache) before the
-    // weights (from memory), so the norm does not wait for the weights
-    __builtin_amdgcn_sched_barrier(0);
-    issue_weights();
-    __builtin_amdgcn_sched_barrier(0);
-    for (int r0 = wave; r0 < M; r0 += NW * RB) {
-      if (r0 != wave) load_rows(r0);
-#pragma unroll
-      for (int b = 0; b < RB; ++b) {
-        const int m = r0 + NW * b;
-        float ss = 0.f;
-#pragma unroll
-        for (int c = 0; c < KC; ++c)
-          if (lane * 4 + 256 * c < K) ss = rms_accumulate(ss, v[b][c]);
-        const float scale = rms_scale(ss, K, eps);
-        if (m < M) {
-#pragma unroll
-          for (int c = 0; c < KC; ++c) {
-            const int k = lane * 4 + 256 * c;
-            if (k < K) {
-              const uint2 hb = make_uint2(pack_bf16x2(v[b][c].x * scale * g[c].x, v[b][c].y * scale * g[c].y),
-                                          pack_bf16x2(v[b][c].z * scale * g[c].z, v[b][c].w * scale * g[c].w));
-              *reinterpret_cast<uint2*>(sA + (size_t)m * lda + k) = hb;
-            }
-          }
-        }
-      }
-    }
-  }
-};
 
 // Rows that do exist in memory (bfloat16 [M, K], row stride lda): copied into LDS once per
 // workgroup, 16 bytes per thread and load, instead of every wavefront fetching its token
@@ -422,6 +352,186 @@ gemm_skinny_staged_kernel(Producer producer, const bf16_t* __restrict__ W, void*
     if (EPI == TI_EPI_ADD_F32) ((float*)out_)[o] = prev + sum;
     if (TI_EPI_ACT(EPI)) ((bf16_t*)out_)[o] = f2bf(epi_act<EPI>(sum));
   }
+}
+
+// ================================== the norm inside the product
+// out (op)= rmsnorm(X; Gw, eps) W^T for M <= 16.  Every workgroup norms all rows for itself into LDS (bfloat16, the bits of the norm's own
+// kernel: lane l of a wavefront holds the float4 pieces l, l + 64, ... of a row) while its weights are on their way into LDS stages of each
+// wavefront's own (staged_rows.h).  G groups of KW wavefronts, a tile of 16 weight rows (SwiGLU: 8 gate and 8 up rows) each, so that a unit
+// norms the rows once for all tiles it has; KW wavefronts split K as the plain kernels do: the same bits as norm and product.
+// KC: float4 pieces of a row a lane holds (K <= 256 KC).  ST: chunks of 64 columns a wavefront has under way.
+// What bounds it: the chain of loads, norm and products of one launch, then the weights' bytes.  A load of 1 KiB keeps the unit that takes
+// addresses for 16 cycles (64 for weights as operands), so rows are asked for only by the wavefronts that norm them, and nothing waits for
+// more than it uses.  Weights as operands straight from memory, norm in front, in a chain of launches with weights from memory, us before
+// and now at 1, 8 and 16 rows: 4096 x 1024 4.0 4.0 5.2 -> 3.2 3.5 4.7, [gate; up] 6144 x 1024 5.6 5.9 7.3 -> 4.2 4.7 5.3, 4096 x 2048 7.5 7.6
+// 9.6 -> 5.3 6.7 8.2, [gate; up] 12288 x 2048 13.6 15.1 18.1 -> 11.7 12.8 16.6, 6144 x 2560 11.7 14.3 20.1 -> 7.4 9.3 11.3, 6144 x 4096
+// at 1 and 8 14.0 16.5 -> 11.3 16.0 (the plain product alone, at 1 row: 3.2, 4.4, 5.6, 10.9, 7.4, 11.3).
+template <int KC, int EPI, int KW, int G, int ST>
+__global__ void __launch_bounds__(64 * KW * G)
+gemm_normed_kernel(const float* __restrict__ X, const bf16_t* __restrict__ W, int M, int N, int K, float eps, const float* __restrict__ Gw,
+                   void* __restrict__ out_) {
+#if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass has no buffer descriptors)
+  constexpr bool SW = (EPI == TI_EPI_SWIGLU);
+  constexpr int NW = KW * G;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];      // the stages, then the rows [M][K + 8]
+  constexpr unsigned ROWS_AT = NW * ST * 2048;
+  static_assert(ST == 4 || ST == 8, "four chunks' operands at a time");
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int kw = wave % KW, group = wave / KW;
+  const int r = lane & 15, j = lane >> 4;
+  const int per = SW ? 8 : 16, tiles = (N + per - 1) / per;
+  const int tile = blockIdx.x * G + group, n0 = min(tile, tiles - 1) * per;      // (a group beyond the last works, and stores nothing)
+  const int chunks = K / 64, steps = (chunks - kw + KW - 1) / KW;
+
+  floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+  asm volatile("" : "+v"(acc));        // (in registers of its own from here: in some that loads went to it would wait for everything under way)
+  // the rows' and the norm's loads, then the weights': they come back in that order.  (As buffer loads whose descriptor ends with the row:
+  // one address for all pieces, and zeros beyond K.)
+  constexpr int RB = KC <= 8 ? 2 : 1;
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  v4f g[KC], v[RB][KC];
+  auto row_at = [&](const float* p) __attribute__((always_inline)) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, K * 4, 0x00020000); };
+  auto load_row = [&](const float* p, v4f (&to)[KC]) __attribute__((always_inline)) {
+    const auto rs = row_at(p);
+#pragma unroll
+    for (int c = 0; c < KC; ++c) to[c] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16 + c * 1024, 0, 0));
+  };
+  auto load_rows = [&](int r0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+      if (r0 + NW * b < M) load_row(X + (size_t)(r0 + NW * b) * K, v[b]);
+  };
+  // (only what is needed: a load of 1 KiB keeps the unit that takes addresses for 16 cycles, and twelve of every wavefront were 0.6 us)
+  if (wave < M) {
+    load_rows(wave);
+    load_row(Gw, g);
+  }
+  const int tok = (threadIdx.x % (64 * KW)) >> 4, row = threadIdx.x & 15;
+  const int n = (SW ? n0 + (row & 7) : n0 + row);
+  float prev = 0.f;
+  if (EPI == TI_EPI_ADD_F32) prev = ((const float*)out_)[(size_t)(tok < M ? tok : 0) * N + (n < N ? n : N - 1)];
+  __builtin_amdgcn_sched_barrier(0);
+  const int lr = lane >> 3, piece = ((lane & 7) ^ lr) * 16;
+  const unsigned v0 = (unsigned)min(lr, N - 1 - n0) * (unsigned)(K * 2) + piece;
+  const unsigned v1 = SW ? v0 : (unsigned)min(8 + lr, N - 1 - n0) * (unsigned)(K * 2) + piece;
+  const auto rows_at = [](const bf16_t* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
+  const auto rsW = rows_at(W + (size_t)n0 * K), rsU = rows_at(W + (size_t)(n0 + (SW ? N : 0)) * K);
+  unsigned char* mine = smem + wave * (ST * 2048);
+  auto load = [&](int step, unsigned stage) __attribute__((always_inline)) {
+    const int at = max(kw + KW * step, 0) * 128;         // (a wavefront without a chunk asks for the first)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsW, (__attribute__((address_space(3))) void*)(mine + stage), 16, v0, at, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsU, (__attribute__((address_space(3))) void*)(mine + stage + 1024), 16, v1, at, 0, 0);
+  };
+  // (without a condition, the last one again where there are fewer: the compiler counts these loads where the rows are waited for)
+#pragma unroll
+  for (int d = 0; d < ST; ++d) load(min(d, steps - 1), d * 2048);
+  __builtin_amdgcn_sched_barrier(0);
+
+  // the norm; written as instructions, or the compiler would have the writes wait for the weights
+  const unsigned rows_lds = (unsigned)(size_t)smem + ROWS_AT, row_bytes = (K + 8) * 2;
+  const bool full = K == 256 * KC;
+  auto norm_rows = [&](int r0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+      const int m = r0 + NW * b;
+      if (b > 0 && m >= M) continue;
+      float ss = 0.f;
+#pragma unroll
+      for (int c = 0; c < KC; ++c) ss = rms_accumulate(ss, make_float4(v[b][c].x, v[b][c].y, v[b][c].z, v[b][c].w));
+      const float scale = rms_scale(ss, K, eps);
+      if (m < M) {
+        const unsigned to = rows_lds + m * row_bytes + lane * 8;
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+          typedef unsigned v2u __attribute__((ext_vector_type(2)));
+          const v2u h = {pack_bf16x2(v[b][c].x * scale * g[c].x, v[b][c].y * scale * g[c].y),
+                         pack_bf16x2(v[b][c].z * scale * g[c].z, v[b][c].w * scale * g[c].w)};
+          if (full || lane * 4 + 256 * c < K) asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(to), "v"(h), "n"(c * 512) : "memory");
+        }
+      }
+    }
+  };
+  if (wave < M) norm_rows(wave);      // (not in the loop, where the compiler would wait for the weights too)
+#pragma clang loop unroll(disable)
+  for (int r0 = wave + NW * RB; r0 < M; r0 += NW * RB) {
+    load_rows(r0);
+    norm_rows(r0);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+
+  // ---- the product: chunks kw, kw + KW, ...
+  const unsigned a_at = rows_lds + (r < M ? r : 0) * row_bytes + j * 32 + kw * 128;
+  const unsigned w_x = (unsigned)(size_t)mine + r * 128 + (((2 * j) ^ (r & 7)) << 4);
+  const unsigned w_y = (unsigned)(size_t)mine + r * 128 + (((2 * j + 1) ^ (r & 7)) << 4);
+  unsigned stage = 0;
+  int i = 0;
+  auto multiply = [&](const RowPieces& w, const v4u& x, const v4u& y) __attribute__((always_inline)) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w.x), __builtin_bit_cast(bf16x8, x), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w.y), __builtin_bit_cast(bf16x8, y), acc, 0, 0, 0);
+  };
+  for (; i + ST < steps; ++i) {
+    wait_vmcnt<2 * (ST - 1)>();
+    RowPieces w, a;
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %6 offset:16\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(w.x), "=&v"(w.y), "=&v"(a.x), "=&v"(a.y) : "v"(w_x + stage), "v"(w_y + stage), "v"(a_at + i * (KW * 128)) : "memory");
+    load(i + ST, stage);
+    multiply(w, a.x, a.y);
+    stage = stage == (ST - 1) * 2048 ? 0 : stage + 2048;
+  }
+  // the last ST: the rows' operands first, which are there
+  v4u a[2 * ST];
+#pragma unroll
+  for (int u = 0; u < ST; u += 4) {
+    const unsigned a0 = a_at + min(i + u, max(steps - 1, 0)) * (KW * 128), a1 = a_at + min(i + u + 1, max(steps - 1, 0)) * (KW * 128),
+                   a2 = a_at + min(i + u + 2, max(steps - 1, 0)) * (KW * 128), a3 = a_at + min(i + u + 3, max(steps - 1, 0)) * (KW * 128);
+    asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:16\n\tds_read_b128 %2, %9\n\tds_read_b128 %3, %9 offset:16\n\t"
+                 "ds_read_b128 %4, %10\n\tds_read_b128 %5, %10 offset:16\n\tds_read_b128 %6, %11\n\tds_read_b128 %7, %11 offset:16\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(a[2 * u]), "=&v"(a[2 * u + 1]), "=&v"(a[2 * u + 2]), "=&v"(a[2 * u + 3]), "=&v"(a[2 * u + 4]), "=&v"(a[2 * u + 5]),
+                   "=&v"(a[2 * u + 6]), "=&v"(a[2 * u + 7])
+                 : "v"(a0), "v"(a1), "v"(a2), "v"(a3) : "memory");
+  }
+  auto last = [&](auto tag) __attribute__((always_inline)) {
+    constexpr int u = decltype(tag)::value;
+    if (i + u >= steps) return false;
+    wait_vmcnt<2 * (ST - 1 - u)>();
+    RowPieces w;
+    read_some_blocks<1>(&w, w_x + stage, w_y + stage);
+    multiply(w, a[2 * u], a[2 * u + 1]);
+    stage = stage == (ST - 1) * 2048 ? 0 : stage + 2048;
+    return true;
+  };
+  auto all = [&](auto... tags) __attribute__((always_inline)) { return (last(tags) && ...); };
+  using std::integral_constant;
+  if (all(integral_constant<int, 0>{}, integral_constant<int, 1>{}, integral_constant<int, 2>{}, integral_constant<int, 3>{}))
+    if constexpr (ST == 8)
+      (void)all(integral_constant<int, 4>{}, integral_constant<int, 5>{}, integral_constant<int, 6>{}, integral_constant<int, 7>{});
+  wait_vmcnt<0>();      // (stages filled and never read: the sums come after the loads)
+  // acc[i]: weight row 4 j + i, token r
+  auto red = [&](int w) -> float (*)[17] { return reinterpret_cast<float (*)[17]>(smem + w * (ST * 2048)); };
+#pragma unroll
+  for (int i = 0; i < 4; ++i) red(wave)[r][4 * j + i] = acc[i];
+  __syncthreads();
+  if (tok >= M || tile >= tiles || n >= N || (SW && row >= 8)) return;
+  if (SW) {
+    float gt = 0.f, up = 0.f;
+#pragma unroll
+    for (int w = 0; w < KW; ++w) {
+      gt += red(group * KW + w)[tok][row];
+      up += red(group * KW + w)[tok][row + 8];
+    }
+    ((bf16_t*)out_)[(size_t)tok * N + n] = f2bf(silu_mul(gt, up));
+  } else {
+    float sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < KW; ++w) sum += red(group * KW + w)[tok][row];
+    const size_t o = (size_t)tok * N + n;
+    if (EPI == TI_EPI_STORE_F32) ((float*)out_)[o] = sum;
+    if (EPI == TI_EPI_ADD_F32) ((float*)out_)[o] = prev + sum;
+    if (TI_EPI_ACT(EPI)) ((bf16_t*)out_)[o] = f2bf(epi_act<EPI>(sum));
+  }
+#endif
 }
 
 // ================================== few tokens, any K: the token rows in pieces, loads never at rest
@@ -1817,6 +1927,33 @@ static int skinny_waves_for(int grid, int K) {
   return g_skinny_waves ? g_skinny_waves : ((grid <= 128 && K >= 1024 && (long)grid * K < (512L << 10)) ? 8 : 4);
 }
 
+static size_t normed_lds(int M, int K, int waves, int stages) { return (size_t)waves * stages * 2048 + (size_t)M * (K + 8) * 2; }
+#define NORMED_LDS (160 << 10)
+template <int KC, int EPI, int KW, int G, int ST>
+static int launch_normed(const float* x, const float* nw, float eps, const bf16_t* w, void* out, int M, int N, int K, int tiles,
+                         hipStream_t stream) {
+  auto kernel = gemm_normed_kernel<KC, EPI, KW, G, ST>;
+  static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, NORMED_LDS);
+  TI_REQUIRE(room == hipSuccess, "gemm_bf16_normed: LDS size refused: %s", hipGetErrorString(room));
+  kernel<<<(tiles + G - 1) / G, 64 * KW * G, normed_lds(M, K, KW * G, ST), stream>>>(x, w, M, N, K, eps, nw, out);
+  TI_LAUNCH_CHECK();
+  return 0;
+}
+static int g_normed_groups = 0;    // a hook for measurements: 1 to 3 groups of wavefronts in the product with the norm inside, 0: by the tiles
+// Groups of four wavefronts: as many as a unit has tiles, three at most; with more two, whose workgroups share a unit.  A long K under two
+// tiles a unit has three as well, for 96 KiB of weights under way instead of 64 (6144 x 4096 at 1 and 4 rows 14.0 14.8 -> 11.3 12.0 us).
+template <int KC, int EPI>
+static int launch_normed_groups(const float* x, const float* nw, float eps, const bf16_t* w, void* out, int M, int N, int K, int tiles,
+                                hipStream_t stream) {
+  const int each = (tiles + compute_units() - 1) / compute_units();
+  int groups = g_normed_groups ? g_normed_groups : each <= 1 ? 1 : each == 3 || (each == 2 && K > 3072) ? 3 : 2;
+  if (groups == 3 && normed_lds(M, K, 12, 4) > NORMED_LDS) groups = 2;
+  if (groups == 3) return launch_normed<KC, EPI, 4, 3, 4>(x, nw, eps, w, out, M, N, K, tiles, stream);
+  if (groups == 2) return launch_normed<KC, EPI, 4, 2, 4>(x, nw, eps, w, out, M, N, K, tiles, stream);
+  if (K > 1024) return launch_normed<KC, EPI, 4, 1, 8>(x, nw, eps, w, out, M, N, K, tiles, stream);
+  return launch_normed<KC, EPI, 4, 1, 4>(x, nw, eps, w, out, M, N, K, tiles, stream);
+}
+
 static bool pieces_serves(int M, int N, int K, int epi);
 #define NORMED_WEIGHT_BELOW (40L << 20)   // weight elements from which the norm stays a kernel of its own
 static long g_normed_weight_below = NORMED_WEIGHT_BELOW;
@@ -1831,6 +1968,10 @@ extern "C" int ti_gemm_bf16_normed(const float* x, const float* nw, float eps, c
   }
   if (epi == TI_EPI_RELU2) {
     ti_set_error("gemm_bf16_normed: this epilogue is left to the norm's kernel and the product's");
+    return 3;
+  }
+  if (normed_lds(M, K, 8, 4) > NORMED_LDS) {
+    ti_set_error("gemm_bf16_normed: %d rows of %d columns do not fit beside the weights", M, K);
     return 3;
   }
   if (row_per_wave_serves(M, N, K, epi)) {
@@ -1856,12 +1997,9 @@ extern "C" int ti_gemm_bf16_normed(const float* x, const float* nw, float eps, c
   const int grid = (epi == TI_EPI_SWIGLU) ? (N + 7) / 8 : (N + 15) / 16;
   const int kc = (K + 255) / 256;
   const int waves = skinny_waves_for(grid, K);
-#define TI_GNK(E, KCV)                                                                                          \
-  return waves == 8                                                                                             \
-             ? launch_staged<NormProducer<KCV>, E, 8>("gemm_bf16_normed", NormProducer<KCV>{x, nw, eps}, w, out, \
-                                                      M, N, K, grid, stream)                                    \
-             : launch_staged<NormProducer<KCV>, E, 4>("gemm_bf16_normed", NormProducer<KCV>{x, nw, eps}, w, out, \
-                                                      M, N, K, grid, stream);
+#define TI_GNK(E, KCV)                                                                                                      \
+  return waves == 8 ? launch_normed<KCV, E, 8, 1, 4>(x, nw, eps, w, out, M, N, K, grid, stream)                             \
+                    : launch_normed_groups<KCV, E>(x, nw, eps, w, out, M, N, K, grid, stream);
 #define TI_GN(E)                        \
   case E:                               \
     if (kc <= 4) TI_GNK(E, 4)           \
@@ -2530,7 +2668,7 @@ extern "C" int ti_gemm_bf16(const void* A, const void* W, void* out, int M, int 
 extern "C" void ti_tuning_reset() {
   g_xcd_rows = 0; g_die_order = 1; g_tiles_160 = 1; g_tiles_256 = 1; g_two_ranges = 1; g_qkv_rows = 0; g_qkv_min_rows = 17; g_force_tile = 0; g_skinny_waves = 0;
   g_skinny_deep = 1; g_use_pipelined = 1; set_tiled_from(280L << 20); g_tiled_from_stored = TILED_FROM_STORED; g_row_per_wave = 1; g_rows_staged = 1;
-  g_normed_weight_below = NORMED_WEIGHT_BELOW; g_skinny_copy = 1; g_wide_rows = 1; g_pieces = 1; g_add_split = 1;
+  g_normed_weight_below = NORMED_WEIGHT_BELOW; g_normed_groups = 0; g_skinny_copy = 1; g_wide_rows = 1; g_pieces = 1; g_add_split = 1;
   g_rows_direct = 1;
   g_wide_rows_min_n = WIDE_ROWS_MIN_N;
   g_wide_rows_grid = 0;
@@ -2538,6 +2676,7 @@ extern "C" void ti_tuning_reset() {
 extern "C" int ti_tuning_set(const char* name, long value) {
   const std::string n = name ? name : "";
   if (n == "force_tile") g_force_tile = (int)value;
+  else if (n == "normed_groups") g_normed_groups = (int)value;
   else if (n == "normed_weight_below") g_normed_weight_below = value > 0 ? value : NORMED_WEIGHT_BELOW;
   else if (n == "tiles_160") g_tiles_160 = (int)value;
   else if (n == "tiles_256") g_tiles_256 = (int)value;

@@ -9,6 +9,7 @@
 //                        11: 256 x 128 by four wavefronts; for SwiGLU alone 5 / 7: 64 x 128, 10: 256 x 256 (another's number:
 //                        128 x 128 for SwiGLU, 128 x 64 for the others); 0: by the shape
 //   normed_weight_below  weights of fewer elements keep the norm inside the product (0: the default)
+//   normed_groups        1 to 3 groups of four wavefronts, a tile each, in the product with the norm inside (0: by the tiles)
 //   tiles_160            0: no tiles of 160 columns
 //   tiles_256            0: no tiles of 256 x 256
 //   two_ranges           0: never split a product's columns between two tiles
