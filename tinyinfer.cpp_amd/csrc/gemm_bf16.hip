@@ -708,64 +708,71 @@ __device__ __forceinline__ float dot2_bf16(unsigned a, unsigned b, float c) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, a), __builtin_bit_cast(bf16x2_t, b), c, false);
 }
 
+// The token rows come by direct loads into LDS, each once a workgroup, and a lane reads back the pieces that go with its own.
+// (Every wavefront asking for them itself, MMAX NL loads of 1 KiB at 16 cycles each of the unit that takes addresses, was what 3 to 8
+// tokens waited for, and the residual, which the compiler asked for at the end.  us in a chain of launches with weights from memory, before and
+// now, at 4 and 8 tokens: 1,024 x 2,048 3.52 4.17 -> 3.16 3.83, 1,024 x 3,072 4.03 4.98 -> 3.59 4.34, 1,024 x 4,096 4.66 6.79 -> 4.04 4.88, 2,048 x
+// 2,048 at 4 4.46 -> 3.98.  Up to two tokens ask for them themselves: the next kernel.)
 template <int EPI, int MMAX, int NL>
 __global__ void __launch_bounds__(256)
 gemv_rows_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ out_, int M, int N,
                  int K, long lda) {
+#if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass has no buffer descriptors)
   static_assert(EPI != TI_EPI_SWIGLU, "no SwiGLU here");
-  extern __shared__ __attribute__((aligned(16))) unsigned char dyn_smem[];
-  bf16_t* sA = reinterpret_cast<bf16_t*>(dyn_smem);          // [M][K]
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  static_assert(MMAX % 4 == 0, "the wavefronts take the token rows in turn");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char dyn_smem[];     // pieces of 1 KiB: [MMAX][NL], then each wavefront's [NL]
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int n = blockIdx.x * 4 + wave;
-  const bf16_t* wp = W + (size_t)(n < N ? n : N - 1) * K;
-  const uint4 zero = make_uint4(0, 0, 0, 0);
-
-  // the residual lane m will add to (row m of the tokens): asked for first
+  // the residual lane m will add to (row m of the tokens)
   float prev = 0.f;
   if (EPI == TI_EPI_ADD_F32) prev = ((const float*)out_)[(size_t)(lane < M ? lane : 0) * N + (n < N ? n : N - 1)];
-  // the token rows (from the cache), 16 bytes per thread and load, all in flight at once; then
-  // this wavefront's weight row (from memory).  Loads come back in the order they were issued.
-  constexpr int PB = (MMAX * NL + 3) / 4;                     // pieces per thread: all of [MMAX][512 NL]
-  const int kp = K >> 3, pieces = M * kp;
-  uint4 av[PB];
+  // The token rows wave, wave + 4, ... (a row beyond M is row 0: read and dropped, so that every load is counted), then the weight row.
+  // All of them direct loads: the waits below count these alone, and whatever else is on its way makes them wait for more, not for less.
+  const auto rows_at = [](const bf16_t* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
 #pragma unroll
-  for (int b = 0; b < PB; ++b) {
-    const int p = threadIdx.x + 256 * b;
-    const int pc = p < pieces ? p : 0;
-    const int m = pc / kp, k8 = pc - m * kp;
-    av[b] = ld16(A + (size_t)m * lda + k8 * 8);
+  for (int t = 0; t < MMAX / 4; ++t) {
+    const int m = wave + 4 * t;
+    const auto rs = rows_at(A + (size_t)(m < M ? m : 0) * lda);
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const int kk = (i * 64 + lane) * 8;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(dyn_smem + (m * NL + i) * 1024), 16,
+                                               (kk < K ? kk : 0) * 2, 0, 0, 0);
+    }
   }
   __builtin_amdgcn_sched_barrier(0);
-  uint4 wv[NL];
+  const auto rsW = rows_at(W + (size_t)(n < N ? n : N - 1) * K);
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
     const int kk = (i * 64 + lane) * 8;
-    wv[i] = ld16(wp + (kk < K ? kk : 0));
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsW, (__attribute__((address_space(3))) void*)(dyn_smem + (MMAX * NL + wave * NL + i) * 1024), 16,
+                                             (kk < K ? kk : 0) * 2, 0, 0, 0);
   }
   __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int b = 0; b < PB; ++b) {
-    const int p = threadIdx.x + 256 * b;
-    if (p < pieces) {
-      const int m = p / kp, k8 = p - m * kp;
-      *reinterpret_cast<uint4*>(sA + (size_t)m * K + k8 * 8) = av[b];
-    }
-  }
-  __syncthreads();
+  wait_vmcnt<NL>();      // the rows have landed; the weights may be on their way
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_sched_barrier(0);
 
-  // rows beyond M repeat row 0 and are dropped: all LDS reads of a piece go out together
   float acc[MMAX];
 #pragma unroll
   for (int m = 0; m < MMAX; ++m) acc[m] = 0.f;
-#pragma unroll
-  for (int i = 0; i < NL; ++i) {
+  const unsigned at = (unsigned)(size_t)dyn_smem + lane * 16, w_at = at + (MMAX + wave) * NL * 1024;
+  auto piece = [&](auto tag) __attribute__((always_inline)) {
+    constexpr int i = decltype(tag)::value;
     const int kk = (i * 64 + lane) * 8;
-    const bool ok = kk < K;
-    const uint4 w = ok ? wv[i] : zero;
-    const bf16_t* ap = sA + (ok ? kk : 0);
-    uint4 a[MMAX];
+    // (read as instructions, or the compiler would have them wait for everything under way)
+    v4u a[MMAX], w;
 #pragma unroll
-    for (int m = 0; m < MMAX; ++m) a[m] = *reinterpret_cast<const uint4*>(ap + (size_t)(m < M ? m : 0) * K);
+    for (int m = 0; m < MMAX; m += 4)
+      asm volatile("ds_read_b128 %0, %4 offset:%5\n\tds_read_b128 %1, %4 offset:%6\n\tds_read_b128 %2, %4 offset:%7\n\t"
+                   "ds_read_b128 %3, %4 offset:%8\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(a[m]), "=&v"(a[m + 1]), "=&v"(a[m + 2]), "=&v"(a[m + 3])
+                   : "v"(at), "n"((m * NL + i) * 1024), "n"(((m + 1) * NL + i) * 1024), "n"(((m + 2) * NL + i) * 1024),
+                     "n"(((m + 3) * NL + i) * 1024)
+                   : "memory");
+    wait_vmcnt<NL - 1 - i>();
+    asm volatile("ds_read_b128 %0, %1 offset:%2\n\ts_waitcnt lgkmcnt(0)" : "=&v"(w) : "v"(w_at), "n"(i * 1024) : "memory");
+    if (kk >= K) w = v4u{0, 0, 0, 0};
 #pragma unroll
     for (int m = 0; m < MMAX; ++m) {
       acc[m] = dot2_bf16(w.x, a[m].x, acc[m]);
@@ -773,7 +780,13 @@ gemv_rows_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, voi
       acc[m] = dot2_bf16(w.z, a[m].z, acc[m]);
       acc[m] = dot2_bf16(w.w, a[m].w, acc[m]);
     }
-  }
+  };
+  static_assert(NL == 2 || NL == 4 || NL == 6 || NL == 8, "pieces of a row");
+  piece(std::integral_constant<int, 0>{}), piece(std::integral_constant<int, 1>{});
+  if constexpr (NL > 2) piece(std::integral_constant<int, 2>{}), piece(std::integral_constant<int, 3>{});
+  if constexpr (NL > 4) piece(std::integral_constant<int, 4>{}), piece(std::integral_constant<int, 5>{});
+  if constexpr (NL > 6) piece(std::integral_constant<int, 6>{}), piece(std::integral_constant<int, 7>{});
+  if (EPI == TI_EPI_ADD_F32) asm volatile("" : "+v"(prev));      // (or the load would move behind the condition below)
   float mine = 0.f;
 #pragma unroll
   for (int m = 0; m < MMAX; ++m) {
@@ -786,15 +799,14 @@ gemv_rows_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, voi
     if (EPI == TI_EPI_ADD_F32) ((float*)out_)[o] = prev + mine;
     if (TI_EPI_ACT(EPI)) ((bf16_t*)out_)[o] = f2bf(epi_act<EPI>(mine));
   }
+#endif
 }
 
-// The same product with the token rows straight from memory into registers: lane l fetches, for every
+// The same product for one or two tokens, their rows straight from memory into registers: lane l fetches, for every
 // token, the pieces of the row that go with its pieces of the weight row (all workgroups read the same few
-// KB: they come from the caches), after its weights have been asked for.  Nothing goes through LDS, so
-// nothing is written, waited for at a barrier and read back between the arrival of the weights and the
-// products (8 tokens, a 1,024 x 2,048 weight, in a chain of dependent launches: 5.3 -> 4.75 us; 1,024 x
-// 3,072: 6.3 -> 5.7 us).  The same order of sums, the same bits.  MMAX * NL * 4 registers hold the token
-// rows: up to NL = 6 (K <= 3,072) at 8 tokens.
+// KB: they come from the caches), after its weights have been asked for.  Nothing is waited for at a barrier and read back between
+// the arrival of the weights and the products.  The same order of sums, the same bits.  (With the residual asked for in front, one token:
+// 1,024 x 2,048 3.14 -> 2.83, 1,024 x 3,072 3.38 -> 3.16.)
 template <int EPI, int MMAX, int NL>
 __global__ void __launch_bounds__(256)
 gemv_rows_direct_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ out_, int M,
@@ -836,6 +848,7 @@ gemv_rows_direct_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__
       acc[m] = dot2_bf16(w.w, a[i][m].w, acc[m]);
     }
   }
+  if (EPI == TI_EPI_ADD_F32) asm volatile("" : "+v"(prev));      // (or the load would move behind the condition below)
   float mine = 0.f;
 #pragma unroll
   for (int m = 0; m < MMAX; ++m) {
@@ -1866,24 +1879,18 @@ static bool row_per_wave_serves(int M, int N, int K, int epi) {
          K <= 64 * 8 * GR_LOADS && (epi == TI_EPI_STORE_F32 || epi == TI_EPI_ADD_F32 || epi == TI_EPI_RELU2);
 }
 
-static int g_rows_direct = 1;     // a hook for measurements: 0: the token rows go through LDS for every K
+static int g_rows_direct = 1;     // a hook for measurements: 0: the rows of one and two tokens go through LDS too
 template <int EPI, int MMAX, int NL>
 static int launch_rows_mk(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda, hipStream_t s) {
-  if constexpr (MMAX * NL <= 48) {
-    if (g_rows_direct) {
-      gemv_rows_direct_kernel<EPI, MMAX, NL><<<(N + 3) / 4, 256, 0, s>>>(A, W, out, M, N, K, lda);
-      return 0;
-    }
+  if constexpr (MMAX <= 2) {
+    gemv_rows_direct_kernel<EPI, MMAX, NL><<<(N + 3) / 4, 256, 0, s>>>(A, W, out, M, N, K, lda);
+  } else {
+    constexpr int lds = (MMAX + 4) * NL * 1024;
+    auto kern = gemv_rows_kernel<EPI, MMAX, NL>;
+    static const hipError_t room = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    TI_REQUIRE(room == hipSuccess, "gemm_bf16: %d bytes of LDS: %s", lds, hipGetErrorString(room));
+    kern<<<(N + 3) / 4, 256, lds, s>>>(A, W, out, M, N, K, lda);
   }
-  const size_t lds = (size_t)M * K * 2;
-  auto kern = gemv_rows_kernel<EPI, MMAX, NL>;
-  static size_t allowed = 48 * 1024;
-  if (lds > allowed) {
-    TI_REQUIRE(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) ==
-                   hipSuccess, "gemm_bf16: LDS size refused");
-    allowed = lds;
-  }
-  kern<<<(N + 3) / 4, 256, lds, s>>>(A, W, out, M, N, K, lda);
   return 0;
 }
 template <int EPI, int MMAX>
@@ -1897,8 +1904,8 @@ static int launch_rows_m(const bf16_t* A, const bf16_t* W, void* out, int M, int
 // the same in all of them
 template <int EPI>
 static int launch_rows(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda, hipStream_t s) {
-  if (M <= 1) return launch_rows_m<EPI, 1>(A, W, out, M, N, K, lda, s);
-  if (M <= 2) return launch_rows_m<EPI, 2>(A, W, out, M, N, K, lda, s);
+  if (M <= 1 && g_rows_direct) return launch_rows_m<EPI, 1>(A, W, out, M, N, K, lda, s);
+  if (M <= 2 && g_rows_direct) return launch_rows_m<EPI, 2>(A, W, out, M, N, K, lda, s);
   if (M <= 4) return launch_rows_m<EPI, 4>(A, W, out, M, N, K, lda, s);
   return launch_rows_m<EPI, GR_MMAX>(A, W, out, M, N, K, lda, s);
 }

@@ -29,7 +29,7 @@
 //   skinny_copy          0: up to 16 tokens, fragments of the token rows straight from memory
 //   pieces               0: up to 16 rows never take the kernel with the token rows in pieces
 //   skinny_deep          0: four chunks of K in flight per wavefront also for a long K
-//   rows_direct          0: the kernel with a weight row per wavefront takes its token rows through LDS for every K
+//   rows_direct          0: the kernel with a weight row per wavefront takes the rows of one and two tokens through LDS too
 //   wide_rows_min_n      the fewest weight rows from which 17..64 rows take the kernel that keeps them in registers (16,384)
 //   wide_rows_grid       its number of workgroups (0: a tile of 16 weight rows each, at most one per compute unit)
 // libti_attention_bf16:
