@@ -1168,6 +1168,7 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   constexpr int V_LOADS = HD / 16;                    // 16 dims (64 bytes each) per wavefront load
   static_assert(K_LOADS % NW == 0 && V_LOADS % NW == 0, "every wavefront takes the same kinds of loads");
   constexpr int MY_K = K_LOADS / NW, MY_LOADS = (K_LOADS + V_LOADS) / NW;   // per wavefront and turn
+  constexpr int QL = NG >= 4 ? TROWS * HD * 2 / 1024 / (NG * NW) : 0;      // loads of queries a wavefront, 0: as operands from memory
   constexpr int KS = HD / 16;                         // k-steps of the first product
   constexpr int DB = HD / 32;                         // 32-dim blocks of the output
 
@@ -1307,13 +1308,29 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
     }
   };
   constexpr int AHEAD = ST - 1;
-  // the first run's blocks and first turns are asked for before the queries: those arrive meanwhile
+  // The queries of a workgroup of many groups, which all take the same rows, come through LDS as well: QL loads a wavefront of whole rows (piece c
+  // of row r in place c ^ (r & (NP - 1))).  As operands from memory, a row in every lane, they were 64 loads a tile of 64 cycles each of the unit that
+  // takes addresses, in front of a tile's first scores.  (us a launch at 16 heads, 8 for keys, before and now: 2,048 tokens 40.0 -> 38.3, 77 8.2
+  // -> 7.5, 504 behind 500 20.6 -> 19.8; 2,048 at 32 heads 74.4 -> 72.2.)
+  if constexpr (QL > 0) {
+    const char* rows = reinterpret_cast<const char*>(q + (size_t)head * HD);
+#pragma unroll
+    for (int j = 0; j < QL; ++j) {
+      const int g = wid + NG * NW * j, r = g * K_ROWS + lane / NP;
+      const char* src = rows + (size_t)min(first + r, row_end - 1) * ((size_t)n_head * HD * 2) + (((lane % NP) ^ (r & (NP - 1))) << 4);
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                       (__attribute__((address_space(3))) void*)(size_t)((unsigned)(size_t)smem + NG * ST * STAGE + g * 1024), 16, 0, 0);
+    }
+  }
+  // the first run's blocks and first turns are asked for before the queries are waited for: those arrive meanwhile
   // (a workgroup whose run of keys is empty walks nothing, and nothing may be on its way into LDS
   // when it goes on to the merge)
+  int under_way = 0;
   if (blk_lo <= blk_hi) {
     const int nblk = min(64, blk_hi + 1 - blk_lo);
     run_blocks(blk_lo, nblk);
     const int my_turns = ((nblk + 1) / 2 - grp + NG - 1) / NG;
+    under_way = min(AHEAD, my_turns);
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i)
       if (i < my_turns) issue(i, i * STAGE);
@@ -1322,6 +1339,19 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   v4u qf[CB][KS];
   int my_pos[CB];
   bool col_ok[CB];
+  if constexpr (QL > 0) {
+    vm_wait_turns<MY_LOADS, ST + 1>(under_way);
+    __builtin_amdgcn_s_barrier();
+    static_assert(CB == 1, "a column block a wavefront");
+    const int r = wave * 32 + r32;
+    const unsigned at = (unsigned)(size_t)smem + NG * ST * STAGE + r * (HD * 2);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      asm volatile("ds_read_b128 %0, %1" : "=v"(qf[0][ks]) : "v"(at + (((ks * 2 + h) ^ (r & (NP - 1))) << 4)));
+    lgkm_wait(0);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[0][ks]));
+  }
 #pragma unroll
   for (int cb = 0; cb < CB; ++cb) {
     const int row = w_first + cb * 32 + r32;
@@ -1329,6 +1359,10 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
     my_pos[cb] = start + (row - row0);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
+      if constexpr (QL > 0) {
+        if (!col_ok[cb]) qf[cb][ks] = v4u{0, 0, 0, 0};
+        continue;
+      }
       qf[cb][ks] = v4u{0, 0, 0, 0};
       if (col_ok[cb]) {
         const uint4 t = *reinterpret_cast<const uint4*>(q + ((size_t)row * n_head + head) * HD + ks * 16 + h * 8);
@@ -1420,7 +1454,10 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
       float bm = sv[0];
 #pragma unroll
       for (int i = 1; i < 16; ++i) bm = fmaxf(bm, sv[i]);
-      bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+      {
+        const LanePair p = lane_pair<32>(bm);
+        bm = fmaxf(p.a, p.b);
+      }
       const float m_new = fmaxf(mx[cb], bm * scale2);
       const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
       float ps = 0.f;
@@ -1565,64 +1602,69 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   } else {
     // The groups merge their partial results through LDS (the stages are free now), each group the
     // values it owns: values VPG g .. VPG (g + 1) - 1 of every lane are group g's.  A group leaves the
-    // values it does not own (in their order), its maximum and its sum in its part of LDS; after a
+    // values it does not own (in their order, four to a slot of 16 bytes a lane), its maximum and its sum in its part of LDS; after a
     // barrier it reads the others' contributions to its own values, merges them with its own and
-    // writes them out.  Which registers a group takes its values from is a choice between registers by
-    // the group's number, which every lane of a wavefront shares: the accumulators stay in registers.
-    constexpr int VALS = DB * 16, VPG = VALS / NG, ML = VALS - VPG, SLOTS = ML + 2;
+    // writes them out.  The code stands once for each group, so that which registers these are is known where it is compiled (as a
+    // choice between registers by the group's number, value by value, a tile's end took 4,400 cycles; 2,048 tokens 38.0 us, now 36.4, 77 7.5,
+    // now 7.05, 2,048 at 32 heads 73.2, now 70.0).
+    constexpr int VALS = DB * 16, VPG = VALS / NG, FOURS = (VALS - VPG) / 4, PART = (FOURS * 16 + 8) * 64;
     static_assert(VALS % NG == 0 && VPG % 4 == 0, "a group owns whole fours of values");
-    static_assert(NG * NW * SLOTS * 64 * 4 <= NG * ST * STAGE, "the partial results fit into the stages");
-    typedef __attribute__((address_space(3))) float lds_float;
-    auto part_of = [&](int g) __attribute__((always_inline)) {
-      return (lds_float*)(size_t)((unsigned)(size_t)smem + (unsigned)(((g * NW + wave) * SLOTS * 64 + lane) * 4));
-    };
+    static_assert(NG * NW * PART <= NG * ST * STAGE, "the partial results fit into the stages");
+    typedef __attribute__((address_space(3))) floatx4 lds_four;
+    typedef __attribute__((address_space(3))) ti_float2v lds_two;
+    // slot i (values 4 i .. of those left) of group g's wavefront, and behind the slots its maximum and sum
+    const unsigned part0 = (unsigned)(size_t)smem + wave * PART;
+    auto four_of = [&](int g, int i) __attribute__((always_inline)) { return (lds_four*)(size_t)(part0 + g * (NW * PART) + i * 1024 + lane * 16); };
+    auto ml_of = [&](int g) __attribute__((always_inline)) { return (lds_two*)(size_t)(part0 + g * (NW * PART) + FOURS * 1024 + lane * 8); };
     // only the workgroup's barrier tells that every group is done with its stages
     if constexpr (NW == 1) __syncthreads();
-    const int first = grp * VPG;                     // this group's first value
+    auto merge = [&](auto tag, int cb) __attribute__((always_inline)) {
+      constexpr int G = decltype(tag)::value, FIRST = G * VPG;      // this group, and its first value
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      if (cb > 0) __syncthreads();                   // the block before has been read
-      lds_float* mine = part_of(grp);
-#pragma unroll
-      for (int sl = 0; sl < ML; ++sl)                // slot sl: value sl below this group's own, sl + VPG above them
-        mine[sl * 64] = (sl < first) ? o[cb][sl >> 4][sl & 15] : o[cb][(sl + VPG) >> 4][(sl + VPG) & 15];
-      mine[ML * 64] = mx[cb];
-      mine[(ML + 1) * 64] = l[cb];
-      __syncthreads();
-      float m_g[NG], l_g[NG];
-#pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        m_g[g] = part_of(g)[ML * 64];
-        l_g[g] = part_of(g)[(ML + 1) * 64];
+      for (int i = 0; i < FOURS; ++i) {
+        constexpr auto at = [](int sl) { return sl < FIRST ? sl : sl + VPG; };
+        const int v = at(4 * i);
+        *four_of(G, i) = floatx4{o[cb][v >> 4][v & 15], o[cb][v >> 4][(v & 15) + 1], o[cb][v >> 4][(v & 15) + 2], o[cb][v >> 4][(v & 15) + 3]};
       }
-      float m_all = m_g[0];
+      *ml_of(G) = ti_float2v{mx[cb], l[cb]};
+      __syncthreads();
+      ti_float2v ml[NG];
 #pragma unroll
-      for (int g = 1; g < NG; ++g) m_all = fmaxf(m_all, m_g[g]);
+      for (int g = 0; g < NG; ++g) ml[g] = *ml_of(g);
+      floatx4 theirs[NG][VPG / 4];
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int j = 0; j < VPG / 4; ++j)
+          if (g != G) theirs[g][j] = *four_of(g, (FIRST + (G > g ? -VPG : 0)) / 4 + j);
+      float m_all = ml[0].x;
+#pragma unroll
+      for (int g = 1; g < NG; ++g) m_all = fmaxf(m_all, ml[g].x);
       const float m_safe = (m_all == -INFINITY) ? 0.f : m_all;
       float a_g[NG], l_all = 0.f;
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
-        a_g[g] = __builtin_amdgcn_exp2f(m_g[g] - m_safe);
-        l_all += l_g[g] * a_g[g];
+        a_g[g] = __builtin_amdgcn_exp2f(ml[g].x - m_safe);
+        l_all += ml[g].y * a_g[g];
       }
       const float a_own = __builtin_amdgcn_exp2f(mx[cb] - m_safe);
       float val[VPG];
 #pragma unroll
-      for (int j = 0; j < VPG; ++j) {
-        float own = o[cb][j >> 4][j & 15];
+      for (int j = 0; j < VPG; ++j) val[j] = o[cb][(FIRST + j) >> 4][(FIRST + j) & 15] * a_own;
 #pragma unroll
-        for (int g = 1; g < NG; ++g)
-          if (grp == g) own = o[cb][(g * VPG + j) >> 4][(g * VPG + j) & 15];
-        val[j] = own * a_own;
-      }
+      for (int g = 0; g < NG; ++g)
 #pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        if (g == grp) continue;                      // the same in every lane
-        const lds_float* theirs = part_of(g) + (first + (grp > g ? -VPG : 0)) * 64;
+        for (int j = 0; j < VPG; ++j)
+          if (g != G) val[j] += theirs[g][j / 4][j % 4] * a_g[g];
+      write_out(cb, val, FIRST, std::integral_constant<int, VPG>{}, m_all, l_all + __shfl_xor(l_all, 32, 64));
+    };
 #pragma unroll
-        for (int j = 0; j < VPG; ++j) val[j] += theirs[j * 64] * a_g[g];
-      }
-      write_out(cb, val, first, std::integral_constant<int, VPG>{}, m_all, l_all + __shfl_xor(l_all, 32, 64));
+    for (int cb = 0; cb < CB; ++cb) {
+      if (cb > 0) __syncthreads();                   // the block before has been read
+      unrolled_while<NG>([&](auto tag) __attribute__((always_inline)) {      // (the same in every lane)
+        if (grp == decltype(tag)::value) merge(tag, cb);
+        return true;
+      });
     }
   }
   // the next tile's loads go into the LDS that the merge has just read
@@ -1878,17 +1920,18 @@ extern "C" int ti_attention_prefill_paired_bf16(const void* q, const void* pool,
              "attention_prefill_paired: 1 to 8 runs of keys, more than one with buffers for their results");
   if (n_tiles == 0) return 0;
   constexpr int NG = 4, NW = 2, ST = 2, CB = 1;
-  const int lds = NG * ST * 2 * PF_KEYS * hd * 2;
+  constexpr int LDS = NG * ST * 2 * PF_KEYS * 2 + 32 * NW * CB * 2;      // per head dimension: the stages, and the queries
+  const int lds = LDS * hd;
   static bool ready = false;          // allow more than 64 KiB of dynamic LDS, once
   if (!ready) {
     if (hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<128, NG, NW, ST, true, CB>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, NG * ST * 2 * PF_KEYS * 128 * 2) != hipSuccess ||
+                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS * 128) != hipSuccess ||
         hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<64, NG, NW, ST, true, CB>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, NG * ST * 2 * PF_KEYS * 64 * 2) != hipSuccess ||
+                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS * 64) != hipSuccess ||
         hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<128, NG, NW, ST, false, CB>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, NG * ST * 2 * PF_KEYS * 128 * 2) != hipSuccess ||
+                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS * 128) != hipSuccess ||
         hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<64, NG, NW, ST, false, CB>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, NG * ST * 2 * PF_KEYS * 64 * 2) != hipSuccess) {
+                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS * 64) != hipSuccess) {
       ti_set_error("attention_prefill_paired: cannot reserve the LDS");
       return 2;
     }
@@ -1991,13 +2034,12 @@ extern "C" int ti_attention_step_bf16(const void* q, const void* pool, const int
   const int parts = (n_head / n_kv + 15) / 16;
   const long grid = (long)n_tiles * n_head + (long)n_runs * n_kv * parts;
   TI_REQUIRE(grid <= 0x7fffffL, "attention_step: too many workgroups");
-  // the runs' LDS is the larger: the same stages, and the merge's maxima and sums
-  static_assert(sizeof(StagedMerge<128, 8, 1>) >= 4 * 2 * 2 * PF_KEYS * 2 * 128 && sizeof(StagedMerge<64, 8, 1>) >= 4 * 2 * 2 * PF_KEYS * 2 * 64,
-                "the tiles' stages fit");
+  constexpr int STAGES = 4 * 2 * 2 * PF_KEYS * 2 + 64 * 2;      // bytes of the tiles' stages and queries per head dimension
+  static_assert(sizeof(StagedMerge<128, 8, 1>) <= STAGES * 128 && sizeof(StagedMerge<64, 8, 1>) <= STAGES * 64, "the runs' stages and merge fit");
   static bool ready = false;          // allow more than 64 KiB of dynamic LDS, once
   if (!ready) {
-    if (hipFuncSetAttribute((const void*)attn_step_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(StagedMerge<128, 8, 1>)) != hipSuccess ||
-        hipFuncSetAttribute((const void*)attn_step_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize, sizeof(StagedMerge<64, 8, 1>)) != hipSuccess) {
+    if (hipFuncSetAttribute((const void*)attn_step_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, STAGES * 128) != hipSuccess ||
+        hipFuncSetAttribute((const void*)attn_step_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize, STAGES * 64) != hipSuccess) {
       ti_set_error("attention_step: cannot reserve the LDS");
       return 2;
     }
@@ -2006,7 +2048,7 @@ extern "C" int ti_attention_step_bf16(const void* q, const void* pool, const int
   const float cap = softcap > 0.f ? softcap : 0.f;
 #define TI_GO(H)                                                                                                              \
   do {                                                                                                                        \
-    attn_step_kernel<H><<<(unsigned)grid, 512, sizeof(StagedMerge<H, 8, 1>), stream>>>((const bf16_t*)q, (const bf16_t*)pool, table, table_stride, \
+    attn_step_kernel<H><<<(unsigned)grid, 512, STAGES * H, stream>>>((const bf16_t*)q, (const bf16_t*)pool, table, table_stride, \
                                                                      tiles, n_tiles, entries, runs, run_stride, n_head / n_kv,  \
                                                                      (bf16_t*)out, part_o, part_ml,                              \
                                                                      n_head, n_kv, page_size, scale, window, cap, g_sink);       \
