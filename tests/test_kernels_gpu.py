@@ -1146,6 +1146,40 @@ def test_linear_bf16_rows_through_lds_up_to_16_rows(ops, M, N, K):
     assert (f64(outs[1][0][:M]) - ref_linear(a.cpu(), w.cpu())).abs().max() < 2e-5 * K
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 8184, 4160), (33, 6168, 1088), (48, 4104, 2048), (49, 8192, 2048), (64, 4112, 64), (64, 40, 4160), (65, 4096, 128),
+                                   (77, 2056, 1088), (80, 24, 64), (81, 6152, 320), (112, 4088, 2112)])
+def test_linear_bf16_rows_through_lds_up_to_112_rows(ops, M, N, K):
+    """One and two groups of weight rows a workgroup: a last workgroup whose second group has few rows or none, four and eight wavefronts,
+    fewer steps than stages and than wavefronts, a first and a last row of a block of 16.  The groups change no bit, the values are
+    float64's within the bound of 32-bit sums, and what lies beyond the rows is left."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = dev((torch.rand(M, K + 8, generator=g) * 2 - 1).to(torch.bfloat16))[:, :K]
+    w = dev((torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    lib, outs = ops.lib("gemm_bf16"), {}
+    lib.ti_tuning_reset()
+    try:
+        for groups in (0, 1, 2):
+            lib.ti_tuning_set(b"skinny_groups", groups)
+            res = [torch.full((M + 1, N if e != "swiglu" else N // 2), 7.0, device="cuda", dtype=torch.float32 if e == "store" else torch.bfloat16)
+                   for e in ("store", "store_act", "swiglu")]
+            for out, e in zip(res, ("store", "store_act", "swiglu")):
+                ops.linear(a, w, out[:M], e)
+            outs[groups] = res
+    finally:
+        lib.ti_tuning_reset()
+    for groups in (1, 2):
+        for x, y in zip(outs[0], outs[groups]):
+            assert torch.equal(x, y), groups
+    store, act, pair = (f64(x) for x in outs[0])
+    assert bool((store[M] == 7.0).all()) and bool((act[M] == 7.0).all()) and bool((pair[M] == 7.0).all())
+    ref = ref_linear(a.cpu(), w.cpu())
+    assert (store[:M] - ref).abs().max() < 2e-5 * K
+    assert (act[:M] - ref).abs().max() < 0.005 * ref.abs().max() + 2e-5 * K
+    gate, up = ref[:, :N // 2], ref[:, N // 2:]
+    ref = gate / (1 + torch.exp(-gate)) * up
+    assert (pair[:M] - ref).abs().max() < 0.005 * ref.abs().max() + 10 * 2e-5 * K
+
+
 @pytest.mark.parametrize("N,K,epi", [(2048, 4096, "store"), (2040, 4096, "store"), (2048, 4096, "swiglu"), (2048, 2048, "store"), (2064, 4096, "store")])
 def test_norm_in_front_of_a_weight_of_8_mi_elements_changes_no_bit(ops, N, K, epi):
     """On either side of the size from which four wavefronts share K in place of eight: the product with the norm inside it and the

@@ -50,22 +50,23 @@ __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f +
 // issued before the first product: out-of-range pieces read a valid address (piece 0 of the
 // row) and get a zeroed weight instead of a branch, so that nothing waits in between.
 // STAGES > 0 (K of whole chunks; up to 16 tokens where staged_16_serves says so): the rows come through LDS (staged_rows.h), a chunk a step; the same sums in the
-// same order.  Every workgroup pulls in all token rows, which as operands from memory was most of its time.  us, before and now, at 17,
+// same order.  G: groups of 16 weight rows a workgroup then takes (skinny_groups_for).  Every workgroup pulls in all token rows, which as operands from memory was most of its time.  us, before and now, at 17,
 // 32, 48 and 64 rows: 4096 x 1024 4.3 4.9 5.9 6.9 -> 3.9 4.0 3.9 4.6; [gate; up] 6144 x 1024 6.7 7.8 9.8 10.0 -> 5.3 5.8 6.9 7.9 (the
-// latter two were tiles); 4096 x 2048 8.7 9.3 10.9 11.9 -> 6.0 6.4 7.2 8.3; 12288 x 2048 16.1 17.0 17.8 18.4 -> 11.5 13.5 16.3 18.6.
+// latter two were tiles; G = 2: 4.9 5.1 5.7 6.4); 4096 x 2048 8.7 9.3 10.9 11.9 -> 6.0 6.4 7.2 8.3; 12288 x 2048 16.1 17.0 17.8 18.4 -> 11.5 13.5 16.3 18.6.
 struct RowPieces { v4u x, y; };
-template <int MT, int EPI, int NW = 4, int UN = 4, int STAGES = 0>
+template <int MT, int EPI, int NW = 4, int UN = 4, int STAGES = 0, int G = 1>
 __global__ void __launch_bounds__(NW * 64)
 gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ out_,
                    int M, int N, int K, long lda) {
 #if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass has no buffer descriptors)
   constexpr bool SW = (EPI == TI_EPI_SWIGLU);
-  constexpr int BLOCKS = MT + 1, STAGED = STAGES * BLOCKS * 2048;      // a wavefront's stages, where its sums lie afterwards
-  static_assert(STAGES == 0 || STAGED >= MT * 16 * 17 * 4, "a wavefront's sums fit into its stages");
+  constexpr int BLOCKS = MT + G, STAGED = STAGES * BLOCKS * 2048;      // a wavefront's stages, where its sums lie afterwards
+  static_assert(STAGES == 0 || STAGED >= G * MT * 16 * 17 * 4, "a wavefront's sums fit into its stages");
+  static_assert(G == 1 || STAGES > 0, "several groups of weight rows: through LDS");
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   __shared__ float s_red[STAGES ? 1 : NW][MT][16][17];
-  const auto red = [&](int w, int t, int a, int b) -> float& {
-    if constexpr (STAGES) return reinterpret_cast<float (*)[16][17]>(smem + w * STAGED)[t][a][b];
+  const auto red = [&](int w, int g, int t, int a, int b) -> float& {
+    if constexpr (STAGES) return reinterpret_cast<float (*)[16][17]>(smem + w * STAGED)[g * MT + t][a][b];
     else return s_red[w][t][a][b];
   };
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -88,30 +89,35 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
   }
   // the residual this thread will add to, asked for before the product
   const int tok = threadIdx.x >> 4, row = threadIdx.x & 15;
-  float prev[MT];
+  float prev[G][MT];
   if (EPI == TI_EPI_ADD_F32) {   // threads without an output element read a valid one: no branch
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      const int m = t * 16 + (tok & 15), n = blockIdx.x * 16 + row;
-      prev[t] = ((const float*)out_)[(size_t)(m < M ? m : 0) * N + (n < N ? n : N - 1)];
-    }
-  }
-  floatx4 acc[MT];
+    for (int g = 0; g < G; ++g)
 #pragma unroll
-  for (int t = 0; t < MT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < MT; ++t) {
+        const int m = t * 16 + (tok & 15), n = blockIdx.x * 16 * G + g * 16 + row;
+        prev[g][t] = ((const float*)out_)[(size_t)(m < M ? m : 0) * N + (n < N ? n : N - 1)];
+      }
+  }
+  floatx4 acc[G][MT];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[g][t] = floatx4{0.f, 0.f, 0.f, 0.f};
 
   const uint4 zero = make_uint4(0, 0, 0, 0);
   // chunk c covers k in [64 c, 64 c + 64); lane group j takes [64 c + 16 j, +16)
   const int chunks = (K + 63) / 64;
   if constexpr (STAGES > 0) {
     const int lr = lane >> 3, piece = ((lane & 7) ^ lr) * 16;
-    const int n0 = blockIdx.x * (SW ? 8 : 16);
+    const int n0 = blockIdx.x * G * (SW ? 8 : 16);
     unsigned voff[BLOCKS][2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      voff[0][h] = (unsigned)min((SW ? 0 : 8 * h) + lr, N - 1 - n0) * (unsigned)(K * 2) + piece;
 #pragma unroll
-      for (int t = 0; t < MT; ++t) voff[1 + t][h] = (unsigned)min(16 * t + 8 * h + lr, M - 1) * (unsigned)(lda * 2) + piece;
+      for (int g = 0; g < G; ++g) voff[g][h] = (unsigned)min((SW ? 8 * g : 16 * g + 8 * h) + lr, N - 1 - n0) * (unsigned)(K * 2) + piece;
+#pragma unroll
+      for (int t = 0; t < MT; ++t) voff[G + t][h] = (unsigned)min(16 * t + 8 * h + lr, M - 1) * (unsigned)(lda * 2) + piece;
     }
     const auto rows_at = [](const bf16_t* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
     const auto rsW = rows_at(W + (size_t)n0 * K + wave * 64), rsU = rows_at(W + (size_t)(n0 + (SW ? N : 0)) * K + wave * 64);
@@ -123,7 +129,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           auto* dst = (__attribute__((address_space(3))) void*)(mine + stage + i * 2048 + h * 1024);      // the same in every lane
-          if (i > 0) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, dst, 16, voff[i][h], step * NW * 128, 0, 0);
+          if (i >= G) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, dst, 16, voff[i][h], step * NW * 128, 0, 0);
           else if (SW && h == 1) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsU, dst, 16, voff[i][h], step * NW * 128, 0, 0);
           else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsW, dst, 16, voff[i][h], step * NW * 128, 0, 0);
         }
@@ -133,10 +139,12 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
     staged_steps<BLOCKS, STAGES, RowPieces>(steps, at + (((2 * j) ^ (r & 7)) << 4), at + (((2 * j + 1) ^ (r & 7)) << 4), load,
                                             [&](const RowPieces* e) {
 #pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, e[0].x), __builtin_bit_cast(bf16x8, e[1 + t].x), acc[t], 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, e[0].y), __builtin_bit_cast(bf16x8, e[1 + t].y), acc[t], 0, 0, 0);
-      }
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, e[g].x), __builtin_bit_cast(bf16x8, e[G + t].x), acc[g][t], 0, 0, 0);
+          acc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, e[g].y), __builtin_bit_cast(bf16x8, e[G + t].y), acc[g][t], 0, 0, 0);
+        }
     });
   }
   if constexpr (STAGES == 0)
@@ -167,16 +175,18 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
       if (!ok1[u]) w1[u].u = zero;
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0[u].v, a0[u][t].v, acc[t], 0, 0, 0);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[u].v, a1[u][t].v, acc[t], 0, 0, 0);
+        acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0[u].v, a0[u][t].v, acc[0][t], 0, 0, 0);
+        acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[u].v, a1[u][t].v, acc[0][t], 0, 0, 0);
       }
     }
   }
-  // acc[t][i]: weight row 4 j + i, token 16 t + r
+  // acc[g][t][i]: row 4 j + i of weight group g, token 16 t + r
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
+  for (int g = 0; g < G; ++g)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red(wave, t, r, 4 * j + i) = acc[t][i];
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red(wave, g, t, r, 4 * j + i) = acc[g][t][i];
   __syncthreads();
   // thread -> (token = tid / 16, row = tid % 16): consecutive threads, consecutive columns
   if (NW > 4 && threadIdx.x >= 256) return;
@@ -185,26 +195,31 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
     const int m = t * 16 + tok;
     if (m >= M) continue;
     if (SW) {
-      if (row >= 8) continue;
-      const int n = blockIdx.x * 8 + row;
-      if (n >= N) continue;
-      float g = 0.f, u = 0.f;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        g += red(w, t, tok, row);
-        u += red(w, t, tok, row + 8);
+      for (int c = row; c < 8 * G; c += 16) {
+        const int n = blockIdx.x * 8 * G + c;
+        if (n >= N) continue;
+        float g = 0.f, u = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+          g += red(w, c >> 3, t, tok, c & 7);
+          u += red(w, c >> 3, t, tok, (c & 7) + 8);
+        }
+        ((bf16_t*)out_)[(size_t)m * N + n] = f2bf(silu_mul(g, u));
       }
-      ((bf16_t*)out_)[(size_t)m * N + n] = f2bf(silu_mul(g, u));
     } else {
-      const int n = blockIdx.x * 16 + row;
-      if (n >= N) continue;
-      float s = 0.f;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) s += red(w, t, tok, row);
-      const size_t o = (size_t)m * N + n;
-      if (EPI == TI_EPI_STORE_F32) ((float*)out_)[o] = s;
-      if (EPI == TI_EPI_ADD_F32) ((float*)out_)[o] = prev[t] + s;
-      if (TI_EPI_ACT(EPI)) ((bf16_t*)out_)[o] = f2bf(epi_act<EPI>(s));
+      for (int g = 0; g < G; ++g) {
+        const int n = blockIdx.x * 16 * G + g * 16 + row;
+        if (n >= N) continue;
+        float s = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) s += red(w, g, t, tok, row);
+        const size_t o = (size_t)m * N + n;
+        if (EPI == TI_EPI_STORE_F32) ((float*)out_)[o] = s;
+        if (EPI == TI_EPI_ADD_F32) ((float*)out_)[o] = prev[g][t] + s;
+        if (TI_EPI_ACT(EPI)) ((bf16_t*)out_)[o] = f2bf(epi_act<EPI>(s));
+      }
     }
   }
 #endif
@@ -1753,18 +1768,39 @@ static bool staged_16_serves(int M, int N, int K, long lda, int epi) {
   const long elements = (epi == TI_EPI_SWIGLU ? 2L * N : (long)N) * K;
   return g_rows_staged && M <= 16 && staged_fits(K, lda) && (M > 8 || elements < (288L << 20));
 }
-// Stages of the kernel for up to 64 rows: all of 1,024 columns under way where a workgroup has its compute unit for itself, room for two
-// workgroups where they share it.
-template <int MT, int EPI, int NW, int STAGES>
+// Stages where a workgroup has four wavefronts, MT blocks of token rows and G of weight rows: as many as fit, up to all of 1,024 columns, where a workgroup
+// has its compute unit for itself; two where that leaves room for a second workgroup and there is one.
+constexpr int skinny_stages(int MT, int G, bool alone) {
+  const int step = 4 * (MT + G) * 2048, most = 160 * 1024 / step;
+  return !alone && 4 * step <= 160 * 1024 ? 2 : most < 4 ? most : 4;
+}
+template <int MT, int EPI, int NW, int STAGES, int G = 1>
 static int launch_skinny_staged(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda, int grid, hipStream_t s) {
-  constexpr int lds = NW * STAGES * (MT + 1) * 2048;
-  auto kernel = gemm_skinny_kernel<MT, EPI, NW, 4, STAGES>;
+  constexpr int lds = NW * STAGES * (MT + G) * 2048;
+  auto kernel = gemm_skinny_kernel<MT, EPI, NW, 4, STAGES, G>;
   static const hipError_t room = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   TI_REQUIRE(room == hipSuccess, "gemm_bf16: %d bytes of LDS: %s", lds, hipGetErrorString(room));
-  kernel<<<grid, NW * 64, lds, s>>>(A, W, out, M, N, K, lda);
+  kernel<<<(grid + G - 1) / G, NW * 64, lds, s>>>(A, W, out, M, N, K, lda);
   return 0;
 }
 
+// Groups of 16 weight rows a workgroup of the staged kernel takes: two where the busiest compute unit then pulls in clearly less (its
+// workgroups' weight rows and, with each workgroup, all token rows).
+// Bound by what a unit pulls in, about 50 bytes a nanosecond.  us, one group and two, weights not in the caches: [gate; up] 6144 x 1024
+// at 23, 48 and 64 rows 5.65 7.10 8.08 and 4.88 5.73 6.36 (three 5.79 6.76 7.62); 6144 x 2560 at 20 and 64 10.6 16.9 and 9.2 13.0; [gate;
+// up] 24576 x 4096 at 20 and 48 41.8 56.9 and 37.5 43.6.  Equal where the loads are no less: 4096 x 2048, a workgroup a unit either way, 6.3
+// 8.5 and 6.7 9.5; up to 16 rows [gate; up] 24576 x 4096 34.1 and 37.6.  Where two groups leave all units one workgroup each, these rows
+// of memory collide (the K of the test; [gate; up] 8192 x 2048 at 17 and 40 rows 8.8 11.5 and 10.7 12.1, 8192 x 4096 15.7 20.1 and 19.6 20.9; but
+// 8192 x 2048 10.4 11.8 and 9.1 10.4).
+static int g_skinny_groups = 0;      // a hook for measurements: 1 or 2 forces them
+static int skinny_rounds(long groups, int G) { return (int)(((groups + G - 1) / G + compute_units() - 1) / compute_units()); }
+static int skinny_groups_for(int M, long groups, int K, bool swiglu) {
+  const int mt = (M + 15) / 16;
+  if (mt == 1) return 1;
+  if (g_skinny_groups) return g_skinny_groups;
+  if (M <= 48 && groups <= 2 * compute_units() && groups * 4 > 7 * compute_units() && K % 4096 == (swiglu ? 2048 : 0)) return 1;
+  return 20 * skinny_rounds(groups, 2) * (mt + 2) <= 17 * skinny_rounds(groups, 1) * (mt + 1) ? 2 : 1;
+}
 static int skinny_waves_for(int grid, int K);
 template <int EPI>
 static int launch_skinny(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda,
@@ -1775,18 +1811,31 @@ static int launch_skinny(const bf16_t* A, const bf16_t* W, void* out, int M, int
   // by the weight's shape only, so that a row's bits do not depend on the rows beside it; up to K = 4,096 and 16 rows as many as the
   // kernels with the norm in front take, so that those give the same bits
   if (waves == 0) waves = mt == 1 && K <= 4096 ? skinny_waves_for(grid, K) : (grid <= 128 && K >= 1024) ? 8 : 4;
+  if (mt > 4) waves = 4;
   const bool staged = (mt > 1 && staged_fits(K, lda)) || staged_16_serves(M, N, K, lda, EPI);
-#define TI_STAGED(MTV)                                                                                      \
-  if (mt == MTV && staged) {                                                                               \
-    if (waves == 8) return launch_skinny_staged<MTV, EPI, 8, 2>(A, W, out, M, N, K, lda, grid, s);          \
-    if (grid <= compute_units()) return launch_skinny_staged<MTV, EPI, 4, 4>(A, W, out, M, N, K, lda, grid, s); \
-    return launch_skinny_staged<MTV, EPI, 4, 2>(A, W, out, M, N, K, lda, grid, s);                          \
+  const int groups = waves == 4 ? skinny_groups_for(M, grid, K, EPI == TI_EPI_SWIGLU) : 1;
+  const bool alone = (grid + groups - 1) / groups <= compute_units();
+#define TI_GO(MTV, GV, ALONE) launch_skinny_staged<MTV, EPI, 4, skinny_stages(MTV, GV, ALONE), GV>(A, W, out, M, N, K, lda, grid, s)
+#define TI_STAGED(MTV)                                                                             \
+  if (mt == MTV && staged) {                                                                       \
+    if (waves == 8) return launch_skinny_staged<MTV, EPI, 8, 2>(A, W, out, M, N, K, lda, grid, s); \
+    if (MTV > 1 && groups == 2) return alone ? TI_GO((MTV > 1 ? MTV : 2), 2, true) : TI_GO((MTV > 1 ? MTV : 2), 2, false); \
+    return alone ? TI_GO(MTV, 1, true) : TI_GO(MTV, 1, false);                                     \
   }
   TI_STAGED(1)
   TI_STAGED(2)
   TI_STAGED(3)
   TI_STAGED(4)
 #undef TI_STAGED
+  if constexpr (EPI != TI_EPI_ADD_F32) {
+#define TI_MORE(MTV) \
+  if (mt == MTV) return groups == 2 ? TI_GO(MTV, 2, true) : TI_GO(MTV, 1, true);
+    TI_MORE(5)
+    TI_MORE(6)
+    TI_MORE(7)
+#undef TI_MORE
+  }
+#undef TI_GO
 #define TI_SKINNY(MTV)                                                               \
   if (mt == MTV) {                                                                   \
     if (waves == 8)                                                                  \
@@ -1859,6 +1908,28 @@ static bool large_weight(int M, int N, int K, int epi) {
   const long rows = (epi == TI_EPI_SWIGLU) ? 2L * N : (long)N;
   if (M <= 12 || M > 64 || K % PBK != 0) return false;
   return rows * K * M >= (M <= 16 ? g_tiled_from_16 : holds_out(M, rows, K, epi) ? g_tiled_from_stored : g_tiled_from);
+}
+// 17 to 112 rows, a product that stores: whether the kernel with its rows through LDS takes it where the line above, or that of 64 rows,
+// gave it to the tiles.  Up to 64 rows as long as two groups of weight rows a workgroup are one round of them (up to K = 4,095 the line
+// above let one group have most of these; us, tiles and this: 6144 x 4096 at 17, 40 and 64 rows 18.0 19.7 22.5 and 15.0 16.6 18.7, 7168 x 5120
+// 22.9 25.2 29.6 and 16.0 19.8 23.7, 4096 x 12288 46 53 62 and 22 30 37, [gate; up] 4096 x 4096 at 40 and 64 27.9 30.4 and 12.1 14.7, 8192 x 4096 at
+// 17, 40 and 64 19.7 21.1 23.7 and 15.8 19.9 22.7); beyond a round only [gate; up], whose tiles cost more (24576 x 4096 at 20, 40 and 64 44.1
+// 44.5 45.6 and 37.5 42.0 49.8; 34816 x 5120 at 20, 40 and 64 89 93 100 and 71 85 106; 19456 x 2560 at 20, 32 and 40 25.7 27.1 27.5 and 24.1 25.8 27.9;
+// 51200 x 5120, seven rounds, at 20 101.5 and 100.4; 12288 x 2048 without [gate; up] at 40 14.1 and 15.6).  65 to 112 rows, five to seven blocks of
+// them beside the tiles' two row tiles: a round of workgroups of one group (4096 x 1024 at 65, 77 and 112 6.8 6.8 7.2 and 5.4 5.5 6.7; 4096 x
+// 4096 17.6 17.9 19.6 and 14.2 14.7 18.3; 1024 x 1024 6.7 at 65, 6.9 at 112 and 5.1, 6.3) or, for [gate; up], two (6144 x 1024 9.1 9.2 10.0 and 6.9 7.0
+// 8.7; 8192 x 2560 22.0 at 77, 23.8 at 100 and 15.6, 18.6); without [gate; up] two groups lose from 77 on (6144 x 2560 13.9
+// and 14.5).  K of 256 and more, so that each of the four wavefronts has a chunk (1024 x 256 at 77 rows 3.6 and 2.7, 4096 x 256 4.1 and 3.3).
+static int g_rows_112 = 1;      // a hook for measurements: 0: only the line above
+static bool staged_112_serves(int M, int N, int K, long lda, int epi) {
+  if (!g_rows_112 || !g_use_pipelined || g_force_tile || g_tiled_from_stored != TILED_FROM_STORED || M <= 16 || M > 112 || epi == TI_EPI_ADD_F32 ||
+      !staged_fits(K, lda) || (M > 64 && lda >= (1L << 23)))      // (112 rows within 2 GiB)
+    return false;
+  const long units = compute_units(), groups = epi == TI_EPI_SWIGLU ? (N + 7) / 8 : (N + 15) / 16;
+  if (M > 64) return K >= 256 && groups <= (epi == TI_EPI_SWIGLU ? 2 : 1) * units;
+  if (groups <= 2 * units) return true;
+  const int rounds = skinny_rounds(groups, 2);
+  return epi == TI_EPI_SWIGLU && rounds <= 5 && M <= (K >= 4096 || rounds == 2 ? 48 : 32);
 }
 
 // 1 (default): up to GR_MMAX tokens and a weight of fewer than GR_ROWS_BELOW rows take the kernel
@@ -2609,7 +2680,7 @@ extern "C" int ti_gemm_bf16(const void* A, const void* W, void* out, int M, int 
   if (M == 0) return 0;
   const bf16_t* a = (const bf16_t*)A;
   const bf16_t* w = (const bf16_t*)W;
-  const bool skinny = M <= 64 && !(large_weight(M, N, K, epi) && g_use_pipelined);
+  const bool skinny = (M <= 64 && !(large_weight(M, N, K, epi) && g_use_pipelined)) || staged_112_serves(M, N, K, lda, epi);
   const bool staged = staged_16_serves(M, N, K, lda, epi) && (skinny || pieces_serves(M, N, K, epi));
   const bool copied = !staged && g_skinny_copy && M <= 16 && K % 64 == 0 && K <= 4096 && skinny;
   if (!staged && pieces_serves(M, N, K, epi)) {
@@ -2675,7 +2746,7 @@ extern "C" int ti_gemm_bf16(const void* A, const void* W, void* out, int M, int 
 extern "C" void ti_tuning_reset() {
   g_xcd_rows = 0; g_die_order = 1; g_tiles_160 = 1; g_tiles_256 = 1; g_two_ranges = 1; g_qkv_rows = 0; g_qkv_min_rows = 17; g_force_tile = 0; g_skinny_waves = 0;
   g_skinny_deep = 1; g_use_pipelined = 1; set_tiled_from(280L << 20); g_tiled_from_stored = TILED_FROM_STORED; g_row_per_wave = 1; g_rows_staged = 1;
-  g_normed_weight_below = NORMED_WEIGHT_BELOW; g_normed_groups = 0; g_skinny_copy = 1; g_wide_rows = 1; g_pieces = 1; g_add_split = 1;
+  g_normed_weight_below = NORMED_WEIGHT_BELOW; g_normed_groups = 0; g_skinny_groups = 0; g_rows_112 = 1; g_skinny_copy = 1; g_wide_rows = 1; g_pieces = 1; g_add_split = 1;
   g_rows_direct = 1;
   g_wide_rows_min_n = WIDE_ROWS_MIN_N;
   g_wide_rows_grid = 0;
@@ -2685,6 +2756,8 @@ extern "C" int ti_tuning_set(const char* name, long value) {
   if (n == "force_tile") g_force_tile = (int)value;
   else if (n == "normed_groups") g_normed_groups = (int)value;
   else if (n == "normed_weight_below") g_normed_weight_below = value > 0 ? value : NORMED_WEIGHT_BELOW;
+  else if (n == "skinny_groups") g_skinny_groups = (int)value;
+  else if (n == "rows_112") g_rows_112 = (int)value;
   else if (n == "tiles_160") g_tiles_160 = (int)value;
   else if (n == "tiles_256") g_tiles_256 = (int)value;
   else if (n == "two_ranges") g_two_ranges = (int)value;

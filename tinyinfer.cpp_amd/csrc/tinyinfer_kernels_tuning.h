@@ -21,10 +21,12 @@
 //   qkv_prep_rows        64 / 128 / 256: the rows of ti_gemm_bf16_qkv_prep's tile; 0: by the shape
 //   wide_rows            0: 17..64 rows times a weight of 16,384 rows or more take the other kernels
 //   tiled_from           17..64 rows x weight elements from which they take the tiled kernels (280 Mi; 1000 Mi for a product that
-//                        stores, K below 4096 and few enough workgroups of 16 rows: set, it holds for both)
+//                        stores, K below 4096 and few enough workgroups of 16 rows: set, it holds for both, and rows_112 is off)
 //   add_split            0: ti_gemm_bf16_add_split serves nothing
 //   use_pipelined        0: the plain tiled kernel for every K
 //   row_per_wave         0: few tokens and a weight of few rows take the 16-row kernels too
+//   skinny_groups        1 or 2 groups of 16 weight rows a workgroup where 17 to 112 rows come through LDS (0: by the shape)
+//   rows_112             0: above 64 rows, and where the weight is large from 17 on, every product takes the tiles
 //   rows_staged          0: up to 16 rows never take the kernel whose rows come through LDS stages of each wavefront's own
 //   skinny_copy          0: up to 16 tokens, fragments of the token rows straight from memory
 //   pieces               0: up to 16 rows never take the kernel with the token rows in pieces
