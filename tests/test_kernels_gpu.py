@@ -84,6 +84,22 @@ def test_rmsnorm_wide_rows(ops, dtype, H):
     assert torch.equal(some, out[rows.long()])
 
 
+@pytest.mark.parametrize("H", [4, 1024, 1028, 2048, 2052, 3072, 3076, 4092, 4096])
+def test_rmsnorm_rows_of_a_wavefront(ops, H):
+    """Widths on either side of each number of pieces a wavefront keeps, a last workgroup of one row, rows in another order: the reference's values, and a row's bits whatever the rows beside it."""
+    g = torch.Generator().manual_seed(H)
+    x, w = torch.randn(1025, H, generator=g), 1 + 0.1 * torch.randn(H, generator=g)
+    ref = ref_rmsnorm(x, w, 1e-6)
+    rows = torch.tensor([1024, 0, 3, 511, 3], dtype=torch.int32)
+    for dtype, tol in ((torch.float32, 1e-5), (torch.bfloat16, 2.0 ** -7)):      # relative; bfloat16 keeps 8 bits
+        many = torch.empty(1025, H, device="cuda", dtype=dtype)
+        ops.rmsnorm(dev(x), dev(w), 1e-6, many)
+        assert ((f64(many) - ref).abs() <= tol * ref.abs() + 1e-6).all()
+        few = torch.full((6, H), 7.0, device="cuda", dtype=dtype)
+        ops.rmsnorm(dev(x), dev(w), 1e-6, few[:5], dev(rows))
+        assert torch.equal(few[:5].cpu(), many.cpu()[rows.long()]) and bool((few[5] == 7.0).all())
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_rmsnorm_gather_odd_width(ops, dtype):
     g = torch.Generator().manual_seed(3)
