@@ -743,6 +743,8 @@ int Ops::decode_splits(int n_rows, int kv_heads, int heads, int context, int typ
 // 36 27.1, 27 25.0; 32 equal runs of them would be 24).  Beside portions eight wavefronts walk a run at 0.2 a block.  Where units hold two runs
 // and others one (33 to 48 rows of 8 heads for keys on 256 units) a block of both takes 0.51: 33 whole rows of 63, 188 and 376 blocks 38, 103 and 199,
 // so that such rows may be cut (33 rows of 3,000 and 6,000 tokens 3,813 and 6,504 us a step whole, 3,334 and 5,214 in three and five runs each).
+// (These are of the decode kernel that read keys and values straight into registers.  For the one through LDS they choose within 1.6 % of the
+// best, refitted to it within 1.5 %: left.)
 static const double RUN_START_US = 6.0, RUN_MERGE_US = 2.7, RUN_BLOCK_US = 0.147, RUN_BLOCK_BESIDE_US = 0.2, RUN_BYTES_US = 6.4e6;
 static const double RUN_BLOCK_SHARED_US = 0.257;
 static const double RUN_MERGE_MANY_US = 3.5;  // rows on more than a round of the units: 33 of 400 tokens are better whole, 48 of 3,000 in two
