@@ -1764,6 +1764,58 @@ def test_decode_records_through_lds(ops, hd, P, nh, nkv, window, stages):
     assert torch.equal(got, want) and torch.equal(staged, straight)
 
 
+def fused_multiply_add(a, b, c):
+    """a b + c of float32 arrays, rounded once."""
+    p, c = a.astype(np.float64) * b.astype(np.float64), c.astype(np.float64)      # 48 bits: exact
+    s = p + c
+    err = (p - (s - (s - p))) + (c - (s - p))                                     # what the sum left out
+    tie = (s.view(np.int64) & ((1 << 29) - 1)) == 1 << 28                         # halfway between two float32: the rest decides
+    return np.where(tie & (err != 0), np.nextafter(s, np.copysign(np.inf, err)), s).astype(np.float32)
+
+
+@pytest.mark.parametrize("shift", range(4))
+@pytest.mark.parametrize("hd", [64, 128])
+def test_prompt_attention_merges_its_groups_in_ascending_order(ops, hd, shift):
+    """Four groups of wavefronts take the turns of 32 keys in rotation and each of them owns a quarter of a lane's values: its own are scaled
+    first, then the other groups' are added in ascending order, each by one multiply-add.  The keys of a group are one vector with a power of two,
+    so that its maximum, sum and outputs are exact and the merge is all that rounds; two runs of keys, whose first leaves its results in 32 bits."""
+    nh, P, start, n_tok, scale = 2, 16, 512, 64, 0.37
+    g = torch.Generator().manual_seed(hd + shift)
+    blocks = (start + n_tok) // 16
+    scores = np.roll(np.array([1, 0.5, 4, 2], dtype=np.float32), shift)
+    values = torch.randn(4, hd, generator=g).to(torch.bfloat16)
+    pool = torch.zeros(blocks, 2, P, hd, dtype=torch.bfloat16)
+    for b in range(blocks):
+        pool[b, 0, :, 0] = float(scores[b // 2 % 4])
+        pool[b, 1] = values[b // 2 % 4].unsqueeze(1).expand(hd, P).reshape(P, hd)      # (values: [hd][P])
+    q = torch.zeros(n_tok, nh, hd, dtype=torch.bfloat16)
+    q[:, :, 0] = 1
+    q, pool, table = dev(q), dev(pool), dev(torch.arange(blocks, dtype=torch.int32).unsqueeze(0))
+    tiles, entries = dev(torch.tensor([[0, 0]], dtype=torch.int32)), dev(torch.tensor([[0, n_tok, start, 0]], dtype=torch.int32))
+    out = torch.empty(n_tok, nh * hd, device="cuda", dtype=torch.bfloat16)
+    part_o, part_ml = torch.full((n_tok, nh, 2, hd), 7.0, device="cuda"), torch.full((n_tok, nh, 2, 2), 7.0, device="cuda")
+    lib, ptr = ops.lib("attention_bf16"), lambda t: t.data_ptr()
+    rc = lib.ti_attention_prefill_paired_bf16(ptr(q), ptr(pool), ptr(table), blocks, ptr(tiles), ptr(entries), ptr(out), 1, nh, 1, hd, P, scale, 0,
+                                              n_tok, ptr(part_o), ptr(part_ml), 2, 0, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.ti_last_error()
+    # the first run: 18 blocks, 9 turns, of which group 0 has three
+    count = np.array([96, 64, 64, 64], dtype=np.float32)
+    m = scores * (np.float32(scale) * np.float32(1.4426950408889634))
+    a = torch.exp2(dev(torch.from_numpy(m - m.max()))).cpu().numpy()
+    o = count[:, None] * values.float().numpy()
+    half = np.float32(0)
+    for k in range(4):
+        half = fused_multiply_add(count[k:k + 1] / 2, a[k:k + 1], np.full(1, half, np.float32))[0]
+    dim = np.arange(hd)
+    owner = (dim // 32 * 16 + dim % 32 // 8 * 4) // (hd // 8)      # a lane holds four consecutive dims of every eight, hd / 2 values, a quarter a group's
+    want = o[owner, dim] * a[owner]
+    for k in range(4):
+        want = np.where(owner == k, want, fused_multiply_add(o[k], np.full(hd, a[k]), want))
+    got, ml = part_o[:, :, 0].cpu().numpy(), part_ml[:, :, 0].cpu().numpy()
+    assert np.array_equal(ml, np.broadcast_to(np.array([m.max(), 2 * half], np.float32), ml.shape))
+    assert np.array_equal(got, np.broadcast_to(want, got.shape)), int((got != want).sum())
+
+
 class FakeCtx:
     """The fields of a step context that the attention dispatch reads."""
 

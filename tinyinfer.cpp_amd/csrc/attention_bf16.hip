@@ -1603,7 +1603,8 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
     // The groups merge their partial results through LDS (the stages are free now), each group the
     // values it owns: values VPG g .. VPG (g + 1) - 1 of every lane are group g's.  A group leaves the
     // values it does not own (in their order, four to a slot of 16 bytes a lane), its maximum and its sum in its part of LDS; after a
-    // barrier it reads the others' contributions to its own values, merges them with its own and
+    // barrier it reads the others' contributions to its own values, adds them to its own (scaled first) in the order of the groups, each by
+    // one multiply-add (written out: left to the compiler, which product of a sum is rounded first changes with the code around it), and
     // writes them out.  The code stands once for each group, so that which registers these are is known where it is compiled (as a
     // choice between registers by the group's number, value by value, a tile's end took 4,400 cycles; 2,048 tokens 38.0 us, now 36.4, 77 7.5,
     // now 7.05, 2,048 at 32 heads 73.2, now 70.0).
@@ -1645,7 +1646,7 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
         a_g[g] = __builtin_amdgcn_exp2f(ml[g].x - m_safe);
-        l_all += ml[g].y * a_g[g];
+        l_all = fmaf(ml[g].y, a_g[g], l_all);
       }
       const float a_own = __builtin_amdgcn_exp2f(mx[cb] - m_safe);
       float val[VPG];
@@ -1655,7 +1656,7 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
       for (int g = 0; g < NG; ++g)
 #pragma unroll
         for (int j = 0; j < VPG; ++j)
-          if (g != G) val[j] += theirs[g][j / 4][j % 4] * a_g[g];
+          if (g != G) val[j] = fmaf(theirs[g][j / 4][j % 4], a_g[g], val[j]);
       write_out(cb, val, FIRST, std::integral_constant<int, VPG>{}, m_all, l_all + __shfl_xor(l_all, 32, 64));
     };
 #pragma unroll
