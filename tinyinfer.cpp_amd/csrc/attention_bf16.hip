@@ -561,10 +561,11 @@ __device__ __forceinline__ float sink_join(const float* __restrict__ sink, int h
 }
 
 #define DEC_TABLE_LDS 1024     // entries of a block-table row that the decode kernel can hold in LDS
-// The workgroup's LDS: what its NW wavefronts leave for the merge (a column's HD values in a row), and their maxima and sums.
+// The workgroup's LDS: what its NW wavefronts leave for the merge (a column's HD values in a row of HD + 4: sixteen lanes write 16 bytes of as
+// many columns at once, and rows of HD floats would put them all into the same banks), and their maxima and sums.
 template <int HD, int NW>
 struct DecodeMerge {
-  float o[NW][16][HD];
+  float o[NW][16][HD + 4];
   float2 ml[NW][16];
 };
 // The same where the operands come through LDS stages: a wavefront leaves its outputs in its own first stage.
@@ -572,7 +573,7 @@ template <int HD, int NW, int ST>
 struct StagedMerge {
   union {
     unsigned char stages[ST][StagedPairs<HD>::BYTES];
-    float o[16][HD];
+    float o[16][HD + 4];
   } w[NW];
   float2 ml[NW][16];
   bf16_t q[16][HD], kv[2][HD];      // the query heads, the row's own key and value (16-byte aligned)
@@ -607,7 +608,7 @@ decode_run(Shared& sm, int ridx, int y, int split, const bf16_t* __restrict__ q,
            const float* __restrict__ sink, DecodeRuns by = DecodeRuns{nullptr, 0}, int group = 0) {
   static_assert(!PREP || NW == 4, "the preparation is written for four wavefronts");
   constexpr bool RUNS = ST > 0;
-  auto s_o = [&](int w) -> float(&)[16][HD] {
+  auto s_o = [&](int w) -> float(&)[16][HD + 4] {
     if constexpr (ST > 0) return sm.w[w].o;
     else return sm.o[w];
   };
@@ -835,13 +836,14 @@ decode_run(Shared& sm, int ridx, int y, int split, const bf16_t* __restrict__ q,
       walk_blocks<HD>(kv, qf, b0 + wave, NW, mine, lo, p_q, p_q, scale * TI_LOG2E, edge, mx, l, o, NoHook{}, NoHook{},
                       softcap * TI_LOG2E);
   }
-  {
-    const LanePair p = lane_pair<16>(l);
-    l = p.a + p.b;
-  }
-  {
-    const LanePair p = lane_pair<32>(l);
-    l = p.a + p.b;
+  if constexpr (ST > 0) {
+    const LanePair near = lane_pair<16>(l);
+    l = near.a + near.b;
+    const LanePair far = lane_pair<32>(l);
+    l = far.a + far.b;
+  } else {      // (with the lanes swapped as above the compiler takes 19 to 34 registers more: at a head size of 64 three wavefronts a SIMD, not four)
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
   }
 
   // merge the wavefronts: what the columns in use hold, four values of a column a thread.  (A wavefront's dims of all sixteen columns,
