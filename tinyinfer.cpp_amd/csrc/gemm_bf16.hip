@@ -195,18 +195,17 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
     const int m = t * 16 + tok;
     if (m >= M) continue;
     if (SW) {
+      static_assert(G <= 2, "a thread a column");
+      if (row >= 8 * G) continue;
+      const int n = blockIdx.x * 8 * G + row, at = G > 1 ? row >> 3 : 0;
+      if (n >= N) continue;
+      float g = 0.f, u = 0.f;
 #pragma unroll
-      for (int c = row; c < 8 * G; c += 16) {
-        const int n = blockIdx.x * 8 * G + c;
-        if (n >= N) continue;
-        float g = 0.f, u = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-          g += red(w, c >> 3, t, tok, c & 7);
-          u += red(w, c >> 3, t, tok, (c & 7) + 8);
-        }
-        ((bf16_t*)out_)[(size_t)m * N + n] = f2bf(silu_mul(g, u));
+      for (int w = 0; w < NW; ++w) {
+        g += red(w, at, t, tok, row & 7);
+        u += red(w, at, t, tok, (row & 7) + 8);
       }
+      ((bf16_t*)out_)[(size_t)m * N + n] = f2bf(silu_mul(g, u));
     } else {
 #pragma unroll
       for (int g = 0; g < G; ++g) {
