@@ -1786,18 +1786,30 @@ static int launch_skinny_staged(const bf16_t* A, const bf16_t* W, void* out, int
 // Groups of 16 weight rows a workgroup of the staged kernel takes: two where the busiest compute unit then pulls in clearly less (its
 // workgroups' weight rows and, with each workgroup, all token rows).
 // Bound by what a unit pulls in, about 50 bytes a nanosecond.  us, one group and two, weights not in the caches: [gate; up] 6144 x 1024
-// at 23, 48 and 64 rows 5.65 7.10 8.08 and 4.88 5.73 6.36 (three 5.79 6.76 7.62); 6144 x 2560 at 20 and 64 10.6 16.9 and 9.2 13.0; [gate;
+// at 17, 32, 48 and 64 rows 5.4 5.9 7.1 8.1 and 4.8 5.2 6.0 6.5 (three at 64 7.6); 6144 x 2560 at 20 and 64 10.6 16.9 and 9.2 13.0; [gate;
 // up] 24576 x 4096 at 20 and 48 41.8 56.9 and 37.5 43.6.  Equal where the loads are no less: 4096 x 2048, a workgroup a unit either way, 6.3
-// 8.5 and 6.7 9.5; up to 16 rows [gate; up] 24576 x 4096 34.1 and 37.6.  Where two groups leave all units one workgroup each, these rows
+// 8.5 and 6.7 9.5; up to 16 rows [gate; up] 24576 x 4096 34.1 and 37.6.
+// Where sums are stored as they are, a short K is starts and ends: two groups only where fewer workgroups then follow one another on a unit (6144 x
+// 256 at 17 and 64 rows, a turn either way, 2.80 3.76 and 3.07 3.77, 8192 x 64 2.23 2.71 and 2.41 3.12; 12288 x 256 at 48, two turns and one, 5.4 and
+// 4.4, at 64, two either way, 6.3 and 6.5); from K = 640 on, 384 from 33 rows on, the bytes decide (6144 x 640 at 17 and 64 4.0 6.2 and 3.9 5.4).
+// Where two groups leave all units one workgroup each, these rows
 // of memory collide (the K of the test; [gate; up] 8192 x 2048 at 17 and 40 rows 8.8 11.5 and 10.7 12.1, 8192 x 4096 15.7 20.1 and 19.6 20.9; but
 // 8192 x 2048 10.4 11.8 and 9.1 10.4).
 static int g_skinny_groups = 0;      // a hook for measurements: 1 or 2 forces them
 static int skinny_rounds(long groups, int G) { return (int)(((groups + G - 1) / G + compute_units() - 1) / compute_units()); }
+// how many workgroups of G groups follow one another in a unit's place, as many side by side as its LDS holds
+static int skinny_turns(int mt, long groups, int G) {
+  const long n = (groups + G - 1) / G, units = compute_units();
+  if (n <= units) return 1;
+  const long beside = units * (160 * 1024 / (skinny_stages(mt, G, false) * 4 * (mt + G) * 2048));
+  return (int)((n + beside - 1) / beside);
+}
 static int skinny_groups_for(int M, long groups, int K, bool swiglu) {
   const int mt = (M + 15) / 16;
   if (mt == 1) return 1;
   if (g_skinny_groups) return g_skinny_groups;
   if (M <= 48 && groups <= 2 * compute_units() && groups * 4 > 7 * compute_units() && K % 4096 == (swiglu ? 2048 : 0)) return 1;
+  if (!swiglu && K < (mt == 2 ? 640 : 384)) return skinny_turns(mt, groups, 2) < skinny_turns(mt, groups, 1) ? 2 : 1;
   return 20 * skinny_rounds(groups, 2) * (mt + 2) <= 17 * skinny_rounds(groups, 1) * (mt + 1) ? 2 : 1;
 }
 static int skinny_waves_for(int grid, int K);
