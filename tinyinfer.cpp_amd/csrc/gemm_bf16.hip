@@ -1792,9 +1792,9 @@ static int launch_skinny_staged(const bf16_t* A, const bf16_t* W, void* out, int
 // Where sums are stored as they are, a short K is starts and ends: two groups only where fewer workgroups then follow one another on a unit (6144 x
 // 256 at 17 and 64 rows, a turn either way, 2.80 3.76 and 3.07 3.77, 8192 x 64 2.23 2.71 and 2.41 3.12; 12288 x 256 at 48, two turns and one, 5.4 and
 // 4.4, at 64, two either way, 6.3 and 6.5); from K = 640 on, 384 from 33 rows on, the bytes decide (6144 x 640 at 17 and 64 4.0 6.2 and 3.9 5.4).
-// Where two groups leave all units one workgroup each, these rows
-// of memory collide (the K of the test; [gate; up] 8192 x 2048 at 17 and 40 rows 8.8 11.5 and 10.7 12.1, 8192 x 4096 15.7 20.1 and 19.6 20.9; but
-// 8192 x 2048 10.4 11.8 and 9.1 10.4).
+// Row strides of 4 KiB and more that are powers of two cost two groups up to a fifth, and up to 32 rows they lose by it where they
+// leave nearly every unit a workgroup: 8192 x 4096 at 17, 32 and 48 15.4 17.2 20.1 and 16.5 16.9 18.1, 8192 x 8192 28.3 32.6 37.8 and 34.1 34.5 36.0,
+// [gate; up] 8192 x 2048 9.0 10.4 12.2 and 9.3 9.7 11.0.  Strides of 12, 20 and 24 KiB do not: no rule here.
 static int g_skinny_groups = 0;      // a hook for measurements: 1 or 2 forces them
 static int skinny_rounds(long groups, int G) { return (int)(((groups + G - 1) / G + compute_units() - 1) / compute_units()); }
 // how many workgroups of G groups follow one another in a unit's place, as many side by side as its LDS holds
@@ -1808,7 +1808,6 @@ static int skinny_groups_for(int M, long groups, int K, bool swiglu) {
   const int mt = (M + 15) / 16;
   if (mt == 1) return 1;
   if (g_skinny_groups) return g_skinny_groups;
-  if (M <= 48 && groups <= 2 * compute_units() && groups * 4 > 7 * compute_units() && K % 4096 == (swiglu ? 2048 : 0)) return 1;
   if (!swiglu && K < (mt == 2 ? 640 : 384)) return skinny_turns(mt, groups, 2) < skinny_turns(mt, groups, 1) ? 2 : 1;
   return 20 * skinny_rounds(groups, 2) * (mt + 2) <= 17 * skinny_rounds(groups, 1) * (mt + 1) ? 2 : 1;
 }
