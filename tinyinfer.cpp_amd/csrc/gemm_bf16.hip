@@ -1838,8 +1838,9 @@ static int launch_skinny(const bf16_t* A, const bf16_t* W, void* out, int M, int
   TI_STAGED(4)
 #undef TI_STAGED
   if constexpr (EPI != TI_EPI_ADD_F32) {
+    constexpr int MORE = EPI == TI_EPI_SWIGLU ? 2 : 1;      // more than a round of single groups: [gate; up] alone (staged_112_serves)
 #define TI_MORE(MTV) \
-  if (mt == MTV) return groups == 2 ? TI_GO(MTV, 2, true) : TI_GO(MTV, 1, true);
+  if (mt == MTV) return groups == 2 ? TI_GO(MTV, MORE, true) : TI_GO(MTV, 1, true);
     TI_MORE(5)
     TI_MORE(6)
     TI_MORE(7)
@@ -2038,8 +2039,7 @@ static int launch_normed_groups(const float* x, const float* nw, float eps, cons
   if (groups == 3 && normed_lds(M, K, 12, 4) > NORMED_LDS) groups = 2;
   if (groups == 3) return launch_normed<KC, EPI, 4, 3, 4>(x, nw, eps, w, out, M, N, K, tiles, stream);
   if (groups == 2) return launch_normed<KC, EPI, 4, 2, 4>(x, nw, eps, w, out, M, N, K, tiles, stream);
-  if (K > 1024) return launch_normed<KC, EPI, 4, 1, 8>(x, nw, eps, w, out, M, N, K, tiles, stream);
-  return launch_normed<KC, EPI, 4, 1, 4>(x, nw, eps, w, out, M, N, K, tiles, stream);
+  return launch_normed<KC, EPI, 4, 1, KC == 4 ? 4 : 8>(x, nw, eps, w, out, M, N, K, tiles, stream);
 }
 
 static bool pieces_serves(int M, int N, int K, int epi);
