@@ -1162,38 +1162,51 @@ def test_linear_bf16_rows_through_lds_up_to_16_rows(ops, M, N, K):
     assert (f64(outs[1][0][:M]) - ref_linear(a.cpu(), w.cpu())).abs().max() < 2e-5 * K
 
 
-@pytest.mark.parametrize("M,N,K", [(17, 8184, 4160), (33, 6168, 1088), (48, 4104, 2048), (49, 8192, 2048), (64, 4112, 64), (64, 40, 4160), (65, 4096, 128),
-                                   (77, 2056, 1088), (80, 24, 64), (81, 6152, 320), (112, 4088, 2112)])
+@pytest.mark.parametrize("M,N,K", [(17, 8184, 4160), (33, 6168, 1088), (48, 4104, 2048), (48, 12280, 128), (49, 8192, 2048), (64, 4112, 64), (64, 40, 4160),
+                                   (65, 4096, 256), (77, 2056, 1088), (80, 24, 256), (81, 4088, 320), (81, 6152, 320), (112, 4088, 2112), (112, 8176, 576),
+                                   (113, 1024, 256), (65, 1024, 192)])
 def test_linear_bf16_rows_through_lds_up_to_112_rows(ops, M, N, K):
     """One and two groups of weight rows a workgroup: a last workgroup whose second group has few rows or none, four and eight wavefronts,
-    fewer steps than stages and than wavefronts, a first and a last row of a block of 16.  The groups change no bit, the values are
-    float64's within the bound of 32-bit sums, and what lies beyond the rows is left."""
+    fewer steps than stages, a first and a last row of a block of 16, and sizes on either side of the rule above 64 rows.  The groups change no
+    bit, the values are float64's within the bound of 32-bit sums, with the rule and without it, and what lies beyond the rows is left.  The
+    kernel's own entry point: `linear` cuts some of these over K."""
+    from tinyinfer_amd.ops.kernels import EPI
     g = torch.Generator().manual_seed(M + N + K)
     a = dev((torch.rand(M, K + 8, generator=g) * 2 - 1).to(torch.bfloat16))[:, :K]
     w = dev((torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16))
     lib, outs = ops.lib("gemm_bf16"), {}
+    ref = ref_linear(a.cpu(), w.cpu())
+    gate, up = ref[:, :N // 2], ref[:, N // 2:]
+    ref_pair = gate / (1 + torch.exp(-gate)) * up
     lib.ti_tuning_reset()
     try:
-        for groups in (0, 1, 2):
+        for groups, rule in ((0, 1), (1, 1), (2, 1), (0, 0)):
             lib.ti_tuning_set(b"skinny_groups", groups)
+            lib.ti_tuning_set(b"rows_112", rule)
             res = [torch.full((M + 1, N if e != "swiglu" else N // 2), 7.0, device="cuda", dtype=torch.float32 if e == "store" else torch.bfloat16)
                    for e in ("store", "store_act", "swiglu")]
             for out, e in zip(res, ("store", "store_act", "swiglu")):
-                ops.linear(a, w, out[:M], e)
-            outs[groups] = res
+                rc = lib.ti_gemm_bf16(a.data_ptr(), w.data_ptr(), out.data_ptr(), M, out.shape[1], K, K + 8, EPI[e],
+                                      torch.cuda.current_stream().cuda_stream)
+                assert rc == 0, lib.ti_last_error()
+            outs[groups, rule] = res
     finally:
         lib.ti_tuning_reset()
     for groups in (1, 2):
-        for x, y in zip(outs[0], outs[groups]):
+        for x, y in zip(outs[0, 1], outs[groups, 1]):
             assert torch.equal(x, y), groups
-    store, act, pair = (f64(x) for x in outs[0])
-    assert bool((store[M] == 7.0).all()) and bool((act[M] == 7.0).all()) and bool((pair[M] == 7.0).all())
-    ref = ref_linear(a.cpu(), w.cpu())
-    assert (store[:M] - ref).abs().max() < 2e-5 * K
-    assert (act[:M] - ref).abs().max() < 0.005 * ref.abs().max() + 2e-5 * K
-    gate, up = ref[:, :N // 2], ref[:, N // 2:]
-    ref = gate / (1 + torch.exp(-gate)) * up
-    assert (pair[:M] - ref).abs().max() < 0.005 * ref.abs().max() + 10 * 2e-5 * K
+    # above 64 rows the rule takes products of one round of workgroups from the tiles: other sums, and elsewhere the same ones
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    if M > 64:
+        by_rule = [65 <= M <= 112 and K >= 256 and groups <= rounds * units for groups, rounds in (((N + 15) // 16, 1), ((N // 2 + 7) // 8, 2))]
+        assert torch.equal(outs[0, 1][0], outs[0, 0][0]) != by_rule[0]
+        assert by_rule[1] or torch.equal(outs[0, 1][2], outs[0, 0][2])
+    for rule in (1, 0):
+        store, act, pair = (f64(x) for x in outs[0, rule])
+        assert bool((store[M] == 7.0).all()) and bool((act[M] == 7.0).all()) and bool((pair[M] == 7.0).all())
+        assert (store[:M] - ref).abs().max() < 2e-5 * K
+        assert (act[:M] - ref).abs().max() < 0.005 * ref.abs().max() + 2e-5 * K
+        assert (pair[:M] - ref_pair).abs().max() < 0.005 * ref_pair.abs().max() + 10 * 2e-5 * K
 
 
 @pytest.mark.parametrize("N,K,epi", [(2048, 4096, "store"), (2040, 4096, "store"), (2048, 4096, "swiglu"), (2048, 2048, "store"), (2064, 4096, "store")])
@@ -1671,13 +1684,13 @@ def test_linear_with_the_norm_inside_by_groups(ops, M, N, K):
 
 
 def test_linear_with_the_norm_inside_refuses_what_it_does_not_serve(ops):
-    """More rows than the kernel holds, a K that is no multiple of 64, or few tokens with a weight
-    of few rows (which another kernel takes): `linear` computes the norm first and the result
+    """More rows than the kernel holds, rows that do not fit into LDS beside the weights, a K that is no multiple of 64, or few tokens with
+    a weight of few rows (which another kernel takes): `linear` computes the norm first and the result
     is that of the norm kernel followed by the product."""
     from tinyinfer_amd.ops.kernels import NormedRows
     assert ops.use_fast_gemm, "the bfloat16 MFMA kernels are switched off or not built"
     g = torch.Generator().manual_seed(9)
-    for M, N, K in ((17, 32, 128), (4, 32, 72), (4, 32, 128), (8, 1024, 2048)):
+    for M, N, K in ((17, 32, 128), (4, 32, 72), (4, 32, 128), (8, 1024, 2048), (16, 6144, 4096), (16, 4104, 3072), (12, 4104, 4096)):
         x = dev(torch.randn(M, K, generator=g))
         nw = dev(1 + 0.1 * torch.randn(K, generator=g))
         w = dev((torch.rand(N, K, generator=g) * 2 - 1).to(torch.bfloat16))
@@ -1686,6 +1699,7 @@ def test_linear_with_the_norm_inside_refuses_what_it_does_not_serve(ops):
         two = torch.empty(M, N, device="cuda")
         ops.linear(h, w, two, "store")
         one = torch.empty(M, N, device="cuda")
+        assert not ops._linear_normed(NormedRows(x, nw, 1e-6, torch.empty_like(h)), w, one, "store")
         ops.linear(NormedRows(x, nw, 1e-6, torch.empty_like(h)), w, one, "store")
         assert torch.equal(one, two)
 
@@ -1719,12 +1733,12 @@ def test_decode_records_say_nothing_beyond_their_runs(ops, hd):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
-@pytest.mark.parametrize("stages", [1, 2])
-@pytest.mark.parametrize("hd,P,nh,nkv,window", [(128, 16, 16, 8, 0), (128, 48, 10, 2, 0), (64, 16, 16, 1, 0), (64, 64, 4, 2, 70), (128, 32, 3, 3, 40)])
+@pytest.mark.parametrize("hd,P,nh,nkv,window,stages", [(128, 16, 16, 8, 0, 1), (128, 16, 16, 8, 0, 2), (128, 48, 10, 2, 0, 1), (128, 48, 10, 2, 0, 2),
+                                                       (128, 32, 3, 3, 40, 1), (128, 32, 3, 3, 40, 2), (64, 16, 16, 1, 0, 2), (64, 64, 4, 2, 70, 2)])
 def test_decode_records_through_lds(ops, hd, P, nh, nkv, window, stages):
     """Keys and values through LDS stages: the bits, and the cache, of the kernel that takes them straight from memory.  Contexts around the
     edges of blocks, of pairs of them, of pages, and beyond the 64 blocks a wavefront holds the page ids of; page ids with the record and
-    behind it."""
+    behind it.  (A head size of 64 has two stages, whatever is asked for.)"""
     g = torch.Generator().manual_seed(hd + P)
     pos = [0, 1, 15, 16, 31, 32, 47, 63, 64, 65, 127, 128, 255, 257, 1000, 4500]
     n, each, width = len(pos), 6, (nh + 2 * nkv) * hd
