@@ -1778,6 +1778,54 @@ def test_decode_records_through_lds(ops, hd, P, nh, nkv, window, stages):
     assert torch.equal(got, want) and torch.equal(staged, straight)
 
 
+@pytest.mark.parametrize("hd,nh,nkv,window", [(128, 4, 2, 0), (128, 16, 1, 8300), (64, 2, 2, 8300), (64, 16, 1, 0)])
+def test_step_records_beyond_64_blocks_a_wavefront(ops, hd, nh, nkv, window):
+    """A portion and single tokens in one launch, the latter's eight wavefronts beyond the 64 blocks whose page ids they hold at once, at the
+    edge, and below it.  A key is seen in full or not at all (scores 0 and -200) and the values are small integers: sums and weights
+    are exact, so that a block lost, walked twice or paired with another's values shows in every dim."""
+    P, each, n_tok, pos = 16, 6, 5, [9000, 8191, 8192, 8207, 700]
+    g = torch.Generator().manual_seed(hd + nh)
+    need = [1] + [p // P + 1 for p in pos]
+    table = torch.zeros(len(need), max(need), dtype=torch.int32)
+    ids = torch.randperm(sum(need), generator=g).to(torch.int32)
+    for r, (a, k) in enumerate(zip(np.cumsum([0] + need), need)):
+        table[r, :k] = ids[a:a + k]
+    seen = torch.rand(sum(need), nkv, P, generator=g) < 0.5
+    seen[:, :, 0] = True
+    seen[int(table[0, 0])] = True
+    values = torch.randint(-8, 9, (sum(need), nkv, hd, P), generator=g)
+    keys = torch.randn(sum(need), nkv, P, hd, generator=g)
+    keys[..., 0] = torch.where(seen, 0.0, -200.0)
+    pool = torch.cat([keys.to(torch.bfloat16), values.to(torch.bfloat16).reshape(sum(need), nkv, P, hd)], dim=1)
+    q = torch.zeros(n_tok + len(pos), nh, hd, dtype=torch.bfloat16)
+    q[:, :, 0] = 1
+    runs = torch.full((len(pos), 8 + 8 * each), -1, dtype=torch.int32)
+    for r, p in enumerate(pos):
+        first = max(0, p - window + 1) // 16 if window else 0
+        blocks = p // 16 + 1 - first
+        runs[r, :8] = torch.tensor([n_tok + r, p, first, blocks, -1, 1 + r, int(table[1 + r, p // P]), 0])
+        for b in range(min(blocks, 8 * each)):
+            runs[r, 8 + (b % 8) * each + b // 8] = table[1 + r, first + b]
+    assert max(int(runs[r, 3]) for r in range(len(pos))) > 8 * 64
+    q, pool, tab, lists = dev(q), dev(pool), dev(table), dev(runs)
+    tiles, entries = dev(torch.tensor([[0, 0]], dtype=torch.int32)), dev(torch.tensor([[0, n_tok, 0, 0]], dtype=torch.int32))
+    out = torch.full((n_tok + len(pos), nh, hd), 7.0, device="cuda", dtype=torch.bfloat16)
+    lib, ptr = ops.lib("attention_bf16"), lambda t: t.data_ptr()
+    rc = lib.ti_attention_step_bf16(ptr(q), ptr(pool), ptr(tab), tab.shape[1], ptr(tiles), ptr(entries), 1, ptr(lists), len(pos), runs.shape[1], None, 0,
+                                    ptr(out), None, None, nh, nkv, hd, P, 1.0, 0.0, window, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.ti_last_error()
+    got = f64(out)
+    for row, (entry, p) in enumerate([(0, i) for i in range(n_tok)] + [(1 + i, p) for i, p in enumerate(pos)]):
+        k = torch.arange(max(0, p - window + 1) if window else 0, p + 1)
+        page, at = table[entry, k // P].long(), k % P
+        for h in range(nh):
+            kv = h // (nh // nkv)
+            m = seen[page, kv, at].double()
+            want = (values[page, kv, :, at].double() * m.unsqueeze(1)).sum(0) / m.sum()
+            # a division, a product and a rounding to 8 bits of an exact sum
+            assert (got[row, h] - want).abs().max() <= 2.0 ** -8 * want.abs().max(), (row, h)
+
+
 def fused_multiply_add(a, b, c):
     """a b + c of float32 arrays, rounded once."""
     p, c = a.astype(np.float64) * b.astype(np.float64), c.astype(np.float64)      # 48 bits: exact
