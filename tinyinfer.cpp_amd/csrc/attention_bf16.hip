@@ -5,12 +5,15 @@
 //
 // Both walk the cache in blocks of 16 positions.  A page holds keys as
 // [row][head_dim] and values transposed as [head_dim][row], so both products
-// read their operands along the dimension they reduce over, straight from memory:
+// read their operands along the dimension they reduce over.  Launches by records (what an
+// engine's decode steps take) and the prompt kernel for head sizes 64 and 128, which works on
+// tiles of 32 x 32, bring them through LDS by direct loads; decode by equal runs and the
+// prompt kernel for head size 32 read them straight from memory.  A tile of 16 columns:
 //   S^T (16 keys x 16 columns)  = K (16 x hd) . Q^T          v_mfma_f32_16x16x32_bf16
 //   O^T (hd x 16 columns)      += V^T (hd x 16 keys) . P^T   v_mfma_f32_16x16x16_bf16
 // The transposed score tile leaves each lane with four keys of one column, which
-// is exactly the operand layout the second product wants for P^T: no shuffles,
-// no LDS between the two.  The softmax statistics of a column are one scalar per
+// is exactly the operand layout the second product wants for P^T: no shuffles and
+// no LDS between the two products.  The softmax statistics of a column are one scalar per
 // lane; scores, statistics and outputs are 32-bit.
 //
 // What the 16 columns are differs:
@@ -2007,7 +2010,7 @@ extern "C" int ti_attention_decode_runs_bf16(const float* qkv, int row_width, co
       runs, run_stride, n_head / n_kv, qkv, row_width, n_kv, (const float2*)rope_table, (const bf16_t*)pool, page_size, table_len, \
       q_w, k_w, table, table_stride, window, inv_freq, write_kv ? (bf16_t*)pool : nullptr, eps, scale, (bf16_t*)out, part_o, part_ml)
   if (hd == 64) TI_GO(64, 2);
-  // two stages (136 KiB) where a unit has one workgroup at most; one (70 KiB) where two share it, so that one walks while the other starts
+  // two stages (133 KiB) where a unit has one workgroup at most; one (69 KiB) where two share it, so that one walks while the other starts
   else if (g_decode_stages ? g_decode_stages == 2 : n_kv * n_runs <= compute_units()) TI_GO(128, 2);
   else TI_GO(128, 1);
 #undef TI_GO

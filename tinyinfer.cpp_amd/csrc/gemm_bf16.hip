@@ -1818,7 +1818,8 @@ static int launch_skinny(const bf16_t* A, const bf16_t* W, void* out, int M, int
   const int grid = (EPI == TI_EPI_SWIGLU) ? (N + 7) / 8 : (N + 15) / 16;
   const int mt = (M + 15) / 16;
   int waves = g_skinny_waves;
-  // by the weight's shape only, so that a row's bits do not depend on the rows beside it; up to K = 4,096 and 16 rows as many as the
+  // by the weight's shape only, so that a row's bits do not depend on the rows beside it (up to 64 of them: above, where the tiles had
+  // them and a row's bits changed too, four wavefronts are what LDS has room for); up to K = 4,096 and 16 rows as many as the
   // kernels with the norm in front take, so that those give the same bits
   if (waves == 0) waves = mt == 1 && K <= 4096 ? skinny_waves_for(grid, K) : (grid <= 128 && K >= 1024) ? 8 : 4;
   if (mt > 4) waves = 4;
@@ -1922,15 +1923,23 @@ static bool large_weight(int M, int N, int K, int epi) {
 }
 // 17 to 112 rows, a product that stores: whether the kernel with its rows through LDS takes it where the line above, or that of 64 rows,
 // gave it to the tiles.  Up to 64 rows as long as two groups of weight rows a workgroup are one round of them (up to K = 4,095 the line
-// above let one group have most of these; us, tiles and this: 6144 x 4096 at 17, 40 and 64 rows 18.0 19.7 22.5 and 15.0 16.6 18.7, 7168 x 5120
-// 22.9 25.2 29.6 and 16.0 19.8 23.7, 4096 x 12288 46 53 62 and 22 30 37, [gate; up] 4096 x 4096 at 40 and 64 27.9 30.4 and 12.1 14.7, 8192 x 4096 at
-// 17, 40 and 64 19.7 21.1 23.7 and 15.8 19.9 22.7); beyond a round only [gate; up], whose tiles cost more (24576 x 4096 at 20, 40 and 64 44.1
+// above let one group have most of these; us, tiles and this: 2048 x 4096 at 48 and 64 rows 18.7 20.5 and 10.5 12.2, [gate; up] 4096 x 4096 at 40 and 64
+// 27.9 30.4 and 12.1 14.7, 8192 x 4096 at 17, 32 and 64, stored in 16 bits, 18.9 19.8 23.3 and 16.5 16.9 19.4); beyond a round only [gate; up], whose tiles
+// cost more (24576 x 4096 at 20, 40 and 64 44.1
 // 44.5 45.6 and 37.5 42.0 49.8; 34816 x 5120 at 20, 40 and 64 89 93 100 and 71 85 106; 19456 x 2560 at 20, 32 and 40 25.7 27.1 27.5 and 24.1 25.8 27.9;
-// 51200 x 5120, seven rounds, at 20 101.5 and 100.4; 12288 x 2048 without [gate; up] at 40 14.1 and 15.6).  65 to 112 rows, five to seven blocks of
+// 51200 x 5120, seven rounds, at 20 101.5 and 100.4; 12288 x 2048 without [gate; up] at 40 14.1 and 15.6).  32-bit sums of large weights from K =
+// 4,096 on seldom come here up to 64 rows: a caller with a workspace asks ti_gemm_bf16_store_split first, which takes them in tiles that share K (with the
+// adding kernel, and here, at 17, 33, 48 and 64 rows: 6144 x 4096 14.9 15.8 16.7 17.7 and 14.1 15.3 16.3 17.7, 8192 x 4096 16.5 17.2 18.0 19.2 and 16.7
+// 17.5 18.3 19.4, 7168 x 5120 18.8 19.9 21.7 22.8 and 16.1 18.7 20.8 24.0, 4096 x 4096 from 33 on 11.3 11.5 11.9 and 10.5 12.0 13.7, 4096 x 12288 24.1
+// 24.8 26.0 27.9 and 22.3 28.2 32.0 36.9: the tiles' cuts are ahead where it matters, and which shapes gain a tenth by leaving them is left).
+// 65 to 112 rows, five to seven blocks of
 // them beside the tiles' two row tiles: a round of workgroups of one group (4096 x 1024 at 65, 77 and 112 6.8 6.8 7.2 and 5.4 5.5 6.7; 4096 x
 // 4096 17.6 17.9 19.6 and 14.2 14.7 18.3; 1024 x 1024 6.7 at 65, 6.9 at 112 and 5.1, 6.3) or, for [gate; up], two (6144 x 1024 9.1 9.2 10.0 and 6.9 7.0
 // 8.7; 8192 x 2560 22.0 at 77, 23.8 at 100 and 15.6, 18.6); without [gate; up] two groups lose from 77 on (6144 x 2560 13.9
-// and 14.5).  K of 256 and more, so that each of the four wavefronts has a chunk (1024 x 256 at 77 rows 3.6 and 2.7, 4096 x 256 4.1 and 3.3).
+// and 14.5).  Measured at 256 to 8192 weight rows and K up to 32,768, where it stays ahead (4096 x 12288 at 65 and 112 46.6 57.7 and 39.6 52.2, 256 x 24576
+// 83 100 and 64 91).  K of 256 and more, so that each of the four wavefronts has a chunk (1024 x 256 at 77 rows 3.6 and 2.7, 4096 x 256 4.1 and 3.3).
+// The sums of four wavefronts, added in their order, are not the tiles' bits, which take K in ascending order in one; relative error of 32-bit results
+// against 64 bits, tiles and this: 1024 x 1024 1.8e-7 and 0.95e-7, 4096 x 4096 4.0e-7 and 1.9e-7, 4096 x 12288 7.1e-7 and 3.4e-7.
 static int g_rows_112 = 1;      // a hook for measurements: 0: only the line above
 static bool staged_112_serves(int M, int N, int K, long lda, int epi) {
   if (!g_rows_112 || !g_use_pipelined || g_force_tile || g_tiled_from_stored != TILED_FROM_STORED || M <= 16 || M > 112 || epi == TI_EPI_ADD_F32 ||
@@ -2029,8 +2038,11 @@ static int launch_normed(const float* x, const float* nw, float eps, const bf16_
   return 0;
 }
 static int g_normed_groups = 0;    // a hook for measurements: 1 to 3 groups of wavefronts in the product with the norm inside, 0: by the tiles
-// Groups of four wavefronts: as many as a unit has tiles, three at most; with more two, whose workgroups share a unit.  A long K under two
-// tiles a unit has three as well, for 96 KiB of weights under way instead of 64 (6144 x 4096 at 1 and 4 rows 14.0 14.8 -> 11.3 12.0 us).
+// Groups of four wavefronts: as many as a unit has tiles, three at most; with more two (us at 1, 4 and 8 rows of K = 1024, two and three groups:
+// 16384 weight rows, four tiles a unit, 6.9 7.3 8.5 and 8.2 8.5 9.1).  Two workgroups of two groups share a unit only where their rows leave room, 16 KiB of
+// them and less (at K = 1024 up to 7 rows, at 2048 up to 3); beyond four tiles a unit three groups would be ahead where they do not (20000 x 1024
+// at 1, 4, 8 and 16 rows 8.8 9.2 11.3 13.0 and 9.1 9.4 9.8 11.3, [gate; up] 17920 x 1536 11.7 12.4 15.7 18.1 and 12.1 12.8 14.0 15.7), which is left.  A long K under two
+// tiles a unit has three as well, for 96 KiB of weights under way instead of 64 (6144 x 4096 at 1 and 4 rows 12.2 13.0 with two, 11.3 12.0).
 template <int KC, int EPI>
 static int launch_normed_groups(const float* x, const float* nw, float eps, const bf16_t* w, void* out, int M, int N, int K, int tiles,
                                 hipStream_t stream) {
@@ -2045,8 +2057,10 @@ static int launch_normed_groups(const float* x, const float* nw, float eps, cons
 static bool pieces_serves(int M, int N, int K, int epi);
 #define NORMED_WEIGHT_BELOW (40L << 20)   // weight elements from which the norm stays a kernel of its own
 static long g_normed_weight_below = NORMED_WEIGHT_BELOW;
-// out = rmsnorm(x; nw, eps) W^T for M <= 16 (see gemm_skinny_staged_kernel).  Returns 3 for
-// sizes it does not serve (M > 16, K not a multiple of 64 or above 4096).
+// out = rmsnorm(x; nw, eps) W^T for M <= 16 (see gemm_normed_kernel).  Returns 3 for what it leaves to the norm's kernel and the product's: M > 16,
+// K not a multiple of 64 or above 4096, operands not 16-byte aligned, rows that do not fit into LDS beside 64 KiB of weights (M (K + 8) above
+// 48 Ki: 16 rows of more than 3,064 columns, 12 of more than 4,088; 6144 x 4096 at 12 and 16 rows 15.5 16.5 us that way, 21.9 24.2 in the kernel
+// that took them before this one), squared relu, and the weights that the rules below name.
 extern "C" int ti_gemm_bf16_normed(const float* x, const float* nw, float eps, const void* W, void* out,
                                    int M, int N, int K, int epi, hipStream_t stream) {
   TI_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_bf16_normed: bad sizes M=%d N=%d K=%d", M, N, K);
@@ -2073,9 +2087,10 @@ extern "C" int ti_gemm_bf16_normed(const float* x, const float* nw, float eps, c
     return 3;
   }
   // Every workgroup here norms all M rows for itself, which pulls as many bytes through the caches as
-  // its share of the weight has.  Under a large weight the kernel that keeps loads in flight gains more
-  // than the norm's own launch costs (Qwen3-8B's gate/up, 100 M elements, at 8 rows: 46 us here, 38 + 5 us
-  // there; Qwen3-4B's, 50 M: 29 against 21 + 2.5; Qwen3-1.7B's, 25 M, and 8B's q/k/v are faster here).
+  // its share of the weight has.  Under a large weight the product alone gains more than the norm's own launch
+  // costs (us at 1, 2, 4 and 8 rows, here and as norm and product: Qwen3-4B's gate/up, 50 M elements, 20.7 21.4 22.9 26.0 and 21.6 21.9
+  // 22.2 22.5; 8B's, 100 M, 35.8 36.9 38.4 41.1 and 36.3 36.6 37.2 38.0; below the line [gate; up] 8192 x 4096, 34 M, 13.4 13.9 14.2 15.5 and 15.8
+  // 16.0 16.6 16.8, Qwen3-1.7B's, 25 M, 12.0 12.1 12.3 12.8 and 13.1 13.3 13.4 13.4).
   if ((long)(epi == TI_EPI_SWIGLU ? 2 : 1) * N * K >= g_normed_weight_below && pieces_serves(M, N, K, epi)) {
     ti_set_error("gemm_bf16_normed: a weight of %d x %d is left to the norm's kernel and the product's", N, K);
     return 3;

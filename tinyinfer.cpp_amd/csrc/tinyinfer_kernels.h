@@ -83,7 +83,8 @@ int ti_gemm_bf16_mblocks_any(const void* A, const void* W, void* out, int M, int
 // epilogue, K a multiple of 64 split ks ways (adding epilogue only; partial f32 [ks][M][N])
 int ti_gemm_bf16_pieces_any(const void* A, const void* W, void* out, int M, int N, int K, long lda, int epi,
                             void* partial, int ks, hipStream_t stream);
-// out (op)= rmsnorm(x; nw, eps) W^T for M <= 16, K a multiple of 64
+// out (op)= rmsnorm(x; nw, eps) W^T for M <= 16, K a multiple of 64 up to 4096.  3: left to the norm's kernel and the product's (other
+// sizes, operands not 16-byte aligned, rows that do not fit into LDS beside the weights, weights that are faster that way): the same bits
 int ti_gemm_bf16_normed(const float* x, const float* nw, float eps, const void* W, void* out, int M, int N, int K, int epi,
                         hipStream_t stream);
 // the q/k/v product of a step (M > 16) that finishes its heads itself: see ti_qk_norm_rope_kv_write
