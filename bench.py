@@ -13,7 +13,7 @@ the live requests) over its time against 8 TB/s.  Beside the fractions of the
 published peaks stand fractions of what this GPU delivers to a kernel that only
 reads memory, and to matrix-core instructions on registers (csrc/measure.hip),
 as the reference times its own kernels against the clock
-(/root/reference/src/selftest.cpp:392-428).
+(src/selftest.cpp:392-428).
 
 `--model 8b` and `--model 32b` run the same with the sizes of Qwen3-8B and
 Qwen3-32B.  `--kernel-times` adds a table of the decode step's calls, timed with

@@ -2,7 +2,7 @@
 reference's formulas.  Whole sequences, no cache, one function per part, numpy
 float64.  It shares no code with the engine: the tests compare the two.
 
-Every function cites the lines of /root/reference it was written from.
+Every function cites the lines of the reference it was written from.
 `rnd(site, array)` is applied where the reference rounds to bfloat16; the
 default rounds nothing, which gives the mathematically exact model.
 """

@@ -1,6 +1,6 @@
 """The logits where the bench runs: the whole depth and vocabulary of Qwen3-0.6B (28 layers, 151,936
 tokens), random weights.  The reference's own whole-model check compares logits of a real checkpoint
-with another implementation (/root/reference/docs/report.md:21-33); here the plain model under tests/
+with another implementation (docs/report.md:21-33); here the plain model under tests/
 stands in, on ~96 tokens: the prompt whole, then its last 32 tokens one by one; one decode step of 64
 requests whose pages lie scattered gives each request the logits it gets alone; the head's product over
 all 151,936 columns against float64; and decode rows at contexts of 2,048 to 4,095 tokens."""

@@ -73,7 +73,7 @@ def test_config_b_mixed_batch_with_temperature(model_folders):
 def test_greedy_generation_with_graphs_equals_eager(model_folders, dtype):
     """Decode steps replayed from captured graphs give the same logits bit for bit
     as eager steps, replay after replay, with eager steps in between (the
-    reference checks the same: /root/reference/src/inference.cu:297-341)."""
+    reference checks the same: src/inference.cu:297-341)."""
     import tinyinfer_amd as ti
     d = model_folders("D", "bfloat16", True)
     prompts = [random_tokens(n, 333, 40 + n) for n in (21, 3, 50)]
@@ -308,7 +308,7 @@ def test_command_line_options(tmp_path):
     """`--random-weights --seed` from a folder with config.json alone, `--num-pages`, `--cuda-graph`, `-t`, `--top-k`,
     `--verbose`: the tokens are the plain model's on the weights `write_model_folder` writes for that seed, drawn with
     the same temperature, cut and seed; --verbose prints the first five and the five largest logits behind each prompt
-    (/root/reference/src/main.cpp:136-158,233-249)."""
+    (src/main.cpp:136-158,233-249)."""
     import json
     import tinyinfer_amd as ti
     cfg = CONFIGS["A"]

@@ -5,7 +5,7 @@ An engine whose longest sequence is 4,096 tokens captures its decode graph with 
 context cut into several runs (chosen for the longest sequence, frozen at capture: the partial
 results' buffers, the number of runs) and replays it over rows of 3 to 2,100 cached tokens while
 requests end and others take their pages.  The reference checks its graph against the eager step
-the same way (/root/reference/src/inference.cu:297-341) and runs its kernels at real dimensions in
+the same way (src/inference.cu:297-341) and runs its kernels at real dimensions in
 src/selftest.cpp:282-390,430-459."""
 import numpy as np
 import pytest

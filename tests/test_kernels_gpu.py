@@ -438,7 +438,7 @@ def test_sample_limits_reduce_to_argmax(ops):
 def test_sample_keeps_every_logit_equal_to_the_kth(ops):
     """Equal logits at the cut: top-k keeps every logit that is no smaller than the k-th largest, so the kept
     set may hold more than k (the reference's nth_element picks among equals arbitrarily and keeps exactly k:
-    /root/reference/src/main.cpp:47-53; which of the equals it keeps is not defined, so parity is unpinned
+    src/main.cpp:47-53; which of the equals it keeps is not defined, so parity is unpinned
     there).  With logits [1, 3, 2, 2, 2, 0] and k = 2 the kept set is {1, 2, 3, 4}: weights e^1 : 1 : 1 : 1 at
     T = 1, and a uniform number near the end of [0, 1) draws index 4, which a cut to exactly two would never do."""
     row = torch.tensor([[1.0, 3.0, 2.0, 2.0, 2.0, 0.0]])

@@ -17,7 +17,7 @@ def rng(seed):
 # -------------------------------------------------------------------- RMSNorm
 def test_rmsnorm_reference_vector():
     """n=1024, rows=3, U(-1,1), eps 1e-6 against the selftest's own loop
-    (/root/reference/src/selftest.cpp:74-100): 1/sqrt(ss/n + eps) * w."""
+    (src/selftest.cpp:74-100): 1/sqrt(ss/n + eps) * w."""
     r = rng(2)
     x, w = r.uniform(-1, 1, (3, 1024)), r.uniform(-1, 1, 1024)
     want = np.stack([x[i] * (1.0 / math.sqrt(float((x[i] ** 2).sum()) / 1024 + 1e-6)) * w for i in range(3)])
@@ -40,7 +40,7 @@ def test_rmsnorm_invariants():
 # ----------------------------------------------------------------------- rope
 def test_rope_reference_vector():
     """rows=2, heads=4, hd=128, theta=1e6, positions {0,5} against the selftest's
-    loop (/root/reference/src/selftest.cpp:102-134): pairs (k, k + hd/2)."""
+    loop (src/selftest.cpp:102-134): pairs (k, k + hd/2)."""
     r = rng(3)
     x = r.uniform(-1, 1, (2, 4, 128))
     want = np.zeros_like(x)

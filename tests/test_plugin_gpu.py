@@ -2,7 +2,7 @@
 builds a kernel library (tests/cpp/toy_relu.hip) and a plugin (tests/cpp/plugin_part.cpp, against
 include/inference.h), and the model made of them is written, loaded, replayed through bin/trace_run
 and stepped through the Python entry point without a change to a file under the framework's folder.
-(The reference's one architecture is a string compare in its loader, /root/reference/src/model.cpp:26-30.)"""
+(The reference's one architecture is a string compare in its loader, src/model.cpp:26-30.)"""
 import json
 import os
 import shutil

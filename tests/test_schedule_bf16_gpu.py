@@ -1,6 +1,6 @@
 """The scheduler's workloads in bfloat16: three requests with prompts of 5, 17 and 33 tokens, portions of
 7 beside decoding requests, pages of 4, temperature 0.8 (the reference's loop with batching:
-/root/reference/src/main.cpp:210-297).  Every step's logits lie inside the bfloat16 bound of the plain
+src/main.cpp:210-297).  Every step's logits lie inside the bfloat16 bound of the plain
 model, and the token drawn is the plain model's wherever its margin exceeds that bound.  Preemption with
 graphs changes no token.  How far the engine's rounding (matrix operands, cached keys/values, and q and
 the softmax weights in addition) is from rounding only where the reference rounds is reported and

@@ -5,7 +5,7 @@
     outs = llm.generate([[1, 2, 3], [4, 5]], max_new_tokens=16, temperature=0.0)
 
 `generate` drives the scheduler, the step function and the device sampler: the
-loop of /root/reference/src/main.cpp:210-297 with admission, portions and
+loop of src/main.cpp:210-297 with admission, portions and
 preemption added (`run_requests`, engine/scheduler.cpp).  Options carry the
 reference's names and meanings (`max_new_tokens` = -n, `temperature` = -t,
 `top_k`, `top_p`, `seed`, `max_seq`).

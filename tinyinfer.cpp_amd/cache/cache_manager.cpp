@@ -3,7 +3,7 @@
 //
 // The reference keeps one slab `[layer][sequence][K/V][kv head][max_seq][head_dim]` that is
 // allocated once for `max_batch x max_seq` tokens and never given back per request
-// (/root/reference/src/inference.cu:146-148,174-176).  Here a token at position `pos` of a
+// (src/inference.cu:146-148,174-176).  Here a token at position `pos` of a
 // request lives in page `table[pos / P]` at row `pos % P`; pages come from a LIFO free list (a
 // page given back is the next one handed out), are given back when the request ends and, in a
 // group whose layers read only a window of keys, as soon as the window has passed them.  Page

@@ -1,5 +1,5 @@
 """Command line in the manner of the reference's `tinyinfer`
-(/root/reference/src/main.cpp:86-162, README.md:88-98):
+(src/main.cpp:86-162, README.md:88-98):
 
     tinyinfer -m MODEL_DIR -n max_tokens -p "prompt" [-p "prompt2" ...] [-f prompts.txt]
               [-t temp] [--top-k K] [--top-p P] [--seed S] [--max-seq N] [--cuda-graph] [--verbose]
@@ -55,7 +55,7 @@ def main(argv: Optional[List[str]] = None) -> int:
     prog, args = argv[0], argv[1:]
     if os.environ.get("TINY_SELFTEST") == "1":
         # every kernel against a CPU computation; the exit code counts the failures
-        # (the reference's QWEN_SELFTEST=1: /root/reference/src/main.cpp:123-125)
+        # (the reference's QWEN_SELFTEST=1: src/main.cpp:123-125)
         from .selftest import run_selftest
         return run_selftest()
     model = None
@@ -163,7 +163,7 @@ def main(argv: Optional[List[str]] = None) -> int:
 
     def show_logits(s, row):
         # the first five logits and the five largest behind each prompt, as the reference's --verbose prints them
-        # (/root/reference/src/main.cpp:233-249)
+        # (src/main.cpp:233-249)
         import numpy as np
         top = np.lexsort((np.arange(row.shape[0]), -row))[:5]            # descending, the lowest id first among equals
         piece = (lambda t: tokenizer.id_to_token(int(t)) or "") if tokenizer is not None else (lambda t: "")

@@ -2,7 +2,7 @@
 // from an architecture's name to its model.
 //
 // The reference fills `Qwen3Config` from GGUF keys and refuses a model whose required sizes are
-// zero (/root/reference/src/model.h:11-21, src/model.cpp:32-47); its architecture gate is one
+// zero (src/model.h:11-21, src/model.cpp:32-47); its architecture gate is one
 // string compare (src/model.cpp:26-30).  Layer order and formulas: src/inference.cu:28-72; tensor
 // names follow the checkpoint convention (`model.layers.{i}.…`), onto which the reference's GGUF
 // names (`blk.{i}.attn_q.weight`, src/model.cpp:120-150) map one to one.
@@ -162,7 +162,7 @@ void Qwen3Config::validate() const {
     throw ConfigError("config.json: 'head_dim' (" + std::to_string(head_dim) +
                       ") must be even (rotation pairs k with k + head_dim/2)");
   // what the attention kernels take (the reference refuses a head size at the launch:
-  // /root/reference/src/cuda/attention.cu:321-324); said here, before any weight is read
+  // src/cuda/attention.cu:321-324); said here, before any weight is read
   if (head_dim % 16 || head_dim > 256)
     throw ConfigError("config.json: 'head_dim' = " + std::to_string(head_dim) +
                       " is not served: the attention kernels take head sizes in steps of 16 up to 256");

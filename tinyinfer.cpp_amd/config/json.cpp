@@ -1,6 +1,6 @@
 // The JSON value of inference.h: a recursive-descent reader and a writer.  It serves config.json,
 // the header of a safetensors file and the parameters of parts; the reference has a reader of the
-// same subset for its server (/root/reference/src/json.h:14-21).
+// same subset for its server (src/json.h:14-21).
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>

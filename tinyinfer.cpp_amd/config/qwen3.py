@@ -1,7 +1,7 @@
 """Typed configuration of the Qwen3 dense decoder.
 
 The reference reads nine hyper-parameters from GGUF keys into `Qwen3Config`
-(/root/reference/src/model.h:11-21, src/model.cpp:32-47) and refuses a model
+(src/model.h:11-21, src/model.cpp:32-47) and refuses a model
 whose required sizes are zero.  Here the same fields come from the
 architecture's `config.json`; reading and validation are the host library's
 (`Qwen3Config::from_json`, config/config.cpp), this class holds the result.

@@ -24,7 +24,7 @@
 //            take four such tiles of the same head, so they walk the same pages
 //            together and share them in the cache.
 // (The reference scans positions with 16-lane groups and FMA for both cases:
-// /root/reference/src/cuda/attention.cu:107-198.)
+// src/cuda/attention.cu:107-198.)
 #include <string>
 #include <type_traits>
 #include <utility>

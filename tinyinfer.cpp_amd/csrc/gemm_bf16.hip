@@ -15,7 +15,7 @@
 // Epilogues: store float, add into a float residual, store bfloat16, or SwiGLU
 // over a stacked [gate; up] weight.  The reduction order of an output element
 // never depends on M within one kernel.  (The reference's two products are
-// /root/reference/src/cuda/gemm.cu:37-85 and 152-261; it reads the weights once
+// src/cuda/gemm.cu:37-85 and 152-261; it reads the weights once
 // per row of A for M <= 32.)
 #include <algorithm>
 #include <string>

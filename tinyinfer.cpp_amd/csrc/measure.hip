@@ -1,7 +1,7 @@
 // What this GPU delivers, measured: the bandwidth of a kernel that only reads memory, and the rate of
 // matrix-core instructions whose operands never leave the registers.  bench.py reports its figures
 // as fractions of these beside the fractions of the published peaks.  The reference times its own
-// GEMV against the clock in the same spirit (/root/reference/src/selftest.cpp:392-428).
+// GEMV against the clock in the same spirit (src/selftest.cpp:392-428).
 #include "common.h"
 #include "tinyinfer_kernels.h"
 

@@ -1,5 +1,5 @@
 // Per-head preparation of queries and keys: RMS-norm over head_dim, then the half-split
-// rotation (/root/reference/src/cuda/rope.cu:31-52: q_norm/k_norm are applied before the
+// rotation (src/cuda/rope.cu:31-52: q_norm/k_norm are applied before the
 // rotation, pairs are (i, i + head_dim / 2)).  The kernel that prepares a whole step's rows
 // and the decode attention kernel that prepares its own query both go through these
 // functions, with the products and sums spelled out, so that they produce the same bits.

@@ -1,6 +1,6 @@
 // Sampling on the device: greedy argmax (of equal logits the lowest index wins,
-// as /root/reference/src/cuda/sample.cu:5-11) and temperature sampling with
-// optional top-k and top-p cuts (/root/reference/src/main.cpp:40-83 does these
+// as src/cuda/sample.cu:5-11) and temperature sampling with
+// optional top-k and top-p cuts (src/main.cpp:40-83 does these
 // on the host with a sort).  Several workgroups read a long row, and one finishes it.
 //
 // Temperature sampling draws by inverse CDF over the index order from one

@@ -5,7 +5,7 @@
 // runs exactly the tokens it is given as one flat batch against the cache that earlier steps
 // left, and returns the logits at the wanted places.  The reference's `Inference::forward` has
 // the same shape (flat tokens with a position and a sequence id each, logits for chosen rows:
-// /root/reference/src/inference.h:26-42, src/inference.cu:178-265) over a non-paged cache; its
+// src/inference.h:26-42, src/inference.cu:178-265) over a non-paged cache; its
 // kernel sequence is src/inference.cu:28-72, its graphs src/inference.cu:267-295.
 //
 // Per-step metadata (tokens, positions, block-table rows, output rows, the parts' own lists) is

@@ -2,7 +2,7 @@
 //
 // The reference has no scheduler: every prompt is prefilled whole in one batch and then every
 // unfinished sequence decodes one token per step, in a cache sized so that nothing can run out
-// (/root/reference/src/main.cpp:210-297).  Here requests wait in a queue, are admitted while a
+// (src/main.cpp:210-297).  Here requests wait in a queue, are admitted while a
 // request slot and pages for their first portion are free, have their prompts cut into portions
 // under a token budget, decode beside the portions of others, and give everything back when they
 // end.
@@ -189,7 +189,7 @@ std::vector<std::shared_ptr<Request>> Scheduler::commit(const Plan& plan, const 
     if (it == sampled.end()) throw SchedulerError("request " + std::to_string(req.number) + " asked for a token and got none");
     const int tok = it->second;
     // the reference drops an end-of-generation token instead of emitting it
-    // (/root/reference/src/main.cpp:255,287) and counts the first token from the prefill step
+    // (src/main.cpp:255,287) and counts the first token from the prefill step
     // towards -n (main.cpp:258,284)
     if (std::find(req.eos_token_ids.begin(), req.eos_token_ids.end(), tok) != req.eos_token_ids.end()) {
       req.finish_reason = "eos";
@@ -223,7 +223,7 @@ void Scheduler::abort_all() {
   for (const auto& r : all) abort(r);
 }
 
-// The loop of /root/reference/src/main.cpp:210-297 with admission, portions and preemption added.
+// The loop of src/main.cpp:210-297 with admission, portions and preemption added.
 void run_requests(Engine& engine, Scheduler& scheduler, Sampler* sampler, GenerationStats* stats,
                   const std::function<void(const Request&, int)>& on_token, bool use_graph, bool run_ahead,
                   const PromptLogits& on_prompt_logits) {

@@ -20,7 +20,7 @@
 // step a line `done <step>` is printed and flushed.  When the input ends the program exits with 0.
 //
 // The reference's tool of this kind writes the last token's logits of one prompt through another
-// library (/root/reference/ref/ref_logits.cpp:13-19,59-67).
+// library (ref/ref_logits.cpp:13-19,59-67).
 #include <cstdio>
 #include <cstring>
 #include <iostream>

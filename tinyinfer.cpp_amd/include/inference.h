@@ -1,8 +1,8 @@
 // tinyinfer for AMD MI355X: the programming interface of the engine, in one header.
 //
 // The reference's counterpart is `class Inference` with `init / forward / reset_kv /
-// set_use_cuda_graph` (/root/reference/src/inference.h:12-44) over `Qwen3Model::load`
-// (/root/reference/src/model.h:39-53).  Here the same step-function shape (a flat batch of
+// set_use_cuda_graph` (src/inference.h:12-44) over `Qwen3Model::load`
+// (src/model.h:39-53).  Here the same step-function shape (a flat batch of
 // tokens with positions, logits at chosen rows) sits on a paged cache with a scheduler above
 // it, and the model is put together from registered parts.
 //
@@ -106,7 +106,7 @@ class Json {
 
 // ----------------------------------------------------------------------------- configuration
 // The hyper-parameters of the Qwen3 dense decoder, read from the keys of its config.json
-// (the reference reads nine of them from GGUF keys: /root/reference/src/model.h:11-21,
+// (the reference reads nine of them from GGUF keys: src/model.h:11-21,
 // src/model.cpp:32-47).  Options that would change the math and are not served
 // (attention_bias, rope_scaling, another hidden_act) are refused by name.
 struct Qwen3Config {
@@ -154,7 +154,7 @@ struct ModelSpec {
 };
 
 // An architecture: config.json -> ModelSpec.  The reference gates on one string
-// (/root/reference/src/model.cpp:26-30); here that compare is a table.
+// (src/model.cpp:26-30); here that compare is a table.
 using SpecBuilder = std::function<ModelSpec(const Json& config)>;
 // The architecture's typed configuration: config.json read, validated and written back with its defaults
 // filled in (what a model folder's config.json says after a round trip).  Optional.
@@ -564,7 +564,7 @@ class Ops {
   void flush();
   int pending_splits() const { return pending_.out ? pending_.splits : 0; }   // 0: no sums are waiting
   // Per-call timing with events (the reference's selftest times its kernels the same way:
-  // /root/reference/src/selftest.cpp:404-424): while on, every call records an event before and
+  // src/selftest.cpp:404-424): while on, every call records an event before and
   // after what it launches; the report waits for them and gives (name with sizes, calls, microseconds).
   void timing(bool on);
   // the same list of calls without the times: nothing is recorded on the stream and no sum is added early, so
@@ -1002,7 +1002,7 @@ class Model {
 // Keys and values in pages with a block table per request, one pool per group of layers with the
 // same need, slots for per-request state of fixed size.  Host bookkeeping only.  The reference
 // keeps one slab for max_batch x max_seq tokens that is never given back per request
-// (/root/reference/src/inference.cu:146-148,174-176).
+// (src/inference.cu:146-148,174-176).
 class PagePool {
  public:
   PagePool(int num_pages, int scatter_window = 0);
@@ -1126,7 +1126,7 @@ class Engine {
 };
 
 // ----------------------------------------------------------------------------------- sampling
-// temperature <= 0: greedy (/root/reference/src/main.cpp:24,31-38); top_k 0 means the reference's
+// temperature <= 0: greedy (src/main.cpp:24,31-38); top_k 0 means the reference's
 // 512 (src/main.cpp:47-48); seed 42 (src/main.cpp:27).  The n-th token of a request is drawn with
 // uniform(seed, request number, n): neither batching nor preemption changes what is sampled.
 struct SamplingParams {
@@ -1162,7 +1162,7 @@ class Sampler {
 // ---------------------------------------------------------------------------------- scheduler
 // Which tokens of which requests the next step runs.  The reference has none: every prompt is
 // prefilled whole in one batch, then every unfinished sequence decodes one token a step
-// (/root/reference/src/main.cpp:210-297).
+// (src/main.cpp:210-297).
 struct Request {
   int64_t number = 0;                  // order of submission; keys the random stream and the cache
   std::vector<int> prompt;
@@ -1220,7 +1220,7 @@ struct GenerationStats {
 // not wait for the host between steps; tokens are the same, `on_token` hears them one step later.
 // `on_prompt_logits`: called with the 32-bit logits (host memory, `vocab` of them) behind the last token of a
 // request's prompt, before its first token is drawn (what the reference's --verbose prints:
-// /root/reference/src/main.cpp:233-249); it costs a copy and a wait per such step.
+// src/main.cpp:233-249); it costs a copy and a wait per such step.
 using PromptLogits = std::function<void(const Request&, const float* logits, int64_t vocab)>;
 void run_requests(Engine& engine, Scheduler& scheduler, Sampler* sampler = nullptr, GenerationStats* stats = nullptr,
                   const std::function<void(const Request&, int token)>& on_token = nullptr, bool use_graph = false,

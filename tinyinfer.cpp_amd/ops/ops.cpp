@@ -8,7 +8,7 @@
 // entries go to the flash-decoding kernel (split over the context so that the launch fills the
 // chip), rows of longer entries to the tiled prefill kernels.  Head or page sizes those do not
 // serve are left to the generic kernel.  The reference runs one kernel for both
-// (/root/reference/src/cuda/attention.cu:89-214).
+// (src/cuda/attention.cu:89-214).
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
 

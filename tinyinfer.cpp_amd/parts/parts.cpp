@@ -1,21 +1,21 @@
 // The parts a model is put together from, and their registry by family and kind.
 //
-//   embedding "table"     x[m, :] = float(E[tok[m], :]), no scaling (/root/reference/src/inference.cu:14-24)
+//   embedding "table"     x[m, :] = float(E[tok[m], :]), no scaling (src/inference.cu:14-24)
 //   norm      "rmsnorm"   y = x * rsqrt(mean(x^2) + eps) * w, eps inside the root, the weight multiplies
-//                         directly (/root/reference/src/cuda/rms_norm.cu:15-25)
+//                         directly (src/cuda/rms_norm.cu:15-25)
 //   pos       "rope_neox" half-split rotation over the whole head: pair (k, k + hd/2) turns by
-//                         pos * theta^(-2k/hd) (/root/reference/src/cuda/attention.cu:38,64-74; the
+//                         pos * theta^(-2k/hd) (src/cuda/attention.cu:38,64-74; the
 //                         adjacent-pair variant is the mistake listed in docs/report.md:91)
 //   mixer     "attention" causal grouped-query attention over the paged cache: fused q/k/v product, per-head
 //                         RMSNorm of q and k with a weight shared by all heads (before rotation; v is left
 //                         alone), rotation, cache write, head h reads kv head h / (heads / kv_heads), scores
 //                         scaled by 1/sqrt(hd), output projection added into the residual
-//                         (/root/reference/src/inference.cu:41-55; src/cuda/attention.cu:12-87,107-198)
+//                         (src/inference.cu:41-55; src/cuda/attention.cu:12-87,107-198)
 //   ffn       "swiglu"    y = silu(h Wg^T) * (h Wu^T); x += y Wd^T, gate and up rows held as one matrix
-//                         (/root/reference/src/inference.cu:60-65,155-160; src/cuda/ffn.cu:13-15)
-//   block     "pre_norm"  x += mixer(norm1(x)); x += ffn(norm2(x)) (/root/reference/src/inference.cu:35-66)
+//                         (src/inference.cu:60-65,155-160; src/cuda/ffn.cu:13-15)
+//   block     "pre_norm"  x += mixer(norm1(x)); x += ffn(norm2(x)) (src/inference.cu:35-66)
 //   head      "linear"    logits = h E_out^T with E_out the embedding itself or a matrix of its own
-//                         (/root/reference/src/cuda/lm_head.cu:5-10; the reference is always tied, src/model.h:42)
+//                         (src/cuda/lm_head.cu:5-10; the reference is always tied, src/model.h:42)
 //
 //
 // Parts no layer of the reference has (their formulas stand at each class):
@@ -421,7 +421,7 @@ class Sinusoidal final : public PositionPart {
 // precision (rounded to float only at the end): a 32-bit angle pos * inv_freq[k] is pos * 2^-23 off, 6e-4
 // five thousand tokens in, and differently at every position, so that not only distances would count.
 // Positions beyond the table (none that an engine serves) have the angle and its sine and cosine in
-// 32-bit on the device, as /root/reference/src/cuda/rope.cu:20-22 has them everywhere.
+// 32-bit on the device, as src/cuda/rope.cu:20-22 has them everywhere.
 //
 // A table never changes and is never freed while anything may read it: captured graphs hold its
 // address in their kernel arguments.  Parts with the same head size and base share the longest table
@@ -722,7 +722,7 @@ class Attention final : public MixerPart {
       src.fill(n_v + ".b", b_qkv.rows(nq + nk, nv));
     }
     // q, k and v go straight into the fused matrix (the reference builds its fused copy beside the
-    // originals and keeps both: /root/reference/src/inference.cu:154-169)
+    // originals and keeps both: src/inference.cu:154-169)
     w_qkv = adopted.defined() ? adopted : src.alloc(src.matrix_dtype, {nq + nk + nv + ng, hidden});      // the gate's rows behind q, k and v: one product
     src.fill(n_q, w_qkv.rows(0, nq));
     if (!shares_kv) {

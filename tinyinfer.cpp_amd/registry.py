@@ -3,7 +3,7 @@
 An entry is a pair: a reader of the architecture's `config.json` into a typed
 configuration, and a builder from that configuration to a `ModelSpec`.  The
 reference gates on one string (`general.architecture == "qwen3"`,
-/root/reference/src/model.cpp:26-30); here that string compare is a table, and
+src/model.cpp:26-30); here that string compare is a table, and
 an unknown name is an error that lists what is registered.  The host library
 has the table of the built-in architecture (config/config.cpp); architectures
 registered from Python are kept here and looked up first.

@@ -3,7 +3,7 @@
 // The reference samples on the host: greedy argmax when the temperature is 0, else the K largest
 // logits (K = --top-k, or 512 when that is 0), weights exp(l/T - max), an optional top-p cut, and
 // one draw from a process-wide mt19937 shared by all sequences in turn
-// (/root/reference/src/main.cpp:23-84).  Here the same options run on the device
+// (src/main.cpp:23-84).  Here the same options run on the device
 // (csrc/sampling.hip), and the random stream is keyed by (seed, request number, index of the
 // generated token): what a request draws does not depend on which other requests share its
 // steps, nor on being preempted.

@@ -1,6 +1,6 @@
 """Sampling parameters, the counter-based random stream, and the device sampler,
 named from Python (sampling/sampler.cpp has them, and what the reference does:
-/root/reference/src/main.cpp:23-84).
+src/main.cpp:23-84).
 """
 from __future__ import annotations
 

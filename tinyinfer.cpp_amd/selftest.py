@@ -1,5 +1,5 @@
 """Operator selftest: every kernel against a plain float64 computation on the CPU, in the
-manner of the reference's `QWEN_SELFTEST=1` (/root/reference/src/selftest.cpp:463-473; its
+manner of the reference's `QWEN_SELFTEST=1` (src/selftest.cpp:463-473; its
 cases and tolerances: 33-72 product, 74-100 RMSNorm, 102-134 rotation, 136-390 per-head
 norm + rotation + cache + attention, 392-459 products of the model's shapes with timings).
 

@@ -4,12 +4,12 @@
 // safetensors: 8 bytes little-endian header length n, n bytes of JSON
 // `{name: {"dtype", "shape", "data_offsets": [begin, end]}, "__metadata__": {...}}`, then the tensor
 // bytes; offsets count from the end of the header.  (The reference's GGUF loader once treated data
-// offsets as file-absolute: /root/reference/docs/report.md:84-91.)  The file is mapped; nothing
+// offsets as file-absolute: docs/report.md:84-91.)  The file is mapped; nothing
 // in it is executed.
 //
 // Every fault of a checkpoint is reported in one error: tensors the model asks for and the files
 // lack, tensors the files hold and nothing asks for, tensors of the wrong shape (the full shape
-// is compared; the reference compares element counts only, /root/reference/src/model.cpp:74-80,
+// is compared; the reference compares element counts only, src/model.cpp:74-80,
 // 104-109, so a transposed matrix would pass there) or of the wrong kind of dtype.
 //
 // Dtypes on the device, by the role a part gives the tensor: a matrix takes the engine's compute
