@@ -2030,6 +2030,27 @@ def test_attention_bf16_random_shapes_and_batches(ops, seed):
         assert (got - want).abs().max() < 2e-2, what
 
 
+@pytest.mark.parametrize("nh,nkv,hd,P", [(16, 8, 128, 16), (6, 3, 128, 48), (8, 8, 64, 32), (4, 2, 64, 16)])
+@pytest.mark.parametrize("variant", ["one group", "two groups", "paired", "a tile each"])
+def test_attention_bf16_portions_at_the_edges_of_runs(ops, nh, nkv, hd, P, variant):
+    """Portions whose keys end at, one before and one behind 64 and 128 blocks of 16 (the addresses of so many are looked up at once,
+    the next ones while they are walked), an odd number of blocks, rows that are a tile, one more and one less; eight heads for
+    keys, which go to the dies by themselves, and other numbers, which do not."""
+    entries = [(64, 960), (65, 959), (63, 962), (17, 1023), (1, 40), (128, 1920), (40, 2009), (2, 2047), (31, 0)]
+    lib = ops.lib("attention_bf16")
+    lib.ti_tuning_set(b"prefill_groups", {"one group": 1, "two groups": 2}.get(variant, 0))
+    ops.use_paired_prefill = variant in ("paired", "a tile each")
+    ops.force_paired_tiles = variant == "paired"
+    try:
+        got, want = fast_attention_case(ops, entries, nh, nkv, hd, P, None, seed=nh + hd + P)
+    finally:
+        lib.ti_tuning_set(b"prefill_groups", 0)
+        ops.use_paired_prefill = True
+        ops.force_paired_tiles = None
+    assert torch.isfinite(got).all()
+    assert (got - want).abs().max() < 2e-2          # as above: weights and results rounded to 8 bits of values of up to 4
+
+
 def test_attention_bf16_far_into_long_contexts(ops):
     """Rows of single tokens behind 20,000 and 32,767 cached tokens (a block table wider than the 1,024 entries
     the decode kernel can hold in LDS, contexts cut into many runs) and portions of prompts deep inside a

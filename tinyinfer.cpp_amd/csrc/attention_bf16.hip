@@ -1139,6 +1139,15 @@ __device__ __forceinline__ void vm_wait_turns(int k) {
 #undef TI_VM
 }
 
+// LDS of a workgroup: every stage of keys of all groups, behind them every stage of values (so that the stage is a constant in a read), and the
+// queries where many groups take the same ones.  The groups' partial results take the stages' place.
+template <int HD, int NG, int NW, int ST>
+struct PrefillLds {
+  static constexpr int TURN = PF_KEYS * HD * 2;                            // a stage: a turn's keys, or its values
+  static constexpr int VALUES = ST * NG * TURN, QUERIES = 2 * VALUES;
+  static constexpr int BYTES = QUERIES + (NG >= 4 ? NW * 32 * HD * 2 : 0);
+};
+
 // NG groups of NW wavefronts in the workgroup.  A tile is 32 NW rows: a column block of 32
 // tokens per wavefront of a group, and every group takes all of the tile's rows.  With more
 // than one group the turns (32 keys) go to the groups in rotation (each group loads and walks
@@ -1166,28 +1175,33 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   constexpr int WROWS = 32 * CB;                      // tokens per wavefront
   constexpr int TROWS = NW * WROWS;                   // tokens per tile
   constexpr int NP = HD / 8;                          // 16-byte pieces per K row
-  constexpr int K_BYTES = PF_KEYS * HD * 2;
-  constexpr int STAGE = 2 * K_BYTES;                  // K tile + V^T tile
+  typedef PrefillLds<HD, NG, NW, ST> Lds;
+  constexpr int NEXT = NG * Lds::TURN;                // from a stage to the next
   constexpr int K_ROWS = 1024 / (HD * 2);             // K rows per wavefront load
   constexpr int K_LOADS = PF_KEYS / K_ROWS;
-  constexpr int V_LOADS = HD / 16;                    // 16 dims (64 bytes each) per wavefront load
+  constexpr int V_LOADS = HD / 16, V_BLOCK = HD / 32;   // 32 dims (the 32 bytes of a block's 16 keys each) per wavefront load
   static_assert(K_LOADS % NW == 0 && V_LOADS % NW == 0, "every wavefront takes the same kinds of loads");
   constexpr int MY_K = K_LOADS / NW, MY_LOADS = (K_LOADS + V_LOADS) / NW;   // per wavefront and turn
   constexpr int QL = NG >= 4 ? TROWS * HD * 2 / 1024 / (NG * NW) : 0;      // loads of queries a wavefront, 0: as operands from memory
   constexpr int KS = HD / 16;                         // k-steps of the first product
   constexpr int DB = HD / 32;                         // 32-dim blocks of the output
 
-  // Which (tile, head) this workgroup takes.  Workgroups go to the eight XCDs in turn (linear id
-  // mod 8) and each XCD has an L2 of its own: with a multiple of eight kv heads, an XCD is given
-  // whole kv heads, so that the keys and values of a head are read into one L2 only.
-  int head = by;
-  if (n_kv % 8 == 0) {
-    const int id = by * gx + bx;
-    const int xcd = id & 7, local = id >> 3;
-    const int per_kv = (n_head / n_kv) * gx;              // workgroups of one kv head
-    const int rest = local % per_kv;
-    head = (xcd + 8 * (local / per_kv)) * (n_head / n_kv) + rest / gx;
-    bx = rest % gx;
+  // Which (tile, head) this workgroup takes: the tiles with the most keys come first in all heads, so that what starts behind the first round
+  // of the units is ever smaller and the units end together.  (With a head's tiles behind one another the last heads' largest tiles started
+  // last.  us, tiles of 64 rows, heads first and tiles first: 32 heads of 700 tokens 21.9 and 16.9, of 1,500 47.6 and 42.8; 16 of 2,048
+  // 37.4 and 35.3.)  Workgroups go to the eight XCDs in turn (linear id mod 8) and each XCD has an L2 of its own: with a multiple of
+  // eight kv heads, an XCD is given whole kv heads, so that the keys and values of a head are read into one L2 only.
+  int head;
+  {
+    const int id = by * gx + bx, group = n_head / n_kv;
+    if (n_kv % 8 == 0) {
+      const int xcd = id & 7, local = id >> 3, heads = n_head / 8, nth = local % heads;      // heads: an XCD's
+      bx = local / heads;
+      head = (xcd + 8 * (nth / group)) * group + nth % group;
+    } else {
+      bx = id / n_head;
+      head = id % n_head;
+    }
   }
   // the wavefront's number in scalar registers: what follows from it (which turns it loads, where they
   // go, which rows are its own) is then worked out once per wavefront, not once per lane
@@ -1197,7 +1211,6 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   const int kvh = head / (n_head / n_kv);
   const size_t page_elems = (size_t)2 * n_kv * P * HD;
   const bf16_t* kpool = pool + (size_t)kvh * P * HD;
-  const bf16_t* vpool = pool + (size_t)(n_kv + kvh) * P * HD;
 
   // scores are kept in units of log 2: softmax weights are then bare exp2
   const float scale2 = scale * 1.4426950408889634f;
@@ -1205,36 +1218,34 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   // what this lane fetches in each of its loads of a turn
   //  K load g: LDS rows K_ROWS g .. + K_ROWS - 1; lane i -> row r = K_ROWS g + i / NP, slot c = i % NP,
   //            holds piece c ^ (r & (NP - 1)) of key 16 (r / 16) + swap23(r % 16)
-  //  V load g: dims 16 g .. 16 g + 15, 64 bytes each; lane i -> dim d = 16 g + i / 4, slot c = i % 4,
-  //            holds piece c ^ ((d >> 2) & 3): keys 16 (piece / 2) + 8 (piece % 2) .. + 7
-  // In bytes from a block's first K row, K load g takes for lane i (lr = i / NP < K_ROWS, c = i % NP)
+  //  V load g of a block: dims 32 g .. 32 g + 31; lane i -> dim 32 g + i / 2, keys 8 (i % 2) .. + 7: in pages of 16 rows 1 KiB of consecutive
+  //            bytes, and in LDS what an operand reads is 1 KiB of consecutive bytes too
+  // K load g starts for lane i (lr = i / NP < K_ROWS, c = i % NP) from its block's first K row at
   //   (k_lane ^ X(g)) + C(g),  k_lane = swap23(lr) * HD * 2 + (c ^ lr) * 16,
   //   X(g) = ((K_ROWS g) & (NP - 1)) * 16,  C(g) = swap23((K_ROWS g) & 15) * HD * 2
-  // (the row number K_ROWS g + lr has g's bits and the lane's bits apart, and so have its pieces), from the
-  // first block of the turn if (K_ROWS g) & 16 is clear, else from the second; and V load g takes, from
-  // the V^T row of a block's first key, v_lane + 32 g P, v_lane = ((i / 4) P + 8 (piece & 1)) * 2, from the
-  // second block in the lanes whose piece is 2 or 3.  One register a kind instead of one a load.
+  // (the row number K_ROWS g + lr has g's bits and the lane's bits apart, and so have its pieces), of the turn's first block if
+  // (K_ROWS g) & 16 is clear, else of the second; V load g at v_lane + 64 g P from the V^T row of the block's first key.  A block has one
+  // descriptor, C(g) and 64 g P go into the scalar offset: a load is one scalar addition, the step of m0, and itself.  (As flat
+  // addresses, two blocks' values in a load, a turn's loads took 75 instructions, most of them scalar ones behind one another, now 35; us a
+  // launch at 16 heads, 8 for keys: 2,048 tokens 33.5 -> 32.6, 6,000 238 -> 229, 77 7.05 -> 6.95.)
   static_assert(K_ROWS <= 16 && (K_ROWS & (K_ROWS - 1)) == 0, "rows of a K load lie in one block of 16");
   auto swap23 = [](int r16) __attribute__((always_inline)) { return ((r16 & 4) << 1) | ((r16 & 8) >> 1) | (r16 & 3); };
   const unsigned k_lane = (unsigned)(swap23(lane / NP) * HD * 2 + (((lane % NP) ^ (lane / NP)) << 4));
-  const int v_piece = (lane & 3) ^ ((lane >> 4) & 3);
-  const unsigned v_lane = (unsigned)((((lane >> 2) * P) + (v_piece & 1) * 8) * 2);
-  const bool v_second = (v_piece >> 1) != 0;
+  const unsigned v_lane = (unsigned)((lane >> 1) * P * 2 + (lane & 1) * 16);
 
-  const unsigned lds0 = (unsigned)(size_t)smem + grp * (ST * STAGE);   // this group's stages
+  const unsigned lds_k = (unsigned)(size_t)smem + grp * Lds::TURN, lds_v = lds_k + Lds::VALUES;      // this group's first stages
   // the wavefronts of a group wait for each other at the workgroup's barrier (a handshake of a group's
   // two wavefronts through a word of LDS, which lets the groups drift apart, was slower: 4.72 ms against
   // 4.59 ms for a prompt of 2,048 tokens at Qwen3-0.6B's sizes)
   auto group_sync = [&]() __attribute__((always_inline)) {
     if constexpr (NW > 1) __builtin_amdgcn_s_barrier();
   };
-  // LDS addresses of this lane's fragments; the stage, and the dim block of a V^T fragment, are
+  // LDS addresses of this lane's fragments; the stage, and the dims and the block of a V^T fragment, are
   // constants in the read instructions
-  unsigned k_addr[KS], v_addr[2];
+  unsigned k_addr[KS];
+  const unsigned v_addr = lds_v + r32 * 32 + h * 16;
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) k_addr[ks] = lds0 + r32 * (HD * 2) + (((ks * 2 + h) ^ (r32 & (NP - 1))) << 4);
-#pragma unroll
-  for (int tt = 0; tt < 2; ++tt) v_addr[tt] = lds0 + K_BYTES + r32 * 64 + (((tt * 2 + h) ^ ((r32 >> 2) & 3)) << 4);
+  for (int ks = 0; ks < KS; ++ks) k_addr[ks] = lds_k + r32 * (HD * 2) + (((ks * 2 + h) ^ (r32 & (NP - 1))) << 4);
 
   for (int slot = 0; slot < (PAIRED ? 2 : 1); ++slot) {
   // ---- this slot's tile
@@ -1264,54 +1275,72 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
     blk_hi = min(blk_hi, blk_lo + per - 1);                         // a run past the end is empty
   }
 
-  // A run is up to 64 blocks.  Lane i keeps where block c0 + i starts in the pool (in elements: the V^T
-  // row of its first key; its first K row lies prow * (HD - 1) further) and the row of its first key in
-  // its page, so that the walk waits for the block table once per run and divides by the page size once
-  // per run.  Blocks past the end stand on page 0, and so do blocks whose page was given back (all their
-  // keys are masked).
-  long base = 0;
-  int prow = 0;
-  auto run_blocks = [&](int c0, int nblk) __attribute__((always_inline)) {
-    const int key = (c0 + lane) * 16, pidx = key / P;
-    prow = key - pidx * P;
-    int page = (lane < nblk) ? tab[pidx] : 0;
-    if (page < 0) page = 0;
-    base = (long)page * (long)page_elems + prow;
+  // A run is 64 blocks.  Lane i keeps where block i of a run starts in the pool (the bytes of its page's first K row of this kv head) and the
+  // row of its first key in that page, for the run that loads are asked from and the next, so that the walk divides by the page size once a
+  // run and waits for the block table once a tile.  Blocks past the end stand on page 0, and so do blocks whose page was given back
+  // (all their keys are masked).
+  unsigned run_lo[2] = {0, 0}, run_hi[2] = {0, 0};
+  int run_row[2] = {0, 0}, asked = 0;
+  const int n_blk = blk_hi + 1 - blk_lo;
+  auto ask_run = [&](int r) __attribute__((always_inline)) {
+    const int b = 64 * r + lane;
+    asked = b < n_blk ? tab[(blk_lo + b) * 16 / P] : 0;
   };
-  // The loads of this group's turn i of the run into a stage (stage_off: its offset, a constant where
-  // the loop is unrolled).  Which blocks, which pages and where in LDS is the same in every lane and
-  // worked out in scalar registers; a lane adds the offset of its piece.  (Asking for a turn in portions
-  // between the steps of the turn before, so that the unit that takes the addresses (64 bytes a cycle
-  // for the whole compute unit) works beside the matrix cores, gained nothing.)
-  auto issue = [&](int i, unsigned stage_off) __attribute__((always_inline)) {
-    const int t = i * NG + grp;
-    const int ja = min(2 * t, 63), jb = min(2 * t + 1, 63);
-    const unsigned lo_a = __builtin_amdgcn_readlane((int)(unsigned)base, ja), hi_a = __builtin_amdgcn_readlane((int)(base >> 32), ja);
-    const unsigned lo_b = __builtin_amdgcn_readlane((int)(unsigned)base, jb), hi_b = __builtin_amdgcn_readlane((int)(base >> 32), jb);
-    const long v_a = (long)(((unsigned long)hi_a << 32) | lo_a), v_b = (long)(((unsigned long)hi_b << 32) | lo_b);
-    const long k_a = v_a + (long)__builtin_amdgcn_readlane(prow, ja) * (HD - 1);
-    const long k_b = v_b + (long)__builtin_amdgcn_readlane(prow, jb) * (HD - 1);
+  auto place_run = [&](int r) __attribute__((always_inline)) {
+    const unsigned long at = (unsigned long)kpool + (unsigned long)max(asked, 0) * (page_elems * 2);
+    const int row = (blk_lo + 64 * r + lane) * 16 % P;
+    if (r & 1) run_lo[1] = (unsigned)at, run_hi[1] = (unsigned)(at >> 32), run_row[1] = row;
+    else run_lo[0] = (unsigned)at, run_hi[0] = (unsigned)(at >> 32), run_row[0] = row;
+  };
+  // The loads of this group's turn i: where its two blocks lie, then one load after another (n < MY_K: keys).  What is the same in every lane
+  // is worked out in scalar registers.
+  unsigned at_lo[2], at_hi[2];
+  int at_row[2];
+  auto find_turn = [&](int i) __attribute__((always_inline)) {
+    const int t = i * NG + grp, j = (2 * t) & 63;
+    if ((t >> 5) & 1) {
 #pragma unroll
-    for (int j = 0; j < MY_LOADS; ++j) {
-      const char* src;
-      unsigned dst;
-      if (j < MY_K) {
-        const int g = wave + NW * j;                              // the same in every lane
-        const int rows = K_ROWS * g;
-        const char* from = reinterpret_cast<const char*>(kpool + ((rows & 16) ? k_b : k_a)) +
-                           swap23(rows & 15) * HD * 2;
-        src = from + (k_lane ^ (unsigned)((rows & (NP - 1)) << 4));
-        dst = g * 1024;
-      } else {
-        const int gv = wave + NW * (j - MY_K);
-        const char* from = reinterpret_cast<const char*>(vpool + (v_second ? v_b : v_a));
-        src = from + v_lane + (size_t)gv * 32 * P;
-        dst = K_BYTES + gv * 1024;
+      for (int x = 0; x < 2; ++x) {
+        at_lo[x] = __builtin_amdgcn_readlane(run_lo[1], j + x);
+        at_hi[x] = __builtin_amdgcn_readlane(run_hi[1], j + x);
+        at_row[x] = __builtin_amdgcn_readlane(run_row[1], j + x);
       }
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                       (__attribute__((address_space(3))) void*)(size_t)(lds0 + stage_off + dst), 16, 0, 0);
+    } else {
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        at_lo[x] = __builtin_amdgcn_readlane(run_lo[0], j + x);
+        at_hi[x] = __builtin_amdgcn_readlane(run_hi[0], j + x);
+        at_row[x] = __builtin_amdgcn_readlane(run_row[0], j + x);
+      }
     }
   };
+  const unsigned v_from = (unsigned)(n_kv * P * HD * 2);             // a page's values behind its keys
+  auto load_one = [&](unsigned stage_off, int n) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass has no buffer descriptors)
+    const bool keys = n < MY_K;
+    const int g = wave + NW * (keys ? n : n - MY_K);                 // the same in every lane
+    const int rows = K_ROWS * g;
+    // which of the turn's blocks: known where it is compiled unless a wavefront's loads of a kind are fewer than the blocks
+    const int x = keys ? (K_ROWS * NW <= 16 ? (K_ROWS * NW * n) >> 4 : rows >> 4) : (NW <= V_BLOCK ? NW * (n - MY_K) / V_BLOCK : g / V_BLOCK);
+    const unsigned lo = x ? at_lo[1] : at_lo[0], hi = x ? at_hi[1] : at_hi[0];
+    const int row = x ? at_row[1] : at_row[0];
+    const auto block = __builtin_amdgcn_make_buffer_rsrc((void*)(((unsigned long)hi << 32) | lo), 0, 0x7fffffff, 0x00020000);
+    if (keys)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(block, (__attribute__((address_space(3))) void*)(size_t)(lds_k + stage_off + g * 1024), 16,
+                                               k_lane ^ (unsigned)((rows & (NP - 1)) << 4), (row + swap23(rows & 15)) * (HD * 2), 0, 0);
+    else
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(block, (__attribute__((address_space(3))) void*)(size_t)(lds_v + stage_off + g * 1024), 16,
+                                               v_lane, v_from + row * 2 + (g % V_BLOCK) * 64 * P, 0, 0);
+#endif
+  };
+  auto issue = [&](int i, unsigned stage_off) __attribute__((always_inline)) {
+    find_turn(i);
+#pragma unroll
+    for (int n = 0; n < MY_LOADS; ++n) load_one(stage_off, n);
+  };
+  // this group's turns are turns grp, grp + NG, ...; i counts them, and turn i goes through stage i % ST
+  const int n_turns = max(0, (n_blk + 1) / 2), n_iter = (n_turns + NG - 1) / NG;      // n_iter: the first group's, the most
+  const int my_turns = max(0, (n_turns - grp + NG - 1) / NG);
   constexpr int AHEAD = ST - 1;
   // The queries of a workgroup of many groups, which all take the same rows, come through LDS as well: QL loads a wavefront of whole rows (piece c
   // of row r in place c ^ (r & (NP - 1))).  As operands from memory, a row in every lane, they were 64 loads a tile of 64 cycles each of the unit that
@@ -1324,21 +1353,20 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
       const int g = wid + NG * NW * j, r = g * K_ROWS + lane / NP;
       const char* src = rows + (size_t)min(first + r, row_end - 1) * ((size_t)n_head * HD * 2) + (((lane % NP) ^ (r & (NP - 1))) << 4);
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                       (__attribute__((address_space(3))) void*)(size_t)((unsigned)(size_t)smem + NG * ST * STAGE + g * 1024), 16, 0, 0);
+                                       (__attribute__((address_space(3))) void*)(size_t)((unsigned)(size_t)smem + Lds::QUERIES + g * 1024), 16, 0, 0);
     }
   }
   // the first run's blocks and first turns are asked for before the queries are waited for: those arrive meanwhile
   // (a workgroup whose run of keys is empty walks nothing, and nothing may be on its way into LDS
   // when it goes on to the merge)
-  int under_way = 0;
-  if (blk_lo <= blk_hi) {
-    const int nblk = min(64, blk_hi + 1 - blk_lo);
-    run_blocks(blk_lo, nblk);
-    const int my_turns = ((nblk + 1) / 2 - grp + NG - 1) / NG;
-    under_way = min(AHEAD, my_turns);
+  const int under_way = min(AHEAD, my_turns);
+  if (n_turns) {
+    ask_run(0);
+    place_run(0);
 #pragma unroll
     for (int i = 0; i < AHEAD; ++i)
-      if (i < my_turns) issue(i, i * STAGE);
+      if (i < my_turns) issue(i, i * NEXT);
+    if (n_blk > 64) ask_run(1);
   }
 
   v4u qf[CB][KS];
@@ -1349,7 +1377,7 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
     __builtin_amdgcn_s_barrier();
     static_assert(CB == 1, "a column block a wavefront");
     const int r = wave * 32 + r32;
-    const unsigned at = (unsigned)(size_t)smem + NG * ST * STAGE + r * (HD * 2);
+    const unsigned at = (unsigned)(size_t)smem + Lds::QUERIES + r * (HD * 2);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
       asm volatile("ds_read_b128 %0, %1" : "=v"(qf[0][ks]) : "v"(at + (((ks * 2 + h) ^ (r & (NP - 1))) << 4)));
@@ -1390,8 +1418,8 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   // One turn of 32 keys from a stage for this wavefront's columns, in two steps: the scores, then the
   // softmax and the second product.  plain (the same in every lane): every key of the turn is visible
   // to every column and written: no compare at all.
-  auto turn_scores = [&](auto stage_tag, floatx16* sc) __attribute__((always_inline)) {
-    constexpr unsigned SOFF = decltype(stage_tag)::value * STAGE;
+  auto turn_scores = [&](auto stage_tag, floatx16* sc, auto between) __attribute__((always_inline)) {
+    constexpr unsigned SOFF = decltype(stage_tag)::value * NEXT;
     // ---- the fragments: keys now, values right behind them
     v4u kf[KS];
 #pragma unroll
@@ -1410,18 +1438,19 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
         }
         sc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kf[ks]),
                                                          __builtin_bit_cast(bf16x8, qf[cb][ks]), sc[cb], 0, 0, 0);
+        if (cb == 0) between(ks);
       }
     }
   };
   auto turn_rest = [&](auto stage_tag, int key0, bool plain, const floatx16* sc) __attribute__((always_inline)) {
-    constexpr unsigned SOFF = decltype(stage_tag)::value * STAGE;
+    constexpr unsigned SOFF = decltype(stage_tag)::value * NEXT;
     // the value fragments are asked for now and waited for after the softmax
     v4u vf[DB][2];
 #pragma unroll
     for (int d = 0; d < DB; ++d)
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
-        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(vf[d][tt]) : "v"(v_addr[tt]), "n"(SOFF + d * 32 * 64));
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(vf[d][tt]) : "v"(v_addr), "n"(SOFF + tt * (HD * 32) + d * 1024));
 
     // ---- masks, the online softmax and O^T += V^T . P^T, column block by column block: the matrix
     // core works on one block's second product while the next block's softmax runs.  The scores stay
@@ -1524,49 +1553,61 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
     }
   };
 
-  for (int c0 = blk_lo; c0 <= blk_hi; c0 += 64) {
-    const int nblk = min(64, blk_hi + 1 - c0);
-    const int n_turns = (nblk + 1) / 2;
-    // this group's turns are turns grp, grp + NG, ... of the run; i counts them, and turn i of a run
-    // goes through stage i % ST
-    const int my_turns = (n_turns - grp + NG - 1) / NG;
-    const int n_iter = (n_turns + NG - 1) / NG;                      // the first group's count: the most
-    if (c0 != blk_lo) {
-      run_blocks(c0, nblk);
+  // Run 1 has been asked for, with the first turns on their way; the others are asked for as the loads enter the run before, and placed a turn
+  // later.
+  int placed = 0, entered = 0;      // the last run placed, and the last that loads have been asked from
+  for (int i0 = 0; i0 < n_iter; i0 += ST) {
+    // ST turns, each with its stage as a constant
+    unrolled_while<ST>([&](auto si_tag) __attribute__((always_inline)) {
+      constexpr int si = decltype(si_tag)::value;
+      const int i = i0 + si;
+      if (i >= n_iter) return false;
+      // this wavefront's part of the group's turn i has landed: only its turns issued after it (at
+      // most AHEAD - 1) may be outstanding.  Then the group's wavefronts wait for each other: the
+      // whole turn has landed, and everyone is done with the turn before, whose stage turn
+      // i + AHEAD goes into.
+      vm_wait_turns<MY_LOADS, ST>(max(0, min(AHEAD - 1, my_turns - 1 - i)));
+      group_sync();
+      const int key0 = (blk_lo + 2 * (i * NG + grp)) * 16;
+      // nothing of this turn is visible to this wavefront: it only helps loading
+      const bool idle = i >= my_turns || w_rows == 0 || key0 > w_pos_last || key0 + PF_KEYS - 1 < w_lo;
+      const bool more = i + AHEAD < my_turns;
+      if (more) {
+        if (placed == entered && 64 * (entered + 1) < n_blk) place_run(++placed);
+        const int r = ((i + AHEAD) * NG + grp) >> 5;
+        find_turn(i + AHEAD);
+        if (idle) {
 #pragma unroll
-      for (int i = 0; i < AHEAD; ++i)
-        if (i < my_turns) issue(i, i * STAGE);
-    }
-    for (int i0 = 0; i0 < n_iter; i0 += ST) {
-      // ST turns, each with its stage as a constant; ends with the run
-      unrolled_while<ST>([&](auto si_tag) __attribute__((always_inline)) {
-        constexpr int si = decltype(si_tag)::value;
-        const int i = i0 + si;
-        if (i >= n_iter) return false;
-        // this wavefront's part of the group's turn i has landed: only its turns issued after it (at
-        // most AHEAD - 1) may be outstanding.  Then the group's wavefronts wait for each other: the
-        // whole turn has landed, and everyone is done with the turn before, whose stage turn
-        // i + AHEAD goes into.
-        vm_wait_turns<MY_LOADS, ST>(max(0, min(AHEAD - 1, my_turns - 1 - i)));
-        group_sync();
-        // turn i + AHEAD goes into the stage that turn i - 1 has left
-        if (i + AHEAD < my_turns) issue(i + AHEAD, ((si + AHEAD) % ST) * STAGE);
-        if (i >= my_turns) return true;
-        const int key0 = (c0 + 2 * (i * NG + grp)) * 16;
-        // nothing of this turn is visible to this wavefront: it only helps loading
-        if (w_rows == 0 || key0 > w_pos_last || key0 + PF_KEYS - 1 < w_lo) return true;
-        const bool plain = (key0 + PF_KEYS - 1 <= w_pos_first) && (w_rows == WROWS) &&
-                           (window <= 0 || key0 >= w_pos_last - window + 1);
-        floatx16 sc[CB];
-        turn_scores(si_tag, sc);
-        turn_rest(si_tag, key0, plain, sc);
-        return true;
-      });
-    }
-    // every wavefront of the group is done with this run's stages before the next run (or the merge)
-    // writes into them
-    group_sync();
+          for (int n = 0; n < MY_LOADS; ++n) load_one(((si + AHEAD) % ST) * NEXT, n);
+        }
+        if (r != entered) {
+          entered = r;
+          if (64 * (r + 1) < n_blk) ask_run(r + 1);
+        }
+      }
+      if (idle) return true;
+      // Turn i + AHEAD goes into the stage that turn i - 1 has left, a load behind each of the first product's matrix instructions: asked for
+      // at once the wavefronts' loads queue at the unit that takes addresses, and nothing is on the matrix cores meanwhile (2,048 tokens
+      // 32.7 us, so 32.0; 6,000 228, 224).
+      constexpr unsigned to = ((si + AHEAD) % ST) * NEXT;
+      floatx16 sc[CB];
+      if (more)
+        turn_scores(si_tag, sc, [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+          for (int n = 0; n < MY_LOADS; ++n)
+            if (n * KS / MY_LOADS == ks) load_one(to, n);
+          __builtin_amdgcn_sched_barrier(0);
+        });
+      else
+        turn_scores(si_tag, sc, [](int) {});
+      const bool plain = (key0 + PF_KEYS - 1 <= w_pos_first) && (w_rows == WROWS) &&
+                         (window <= 0 || key0 >= w_pos_last - window + 1);
+      turn_rest(si_tag, key0, plain, sc);
+      return true;
+    });
   }
+  // every wavefront of the group is done with the stages before the merge (or the next tile) writes into them
+  group_sync();
 
   // ---- the result: o[cb][d][i] is dim 32 d + 8 (i / 4) + 4 h + i % 4 of token (column) r32 of block cb.
   // `first_val`, `count_tag`: which of a lane's DB * 16 values of a block (value v = 16 d + i) these are; a
@@ -1615,7 +1656,7 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
     // now 7.05, 2,048 at 32 heads 73.2, now 70.0).
     constexpr int VALS = DB * 16, VPG = VALS / NG, FOURS = (VALS - VPG) / 4, PART = (FOURS * 16 + 8) * 64;
     static_assert(VALS % NG == 0 && VPG % 4 == 0, "a group owns whole fours of values");
-    static_assert(NG * NW * PART <= NG * ST * STAGE, "the partial results fit into the stages");
+    static_assert(NG * NW * PART <= Lds::QUERIES, "the partial results fit into the stages");
     typedef __attribute__((address_space(3))) floatx4 lds_four;
     typedef __attribute__((address_space(3))) ti_float2v lds_two;
     // slot i (values 4 i .. of those left) of group g's wavefront, and behind the slots its maximum and sum
@@ -1841,13 +1882,16 @@ extern "C" int ti_attention_decode_prepared_bf16(const float* qkv, int row_width
                              n_head, n_kv, hd, page_size, scale, window, n_splits, prep, stream);
 }
 
+// What the kernels through LDS reach behind a block's descriptor: a page of all heads' keys and values.
+static bool prefill_page_fits(int n_kv, int hd, int P) { return 4L * n_kv * P * hd < 0x7fffffffL; }
+
 static int g_prefill_groups = 0;   // for measurements: 1 or 2 wavefront groups per workgroup, 0 = by the launch
 static int g_prefill_lds = 1;
 static int g_decode_stages = 0;    // LDS stages a wavefront of the decode kernel by records at a head size of 128, 0 = by the launch
 // 1: head sizes 64 and 128 take the kernel that shares keys and values through LDS
 // (default); 0: every head size takes the kernel that reads them per wavefront
 
-// Portions of prompts.  tiles: int [n_tiles, 2] = (entry, first row), each tile 128 rows;
+// Portions of prompts.  tiles: int [n_tiles, 2] = (entry, first row), each tile 128 rows, best from the one that sees the most keys on;
 // entries: int [n_entries, 4] = (row0, n_tokens, start_pos, -); table row e belongs to entry e.
 extern "C" int ti_attention_prefill_bf16(const void* q, const void* pool, const int* table, int table_stride,
                                          const int* tiles, const int* entries, void* out, int n_tiles,
@@ -1858,7 +1902,7 @@ extern "C" int ti_attention_prefill_bf16(const void* q, const void* pool, const 
   TI_REQUIRE(n_head <= 65535, "attention_prefill: too many heads");
   if (n_tiles == 0) return 0;
   dim3 grid(n_tiles, n_head);
-  if (g_prefill_lds && (hd == 64 || hd == 128)) {
+  if (g_prefill_lds && (hd == 64 || hd == 128) && prefill_page_fits(n_kv, hd, page_size)) {
     // two groups of wavefronts per workgroup when the launch would else leave a SIMD with one wavefront
     const int groups = g_prefill_groups ? g_prefill_groups : ((long)n_tiles * n_head < 512 ? 2 : 1);
     const int lds = groups * PF_STAGES * 2 * PF_KEYS * hd * 2;
@@ -1921,23 +1965,26 @@ extern "C" int ti_attention_prefill_paired_bf16(const void* q, const void* pool,
     ti_set_error("attention_prefill_paired: head_dim 32 is not served (64, 128)");
     return 3;
   }
+  if (!prefill_page_fits(n_kv, hd, page_size)) {
+    ti_set_error("attention_prefill_paired: pages of 2 GiB and more are not served");
+    return 3;
+  }
   TI_REQUIRE(n_head <= 65535, "attention_prefill_paired: too many heads");
   TI_REQUIRE(n_splits >= 1 && n_splits <= 8 && (n_splits == 1 || (part_o && part_ml && n_rows > 0)),
              "attention_prefill_paired: 1 to 8 runs of keys, more than one with buffers for their results");
   if (n_tiles == 0) return 0;
   constexpr int NG = 4, NW = 2, ST = 2, CB = 1;
-  constexpr int LDS = NG * ST * 2 * PF_KEYS * 2 + 32 * NW * CB * 2;      // per head dimension: the stages, and the queries
-  const int lds = LDS * hd;
+  const int lds = hd == 128 ? PrefillLds<128, NG, NW, ST>::BYTES : PrefillLds<64, NG, NW, ST>::BYTES;
   static bool ready = false;          // allow more than 64 KiB of dynamic LDS, once
   if (!ready) {
     if (hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<128, NG, NW, ST, true, CB>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS * 128) != hipSuccess ||
+                            hipFuncAttributeMaxDynamicSharedMemorySize, PrefillLds<128, NG, NW, ST>::BYTES) != hipSuccess ||
         hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<64, NG, NW, ST, true, CB>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS * 64) != hipSuccess ||
+                            hipFuncAttributeMaxDynamicSharedMemorySize, PrefillLds<64, NG, NW, ST>::BYTES) != hipSuccess ||
         hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<128, NG, NW, ST, false, CB>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS * 128) != hipSuccess ||
+                            hipFuncAttributeMaxDynamicSharedMemorySize, PrefillLds<128, NG, NW, ST>::BYTES) != hipSuccess ||
         hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<64, NG, NW, ST, false, CB>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, LDS * 64) != hipSuccess) {
+                            hipFuncAttributeMaxDynamicSharedMemorySize, PrefillLds<64, NG, NW, ST>::BYTES) != hipSuccess) {
       ti_set_error("attention_prefill_paired: cannot reserve the LDS");
       return 2;
     }
@@ -2034,18 +2081,23 @@ extern "C" int ti_attention_step_bf16(const void* q, const void* pool, const int
     ti_set_error("attention_step: head_dim 32 is not served (64, 128)");
     return 3;
   }
+  if (!prefill_page_fits(n_kv, hd, page_size)) {
+    ti_set_error("attention_step: pages of 2 GiB and more are not served");
+    return 3;
+  }
   TI_REQUIRE(n_tiles > 0 && tiles && entries, "attention_step: no tiles");
   rc = check_runs("attention_step", runs, n_runs, run_stride, rows, n_rows, part_o, part_ml);
   if (rc) return rc;
   const int parts = (n_head / n_kv + 15) / 16;
   const long grid = (long)n_tiles * n_head + (long)n_runs * n_kv * parts;
   TI_REQUIRE(grid <= 0x7fffffL, "attention_step: too many workgroups");
-  constexpr int STAGES = 4 * 2 * 2 * PF_KEYS * 2 + 64 * 2;      // bytes of the tiles' stages and queries per head dimension
-  static_assert(sizeof(StagedMerge<128, 8, 1>) <= STAGES * 128 && sizeof(StagedMerge<64, 8, 1>) <= STAGES * 64, "the runs' stages and merge fit");
+  typedef PrefillLds<128, 4, 2, 2> Lds128;
+  typedef PrefillLds<64, 4, 2, 2> Lds64;
+  static_assert(sizeof(StagedMerge<128, 8, 1>) <= Lds128::BYTES && sizeof(StagedMerge<64, 8, 1>) <= Lds64::BYTES, "the runs' stages and merge fit");
   static bool ready = false;          // allow more than 64 KiB of dynamic LDS, once
   if (!ready) {
-    if (hipFuncSetAttribute((const void*)attn_step_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, STAGES * 128) != hipSuccess ||
-        hipFuncSetAttribute((const void*)attn_step_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize, STAGES * 64) != hipSuccess) {
+    if (hipFuncSetAttribute((const void*)attn_step_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, Lds128::BYTES) != hipSuccess ||
+        hipFuncSetAttribute((const void*)attn_step_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize, Lds64::BYTES) != hipSuccess) {
       ti_set_error("attention_step: cannot reserve the LDS");
       return 2;
     }
@@ -2054,7 +2106,7 @@ extern "C" int ti_attention_step_bf16(const void* q, const void* pool, const int
   const float cap = softcap > 0.f ? softcap : 0.f;
 #define TI_GO(H)                                                                                                              \
   do {                                                                                                                        \
-    attn_step_kernel<H><<<(unsigned)grid, 512, STAGES * H, stream>>>((const bf16_t*)q, (const bf16_t*)pool, table, table_stride, \
+    attn_step_kernel<H><<<(unsigned)grid, 512, Lds##H::BYTES, stream>>>((const bf16_t*)q, (const bf16_t*)pool, table, table_stride, \
                                                                      tiles, n_tiles, entries, runs, run_stride, n_head / n_kv,  \
                                                                      (bf16_t*)out, part_o, part_ml,                              \
                                                                      n_head, n_kv, page_size, scale, window, cap, g_sink);       \

@@ -660,9 +660,9 @@ struct AttentionWork {
   const int* positions = nullptr;    // [M]
   const int* slots = nullptr;        // [M] row of the block table
   const int* entry_meta = nullptr;   // [R][4] = (row0, n_tokens, start_pos, state slot)
-  const int* tiles = nullptr;        // [n_tiles][2] = (entry, first row) of 128 query rows
+  const int* tiles = nullptr;        // [n_tiles][2] = (entry, first row) of 128 query rows, from the most visible keys to the fewest
   int n_tiles = 0;
-  const int* tiles_small = nullptr;  // the same in tiles of 64 rows, from the most visible keys to the fewest
+  const int* tiles_small = nullptr;  // the same in tiles of 64 rows
   int n_tiles_small = 0;
   const int* decode_rows = nullptr;  // rows of single-token entries (null when every entry is one)
   int n_decode_rows = 0;

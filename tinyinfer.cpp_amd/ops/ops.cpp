@@ -930,13 +930,16 @@ static const int PORTION_SPLIT_KEYS = 512;   // a portion's keys are cut into ru
 static const int PORTION_SPLIT_MAX = 8;      // ... at most this many runs
 static const int PAIRED_BELOW = 1025;        // (tiles of 128 rows) x heads below which a launch takes the paired kernel
 
-// A launch whose tiles all find a compute unit at once gives each tile a workgroup of its own (it
-// lasts as long as its heaviest tile then); a larger one pairs the heaviest tile with the lightest.
+// Tiles of 64 rows get a workgroup each, the heaviest first.  Where they are two rounds of the units, or nearly, a workgroup takes the heaviest
+// and the lightest of those left, which spares the second round's starts (us, pairs and a workgroup each: 16 heads of 2,048 tokens 34.3
+// and 35.3, of 1,984 32.9 and 33.9, of 1,920 33.3 and 33.3, of 1,792 31.2 and 30.7, of 1,500 29.6 and 25.7, of 2,176 63.6 and 41.9, of
+// 3,000 81 and 66.5; 32 heads of 1,024 23.1 and 24.1).
 // The keys are cut into runs when the launch would leave most units idle (a short portion) while
 // every workgroup walks a long context.
 int Ops::portion_launch(int n_tiles_small, int heads, int portion_context, int window, int units, bool* paired) {
   const int context = window == 0 ? portion_context : std::min(portion_context, window + 64);
-  const bool pair = n_tiles_small * heads > units;
+  const long tiles = (long)n_tiles_small * heads;
+  const bool pair = 10 * tiles > 19L * units && tiles <= 2L * units;
   if (paired) *paired = pair;
   const int workgroups = std::max(1, (pair ? (n_tiles_small + 1) / 2 : n_tiles_small) * heads);
   if (workgroups * 2 > units || context < 2 * PORTION_SPLIT_KEYS) return 1;
@@ -1050,8 +1053,6 @@ bool Ops::attention(const AttentionWork& work, Workspace& ws, const CacheView& v
       // the rows of single tokens get their own result afterwards
       if (work.n_tiles && (head_dim == 64 || head_dim == 128) && work.n_tiles * heads < PAIRED_BELOW && work.tiles_small &&
           use.paired_prefill) {
-        // few tiles: under a causal mask they differ much in work, and a launch lasts as long as its
-        // heaviest workgroup; the paired kernel gives every workgroup a heavy and a light tile
         bool paired = false;
         int S = portion_launch(work.n_tiles_small, heads, work.portion_context, window, units, &paired);
         if (!use.portion_splits) S = 1;

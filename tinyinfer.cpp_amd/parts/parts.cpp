@@ -762,9 +762,9 @@ class Attention final : public MixerPart {
     return n;
   }
 
-  // The work lists of the attention kernels for this step: query tiles of 128 rows in order,
-  // tiles of 64 rows from the one whose last row sees the most keys to the one that sees the
-  // fewest, and the rows of single-token entries.  Every attention part of a model asks for the
+  // The work lists of the attention kernels for this step: query tiles of 128 and of 64 rows, from
+  // the one whose last row sees the most keys to the one that sees the fewest, and the rows of
+  // single-token entries.  Every attention part of a model asks for the
   // same lists; the first one builds them.
   void plan(StepPlan& plan) const override {
     if (!plan.decode_only() && !plan.has("attention.tiles")) plan_tiles(plan);
@@ -857,30 +857,30 @@ class Attention final : public MixerPart {
     int* tiles = plan.ints("attention.tiles", 2 * n_tiles);
     int* small = plan.ints("attention.tiles_small", 2 * n_small);
     int* dec = plan.ints("attention.decode_rows", n_dec);
-    struct Small { int last, entry, row; };
-    std::vector<Small> order;
-    order.reserve(n_small);
+    struct Tile { int last, entry, row; };
+    std::vector<Tile> large, little;
+    large.reserve(n_tiles);
+    little.reserve(n_small);
     int portion_context = 0;
-    size_t t = 0, d = 0;
+    size_t d = 0;
     for (size_t i = 0; i < entries.size(); ++i) {
       const auto& e = entries[i];
       if (e.n_tokens > 1) {
-        for (int q0 = 0; q0 < e.n_tokens; q0 += PREFILL_TILE_Q) {
-          tiles[t++] = (int)i;
-          tiles[t++] = e.row0 + q0;
-        }
+        for (int q0 = 0; q0 < e.n_tokens; q0 += PREFILL_TILE_Q)
+          large.push_back({e.start + std::min(q0 + PREFILL_TILE_Q, e.n_tokens) - 1, (int)i, e.row0 + q0});
         for (int q0 = 0; q0 < e.n_tokens; q0 += PREFILL_TILE_SMALL)
-          order.push_back({e.start + std::min(q0 + PREFILL_TILE_SMALL, e.n_tokens) - 1, (int)i, e.row0 + q0});
+          little.push_back({e.start + std::min(q0 + PREFILL_TILE_SMALL, e.n_tokens) - 1, (int)i, e.row0 + q0});
         portion_context = std::max(portion_context, e.start + e.n_tokens);
       } else {
         dec[d++] = e.row0;
       }
     }
-    std::stable_sort(order.begin(), order.end(), [](const Small& a, const Small& b) { return a.last > b.last; });
-    for (size_t i = 0; i < order.size(); ++i) {
-      small[2 * i] = order[i].entry;
-      small[2 * i + 1] = order[i].row;
-    }
+    const auto list = [](std::vector<Tile>& order, int* out) {
+      std::stable_sort(order.begin(), order.end(), [](const Tile& a, const Tile& b) { return a.last > b.last; });
+      for (const Tile& t : order) *out++ = t.entry, *out++ = t.row;
+    };
+    list(large, tiles);
+    list(little, small);
     plan.set_value("attention.portion_context", portion_context);
   }
 
