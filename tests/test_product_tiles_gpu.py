@@ -41,6 +41,65 @@ def test_every_tile_over_few_k_tiles(ops, M, N, K):  # noqa: F811
     assert ((f64(want[0]) - ref).abs() <= (K + 1) * 2.0 ** -24 * size).all()
 
 
+@pytest.mark.parametrize("tile", [10, 12])
+@pytest.mark.parametrize("M,F,K,shift", [(255, 128, 64, 0), (257, 136, 128, 0), (256, 130, 192, 0), (513, 264, 256, 0), (64, 8, 576, 0), (300, 136, 320, 4)])
+def test_tiles_of_256_by_quarters(ops, tile, M, F, K, shift):  # noqa: F811
+    """The loop by quarters over one k-tile and more than its two stages, rows and columns a tile, one more and one less, columns in
+    whole pieces of 16 bytes and not (130), a result that starts between two pieces (shift): the bits of the 128 x 128 tile."""
+    lib = ops.lib("gemm_bf16")
+    g = torch.Generator().manual_seed(M + F + K)
+    a = dev((torch.rand(M, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    w = dev((torch.rand(2 * F, K, generator=g) * 2 - 1).to(torch.bfloat16))
+    outs = []
+    lib.ti_tuning_set(b"rows_112", 0)
+    lib.ti_tuning_set(b"tiled_from", 1)
+    try:
+        for force in (2, tile):
+            lib.ti_tuning_set(b"force_tile", force)
+            room = torch.full((M * F + 16,), 7.0, device="cuda", dtype=torch.bfloat16)
+            out = room[shift:shift + M * F].view(M, F)
+            ops.linear(a, w, out, "swiglu")
+            assert bool((room[:shift] == 7.0).all()) and bool((room[shift + M * F:] == 7.0).all())
+            outs.append(out.clone())
+    finally:
+        lib.ti_tuning_reset()
+    assert torch.equal(outs[0], outs[1])
+    gate, up = (ref_linear(a.cpu(), w[i * F:(i + 1) * F].cpu()) for i in (0, 1))
+    want = torch.nn.functional.silu(gate) * up
+    # sums of K products within K 2^-24 of their sizes, a result rounded to 8 bits
+    assert ((f64(outs[1]) - want).abs() <= 2.0 ** -8 * want.abs() + (K + 8) * 2.0 ** -24 * K * (1 + up.abs() + gate.abs())).all()
+
+
+@pytest.mark.parametrize("M,F,K,tile", [(2048, 3072, 1024, 10), (2048, 12288, 4096, 12), (512, 3072, 1024, 0), (2000, 2565, 2048, 10)])
+def test_which_gate_up_products_go_by_quarters(ops, M, F, K, tile):  # noqa: F811
+    """Where the costs say so, and with the bits of what is taken without them: two tile shapes for two ranges of columns, or one."""
+    lib = ops.lib("gemm_bf16")
+    assert lib.ti_gemm_bf16_quarters_choice(M, F, K) == tile
+    g = torch.Generator(device="cuda").manual_seed(M + F)
+    a = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(2 * F, K, device="cuda", generator=g) * 0.1).to(torch.bfloat16)
+    outs = []
+    try:
+        for on, ranges in ((1, 1), (0, 1), (0, 0)):
+            lib.ti_tuning_set(b"tiles_256", on)
+            lib.ti_tuning_set(b"two_ranges", ranges)
+            outs.append(torch.empty(M, F, device="cuda", dtype=torch.bfloat16))
+            ops.linear(a, w, outs[-1], "swiglu")
+    finally:
+        lib.ti_tuning_reset()
+    assert torch.isfinite(outs[0]).all()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("M,nh,nkv,hd,K,P,norm,rope", [
+    (300, 3, 1, 128, 128, 16, True, "table"), (513, 5, 1, 64, 256, 32, True, None), (257, 4, 0, 128, 64, 16, False, "computed"),
+    (100, 2, 2, 64, 192, 48, False, "table")])
+def test_qkv_product_in_tiles_of_256_by_256(ops, M, nh, nkv, hd, K, P, norm, rope):  # noqa: F811
+    """The heads finished in two ranges of 128 columns: whole tiles, a second range beyond the last head, rows that are no
+    multiple of the tile.  The bits of the product and the kernel that prepares whole steps."""
+    qkv_prepared_case(ops, 512, M, nh, nkv, hd, K, P, norm, rope)
+
+
 @pytest.mark.parametrize("M,N,K", [(1024, 1024, 128), (2048, 512, 128), (512, 2048, 64), (384, 1152, 64)])
 def test_dies_blocks_cover_every_tile_once(ops, M, N, K):  # noqa: F811
     """Grids that the eight dies cut by rows, by columns and by both, and one that none of the cuts divides."""

@@ -1103,6 +1103,9 @@ __device__ __forceinline__ void qkv_rows_by_lanes(const QKVEpilogue& ep, float* 
     qkv_rows_by_lanes<HD, BM, NWV, FS, false, false>(ep, ft, s_pos, s_page, s_prow, s_live, hh, u, m0);
 }
 
+// LDS of that epilogue: 128 columns of a tile of bm rows in 32-bit, and four words a row.
+constexpr int qkv_prep_lds(int bm, int bn) { return bm * ((bn < 128 ? bn : 128) + 8) * 4 + 4 * bm * 4; }
+
 // tile(n_k - LEFT, LEFT) for LEFT = STAGES - 2, ..., 0, as far as there are tiles
 template <class Tile, int... I>
 __device__ __forceinline__ void last_tiles(int n_k, Tile&& tile, std::integer_sequence<int, I...>) {
@@ -1110,7 +1113,8 @@ __device__ __forceinline__ void last_tiles(int n_k, Tile&& tile, std::integer_se
   ((n_k >= N - I ? (tile(n_k - (N - I), std::integral_constant<int, N - 1 - I>{}), 0) : 0), ...);
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int STAGES = PSTAGES>
+// PHASED: the multiply loop goes by quarters of a wavefront's tile, for tiles of 256 x 256 (see the loop).
+template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int STAGES = PSTAGES, bool PHASED = false>
 __global__ void __launch_bounds__(WAVES_M * WAVES_N * 64)
 gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ out_arg,
                       int M, int N, int K, long lda, int n_first, int xcd_rows, int die_rows, QKVEpilogue ep = QKVEpilogue{}) {
@@ -1162,19 +1166,31 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
   const int n0 = n_first + bx * (SW ? BN / 2 : BN);
   const int lr = lane / CPR, lc = lane % CPR;                // row within a load's group of rows, slot within the row
 
+  // Which group of RPL rows this wavefront's load i brings: 0 .. GROUPS_A - 1 of A, then of B, the weight's rows or, SwiGLU, its up rows.
+  // PHASED: the first half of the loads brings the first halves of every wavefront's rows of A and of B, the second half the others.
+  constexpr int span = BN / WAVES_N, half = span / 2;        // SwiGLU: a wavefront's columns are gate rows, then up rows
+  constexpr int HA = GROUPS_A / 2 / NWV, HB = GROUPS_B / 2 / NWV;
+  auto half_group = [](int rows, int second, int x) { return x / (rows / 2 / RPL) * (rows / RPL) + second * (rows / 2 / RPL) + x % (rows / 2 / RPL); };
+  auto group_of = [&](int i) {
+    if constexpr (!PHASED) return wave + NWV * i;
+    else if (i < HA) return half_group(BM / WAVES_M, 0, wave + NWV * i);
+    else if (i < HA + 2 * HB) return GROUPS_A + half_group(span, i < HA + HB ? 0 : 1, wave + NWV * ((i - HA) % HB));
+    else return half_group(BM / WAVES_M, 1, wave + NWV * (i - HA - 2 * HB));
+  };
+  auto of_a = [&](int i, int g) { return PHASED ? i < HA || i >= HA + 2 * HB : g < GROUPS_A; };
+  auto of_up = [&](int i, int g) { return SW && (PHASED ? i >= HA + HB : ((g - GROUPS_A) * RPL) % span >= half); };      // (of B's)
   // A load's rows lie behind one of three descriptors (tokens, weight rows, up rows), which are scalar, as is where a k-tile
   // starts; a lane's own offset stays the same from tile to tile, so that a load costs no vector arithmetic.  Rows beyond
   // the matrix are clamped into it: they are computed and thrown away.
   unsigned voff[LOADS];
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
-    const int g = wave + NWV * i;                            // groups 0..GROUPS_A-1: A, then B
-    if (g < GROUPS_A) {
+    const int g = group_of(i);
+    if (of_a(i, g)) {
       const int row = g * RPL + lr;
       voff[i] = (unsigned)min(row, M - 1 - m0) * (unsigned)(lda * 2) + (lc ^ swz(row)) * 16;
     } else {
       const int row = (g - GROUPS_A) * RPL + lr;
-      constexpr int span = BN / WAVES_N, half = span / 2;    // SwiGLU: a wavefront's columns are gate rows, then up rows
       const int n = SW ? (row / span) * half + (row % half) : row;
       voff[i] = (unsigned)min(n, N - 1 - n0) * (unsigned)(K * 2) + (lc ^ swz(row)) * 16;
     }
@@ -1185,11 +1201,10 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
   const auto rsU = rows_at(W + (size_t)(n0 + (SW ? N : 0)) * K + (size_t)kt0 * KT);
   // load i of this wavefront's LOADS loads of k-tile kt, into the stage at that byte
   auto issue_one = [&](int kt, unsigned stage, int i) {
-    const int g = wave + NWV * i;
+    const int g = group_of(i);
     auto* dst = (__attribute__((address_space(3))) void*)(smem + stage + g * 1024);      // the same in every lane
-    constexpr int span = BN / WAVES_N;
-    if (g < GROUPS_A) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, dst, 16, voff[i], kt * KT * 2, 0, 0);
-    else if (SW && ((g - GROUPS_A) * RPL) % span >= span / 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsU, dst, 16, voff[i], kt * KT * 2, 0, 0);
+    if (of_a(i, g)) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, dst, 16, voff[i], kt * KT * 2, 0, 0);
+    else if (of_up(i, g)) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsU, dst, 16, voff[i], kt * KT * 2, 0, 0);
     else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsW, dst, 16, voff[i], kt * KT * 2, 0, 0);
   };
 
@@ -1230,102 +1245,236 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
   // the residual an adding epilogue adds to: asked for while the last k-tile is multiplied
   // (elements outside the matrix read a valid one and are not stored)
   // (a tile of many accumulators has no registers for it and reads the residual in the epilogue)
-  constexpr bool PREV = EPI == TI_EPI_ADD_F32 && (NWV == 4 || TM * TN <= 4);
+  constexpr bool PREV = !PHASED && EPI == TI_EPI_ADD_F32 && (NWV == 4 || TM * TN <= 4);
   float prev[PREV ? TM : 1][PREV ? TN : 1][16];
-  constexpr int NR = TM + TN, NM = TM * TN;                  // fragment reads and matrix instructions of a k-step
-  constexpr int GB = NM >= 8 ? 2 : 0;
-  // matrix instructions of a k-tile that its loads are spread over: up to the barrier; where only one k-tile is ahead the
-  // first quarter, so that the loads have the rest of the tile to arrive in
-  constexpr int SPAN = STAGES == 2 ? NM : (KSTEPS - 1) * NM + GB + 1;
-  v4u fa[2][TM], fb[2][TN];
-  // fragment j of k-step ks of the stage at byte st
-  auto read_one = [&](unsigned st, int ks, int set, int j) {
-    const unsigned pa = rowA + st + xo[ks], pb = rowB + st + xo[ks];
-#pragma unroll
-    for (int a = 0; a < TM; ++a)
-      if (a == j) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][a]) : "v"(pa), "n"(a * 32 * ROWB));
-#pragma unroll
-    for (int b = 0; b < TN; ++b)
-      if (b == j - TM) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[set][b]) : "v"(pb), "n"(b * 32 * ROWB));
-  };
-#pragma unroll
-  for (int t = 0; t < STAGES - 1; ++t)
-    if (t < n_k) {
-#pragma unroll
-      for (int i = 0; i < LOADS; ++i) issue_one(t, t * STAGE_BYTES, i);
-    }
-  if (n_k >= STAGES - 1) wait_vmcnt<(STAGES - 2) * LOADS>();
-  else wait_vmcnt<0>();
-  __builtin_amdgcn_s_barrier();
-  if (n_k > 0) {
-#pragma unroll
-    for (int j = 0; j < NR; ++j) read_one(0, 0, 0, j);
-  }
-  unsigned st = 0, st_new = (STAGES - 1) * STAGE_BYTES;      // where tile kt lies, where tile kt + STAGES - 1 goes
-  // LEFT: how many tiles follow tile kt (STAGES: at least STAGES - 1)
-  auto tile = [&](int kt, auto left) {
-    constexpr int LEFT = decltype(left)::value;
-    constexpr bool MORE = LEFT >= STAGES - 1, NEXT = LEFT >= 1;
-    const unsigned st_next = st == (STAGES - 1) * STAGE_BYTES ? 0 : st + STAGE_BYTES;
-    if constexpr (PREV && LEFT == 0) {
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int m = m0 + wm * (BM / WAVES_M) + a * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-            const int n = n0 + wn * (BN / WAVES_N) + b * 32 + (lane & 31);
-            prev[a][b][i] = ((const float*)out_)[(size_t)min(m, M - 1) * N + min(n, N - 1)];
-          }
-    }
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      const int set = ks & 1;
-      constexpr int LAST = KSTEPS - 1;
-      // this step's fragments have arrived (the next step's are asked for below); tied to the wait, so that no
-      // matrix instruction is moved above it
+  if constexpr (PHASED) {
+    // By quarters: a phase multiplies half of the wavefront's rows of A with half of its rows of B over the whole k-tile, and the fragments of
+    // a half stay in registers as long as they are used, so that a half's bytes of LDS are free again when they have been read once:
+    //   lo x lo (reads B hi)   lo x hi (reads A hi)   hi x lo (reads the next k-tile's A lo)   hi x hi (reads its B lo)
+    // The workgroup meets twice a k-tile.  In the first phase A lo and B lo are free, and B hi and A hi have landed; in the third the other
+    // way round, of the next k-tile.  What is freed is asked for again at once: with two stages, which are all that LDS holds
+    // of this tile, a load has a k-tile and a half to arrive in.  (In the loop below it has three quarters of one, and a k-tile of 256 x 256 takes
+    // as long as memory does: 1.60 us on all units, 1.09 on eight, matrix instructions alone 1.17 and 0.87; by quarters 1.54 and 0.95 by
+    // eight wavefronts, 1.45 and 0.92 by four, which read LDS the least.  Tiles of 256 x 128 and 128 x 128, whose three
+    // and four stages are as deep as that, gain nothing.)  The sums are taken in the same order: the same bits.
+    constexpr int HM = TM / 2, HN = TN / 2, G = HA + HB;     // blocks of a half; loads of half a stage
+    constexpr int NP = KSTEPS * HM * HN;                     // matrix instructions of a phase
+    constexpr int AR = KSTEPS * HM, BR = KSTEPS * HN;        // reads of a half
+    constexpr int GB = 1;                                    // matrix instructions in front of a meeting
+    static_assert(GROUPS_A % (2 * NWV) == 0 && GROUPS_B % (2 * NWV) == 0 && TM % 2 == 0 && TN % 2 == 0, "halves of whole loads and blocks");
+    static_assert(LOADS == 2 * G && NP > GB, "two groups of loads a k-tile");
+    v4u fa[2][HM][KSTEPS], fb[2][HN][KSTEPS];
+    auto read_a = [&](unsigned st, int h, int j) {
+      const int ks = j / HM, a = j % HM;
+      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[h][a][ks]) : "v"(rowA + st + xo[ks]), "n"((h * HM + a) * 32 * ROWB));
+    };
+    auto read_b = [&](unsigned st, int h, int j) {
+      const int ks = j / HN, b = j % HN;
+      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[h][b][ks]) : "v"(rowB + st + xo[ks]), "n"((h * HN + b) * 32 * ROWB));
+    };
+    // all reads asked for have arrived; tied to the wait, so that no matrix instruction is moved above it
+    auto arrived = [&](int a_half, int b_half) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (a_half >= 0) {
 #pragma unroll
-      for (int a = 0; a < TM; ++a) asm volatile("" : "+v"(fa[set][a]));
+        for (int j = 0; j < AR; ++j) asm volatile("" : "+v"(fa[a_half][j % HM][j / HM]));
+      }
+      if (b_half >= 0) {
 #pragma unroll
-      for (int b = 0; b < TN; ++b) asm volatile("" : "+v"(fb[set][b]));
+        for (int j = 0; j < BR; ++j) asm volatile("" : "+v"(fb[b_half][j % HN][j / HN]));
+      }
+    };
+    auto meet = [&]() {
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto phase = [&](int ah, int bh, auto behind) {          // behind(g): what follows matrix instruction g
 #pragma unroll
-      for (int g = 0; g < NM; ++g) {
-        const int a = g / TN, b = g % TN;
-        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[set][a]),
-                                                            __builtin_bit_cast(bf16x8, fb[set][b]), acc[a][b], 0, 0, 0);
+      for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+        for (int a = 0; a < HM; ++a)
+#pragma unroll
+          for (int b = 0; b < HN; ++b) {
+            floatx16& c = acc[ah * HM + a][bh * HN + b];
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[ah][a][ks]), __builtin_bit_cast(bf16x8, fb[bh][b][ks]), c, 0, 0, 0);
+            behind((ks * HM + a) * HN + b);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+    };
+#pragma unroll
+    for (int t = 0; t < STAGES; ++t)
+      if (t < n_k) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) issue_one(t, t * STAGE_BYTES, i);
+      }
+    if (n_k >= STAGES) wait_vmcnt<(2 * STAGES - 1) * G>();
+    else wait_vmcnt<0>();
+    meet();
+    if (n_k > 0) {
+#pragma unroll
+      for (int j = 0; j < AR; ++j) read_a(0, 0, j);
+#pragma unroll
+      for (int j = 0; j < BR; ++j) read_b(0, 0, j);
+      arrived(0, 0);
+    }
+    unsigned st = 0;                                         // where tile kt lies
+    // LEFT: how many tiles follow tile kt (STAGES: at least STAGES)
+    auto tile = [&](int kt, auto left) {
+      constexpr int LEFT = decltype(left)::value;
+      constexpr bool MORE = LEFT >= STAGES, AFTER = LEFT >= 1;
+      const unsigned st_next = st == (STAGES - 1) * STAGE_BYTES ? 0 : st + STAGE_BYTES;
+      // what has been asked for behind this tile's second group of loads, and behind the next tile's first
+      constexpr int BEHIND_2 = 2 * (LEFT < STAGES - 1 ? LEFT : STAGES - 1) * G;
+      constexpr int BEHIND_1 = AFTER ? (1 + 2 * (LEFT - 1 < STAGES - 2 ? LEFT - 1 : STAGES - 2) + (MORE ? 1 : 0)) * G : 0;
+      auto at = [](int j, int count, int from) { return from + j * (NP / 2) / count; };      // reads behind the first half of a phase
+      phase(0, 0, [&](int g) {
+        if (g == GB) {
+          __builtin_amdgcn_sched_barrier(0);
+          wait_vmcnt<BEHIND_2>();
+          meet();
+        }
+#pragma unroll
+        for (int j = 0; j < BR; ++j)
+          if (at(j, BR, GB) == g) read_b(st, 1, j);
         if (MORE) {
 #pragma unroll
-          for (int i = 0; i < LOADS; ++i)
-            if ((2 * i + 1) * SPAN / (2 * LOADS) == ks * NM + g) issue_one(kt + STAGES - 1, st_new, i);
+          for (int i = 0; i < G; ++i)
+            if (GB + i * (NP - GB) / G == g) issue_one(kt + STAGES, st, i);
         }
-        if (ks < LAST) {
+      });
+      arrived(-1, 1);
+      phase(0, 1, [&](int g) {
 #pragma unroll
-          for (int j = 0; j < NR; ++j)
-            if (j * (NM - 1) / NR == g) read_one(st, ks + 1, set ^ 1, j);
-        } else if (NEXT) {
+        for (int j = 0; j < AR; ++j)
+          if (at(j, AR, 0) == g) read_a(st, 1, j);
+      });
+      arrived(1, -1);
+      phase(1, 0, [&](int g) {
+        if (AFTER) {
           if (g == GB) {
-            // the loads of the tiles behind kt + 1 may still be out
             __builtin_amdgcn_sched_barrier(0);
-            wait_vmcnt<(MORE ? STAGES - 2 : LEFT >= 1 ? LEFT - 1 : 0) * LOADS>();
-            __builtin_amdgcn_s_barrier();
-            __builtin_amdgcn_sched_barrier(0);
+            wait_vmcnt<BEHIND_1>();
+            meet();
           }
-          if (g >= GB) {
+#pragma unroll
+          for (int j = 0; j < AR; ++j)
+            if (at(j, AR, GB) == g) read_a(st_next, 0, j);
+        }
+        if (MORE) {
+#pragma unroll
+          for (int i = 0; i < G; ++i)
+            if (GB + i * (NP - GB) / G == g) issue_one(kt + STAGES, st, G + i);
+        }
+      });
+      phase(1, 1, [&](int g) {
+        if (AFTER) {
+#pragma unroll
+          for (int j = 0; j < BR; ++j)
+            if (at(j, BR, 0) == g) read_b(st_next, 0, j);
+        }
+      });
+      if (AFTER) arrived(0, 0);
+      st = st_next;
+    };
+    for (int kt = 0; kt + STAGES < n_k; ++kt) tile(kt, std::integral_constant<int, STAGES>{});
+    last_tiles(n_k, tile, std::make_integer_sequence<int, STAGES>{});
+  } else {
+    constexpr int NR = TM + TN, NM = TM * TN;                  // fragment reads and matrix instructions of a k-step
+    constexpr int GB = NM >= 8 ? 2 : 0;
+    // matrix instructions of a k-tile that its loads are spread over: up to the barrier; where only one k-tile is ahead the
+    // first quarter, so that the loads have the rest of the tile to arrive in
+    constexpr int SPAN = STAGES == 2 ? NM : (KSTEPS - 1) * NM + GB + 1;
+    v4u fa[2][TM], fb[2][TN];
+    // fragment j of k-step ks of the stage at byte st
+    auto read_one = [&](unsigned st, int ks, int set, int j) {
+      const unsigned pa = rowA + st + xo[ks], pb = rowB + st + xo[ks];
+#pragma unroll
+      for (int a = 0; a < TM; ++a)
+        if (a == j) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[set][a]) : "v"(pa), "n"(a * 32 * ROWB));
+#pragma unroll
+      for (int b = 0; b < TN; ++b)
+        if (b == j - TM) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[set][b]) : "v"(pb), "n"(b * 32 * ROWB));
+    };
+#pragma unroll
+    for (int t = 0; t < STAGES - 1; ++t)
+      if (t < n_k) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) issue_one(t, t * STAGE_BYTES, i);
+      }
+    if (n_k >= STAGES - 1) wait_vmcnt<(STAGES - 2) * LOADS>();
+    else wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    if (n_k > 0) {
+#pragma unroll
+      for (int j = 0; j < NR; ++j) read_one(0, 0, 0, j);
+    }
+    unsigned st = 0, st_new = (STAGES - 1) * STAGE_BYTES;      // where tile kt lies, where tile kt + STAGES - 1 goes
+    // LEFT: how many tiles follow tile kt (STAGES: at least STAGES - 1)
+    auto tile = [&](int kt, auto left) {
+      constexpr int LEFT = decltype(left)::value;
+      constexpr bool MORE = LEFT >= STAGES - 1, NEXT = LEFT >= 1;
+      const unsigned st_next = st == (STAGES - 1) * STAGE_BYTES ? 0 : st + STAGE_BYTES;
+      if constexpr (PREV && LEFT == 0) {
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+          for (int b = 0; b < TN; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const int m = m0 + wm * (BM / WAVES_M) + a * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
+              const int n = n0 + wn * (BN / WAVES_N) + b * 32 + (lane & 31);
+              prev[a][b][i] = ((const float*)out_)[(size_t)min(m, M - 1) * N + min(n, N - 1)];
+            }
+      }
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) {
+        const int set = ks & 1;
+        constexpr int LAST = KSTEPS - 1;
+        // this step's fragments have arrived (the next step's are asked for below); tied to the wait, so that no
+        // matrix instruction is moved above it
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int a = 0; a < TM; ++a) asm volatile("" : "+v"(fa[set][a]));
+#pragma unroll
+        for (int b = 0; b < TN; ++b) asm volatile("" : "+v"(fb[set][b]));
+#pragma unroll
+        for (int g = 0; g < NM; ++g) {
+          const int a = g / TN, b = g % TN;
+          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[set][a]),
+                                                              __builtin_bit_cast(bf16x8, fb[set][b]), acc[a][b], 0, 0, 0);
+          if (MORE) {
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i)
+              if ((2 * i + 1) * SPAN / (2 * LOADS) == ks * NM + g) issue_one(kt + STAGES - 1, st_new, i);
+          }
+          if (ks < LAST) {
 #pragma unroll
             for (int j = 0; j < NR; ++j)
-              if (GB + j * (NM - 1 - GB) / NR == g) read_one(st_next, 0, set ^ 1, j);
+              if (j * (NM - 1) / NR == g) read_one(st, ks + 1, set ^ 1, j);
+          } else if (NEXT) {
+            if (g == GB) {
+              // the loads of the tiles behind kt + 1 may still be out
+              __builtin_amdgcn_sched_barrier(0);
+              wait_vmcnt<(MORE ? STAGES - 2 : LEFT >= 1 ? LEFT - 1 : 0) * LOADS>();
+              __builtin_amdgcn_s_barrier();
+              __builtin_amdgcn_sched_barrier(0);
+            }
+            if (g >= GB) {
+#pragma unroll
+              for (int j = 0; j < NR; ++j)
+                if (GB + j * (NM - 1 - GB) / NR == g) read_one(st_next, 0, set ^ 1, j);
+            }
           }
+          __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
       }
-    }
-    st_new = st;
-    st = st_next;
-  };
-  for (int kt = 0; kt + STAGES - 1 < n_k; ++kt) tile(kt, std::integral_constant<int, STAGES>{});
-  last_tiles(n_k, tile, std::make_integer_sequence<int, STAGES - 1>{});
+      st_new = st;
+      st = st_next;
+    };
+    for (int kt = 0; kt + STAGES - 1 < n_k; ++kt) tile(kt, std::integral_constant<int, STAGES>{});
+    last_tiles(n_k, tile, std::make_integer_sequence<int, STAGES - 1>{});
+  }
 
   // acc[a][b][i]: row wm*(BM/WAVES_M) + a*32 + 8*(i/4) + 4*(lane/32) + i%4, column wn*(BN/WAVES_N) + b*32 + lane%32
   const int ccol = lane & 31, crow = (lane >> 5) * 4;
@@ -1334,20 +1483,26 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
     // lanes finish a row of a q or k head (the arithmetic of the kernel that prepares whole steps; a
     // row's eight lanes read its angles and write its result as runs of consecutive bytes), and a
     // thread a dim of a v head.
+    // (A tile of 256 columns goes in two ranges of 128, which is what LDS holds in 32-bit.)
     static_assert(BM % 64 == 0 && BM <= 256 && NWV == 8, "the first wavefronts look up a row each; 64 rows per pass of all eight");
-    constexpr int FS = BN + 8;                              // row stride: the eight rows x eight lanes of a wavefront
+    constexpr int COLS = BN < 128 ? BN : 128, RANGES = BN / COLS, WN = BN / WAVES_N;
+    static_assert(BN % COLS == 0 && COLS % WN == 0, "a range is whole wavefronts' columns");
+    constexpr int FS = COLS + 8;                            // row stride: the eight rows x eight lanes of a wavefront
                                                             // read 64 different banks
-    static_assert(BM * FS * 4 + 4 * BM * 4 <= STAGES * STAGE_BYTES, "the 32-bit tile fits into the stages");
+    static_assert(qkv_prep_lds(BM, BN) <= (160 << 10), "the 32-bit tile fits into LDS");
     float* ft = reinterpret_cast<float*>(smem);
+#pragma unroll 1
+    for (int range = 0; range < RANGES; ++range) {
     __syncthreads();
+    if (RANGES == 1 || wn * WN / COLS == range) {
 #pragma unroll
-    for (int a = 0; a < TM; ++a)
+      for (int a = 0; a < TM; ++a)
 #pragma unroll
-      for (int i = 0; i < 16; ++i)
+        for (int i = 0; i < 16; ++i)
 #pragma unroll
-        for (int b = 0; b < TN; ++b)
-          ft[(wm * (BM / WAVES_M) + a * 32 + (i >> 2) * 8 + crow + (i & 3)) * FS + wn * (BN / WAVES_N) + b * 32 + ccol] =
-              acc[a][b][i];
+          for (int b = 0; b < TN; ++b)
+            ft[(wm * (BM / WAVES_M) + a * 32 + (i >> 2) * 8 + crow + (i & 3)) * FS + wn * WN % COLS + b * 32 + ccol] = acc[a][b][i];
+    }
     // each row's position, and where its key and value go
     int* s_page = reinterpret_cast<int*>(ft + BM * FS);     // [BM] page of the row's position, -1: none
     int* s_prow = s_page + BM;                              // [BM] row of the position in that page
@@ -1365,8 +1520,8 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
       s_pos[tid] = p;
     }
     __syncthreads();
-    for (int hh = 0; hh < BN / hd; ++hh) {
-      const int u = n0 / hd + hh;                            // the same in every thread
+    for (int hh = 0; hh < COLS / hd; ++hh) {
+      const int u = (n0 + range * COLS) / hd + hh;           // the same in every thread
       if (u >= units) break;
       const bool is_q = u < ep.n_head, is_v = u >= ep.n_head + ep.n_kv;
       if (is_v) {
@@ -1405,7 +1560,38 @@ gemm_pipelined_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W
       else
         qkv_rows_by_lanes<64, BM, NWV, FS>(ep, ft, s_pos, s_page, s_prow, s_live, hh, u, m0);
     }
+    }
     return;
+  }
+  if constexpr (SW) {
+    // Whole pieces of 16 bytes: a wavefront's results through LDS (the stages are free now), and out as runs of its columns.  (Two bytes a lane: 2,048
+    // rows of 6144 x 1024 in tiles of 256 x 256 29.5 us, so 28.2; of 24576 x 4096 by four wavefronts 316 and 305; 512 rows in tiles of 128 x 128
+    // 12.0 and 11.7.)
+    if (N % 8 == 0 && ((uintptr_t)out_ & 15) == 0) {
+      constexpr int ROWS = BM / WAVES_M, COLS = half, LDB = COLS * 2 + 16;      // a wavefront's part, and the bytes from row to row
+      static_assert(NWV * ROWS * LDB <= STAGES * STAGE_BYTES && COLS % 8 == 0 && 64 % (COLS / 8) == 0, "it fits into the stages, rows of whole pieces");
+      __syncthreads();
+      unsigned char* mine = smem + wave * (ROWS * LDB);
+#pragma unroll
+      for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+#pragma unroll
+          for (int b = 0; b < TN / 2; ++b)
+            *reinterpret_cast<bf16_t*>(mine + (a * 32 + (i >> 2) * 8 + crow + (i & 3)) * LDB + (b * 32 + ccol) * 2) =
+                f2bf(silu_mul(acc[a][b][i], acc[a][b + TN / 2][i]));
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      constexpr int EACH = COLS / 8, PASS = 64 / EACH;       // lanes a row, rows a pass
+      const int col = (lane % EACH) * 8, n = n0 + wn * COLS + col;
+#pragma unroll
+      for (int r0 = 0; r0 < ROWS; r0 += PASS) {
+        const int r = r0 + lane / EACH, m = m0 + wm * ROWS + r;
+        const uint4 v = *reinterpret_cast<const uint4*>(mine + r * LDB + col * 2);
+        if (r < ROWS && m < M && n < N) *reinterpret_cast<uint4*>((bf16_t*)out_ + (size_t)m * N + n) = v;
+      }
+      return;
+    }
   }
 #pragma unroll
   for (int a = 0; a < TM; ++a) {
@@ -1468,11 +1654,11 @@ static DieOrder die_order(const dim3& grid, long A, long W) {
   return o;
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int STAGES = PSTAGES>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int EPI, int STAGES = PSTAGES, bool PHASED = false>
 static int launch_pipelined(const bf16_t* A, const bf16_t* W, void* out, int M, int N, int K, long lda,
                             hipStream_t s, int ksplit = 1, int n_first = 0, int n_end = -1) {
   constexpr int bytes = STAGES * (BM + BN) * PBK * 2;
-  auto kernel = gemm_pipelined_kernel<BM, BN, WAVES_M, WAVES_N, EPI, STAGES>;
+  auto kernel = gemm_pipelined_kernel<BM, BN, WAVES_M, WAVES_N, EPI, STAGES, PHASED>;
   static bool ready = false;          // per instantiation: allow more than 64 KiB of dynamic LDS
   if (!ready) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
@@ -1493,7 +1679,7 @@ static int launch_pipelined(const bf16_t* A, const bf16_t* W, void* out, int M, 
 static int g_tiles_160 = 1;      // a hook for measurements: 0 = no tiles of 160 columns
 static int g_tiles_256 = 1;      // a hook for measurements: 0 = no tiles of 256 x 256
 static int g_two_ranges = 1;     // a hook for measurements: 0 = never split the columns between two tile shapes
-static int g_qkv_rows = 0;       // hooks for measurements: 64, 128 or 256 forces the tile's rows;
+static int g_qkv_rows = 0;       // hooks for measurements: 64, 128 or 256 forces the tile's rows, 512 tiles of 256 x 256;
 static int g_qkv_min_rows = 17;  // the fewest rows served (fewer take the kernels with the norm in front)
 
 // What the pipelined kernel takes: k-tiles of 64, and rows whose offsets inside a tile fit its 32-bit load offsets.
@@ -1510,12 +1696,11 @@ static int compute_units() {
   return n;
 }
 
-template <int BM, int WAVES_M, int WAVES_N, int STAGES>
+template <int BM, int WAVES_M, int WAVES_N, int STAGES, int BN = 128, bool PHASED = false>
 static int launch_qkv_prep(const void* A, const void* W, int M, int N, int K, long lda, const QKVEpilogue& ep,
                            hipStream_t stream, int n_first = 0, int n_end = -1) {
-  constexpr int BN = 128;
-  constexpr int bytes = STAGES * (BM + BN) * PBK * 2;
-  auto kernel = gemm_pipelined_kernel<BM, BN, WAVES_M, WAVES_N, TI_EPI_QKV_PREP, STAGES>;
+  constexpr int stages = STAGES * (BM + BN) * PBK * 2, bytes = stages > qkv_prep_lds(BM, BN) ? stages : qkv_prep_lds(BM, BN);
+  auto kernel = gemm_pipelined_kernel<BM, BN, WAVES_M, WAVES_N, TI_EPI_QKV_PREP, STAGES, PHASED>;
   static bool ready = false;
   if (!ready) {
     if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
@@ -1555,9 +1740,13 @@ static const TileRate TILES_PLAIN[] = {
     {3, 128, 64, 2.17f, 0.38f, 0.06f, 3.48f, 0.26f, 0.39f}, {6, 64, 64, 1.27f, 0.20f, 0.05f, 1.96f, 0.19f, 0.22f},
     {8, 128, 160, 4.98f, 0.51f, 0.13f, 0.f, 0.f, 0.f},     {9, 256, 160, 8.03f, 0.63f, 0.35f, 0.f, 0.f, 0.f}};
 static const TileRate TILES_SWIGLU[] = {
-    {10, 256, 256, 5.46f, 1.39f, 0.20f, 0.f, 0.f, 0.f},    {1, 256, 128, 3.08f, 0.56f, 0.28f, 0.f, 0.f, 0.f},
+    {1, 256, 128, 3.08f, 0.56f, 0.28f, 0.f, 0.f, 0.f},
     {2, 128, 128, 0.f, 0.54f, 0.05f, 0.f, 0.f, 0.f},       {7, 64, 128, 0.f, 0.40f, 0.03f, 0.f, 0.f, 0.f},
     {5, 64, 128, 0.f, 0.45f, 0.09f, 0.f, 0.55f, 0.20f}};
+// SwiGLU in tiles of 256 x 256 by quarters, eight wavefronts and four (fitted to 52 products, 200 to 6,000 rows times the four sizes' gate/up: the
+// median error is 1.5 %, and what the costs choose is on average 0.2 % slower than the fastest).  They are chosen against the others' best, whole or in two ranges.
+static const TileRate TILES_QUARTERS[] = {
+    {10, 256, 256, 5.76f, 0.91f, 0.60f, 0.f, 0.f, 0.f}, {12, 256, 256, 8.00f, 0.91f, 0.55f, 0.f, 0.f, 0.f}};
 static const double LAUNCH_US = 2.0;
 
 static double tile_us(const TileRate& t, long workgroups, int k_tiles) {
@@ -1582,7 +1771,7 @@ struct TileChoice {
 static TileChoice choose_tile(bool swiglu, int M, int rows, int k_tiles, int copies, bool two_ranges) {
   const TileRate* tiles = swiglu ? TILES_SWIGLU : TILES_PLAIN;
   const int n = swiglu ? (int)(sizeof(TILES_SWIGLU) / sizeof(TileRate)) : (int)(sizeof(TILES_PLAIN) / sizeof(TileRate));
-  auto allowed = [&](const TileRate& t) { return !((t.id == 10 && !g_tiles_256) || (t.bn == 160 && !g_tiles_160)); };
+  auto allowed = [&](const TileRate& t) { return t.bn != 160 || g_tiles_160; };
   auto row_tiles = [&](const TileRate& t) { return (long)((M + t.bm - 1) / t.bm); };
   auto us = [&](const TileRate& t, int r) { return LAUNCH_US + tile_us(t, row_tiles(t) * ((r + t.bn - 1) / t.bn) * copies, k_tiles); };
   TileChoice best;
@@ -1608,6 +1797,17 @@ static TileChoice choose_tile(bool swiglu, int M, int rows, int k_tiles, int cop
   return best;
 }
 
+// ... by quarters: the cheaper of the two (id 0: neither)
+static TileChoice choose_quarters(int M, int rows, int k_tiles) {
+  TileChoice best;
+  if (!g_tiles_256) return best;
+  for (const TileRate& t : TILES_QUARTERS) {
+    const double us = LAUNCH_US + tile_us(t, (long)((M + 255) / 256) * ((rows + 255) / 256), k_tiles);
+    if (!best.id || us < best.us) best = {t.id, us, 0, 0};
+  }
+  return best;
+}
+
 // The tile of the q/k/v product that finishes its heads: of 64, 128 or 256 rows the one whose launch costs the least,
 // 256-row tiles also as whole rounds of the units with the heads left over in 128-row tiles behind them (Qwen3-8B's 48 heads
 // over 2,048 rows), beside the plain product in its own best tile followed by the kernel that prepares whole steps, which
@@ -1615,7 +1815,7 @@ static TileChoice choose_tile(bool swiglu, int M, int rows, int k_tiles, int cop
 // tiles of 128 x 128: 18.9 us; of 64 x 128, on all units: 12).  Steps of up to 64 rows whose tiles leave most units idle
 // always go to the product.
 struct QKVChoice {
-  int rows = 0;             // of a tile; 0: left to the product and the preparation kernel
+  int rows = 0;             // of a tile; 512: tiles of 256 x 256; 0: left to the product and the preparation kernel
   int n_big = 0;            // > 0: that many columns in 256-row tiles, the others in 128-row tiles
 };
 static QKVChoice qkv_choice(int M, int N, int K) {
@@ -1644,6 +1844,16 @@ static QKVChoice qkv_choice(int M, int N, int K) {
       c = {256, cols * 128};
     }
   }
+  // Tiles of 256 x 256 read A and W the least; they finish twice the heads, 7 us (us, the best of the others and they: 2,048 rows of 6144 x 4096
+  // 103 and 97, of 6144 x 2560 75 and 67, 1,500 of 6144 x 4096 97 and 86).  Under a shorter K the heads weigh more and less is left to gain
+  // (6144 x 2048 64 and 60, 5120 x 2048 60 and 58; 3,000 rows of 6144 x 2048 95 and 115).
+  if (g_tiles_256 && k_tiles >= 40) {
+    const double wide = LAUNCH_US + 7.0 + tile_us(TILES_QUARTERS[0], row_tiles * ((N + 255) / 256), k_tiles);
+    if (wide < least) {
+      least = wide;
+      c = {512, 0};
+    }
+  }
   const double apart = choose_tile(false, M, N, k_tiles, 1, true).us + LAUNCH_US + 2.0 + 2.0 * M * N * 4 / 4.0e6;
   if (M <= 64 ? (long)((M + 127) / 128) * col_tiles * 2 < units : apart < least) c = {0, 0};
   return c;
@@ -1656,6 +1866,11 @@ extern "C" int ti_gemm_bf16_tile_choice(int swiglu, int M, int N, int K, int* re
   *rest = c.rest;
   *n_big = swiglu ? c.n_big / 2 : c.n_big;
   return c.id;
+}
+// ... what SwiGLU takes in its place: 10 or 12, or 0: that choice.
+extern "C" int ti_gemm_bf16_quarters_choice(int M, int N, int K) {
+  const TileChoice q = choose_quarters(M, 2 * N, K / PBK);
+  return q.id && q.us < choose_tile(true, M, 2 * N, K / PBK, 1, true).us ? q.id : 0;
 }
 extern "C" int ti_gemm_bf16_qkv_choice(int M, int N, int K, int* n_big) {
   const QKVChoice c = qkv_choice(M, N, K);
@@ -1695,6 +1910,8 @@ extern "C" int ti_gemm_bf16_qkv_prep(const void* A, const void* W, int M, int K,
   if (c.n_big) {
     rc_ = launch_qkv_prep<256, 4, 2, 3>(A, W, M, N, K, lda, ep, stream, 0, c.n_big);
     if (!rc_) rc_ = launch_qkv_prep<128, 4, 2, 4>(A, W, M, N, K, lda, ep, stream, c.n_big, N);
+  } else if (c.rows == 512) {      // (256 x 256)
+    rc_ = launch_qkv_prep<256, 2, 4, 2, 256, true>(A, W, M, N, K, lda, ep, stream);
   } else if (c.rows == 64) {
     rc_ = launch_qkv_prep<64, 2, 4, 4>(A, W, M, N, K, lda, ep, stream);
   } else if (c.rows == 128) {
@@ -1719,7 +1936,8 @@ static int launch_tile(int id, const bf16_t* A, const bf16_t* W, void* out, int 
     switch (id) {
       case 5: return launch_pipelined<64, 128, 2, 2, EPI>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
       case 7: return launch_pipelined<64, 128, 2, 2, EPI, 4>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
-      case 10: return launch_pipelined<256, 256, 4, 2, EPI, 2>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+      case 10: return launch_pipelined<256, 256, 2, 4, EPI, 2, true>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
+      case 12: return launch_pipelined<256, 256, 2, 2, EPI, 2, true>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);     // for a long K
     }
     // (a forced tile that it does not have)
     return launch_pipelined<128, 128, 4, 2, EPI, 4>(A, W, out, M, N, K, lda, s, ksplit, n_first, n_end);
@@ -1741,6 +1959,10 @@ static int launch_tiled_best(const bf16_t* A, const bf16_t* W, void* out, int M,
   constexpr bool SW = EPI == TI_EPI_SWIGLU;
   if (g_force_tile) return launch_tile<EPI>(g_force_tile, A, W, out, M, N, K, lda, s);
   const TileChoice c = choose_tile(SW, M, SW ? 2 * N : N, K / PBK, 1, true);
+  if constexpr (SW) {
+    const TileChoice q = choose_quarters(M, 2 * N, K / PBK);
+    if (q.id && q.us < c.us) return launch_tile<EPI>(q.id, A, W, out, M, N, K, lda, s);
+  }
   if (!c.n_big) return launch_tile<EPI>(c.id, A, W, out, M, N, K, lda, s);
   const int n_big = SW ? c.n_big / 2 : c.n_big;
   if (int rc = launch_tile<EPI>(c.id, A, W, out, M, N, K, lda, s, 1, 0, n_big)) return rc;

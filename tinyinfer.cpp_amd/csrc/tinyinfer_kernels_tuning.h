@@ -6,7 +6,7 @@
 //
 // libti_gemm_bf16:
 //   force_tile           1: 256 x 128, 2: 128 x 128; not for SwiGLU 3 / 4: 128 x 64, 6: 64 x 64, 8: 128 x 160, 9: 256 x 160,
-//                        11: 256 x 128 by four wavefronts; for SwiGLU alone 5 / 7: 64 x 128, 10: 256 x 256 (another's number:
+//                        11: 256 x 128 by four wavefronts; for SwiGLU alone 5 / 7: 64 x 128, 10 / 12: 256 x 256 (another's number:
 //                        128 x 128 for SwiGLU, 128 x 64 for the others); 0: by the shape
 //   normed_weight_below  weights of fewer elements keep the norm inside the product (0: the default)
 //   normed_groups        1 to 3 groups of four wavefronts, a tile each, in the product with the norm inside (0: by the tiles)
@@ -18,7 +18,7 @@
 //   die_order            0: the dies take the tiles of a small weight in the grid's order
 //   skinny_waves         4 or 8 wavefronts in the kernel for M <= 64 (0: by the shape)
 //   qkv_prep_min_rows    the fewest rows ti_gemm_bf16_qkv_prep serves (17)
-//   qkv_prep_rows        64 / 128 / 256: the rows of ti_gemm_bf16_qkv_prep's tile; 0: by the shape
+//   qkv_prep_rows        64 / 128 / 256: the rows of ti_gemm_bf16_qkv_prep's tile, 512: tiles of 256 x 256; 0: by the shape
 //   wide_rows            0: 17..64 rows times a weight of 16,384 rows or more take the other kernels
 //   tiled_from           17..64 rows x weight elements from which they take the tiled kernels (280 Mi; 1000 Mi for a product that
 //                        stores, K below 4096 and few enough workgroups of 16 rows: set, it holds for both, and rows_112 is off)
@@ -46,9 +46,11 @@ int ti_tuning_set(const char* name, long value);     // 0, or 1 for a name the l
 void ti_tuning_reset();                              // every choice back to the library's own
 // libti_gemm_bf16: what is chosen for M rows times N output columns.  The tile (by its number above) and, where the columns are
 // split between two (n_big > 0), the second one from column n_big on; the rows of the q/k/v product's tile (0: left to the
-// product and the preparation kernel), 256 and 128 where n_big > 0.
+// product and the preparation kernel; 512: tiles of 256 x 256), 256 and 128 where n_big > 0.
 int ti_gemm_bf16_tile_choice(int swiglu, int M, int N, int K, int* rest, int* n_big);
 int ti_gemm_bf16_qkv_choice(int M, int N, int K, int* n_big);
+// ... SwiGLU, in place of the first: a tile of 256 x 256 (10, 12), or 0
+int ti_gemm_bf16_quarters_choice(int M, int N, int K);
 #ifdef __cplusplus
 }
 #endif
