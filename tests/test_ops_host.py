@@ -92,6 +92,35 @@ def test_what_the_rows_of_a_draw_ask_for_packs_from_any_iterable():
     assert bytes(Sampler._arguments(2, params, iter([11 + (1 << 64), 5]), [0, 2])[4]) == want[4]
 
 
+def test_records_of_a_draw_say_what_the_lists_say():
+    """A record's fields are the lists' elements; parameters and numbers that a record cannot hold go by the lists (None)."""
+    import copy
+    import dataclasses
+    import pickle
+    import struct
+
+    import numpy as np
+    from tinyinfer_amd.sampling import Sampler, SamplingParams
+
+    class Lists:                                      # parameters of a caller's own
+        temperature, top_k, top_p, seed = 0.5, 7, 0.9, 1
+    params = [SamplingParams(0.5, 7, 0.9, -3), SamplingParams(1, 0, 1, 1 << 63), dataclasses.replace(SamplingParams(0.5, 7), top_k=9),
+              pickle.loads(pickle.dumps(SamplingParams(0.25, 3, 0.5, 4))), copy.copy(SamplingParams(1e39))]
+    n = len(params)
+    records, requests, counters = Sampler._records(n, params, (1, 2, 3, 4, 5), (0,) * n)
+    lists = Sampler._arguments(n, params, (1, 2, 3, 4, 5), (0,) * n)
+    fields = list(struct.iter_unpack("@fif4xQ", records))
+    assert len(records) == 24 * n
+    for i, kind in enumerate("fifQ"):
+        assert struct.pack(f"{n}{kind}", *[f[i] for f in fields]) == lists[i]
+    assert (requests, counters) == lists[4:]
+    for odd in (Lists(), SamplingParams(0.5, 1 << 40), SamplingParams(0.5, 2.0), SamplingParams(np.float32(0.5))):
+        assert Sampler._records(2, [odd, params[0]], (1, 2), (0, 0)) is None
+    assert Sampler._records(2, params[:2], (1 << 64, 2), (0, 0)) is None
+    assert Sampler._records(2, params[:2], (1,), (0, 0)) is None
+    assert SamplingParams(0.5, 7) == SamplingParams(0.5, 7) and repr(SamplingParams()).count("record") == 0
+
+
 @pytest.mark.parametrize("heads,rows,context,tokens,behind,one", [
     # whole portions: enough units left, or short rows; then long rows beside portions on most units or all, which took up to 12 % longer in one launch
     (16, 2, 2000, 512, 0, True), (16, 2, 2000, 768, 0, True), (16, 2, 12000, 768, 4000, True), (16, 4, 500, 1024, 8000, True),

@@ -908,19 +908,51 @@ int ti_sampler_sample(void* sampler, const ti_tensor* logits, int n, const float
   memcpy(out, ids.data(), (size_t)n * 4);
   TI_END
 }
+// where a call's ids go beside the host: an engine's token feedback, or nowhere
+static int* feedback_of(void* feed_engine, int n) {
+  if (!feed_engine) return nullptr;
+  Engine& e = *static_cast<Engine*>(feed_engine);
+  if (!e.token_feedback()) throw EngineError("this engine has no token feedback (its model has parts from outside the library)");
+  if (n > e.feedback_rows())
+    throw EngineError(std::to_string(n) + " rows of logits but the token feedback holds " + std::to_string(e.feedback_rows()));
+  return e.token_feedback();
+}
 int ti_sampler_sample_async(void* sampler, const ti_tensor* logits, int n, const float* temperature, const int* top_k,
                             const float* top_p, const uint64_t* seeds, const int64_t* requests, const int64_t* counters,
                             void* feed_engine, uint64_t* out_ticket) {
   TI_BEGIN
-  int* feed = nullptr;
-  if (feed_engine) {
-    Engine& e = *static_cast<Engine*>(feed_engine);
-    if (!e.token_feedback()) throw EngineError("this engine has no token feedback (its model has parts from outside the library)");
-    if (n > e.feedback_rows())
-      throw EngineError(std::to_string(n) + " rows of logits but the token feedback holds " + std::to_string(e.feedback_rows()));
-    feed = e.token_feedback();
-  }
+  int* feed = feedback_of(feed_engine, n);
   *out_ticket = static_cast<Sampler*>(sampler)->sample_async(T(logits, 0), sampling_params(n, temperature, top_k, top_p, seeds),
+                                                             std::vector<int64_t>(requests, requests + n),
+                                                             std::vector<int64_t>(counters, counters + n), feed);
+  TI_END
+}
+static std::vector<SamplingParams> recorded_params(int n, const ti_sampling_record* records) {
+  std::vector<SamplingParams> params(n);
+  for (int i = 0; i < n; ++i) {
+    ti_sampling_record r;
+    memcpy(&r, (const char*)records + i * sizeof r, sizeof r);      // (bytes of the caller's, on any boundary)
+    params[i].temperature = r.temperature;
+    params[i].top_k = r.top_k;
+    params[i].top_p = r.top_p;
+    params[i].seed = r.seed;
+  }
+  return params;
+}
+int ti_sampler_sample_records(void* sampler, const ti_tensor* logits, int n, const ti_sampling_record* records, const int64_t* requests,
+                              const int64_t* counters, int* out) {
+  TI_BEGIN
+  const std::vector<int> ids = static_cast<Sampler*>(sampler)->sample(T(logits, 0), recorded_params(n, records),
+                                                                      std::vector<int64_t>(requests, requests + n),
+                                                                      std::vector<int64_t>(counters, counters + n));
+  memcpy(out, ids.data(), (size_t)n * 4);
+  TI_END
+}
+int ti_sampler_sample_records_async(void* sampler, const ti_tensor* logits, int n, const ti_sampling_record* records,
+                                    const int64_t* requests, const int64_t* counters, void* feed_engine, uint64_t* out_ticket) {
+  TI_BEGIN
+  int* feed = feedback_of(feed_engine, n);
+  *out_ticket = static_cast<Sampler*>(sampler)->sample_async(T(logits, 0), recorded_params(n, records),
                                                              std::vector<int64_t>(requests, requests + n),
                                                              std::vector<int64_t>(counters, counters + n), feed);
   TI_END

@@ -1354,6 +1354,17 @@ int ti_sampler_sample(void* sampler, const ti_tensor* logits, int n, const float
 int ti_sampler_sample_async(void* sampler, const ti_tensor* logits, int n, const float* temperature, const int* top_k,
                             const float* top_p, const uint64_t* seeds, const int64_t* requests, const int64_t* counters,
                             void* feed_engine, uint64_t* out_ticket);
+// the same with what each row asks for in one record (a caller that keeps a request's record packs nothing at a call)
+typedef struct {
+  float temperature;
+  int32_t top_k;
+  float top_p;
+  uint64_t seed;      // on a boundary of 8: 24 bytes in all
+} ti_sampling_record;
+int ti_sampler_sample_records(void* sampler, const ti_tensor* logits, int n, const ti_sampling_record* records, const int64_t* requests,
+                              const int64_t* counters, int* out);
+int ti_sampler_sample_records_async(void* sampler, const ti_tensor* logits, int n, const ti_sampling_record* records,
+                                    const int64_t* requests, const int64_t* counters, void* feed_engine, uint64_t* out_ticket);
 int ti_sampler_collect(void* sampler, uint64_t ticket, int n, int* out);
 int ti_scheduler_create(void* cache, int max_batched_tokens, int chunk_size, int max_running, void** out);
 void ti_scheduler_release(void* scheduler);

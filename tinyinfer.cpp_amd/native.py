@@ -149,6 +149,8 @@ _SIGNATURES = {
     "ti_sampler_create": [c_void_p, _OUT_PTR],
     # (the rows' arrays as ctypes arrays or as packed bytes)
     "ti_sampler_sample": [c_void_p, _TT, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, P(c_int)],
+    "ti_sampler_sample_records": [c_void_p, _TT, c_int, c_void_p, c_void_p, c_void_p, P(c_int)],
+    "ti_sampler_sample_records_async": [c_void_p, _TT, c_int, c_void_p, c_void_p, c_void_p, c_void_p, P(c_u64)],
     "ti_sampler_sample_async": [c_void_p, _TT, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, P(c_u64)],
     "ti_sampler_collect": [c_void_p, c_u64, c_int, P(c_int)],
     "ti_scheduler_create": [c_void_p, c_int, c_int, c_int, _OUT_PTR],
