@@ -217,6 +217,40 @@ def test_qk_norm_rope_kv_write(ops, dtype, hd, nh, nkv, P, table_len):
     assert keys[mask].abs().max() == 0 and vals[mask].abs().max() == 0
 
 
+# rows around a block of sixteen values, and around one, two and three heads a wavefront (3,072 and 9,600 query and key heads)
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("M,nh,nkv,P,normed", [(1, 16, 8, 16, True), (15, 16, 8, 16, True), (17, 5, 2, 4, False), (128, 16, 8, 16, True),
+                                               (129, 16, 8, 16, True), (400, 16, 8, 8, True), (401, 16, 8, 16, True), (33, 3, 1, 16, True),
+                                               (40, 4, 0, 16, True), (1923, 3, 2, 16, True)])
+def test_heads_of_128_are_finished_as_the_general_kernel_does(ops, dtype, M, nh, nkv, P, normed):
+    """The same bits from the kernel for heads of 128 and from the general one, which takes projections off a boundary of 16 bytes: three
+    requests whose rows begin inside a page, positions within and beyond the table, a page that is not reserved."""
+    g = torch.Generator().manual_seed(M)
+    hd, width = 128, (nh + 2 * nkv) * 128
+    qkv = torch.randn(M, width, generator=g)
+    qw, kw = (dev(1 + 0.1 * torch.randn(hd, generator=g)) if normed else None for _ in range(2))
+    cuts = [0, M // 3, M // 2, M]
+    slot = torch.cat([torch.full((cuts[i + 1] - cuts[i],), i, dtype=torch.int32) for i in range(3)])
+    pos = torch.cat([torch.arange(cuts[i + 1] - cuts[i], dtype=torch.int32) + 3 * i + 1 for i in range(3)])
+    W = int(pos.max()) // P + 1
+    table = torch.randperm(3 * W, generator=g).to(torch.int32).view(3, W)
+    if M > 1:
+        table[2, 0] = -1                                      # nothing is written there
+    freqs = dev(inv_freq(hd, 1e6))
+    rope_table = ops.rope_table(freqs, max(1, W * P // 2))
+    results = []
+    for off in (0, 1):
+        buffer = torch.empty(M * width + 4, device="cuda")
+        there = buffer[off:off + M * width].view(M, width)
+        there.copy_(qkv)
+        pool = torch.zeros(3 * W, 2, max(nkv, 1), P, hd, dtype=DT[dtype], device="cuda")
+        q_out = torch.zeros(M, nh * hd, dtype=DT[dtype], device="cuda")
+        ops.qk_norm_rope_kv_write(there, qw, kw, 1e-6, freqs, dev(pos), dev(slot), View(dev(table)), pool, q_out, nh, nkv, hd, rope_table)
+        results.append((q_out, pool))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    assert results[0][0].abs().max() > 0 and (nkv == 0) == (results[0][1].abs().max().item() == 0)
+
+
 # -------------------------------------------------------------- matrix products
 def test_qk_norm_in_place(ops):
     """The per-head norm alone, in place on 32-bit projections: the same numbers as the fused

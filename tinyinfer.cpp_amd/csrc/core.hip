@@ -527,36 +527,6 @@ qk_norm_rope_kv_write_kernel(
   const bool is_q = u < n_head;
   const bool is_v = u >= n_head + n_kv;
   const float* src = row + (size_t)u * hd;
-  if (hd == 2 * TI_WAVE) {
-    // a pair a lane: everything is asked for before anything is waited for (the same arithmetic and bits as below).  What bounds it is a
-    // wavefront's chain of loads, and the values' scattered stores: 24 heads of 77, 300 and 1,000 rows, in turn with the loops below, us: 3.6 -> 3.1,
-    // 7.5 -> 6.1, 16.0 -> 14.5, in float32 3.9 -> 3.4, 8.9 -> 7.5, 21.3 -> 18.3.
-    const float* w = is_v ? nullptr : is_q ? q_w : k_w;
-    float lo = src[lane], hi = src[lane + TI_WAVE], wl = 1.f, wh = 1.f;
-    if (w) {
-      wl = w[lane];
-      wh = w[lane + TI_WAVE];
-    }
-    const bool rotate = inv_freq && !is_v;
-    float2 cs = make_float2(1.f, 0.f);
-    if (rotate) cs = qk_cos_sin(lane, TI_WAVE, p, inv_freq, rope_table, table_len);
-    const int page = is_q ? 0 : table[(size_t)slot[m] * table_stride + p / P];
-    if (w) {
-      const float scale = qk_norm_scale(group_sum<TI_WAVE>(qk_pair_square(lo, hi)), hd, eps);
-      lo *= scale;
-      hi *= scale;
-      lo *= wl;
-      hi *= wh;
-    }
-    if (rotate) qk_rotate(lo, hi, cs);
-    if (page < 0) return;   // the host reserves pages first; never write astray
-    T* dst = q_out + (size_t)m * nq + (size_t)u * hd;
-    if (!is_q) dst = kv_page_slot<T>(pool, page, is_v ? 1 : 0, is_v ? u - n_head - n_kv : u - n_head, p % P, n_kv, P, hd);
-    const size_t step = is_v ? P : 1;
-    st<T>(dst + (size_t)lane * step, lo);
-    st<T>(dst + (size_t)(lane + TI_WAVE) * step, hi);
-    return;
-  }
   if (is_q) {
     qk_head_wave<T>(src, q_out + (size_t)m * nq + (size_t)u * hd, 1, q_w, eps, inv_freq, rope_table, table_len, p,
                     hd);
@@ -572,6 +542,90 @@ qk_norm_rope_kv_write_kernel(
     qk_head_wave<T>(src, dst, 1, k_w, eps, inv_freq, rope_table, table_len, p, hd);
 }
 
+// The same for heads of 128, a pair a lane; the same arithmetic and bits.  What bounds it is how many loads wait for one another, and stores.
+// A wavefront takes HEADS neighbouring query and key heads of a row, whose position, angles and page are looked up once and whose loads are
+// all under way together.  Values go sixteen rows at a time, a workgroup a head: where the rows are neighbours of a page a dim's sixteen
+// elements are consecutive bytes, which a head a wavefront stored 64 bytes apart (one store of a wavefront: 64 lines).
+// Grid: workgroups of query and key heads, then those of values.
+// One head a wavefront while the units hold all wavefronts with room to spare, then two and three, so that fewer come and go.  us, 24 heads, a head of any
+// kind a wavefront, then 1, 2 and 3: float32 77 rows 3.2, 2.5 2.7 2.9, 112 3.7, 2.7 2.9 3.0, 170 4.6, 3.2 3.1 3.4, 300 6.9, 4.5 4.0 4.1, 450
+// 9.0, 6.0 5.0 4.9, 2,000 26.3, 16.2 12.8 12.5; bfloat16 77 2.8, 2.5 2.7 2.8, 300 5.2, 4.2 3.8 3.8, 2,000 20.2, 15.4 11.9 11.1.
+#define QK_ONE_EACH 3072
+#define QK_TWO_EACH 9600
+template <typename T, int HEADS>
+__global__ void __launch_bounds__(256)
+qk_norm_rope_kv_write_128_kernel(
+    const float* __restrict__ qkv, const float* __restrict__ q_w, const float* __restrict__ k_w,
+    const float* __restrict__ inv_freq, const float2* __restrict__ rope_table, int table_len,
+    const int* __restrict__ pos, const int* __restrict__ slot,
+    const int* __restrict__ table, int table_stride, T* __restrict__ pool, T* __restrict__ q_out,
+    int M, int n_head, int n_kv, int P, float eps) {
+  constexpr int HD = 2 * TI_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / TI_WAVE), lane = threadIdx.x % TI_WAVE;
+  const int qk = n_head + n_kv, per_row = (qk + 4 * HEADS - 1) / (4 * HEADS), width = (qk + n_kv) * HD;
+  const int id = blockIdx.x;
+  if (id < M * per_row) {
+    const int m = id / per_row, u0 = ((id - m * per_row) * 4 + wave) * HEADS, heads = min(HEADS, qk - u0);
+    if (heads <= 0) return;
+    const float* src = qkv + (size_t)m * width + (size_t)u0 * HD;
+    float lo[HEADS], hi[HEADS];
+#pragma unroll
+    for (int j = 0; j < HEADS; ++j) {
+      const int at = min(j, heads - 1) * HD + lane;
+      lo[j] = src[at];
+      hi[j] = src[at + TI_WAVE];
+    }
+    const int p = pos[m];
+    float qwl = 1.f, qwh = 1.f, kwl = 1.f, kwh = 1.f;
+    if (q_w) {
+      qwl = q_w[lane];
+      qwh = q_w[lane + TI_WAVE];
+    }
+    if (k_w) {
+      kwl = k_w[lane];
+      kwh = k_w[lane + TI_WAVE];
+    }
+    float2 cs = make_float2(1.f, 0.f);
+    if (inv_freq) cs = qk_cos_sin(lane, TI_WAVE, p, inv_freq, rope_table, table_len);
+    const int page = u0 + heads > n_head ? table[(size_t)slot[m] * table_stride + p / P] : 0;
+#pragma unroll
+    for (int j = 0; j < HEADS; ++j) {
+      if (j >= heads) break;
+      const int u = u0 + j;
+      const bool is_q = u < n_head;
+      if (is_q ? q_w != nullptr : k_w != nullptr) {
+        const float scale = qk_norm_scale(group_sum<TI_WAVE>(qk_pair_square(lo[j], hi[j])), HD, eps);
+        lo[j] *= scale;
+        hi[j] *= scale;
+        lo[j] *= is_q ? qwl : kwl;
+        hi[j] *= is_q ? qwh : kwh;
+      }
+      if (inv_freq) qk_rotate(lo[j], hi[j], cs);
+      if (page < 0 && !is_q) continue;      // the host reserves pages first; never write astray
+      T* dst = is_q ? q_out + (size_t)m * n_head * HD + (size_t)u * HD : kv_page_slot<T>(pool, page, 0, u - n_head, p % P, n_kv, P, HD);
+      st<T>(dst + lane, lo[j]);
+      st<T>(dst + lane + TI_WAVE, hi[j]);
+    }
+    return;
+  }
+  // values: row lane % 16 of the block, dims 32 wave + 16 i + 4 (lane / 16) ..+3
+  const int v = id - M * per_row, kvh = v % n_kv, m = v / n_kv * 16 + (lane & 15);
+  if (m >= M) return;
+  const int d0 = 32 * wave + 4 * (lane >> 4);
+  const float* src = qkv + (size_t)m * width + (size_t)(qk + kvh) * HD + d0;
+  const float4 x[2] = {*reinterpret_cast<const float4*>(src), *reinterpret_cast<const float4*>(src + 16)};
+  const int p = pos[m], page = table[(size_t)slot[m] * table_stride + p / P];
+  if (page < 0) return;
+  T* dst = kv_page_slot<T>(pool, page, 1, kvh, p % P, n_kv, P, HD) + (size_t)d0 * P;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    st<T>(dst + (size_t)(16 * i) * P, x[i].x);
+    st<T>(dst + (size_t)(16 * i + 1) * P, x[i].y);
+    st<T>(dst + (size_t)(16 * i + 2) * P, x[i].z);
+    st<T>(dst + (size_t)(16 * i + 3) * P, x[i].w);
+  }
+}
+
 extern "C" int ti_qk_norm_rope_kv_write(int dtype, const float* qkv, const float* q_w, const float* k_w,
                                         const float* inv_freq, const float* rope_table, int table_len,
                                         const int* pos, const int* slot,
@@ -585,17 +639,35 @@ extern "C" int ti_qk_norm_rope_kv_write(int dtype, const float* qkv, const float
   if (M == 0) return 0;
   const int units = n_head + 2 * n_kv;
   TI_REQUIRE((units + 3) / 4 <= 65535, "qk_norm_rope_kv_write: too many heads");
+  TI_REQUIRE(dtype == TI_F32 || dtype == TI_BF16, "qk_norm_rope_kv_write: unknown dtype %d", dtype);
+  // heads of 128, values as 16-byte pieces
+  if (hd == 2 * TI_WAVE && ((uintptr_t)qkv & 15) == 0) {
+    const long heads = (long)M * (n_head + n_kv);
+    const auto go = [&](auto kernel, auto* to_pool, auto* to_q, int each) {
+      const long groups = (long)M * ((n_head + n_kv + 4 * each - 1) / (4 * each)) + (long)((M + 15) / 16) * n_kv;
+      if (groups > 0x7fffffff) return false;
+      kernel<<<(unsigned)groups, 256, 0, stream>>>(qkv, q_w, k_w, inv_freq, (const float2*)rope_table, table_len, pos, slot, table,
+                                                   table_stride, to_pool, to_q, M, n_head, n_kv, page_size, eps);
+      return true;
+    };
+#define TI_GO(T, EACH) go(qk_norm_rope_kv_write_128_kernel<T, EACH>, (T*)pool, (T*)q_out, EACH)
+#define TI_ROWS(T) (heads <= QK_ONE_EACH ? TI_GO(T, 1) : heads <= QK_TWO_EACH ? TI_GO(T, 2) : TI_GO(T, 3))
+    if (dtype == TI_F32 ? TI_ROWS(float) : TI_ROWS(bf16_t)) {
+      TI_LAUNCH_CHECK();
+      return 0;
+    }
+#undef TI_ROWS
+#undef TI_GO
+  }
   dim3 grid(M, (units + 3) / 4);
   if (dtype == TI_F32)
     qk_norm_rope_kv_write_kernel<float><<<grid, 256, 0, stream>>>(
         qkv, q_w, k_w, inv_freq, (const float2*)rope_table, table_len, pos, slot, table, table_stride,
         (float*)pool, (float*)q_out, n_head, n_kv, hd, page_size, eps);
-  else if (dtype == TI_BF16)
+  else
     qk_norm_rope_kv_write_kernel<bf16_t><<<grid, 256, 0, stream>>>(
         qkv, q_w, k_w, inv_freq, (const float2*)rope_table, table_len, pos, slot, table, table_stride,
         (bf16_t*)pool, (bf16_t*)q_out, n_head, n_kv, hd, page_size, eps);
-  else
-    TI_REQUIRE(false, "qk_norm_rope_kv_write: unknown dtype %d", dtype);
   TI_LAUNCH_CHECK();
   return 0;
 }
