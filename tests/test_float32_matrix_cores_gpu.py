@@ -1,5 +1,6 @@
 """The float32 product and attention on the matrix cores, against float64 and against themselves under other cuts of
 the same rows: a row's bits do not depend on the rows beside it."""
+import ctypes
 import math
 
 import pytest
@@ -43,6 +44,38 @@ def test_product_at_the_edges_of_its_tiles(ops, N, K):  # noqa: F811
             gate, up = f64(full[:M, :N // 2]), f64(full[:M, N // 2:])
             want = gate / (1 + torch.exp(-gate)) * up
             assert ((f64(out) - want).abs() <= 16 * EPS * want.abs() + 1e-30).all(), M
+
+
+# a last tile of few rows and of few columns, columns that are no whole float4, runs of K of 1 to 5 steps, an odd number of steps, rows further apart than K
+@pytest.mark.parametrize("swiglu,M,N,K,lda", [(0, 321, 8194, 1056, 1056), (0, 130, 40003, 320, 320), (0, 4000, 8194, 64, 64), (0, 64, 151936, 1024, 1056),
+                                              (1, 300, 3072, 1024, 1024), (1, 250, 3039, 1056, 1060)])
+def test_product_whose_wavefronts_split_together(ops, swiglu, M, N, K, lda):  # noqa: F811
+    """The bits of sixteen rows at a time, which go to the kernel whose wavefronts split for themselves, with every epilogue; infinite, NaN
+    and the largest floats among the operands.  Within the bound of a 32-bit sum of float64."""
+    choice = ops.lib("gemm_generic").ti_gemm_generic_f32_choice
+    choice.argtypes = [ctypes.c_int] * 4 + [ctypes.c_long]
+    assert choice(swiglu, M, N, K, lda) == 1 and choice(swiglu, 16, N, K, lda) == 0
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    rows = torch.randn(M, lda, device="cuda", generator=g)
+    w = torch.randn(N * (1 + swiglu), K, device="cuda", generator=g) * 0.05
+    rows[M - 1, K - 1], rows[M // 2, 3], rows[1, K // 2] = float("inf"), float("nan"), 3.39e38
+    w[N - 1, 5] = float("-inf")
+    a = rows[:, :K]
+    bits = lambda t: t.view(torch.int32)                      # noqa: E731
+    for epilogue in ("swiglu",) if swiglu else ("store", "add", "relu2"):
+        full, parts = torch.full((M + 1, N), 0.5, device="cuda"), torch.full((M, N), 0.5, device="cuda")
+        ops.linear(a, w, full[:M], epilogue)
+        assert bool((full[M] == 0.5).all())
+        for m in range(0, M, 16):
+            ops.linear(a[m:m + 16], w, parts[m:m + 16], epilogue)
+        same = (bits(full[:M]) == bits(parts)) | (torch.isnan(full[:M]) & torch.isnan(parts))
+        assert bool(same.all()), epilogue
+        if epilogue == "store":
+            m = min(M, 400)
+            ref, size = a[:m].double() @ w.double().t().contiguous(), a[:m].double().abs() @ w.double().abs().t().contiguous()
+            fine = torch.isfinite(ref) & (ref.abs() < 1e38)
+            assert bool(((full[:m].double() - ref).abs() <= (K + 1) * EPS * size)[fine].all())
+            assert torch.equal(torch.isnan(full[:m]), torch.isnan(ref))
 
 
 @pytest.mark.parametrize("M,N,K", [(7, 64, 20), (37, 132, 1056), (300, 96, 260)])

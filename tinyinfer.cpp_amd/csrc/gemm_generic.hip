@@ -188,6 +188,36 @@ __device__ __forceinline__ float dot_by_fma(const float* __restrict__ a, const f
   return total;
 }
 
+// Four neighbouring results of one token, from the sums of all runs to `o`: what is not finite is computed again, SwiGLU, the store.
+template <bool SW>
+__device__ __forceinline__ void f32_finish(gf4 v, gf4 u, const float* __restrict__ a, const float* __restrict__ W, float* __restrict__ o,
+                                           int n, int N, int K, int run, int epi, int wide_out) {
+  const auto settle = [&](gf4& x, size_t row0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (fabsf(x[i]) <= FLT_MAX) x[i] *= 1.f / (GF_SCALE * GF_SCALE);
+      else if (n + i < N) x[i] = dot_by_fma(a, W + (row0 + n + i) * K, K, run);
+  };
+  settle(v, 0);
+  if (SW) {
+    settle(u, N);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = v[i] / (1.0f + expf(-v[i])) * u[i];
+  }
+  if (epi == TI_EPI_RELU2) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = epi_act<TI_EPI_RELU2>(v[i]);
+  }
+  if (wide_out) {
+    if (epi == TI_EPI_ADD_F32) v += *reinterpret_cast<const gf4*>(o);
+    *reinterpret_cast<gf4*>(o) = v;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (n + i < N) o[i] = epi == TI_EPI_ADD_F32 ? o[i] + v[i] : v[i];
+  }
+}
+
 struct Eight { gf4 x, y; };      // eight consecutive k of one row
 
 template <int RB, int NB, bool SW> struct F32Tile {
@@ -316,35 +346,205 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
       const gf4 x = *reinterpret_cast<const gf4*>(&s_tile[w][0][t][c]);
       v = w & 1 ? v - x : v + x;
     }
-    const auto settle = [&](gf4& x, size_t row0) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (fabsf(x[i]) <= FLT_MAX) x[i] *= 1.f / (GF_SCALE * GF_SCALE);
-        else if (n + i < N) x[i] = dot_by_fma(A + (size_t)m * lda, W + (row0 + n + i) * K, K, run);
-    };
-    settle(v, 0);
+    gf4 u = v;
     if (SW) {
-      gf4 u = *reinterpret_cast<const gf4*>(&s_tile[0][PL - 1][t][c]);
+      u = *reinterpret_cast<const gf4*>(&s_tile[0][PL - 1][t][c]);
       for (int w = 1; w < runs; ++w) {
         const gf4 x = *reinterpret_cast<const gf4*>(&s_tile[w][PL - 1][t][c]);
         u = w & 1 ? u - x : u + x;
       }
-      settle(u, N);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = v[i] / (1.0f + expf(-v[i])) * u[i];
     }
-    if (epi == TI_EPI_RELU2) {
+    f32_finish<SW>(v, u, A + (size_t)m * lda, W, out + (size_t)m * N + n, n, N, K, run, epi, wide_out);
+  }
+#endif
+}
+
+// ---------------------------------------------------------------------------------- float32, more tokens: shared splits
+// In gemm_f32_kernel every wavefront splits what it multiplies, 52 vector instructions a block, twice the time of its matrix instructions.
+// Here WR x WT wavefronts own a tile together, each RB blocks of weight rows (SwiGLU: of gates and of their ups) x NB of tokens: a
+// k-step's floats come into registers eight lanes to a row's 128 bytes, are split once for the workgroup and go as pieces into one of
+// two stages of LDS, in the order in which a matrix instruction takes them.  While one stage is multiplied the next is split, and the
+// loads of the two after that are out; a step has one barrier.  A wavefront alone on its SIMD issues a vector instruction every 8
+// cycles, two one every 4.7: two workgroups of four wavefronts to a unit, or eight wavefronts.
+// The runs of K are those of gemm_f32_kernel, one after the other in the same wavefront, each with sums of its own that are
+// added to (or subtracted from) the total at its end: the same bits, whichever kernel takes a product.
+// Piece (k / 8, row) of a block's plane lies in place (k / 8) * 16 + (row ^ 2 (k / 8)).  A wavefront's read of a plane takes 1.8 ns a unit so, as
+// in a row, and its write of 512 bytes 3.0; exchanged by 4 (k / 8) 3.5 and 3.4, not exchanged 1.9 and 6.8.
+// What bounds it: vector and matrix instructions of a step hardly overlap (tiles of 64 x 128, two to a unit: 1.83 us a step of both, of which
+// matrix instructions alone take 0.7 and vector instructions 0.8; in which order they stand changes nothing).
+// us a call, there and here: 300 rows x 151936 x 1024 868 -> 680, [gate; up] 6144 x 1024 37.4 -> 31.7; 64 rows x 151936 x 1024 208 -> 178;
+// 1,000 rows x 4096 x 1024 79 -> 62, x 151936 x 1024 2,490 -> 2,080.
+template <int WR, int WT, int RB, int NB, bool SW> struct F32Shared {
+  static constexpr int WAVES = WR * WT, PL = SW ? 2 : 1, ROWS = WR * RB, TOKENS = WT * NB;      // blocks of 16: weight rows of a plane, tokens
+  static constexpr int BLOCKS = PL * ROWS + TOKENS, LOADS = 2 * BLOCKS / WAVES;      // half blocks of 8 rows a wavefront asks for
+  static constexpr int STAGE = BLOCKS * 3072, LDS = 2 * STAGE;
+  static_assert(ROWS % (WAVES / 2) == 0 && TOKENS % (WAVES / 2) == 0, "a load of all wavefronts is rows of one kind");
+};
+
+// Four floats, times `factor`, as three bfloat16 each: split_planes for half an operand.
+struct HalfPlanes {
+  uint2 p[3];
+};
+__device__ __forceinline__ HalfPlanes split_half(const gf4& x, float factor) {
+  HalfPlanes s;
+  float r[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = epi_act<TI_EPI_RELU2>(v[i]);
+  for (int i = 0; i < 4; ++i) r[i] = x[i] * factor;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    s.p[j] = make_uint2(pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]));
+    if (j < 2) {
+      r[0] -= __uint_as_float(s.p[j].x << 16);
+      r[1] -= __uint_as_float(s.p[j].x & 0xffff0000u);
+      r[2] -= __uint_as_float(s.p[j].y << 16);
+      r[3] -= __uint_as_float(s.p[j].y & 0xffff0000u);
     }
-    float* o = out + (size_t)m * N + n;
-    if (wide_out) {
-      if (epi == TI_EPI_ADD_F32) v += *reinterpret_cast<const gf4*>(o);
-      *reinterpret_cast<gf4*>(o) = v;
-    } else {
+  }
+  return s;
+}
+
+template <int WR, int WT, int RB, int NB, bool SW>
+__global__ void __launch_bounds__(64 * WR * WT, 2)
+gemm_f32_shared_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ out, int M, int N, int K,
+                       long lda, int run, int m_tiles, int n_tiles, int epi, int wide_out) {
+#if defined(__HIP_DEVICE_COMPILE__)      // (the host's pass has no buffer descriptors)
+  using T = F32Shared<WR, WT, RB, NB, SW>;
+  constexpr int WAVES = T::WAVES, PL = T::PL, ROWS = T::ROWS, LOADS = T::LOADS, STAGE = T::STAGE;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int die = blockIdx.x & 7, local = blockIdx.x >> 3;      // (as in gemm_f32_kernel)
+  const int nt = m_tiles == 1 ? (int)blockIdx.x : (local / m_tiles) * 8 + die;
+  const int mt = m_tiles == 1 ? 0 : local % m_tiles;
+  if (nt >= n_tiles) return;
+  const int n0 = nt * 16 * ROWS, m0 = mt * 16 * T::TOKENS;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r16 = lane & 15, quad = lane >> 4;
+  const int wr = wave % WR, wt = wave / WR;                      // this wavefront's part of the rows, of the tokens
+
+  // what this wavefront brings: half blocks WAVES i + wave.  Rows past the end repeat the last one; their sums are not stored.
+  unsigned voff[LOADS], put[LOADS];
+  const int lr = lane >> 3, c = lane & 7;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (n + i < N) o[i] = epi == TI_EPI_ADD_F32 ? o[i] + v[i] : v[i];
+  for (int i = 0; i < LOADS; ++i) {
+    const int hb = WAVES * i + wave, block = hb >> 1, row8 = (hb & 1) * 8 + lr;
+    const bool tokens = block >= PL * ROWS;
+    const int row = (tokens ? block - PL * ROWS : block % ROWS) * 16 + row8;
+    voff[i] = (tokens ? (unsigned)min(row, M - 1 - m0) * (unsigned)(lda * 4) : (unsigned)min(row, N - 1 - n0) * (unsigned)(K * 4)) + c * 16;
+    put[i] = block * 3072 + (c >> 1) * 256 + (row8 ^ ((c >> 1) * 2)) * 16 + (c & 1) * 8;
+  }
+  const auto rows_at = [](const float* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
+  const auto rsW = rows_at(W + (size_t)n0 * K), rsU = rows_at(W + (size_t)(n0 + (SW ? N : 0)) * K), rsA = rows_at(A + (size_t)m0 * lda);
+  const auto load = [&](gf4* g, int step) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const auto& rs = WAVES / 2 * i >= PL * ROWS ? rsA : WAVES / 2 * i >= ROWS ? rsU : rsW;
+      g[i] = __builtin_bit_cast(gf4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff[i], step * GF_STEP * 4, 0));
+    }
+  };
+  const auto split = [&](const gf4* g, unsigned stage, float turned) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const HalfPlanes h = split_half(g[i], WAVES / 2 * i >= PL * ROWS ? turned : GF_SCALE);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) *reinterpret_cast<uint2*>(smem + stage + put[i] + j * 1024) = h.p[j];
+    }
+  };
+
+  gf4 acc[PL][RB][NB], fine[PL][RB][NB], total[PL][RB][NB];       // the leading products, the others, the runs before
+#pragma unroll
+  for (int p = 0; p < PL; ++p)
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[p][r][b] = fine[p][r][b] = total[p][r][b] = gf4{0.f, 0.f, 0.f, 0.f};
+  const unsigned read_at = quad * 256 + (r16 ^ (quad * 2)) * 16;
+  struct Pieces {
+    gbf8 w[PL][RB][3], t[NB][3];
+  };
+  const auto read = [&](Pieces& f, unsigned stage) {
+    const auto piece = [&](int block, int j) { return *reinterpret_cast<const gbf8*>(smem + stage + read_at + block * 3072 + j * 1024); };
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) f.t[b][j] = piece(PL * ROWS + wt * NB + b, j);
+#pragma unroll
+      for (int p = 0; p < PL; ++p)
+#pragma unroll
+        for (int r = 0; r < RB; ++r) f.w[p][r][j] = piece(p * ROWS + wr * RB + r, j);
+    }
+  };
+  const auto multiply = [&](const Pieces& f) {
+    constexpr int WJ[6] = {2, 0, 1, 1, 0, 0}, AJ[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+#pragma unroll
+      for (int p = 0; p < PL; ++p)
+#pragma unroll
+        for (int r = 0; r < RB; ++r)
+#pragma unroll
+          for (int b = 0; b < NB; ++b) {
+            gf4& sum = j < 5 ? fine[p][r][b] : acc[p][r][b];
+            sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[p][r][WJ[j]], f.t[b][AJ[j]], sum, 0, 0, 0);
+          }
+  };
+  const int steps = K / GF_STEP, run_steps = run / GF_STEP, end = steps - 1;
+  int left = run_steps, split_left = run_steps;                   // steps of the run that is multiplied, of the run that is split
+  float sign = 1.f, turned = GF_SCALE;
+  const auto split_next = [&](const gf4* g, unsigned stage) {
+    split(g, stage, turned);
+    if (--split_left == 0) split_left = run_steps, turned = -turned;
+  };
+  const auto end_of_run = [&]() {
+#pragma unroll
+    for (int p = 0; p < PL; ++p)
+#pragma unroll
+      for (int r = 0; r < RB; ++r)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) total[p][r][b][i] = fmaf(acc[p][r][b][i] + fine[p][r][b][i], sign, total[p][r][b][i]);
+          acc[p][r][b] = fine[p][r][b] = gf4{0.f, 0.f, 0.f, 0.f};
+        }
+    left = run_steps;
+    sign = -sign;
+  };
+  // One step: `g`, the step behind it, is split into the other stage and asked for anew two steps further on.  (Past the end the last step is
+  // loaded and split again, into a stage that nothing multiplies.)
+  Pieces pieces;
+  const auto step = [&](int s, gf4* g, unsigned stage) {
+    __syncthreads();
+    read(pieces, stage);
+    __builtin_amdgcn_sched_barrier(0);
+    split_next(g, STAGE - stage);
+    load(g, min(s + 3, end));
+    multiply(pieces);
+    __builtin_amdgcn_sched_barrier(0);
+    if (--left == 0 || s == end) end_of_run();
+  };
+  gf4 g0[LOADS], g1[LOADS];                                       // steps of even and of odd number
+  load(g0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  load(g1, min(1, end));
+  __builtin_amdgcn_sched_barrier(0);
+  split_next(g0, 0);
+  load(g0, min(2, end));
+  __builtin_amdgcn_sched_barrier(0);
+  int s = 0;
+  for (; s + 2 <= steps; s += 2) {
+    step(s, g1, 0);
+    step(s + 1, g0, STAGE);
+  }
+  if (s < steps) step(s, g1, 0);
+
+  // a lane holds four weight rows of one token
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const int m = m0 + (wt * NB + b) * 16 + r16;
+    if (m >= M) continue;
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      const int n = n0 + (wr * RB + r) * 16 + quad * 4;
+      if (n >= N) continue;
+      f32_finish<SW>(total[0][r][b], total[PL - 1][r][b], A + (size_t)m * lda, W, out + (size_t)m * N + n, n, N, K, run, epi, wide_out);
     }
   }
 #endif
@@ -361,6 +561,19 @@ static int compute_units() {
   return n;
 }
 
+template <int WR, int WT, int RB, int NB, bool SW>
+static int launch_f32_shared(const float* A, const float* W, float* out, int M, int N, int K, long lda, int run, int epi, int wide_out,
+                             hipStream_t stream) {
+  using T = F32Shared<WR, WT, RB, NB, SW>;
+  static const hipError_t room = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_f32_shared_kernel<WR, WT, RB, NB, SW>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
+  TI_REQUIRE(room == hipSuccess, "gemm_generic: %d bytes of LDS: %s", T::LDS, hipGetErrorString(room));
+  const int m_tiles = (M + 16 * T::TOKENS - 1) / (16 * T::TOKENS), n_tiles = (N + 16 * T::ROWS - 1) / (16 * T::ROWS);
+  const long grid = m_tiles == 1 ? n_tiles : (long)((n_tiles + 7) / 8) * 8 * m_tiles;
+  gemm_f32_shared_kernel<WR, WT, RB, NB, SW><<<(unsigned)grid, 64 * T::WAVES, T::LDS, stream>>>(A, W, out, M, N, K, lda, run, m_tiles, n_tiles, epi, wide_out);
+  return 0;
+}
+
 // The tile: of those that are built, the one whose rounds of the compute units take the least time in all.  A round costs a
 // start, its products (RB NB) and its operands (RB + NB blocks to split, four times a product's weight each).
 // Fitted to 1 to 1,000 rows times the weights of Qwen3-0.6B's sizes: the tile it picks is on average 0.9 % slower than the
@@ -372,10 +585,23 @@ static long f32_tile_cost(int rb, int nb, bool sw, int M, int N, int units) {
   return rounds * (2 + pl * rb * nb + 4 * (pl * rb + nb));
 }
 
-static int launch_f32(const float* A, const float* W, float* out, int M, int N, int K, long lda, int epi, hipStream_t stream) {
+// Whether the tiles with shared splits take it, 64 tokens x 128 weight rows (SwiGLU: 64 gates and their ups).  Their launch: 4 us, and a k-step
+// 1.83 us where a unit has two of them, 1.07 (SwiGLU 0.87) where it has one; a unit of the other's cost 0.37 us a thousand of K, 0.30 of a
+// K beyond 2,048.  A tenth in favour of the other, which stays where a round of tiles leaves units idle.  us, the other and this: 40 rows x
+// 151936 x 1024 241 196, 65 278 (278, left), 200 711 563, [gate; up] 6144 x 1024 under 200 rows 32 (left), 256 36.3 31.9, 512 56 (left), 1,000
+// 112 96, 12288 x 2048 under 300 125 115; 4096 x 1024 under 300 29 (38, left), 1,000 79 64, 2,000 159 120; 6144 x 4096 under 300 110 (114, left).
+static bool f32_shared_serves(long other_cost, bool sw, int M, int N, int K, long lda) {
+  // whole k-steps, and a tile's rows within what a buffer's descriptor spans
+  if (K % GF_STEP || K >= (1 << 20) || lda >= (1 << 20)) return false;
+  const long tiles = (long)((M + 63) / 64) * ((N + (sw ? 63 : 127)) / (sw ? 64 : 128)), units = compute_units();
+  const long rest = tiles % (2 * units);
+  const double step = 1.83 * (tiles / (2 * units)) + (rest == 0 ? 0.0 : rest > units ? 1.83 : sw ? 0.87 : 1.07);
+  return 4.0 + step * (K / GF_STEP) < 0.9 * (K > 2048 ? 0.30 : 0.37) * other_cost * K / 1024;
+}
+
+// the tile of gemm_f32_kernel that costs the least, and its cost
+static long f32_best_tile(bool sw, int M, int N, int& rb, int& nb) {
   static const int TILES[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 5}, {2, 2}, {2, 3}, {2, 4}, {2, 5}, {4, 2}, {4, 4}};
-  const bool sw = epi == TI_EPI_SWIGLU;
-  int rb = 1, nb = 1;
   long best = -1;
   for (const auto& t : TILES) {
     if (sw && t[0] * t[1] > 8) continue;           // two planes of it would not fit in LDS
@@ -386,8 +612,24 @@ static int launch_f32(const float* A, const float* W, float* out, int M, int N, 
       nb = t[1];
     }
   }
+  return best;
+}
+
+// What is chosen, for tests: 1: the tiles with shared splits.
+extern "C" int ti_gemm_generic_f32_choice(int swiglu, int M, int N, int K, long lda) {
+  int rb, nb;
+  return f32_shared_serves(f32_best_tile(swiglu != 0, M, N, rb, nb), swiglu != 0, M, N, K, lda) ? 1 : 0;
+}
+
+static int launch_f32(const float* A, const float* W, float* out, int M, int N, int K, long lda, int epi, hipStream_t stream) {
+  const bool sw = epi == TI_EPI_SWIGLU;
+  int rb, nb;
+  const long best = f32_best_tile(sw, M, N, rb, nb);
   const int wide_out = N % 4 == 0 && ((uintptr_t)out & 15) == 0;
   const int run = ((K + GF_RUNS - 1) / GF_RUNS + GF_STEP - 1) / GF_STEP * GF_STEP;
+  if (f32_shared_serves(best, sw, M, N, K, lda))
+    return sw ? launch_f32_shared<4, 2, 1, 2, true>(A, W, out, M, N, K, lda, run, epi, wide_out, stream)
+              : launch_f32_shared<2, 2, 4, 2, false>(A, W, out, M, N, K, lda, run, epi, wide_out, stream);
   const int m_tiles = (M + 16 * nb - 1) / (16 * nb), n_tiles = (N + 16 * rb - 1) / (16 * rb);
   const long grid = m_tiles == 1 ? n_tiles : (long)((n_tiles + 7) / 8) * 8 * m_tiles;
 #define GF_LAUNCH(R, B, S)                                                                                                \

@@ -51,6 +51,8 @@ int ti_gemm_bf16_tile_choice(int swiglu, int M, int N, int K, int* rest, int* n_
 int ti_gemm_bf16_qkv_choice(int M, int N, int K, int* n_big);
 // ... SwiGLU, in place of the first: a tile of 256 x 256 (10, 12), or 0
 int ti_gemm_bf16_quarters_choice(int M, int N, int K);
+// libti_gemm_generic: 1 where float32 rows take the tiles whose wavefronts split their floats together
+int ti_gemm_generic_f32_choice(int swiglu, int M, int N, int K, long lda);
 #ifdef __cplusplus
 }
 #endif
