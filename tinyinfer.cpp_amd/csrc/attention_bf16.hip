@@ -304,7 +304,8 @@ __device__ __forceinline__ void unrolled_while(F&& f) {
 //
 // Row R of a pair's keys (block A's 16, then block B's) lies at R HD 2 bytes with piece c (16 bytes) in place c ^ f(R),
 // f(R) = R % 4 + 4 ((R / 8) % 4): the rows that sixteen lanes read together differ in it.  The values of a block lie as in a page of 16
-// rows, 32 bytes a dim, with the two halves of dim d changed where bits 2 and 3 of d differ.
+// rows, 32 bytes a dim: LDS serves lanes 0 to 3, 12 to 15 and 20 to 27 together, which are dims 0 to 3 and 12 to 15 of one half and 4 to 11 of
+// the other, sixteen different places (1.8 ns a read of a unit; with the halves of some dims exchanged 3.4).
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 template <int HD> struct StagedPairs {
@@ -325,10 +326,10 @@ template <int HD> struct StagedPairs {
     const int f = r16 & (NP - 1);                        // f(R): bits 0, 1 and 3, 4 of R
 #pragma unroll
     for (int s = 0; s < HD / 32; ++s) k_at[s] = lds + R * (HD * 2) + (((s * 4 + quad) ^ f) << 4);
-    v_at = lds + K_BYTES + (quad >> 1) * V_BYTES + r16 * 32 + ((((quad & 1) ^ (r16 >> 2) ^ (r16 >> 3)) & 1) << 4);
+    v_at = lds + K_BYTES + (quad >> 1) * V_BYTES + r16 * 32 + ((quad & 1) << 4);
     const int row = lane / NP, c = lane % NP;            // of a load's rows; bits 2 of R and above come with the load's number
     k_lane = (unsigned)(row * HD * 2 + ((c ^ (row & 3)) << 4));
-    v_lane = (unsigned)((lane >> 1) * P * 2 + (((lane ^ (lane >> 3) ^ (lane >> 4)) & 1) << 4));
+    v_lane = (unsigned)((lane >> 1) * P * 2 + ((lane & 1) << 4));
   }
   // the loads of a pair into the stage at `stage` (bytes); pages that exist, as for load_pair
   __device__ __forceinline__ void ask(const PagedKV& kv, int pageA, int keyA, int pageB, int keyB, unsigned stage) const {
@@ -1218,8 +1219,9 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   // what this lane fetches in each of its loads of a turn
   //  K load g: LDS rows K_ROWS g .. + K_ROWS - 1; lane i -> row r = K_ROWS g + i / NP, slot c = i % NP,
   //            holds piece c ^ (r & (NP - 1)) of key 16 (r / 16) + swap23(r % 16)
-  //  V load g of a block: dims 32 g .. 32 g + 31; lane i -> dim 32 g + i / 2, keys 8 (i % 2) .. + 7: in pages of 16 rows 1 KiB of consecutive
-  //            bytes, and in LDS what an operand reads is 1 KiB of consecutive bytes too
+  //  V load g of a block: dims 32 g .. 32 g + 31; lane i -> dim 32 g + i / 2, keys 8 ((i + i / 32) % 2) .. + 7: in pages of 16 rows 1 KiB of
+  //            consecutive bytes, and in LDS what an operand reads is 1 KiB of consecutive bytes too, dims 16 to 31 with their halves exchanged:
+  //            of the lanes that LDS serves together, 0 to 3 and 12 to 15 with 20 to 27, no two meet in a bank so (1.8 ns a read of a unit, 3.5 without)
   // K load g starts for lane i (lr = i / NP < K_ROWS, c = i % NP) from its block's first K row at
   //   (k_lane ^ X(g)) + C(g),  k_lane = swap23(lr) * HD * 2 + (c ^ lr) * 16,
   //   X(g) = ((K_ROWS g) & (NP - 1)) * 16,  C(g) = swap23((K_ROWS g) & 15) * HD * 2
@@ -1231,7 +1233,7 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   static_assert(K_ROWS <= 16 && (K_ROWS & (K_ROWS - 1)) == 0, "rows of a K load lie in one block of 16");
   auto swap23 = [](int r16) __attribute__((always_inline)) { return ((r16 & 4) << 1) | ((r16 & 8) >> 1) | (r16 & 3); };
   const unsigned k_lane = (unsigned)(swap23(lane / NP) * HD * 2 + (((lane % NP) ^ (lane / NP)) << 4));
-  const unsigned v_lane = (unsigned)((lane >> 1) * P * 2 + (lane & 1) * 16);
+  const unsigned v_lane = (unsigned)((lane >> 1) * P * 2 + ((lane ^ (lane >> 5)) & 1) * 16);
 
   const unsigned lds_k = (unsigned)(size_t)smem + grp * Lds::TURN, lds_v = lds_k + Lds::VALUES;      // this group's first stages
   // the wavefronts of a group wait for each other at the workgroup's barrier (a handshake of a group's
@@ -1243,7 +1245,7 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   // LDS addresses of this lane's fragments; the stage, and the dims and the block of a V^T fragment, are
   // constants in the read instructions
   unsigned k_addr[KS];
-  const unsigned v_addr = lds_v + r32 * 32 + h * 16;
+  const unsigned v_addr = lds_v + r32 * 32 + ((h ^ (r32 >> 4)) & 1) * 16;
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) k_addr[ks] = lds_k + r32 * (HD * 2) + (((ks * 2 + h) ^ (r32 & (NP - 1))) << 4);
 

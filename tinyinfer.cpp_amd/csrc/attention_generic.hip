@@ -169,7 +169,8 @@ template <int DB> __device__ __forceinline__ void read_slices(af4* e, unsigned a
 // rows x 64 bytes for the keys and as many for the values.  As operands straight from memory, neighbouring lanes in different rows, a load
 // takes the unit that takes addresses 64 cycles, and a compute unit's eight wavefronts share it: some 3.4 us a round of eight blocks of
 // heads of 128; four lanes to a row's 64 bytes take 16.  A slice is asked for again, for the wavefront's next block, as soon as it has been
-// read.  Piece c (16 bytes) of row r lies in place 4 r + (c ^ (r / 4)), so that a quarter of the wavefront reads from different banks.  The
+// read.  Piece c (16 bytes) of row r lies in place 4 r + (c ^ (-(r / 4) % 4)): the sixteen lanes that LDS serves together are rows 0 to 3 and 12 to 15 of
+// one quarter and 4 to 11 of the next, and read from different banks so (from places c ^ (r / 4) a read takes twice as long).  The
 // arithmetic is the same, and so are the bits.  us, straight from memory, so, and with the order of tiles below: a portion
 // of 300 tokens, 16 heads of 128 on 8, 27.7, 20.8, 15.9; 512 tokens behind 300 63.5, 46.9, 43.3; 300 tokens with 32 heads of 64 23.8, 19.8,
 // 17.7; 8 single tokens of 900 31.6 -> 25.7.  Left: 304 workgroups on 256 units, one a unit, and each one's start and merge.
@@ -323,10 +324,10 @@ attention_f32_kernel(const float* __restrict__ q, const float* __restrict__ pool
   if (b <= b_last) {
     Block f0;
     if constexpr (STAGED) {
-      const int row = lane >> 2, piece = (lane & 3) ^ ((row >> 2) & 3);
+      const int row = lane >> 2, piece = (lane & 3) ^ (-(row >> 2) & 3);
       const unsigned k_off = (unsigned)row * (HD * 4) + piece * 16, v_off = (unsigned)row * (unsigned)(P * 4) + piece * 16;
       unsigned char* mine = smem + wave * STAGE;
-      const unsigned at = (unsigned)(size_t)mine + r16 * 64 + ((quad ^ (r16 >> 2)) << 4);
+      const unsigned at = (unsigned)(size_t)mine + r16 * 64 + ((quad ^ (-(r16 >> 2) & 3)) << 4);
       const auto rows_at = [](const float* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
       const auto page_of = [&](int block) { return __builtin_amdgcn_readfirstlane(tab[block * 16 / P]); };
       const auto ask_keys = [&](int page, int block) {

@@ -109,7 +109,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
   // chunk c covers k in [64 c, 64 c + 64); lane group j takes [64 c + 16 j, +16)
   const int chunks = (K + 63) / 64;
   if constexpr (STAGES > 0) {
-    const int lr = lane >> 3, piece = ((lane & 7) ^ lr) * 16;
+    const int lr = lane >> 3, piece = piece_of((lane & 7) ^ lr) * 16;
     const int n0 = blockIdx.x * G * (SW ? 8 : 16);
     unsigned voff[BLOCKS][2];
 #pragma unroll
@@ -136,7 +136,7 @@ gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, v
     };
     const unsigned at = (unsigned)(size_t)mine + r * 128;
     const int steps = wave < chunks ? (chunks - wave + NW - 1) / NW : 0;
-    staged_steps<BLOCKS, STAGES, RowPieces>(steps, at + (((2 * j) ^ (r & 7)) << 4), at + (((2 * j + 1) ^ (r & 7)) << 4), load,
+    staged_steps<BLOCKS, STAGES, RowPieces>(steps, at + ((j ^ (r & 7)) << 4), at + (((j + 4) ^ (r & 7)) << 4), load,
                                             [&](const RowPieces* e) {
 #pragma unroll
       for (int g = 0; g < G; ++g)
@@ -425,7 +425,7 @@ gemm_normed_kernel(const float* __restrict__ X, const bf16_t* __restrict__ W, in
   float prev = 0.f;
   if (EPI == TI_EPI_ADD_F32) prev = ((const float*)out_)[(size_t)(tok < M ? tok : 0) * N + (n < N ? n : N - 1)];
   __builtin_amdgcn_sched_barrier(0);
-  const int lr = lane >> 3, piece = ((lane & 7) ^ lr) * 16;
+  const int lr = lane >> 3, piece = piece_of((lane & 7) ^ lr) * 16;
   const unsigned v0 = (unsigned)min(lr, N - 1 - n0) * (unsigned)(K * 2) + piece;
   const unsigned v1 = SW ? v0 : (unsigned)min(8 + lr, N - 1 - n0) * (unsigned)(K * 2) + piece;
   const auto rows_at = [](const bf16_t* p) { return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, 0x7fffffff, 0x00020000); };
@@ -476,8 +476,8 @@ gemm_normed_kernel(const float* __restrict__ X, const bf16_t* __restrict__ W, in
 
   // ---- the product: chunks kw, kw + KW, ...
   const unsigned a_at = rows_lds + (r < M ? r : 0) * row_bytes + j * 32 + kw * 128;
-  const unsigned w_x = (unsigned)(size_t)mine + r * 128 + (((2 * j) ^ (r & 7)) << 4);
-  const unsigned w_y = (unsigned)(size_t)mine + r * 128 + (((2 * j + 1) ^ (r & 7)) << 4);
+  const unsigned w_x = (unsigned)(size_t)mine + r * 128 + ((j ^ (r & 7)) << 4);
+  const unsigned w_y = (unsigned)(size_t)mine + r * 128 + (((j + 4) ^ (r & 7)) << 4);
   unsigned stage = 0;
   int i = 0;
   auto multiply = [&](const RowPieces& w, const v4u& x, const v4u& y) __attribute__((always_inline)) {

@@ -286,7 +286,7 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
   if (steps > 0) {
     // Rows past the end repeat the last one; their sums are not stored.
     unsigned voff[BLOCKS][2];
-    const int lr = lane >> 3, piece = (lane & 7) ^ lr;
+    const int lr = lane >> 3, piece = piece_of((lane & 7) ^ lr);
 #pragma unroll
     for (int i = 0; i < BLOCKS; ++i)
 #pragma unroll
@@ -308,7 +308,7 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
           else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, dst, 16, voff[i][h], step * GF_STEP * 4, 0, 0);
         }
     };
-    const unsigned at = (unsigned)(size_t)mine + r16 * 128, x = at + (((2 * quad) ^ (r16 & 7)) << 4), y = at + (((2 * quad + 1) ^ (r16 & 7)) << 4);
+    const unsigned at = (unsigned)(size_t)mine + r16 * 128, x = at + ((quad ^ (r16 & 7)) << 4), y = at + (((quad + 4) ^ (r16 & 7)) << 4);
     staged_steps<BLOCKS, STAGES, Eight>(steps, x, y, load, multiply);
   }
   if (k1 > k0 && (k1 - k0) % GF_STEP) {

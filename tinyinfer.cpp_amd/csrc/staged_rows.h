@@ -3,10 +3,16 @@
 // every tile of the float32 product, 16 bytes a cycle for a whole compute unit).  Direct loads with eight lanes to a row's 128 bytes
 // take 16, and reading the operand back from LDS 8.  A wavefront has stages of its own: it waits for its own loads and meets no barrier.
 //
-// A block is 16 rows of 128 bytes (2 KiB): two loads of eight rows.  Piece c (16 bytes) of row r lies in place c ^ (r & 7), so that the
-// sixteen rows read together lie in different banks.
+// A block is 16 rows of 128 bytes (2 KiB): two loads of eight rows.  What stands c-th in a row r lies in place c ^ (r & 7).  A read of 16 bytes a lane
+// takes its lanes sixteen at a time, but not in their order: rows 0 to 3 and 12 to 15 of one operand piece go with rows 4 to 11 of the next
+// quarter's.  Those meet in no bank if the quarters of a wavefront read neighbouring places: pieces q and q + 4 by quarter q, 1.8 ns a read
+// of a unit (linear 1.8).  Pieces 2 q and 2 q + 1, two halves of 16 consecutive k, took 3.4 from places 2 q and 2 q + 1; where an operand is such a
+// pair the loads put piece 2 q into place q and piece 2 q + 1 into place q + 4 (piece_of).
 #pragma once
 #include <hip/hip_runtime.h>
+
+// the piece of a row's eight that stands c-th where a lane's operand is pieces 2 q and 2 q + 1
+__device__ __forceinline__ int piece_of(int c) { return ((c & 3) << 1) | (c >> 2); }
 
 // s_waitcnt with only vmcnt set (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14)
 template <int N> __device__ __forceinline__ void wait_vmcnt() {
