@@ -645,7 +645,7 @@ extern "C" int ti_qk_norm_rope_kv_write(int dtype, const float* qkv, const float
     const long heads = (long)M * (n_head + n_kv);
     const auto go = [&](auto kernel, auto* to_pool, auto* to_q, int each) {
       const long groups = (long)M * ((n_head + n_kv + 4 * each - 1) / (4 * each)) + (long)((M + 15) / 16) * n_kv;
-      if (groups > 0x7fffffff) return false;
+      if (groups <= 0 || groups > 0x7fffffff) return false;
       kernel<<<(unsigned)groups, 256, 0, stream>>>(qkv, q_w, k_w, inv_freq, (const float2*)rope_table, table_len, pos, slot, table,
                                                    table_stride, to_pool, to_q, M, n_head, n_kv, page_size, eps);
       return true;

@@ -8,6 +8,7 @@
 //
 //   gemm_f32_kernel      float32 with rows of whole, aligned float4s: matrix
 //                        instructions on the floats cut into three bfloat16
+//   gemm_f32_shared_kernel  the same bits, cut once a workgroup: many tiles
 //   gemm_generic_kernel  everything else: one fused multiply-add at a time, in
 //                        ascending k
 #include <float.h>
