@@ -121,6 +121,44 @@ def test_records_of_a_draw_say_what_the_lists_say():
     assert SamplingParams(0.5, 7) == SamplingParams(0.5, 7) and repr(SamplingParams()).count("record") == 0
 
 
+def test_parameters_of_a_draw_hold_what_they_were_given():
+    """Drawn with or not, a SamplingParams' attributes are its four, in vars, in a pickle and in a copy; parameters of a caller's own class, whose
+    numbers may change between draws, go by the lists whether or not it derives from SamplingParams."""
+    import copy
+    import pickle
+
+    from tinyinfer_amd.sampling import Sampler, SamplingParams
+    p = SamplingParams(0.5, 7, 0.9, -3)
+    given = {"temperature": 0.5, "top_k": 7, "top_p": 0.9, "seed": -3}
+    fresh = pickle.dumps(p)
+    for _ in range(2):
+        assert vars(p) == given and SamplingParams(**vars(p)) == p and pickle.dumps(p) == fresh
+        first = Sampler._records(1, [p], (1,), (0,))
+        again = Sampler._records(2, [pickle.loads(fresh), copy.copy(p)], (1, 1), (0, 0))
+        assert again[0] == 2 * first[0] and len(first[0]) == 24
+
+    class Cooling(SamplingParams):
+        calls = 0
+
+        @property
+        def top_p(self):
+            Cooling.calls += 1
+            return 1.0 / Cooling.calls
+
+        @top_p.setter
+        def top_p(self, value):
+            pass
+
+    class Named(SamplingParams):
+        _record = b"not a record"
+    for own in (Cooling, Named):
+        assert Sampler._records(1, [own.__new__(own)], (1,), (0,)) is None
+    bad = SamplingParams(0.5, 1 << 40)                    # cut to 32 bits by the lists, at every call
+    for _ in range(2):
+        assert Sampler._records(2, [p, bad], (1, 2), (0, 0)) is None
+    assert Sampler._records(1, [p], (1,), (0,)) == first
+
+
 @pytest.mark.parametrize("heads,rows,context,tokens,behind,one", [
     # whole portions: enough units left, or short rows; then long rows beside portions on most units or all, which took up to 12 % longer in one launch
     (16, 2, 2000, 512, 0, True), (16, 2, 2000, 768, 0, True), (16, 2, 12000, 768, 4000, True), (16, 4, 500, 1024, 8000, True),

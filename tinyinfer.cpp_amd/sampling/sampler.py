@@ -15,25 +15,26 @@ _RECORD = struct.Struct("@fif4xQ")      # a SamplingParams of the library's
 DEFAULT_TOP_K = 512          # the reference's cut when --top-k is 0: src/main.cpp:47-48
 
 
+class _Recorded:
+    """Where a SamplingParams keeps its record: beside its attributes, which are what it is given."""
+    __slots__ = ("_record",)
+
+
 @dataclass(frozen=True)
-class SamplingParams:
+class SamplingParams(_Recorded):
     temperature: float = 0.0     # <= 0: greedy (src/main.cpp:24,31-38)
     top_k: int = 0               # 0: the reference's default of 512
     top_p: float = 1.0
     seed: int = 42               # src/main.cpp:27
 
-    def __post_init__(self):
-        # what the library reads, packed once: four lists of a number a request each took longer at every call than its kernels' launches
-        # (numbers of other types, or out of their type's range, are converted at the call: None)
-        plain = (type(self.temperature) in (int, float) and type(self.top_k) is int and type(self.top_p) in (int, float) and type(self.seed) is int)
-        try:
-            record = _RECORD.pack(self.temperature, self.top_k, self.top_p, self.seed & ((1 << 64) - 1)) if plain else None
-        except (struct.error, OverflowError):
-            record = None
-        object.__setattr__(self, "_record", record)
+    def __getstate__(self):
+        return self.__dict__
 
     def effective_top_k(self) -> int:
         return self.top_k if self.top_k > 0 else DEFAULT_TOP_K
+
+
+_keep = _Recorded._record.__set__
 
 
 def uniform(seed: int, request: int, n_generated: int) -> float:
@@ -75,12 +76,25 @@ class Sampler:
 
     @staticmethod
     def _records(n, params, requests, counters):
-        """The same from the parameters' own records, or None where one of them has none or a number does not fit (64 rows: 4 us, 17 above; a whole call of 64 rows of 151,936 61.6 -> 55.3)."""
+        """The same from the parameters' own records, or None where one of them can have none or a number does not fit.  A record is packed at its
+        first draw (64 rows: kept ones 5 us, new ones 29, the lists above 17; a whole call of 64 rows of 151,936 with kept ones 61.6 -> 55.3)."""
         try:
-            if not len(params) == len(requests) == len(counters) == n:
+            if not len(params) == len(requests) == len(counters) == n or (n and {*map(type, params)} != {SamplingParams}):
                 return None
             words = f"{n}q"
-            return b"".join([p._record for p in params]), struct.pack(words, *requests), struct.pack(words, *counters)
+            words = struct.pack(words, *requests), struct.pack(words, *counters)
+            try:
+                records = [p._record for p in params]
+            except AttributeError:
+                for p in params:
+                    t, k, q, s = p.temperature, p.top_k, p.top_p, p.seed
+                    try:      # (numbers of other types, or out of their type's range, are converted at every call)
+                        plain = type(k) is type(s) is int and (type(t) is float or type(t) is int) and (type(q) is float or type(q) is int)
+                        _keep(p, _RECORD.pack(t, k, q, s & ((1 << 64) - 1)) if plain else None)
+                    except (struct.error, OverflowError):
+                        _keep(p, None)
+                records = [p._record for p in params]
+            return (b"".join(records),) + words
         except (AttributeError, TypeError, struct.error, OverflowError):
             return None
 
