@@ -91,6 +91,30 @@ def test_which_gate_up_products_go_by_quarters(ops, M, F, K, tile):  # noqa: F81
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
+# whole rounds by quarters of four or eight wavefronts, the columns left in another tile: of no whole tile and no whole piece of 16 bytes (9717)
+@pytest.mark.parametrize("M,F,K", [(1000, 9728, 2560), (800, 9717, 2560), (1792, 9728, 2560), (1300, 6144, 2048), (1300, 12288, 4096), (2304, 12288, 4096)])
+def test_gate_up_products_by_quarters_in_two_ranges(ops, M, F, K):  # noqa: F811
+    """Rows and weights whose tiles of 256 x 256 are no whole rounds of the units: the bits of one tile of 128 x 128 everywhere."""
+    lib = ops.lib("gemm_bf16")
+    rest, n_big = ctypes.c_int(), ctypes.c_int()
+    tile = lib.ti_gemm_bf16_quarters_ranges(M, F, K, ctypes.byref(rest), ctypes.byref(n_big))
+    assert tile in (10, 12) and 0 < n_big.value < F and n_big.value % 128 == 0 and rest.value > 0
+    g = torch.Generator(device="cuda").manual_seed(M + F)
+    a = torch.randn(M, K, device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn(2 * F, K, device="cuda", generator=g) * 0.1).to(torch.bfloat16)
+    outs = []
+    try:
+        for force in (0, 2):
+            lib.ti_tuning_set(b"force_tile", force)
+            room = torch.full((M * F + 8,), 7.0, device="cuda", dtype=torch.bfloat16)
+            ops.linear(a, w, room[:M * F].view(M, F), "swiglu")
+            assert bool((room[M * F:] == 7.0).all())
+            outs.append(room)
+    finally:
+        lib.ti_tuning_reset()
+    assert torch.isfinite(outs[0]).all() and torch.equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("M,nh,nkv,hd,K,P,norm,rope", [
     (300, 3, 1, 128, 128, 16, True, "table"), (513, 5, 1, 64, 256, 32, True, None), (257, 4, 0, 128, 64, 16, False, "computed"),
     (100, 2, 2, 64, 192, 48, False, "table")])

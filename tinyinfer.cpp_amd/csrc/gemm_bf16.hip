@@ -1742,11 +1742,16 @@ static const TileRate TILES_PLAIN[] = {
 static const TileRate TILES_SWIGLU[] = {
     {1, 256, 128, 3.08f, 0.56f, 0.28f, 0.f, 0.f, 0.f},
     {2, 128, 128, 0.f, 0.54f, 0.05f, 0.f, 0.f, 0.f},       {7, 64, 128, 0.f, 0.40f, 0.03f, 0.f, 0.f, 0.f},
-    {5, 64, 128, 0.f, 0.45f, 0.09f, 0.f, 0.55f, 0.20f}};
-// SwiGLU in tiles of 256 x 256 by quarters, eight wavefronts and four (fitted to 52 products, 200 to 6,000 rows times the four sizes' gate/up: the
-// median error is 1.5 %, and what the costs choose is on average 0.2 % slower than the fastest).  They are chosen against the others' best, whole or in two ranges.
-static const TileRate TILES_QUARTERS[] = {
-    {10, 256, 256, 5.76f, 0.91f, 0.60f, 0.f, 0.f, 0.f}, {12, 256, 256, 8.00f, 0.91f, 0.55f, 0.f, 0.f, 0.f}};
+    {5, 64, 128, 0.f, 0.45f, 0.09f, 0.f, 0.55f, 0.20f},
+    // by quarters, eight wavefronts and four
+    {10, 256, 256, 5.76f, 0.93f, 0.60f, 0.f, 0.f, 0.f},    {12, 256, 256, 8.00f, 0.93f, 0.55f, 0.f, 0.f, 0.f}};
+// Two SwiGLU ranges, of which the first goes by quarters as a rule, take more than their launches' costs by this share and this time.  Over 122 products, 200
+// to 6,000 rows times the four sizes' gate/up, up to nine plans each in turns, what the costs choose is on average 0.5 % slower than the fastest, 1.6 % faster than
+// the better of no tiles by quarters and only whole launches of them, and never slower than either beyond noise (without this share and time 0.65 % slower than
+// so, 2048-wide gate/up under 1,650 to 1,792 and 3,000 to 3,300 rows by 2 to 5 %).  us, 256 x 256 in the older loop, quarters as whole launches alone, and
+// so: 4B's gate/up under 800 and 1,000 rows 100 102 93, 106 110 99, under 1,650 176 176 165; 1.7B's under 1,300 77 79 74; 8B's under 650, 1,000, 1,300 and
+// 2,304 rows 149 147 136, 179 177 168, 266 263 246, 395 396 373.
+static const double RANGES_SHARE = 1.04, RANGES_US = 3.0;
 static const double LAUNCH_US = 2.0;
 
 static double tile_us(const TileRate& t, long workgroups, int k_tiles) {
@@ -1767,11 +1772,12 @@ struct TileChoice {
   int rest = 0;
 };
 // The cheapest tile for M rows times `rows` rows of W (for SwiGLU both halves), k_tiles deep, the launch `copies` times as
-// large (K split).  two_ranges: also two launches, whole rounds of one tile and the columns left over in another.
-static TileChoice choose_tile(bool swiglu, int M, int rows, int k_tiles, int copies, bool two_ranges) {
+// large (K split).  two_ranges: also two launches, whole rounds of one tile and the columns left over in another.  quarters: SwiGLU by
+// quarters as well, whole or for either range.
+static TileChoice choose_tile(bool swiglu, int M, int rows, int k_tiles, int copies, bool two_ranges, bool quarters = false) {
   const TileRate* tiles = swiglu ? TILES_SWIGLU : TILES_PLAIN;
   const int n = swiglu ? (int)(sizeof(TILES_SWIGLU) / sizeof(TileRate)) : (int)(sizeof(TILES_PLAIN) / sizeof(TileRate));
-  auto allowed = [&](const TileRate& t) { return t.bn != 160 || g_tiles_160; };
+  auto allowed = [&](const TileRate& t) { return t.bn == 160 ? g_tiles_160 != 0 : t.bn != 256 || (quarters && g_tiles_256); };
   auto row_tiles = [&](const TileRate& t) { return (long)((M + t.bm - 1) / t.bm); };
   auto us = [&](const TileRate& t, int r) { return LAUNCH_US + tile_us(t, row_tiles(t) * ((r + t.bn - 1) / t.bn) * copies, k_tiles); };
   TileChoice best;
@@ -1790,20 +1796,10 @@ static TileChoice choose_tile(bool swiglu, int M, int rows, int k_tiles, int cop
     const double first = us(t, n_big);
     for (int j = 0; j < n; ++j) {
       if (!allowed(tiles[j])) continue;
-      const double c = first + us(tiles[j], rows - n_big);
+      double c = first + us(tiles[j], rows - n_big);
+      if (quarters) c = c * RANGES_SHARE + RANGES_US;
       if (c < best.us) best = {t.id, c, n_big, tiles[j].id};
     }
-  }
-  return best;
-}
-
-// ... by quarters: the cheaper of the two (id 0: neither)
-static TileChoice choose_quarters(int M, int rows, int k_tiles) {
-  TileChoice best;
-  if (!g_tiles_256) return best;
-  for (const TileRate& t : TILES_QUARTERS) {
-    const double us = LAUNCH_US + tile_us(t, (long)((M + 255) / 256) * ((rows + 255) / 256), k_tiles);
-    if (!best.id || us < best.us) best = {t.id, us, 0, 0};
   }
   return best;
 }
@@ -1818,6 +1814,7 @@ struct QKVChoice {
   int rows = 0;             // of a tile; 512: tiles of 256 x 256; 0: left to the product and the preparation kernel
   int n_big = 0;            // > 0: that many columns in 256-row tiles, the others in 128-row tiles
 };
+static const TileRate TILE_QKV_256 = {512, 256, 256, 5.76f, 0.91f, 0.60f, 0.f, 0.f, 0.f};
 static QKVChoice qkv_choice(int M, int N, int K) {
   QKVChoice c{g_qkv_rows, 0};
   if (c.rows) return c;                             // (a test asks for a tile)
@@ -1848,7 +1845,7 @@ static QKVChoice qkv_choice(int M, int N, int K) {
   // 103 and 97, of 6144 x 2560 75 and 67, 1,500 of 6144 x 4096 97 and 86).  Under a shorter K the heads weigh more and less is left to gain
   // (6144 x 2048 64 and 60, 5120 x 2048 60 and 58; 3,000 rows of 6144 x 2048 95 and 115).
   if (g_tiles_256 && k_tiles >= 40) {
-    const double wide = LAUNCH_US + 7.0 + tile_us(TILES_QUARTERS[0], row_tiles * ((N + 255) / 256), k_tiles);
+    const double wide = LAUNCH_US + 7.0 + tile_us(TILE_QKV_256, row_tiles * ((N + 255) / 256), k_tiles);
     if (wide < least) {
       least = wide;
       c = {512, 0};
@@ -1867,10 +1864,16 @@ extern "C" int ti_gemm_bf16_tile_choice(int swiglu, int M, int N, int K, int* re
   *n_big = swiglu ? c.n_big / 2 : c.n_big;
   return c.id;
 }
-// ... what SwiGLU takes in its place: 10 or 12, or 0: that choice.
+// ... where SwiGLU goes by quarters in its place, whole or in a range: likewise, 0 where it does not.
+extern "C" int ti_gemm_bf16_quarters_ranges(int M, int N, int K, int* rest, int* n_big) {
+  const TileChoice c = choose_tile(true, M, 2 * N, K / PBK, 1, true, true);
+  *rest = c.rest;
+  *n_big = c.n_big / 2;
+  return c.id >= 10 || c.rest >= 10 ? c.id : 0;
+}
 extern "C" int ti_gemm_bf16_quarters_choice(int M, int N, int K) {
-  const TileChoice q = choose_quarters(M, 2 * N, K / PBK);
-  return q.id && q.us < choose_tile(true, M, 2 * N, K / PBK, 1, true).us ? q.id : 0;
+  int rest, n_big;
+  return ti_gemm_bf16_quarters_ranges(M, N, K, &rest, &n_big);
 }
 extern "C" int ti_gemm_bf16_qkv_choice(int M, int N, int K, int* n_big) {
   const QKVChoice c = qkv_choice(M, N, K);
@@ -1958,11 +1961,7 @@ static int launch_tiled_best(const bf16_t* A, const bf16_t* W, void* out, int M,
                              hipStream_t s) {
   constexpr bool SW = EPI == TI_EPI_SWIGLU;
   if (g_force_tile) return launch_tile<EPI>(g_force_tile, A, W, out, M, N, K, lda, s);
-  const TileChoice c = choose_tile(SW, M, SW ? 2 * N : N, K / PBK, 1, true);
-  if constexpr (SW) {
-    const TileChoice q = choose_quarters(M, 2 * N, K / PBK);
-    if (q.id && q.us < c.us) return launch_tile<EPI>(q.id, A, W, out, M, N, K, lda, s);
-  }
+  const TileChoice c = choose_tile(SW, M, SW ? 2 * N : N, K / PBK, 1, true, SW);
   if (!c.n_big) return launch_tile<EPI>(c.id, A, W, out, M, N, K, lda, s);
   const int n_big = SW ? c.n_big / 2 : c.n_big;
   if (int rc = launch_tile<EPI>(c.id, A, W, out, M, N, K, lda, s, 1, 0, n_big)) return rc;

@@ -49,7 +49,8 @@ void ti_tuning_reset();                              // every choice back to the
 // product and the preparation kernel; 512: tiles of 256 x 256), 256 and 128 where n_big > 0.
 int ti_gemm_bf16_tile_choice(int swiglu, int M, int N, int K, int* rest, int* n_big);
 int ti_gemm_bf16_qkv_choice(int M, int N, int K, int* n_big);
-// ... SwiGLU, in place of the first: a tile of 256 x 256 (10, 12), or 0
+// ... SwiGLU by quarters (tiles 10 and 12), in place of the first; 0: that one
+int ti_gemm_bf16_quarters_ranges(int M, int N, int K, int* rest, int* n_big);
 int ti_gemm_bf16_quarters_choice(int M, int N, int K);
 // libti_gemm_generic: 1 where float32 rows take the tiles whose wavefronts split their floats together
 int ti_gemm_generic_f32_choice(int swiglu, int M, int N, int K, long lda);
