@@ -78,6 +78,18 @@ def test_product_whose_wavefronts_split_together(ops, swiglu, M, N, K, lda):  # 
             assert torch.equal(torch.isnan(full[:m]), torch.isnan(ref))
 
 
+@pytest.mark.parametrize("swiglu,M,N,K,together", [
+    # one workgroup a unit: a round that is nearly full, and one that has just begun; 600 rows begin a fourth round of the dies with the most columns
+    (1, 256, 3072, 1024, 1), (1, 512, 3072, 1024, 0), (1, 384, 4864, 896, 1), (1, 600, 4864, 896, 0), (1, 64, 9728, 2560, 1), (1, 100, 9728, 2560, 0),
+    # two workgroups a unit
+    (0, 512, 4096, 1024, 0), (0, 1000, 4096, 1024, 1), (0, 1280, 4096, 1024, 0), (0, 300, 6144, 4096, 0), (0, 2048, 6144, 4096, 1)])
+def test_which_products_split_together(ops, swiglu, M, N, K, together):  # noqa: F811
+    """The faster of the two kernels, as measured on either side of the line."""
+    choice = ops.lib("gemm_generic").ti_gemm_generic_f32_choice
+    choice.argtypes = [ctypes.c_int] * 4 + [ctypes.c_long]
+    assert choice(swiglu, M, N, K, K) == together
+
+
 @pytest.mark.parametrize("M,N,K", [(7, 64, 20), (37, 132, 1056), (300, 96, 260)])
 def test_product_of_what_three_bfloat16_do_not_hold(ops, M, N, K):  # noqa: F811
     """Operands from 1e-30 to the largest float, infinite ones and NaN, beside zeros: what float64 gives in 32 bits is what comes out, of

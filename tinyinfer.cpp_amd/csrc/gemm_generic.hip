@@ -586,18 +586,26 @@ static long f32_tile_cost(int rb, int nb, bool sw, int M, int N, int units) {
   return rounds * (2 + pl * rb * nb + 4 * (pl * rb + nb));
 }
 
-// Whether the tiles with shared splits take it, 64 tokens x 128 weight rows (SwiGLU: 64 gates and their ups).  Their launch: 4 us, and a k-step
-// 1.83 us where a unit has two of them, 1.07 (SwiGLU 0.87) where it has one; a unit of the other's cost 0.37 us a thousand of K, 0.30 of a
-// K beyond 2,048.  A tenth in favour of the other, which stays where a round of tiles leaves units idle.  us, the other and this: 40 rows x
-// 151936 x 1024 241 196, 65 278 (278, left), 200 711 563, [gate; up] 6144 x 1024 under 200 rows 32 (left), 256 36.3 31.9, 512 56 (left), 1,000
-// 112 96, 12288 x 2048 under 300 125 115; 4096 x 1024 under 300 29 (38, left), 1,000 79 64, 2,000 159 120; 6144 x 4096 under 300 110 (114, left).
+// Whether the tiles with shared splits take it, 64 tokens x 128 weight rows (SwiGLU: 64 gates and their ups).  The dies take columns of tiles in turn, so
+// what counts is the rounds of the die that has the most.  A unit holds two workgroups of the former (four wavefronts of 242 registers): a round is 3 us
+// and 1.6 a k-step of both, 1.05 where there is one each.  Of the latter (eight wavefronts of 145) it holds one: 2.5 us and 0.86 a k-step a round.
+// The other kernel's cost is worth 0.075 us and 0.256 a thousand of K.  Over 232 products of thirteen weights, 40 to 3,000 rows, what this chooses is on
+// average 0.04 % slower than the faster of the two, at worst 2.3 % (rounds of all units at one rate, a tenth in favour of the other: 0.7 and 17 %).
+// us, the other and this: 64 rows of 151936 x 1024 214 172, 300 790 654; [gate; up] 6144 x 1024 under 200 rows 30.4 31.0, 256 34.6 29.9, 512 51 58, 1,000
+// 104 90, 9728 x 896 under 600 92 102, 384 64 52, 19456 x 2560 under 64 79 67, 512 365 342; 4096 x 1024 under 512 37.1 38.5, 1,000 73 60, 2,000 153 114;
+// 6144 x 4096 under 300 108 135, 2,048 699 665.
 static bool f32_shared_serves(long other_cost, bool sw, int M, int N, int K, long lda) {
   // whole k-steps, and a tile's rows within what a buffer's descriptor spans
   if (K % GF_STEP || K >= (1 << 20) || lda >= (1 << 20)) return false;
-  const long tiles = (long)((M + 63) / 64) * ((N + (sw ? 63 : 127)) / (sw ? 64 : 128)), units = compute_units();
-  const long rest = tiles % (2 * units);
-  const double step = 1.83 * (tiles / (2 * units)) + (rest == 0 ? 0.0 : rest > units ? 1.83 : sw ? 0.87 : 1.07);
-  return 4.0 + step * (K / GF_STEP) < 0.9 * (K > 2048 ? 0.30 : 0.37) * other_cost * K / 1024;
+  const long columns = (N + (sw ? 63 : 127)) / (sw ? 64 : 128), tiles = (long)((M + 63) / 64) * ((columns + 7) / 8), units = (compute_units() + 7) / 8;      // of a die
+  const double steps = K / GF_STEP;
+  double us = 1.0;
+  if (sw) us += (double)((tiles + units - 1) / units) * (2.5 + 0.86 * steps);
+  else {
+    const long rest = tiles % (2 * units);
+    us += (double)(tiles / (2 * units) + (rest > units)) * (3.0 + 1.6 * steps) + (rest > 0 && rest <= units ? 3.0 + 1.05 * steps : 0.0);
+  }
+  return us < 2.7 + other_cost * (0.075 + 0.256 * K / 1024);
 }
 
 // the tile of gemm_f32_kernel that costs the least, and its cost
