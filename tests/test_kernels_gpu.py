@@ -2085,6 +2085,40 @@ def test_attention_bf16_portions_at_the_edges_of_runs(ops, nh, nkv, hd, P, varia
     assert (got - want).abs().max() < 2e-2          # as above: weights and results rounded to 8 bits of values of up to 4
 
 
+@pytest.mark.parametrize("nh,nkv,P", [(32, 32, 131072), (2, 1, 1 << 23)])
+def test_attention_bf16_portions_in_pages_of_2_gib_and_more(ops, nh, nkv, P):
+    """Pages of more than a buffer descriptor spans, which the kernel takes that reads flat addresses: what pages of 16 rows give, with a sink in
+    the denominator."""
+    g = torch.Generator(device="cuda").manual_seed(nh)
+    hd, entries = 128, [(70, 300), (130, 0)]
+    q = torch.randn(200, nh * hd, device="cuda", generator=g).to(torch.bfloat16)
+    sink = torch.randn(nh, device="cuda", generator=g) + 3
+    k, v = (torch.randn(2, 384, nkv, hd, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+    lib, results = ops.lib("attention_bf16"), []
+    lib.ti_attention_bf16_sink.argtypes = [ctypes.c_void_p]
+    for rows in (16, P):
+        each = -(-384 // rows)
+        pool = torch.zeros(2 * each, 2, nkv, rows, hd, device="cuda", dtype=torch.bfloat16)
+        for e in range(2):
+            for n in range(each):
+                at, m = slice(n * rows, (n + 1) * rows), min(rows, 384)
+                pool[e * each + n, 0, :, :m] = k[e, at].transpose(0, 1)
+                pool[e * each + n, 1].view(nkv, hd, rows)[:, :, :m] = v[e, at].permute(1, 2, 0)
+        table = torch.arange(2 * each, dtype=torch.int32).view(2, each)
+        out = torch.zeros_like(q)
+        lib.ti_attention_bf16_sink(sink.data_ptr())
+        try:
+            assert run_attention(ops, FakeCtx(entries), View(dev(table)), q, pool, out, nh, nkv, hd, hd ** -0.5, None)
+            torch.cuda.synchronize()
+        finally:
+            lib.ti_attention_bf16_sink(None)
+        results.append(out)
+        del pool
+    torch.cuda.empty_cache()
+    assert results[0].abs().max() > 0.1
+    assert (f64(results[0]) - f64(results[1])).abs().max() < 2e-2      # as above: weights and results rounded to 8 bits
+
+
 def test_attention_bf16_far_into_long_contexts(ops):
     """Rows of single tokens behind 20,000 and 32,767 cached tokens (a block table wider than the 1,024 entries
     the decode kernel can hold in LDS, contexts cut into many runs) and portions of prompts deep inside a

@@ -1051,6 +1051,7 @@ bool Ops::attention(const AttentionWork& work, Workspace& ws, const CacheView& v
       }
       // the portions first: with their keys cut into runs, the merge writes every row of the step, and
       // the rows of single tokens get their own result afterwards
+      bool portions_left = work.n_tiles != 0;
       if (work.n_tiles && (head_dim == 64 || head_dim == 128) && work.n_tiles * heads < PAIRED_BELOW && work.tiles_small &&
           use.paired_prefill) {
         bool paired = false;
@@ -1066,9 +1067,12 @@ bool Ops::attention(const AttentionWork& work, Workspace& ws, const CacheView& v
             q.data, pool.data, view.table, view.table_width, work.tiles_small, work.entry_meta, out.data, work.n_tiles_small,
             heads, kv_heads, head_dim, P, scale, softcap, window, (int)work.M, part_o, part_ml, S, paired ? 1 : 0,
             (hipStream_t)stream);
-        if (rc == 3) done = false;
-        else check("attention_bf16", rc, "attention(prefill, paired)");
-      } else if (work.n_tiles) {
+        if (rc != 3) {
+          check("attention_bf16", rc, "attention(prefill, paired)");
+          portions_left = false;
+        }
+      }
+      if (portions_left) {
         int rc = KERNEL("attention_bf16", ti_attention_prefill_capped_bf16)(
             q.data, pool.data, view.table, view.table_width, work.tiles, work.entry_meta, out.data, work.n_tiles, heads,
             kv_heads, head_dim, P, scale, softcap, window, (hipStream_t)stream);
