@@ -124,6 +124,31 @@ def test_qkv_product_in_tiles_of_256_by_256(ops, M, nh, nkv, hd, K, P, norm, rop
     qkv_prepared_case(ops, 512, M, nh, nkv, hd, K, P, norm, rope)
 
 
+@pytest.mark.parametrize("M,N,K,wide", [
+    # both sides of the line: rounds of 256 x 256 nearly full, and ones that have just begun
+    (2048, 6144, 2560, 1), (3000, 6144, 2560, 0), (6000, 6144, 2560, 0), (2048, 6144, 4096, 1), (6000, 6144, 4096, 0), (2048, 4096, 2048, 0),
+    (3000, 4096, 2048, 1), (6000, 4096, 2048, 0), (4096, 4096, 1024, 1), (2048, 4096, 1024, 0), (3500, 10240, 5120, 0), (2048, 5120, 2048, 1)])
+def test_which_qkv_products_take_tiles_of_256_by_256(ops, M, N, K, wide):  # noqa: F811
+    """By their costs, at any K."""
+    assert ops.lib("gemm_bf16").ti_gemm_bf16_qkv_wide(M, N, K) == wide
+
+
+@pytest.mark.parametrize("M,nh,nkv,hd,ranges,wide", [(2048, 32, 4, 128, 1, 1), (1900, 70, 5, 64, 1, 1), (3000, 32, 8, 128, 1, 0), (3000, 16, 8, 128, 0, 1)])
+def test_qkv_product_as_chosen_with_and_without_tiles_of_256_by_256(ops, M, nh, nkv, hd, ranges, wide):  # noqa: F811
+    """Tiles of 256 x 256 where they are chosen, and without them 256-row tiles, with the heads left over in 128-row tiles where `ranges`: the bits
+    of the product and the kernel that prepares whole steps."""
+    lib, n_big, K = ops.lib("gemm_bf16"), ctypes.c_int(0), 2048
+    N = (nh + 2 * nkv) * hd
+    assert lib.ti_gemm_bf16_qkv_choice(M, N, K, ctypes.byref(n_big)) == 256 and (0 < n_big.value < N) == ranges
+    assert lib.ti_gemm_bf16_qkv_wide(M, N, K) == wide
+    try:
+        for on in (1, 0):
+            lib.ti_tuning_set(b"tiles_256", on)
+            qkv_prepared_case(ops, 0, M, nh, nkv, hd, K, 16, True, "table")
+    finally:
+        lib.ti_tuning_set(b"tiles_256", 1)
+
+
 @pytest.mark.parametrize("M,N,K", [(1024, 1024, 128), (2048, 512, 128), (512, 2048, 64), (384, 1152, 64)])
 def test_dies_blocks_cover_every_tile_once(ops, M, N, K):  # noqa: F811
     """Grids that the eight dies cut by rows, by columns and by both, and one that none of the cuts divides."""

@@ -1814,8 +1814,13 @@ struct QKVChoice {
   int rows = 0;             // of a tile; 512: tiles of 256 x 256; 0: left to the product and the preparation kernel
   int n_big = 0;            // > 0: that many columns in 256-row tiles, the others in 128-row tiles
 };
-static const TileRate TILE_QKV_256 = {512, 256, 256, 5.76f, 0.91f, 0.60f, 0.f, 0.f, 0.f};
-static QKVChoice qkv_choice(int M, int N, int K) {
+// Tiles of 256 x 256 read A and W the least, but every round of them ends with two ranges of heads, some 10 us: its start here.  Fitted to 128 products, 200 to
+// 6,000 rows times q/k/v of 4096 to 10240 rows at K of 1,024 to 5,120 (median error 0.7 %); what is chosen is on average 0.1 % slower than the faster of
+// this tile and the others' best, at worst 8 %.  us, the others and this tile: 6144 x 2560 under 2,048 rows 78 72, 3,000 117 134, 6,000 203 214; 6144 x 4096
+// under 1,300 (product and preparation apart; this tile 97), 2,048 106 104, 6,000 288 313; 4096 x 2048 under 2,048 rows 38 57, 3,000 68 61, 6,000 106 121;
+// 5120 x 2048 under 3,000 71 67; 4096 x 1024 under 4,096 48 44, 7168 x 5120 under 2,048 144 133, 10240 x 5120 under 3,500 360 374.
+static const TileRate TILE_QKV_256 = {512, 256, 256, 16.1f, 0.91f, 0.61f, 0.f, 0.f, 0.f};
+static QKVChoice qkv_choice(int M, int N, int K, bool wide_tiles) {
   QKVChoice c{g_qkv_rows, 0};
   if (c.rows) return c;                             // (a test asks for a tile)
   const long units = compute_units();
@@ -1841,11 +1846,9 @@ static QKVChoice qkv_choice(int M, int N, int K) {
       c = {256, cols * 128};
     }
   }
-  // Tiles of 256 x 256 read A and W the least; they finish twice the heads, 7 us (us, the best of the others and they: 2,048 rows of 6144 x 4096
-  // 103 and 97, of 6144 x 2560 75 and 67, 1,500 of 6144 x 4096 97 and 86).  Under a shorter K the heads weigh more and less is left to gain
-  // (6144 x 2048 64 and 60, 5120 x 2048 60 and 58; 3,000 rows of 6144 x 2048 95 and 115).
-  if (g_tiles_256 && k_tiles >= 40) {
-    const double wide = LAUNCH_US + 7.0 + tile_us(TILE_QKV_256, row_tiles * ((N + 255) / 256), k_tiles);
+  // (the others' is the least of several costs, which is on average a fiftieth too low)
+  if (wide_tiles && g_tiles_256) {
+    const double wide = (LAUNCH_US + tile_us(TILE_QKV_256, row_tiles * ((N + 255) / 256), k_tiles)) / 1.02;
     if (wide < least) {
       least = wide;
       c = {512, 0};
@@ -1876,10 +1879,12 @@ extern "C" int ti_gemm_bf16_quarters_choice(int M, int N, int K) {
   return ti_gemm_bf16_quarters_ranges(M, N, K, &rest, &n_big);
 }
 extern "C" int ti_gemm_bf16_qkv_choice(int M, int N, int K, int* n_big) {
-  const QKVChoice c = qkv_choice(M, N, K);
+  const QKVChoice c = qkv_choice(M, N, K, false);
   *n_big = c.n_big;
   return c.rows;
 }
+// ... 1: tiles of 256 x 256 in its place.
+extern "C" int ti_gemm_bf16_qkv_wide(int M, int N, int K) { return qkv_choice(M, N, K, true).rows == 512; }
 
 // The fused q/k/v projection of a step's rows with the per-head work in its epilogue (see
 // QKVEpilogue): A [M, K] bf16, W [(n_head + 2 n_kv) hd, K] bf16 (n_kv = 0: q heads only, nothing is
@@ -1904,7 +1909,7 @@ extern "C" int ti_gemm_bf16_qkv_prep(const void* A, const void* W, int M, int K,
   QKVEpilogue ep{q_w, k_w, eps, inv_freq, (const float2*)rope_table, table_len, pos, slot, table, table_stride,
                  (bf16_t*)pool, (bf16_t*)q_out, n_head, n_kv, hd, page_size};
   const int N = (n_head + 2 * n_kv) * hd;
-  const QKVChoice c = qkv_choice(M, N, K);
+  const QKVChoice c = qkv_choice(M, N, K, true);
   if (!c.rows) {
     ti_set_error("gemm_bf16_qkv_prep: %d rows are left to the product and the preparation kernel", M);
     return 3;

@@ -46,9 +46,10 @@ int ti_tuning_set(const char* name, long value);     // 0, or 1 for a name the l
 void ti_tuning_reset();                              // every choice back to the library's own
 // libti_gemm_bf16: what is chosen for M rows times N output columns.  The tile (by its number above) and, where the columns are
 // split between two (n_big > 0), the second one from column n_big on; the rows of the q/k/v product's tile (0: left to the
-// product and the preparation kernel; 512: tiles of 256 x 256), 256 and 128 where n_big > 0.
+// product and the preparation kernel), 256 and 128 where n_big > 0.
 int ti_gemm_bf16_tile_choice(int swiglu, int M, int N, int K, int* rest, int* n_big);
 int ti_gemm_bf16_qkv_choice(int M, int N, int K, int* n_big);
+int ti_gemm_bf16_qkv_wide(int M, int N, int K);      // 1: tiles of 256 x 256 in its place
 // ... SwiGLU by quarters (tiles 10 and 12), in place of the first; 0: that one
 int ti_gemm_bf16_quarters_ranges(int M, int N, int K, int* rest, int* n_big);
 int ti_gemm_bf16_quarters_choice(int M, int N, int K);
