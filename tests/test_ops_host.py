@@ -80,6 +80,18 @@ def test_context_splits_of_the_decode_kernel(monkeypatch):
             assert 1 <= s <= max(1, min(-(-context // 16) // a.MIN_BLOCKS_PER_SPLIT, a.MAX_SPLITS))
 
 
+@pytest.mark.parametrize("heads,tiles,paired", [
+    (16, 1, False), (16, 17, False), (16, 30, False), (16, 31, True), (16, 32, True), (16, 33, False), (32, 15, False), (32, 16, True), (32, 17, False),
+    (3, 162, False), (3, 163, True), (3, 170, True), (3, 171, False), (1, 486, False), (1, 487, True), (1, 512, True), (1, 513, False), (64, 1 << 20, False)])
+def test_two_tiles_a_workgroup_where_they_are_two_rounds_of_the_units(heads, tiles, paired):
+    """More than 1.9 and up to 2 tiles a unit (256): 487 to 512, whatever their keys; the keys of as many tiles are never cut into runs."""
+    from tinyinfer_amd import native
+    said = ctypes.c_int()
+    for context, window in ((2048, 0), (64, 0), (40000, 0), (40000, 256)):
+        runs = native.lib().ti_portion_launch(tiles, heads, context, window, 256, ctypes.byref(said))
+        assert bool(said.value) == paired and (runs == 1 or 2 * tiles * heads <= 256)
+
+
 def test_what_the_rows_of_a_draw_ask_for_packs_from_any_iterable():
     """Requests and counters as lists, tuples, views and iterators give the same bytes, numbers beyond their type's range what ctypes
     makes of them."""

@@ -1951,11 +1951,10 @@ extern "C" int ti_attention_prefill_bf16(const void* q, const void* pool, const 
   return 0;
 }
 
-// The same for launches of few tiles, with the work evened out under a causal mask.  tiles: int
-// [n_tiles, 2] = (entry, first row) of tiles of 64 rows, ordered from the tile that sees the most
-// keys to the one that sees the fewest; a workgroup takes tile b and tile n_tiles - 1 - b, one
-// after the other, with four groups of two wavefronts taking the turns of keys in rotation.
-// Returns 3 for head sizes other than 64 and 128.
+// The same for launches of few tiles.  tiles: int [n_tiles, 2] = (entry, first row) of tiles of 64 rows, ordered from the
+// tile that sees the most keys to the one that sees the fewest.  A workgroup takes a tile, the heaviest ones of all heads
+// first, or where the caller asks for pairs tile b and tile n_tiles - 1 - b, one after the other; four groups of
+// two wavefronts take the turns of keys in rotation.  Returns 3 for head sizes other than 64 and 128 and for pages of 2 GiB and more.
 extern "C" int ti_attention_prefill_paired_bf16(const void* q, const void* pool, const int* table, int table_stride,
                                                 const int* tiles, const int* entries, void* out, int n_tiles,
                                                 int n_head, int n_kv, int hd, int page_size, float scale,
@@ -1992,8 +1991,7 @@ extern "C" int ti_attention_prefill_paired_bf16(const void* q, const void* pool,
     }
     ready = true;
   }
-  // paired = 0: a workgroup per tile (a launch that fits the chip in one round lasts as long as its
-  // heaviest tile then, not as the heaviest and the lightest together)
+  // (pairs: for about two rounds of the units, see the caller's rule)
   dim3 grid(paired ? (n_tiles + 1) / 2 : n_tiles, n_head, n_splits);
 #define TI_GO(H, PAIRED)                                                                                          \
   attn_prefill_lds_kernel<H, NG, NW, ST, PAIRED, CB><<<grid, 64 * NW * NG, lds, stream>>>(                            \

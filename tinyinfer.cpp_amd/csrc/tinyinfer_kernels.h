@@ -467,13 +467,12 @@ enum { TI_RUN_ROW, TI_RUN_POS, TI_RUN_FIRST, TI_RUN_BLOCKS, TI_RUN_PART, TI_RUN_
 int ti_attention_prefill_bf16(const void* q, const void* pool, const int* table, int table_stride, const int* tiles,
                               const int* entries, void* out, int n_tiles, int n_head, int n_kv, int hd, int page_size,
                               float scale, int window, hipStream_t stream);
-// the same for launches of few tiles (head sizes 64, 128): tiles of 64 rows ordered from the most visible
-// keys to the fewest; a workgroup takes tile b and tile n_tiles - 1 - b, so that all have about the same work
+// the same for launches of few tiles (head sizes 64, 128; pages of less than 2 GiB): tiles of 64 rows ordered from the most
+// visible keys to the fewest.  A workgroup takes a tile, the heaviest of all heads first; paired: tile b and tile n_tiles - 1 - b
 // n_splits > 1 (up to 8): the keys of every tile are cut into that many runs, each with a workgroup of its
 // own, for launches of few tiles against a long context; their results go through part_o [n_rows][n_head]
 // [n_splits][hd] and part_ml [n_rows][n_head][n_splits][2] and are merged into out for all n_rows rows of the
 // step (rows of no tile get what lies in the buffers: whoever owns them writes them afterwards).
-// paired = 0: the same kernel with a workgroup per tile, for launches that fit the chip in one round.
 int ti_attention_prefill_paired_bf16(const void* q, const void* pool, const int* table, int table_stride,
                                      const int* tiles, const int* entries, void* out, int n_tiles, int n_head,
                                      int n_kv, int hd, int page_size, float scale, int window, int n_rows,

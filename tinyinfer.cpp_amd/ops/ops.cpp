@@ -928,12 +928,14 @@ static int typical_context(const AttentionWork& w) {
 
 static const int PORTION_SPLIT_KEYS = 512;   // a portion's keys are cut into runs of at least this many ...
 static const int PORTION_SPLIT_MAX = 8;      // ... at most this many runs
-static const int PAIRED_BELOW = 1025;        // (tiles of 128 rows) x heads below which a launch takes the paired kernel
+static const int PAIRED_BELOW = 1025;        // (tiles of 128 rows) x heads below which a launch takes the kernel with 64-row tiles
 
 // Tiles of 64 rows get a workgroup each, the heaviest first.  Where they are two rounds of the units, or nearly, a workgroup takes the heaviest
 // and the lightest of those left, which spares the second round's starts (us, pairs and a workgroup each: 16 heads of 2,048 tokens 34.3
 // and 35.3, of 1,984 32.9 and 33.9, of 1,920 33.3 and 33.3, of 1,792 31.2 and 30.7, of 1,500 29.6 and 25.7, of 2,176 63.6 and 41.9, of
-// 3,000 81 and 66.5; 32 heads of 1,024 23.1 and 24.1).
+// 3,000 81 and 66.5; 32 heads of 1,024 23.1 and 24.1).  What the tiles see hardly matters: of 40 other steps of 490 to 512 tiles none takes longer in pairs
+// than 1 % (16 heads: 2,048 tokens behind 500 42.7 and 43.2, 2,000 74.9 and 75.0, 8,000 196.9 and 196.2, under a window of 256 18.7 and 19.3;
+// 2 prompts of 1,024 22.4 and 23.0, 4 of 512 17.3 and 18.2, 32 of 64 13.1 and 14.0; 1,024 fresh and 1,024 behind 4,000 65.6 and 65.9).
 // The keys are cut into runs when the launch would leave most units idle (a short portion) while
 // every workgroup walks a long context.
 int Ops::portion_launch(int n_tiles_small, int heads, int portion_context, int window, int units, bool* paired) {
