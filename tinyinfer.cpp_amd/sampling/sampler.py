@@ -27,6 +27,10 @@ class SamplingParams(_Recorded):
     top_p: float = 1.0
     seed: int = 42               # src/main.cpp:27
 
+    def __post_init__(self):
+        if type(self) is SamplingParams:      # (a class derived from it may not have its numbers yet, or change them)
+            _pack(self)
+
     def __getstate__(self):
         return self.__dict__
 
@@ -35,6 +39,17 @@ class SamplingParams(_Recorded):
 
 
 _keep = _Recorded._record.__set__
+
+
+def _pack(p):
+    """What the library reads of a request, once: four lists of a number a request each took longer at every call than its kernels' launches.  None for
+    numbers of other types or out of their type's range, which are converted at every call."""
+    t, k, q, s = p.temperature, p.top_k, p.top_p, p.seed
+    try:
+        plain = type(k) is type(s) is int and (type(t) is float or type(t) is int) and (type(q) is float or type(q) is int)
+        _keep(p, _RECORD.pack(t, k, q, s & ((1 << 64) - 1)) if plain else None)
+    except (struct.error, OverflowError):
+        _keep(p, None)
 
 
 def uniform(seed: int, request: int, n_generated: int) -> float:
@@ -76,8 +91,8 @@ class Sampler:
 
     @staticmethod
     def _records(n, params, requests, counters):
-        """The same from the parameters' own records, or None where one of them can have none or a number does not fit.  A record is packed at its
-        first draw (64 rows: kept ones 5 us, new ones 29, the lists above 17; a whole call of 64 rows of 151,936 with kept ones 61.6 -> 55.3)."""
+        """The same from the parameters' own records, or None where one of them can have none or a number does not fit (64 rows: 5 us, 17 above; a whole
+        call of 64 rows of 151,936 61.6 -> 55.3)."""
         try:
             if not len(params) == len(requests) == len(counters) == n or (n and {*map(type, params)} != {SamplingParams}):
                 return None
@@ -86,13 +101,8 @@ class Sampler:
             try:
                 records = [p._record for p in params]
             except AttributeError:
-                for p in params:
-                    t, k, q, s = p.temperature, p.top_k, p.top_p, p.seed
-                    try:      # (numbers of other types, or out of their type's range, are converted at every call)
-                        plain = type(k) is type(s) is int and (type(t) is float or type(t) is int) and (type(q) is float or type(q) is int)
-                        _keep(p, _RECORD.pack(t, k, q, s & ((1 << 64) - 1)) if plain else None)
-                    except (struct.error, OverflowError):
-                        _keep(p, None)
+                for p in params:              # (of a pickle or a copy)
+                    _pack(p)
                 records = [p._record for p in params]
             return (b"".join(records),) + words
         except (AttributeError, TypeError, struct.error, OverflowError):
