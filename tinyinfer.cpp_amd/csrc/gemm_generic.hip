@@ -579,22 +579,25 @@ static int launch_f32_shared(const float* A, const float* W, float* out, int M, 
 // start, its products (RB NB) and its operands (RB + NB blocks to split, four times a product's weight each).
 // Fitted to 1 to 1,000 rows times the weights of Qwen3-0.6B's sizes: the tile it picks is on average 0.9 % slower than the
 // fastest (300 x 1024 x 3072: 32 x 48 20.2 us, 16 x 80 22.4), and 0.3 % over those and the 1.7B to 4B sizes with the present kernel.
-static long f32_tile_cost(int rb, int nb, bool sw, int M, int N, int units) {
-  const long tiles = (long)((M + 16 * nb - 1) / (16 * nb)) * ((N + 16 * rb - 1) / (16 * rb));
+// dies = 8: by the rounds of the die that has the most columns of tiles.
+static long f32_tile_cost(int rb, int nb, bool sw, int M, int N, int units, int dies = 1) {
+  const long columns = (N + 16 * rb - 1) / (16 * rb), tiles = (long)((M + 16 * nb - 1) / (16 * nb)) * ((columns + dies - 1) / dies);
   const int pl = sw ? 2 : 1;
+  units = (units + dies - 1) / dies;
   const long rounds = (tiles + units - 1) / units;
   return rounds * (2 + pl * rb * nb + 4 * (pl * rb + nb));
 }
 
 // Whether the tiles with shared splits take it, 64 tokens x 128 weight rows (SwiGLU: 64 gates and their ups).  The dies take columns of tiles in turn, so
-// what counts is the rounds of the die that has the most.  A unit holds two workgroups of the former (four wavefronts of 242 registers): a round is 3 us
-// and 1.6 a k-step of both, 1.05 where there is one each.  Of the latter (eight wavefronts of 145) it holds one: 2.5 us and 0.86 a k-step a round.
-// The other kernel's cost is worth 0.075 us and 0.256 a thousand of K.  Over 232 products of thirteen weights, 40 to 3,000 rows, what this chooses is on
-// average 0.04 % slower than the faster of the two, at worst 2.3 % (rounds of all units at one rate, a tenth in favour of the other: 0.7 and 17 %).
+// what counts is the rounds of the die that has the most.  A unit holds two workgroups of the former (four wavefronts of 242 registers): a round is 4 us
+// and 1.55 a k-step of both, 1.05 where there is one each.  Of the latter (eight wavefronts of 145) it holds one: 2.5 us and 0.86 a k-step a round.
+// The other kernel's cost, counted so, is worth 0.075 us and 0.256 a thousand of K (95 of 100 within 13 %).  Over 307 products, thirteen weights under 40
+// to 3,000 rows and 60 of random sizes, what this chooses is on average 0.13 % slower than the faster of the two, at worst 9 % (rounds of all units at one
+// rate, a tenth in favour of the other: 1.1 and 52 %).
 // us, the other and this: 64 rows of 151936 x 1024 214 172, 300 790 654; [gate; up] 6144 x 1024 under 200 rows 30.4 31.0, 256 34.6 29.9, 512 51 58, 1,000
 // 104 90, 9728 x 896 under 600 92 102, 384 64 52, 19456 x 2560 under 64 79 67, 512 365 342; 4096 x 1024 under 512 37.1 38.5, 1,000 73 60, 2,000 153 114;
 // 6144 x 4096 under 300 108 135, 2,048 699 665.
-static bool f32_shared_serves(long other_cost, bool sw, int M, int N, int K, long lda) {
+static bool f32_shared_serves(int rb, int nb, bool sw, int M, int N, int K, long lda) {
   // whole k-steps, and a tile's rows within what a buffer's descriptor spans
   if (K % GF_STEP || K >= (1 << 20) || lda >= (1 << 20)) return false;
   const long columns = (N + (sw ? 63 : 127)) / (sw ? 64 : 128), tiles = (long)((M + 63) / 64) * ((columns + 7) / 8), units = (compute_units() + 7) / 8;      // of a die
@@ -603,13 +606,13 @@ static bool f32_shared_serves(long other_cost, bool sw, int M, int N, int K, lon
   if (sw) us += (double)((tiles + units - 1) / units) * (2.5 + 0.86 * steps);
   else {
     const long rest = tiles % (2 * units);
-    us += (double)(tiles / (2 * units) + (rest > units)) * (3.0 + 1.6 * steps) + (rest > 0 && rest <= units ? 3.0 + 1.05 * steps : 0.0);
+    us += (double)(tiles / (2 * units) + (rest > units)) * (4.0 + 1.55 * steps) + (rest > 0 && rest <= units ? 4.0 + 1.05 * steps : 0.0);
   }
-  return us < 2.7 + other_cost * (0.075 + 0.256 * K / 1024);
+  return us < 2.7 + f32_tile_cost(rb, nb, sw, M, N, compute_units(), 8) * (0.075 + 0.256 * K / 1024);
 }
 
-// the tile of gemm_f32_kernel that costs the least, and its cost
-static long f32_best_tile(bool sw, int M, int N, int& rb, int& nb) {
+// the tile of gemm_f32_kernel that costs the least
+static void f32_best_tile(bool sw, int M, int N, int& rb, int& nb) {
   static const int TILES[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 5}, {2, 2}, {2, 3}, {2, 4}, {2, 5}, {4, 2}, {4, 4}};
   long best = -1;
   for (const auto& t : TILES) {
@@ -621,22 +624,22 @@ static long f32_best_tile(bool sw, int M, int N, int& rb, int& nb) {
       nb = t[1];
     }
   }
-  return best;
 }
 
 // What is chosen, for tests: 1: the tiles with shared splits.
 extern "C" int ti_gemm_generic_f32_choice(int swiglu, int M, int N, int K, long lda) {
   int rb, nb;
-  return f32_shared_serves(f32_best_tile(swiglu != 0, M, N, rb, nb), swiglu != 0, M, N, K, lda) ? 1 : 0;
+  f32_best_tile(swiglu != 0, M, N, rb, nb);
+  return f32_shared_serves(rb, nb, swiglu != 0, M, N, K, lda) ? 1 : 0;
 }
 
 static int launch_f32(const float* A, const float* W, float* out, int M, int N, int K, long lda, int epi, hipStream_t stream) {
   const bool sw = epi == TI_EPI_SWIGLU;
   int rb, nb;
-  const long best = f32_best_tile(sw, M, N, rb, nb);
+  f32_best_tile(sw, M, N, rb, nb);
   const int wide_out = N % 4 == 0 && ((uintptr_t)out & 15) == 0;
   const int run = ((K + GF_RUNS - 1) / GF_RUNS + GF_STEP - 1) / GF_STEP * GF_STEP;
-  if (f32_shared_serves(best, sw, M, N, K, lda))
+  if (f32_shared_serves(rb, nb, sw, M, N, K, lda))
     return sw ? launch_f32_shared<4, 2, 1, 2, true>(A, W, out, M, N, K, lda, run, epi, wide_out, stream)
               : launch_f32_shared<2, 2, 4, 2, false>(A, W, out, M, N, K, lda, run, epi, wide_out, stream);
   const int m_tiles = (M + 16 * nb - 1) / (16 * nb), n_tiles = (N + 16 * rb - 1) / (16 * rb);
