@@ -2085,6 +2085,31 @@ def test_attention_bf16_portions_at_the_edges_of_runs(ops, nh, nkv, hd, P, varia
     assert (got - want).abs().max() < 2e-2          # as above: weights and results rounded to 8 bits of values of up to 4
 
 
+@pytest.mark.parametrize("nh,nkv,hd", [(32, 4, 128), (16, 2, 128), (28, 4, 64), (8, 1, 128), (15, 3, 128), (5, 5, 64), (12, 12, 64), (16, 8, 128)])
+@pytest.mark.parametrize("portions", [1, 3, 8])
+def test_attention_bf16_tiles_whose_heads_stand_together(ops, nh, nkv, hd, portions):
+    """Every head of every tile once, with the bits of the heads dealt out one by one, whole and in runs of keys, for numbers of tiles times kv heads
+    that eight divides and others."""
+    g = torch.Generator().manual_seed(nh + portions)
+    entries = [(64 + 37 * e, 100 * e) for e in range(portions)]
+    ctx, pages = FakeCtx(entries), 64
+    pool = dev(torch.randn(portions * pages, 2, nkv, 16, hd, generator=g).to(torch.bfloat16))
+    table = dev(torch.randperm(portions * pages, generator=g).to(torch.int32).view(portions, pages))
+    q = dev(torch.randn(ctx.M, nh * hd, generator=g).to(torch.bfloat16))
+    lib, ptr = ops.lib("attention_bf16"), lambda t: t.data_ptr()
+    part_o, part_ml = torch.zeros(ctx.M, nh, 2, hd, device="cuda"), torch.zeros(ctx.M, nh, 2, 2, device="cuda")
+    for runs in (1, 2):
+        outs = []
+        for order in (0, 2):
+            out = torch.full_like(q, 7.0)
+            rc = lib.ti_attention_prefill_paired_bf16(ptr(q), ptr(pool), ptr(table), pages, ptr(ctx.tiles_small), ptr(ctx.entry_meta), ptr(out),
+                                                      ctx.n_tiles_small, nh, nkv, hd, 16, hd ** -0.5, 0, ctx.M, ptr(part_o), ptr(part_ml), runs, order,
+                                                      torch.cuda.current_stream().cuda_stream)
+            assert rc == 0, lib.ti_last_error()
+            outs.append(out)
+        assert torch.equal(outs[0], outs[1]) and not bool((outs[0] == 7.0).all(dim=1).any())
+
+
 @pytest.mark.parametrize("nh,nkv,P", [(32, 32, 131072), (2, 1, 1 << 23)])
 def test_attention_bf16_portions_in_pages_of_2_gib_and_more(ops, nh, nkv, P):
     """Pages of more than a buffer descriptor spans, which the kernel takes that reads flat addresses: what pages of 16 rows give, with a sink in

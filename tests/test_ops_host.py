@@ -92,6 +92,17 @@ def test_two_tiles_a_workgroup_where_they_are_two_rounds_of_the_units(heads, til
         assert bool(said.value) == paired and (runs == 1 or 2 * tiles * heads <= 256)
 
 
+@pytest.mark.parametrize("portions,tokens,start,kv_heads,together", [
+    (12, 64, 500, 4, True), (12, 64, 500, 2, True), (32, 64, 1500, 4, True), (8, 500, 0, 4, True), (5, 130, 700, 4, True), (12, 64, 500, 3, True),
+    (12, 64, 500, 8, False), (12, 64, 500, 16, False), (12, 100, 0, 4, False), (6, 200, 0, 4, False), (3, 500, 0, 4, False), (1, 2048, 0, 4, False),
+    (1, 64, 100000, 4, False), (2, 1000, 0, 4, False), (2, 512, 8000, 4, True), (0, 0, 0, 4, False)])
+def test_which_tiles_have_their_heads_on_one_die(portions, tokens, start, kv_heads, together):
+    """Several portions of up to eight tiles each, whose keys and values are more than 4 MiB, under kv heads that eight does not divide."""
+    from tinyinfer_amd import native
+    tiles = portions * -(-tokens // 64)
+    assert native.lib().ti_heads_together(portions, portions * (tokens + start), tiles, kv_heads, 128) == together
+
+
 def test_what_the_rows_of_a_draw_ask_for_packs_from_any_iterable():
     """Requests and counters as lists, tuples, views and iterators give the same bytes, numbers beyond their type's range what ctypes
     makes of them."""

@@ -1166,7 +1166,7 @@ struct PrefillLds {
 //   n_splits > 1: the keys a tile sees are cut into n_splits runs of whole turns, the workgroup takes
 //   run `split` and leaves its maxima, sums and unscaled outputs in part_ml [row][head][split] = (m, l) and
 //   part_o [row][head][split][HD] for the kernel that merges them
-template <int HD, int NG, int NW, int ST, bool PAIRED, int CB>
+template <int HD, int NG, int NW, int ST, bool PAIRED, int CB, bool TOGETHER>
 __device__ __forceinline__ void
 prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int split, const bf16_t* __restrict__ q,
               const bf16_t* __restrict__ pool, const int* __restrict__ table, int table_stride,
@@ -1191,7 +1191,9 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   // of the units is ever smaller and the units end together.  (With a head's tiles behind one another the last heads' largest tiles started
   // last.  us, tiles of 64 rows, heads first and tiles first: 32 heads of 700 tokens 21.9 and 16.9, of 1,500 47.6 and 42.8; 16 of 2,048
   // 37.4 and 35.3.)  Workgroups go to the eight XCDs in turn (linear id mod 8) and each XCD has an L2 of its own: with a multiple of
-  // eight kv heads, an XCD is given whole kv heads, so that the keys and values of a head are read into one L2 only.
+  // eight kv heads, an XCD is given whole kv heads, so that the keys and values of a head are read into one L2 only.  With others a tile's heads
+  // are dealt out one by one and every L2 reads all kv heads, which costs nothing while they fit; TOGETHER: the heads that read a tile's keys
+  // stand behind one another on one XCD, and what is no multiple of eight such groups comes last.
   int head;
   {
     const int id = by * gx + bx, group = n_head / n_kv;
@@ -1199,6 +1201,11 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
       const int xcd = id & 7, local = id >> 3, heads = n_head / 8, nth = local % heads;      // heads: an XCD's
       bx = local / heads;
       head = (xcd + 8 * (nth / group)) * group + nth % group;
+    } else if (TOGETHER) {
+      const int spread = (gx * n_kv) & ~7, rest = id - spread * group, local = rest < 0 ? id >> 3 : rest;
+      const int unit = rest < 0 ? (local / group) * 8 + (id & 7) : spread + local / group;
+      bx = unit / n_kv;
+      head = (unit % n_kv) * group + local % group;
     } else {
       bx = id / n_head;
       head = id % n_head;
@@ -1721,7 +1728,7 @@ prefill_tiles(unsigned char* smem, int bx, int by, int gx, int n_splits, int spl
   }   // slot
 }
 
-template <int HD, int NG, int NW = 4, int ST = PF_STAGES, bool PAIRED = false, int CB = 1>
+template <int HD, int NG, int NW = 4, int ST = PF_STAGES, bool PAIRED = false, int CB = 1, bool TOGETHER = false>
 __global__ void __launch_bounds__(64 * NW * NG)
 attn_prefill_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool,
                         const int* __restrict__ table, int table_stride, const int* __restrict__ tiles,
@@ -1729,7 +1736,7 @@ attn_prefill_lds_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__
                         int n_kv, int P, float scale, int window, float* __restrict__ part_o = nullptr,
                         float* __restrict__ part_ml = nullptr, float softcap = 0.f, const float* __restrict__ sink = nullptr) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  prefill_tiles<HD, NG, NW, ST, PAIRED, CB>(smem, blockIdx.x, blockIdx.y, gridDim.x, gridDim.z, blockIdx.z, q, pool, table,
+  prefill_tiles<HD, NG, NW, ST, PAIRED, CB, TOGETHER>(smem, blockIdx.x, blockIdx.y, gridDim.x, gridDim.z, blockIdx.z, q, pool, table,
                                             table_stride, tiles, n_tiles, entries, out, n_head, n_kv, P, scale, window, part_o,
                                             part_ml, softcap, sink);
 }
@@ -1748,7 +1755,7 @@ attn_step_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ pool, 
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   const int n_pre = n_tiles * n_head, id = blockIdx.x;
   if (id < n_pre) {
-    prefill_tiles<HD, 4, 2, 2, false, 1>(smem, id % n_tiles, id / n_tiles, n_tiles, 1, 0, q, pool, table, table_stride, tiles,
+    prefill_tiles<HD, 4, 2, 2, false, 1, false>(smem, id % n_tiles, id / n_tiles, n_tiles, 1, 0, q, pool, table, table_stride, tiles,
                                          n_tiles, entries, out, n_head, n_kv, P, scale, window, nullptr, nullptr, softcap, sink);
   } else {
     const int at = id - n_pre, ways = n_kv * ((group + 15) / 16);
@@ -1953,8 +1960,8 @@ extern "C" int ti_attention_prefill_bf16(const void* q, const void* pool, const 
 
 // The same for launches of few tiles.  tiles: int [n_tiles, 2] = (entry, first row) of tiles of 64 rows, ordered from the
 // tile that sees the most keys to the one that sees the fewest.  A workgroup takes a tile, the heaviest ones of all heads
-// first, or where the caller asks for pairs tile b and tile n_tiles - 1 - b, one after the other; four groups of
-// two wavefronts take the turns of keys in rotation.  Returns 3 for head sizes other than 64 and 128 and for pages of 2 GiB and more.
+// first, or where the caller asks for pairs (1) tile b and tile n_tiles - 1 - b, one after the other; 2: a tile, its heads together (see
+// prefill_tiles); four groups of two wavefronts take the turns of keys in rotation.  Returns 3 for head sizes other than 64 and 128 and for pages of 2 GiB and more.
 extern "C" int ti_attention_prefill_paired_bf16(const void* q, const void* pool, const int* table, int table_stride,
                                                 const int* tiles, const int* entries, void* out, int n_tiles,
                                                 int n_head, int n_kv, int hd, int page_size, float scale,
@@ -1984,6 +1991,10 @@ extern "C" int ti_attention_prefill_paired_bf16(const void* q, const void* pool,
                             hipFuncAttributeMaxDynamicSharedMemorySize, PrefillLds<64, NG, NW, ST>::BYTES) != hipSuccess ||
         hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<128, NG, NW, ST, false, CB>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, PrefillLds<128, NG, NW, ST>::BYTES) != hipSuccess ||
+        hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<128, NG, NW, ST, false, CB, true>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, PrefillLds<128, NG, NW, ST>::BYTES) != hipSuccess ||
+        hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<64, NG, NW, ST, false, CB, true>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, PrefillLds<64, NG, NW, ST>::BYTES) != hipSuccess ||
         hipFuncSetAttribute((const void*)attn_prefill_lds_kernel<64, NG, NW, ST, false, CB>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, PrefillLds<64, NG, NW, ST>::BYTES) != hipSuccess) {
       ti_set_error("attention_prefill_paired: cannot reserve the LDS");
@@ -1991,16 +2002,19 @@ extern "C" int ti_attention_prefill_paired_bf16(const void* q, const void* pool,
     }
     ready = true;
   }
-  // (pairs: for about two rounds of the units, see the caller's rule)
-  dim3 grid(paired ? (n_tiles + 1) / 2 : n_tiles, n_head, n_splits);
-#define TI_GO(H, PAIRED)                                                                                          \
-  attn_prefill_lds_kernel<H, NG, NW, ST, PAIRED, CB><<<grid, 64 * NW * NG, lds, stream>>>(                            \
+  const bool pairs = paired == 1;
+  dim3 grid(pairs ? (n_tiles + 1) / 2 : n_tiles, n_head, n_splits);
+#define TI_GO(H, PAIRED, TOGETHER)                                                                                \
+  attn_prefill_lds_kernel<H, NG, NW, ST, PAIRED, CB, TOGETHER><<<grid, 64 * NW * NG, lds, stream>>>(                            \
       (const bf16_t*)q, (const bf16_t*)pool, table, table_stride, tiles, n_tiles, entries, (bf16_t*)out, n_head, \
       n_kv, page_size, scale, window, part_o, part_ml, g_softcap, g_sink)
-  if (hd == 128 && paired) TI_GO(128, true);
-  else if (hd == 128) TI_GO(128, false);
-  else if (paired) TI_GO(64, true);
-  else TI_GO(64, false);
+  const bool together = paired == 2 && n_kv % 8 != 0;
+  if (hd == 128 && pairs) TI_GO(128, true, false);
+  else if (hd == 128 && together) TI_GO(128, false, true);
+  else if (hd == 128) TI_GO(128, false, false);
+  else if (pairs) TI_GO(64, true, false);
+  else if (together) TI_GO(64, false, true);
+  else TI_GO(64, false, false);
 #undef TI_GO
   if (n_splits > 1) {
     // every row of the step has its runs (rows of single tokens too: theirs are not read by anyone)

@@ -468,7 +468,8 @@ int ti_attention_prefill_bf16(const void* q, const void* pool, const int* table,
                               const int* entries, void* out, int n_tiles, int n_head, int n_kv, int hd, int page_size,
                               float scale, int window, hipStream_t stream);
 // the same for launches of few tiles (head sizes 64, 128; pages of less than 2 GiB): tiles of 64 rows ordered from the most
-// visible keys to the fewest.  A workgroup takes a tile, the heaviest of all heads first; paired: tile b and tile n_tiles - 1 - b
+// visible keys to the fewest.  A workgroup takes a tile, the heaviest of all heads first; paired = 1: tile b and tile n_tiles - 1 - b;
+// 2: a tile, the heads that read its keys behind one another on a die (kv heads that are no multiple of eight)
 // n_splits > 1 (up to 8): the keys of every tile are cut into that many runs, each with a workgroup of its
 // own, for launches of few tiles against a long context; their results go through part_o [n_rows][n_head]
 // [n_splits][hd] and part_ml [n_rows][n_head][n_splits][2] and are merged into out for all n_rows rows of the

@@ -1561,6 +1561,9 @@ int ti_portion_launch(int n_tiles_small, int heads, int portion_context, int win
   if (paired) *paired = p ? 1 : 0;
   return s;
 }
+int ti_heads_together(int portions, int64_t portion_keys, int n_tiles_small, int kv_heads, int head_dim) {
+  return Ops::heads_together(portions, (long)portion_keys, n_tiles_small, kv_heads, head_dim) ? 1 : 0;
+}
 int ti_portions_with_rows(int n_tiles_small, int context, int least_context, int n_rows, int longest_blocks, long row_blocks, int max_seq, int heads,
                           int kv_heads, int window, int units, int head_dim) {
   Ops::PortionsLaunch p;

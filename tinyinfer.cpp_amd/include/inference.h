@@ -611,6 +611,7 @@ class Ops {
   static double portion_us(int portion_context, int window);
   // runs of keys for the prefill kernel with 64-row tiles, and whether it pairs a heavy with a light tile
   static int portion_launch(int n_tiles_small, int heads, int portion_context, int window, int units, bool* paired);
+  static bool heads_together(int portions, long portion_keys, int n_tiles_small, int kv_heads, int head_dim);
 
  private:
   void* launch_stream();
@@ -675,6 +676,8 @@ struct AttentionWork {
   bool slots_are_rows = false;       // slots[m] == m for every row (a step of single tokens, one entry a row)
   int max_context = 0;               // longest context any row reads
   int portion_context = 0;           // ... over rows of entries of several tokens
+  int portions = 0;                  // entries of several tokens (0: not known)
+  long portion_keys = 0;             // the positions that those see, all together
   int split_context = 0;             // the context the decode kernel's runs are sized for
 };
 
@@ -1393,6 +1396,7 @@ int ti_ops_call(void* ops, const char* op, const ti_tensor* t, int n_t, const do
                 const char* text, ti_tensor* result);
 int ti_ops_timing_report(void* ops, const char** out_json);     // [{"name", "calls", "us"}] since timing was switched on
 int ti_decode_splits(int n_rows, int kv_heads, int heads, int context, int typical, int units, int head_dim);
+int ti_heads_together(int portions, int64_t portion_keys, int n_tiles_small, int kv_heads, int head_dim);
 int ti_portion_launch(int n_tiles_small, int heads, int portion_context, int window, int units, int* paired);
 // the runs that a step of n_rows single tokens is cut into, each behind `blocks` blocks of 16 (Ops::plan_runs)
 int ti_decode_runs(int n_rows, int blocks, int max_seq, int heads, int kv_heads, int units, int head_dim);

@@ -203,6 +203,8 @@ def lib() -> ctypes.CDLL:
         handle.ti_uniform.argtypes = [c_u64, c_u64, c_u64]
         handle.ti_decode_splits.restype = c_int
         handle.ti_decode_splits.argtypes = [c_int] * 7
+        handle.ti_heads_together.restype = c_int
+        handle.ti_heads_together.argtypes = [c_int, ctypes.c_int64, c_int, c_int, c_int]
         handle.ti_portion_launch.restype = c_int
         handle.ti_portion_launch.argtypes = [c_int] * 5 + [P(c_int)]
         handle.ti_decode_runs.restype = c_int

@@ -948,6 +948,15 @@ int Ops::portion_launch(int n_tiles_small, int heads, int portion_context, int w
   return std::max(1, std::min({PORTION_SPLIT_MAX, units / workgroups, context / PORTION_SPLIT_KEYS}));
 }
 
+// Whether a tile's heads stand together on a die where the kv heads are no multiple of eight: for several portions of few tiles whose keys and
+// values are more than a die's L2, which eight of them would else all bring in.  Up to that size, and for few long portions, whose tiles
+// walk the same keys side by side, the heads dealt out one by one are the faster.  us, dealt out and together, 32 heads on 4: 12 portions of 64 tokens behind 500
+// 29.1 25.1, behind 1,500 55.6 45.2, 32 of 64 behind 1,500 127 90, 12 of 130 behind 700 84 68, 8 of 500 74 68, 8 of 300 41 39; 12 of 100 20.4 21.3, 6 of
+// 200 21.3 22.0, 3 of 500 26.9 27.4, one of 2,048 63 66; 16 on 2: 12 of 64 behind 500 16.3 14.1.
+bool Ops::heads_together(int portions, long portion_keys, int n_tiles_small, int kv_heads, int head_dim) {
+  return kv_heads % 8 != 0 && portions > 1 && n_tiles_small <= 8 * portions && portion_keys * kv_heads * head_dim * 4 > (4L << 20);
+}
+
 bool Ops::attention_from_projections(const AttentionWork& work, Workspace& ws, const CacheView& view, const Tensor& qkv,
                                      const float* q_w, const float* k_w, float eps, const Rotation& rot,
                                      const Tensor& pool, bool write_kv, const Tensor& out, int heads, int kv_heads,
@@ -1060,6 +1069,7 @@ bool Ops::attention(const AttentionWork& work, Workspace& ws, const CacheView& v
         int S = portion_launch(work.n_tiles_small, heads, work.portion_context, window, units, &paired);
         if (!use.portion_splits) S = 1;
         if (use.force_paired_tiles >= 0) paired = use.force_paired_tiles != 0;
+        const int each = heads_together(work.portions, work.portion_keys, work.n_tiles_small, kv_heads, head_dim) ? 2 : 0;
         float *part_o = nullptr, *part_ml = nullptr;
         if (S > 1) {
           part_o = (float*)ws.get("attn.portion_o", (size_t)work.M * heads * S * head_dim * 4);
@@ -1067,7 +1077,7 @@ bool Ops::attention(const AttentionWork& work, Workspace& ws, const CacheView& v
         }
         int rc = KERNEL("attention_bf16", ti_attention_prefill_paired_capped_bf16)(
             q.data, pool.data, view.table, view.table_width, work.tiles_small, work.entry_meta, out.data, work.n_tiles_small,
-            heads, kv_heads, head_dim, P, scale, softcap, window, (int)work.M, part_o, part_ml, S, paired ? 1 : 0,
+            heads, kv_heads, head_dim, P, scale, softcap, window, (int)work.M, part_o, part_ml, S, paired ? 1 : each,
             (hipStream_t)stream);
         if (rc != 3) {
           check("attention_bf16", rc, "attention(prefill, paired)");

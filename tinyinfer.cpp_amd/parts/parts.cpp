@@ -861,7 +861,8 @@ class Attention final : public MixerPart {
     std::vector<Tile> large, little;
     large.reserve(n_tiles);
     little.reserve(n_small);
-    int portion_context = 0;
+    int portion_context = 0, portions = 0;
+    long portion_keys = 0;
     size_t d = 0;
     for (size_t i = 0; i < entries.size(); ++i) {
       const auto& e = entries[i];
@@ -871,6 +872,8 @@ class Attention final : public MixerPart {
         for (int q0 = 0; q0 < e.n_tokens; q0 += PREFILL_TILE_SMALL)
           little.push_back({e.start + std::min(q0 + PREFILL_TILE_SMALL, e.n_tokens) - 1, (int)i, e.row0 + q0});
         portion_context = std::max(portion_context, e.start + e.n_tokens);
+        portions += 1;
+        portion_keys += e.start + e.n_tokens;
       } else {
         dec[d++] = e.row0;
       }
@@ -882,6 +885,8 @@ class Attention final : public MixerPart {
     list(large, tiles);
     list(little, small);
     plan.set_value("attention.portion_context", portion_context);
+    plan.set_value("attention.portions", portions);
+    plan.set_value("attention.portion_keys", portion_keys);
   }
 
   AttentionWork work(const StepContext& ctx) const {
@@ -902,6 +907,8 @@ class Attention final : public MixerPart {
       w.decode_rows = ctx.planned("attention.decode_rows");
       w.n_decode_rows = (int)ctx.planned_size("attention.decode_rows");
       w.portion_context = (int)ctx.value("attention.portion_context");
+      w.portions = (int)ctx.value("attention.portions");
+      w.portion_keys = (long)ctx.value("attention.portion_keys");
     }
     if (ctx.plan && ctx.engine && !general && !gated) {
       const std::string key = runs_key(ctx.binding(this).first);
