@@ -80,16 +80,20 @@ def test_context_splits_of_the_decode_kernel(monkeypatch):
             assert 1 <= s <= max(1, min(-(-context // 16) // a.MIN_BLOCKS_PER_SPLIT, a.MAX_SPLITS))
 
 
-@pytest.mark.parametrize("heads,tiles,paired", [
-    (16, 1, False), (16, 17, False), (16, 30, False), (16, 31, True), (16, 32, True), (16, 33, False), (32, 15, False), (32, 16, True), (32, 17, False),
-    (3, 162, False), (3, 163, True), (3, 170, True), (3, 171, False), (1, 486, False), (1, 487, True), (1, 512, True), (1, 513, False), (64, 1 << 20, False)])
-def test_two_tiles_a_workgroup_where_they_are_two_rounds_of_the_units(heads, tiles, paired):
-    """More than 1.9 and up to 2 tiles a unit (256): 487 to 512, whatever their keys; the keys of as many tiles are never cut into runs."""
+@pytest.mark.parametrize("heads,tiles,paired,light", [
+    (16, 1, 0, 0), (16, 16, 0, 0), (16, 17, 0, 0), (16, 19, 0, 0), (16, 20, 0, 1), (16, 21, 0, 1), (16, 30, 0, 1), (16, 31, 1, 1), (16, 32, 1, 1), (16, 33, 0, 0),
+    (16, 48, 0, 0), (16, 51, 0, 0), (16, 52, 0, 1), (16, 62, 0, 1), (16, 63, 1, 1), (16, 64, 1, 1), (16, 65, 0, 0), (16, 96, 1, 1), (16, 112, 0, 0), (16, 128, 1, 1),
+    (32, 15, 0, 1), (32, 16, 1, 1), (32, 17, 0, 0), (3, 162, 0, 1), (3, 163, 1, 1), (3, 170, 1, 1), (3, 171, 0, 0), (1, 319, 0, 0), (1, 320, 0, 1), (0, 0, 0, 0),
+    (64, 1 << 20, 1, 1)])
+def test_two_tiles_a_workgroup_where_they_are_an_even_number_of_rounds(heads, tiles, paired, light):
+    """On 256 units, in the last tenth of an even round; light tiles (up to 256 keys, by their context or their window) from its first quarter on.  The keys
+    of as many tiles are never cut into runs."""
     from tinyinfer_amd import native
     said = ctypes.c_int()
-    for context, window in ((2048, 0), (64, 0), (40000, 0), (40000, 256)):
+    for context, window, want in ((2048, 0, paired), (257, 0, paired), (40000, 0, paired), (40000, 256, paired), (256, 0, light), (64, 0, light), (40000, 128, light)):
         runs = native.lib().ti_portion_launch(tiles, heads, context, window, 256, ctypes.byref(said))
-        assert bool(said.value) == paired and (runs == 1 or 2 * tiles * heads <= 256)
+        assert bool(said.value) == want, (context, window)
+        assert runs == 1 or (not want and 2 * tiles * heads <= 256)
 
 
 @pytest.mark.parametrize("portions,tokens,start,kv_heads,together", [

@@ -930,18 +930,23 @@ static const int PORTION_SPLIT_KEYS = 512;   // a portion's keys are cut into ru
 static const int PORTION_SPLIT_MAX = 8;      // ... at most this many runs
 static const int PAIRED_BELOW = 1025;        // (tiles of 128 rows) x heads below which a launch takes the kernel with 64-row tiles
 
-// Tiles of 64 rows get a workgroup each, the heaviest first.  Where they are two rounds of the units, or nearly, a workgroup takes the heaviest
-// and the lightest of those left, which spares the second round's starts (us, pairs and a workgroup each: 16 heads of 2,048 tokens 34.3
-// and 35.3, of 1,984 32.9 and 33.9, of 1,920 33.3 and 33.3, of 1,792 31.2 and 30.7, of 1,500 29.6 and 25.7, of 2,176 63.6 and 41.9, of
-// 3,000 81 and 66.5; 32 heads of 1,024 23.1 and 24.1).  What the tiles see hardly matters: of 40 other steps of 490 to 512 tiles none takes longer in pairs
-// than 1 % (16 heads: 2,048 tokens behind 500 42.7 and 43.2, 2,000 74.9 and 75.0, 8,000 196.9 and 196.2, under a window of 256 18.7 and 19.3;
-// 2 prompts of 1,024 22.4 and 23.0, 4 of 512 17.3 and 18.2, 32 of 64 13.1 and 14.0; 1,024 fresh and 1,024 behind 4,000 65.6 and 65.9).
+// Tiles of 64 rows get a workgroup each, the heaviest first.  Two of them in one, the heaviest and the lightest of those left, spare a start, and
+// take as many rounds where the tiles are an even number of them, the last one nearly full, or in any even one from its first quarter on where
+// all tiles are light (keys of up to 256).  Otherwise they cost a round, or the units that are through with a light tile wait for the end of a heavy
+// pair.  us, pairs and a workgroup each, heads of 128: 2 rounds: 16 heads of 2,048 tokens 34.3 and 35.3, of 1,984 32.9 and 33.9, of 1,920 33.3
+// and 33.3, of 1,792 31.2 and 30.7, of 1,500 29.6 and 25.7, 2,048 behind 500 42.7 and 43.2, behind 8,000 196.9 and 196.2, 32 portions of 64
+// 13.1 and 14.0; 3: 16 heads of 2,176 63.6 and 41.9, of 3,000 81 and 66.5, 32 heads, 20 portions of 64 24.0 and 20.3; 4: 32 heads of 2,048 63.3 and
+// 64.3, 8 of 200 27.4 and 29.0, 64 heads of 1,024 42.4 and 43.9; 6: 64 heads, 12 of 100 37.3 and 39.3; 8: 32 heads, 8 of 500 65.5 and 67.4.  Light
+// tiles: 16 heads, 20 of 64 (320 tiles) 12.5 and 13.5, 12 of 100 (384) 13.0 and 13.8, 5 of 200 (320) 13.9 and 13.8, 6 of 200 on 12 heads (288) 14.1 and 13.4.
+// Of 90 launches that the rule pairs none takes longer than 2 % by it.  Heads of 64 are two workgroups to a unit, and pairs leave half of them out: a
+// workgroup each (the caller's).
 // The keys are cut into runs when the launch would leave most units idle (a short portion) while
 // every workgroup walks a long context.
 int Ops::portion_launch(int n_tiles_small, int heads, int portion_context, int window, int units, bool* paired) {
   const int context = window == 0 ? portion_context : std::min(portion_context, window + 64);
-  const long tiles = (long)n_tiles_small * heads;
-  const bool pair = 10 * tiles > 19L * units && tiles <= 2L * units;
+  const long tiles = (long)n_tiles_small * heads, rounds = (tiles + units - 1) / units;
+  const bool pair = rounds > 0 && rounds % 2 == 0 &&
+                    (context <= 256 ? 4 * tiles >= (4 * rounds - 3) * units : 10 * tiles > (10 * rounds - 1) * units);
   if (paired) *paired = pair;
   const int workgroups = std::max(1, (pair ? (n_tiles_small + 1) / 2 : n_tiles_small) * heads);
   if (workgroups * 2 > units || context < 2 * PORTION_SPLIT_KEYS) return 1;
@@ -951,7 +956,7 @@ int Ops::portion_launch(int n_tiles_small, int heads, int portion_context, int w
 // Whether a tile's heads stand together on a die where the kv heads are no multiple of eight: for several portions of few tiles whose keys and
 // values are more than a die's L2, which eight of them would else all bring in.  Up to that size, and for few long portions, whose tiles
 // walk the same keys side by side, the heads dealt out one by one are the faster.  us, dealt out and together, 32 heads on 4: 12 portions of 64 tokens behind 500
-// 29.1 25.1, behind 1,500 55.6 45.2, 32 of 64 behind 1,500 127 90, 12 of 130 behind 700 84 68, 8 of 500 74 68, 8 of 300 41 39; 12 of 100 20.4 21.3, 6 of
+// 29.1 25.1, behind 1,500 55.6 45.2, 32 of 64 behind 1,500 127 90 (two tiles a workgroup 127), 12 of 130 behind 700 84 68, 8 of 500 74 68, 8 of 300 41 39; 12 of 100 20.4 21.3, 6 of
 // 200 21.3 22.0, 3 of 500 26.9 27.4, one of 2,048 63 66; 16 on 2: 12 of 64 behind 500 16.3 14.1.
 bool Ops::heads_together(int portions, long portion_keys, int n_tiles_small, int kv_heads, int head_dim) {
   return kv_heads % 8 != 0 && portions > 1 && n_tiles_small <= 8 * portions && portion_keys * kv_heads * head_dim * 4 > (4L << 20);
@@ -1068,8 +1073,9 @@ bool Ops::attention(const AttentionWork& work, Workspace& ws, const CacheView& v
         bool paired = false;
         int S = portion_launch(work.n_tiles_small, heads, work.portion_context, window, units, &paired);
         if (!use.portion_splits) S = 1;
-        if (use.force_paired_tiles >= 0) paired = use.force_paired_tiles != 0;
         const int each = heads_together(work.portions, work.portion_keys, work.n_tiles_small, kv_heads, head_dim) ? 2 : 0;
+        paired = paired && head_dim == 128 && !each;
+        if (use.force_paired_tiles >= 0) paired = use.force_paired_tiles != 0;
         float *part_o = nullptr, *part_ml = nullptr;
         if (S > 1) {
           part_o = (float*)ws.get("attn.portion_o", (size_t)work.M * heads * S * head_dim * 4);
