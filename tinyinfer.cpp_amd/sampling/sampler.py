@@ -94,17 +94,20 @@ class Sampler:
         """The same from the parameters' own records, or None where one of them can have none or a number does not fit (64 rows: 5 us, 17 above; a whole
         call of 64 rows of 151,936 61.6 -> 55.3)."""
         try:
-            if not len(params) == len(requests) == len(counters) == n or (n and {*map(type, params)} != {SamplingParams}):
+            if not len(params) == len(requests) == len(counters) == n:
                 return None
             words = f"{n}q"
-            words = struct.pack(words, *requests), struct.pack(words, *counters)
             try:
-                records = [p._record for p in params]
+                records = b"".join([p._record for p in params])
             except AttributeError:
+                if {*map(type, params)} != {SamplingParams}:
+                    return None
                 for p in params:              # (of a pickle or a copy)
                     _pack(p)
-                records = [p._record for p in params]
-            return (b"".join(records),) + words
+                records = b"".join([p._record for p in params])
+            if len(records) != n * _RECORD.size:      # (somebody else's attribute)
+                return None
+            return records, struct.pack(words, *requests), struct.pack(words, *counters)
         except (AttributeError, TypeError, struct.error, OverflowError):
             return None
 
